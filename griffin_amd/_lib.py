@@ -115,10 +115,30 @@ def load():
         return _lib
 
 
-def available() -> bool:
-    """True when the shared library exists and loads (says nothing about a GPU being present)."""
-    try:
+_native_module = None
+
+
+def native():
+    """The PyTorch operators over the library (csrc/torch_ops.cpp, built next to it); raises RuntimeError when either
+    of the two is missing."""
+    global _native_module, _load_error
+    if _native_module is None:
         load()
+        try:
+            from . import _native
+        except ImportError as error:
+            _load_error = f"its PyTorch operators do not load ({error}); run `python -m griffin_amd.build`"
+            raise RuntimeError("RG-LRU HIP library unavailable: " + _load_error) from error
+        _native_module = _native
+    return _native_module
+
+
+def available() -> bool:
+    """True when the shared library and its operators exist and load (says nothing about a GPU being present)."""
+    if _native_module is not None:
+        return True
+    try:
+        native()
     except RuntimeError:
         return False
     return True

@@ -1,6 +1,7 @@
-"""Build librglru_hip.so (hand-written gfx950 kernels + the C ABI) in-tree with hipcc.
+"""Build librglru_hip.so (hand-written gfx950 kernels + the C ABI) in-tree with hipcc, and _native.so (the PyTorch
+operators over it, host code only) with the host compiler.
 
-    python -m griffin_amd.build            # compile griffin_amd/librglru_hip.so
+    python -m griffin_amd.build            # compile griffin_amd/librglru_hip.so and griffin_amd/_native.so
 
 hipcc cross-compiles without a GPU present, so this runs on a CPU-only machine.
 """
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
@@ -20,6 +22,8 @@ LIB_NAME = "librglru_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 SOURCES = ["rglru_scan.hip", "rglru_fused.hip", "rglru_fused_bwd.hip", "rglru_decode.hip", "rglru_gate_gemm.hip",
            "rglru_block_ops.hip"]
+NATIVE_PATH = os.path.join(HERE, "_native.so")
+NATIVE_SOURCE = "torch_ops.cpp"
 ARCH = "gfx950"
 
 
@@ -33,8 +37,29 @@ def hipcc_path() -> str:
     raise RuntimeError("hipcc not found: the RG-LRU HIP library cannot be built")
 
 
+def _native_commands(obj: str, out: str) -> tuple[list[str], list[str]]:
+    """Compile and link lines of the operator module.  It finds librglru_hip.so next to itself ($ORIGIN)."""
+    import torch                                             # its headers and libraries, found through the package
+
+    root = torch.__path__[0]
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    compiler = shutil.which("g++") or os.path.join(rocm, "llvm", "bin", "clang++")
+    compile_line = [
+        compiler, "-c", "-O2", "-std=c++17", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        "-I", os.path.join(root, "include"), "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+        "-I", os.path.join(rocm, "include"), "-I", sysconfig.get_path("include"), os.path.join(CSRC, NATIVE_SOURCE), "-o", obj,
+    ]
+    link_line = [
+        compiler, "-shared", obj, "-o", out, "-L", HERE, f"-l:{LIB_NAME}", "-L", os.path.join(root, "lib"), "-ltorch_python",
+        "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN",
+    ]
+    return compile_line, link_line
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every kernel for gfx950 and link the shared library; returns its path."""
+    """Compile every kernel for gfx950, link the shared library and the operator module over it; returns the
+    library's path."""
     flags = [
         "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -50,7 +75,7 @@ def build(verbose: bool = False) -> str:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         log = "\n".join(line for line in (proc.stdout + proc.stderr).splitlines() if noise not in line)
         if proc.returncode != 0:
-            raise RuntimeError("hipcc failed:\n" + log)
+            raise RuntimeError(f"{os.path.basename(cmd[0])} failed:\n" + log)
         if log.strip():
             logs.append(log)
 
@@ -58,21 +83,25 @@ def build(verbose: bool = False) -> str:
     tmp = LIB_PATH + ".tmp"
     with tempfile.TemporaryDirectory(prefix="rglru_build_") as objdir:
         objects = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
-        jobs = [[hipcc_path(), *flags, "-c", os.path.join(CSRC, s), "-o", o] for s, o in zip(SOURCES, objects)]
+        native_obj, native_tmp = os.path.join(objdir, "torch_ops.o"), NATIVE_PATH + ".tmp"
+        native_compile, native_link = _native_commands(native_obj, native_tmp)
+        jobs = [native_compile] + [[hipcc_path(), *flags, "-c", os.path.join(CSRC, s), "-o", o] for s, o in zip(SOURCES, objects)]
         with ThreadPoolExecutor(max_workers=min(len(jobs), os.cpu_count() or 1)) as pool:
             list(pool.map(run, jobs))
         run([hipcc_path(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objects, "-o", tmp])
+        # A kernel template whose body the host pass cannot instantiate (seen with a target builtin called directly in a
+        # __global__ template) loses its launch stub without any diagnostic; the library then links but does not load.
+        missing = [line.split()[-1] for line in
+                   subprocess.run(["nm", "-D", "--undefined-only", tmp], capture_output=True, text=True).stdout.splitlines()
+                   if "__device_stub__" in line]
+        if missing:
+            os.remove(tmp)
+            raise RuntimeError("hipcc produced a library with undefined kernel stubs (would not load): " + ", ".join(missing[:4]))
+        os.replace(tmp, LIB_PATH)
+        run(native_link)
+        os.replace(native_tmp, NATIVE_PATH)
     if verbose and logs:
         print("\n".join(logs))
-    # A kernel template whose body the host pass cannot instantiate (seen with a target builtin called directly in a
-    # __global__ template) loses its launch stub without any diagnostic; the library then links but does not load.
-    missing = [line.split()[-1] for line in
-               subprocess.run(["nm", "-D", "--undefined-only", tmp], capture_output=True, text=True).stdout.splitlines()
-               if "__device_stub__" in line]
-    if missing:
-        os.remove(tmp)
-        raise RuntimeError("hipcc produced a library with undefined kernel stubs (would not load): " + ", ".join(missing[:4]))
-    os.replace(tmp, LIB_PATH)
     return LIB_PATH
 
 

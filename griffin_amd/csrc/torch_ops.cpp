@@ -1,0 +1,1085 @@
+// PyTorch operators over the C ABI of librglru_hip.so: argument checks, allocation and autograd in C++.
+//
+// Why native: a training step of a small layer is a handful of launches of 3-10 us, and the same glue in Python
+// (autograd.Function, one torch.empty per buffer, ctypes calls of twenty arguments) kept the host busy for 190 us of
+// a 50 us step and 790 us of a 560 us block step.  Here an operator costs its allocations and launches.
+// Buffers that live and die together are parts of one allocation.
+//
+// Errors follow the reference's operator module (griffin/triton_scan.py:213-224): RuntimeError for a missing GPU,
+// ValueError for shapes, TypeError for types.
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/extension.h>
+
+#include <optional>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "../../include/rglru_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+using MaybeTensor = std::optional<Tensor>;
+
+// ---- small helpers ---------------------------------------------------------------------------------------------
+
+Tensor opt(const MaybeTensor& t) { return t.has_value() ? *t : Tensor(); }
+MaybeTensor maybe(const Tensor& t) { return t.defined() ? MaybeTensor(t) : MaybeTensor(); }
+
+void check(int code, const char* what) {
+  if (code == RGLRU_OK) return;
+  const char* why = rglru_hip_last_error();
+  if (code == RGLRU_E_ARG || code == RGLRU_E_UNSUPPORTED) TORCH_CHECK_VALUE(false, what, " failed: ", why);
+  TORCH_CHECK(false, what, " failed: ", why);
+}
+
+bool known(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
+
+int code_of(at::ScalarType t) {
+  TORCH_CHECK_TYPE(known(t), "hip RG-LRU supports float32 and bfloat16 activations, got ", t);
+  return t == at::kBFloat16 ? RGLRU_BF16 : RGLRU_F32;
+}
+
+void require_gpu(const char* name, std::initializer_list<const Tensor*> tensors) {
+  for (const Tensor* t : tensors)
+    TORCH_CHECK(!t->defined() || t->is_cuda(), name, " requires CUDA/HIP tensors, got a ", t->device().type(), " tensor");
+}
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+float* fptr(const Tensor& t) { return t.defined() ? static_cast<float*>(t.data_ptr()) : nullptr; }
+const int64_t* iptr(const Tensor& t) { return t.defined() ? static_cast<const int64_t*>(t.data_ptr()) : nullptr; }
+const uint8_t* bptr(const Tensor& t) { return t.defined() ? static_cast<const uint8_t*>(t.data_ptr()) : nullptr; }
+
+const uint8_t* flags_ptr(const Tensor& flags, bool first_reset) {
+  return first_reset ? RGLRU_FLAGS_FIRST_RESET : bptr(flags);
+}
+
+Tensor fresh(at::IntArrayRef size, at::ScalarType dtype, const Tensor& like) {
+  return Tensor(at::detail::empty_cuda(size, dtype, like.device(), std::nullopt));
+}
+Tensor fresh_like(const Tensor& t) { return fresh(t.sizes(), t.scalar_type(), t); }
+Tensor bytes(size_t n, const Tensor& like) { return fresh({static_cast<int64_t>(n)}, at::kByte, like); }
+
+size_t round_up(size_t n) { return (n + 255) & ~size_t(255); }
+
+// Contiguous and on a 16-byte boundary (what every fresh allocation is): a view at an odd offset costs one copy
+// instead of sending the whole call to the portable kernels, which are several times slower.
+Tensor aligned(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 16 == 0 ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+bool is_aligned(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; }
+
+Tensor as(const Tensor& t, at::ScalarType dtype) {
+  if (!t.defined()) return t;
+  return t.scalar_type() == dtype ? t.contiguous() : t.to(dtype).contiguous();
+}
+
+// A parameter as the library reads it: its own type when that is fp32 or bf16, else converted.
+Tensor operand(const Tensor& t, at::ScalarType like) {
+  if (!t.defined()) return t;
+  return as(t, known(t.scalar_type()) ? t.scalar_type() : like);
+}
+
+bool wants_grad(std::initializer_list<const Tensor*> tensors) {
+  if (!at::GradMode::is_enabled()) return false;
+  for (const Tensor* t : tensors)
+    if (t->defined() && t->requires_grad()) return true;
+  return false;
+}
+
+// The gradients of a first-order operator: a second differentiation meets an error instead of a wrong number.
+variable_list once(variable_list grads) {
+  if (!at::GradMode::is_enabled()) return grads;
+  variable_list marked;
+  marked.reserve(grads.size());
+  for (auto& g : grads) marked.push_back(g.defined() ? g.detach().set_requires_grad(true) : Tensor());
+  auto error = std::make_shared<torch::autograd::DelayedError>(
+      "trying to differentiate twice a function that was marked with @once_differentiable", marked.size());
+  return error->apply(std::move(marked));
+}
+
+// ---- RG-LRU ----------------------------------------------------------------------------------------------------
+
+// The five parameters as the library reads them: gate weights in the storage type; biases and Lambda in their own
+// type when the three agree on one the library knows, so the usual cases launch no conversion kernels.
+struct Operands {
+  Tensor w_a, b_a, w_x, b_x, lam;
+  int vec;
+  Operands(const Tensor& wa, const Tensor& ba, const Tensor& wx, const Tensor& bx, const Tensor& l, at::ScalarType dtype) {
+    auto v = ba.scalar_type();
+    if (bx.scalar_type() != v || l.scalar_type() != v || !known(v)) v = at::kFloat;
+    w_a = as(wa, dtype), b_a = as(ba, v), w_x = as(wx, dtype), b_x = as(bx, v), lam = as(l, v);
+    vec = v == at::kBFloat16 ? RGLRU_BF16 : RGLRU_F32;
+  }
+};
+
+size_t prep_bytes(int64_t W, int64_t nb, int code) {
+  const size_t n = rglru_hip_prep_bytes(W, nb, code);
+  if (n == 0) check(RGLRU_E_UNSUPPORTED, "rglru_hip_prep_bytes");
+  return n;
+}
+
+int64_t kernel_path(int64_t B, int64_t T, int64_t W, int64_t nb, at::ScalarType dtype, bool on_boundary) {
+  const int path = rglru_hip_backward_path(B, T, W, nb, code_of(dtype), on_boundary ? 1 : 0);
+  if (path < 0) check(RGLRU_E_UNSUPPORTED, "rglru_hip_backward_path");
+  return path;
+}
+
+Tensor prepare(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam, double c,
+               at::ScalarType dtype) {
+  const int64_t nb = w_a.size(0), W = nb * w_a.size(1);
+  const int code = code_of(dtype);
+  c10::DeviceGuard guard(w_a.device());
+  at::NoGradGuard no_grad;
+  Operands p(w_a, b_a, w_x, b_x, lam, dtype);
+  Tensor image = bytes(prep_bytes(W, nb, code), w_a);
+  check(rglru_hip_prepare(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), W, nb, code,
+                          p.vec, ptr(image), stream_of(w_a)), "rglru_hip_prepare");
+  return image;
+}
+
+void check_fused(const Tensor& x, const Tensor& w_a, const Tensor& h0, const Tensor& flags) {
+  TORCH_CHECK_VALUE(x.dim() == 3, "hip RG-LRU expects [batch, sequence, width], got ", x.sizes());
+  const int64_t B = x.size(0), T = x.size(1), W = x.size(2);
+  TORCH_CHECK_VALUE(w_a.dim() == 3 && w_a.size(1) == w_a.size(2) && w_a.size(0) * w_a.size(1) == W, "gate weights ",
+                    w_a.sizes(), " do not match width ", W);
+  TORCH_CHECK_VALUE(!h0.defined() || (h0.dim() == 2 && h0.size(0) == B && h0.size(1) == W), "initial state must have shape (",
+                    B, ", ", W, ")");
+  TORCH_CHECK_VALUE(!flags.defined() || (flags.dim() == 2 && flags.size(0) == B && flags.size(1) == T),
+                    "token flags must have shape (", B, ", ", T, ")");
+  TORCH_CHECK_VALUE(T > 0 && B > 0, "hip RG-LRU does not accept empty batches or sequences");
+  code_of(x.scalar_type());
+}
+
+// What a forward pass keeps for its backward: the parameter image and the workspace in one allocation.
+struct Kept {
+  Tensor buffer;
+  void *image = nullptr, *ws = nullptr;
+  Kept(const Tensor& held, int64_t W, int64_t nb, int code) : buffer(held) {
+    image = held.data_ptr();
+    ws = static_cast<char*>(image) + round_up(prep_bytes(W, nb, code));
+  }
+  Kept(const Tensor& like, int64_t B, int64_t T, int64_t W, int64_t nb, int code)
+      : Kept(bytes(round_up(prep_bytes(W, nb, code)) + rglru_hip_workspace_bytes(B, T, W, nb), like), W, nb, code) {}
+};
+
+struct ForwardResult {
+  Tensor x, h0, y, h_last, kept;
+};
+
+ForwardResult rglru_forward(const Tensor& x_in, const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x,
+                            const Tensor& lam, const Tensor& h0_in, const Tensor& flags, bool first_reset, double c, int64_t path) {
+  ForwardResult r;
+  c10::DeviceGuard guard(x_in.device());
+  r.x = aligned(x_in);
+  const int64_t B = r.x.size(0), T = r.x.size(1), W = r.x.size(2), nb = w_a.size(0);
+  const int code = code_of(r.x.scalar_type());
+  Operands p(w_a, b_a, w_x, b_x, lam, r.x.scalar_type());
+  r.h0 = as(h0_in, at::kFloat);
+  r.y = fresh_like(r.x);
+  r.h_last = fresh({B, W}, at::kFloat, r.x);
+  Kept kept(r.x, B, T, W, nb, code);
+  r.kept = kept.buffer;
+  void* stream = stream_of(r.x);
+  const uint8_t* fl = flags_ptr(flags, first_reset);
+  if (path == RGLRU_PATH_PRE) {
+    Tensor pre = fresh({nb, B * T, 2 * (W / nb)}, r.x.scalar_type(), r.x);  // scratch of the call
+    check(rglru_hip_prepare(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), W, nb, code,
+                            p.vec, kept.image, stream), "rglru_hip_prepare");
+    check(rglru_hip_fwd_pre(ptr(r.x), ptr(pre), kept.image, fptr(r.h0), fl, ptr(r.y), fptr(r.h_last), kept.ws, B, T, W, nb,
+                            code, stream), "rglru_hip_fwd_pre");
+  } else {
+    // parameter conversion, workspace clearing and the forward kernel: two launches, or one where the forward kernel
+    // does all three (batch-rich shapes)
+    check(rglru_hip_prepare_fwd(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), p.vec,
+                                kept.image, ptr(r.x), fptr(r.h0), fl, ptr(r.y), fptr(r.h_last), kept.ws, B, T, W, nb, code,
+                                stream), "rglru_hip_prepare_fwd");
+  }
+  return r;
+}
+
+struct ParamGrads {
+  Tensor dx, dw_a, db_a, dw_x, db_x, dlam, dh0;
+};
+
+// Backward pass of the RG-LRU on what its forward kept; the parameter gradients come back in the parameters' types
+// (w_a, b_a, w_x, b_x, lam).
+ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Tensor& h0, const Tensor& flags, bool first_reset,
+                          const Tensor& held, const Tensor& dy_in, const Tensor& dh_last_in,
+                          const std::array<at::ScalarType, 5>& types, bool need_dh0) {
+  ParamGrads g;
+  c10::DeviceGuard guard(x.device());
+  const int64_t B = x.size(0), T = x.size(1), W = x.size(2), bw = W / nb;
+  const auto dtype = x.scalar_type();
+  const int code = code_of(dtype);
+  Kept kept(held, W, nb, code);
+  Tensor dy = dy_in.defined() ? aligned(dy_in.to(dtype)) : at::zeros_like(x);
+  Tensor dh_last = as(dh_last_in, at::kFloat);
+  // one type for all five gradients where the parameters share one that the library writes; else fp32, converted below
+  auto gt = types[0];
+  for (auto t : types)
+    if (t != gt) gt = at::kFloat;
+  if (!known(gt)) gt = at::kFloat;
+  const int gcode = code_of(gt);
+  g.dx = fresh_like(x);
+  g.dw_a = fresh({nb, bw, bw}, gt, x);
+  g.dw_x = fresh({nb, bw, bw}, gt, x);
+  g.db_a = fresh({nb, bw}, gt, x);
+  g.db_x = fresh({nb, bw}, gt, x);
+  g.dlam = fresh({W}, gt, x);
+  if (need_dh0) g.dh0 = fresh({B, W}, at::kFloat, x);
+  void* stream = stream_of(x);
+  const uint8_t* fl = flags_ptr(flags, first_reset);
+  const int64_t path = kernel_path(B, T, W, nb, dtype, is_aligned(x) && is_aligned(y) && is_aligned(dy));
+  const size_t scratch_bytes = round_up(rglru_hip_bwd_scratch_bytes(B, T, W, nb, code));
+  const size_t tensor_bytes = round_up(x.numel() * x.element_size());
+  // scratch of this call, the operand tensors of the paths that keep some in memory behind it
+  const int extra = path == RGLRU_PATH_PRE ? 4 : path == RGLRU_PATH_PORTABLE ? 2 : 0;
+  Tensor scratch = bytes(scratch_bytes + extra * tensor_bytes, x);
+  char* sp = static_cast<char*>(scratch.data_ptr());
+  char* more = sp + scratch_bytes;
+  if (path == RGLRU_PATH_FAST_CHAIN || path == RGLRU_PATH_FAST_TILED) {
+    check(rglru_hip_bwd_full(ptr(x), ptr(y), kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx),
+                             ptr(g.dw_a), ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam), fptr(g.dh0), B, T, W, nb, code,
+                             gcode, stream), "rglru_hip_bwd_full");
+  } else if (path == RGLRU_PATH_WIDE) {
+    check(rglru_hip_bwd_wide(ptr(x), kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx), ptr(g.dw_a),
+                             ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam), fptr(g.dh0), B, T, W, nb, code, gcode,
+                             stream), "rglru_hip_bwd_wide");
+  } else if (path == RGLRU_PATH_PRE) {
+    check(rglru_hip_bwd_pre(ptr(x), more, kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx),
+                            more + 2 * tensor_bytes, ptr(g.dw_a), ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam),
+                            fptr(g.dh0), B, T, W, nb, code, gcode, stream), "rglru_hip_bwd_pre");
+  } else {
+    check(rglru_hip_bwd(ptr(x), kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx), more,
+                        more + tensor_bytes, ptr(g.dw_a), ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam), fptr(g.dh0), B,
+                        T, W, nb, code, gcode, stream), "rglru_hip_bwd");
+  }
+  Tensor* out[5] = {&g.dw_a, &g.db_a, &g.dw_x, &g.db_x, &g.dlam};
+  for (int i = 0; i < 5; ++i)
+    if (types[i] != gt) *out[i] = out[i]->to(types[i]);
+  return g;
+}
+
+std::array<at::ScalarType, 5> types_of(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x,
+                                       const Tensor& lam) {
+  return {w_a.scalar_type(), b_a.scalar_type(), w_x.scalar_type(), b_x.scalar_type(), lam.scalar_type()};
+}
+
+void pack(AutogradContext* ctx, std::initializer_list<int64_t> values) {
+  ctx->saved_data["meta"] = c10::List<int64_t>(values);
+}
+std::vector<int64_t> unpack(AutogradContext* ctx) { return ctx->saved_data["meta"].toIntVector(); }
+at::ScalarType type_at(const std::vector<int64_t>& m, size_t i) { return static_cast<at::ScalarType>(m[i]); }
+constexpr int64_t kNone = -1;
+
+// Whether the gradient of tensor argument i of a Function's forward is asked for.  The node has an edge only for the
+// arguments that were there, so an optional argument in front shifts the ones behind it: forward notes which were.
+void note_arguments(AutogradContext* ctx, std::initializer_list<bool> present) {
+  c10::List<int64_t> edges;
+  int64_t next = 0;
+  for (bool p : present) edges.push_back(p ? next++ : kNone);
+  ctx->saved_data["edges"] = edges;
+}
+struct Needs {
+  AutogradContext* ctx;
+  std::vector<int64_t> edges;
+  explicit Needs(AutogradContext* c) : ctx(c), edges(c->saved_data["edges"].toIntVector()) {}
+  bool operator()(size_t i) const { return edges[i] != kNone && ctx->needs_input_grad(edges[i]); }
+};
+
+int64_t type_or_none(const Tensor& t) { return t.defined() ? static_cast<int64_t>(t.scalar_type()) : kNone; }
+
+struct RGLRU : torch::autograd::Function<RGLRU> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w_a, const Tensor& b_a, const Tensor& w_x,
+                               const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_, const MaybeTensor& flags_, bool first_reset,
+                               double c, int64_t path) {
+    Tensor h0 = opt(h0_), flags = opt(flags_);
+    note_arguments(ctx, {true, true, true, true, true, true, h0.defined()});
+    ForwardResult r = rglru_forward(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_reset, c, path);
+    ctx->save_for_backward({r.x, r.h0, flags, r.kept, r.y});
+    auto t = types_of(w_a, b_a, w_x, b_x, lam);
+    pack(ctx, {first_reset, w_a.size(0), type_or_none(h0), (int64_t)t[0], (int64_t)t[1], (int64_t)t[2], (int64_t)t[3], (int64_t)t[4]});
+    ctx->set_materialize_grads(false);  // an unused output arrives undefined, not as a tensor of zeros
+    return {r.y, r.h_last};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto saved = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    ParamGrads g;
+    {
+      at::NoGradGuard no_grad;
+      g = rglru_backward(saved[0], saved[4], m[1], saved[1], saved[2], m[0], saved[3], grads[0], grads[1],
+                         {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)},
+                         Needs(ctx)(6));
+      if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
+    }
+    return once({g.dx, g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam, g.dh0, Tensor(), Tensor(), Tensor(), Tensor()});
+  }
+};
+
+std::tuple<Tensor, Tensor> rglru(const Tensor& x, const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x,
+                                 const Tensor& lam, const MaybeTensor& h0_, const MaybeTensor& flags_, bool first_reset,
+                                 double c, int64_t path) {
+  Tensor h0 = opt(h0_), flags = opt(flags_);
+  require_gpu("hip RG-LRU", {&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0, &flags});
+  check_fused(x, w_a, h0, flags);
+  if (wants_grad({&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0})) {
+    auto out = RGLRU::apply(x, w_a, b_a, w_x, b_x, lam, maybe(h0), maybe(flags), first_reset, c, path);
+    return {out[0], out[1]};
+  }
+  at::NoGradGuard no_grad;
+  ForwardResult r = rglru_forward(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_reset, c, path);
+  return {r.y, r.h_last};
+}
+
+// Storage addresses and version counters of some tensors, one after the other: unchanged while nobody replaced one or
+// wrote to it through PyTorch.
+py::tuple fingerprint(const std::vector<Tensor>& tensors) {
+  py::tuple out(2 * tensors.size());
+  for (size_t i = 0; i < tensors.size(); ++i) {
+    out[2 * i] = reinterpret_cast<uintptr_t>(tensors[i].data_ptr());
+    out[2 * i + 1] = tensors[i]._version();
+  }
+  return out;
+}
+
+// ---- decode steps ----------------------------------------------------------------------------------------------
+
+Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
+  Tensor flags = opt(flags_);
+  require_gpu("hip RG-LRU step", {&x_in, &state, &flags});
+  TORCH_CHECK_VALUE(state.sizes() == x_in.sizes() && state.scalar_type() == at::kFloat && state.is_contiguous(),
+                    "step expects a contiguous fp32 state of the same shape as x");
+  c10::DeviceGuard guard(x_in.device());
+  Tensor x = x_in.contiguous();
+  Tensor y = fresh_like(x);
+  check(rglru_hip_step(ptr(x), ptr(image), fptr(state), bptr(flags), ptr(y), x.size(0), x.size(1), blocks,
+                       code_of(x.scalar_type()), stream_of(x)), "rglru_hip_step");
+  return y;
+}
+
+Tensor rglru_steps(const Tensor& xs_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
+  Tensor flags = opt(flags_);
+  require_gpu("hip RG-LRU steps", {&xs_in, &state, &flags});
+  c10::DeviceGuard guard(xs_in.device());
+  Tensor xs = xs_in.contiguous();
+  Tensor ys = fresh_like(xs);
+  Tensor fl = flags.defined() ? flags.contiguous() : flags;
+  if (xs.size(0) > 0 && xs.size(1) > 0)
+    check(rglru_hip_steps(ptr(xs), ptr(image), fptr(state), bptr(fl), ptr(ys), xs.size(0), xs.size(1), xs.size(2), blocks,
+                          code_of(xs.scalar_type()), stream_of(xs)), "rglru_hip_steps");
+  return ys;
+}
+
+// One token per row of the bare layer: y and the new state, the old one untouched (x [B, 1, W]).  The kernel takes the
+// state in place, so the copy into the new buffer is the only other launch.
+std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x, const Tensor& image, int64_t blocks, const MaybeTensor& state_,
+                                             const MaybeTensor& flags_) {
+  Tensor flags = opt(flags_);
+  require_gpu("hip RG-LRU step", {&x, &flags});
+  c10::DeviceGuard guard(x.device());
+  const int64_t B = x.size(0), W = x.size(2);
+  Tensor h = fresh({B, W}, at::kFloat, x);
+  if (state_.has_value()) h.copy_(*state_);
+  else h.zero_();
+  Tensor xc = x.contiguous();
+  Tensor y = fresh({B, 1, W}, x.scalar_type(), x);
+  check(rglru_hip_step(ptr(xc), ptr(image), fptr(h), bptr(flags), ptr(y), B, W, blocks, code_of(x.scalar_type()),
+                       stream_of(x)), "rglru_hip_step");
+  return {y, h};
+}
+
+// ---- scan-only operator: h_t = a_t h_{t-1} + z_t (griffin/triton_scan.py:207-276) --------------------------------
+
+Tensor scan_forward(const Tensor& a, const Tensor& z, const Tensor& h0, Tensor* ws_out) {
+  Tensor out = fresh_like(z);
+  if (out.numel() == 0) return out;
+  const int64_t B = a.size(0), T = a.size(1), W = a.size(2);
+  Tensor ws = bytes(rglru_hip_scan_workspace_bytes(B, T, W), a);
+  check(rglru_hip_scan_fwd(fptr(a), fptr(z), fptr(h0), fptr(out), ptr(ws), B, T, W, stream_of(a)), "rglru_hip_scan_fwd");
+  if (ws_out != nullptr) *ws_out = ws;
+  return out;
+}
+
+struct Scan : torch::autograd::Function<Scan> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& a_in, const Tensor& z, const Tensor& h0_in) {
+    c10::DeviceGuard guard(a_in.device());
+    Tensor a = a_in.contiguous(), h0 = h0_in.contiguous(), ws;
+    Tensor out = scan_forward(a, z.contiguous(), h0, &ws);
+    ctx->save_for_backward({a, h0, out});
+    // the forward call has cleared the backward part of the workspace too: the first backward call over this forward
+    // finds it clear (a repeated one clears its part itself)
+    if (ws.defined()) ctx->saved_data["ws"] = ws;
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto saved = ctx->get_saved_variables();
+    const Tensor &a = saved[0], &h0 = saved[1], &out = saved[2];
+    Tensor da, dz, dh0;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(a.device());
+      Tensor dh = grads[0].contiguous();
+      const int64_t B = a.size(0), T = a.size(1), W = a.size(2);
+      da = fresh_like(a), dz = fresh_like(a), dh0 = fresh_like(h0);
+      if (a.numel() == 0) {
+        dh0.zero_();
+      } else {
+        auto held = ctx->saved_data.find("ws");
+        const bool clear = held != ctx->saved_data.end();
+        Tensor ws = clear ? held->second.toTensor() : bytes(rglru_hip_scan_workspace_bytes(B, T, W), a);
+        if (clear) ctx->saved_data.erase(held);
+        check(rglru_hip_scan_bwd(fptr(a), fptr(h0), fptr(out), fptr(dh), fptr(da), fptr(dz), fptr(dh0), ptr(ws), clear ? 1 : 0, B,
+                                 T, W, stream_of(a)), "rglru_hip_scan_bwd");
+      }
+    }
+    return once({da, dz, dh0});
+  }
+};
+
+Tensor scan(const Tensor& a, const Tensor& z, const Tensor& h0) {
+  require_gpu("hip_rglru_scan", {&a, &z, &h0});
+  TORCH_CHECK_VALUE(a.dim() == 3 && a.sizes() == z.sizes(), "decay and current_input must share shape [batch, sequence, width]");
+  TORCH_CHECK_VALUE(h0.dim() == 2 && h0.size(0) == a.size(0) && h0.size(1) == a.size(2), "initial_state must have shape [batch, width]");
+  TORCH_CHECK_TYPE(a.scalar_type() == at::kFloat && z.scalar_type() == at::kFloat, "hip_rglru_scan expects fp32 decay and normalized input");
+  TORCH_CHECK_TYPE(h0.scalar_type() == at::kFloat, "hip_rglru_scan expects fp32 recurrent state");
+  if (wants_grad({&a, &z, &h0})) return Scan::apply(a, z, h0);
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(a.device());
+  return scan_forward(a.contiguous(), z.contiguous(), h0.contiguous(), nullptr);
+}
+
+// ---- causal depthwise convolution (griffin/griffin.py:474-510) ----------------------------------------------------
+
+struct ConvMeta {  // types of the forward's arguments (kNone: absent)
+  int64_t state, weight, bias;
+};
+
+// Reverse mode of the dense convolution on contiguous operands.  `du_out`: where to write du instead of a new tensor --
+// [B, T, W] with unit stride along W and rows a common distance apart (a column range of a wider matrix).
+variable_list conv_backward(const Tensor& u, const Tensor& state, const Tensor& taps, const Tensor& pos, const Tensor& dout_in,
+                            ConvMeta meta, bool need_u, bool need_state, bool need_w, bool need_b, const Tensor& du_out) {
+  const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = taps.size(2);
+  Tensor dout = as(dout_in, u.scalar_type());
+  const auto gt = taps.scalar_type();
+  Tensor du = du_out.defined() ? du_out : fresh_like(u);
+  Tensor dstate, dtaps, dbias;
+  if (need_state && state.defined()) dstate = fresh_like(state);
+  if (need_w) dtaps = fresh({W, 1, K}, gt, u);
+  if (need_b && meta.bias != kNone) dbias = fresh({W}, gt, u);
+  Tensor scratch = bytes(rglru_hip_conv_scratch_bytes(B, T, W, K), u);
+  check(rglru_hip_conv_bwd(ptr(u), ptr(state), ptr(taps), iptr(pos), ptr(dout), ptr(scratch), ptr(du), du.stride(1), ptr(dstate),
+                           ptr(dtaps), ptr(dbias), B, T, W, K, code_of(u.scalar_type()), code_of(gt), code_of(gt), stream_of(u)),
+        "rglru_hip_conv_bwd");
+  if (dtaps.defined()) dtaps = dtaps.to(static_cast<at::ScalarType>(meta.weight));
+  if (dbias.defined()) dbias = dbias.to(static_cast<at::ScalarType>(meta.bias));
+  if (need_state && meta.state != kNone)
+    dstate = (dstate.defined() ? dstate : at::zeros({B, K - 1, W}, u.options())).to(static_cast<at::ScalarType>(meta.state));
+  return {need_u ? du : Tensor(), dstate, dtaps, dbias};
+}
+
+void check_conv(const char* name, const Tensor& u, const Tensor& state, const Tensor& weight, const Tensor& bias,
+                const Tensor& pos) {
+  TORCH_CHECK_VALUE(u.dim() == 3, name, " expects [batch, sequence, width], got ", u.sizes());
+  const int64_t B = u.size(0), T = u.size(1), W = u.size(2);
+  TORCH_CHECK_VALUE(weight.dim() == 3 && weight.size(0) == W && weight.size(1) == 1,
+                    "weight must be that of a depthwise Conv1d: [width, 1, kernel_size]");
+  TORCH_CHECK_VALUE(!bias.defined() || (bias.dim() == 1 && bias.size(0) == W), "bias must have shape [width]");
+  TORCH_CHECK_VALUE(!state.defined() || (state.dim() == 3 && state.size(0) == B && state.size(1) == weight.size(2) - 1 && state.size(2) == W),
+                    "state must have shape [batch, kernel_size - 1, width]");
+  TORCH_CHECK_VALUE(pos.dim() == 2 && pos.size(0) == B && pos.size(1) == T, "segment_pos must have shape [batch, sequence]");
+  code_of(u.scalar_type());
+}
+
+struct ConvOperands {
+  Tensor u, state, taps, bias, pos;
+  ConvOperands(const Tensor& u_in, const Tensor& st, const Tensor& weight, const Tensor& b, const Tensor& segment_pos) {
+    u = u_in.contiguous();
+    state = weight.size(2) == 1 ? Tensor() : as(st, u.scalar_type());
+    taps = operand(weight, u.scalar_type());
+    bias = as(b, taps.scalar_type());
+    pos = segment_pos.to(u.device(), at::kLong).contiguous();
+  }
+};
+
+struct CausalConv : torch::autograd::Function<CausalConv> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& u, const MaybeTensor& state_, const Tensor& weight,
+                        const MaybeTensor& bias_, const Tensor& pos) {
+    Tensor state = opt(state_), bias = opt(bias_);
+    note_arguments(ctx, {true, state.defined(), true, bias.defined()});
+    c10::DeviceGuard guard(u.device());
+    ConvOperands o(u, state, weight, bias, pos);
+    Tensor out = fresh_like(o.u);
+    check(rglru_hip_conv_fwd(ptr(o.u), ptr(o.state), ptr(o.taps), ptr(o.bias), iptr(o.pos), ptr(out), nullptr, u.size(0),
+                             u.size(1), u.size(2), weight.size(2), code_of(u.scalar_type()), code_of(o.taps.scalar_type()),
+                             stream_of(u)), "rglru_hip_conv_fwd");
+    ctx->save_for_backward({o.u, o.state, o.taps, o.pos});
+    pack(ctx, {type_or_none(state), type_or_none(weight), type_or_none(bias)});
+    ctx->set_materialize_grads(false);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    if (!grads[0].defined()) return variable_list(5);
+    auto s = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    variable_list g;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(s[0].device());
+      Needs need(ctx);
+      g = conv_backward(s[0], s[1], s[2], s[3], grads[0], {m[0], m[1], m[2]}, need(0), need(1), need(2), need(3), Tensor());
+    }
+    g.emplace_back();
+    return once(std::move(g));
+  }
+};
+
+Tensor causal_conv(const Tensor& u, const MaybeTensor& state_, const Tensor& weight, const MaybeTensor& bias_, const Tensor& pos) {
+  Tensor state = opt(state_), bias = opt(bias_);
+  require_gpu("hip_causal_conv", {&u, &state, &weight, &bias, &pos});
+  check_conv("hip_causal_conv", u, state, weight, bias, pos);
+  return CausalConv::apply(u, maybe(state), weight, maybe(bias), pos);
+}
+
+struct CausalConvPadded : torch::autograd::Function<CausalConvPadded> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& u, const MaybeTensor& state_, const Tensor& weight,
+                               const MaybeTensor& bias_, const Tensor& pos, const Tensor& active) {
+    Tensor state = opt(state_), bias = opt(bias_);
+    note_arguments(ctx, {true, state.defined(), true, bias.defined()});
+    c10::DeviceGuard guard(u.device());
+    ConvOperands o(u, state, weight, bias, pos);
+    Tensor live = active.to(u.device(), at::kByte).contiguous();
+    const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = weight.size(2);
+    Tensor out = fresh_like(o.u);
+    Tensor new_state = fresh({B, K - 1, W}, u.scalar_type(), u);
+    Tensor scratch = bytes(rglru_hip_conv_padded_scratch_bytes(B, T), u);
+    check(rglru_hip_conv_padded_fwd(ptr(o.u), ptr(o.state), ptr(o.taps), ptr(o.bias), iptr(o.pos), bptr(live), ptr(scratch),
+                                    ptr(out), K > 1 ? ptr(new_state) : nullptr, B, T, W, K, code_of(u.scalar_type()),
+                                    code_of(o.taps.scalar_type()), stream_of(u)), "rglru_hip_conv_padded_fwd");
+    ctx->save_for_backward({o.u, o.state, o.taps, o.pos, live});
+    pack(ctx, {type_or_none(state), type_or_none(weight), type_or_none(bias)});
+    ctx->mark_non_differentiable({new_state});
+    ctx->set_materialize_grads(false);
+    return {out, new_state};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    if (!grads[0].defined()) return variable_list(6);
+    auto s = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    const Tensor &u = s[0], &state = s[1], &taps = s[2], &pos = s[3], &live = s[4];
+    Tensor du, dstate, dtaps, dbias;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(u.device());
+      const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = taps.size(2);
+      Needs need(ctx);
+      const bool need_state = need(1);
+      Tensor dout = as(grads[0], u.scalar_type());
+      const auto gt = taps.scalar_type();
+      du = fresh_like(u);
+      if (need_state && K > 1) dstate = fresh({B, K - 1, W}, u.scalar_type(), u);
+      if (need(2)) dtaps = fresh({W, 1, K}, gt, u);
+      if (need(3) && m[2] != kNone) dbias = fresh({W}, gt, u);
+      const size_t index_bytes = round_up(rglru_hip_conv_padded_scratch_bytes(B, T));
+      Tensor scratch = bytes(index_bytes + rglru_hip_conv_scratch_bytes(B, T, W, K), u);
+      char* sp = static_cast<char*>(scratch.data_ptr());
+      check(rglru_hip_conv_padded_bwd(ptr(u), ptr(state), ptr(taps), iptr(pos), bptr(live), ptr(dout), sp, sp + index_bytes,
+                                      ptr(du), ptr(dstate), ptr(dtaps), ptr(dbias), B, T, W, K, code_of(u.scalar_type()),
+                                      code_of(gt), code_of(gt), stream_of(u)), "rglru_hip_conv_padded_bwd");
+      if (dtaps.defined()) dtaps = dtaps.to(type_at(m, 1));
+      if (dbias.defined()) dbias = dbias.to(type_at(m, 2));
+      if (need_state && m[0] != kNone)
+        dstate = (dstate.defined() ? dstate : at::zeros({B, K - 1, W}, u.options())).to(type_at(m, 0));
+      else
+        dstate = Tensor();
+      if (!need(0)) du = Tensor();
+    }
+    return once({du, dstate, dtaps, dbias, Tensor(), Tensor()});
+  }
+};
+
+std::tuple<Tensor, Tensor> causal_conv_padded(const Tensor& u, const MaybeTensor& state_, const Tensor& weight,
+                                              const MaybeTensor& bias_, const Tensor& pos, const Tensor& active) {
+  Tensor state = opt(state_), bias = opt(bias_);
+  require_gpu("hip_causal_conv_padded", {&u, &state, &weight, &bias, &pos, &active});
+  check_conv("hip_causal_conv_padded", u, state, weight, bias, pos);
+  TORCH_CHECK_VALUE(active.sizes() == pos.sizes(), "segment_pos and active_mask must have shape [batch, sequence]");
+  auto out = CausalConvPadded::apply(u, maybe(state), weight, maybe(bias), pos, active);
+  return {out[0], out[1]};
+}
+
+// ---- output gate h * gelu_tanh(v) (griffin/griffin.py:464, :520) --------------------------------------------------
+
+struct GeluGate : torch::autograd::Function<GeluGate> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& h_in, const Tensor& v_in) {
+    c10::DeviceGuard guard(h_in.device());
+    Tensor h = h_in.contiguous(), v = v_in.contiguous();
+    Tensor out = fresh_like(h);
+    if (h.numel() > 0)
+      check(rglru_hip_gelu_gate_fwd(ptr(h), ptr(v), ptr(out), h.numel(), code_of(h.scalar_type()), stream_of(h)),
+            "rglru_hip_gelu_gate_fwd");
+    ctx->save_for_backward({h, v});
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto s = ctx->get_saved_variables();
+    const Tensor &h = s[0], &v = s[1];
+    Tensor dh, dv;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(h.device());
+      Tensor dout = as(grads[0], h.scalar_type());
+      dh = fresh_like(h), dv = fresh_like(v);
+      if (h.numel() > 0)
+        check(rglru_hip_gelu_gate_bwd(ptr(dout), ptr(h), ptr(v), ptr(dh), ptr(dv), h.numel(), h.size(-1), 0,
+                                      code_of(h.scalar_type()), stream_of(h)), "rglru_hip_gelu_gate_bwd");
+    }
+    return once({dh, dv});
+  }
+};
+
+Tensor gelu_gate(const Tensor& h, const Tensor& v) {
+  require_gpu("hip_gelu_gate", {&h, &v});
+  TORCH_CHECK_VALUE(h.sizes() == v.sizes(), "hip_gelu_gate expects equal shapes, got ", h.sizes(), " and ", v.sizes());
+  TORCH_CHECK_TYPE(h.scalar_type() == v.scalar_type(), "hip_gelu_gate expects equal dtypes, got ", h.scalar_type(), " and ", v.scalar_type());
+  code_of(h.scalar_type());
+  return GeluGate::apply(h, v);
+}
+
+// ---- convolution, RG-LRU and output gate of the block in one forward launch ---------------------------------------
+
+// [B, T, W] as the library addresses it: channels contiguous, one row stride for all tokens, rows on 16 bytes.
+Tensor row_view(const Tensor& t) {
+  const int64_t B = t.size(0), T = t.size(1), W = t.size(2);
+  if (t.stride(2) == 1 && t.stride(1) >= W && (B == 1 || t.stride(0) == T * t.stride(1)) &&
+      (t.stride(1) * t.element_size()) % 16 == 0 && is_aligned(t))
+    return t;
+  return t.contiguous();
+}
+
+Tensor block_flags(const Tensor& segment_pos) {
+  require_gpu("hip_block_flags", {&segment_pos});
+  c10::DeviceGuard guard(segment_pos.device());
+  Tensor pos = segment_pos.to(at::kLong).contiguous();
+  Tensor flags = fresh(pos.sizes(), at::kByte, pos);
+  if (pos.numel() > 0)
+    check(rglru_hip_block_flags(iptr(pos), static_cast<uint8_t*>(flags.data_ptr()), pos.numel(), stream_of(pos)),
+          "rglru_hip_block_flags");
+  return flags;
+}
+
+struct BlockResult {
+  Tensor u, v, state, taps, pos, x_conv, y, h0, flags, kept, gated, h_last, new_conv;
+};
+
+BlockResult block_forward_pass(const Tensor& u, const Tensor& v, const Tensor& conv_state, const Tensor& weight,
+                               const Tensor& bias, const Tensor& segment_pos, const Tensor& flags, bool first_reset,
+                               const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam,
+                               const Tensor& h0, double c, const Tensor& image, bool training) {
+  BlockResult r;
+  c10::DeviceGuard guard(u.device());
+  const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = weight.size(2), nb = w_a.size(0);
+  const auto dtype = u.scalar_type();
+  const int code = code_of(dtype);
+  r.u = row_view(u), r.v = row_view(v);
+  r.state = K == 1 ? Tensor() : as(conv_state, dtype);
+  r.taps = operand(weight, dtype);
+  Tensor b = as(bias, r.taps.scalar_type());
+  r.pos = segment_pos.to(u.device(), at::kLong).contiguous();
+  r.h0 = as(h0, at::kFloat);
+  r.flags = first_reset ? Tensor() : flags.defined() ? flags : block_flags(r.pos);
+  r.gated = fresh({B, T, W}, dtype, u);
+  if (training) r.x_conv = fresh({B, T, W}, dtype, u), r.y = fresh({B, T, W}, dtype, u);
+  r.new_conv = fresh({B, K - 1, W}, dtype, u);
+  r.h_last = fresh({B, W}, at::kFloat, u);
+  void* stream = stream_of(u);
+  void* new_conv = K > 1 ? ptr(r.new_conv) : nullptr;
+  const uint8_t* fl = flags_ptr(r.flags, first_reset);
+  if (training || !image.defined()) {
+    Operands p(w_a, b_a, w_x, b_x, lam, dtype);
+    Kept kept(u, B, T, W, nb, code);
+    r.kept = kept.buffer;
+    check(rglru_hip_prepare_block_fwd(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), p.vec,
+                                      kept.image, ptr(r.u), r.u.stride(1), ptr(r.v), r.v.stride(1), ptr(r.state), ptr(r.taps),
+                                      ptr(b), K, fptr(r.h0), fl, ptr(r.x_conv), ptr(r.y), ptr(r.gated), new_conv,
+                                      fptr(r.h_last), kept.ws, B, T, W, nb, code, stream), "rglru_hip_prepare_block_fwd");
+  } else {
+    Tensor ws = bytes(rglru_hip_workspace_bytes(B, T, W, nb), u);
+    check(rglru_hip_block_fwd(ptr(r.u), r.u.stride(1), ptr(r.v), r.v.stride(1), ptr(r.state), ptr(r.taps), ptr(b), K,
+                              code_of(r.taps.scalar_type()), ptr(image), fptr(r.h0), fl, ptr(r.x_conv), ptr(r.y), ptr(r.gated),
+                              new_conv, fptr(r.h_last), ptr(ws), B, T, W, nb, code, stream), "rglru_hip_block_fwd");
+  }
+  return r;
+}
+
+// The backward pass runs the three reverse kernels one after the other on the x and y the forward kept.
+struct BlockForward : torch::autograd::Function<BlockForward> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& u, const Tensor& v, const MaybeTensor& conv_state_,
+                               const Tensor& weight, const MaybeTensor& bias_, const Tensor& segment_pos,
+                               const MaybeTensor& flags_, bool first_reset, const Tensor& w_a, const Tensor& b_a,
+                               const Tensor& w_x, const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_, double c) {
+    Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_);
+    note_arguments(ctx, {true, true, conv_state.defined(), true, bias.defined(), true, flags.defined(), true, true, true, true,
+                         true, h0.defined()});
+    BlockResult r = block_forward_pass(u, v, conv_state, weight, bias, segment_pos, flags, first_reset, w_a, b_a, w_x, b_x, lam,
+                                       h0, c, Tensor(), true);
+    ctx->save_for_backward({r.u, r.v, r.state, r.taps, r.pos, r.x_conv, r.y, r.h0, r.flags, r.kept});
+    auto t = types_of(w_a, b_a, w_x, b_x, lam);
+    pack(ctx, {first_reset, w_a.size(0), type_or_none(h0), (int64_t)t[0], (int64_t)t[1], (int64_t)t[2], (int64_t)t[3], (int64_t)t[4],
+               type_or_none(conv_state), type_or_none(weight), type_or_none(bias)});
+    ctx->mark_non_differentiable({r.new_conv});
+    ctx->set_materialize_grads(false);
+    return {r.gated, r.h_last, r.new_conv};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto s = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    const Tensor &u = s[0], &v = s[1], &state = s[2], &taps = s[3], &pos = s[4], &x_conv = s[5], &y = s[6], &h0 = s[7],
+                 &flags = s[8], &kept = s[9];
+    Needs need(ctx);  // by tensor argument of forward: u, v, conv_state, weight, bias, ... (12: h0)
+    const bool need_u = need(0), need_v = need(1);
+    Tensor dv;
+    ParamGrads g;
+    variable_list conv;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(y.device());
+      const int64_t B = y.size(0), T = y.size(1), W = y.size(2);
+      const auto dtype = y.scalar_type();
+      Tensor dy, du_out;
+      if (grads[0].defined()) {
+        Tensor dout = as(grads[0], dtype);
+        Tensor v_c = v.contiguous();
+        dy = fresh_like(y);
+        const int64_t row_bytes = W * y.element_size();
+        if (need_u && need_v && row_bytes % 16 == 0 && B * T * 2 * row_bytes < (int64_t(1) << 31)) {
+          // The gradients of the two projections as the halves of ONE [B, T, 2 W] matrix: the Linear layers' backward
+          // then runs one GEMM each for dx and dW and one column sum (linear_pair).
+          Tensor both = fresh({B, T, 2 * W}, dtype, y);
+          du_out = both.narrow(2, 0, W), dv = both.narrow(2, W, W);
+        } else {
+          dv = fresh_like(v_c);
+        }
+        check(rglru_hip_gelu_gate_bwd(ptr(dout), ptr(y), ptr(v_c), ptr(dy), ptr(dv), y.numel(), W, dv.stride(1), code_of(dtype),
+                                      stream_of(y)), "rglru_hip_gelu_gate_bwd");
+      }
+      g = rglru_backward(x_conv, y, m[1], h0, flags, m[0], kept, dy, grads[1],
+                         {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)}, need(12));
+      if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
+      conv = conv_backward(u.contiguous(), state, taps, pos, g.dx, {m[8], m[9], m[10]}, need_u, need(2), need(3),
+                           need(4), du_out);
+      if (!need_v) dv = Tensor();
+    }
+    return once({conv[0], dv, conv[1], conv[2], conv[3], Tensor(), Tensor(), Tensor(), g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam,
+                 g.dh0, Tensor()});
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& v, const MaybeTensor& conv_state_,
+                                                 const Tensor& weight, const MaybeTensor& bias_, const Tensor& segment_pos,
+                                                 const MaybeTensor& flags_, bool first_reset, const Tensor& w_a, const Tensor& b_a,
+                                                 const Tensor& w_x, const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_,
+                                                 double c, const MaybeTensor& image_) {
+  Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_);
+  require_gpu("hip_block_forward", {&u, &v, &conv_state, &weight, &bias, &segment_pos, &w_a, &b_a, &w_x, &b_x, &lam, &h0});
+  TORCH_CHECK_VALUE(u.dim() == 3 && u.sizes() == v.sizes() && u.scalar_type() == v.scalar_type(),
+                    "hip_block_forward expects two [batch, sequence, width] tensors of one dtype");
+  const int64_t B = u.size(0), T = u.size(1), W = u.size(2);
+  check_conv("hip_block_forward", u, conv_state, weight, Tensor(), segment_pos);
+  TORCH_CHECK_VALUE(!h0.defined() || (h0.dim() == 2 && h0.size(0) == B && h0.size(1) == W), "initial state must have shape (", B, ", ", W, ")");
+  TORCH_CHECK_VALUE(!flags.defined() || (flags.dim() == 2 && flags.size(0) == B && flags.size(1) == T && flags.scalar_type() == at::kByte && flags.is_contiguous()),
+                    "flags must be a contiguous uint8 tensor of shape [batch, sequence]");
+  if (wants_grad({&u, &v, &conv_state, &weight, &bias, &w_a, &b_a, &w_x, &b_x, &lam, &h0})) {
+    auto out = BlockForward::apply(u, v, maybe(conv_state), weight, maybe(bias), segment_pos, maybe(flags), first_reset, w_a,
+                                   b_a, w_x, b_x, lam, maybe(h0), c);
+    return {out[0], out[1], out[2]};
+  }
+  at::NoGradGuard no_grad;
+  BlockResult r = block_forward_pass(u, v, conv_state, weight, bias, segment_pos, flags, first_reset, w_a, b_a, w_x, b_x, lam, h0, c,
+                                     opt(image_), false);
+  return {r.gated, r.h_last, r.new_conv};
+}
+
+// One token per row through conv -> RG-LRU step -> output gate (no autograd), two kernel launches.
+std::tuple<Tensor, Tensor, Tensor, Tensor> block_decode_step(const Tensor& u_in, const Tensor& v_in, const MaybeTensor& conv_state_,
+                                                             const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& prev_pos_,
+                                                             const MaybeTensor& segment_pos_, const MaybeTensor& active_,
+                                                             const Tensor& image, int64_t width, int64_t blocks, at::ScalarType prep_dtype,
+                                                             const MaybeTensor& rnn_state_) {
+  Tensor conv_state = opt(conv_state_), bias = opt(bias_), prev_pos = opt(prev_pos_), segment_pos = opt(segment_pos_),
+         active = opt(active_), rnn_state = opt(rnn_state_);
+  require_gpu("hip_block_decode_step", {&u_in, &v_in, &conv_state, &weight, &bias, &prev_pos, &segment_pos, &active, &rnn_state});
+  TORCH_CHECK_VALUE(u_in.dim() == 2 && u_in.sizes() == v_in.sizes() && u_in.scalar_type() == v_in.scalar_type(),
+                    "hip_block_decode_step expects two [batch, width] tensors of one dtype");
+  const int64_t B = u_in.size(0), W = u_in.size(1), K = weight.size(2);
+  TORCH_CHECK_VALUE(W == width && u_in.scalar_type() == prep_dtype, "the prepared RG-LRU parameters do not match the activations");
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(u_in.device());
+  const auto dtype = u_in.scalar_type();
+  const int code = code_of(dtype);
+  // rows may be views into a wider buffer (the two halves of one fused projection)
+  auto rows = [W](const Tensor& t) { return t.stride(1) == 1 && t.stride(0) >= W ? t : t.contiguous(); };
+  Tensor u = rows(u_in), v = rows(v_in);
+  Tensor state = K == 1 ? Tensor() : as(conv_state, dtype);
+  Tensor taps = operand(weight, dtype);
+  Tensor b = as(bias, taps.scalar_type());
+  Tensor new_conv = fresh({B, K - 1, W}, dtype, u);
+  Tensor new_pos = fresh({B}, at::kLong, u);
+  Tensor h_in = rnn_state.defined() ? as(rnn_state, at::kFloat) : at::zeros({B, W}, u.options().dtype(at::kFloat));
+  Tensor h_out = fresh({B, W}, at::kFloat, u);
+  Tensor out = fresh({B, W}, dtype, u);
+  const size_t x_bytes = round_up(B * W * u.element_size());
+  Tensor scratch = bytes(x_bytes + B, u);
+  char* x = static_cast<char*>(scratch.data_ptr());
+  uint8_t* flags = reinterpret_cast<uint8_t*>(x + x_bytes);
+  void* stream = stream_of(u);
+  check(rglru_hip_decode_prepare(ptr(u), u.stride(0), ptr(state), ptr(taps), ptr(b), iptr(prev_pos), iptr(segment_pos), bptr(active),
+                                 x, K > 1 ? ptr(new_conv) : nullptr, static_cast<int64_t*>(new_pos.data_ptr()), flags, B, W, K, code,
+                                 code_of(taps.scalar_type()), stream), "rglru_hip_decode_prepare");
+  check(rglru_hip_step_gated(x, ptr(image), fptr(h_in), fptr(h_out), flags, ptr(v), v.stride(0), ptr(out), B, W, blocks, code, stream),
+        "rglru_hip_step_gated");
+  return {out, h_out, new_conv, new_pos};
+}
+
+// ---- Linear layers of the block (griffin/griffin.py:379-389) ------------------------------------------------------
+
+// sets.sum(0) of a contiguous [sets, ...] tensor in one pass; anything the kernel does not take goes to the generic one.
+Tensor sum_sets(const Tensor& sets) {
+  if (!sets.is_cuda() || !known(sets.scalar_type()) || !sets.is_contiguous() || sets.numel() == 0) return sets.sum(0);
+  c10::DeviceGuard guard(sets.device());
+  Tensor out = fresh(sets.sizes().slice(1), sets.scalar_type(), sets);
+  check(rglru_hip_sum_sets(ptr(sets), ptr(out), sets.size(0), out.numel(), code_of(sets.scalar_type()), stream_of(sets)),
+        "rglru_hip_sum_sets");
+  return out;
+}
+
+// (dW, db) of y = x W^T + b for the incoming dy; bias_type kNone skips db.
+std::tuple<Tensor, Tensor> linear_parameter_grads(const Tensor& x, at::ScalarType weight_type, const Tensor& dy, bool need_w, int64_t bias_type) {
+  Tensor dy2 = dy.reshape({-1, dy.size(-1)});
+  Tensor dw, db;
+  const int64_t rows = dy2.size(0), width = dy2.size(1);
+  if (need_w) {
+    Tensor x2 = x.reshape({-1, x.size(-1)}).to(dy.scalar_type());
+    // dW = dy^T x contracts over all tokens: one GEMM with K = rows runs at a fraction of the rate of the same work as
+    // a batch of GEMMs with K = 2048 whose results are added (100 us against 43 us for 16384 x 1024 x 768 in bf16 on
+    // this library), so long contractions are split
+    int64_t chunks = (rows % 2048 == 0 && dy2.is_contiguous() && x2.is_contiguous()) ? rows / 2048 : 1;
+    while (chunks > 16 && chunks % 2 == 0) chunks /= 2;
+    if (chunks > 1) {
+      const int64_t per = rows / chunks;
+      dw = sum_sets(at::bmm(dy2.view({chunks, per, width}).transpose(1, 2), x2.view({chunks, per, x2.size(1)})));
+    } else {
+      dw = at::mm(dy2.t(), x2);
+    }
+    if (dw.scalar_type() != weight_type) dw = dw.to(weight_type);
+  }
+  if (bias_type != kNone) {
+    const auto bt = static_cast<at::ScalarType>(bias_type);
+    const auto ot = known(bt) ? bt : at::kFloat;
+    Tensor dy_c = dy2.contiguous();
+    db = fresh({width}, ot, dy);
+    Tensor scratch = bytes(rglru_hip_colsum_scratch_bytes(rows, width), dy);
+    check(rglru_hip_colsum(ptr(dy_c), ptr(scratch), ptr(db), rows, width, code_of(dy.scalar_type()), code_of(ot), stream_of(dy)),
+          "rglru_hip_colsum");
+    if (ot != bt) db = db.to(bt);
+  }
+  return {dw, db};
+}
+
+struct Linear : torch::autograd::Function<Linear> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const MaybeTensor& bias) {
+    ctx->save_for_backward({x, weight});
+    note_arguments(ctx, {true, true, bias.has_value()});
+    pack(ctx, {type_or_none(opt(bias))});
+    return at::linear(x, weight, bias);
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto s = ctx->get_saved_variables();
+    Tensor dx, dw, db;
+    {
+      at::NoGradGuard no_grad;
+      const Tensor &x = s[0], &weight = s[1], &dy = grads[0];
+      c10::DeviceGuard guard(x.device());
+      Needs need(ctx);
+      if (need(0)) dx = at::matmul(dy, weight.to(dy.scalar_type()));
+      std::tie(dw, db) = linear_parameter_grads(x, weight.scalar_type(), dy, need(1), need(2) ? unpack(ctx)[0] : kNone);
+    }
+    return once({dx, dw, db});
+  }
+};
+
+Tensor linear(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_) {
+  Tensor bias = opt(bias_);
+  require_gpu("hip_linear", {&x, &weight, &bias});
+  code_of(x.scalar_type());
+  return Linear::apply(x, weight, maybe(bias));
+}
+
+// The [rows, 2 W] matrix whose column halves `a` and `b` ([..., W] each) are, or an undefined tensor if they are not
+// laid out that way (same storage, b starts W elements behind a, rows 2 W elements apart).
+Tensor stacked_halves(const Tensor& a, const Tensor& b) {
+  if (!a.defined() || !b.defined() || a.sizes() != b.sizes() || a.scalar_type() != b.scalar_type() || a.dim() < 2 || a.numel() == 0)
+    return Tensor();
+  const int64_t W = a.size(-1);
+  if (a.strides() != b.strides() || a.stride(-1) != 1 || b.storage_offset() != a.storage_offset() + W) return Tensor();
+  if (!a.is_alias_of(b)) return Tensor();
+  int64_t expect = 2 * W;  // every leading axis must continue the rows of the one before
+  for (int64_t d = a.dim() - 2; d >= 0; --d) {
+    if (a.size(d) != 1 && a.stride(d) != expect) return Tensor();
+    expect *= a.size(d);
+  }
+  return a.as_strided({a.numel() / W, 2 * W}, {2 * W, 1}, a.storage_offset());
+}
+
+// Two Linear layers on one input (the block's two branches).  Their input gradients are one GEMM that accumulates into
+// the other's result instead of two results and an addition.
+struct LinearPair : torch::autograd::Function<LinearPair> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2,
+                               const MaybeTensor& b2) {
+    ctx->save_for_backward({x, w1, w2});
+    note_arguments(ctx, {true, true, b1.has_value(), true, b2.has_value()});
+    pack(ctx, {type_or_none(opt(b1)), type_or_none(opt(b2))});
+    ctx->set_materialize_grads(false);
+    return {at::linear(x, w1, b1), at::linear(x, w2, b2)};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto s = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    const Tensor &x = s[0], &w1 = s[1], &w2 = s[2];
+    Needs need(ctx);
+    const bool need_x = need(0), need_w1 = need(1), need_b1 = need(2), need_w2 = need(3), need_b2 = need(4);
+    Tensor dx, dw1, db1, dw2, db2;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(x.device());
+      Tensor both = stacked_halves(grads[0], grads[1]);
+      if (both.defined() && w1.scalar_type() == w2.scalar_type() && w1.sizes() == w2.sizes() && need_w1 == need_w2 &&
+          need_b1 == need_b2 && m[0] == m[1]) {
+        // The halves of one matrix (the block's backward writes them so): one GEMM for dx against the stacked weights,
+        // one for both weight gradients, one column sum.  At 16384 rows, 768 -> 2 x 1024: 49 against 65 us (dx), 60
+        // against 83 us (dW), two launches instead of four (db).
+        const int64_t n = w1.size(0);
+        if (need_x) dx = at::mm(both, at::cat({w1, w2}).to(both.scalar_type())).view(x.sizes());
+        Tensor dw, db;
+        std::tie(dw, db) = linear_parameter_grads(x, w1.scalar_type(), both, need_w1, need_b1 ? m[0] : kNone);
+        if (dw.defined()) dw1 = dw.narrow(0, 0, n), dw2 = dw.narrow(0, n, n);
+        if (db.defined()) db1 = db.narrow(0, 0, n), db2 = db.narrow(0, n, n);
+      } else {
+        for (int i = 0; i < 2; ++i) {
+          const Tensor& dy = grads[i];
+          if (!need_x || !dy.defined()) continue;
+          Tensor flat = dy.reshape({-1, dy.size(-1)});
+          Tensor w = (i == 0 ? w1 : w2).to(dy.scalar_type());
+          if (dx.defined()) dx.addmm_(flat, w);
+          else dx = at::mm(flat, w);
+        }
+        if (dx.defined()) dx = dx.view(x.sizes());
+        if (grads[0].defined()) std::tie(dw1, db1) = linear_parameter_grads(x, w1.scalar_type(), grads[0], need_w1, need_b1 ? m[0] : kNone);
+        if (grads[1].defined()) std::tie(dw2, db2) = linear_parameter_grads(x, w2.scalar_type(), grads[1], need_w2, need_b2 ? m[1] : kNone);
+      }
+    }
+    return once({dx, dw1, db1, dw2, db2});
+  }
+};
+
+std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const MaybeTensor& b1_, const Tensor& w2, const MaybeTensor& b2_) {
+  Tensor b1 = opt(b1_), b2 = opt(b2_);
+  require_gpu("hip_linear_pair", {&x, &w1, &b1, &w2, &b2});
+  code_of(x.scalar_type());
+  auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2));
+  return {out[0], out[1]};
+}
+
+// ---- RMSNorm (griffin/griffin.py:68-80) ---------------------------------------------------------------------------
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> rmsnorm_forward(const Tensor& x_in, const Tensor& g, double eps) {
+  c10::DeviceGuard guard(x_in.device());
+  Tensor x = x_in.contiguous();
+  Tensor scale = operand(g, x.scalar_type());
+  const int64_t D = x.size(-1), rows = x.numel() / D;
+  Tensor y = fresh_like(x);
+  Tensor inv = fresh({rows}, at::kFloat, x);
+  if (rows > 0)
+    check(rglru_hip_rmsnorm_fwd(ptr(x), ptr(scale), ptr(y), fptr(inv), rows, D, static_cast<float>(eps), code_of(x.scalar_type()),
+                                code_of(scale.scalar_type()), stream_of(x)), "rglru_hip_rmsnorm_fwd");
+  return {x, scale, y, inv};
+}
+
+struct RmsNorm : torch::autograd::Function<RmsNorm> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& g, double eps) {
+    auto [x, scale, y, inv] = rmsnorm_forward(x_in, g, eps);
+    ctx->save_for_backward({x, scale, inv});
+    pack(ctx, {type_or_none(g)});
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto s = ctx->get_saved_variables();
+    const Tensor &x = s[0], &scale = s[1], &inv = s[2];
+    Tensor dx, dg;
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(x.device());
+      const int64_t D = x.size(-1), rows = x.numel() / D;
+      Tensor dy = as(grads[0], x.scalar_type());
+      const auto gt = scale.scalar_type();
+      dx = fresh_like(x);
+      if (ctx->needs_input_grad(1)) dg = fresh({D}, gt, x);
+      if (rows > 0) {
+        Tensor scratch = bytes(rglru_hip_rmsnorm_scratch_bytes(rows, D), x);
+        check(rglru_hip_rmsnorm_bwd(ptr(x), ptr(scale), fptr(inv), ptr(dy), ptr(scratch), ptr(dx), ptr(dg), rows, D,
+                                    code_of(x.scalar_type()), code_of(gt), code_of(gt), stream_of(x)), "rglru_hip_rmsnorm_bwd");
+      } else if (dg.defined()) {
+        dg.zero_();
+      }
+      if (dg.defined()) dg = dg.to(type_at(unpack(ctx), 0));
+    }
+    return once({dx, dg, Tensor()});
+  }
+};
+
+Tensor rmsnorm(const Tensor& x, const Tensor& g, double eps) {
+  require_gpu("hip_rmsnorm", {&x, &g});
+  TORCH_CHECK_VALUE(g.dim() == 1 && x.dim() >= 1 && x.size(-1) == g.numel(), "hip_rmsnorm expects a scale of shape [",
+                    x.dim() >= 1 ? x.size(-1) : 0, "], got ", g.sizes());
+  code_of(x.scalar_type());
+  if (wants_grad({&x, &g})) return RmsNorm::apply(x, g, eps);
+  at::NoGradGuard no_grad;
+  return std::get<2>(rmsnorm_forward(x, g, eps));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m) {
+#define EXPORT(name) m.def(#name, torch::wrap_pybind_function(name))
+  EXPORT(kernel_path);
+  EXPORT(prepare);
+  EXPORT(fingerprint);
+  EXPORT(rglru);
+  EXPORT(rglru_step);
+  EXPORT(rglru_steps);
+  EXPORT(rglru_module_step);
+  EXPORT(scan);
+  EXPORT(causal_conv);
+  EXPORT(causal_conv_padded);
+  EXPORT(gelu_gate);
+  EXPORT(block_flags);
+  EXPORT(block_forward);
+  EXPORT(block_decode_step);
+  EXPORT(sum_sets);
+  EXPORT(stacked_halves);
+  EXPORT(linear);
+  EXPORT(linear_pair);
+  EXPORT(rmsnorm);
+#undef EXPORT
+}

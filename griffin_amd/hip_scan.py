@@ -10,14 +10,12 @@ There is no CPU fallback in this file: every operator raises when the library or
 
 from __future__ import annotations
 
-import weakref
-
 import threading
 import warnings
+import weakref
 
 import torch
 from torch import Tensor
-from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -47,7 +45,6 @@ def set_chain_forward(mode: int) -> int:
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-_raw_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _stream_ptr(device: torch.device) -> int:
@@ -56,25 +53,6 @@ def _stream_ptr(device: torch.device) -> int:
     if _raw_stream is not None and index is not None:
         return _raw_stream(index)                        # no Stream object: a fraction of a microsecond
     return torch.cuda.current_stream(device).cuda_stream
-
-
-class _NoSwitch:
-    def __enter__(self):
-        return None
-
-    def __exit__(self, *exc):
-        return False
-
-
-_NO_SWITCH = _NoSwitch()
-
-
-def _on_device(device: torch.device):
-    """``torch.cuda.device(device)`` without the cost of the guard when ``device`` is current already
-    (the usual case; the guard costs several microseconds per call, as much as a decode step's kernel)."""
-    if _raw_device is not None and device.index is not None and _raw_device() == device.index:
-        return _NO_SWITCH
-    return torch.cuda.device(device)
 
 
 class _FirstTokenReset:
@@ -88,24 +66,12 @@ class _FirstTokenReset:
 FIRST_TOKEN_RESET = _FirstTokenReset()
 
 
-def _flags_ptr(flags) -> int | None:
-    return 1 if flags is FIRST_TOKEN_RESET else _ptr(flags)
-
-
 def _ptr(t: Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-_gpu_seen = False
-
-
 def _require_gpu(name: str, *tensors: Tensor) -> None:
-    global _gpu_seen
-    if not _gpu_seen:
-        _lib.load()  # raises RuntimeError when the extension is missing
-        if not torch.cuda.is_available():
-            raise RuntimeError(f"{name} requires a CUDA/HIP device, none is available")
-        _gpu_seen = True                                 # both facts hold for the life of the process
+    _lib.native()  # raises RuntimeError when the library or its binding is missing
     for t in tensors:
         if t is not None and not t.is_cuda:
             raise RuntimeError(f"{name} requires CUDA/HIP tensors, got a {t.device.type} tensor")
@@ -114,66 +80,9 @@ def _require_gpu(name: str, *tensors: Tensor) -> None:
 # ----------------------------------------------------------------------------------------------
 # scan-only operator: h_t = a_t h_{t-1} + z_t
 # ----------------------------------------------------------------------------------------------
-class _HipScan(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, decay: Tensor, current_input: Tensor, initial_state: Tensor) -> Tensor:
-        _require_gpu("hip_rglru_scan", decay, current_input, initial_state)
-        if decay.dim() != 3 or decay.shape != current_input.shape:
-            raise ValueError("decay and current_input must share shape [batch, sequence, width]")
-        if initial_state.shape != (decay.size(0), decay.size(2)):
-            raise ValueError("initial_state must have shape [batch, width]")
-        if decay.dtype != torch.float32 or current_input.dtype != torch.float32:
-            raise TypeError("hip_rglru_scan expects fp32 decay and normalized input")
-        if initial_state.dtype != torch.float32:
-            raise TypeError("hip_rglru_scan expects fp32 recurrent state")
-        lib = _lib.load()
-        decay = decay.contiguous()
-        current_input = current_input.contiguous()
-        initial_state = initial_state.contiguous()
-        B, T, W = decay.shape
-        out = torch.empty_like(current_input)
-        if out.numel() == 0:
-            ctx.save_for_backward(decay, initial_state, out)
-            return out
-        with _on_device(decay.device):
-            ws = torch.empty(lib.rglru_hip_scan_workspace_bytes(B, T, W), dtype=torch.uint8, device=decay.device)
-            _lib.check(lib.rglru_hip_scan_fwd(decay.data_ptr(), current_input.data_ptr(), initial_state.data_ptr(),
-                                              out.data_ptr(), ws.data_ptr(), B, T, W, _stream_ptr(decay.device)),
-                       "rglru_hip_scan_fwd")
-        ctx.save_for_backward(decay, initial_state, out)
-        # the forward call has cleared the backward part of the workspace too: the first backward call over this
-        # forward finds it clear (a repeated one clears its part itself)
-        ctx.workspace = [ws]
-        return out
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, grad_out: Tensor):
-        decay, initial_state, out = ctx.saved_tensors
-        lib = _lib.load()
-        grad_out = grad_out.contiguous()
-        B, T, W = decay.shape
-        d_decay = torch.empty_like(decay)
-        d_input = torch.empty_like(decay)
-        d_state = torch.empty_like(initial_state)
-        if decay.numel() == 0:
-            return d_decay, d_input, d_state.zero_()
-        with _on_device(decay.device):
-            held = getattr(ctx, "workspace", None)
-            fresh = bool(held)
-            ws = held.pop() if fresh else torch.empty(lib.rglru_hip_scan_workspace_bytes(B, T, W), dtype=torch.uint8,
-                                                      device=decay.device)
-            _lib.check(lib.rglru_hip_scan_bwd(decay.data_ptr(), initial_state.data_ptr(), out.data_ptr(),
-                                              grad_out.data_ptr(), d_decay.data_ptr(), d_input.data_ptr(),
-                                              d_state.data_ptr(), ws.data_ptr(), 1 if fresh else 0, B, T, W,
-                                              _stream_ptr(decay.device)),
-                       "rglru_hip_scan_bwd")
-        return d_decay, d_input, d_state
-
-
 def hip_rglru_scan(decay: Tensor, current_input: Tensor, initial_state: Tensor) -> Tensor:
     """Differentiable linear recurrence on the GPU (contract of griffin/triton_scan.py:274-276)."""
-    return _HipScan.apply(decay, current_input, initial_state)
+    return _lib.native().scan(decay, current_input, initial_state)
 
 
 # ----------------------------------------------------------------------------------------------
@@ -219,65 +128,17 @@ def pack_flags(reset_mask: Tensor | None, active_mask: Tensor | None) -> Tensor 
     return None if flags is None else flags.contiguous()
 
 
-def _parameter_operands(w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor, lam: Tensor, dtype: torch.dtype):
-    """The five parameters as the library reads them: gate weights in the storage type; biases and
-    Lambda in their own type when the library knows it (fp32 or bf16), so the usual cases launch no
-    conversion kernels.  Returns the tensors (kept alive by the caller) and the vector dtype code."""
-    vec_dtype = b_a.dtype if (b_a.dtype == b_x.dtype == lam.dtype and b_a.dtype in _DTYPE_CODES) else torch.float32
-    tensors = (w_a.detach().to(dtype).contiguous(), b_a.detach().to(vec_dtype).contiguous(),
-               w_x.detach().to(dtype).contiguous(), b_x.detach().to(vec_dtype).contiguous(),
-               lam.detach().to(vec_dtype).contiguous())
-    return tensors, _DTYPE_CODES[vec_dtype]
-
-
-def _prep_bytes(width: int, blocks: int, code: int) -> int:
-    size = _lib.load().rglru_hip_prep_bytes(width, blocks, code)
-    if size == 0:
-        _lib.check(2, "rglru_hip_prep_bytes")
-    return size
-
-
 class PreparedParams:
     """Kernel-side image of the RG-LRU parameters (see rglru_hip_prepare)."""
 
     def __init__(self, w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor, lam: Tensor, c: float, dtype: torch.dtype):
-        lib = _lib.load()
         nb, bw, _ = w_a.shape
         self.width = nb * bw
         self.blocks = nb
         self.dtype = dtype
         self.c = float(c)
-        code = _dtype_code(dtype)
-        size = _prep_bytes(self.width, nb, code)
-        device = w_a.device
-        operands, vec_code = _parameter_operands(w_a, b_a, w_x, b_x, lam, dtype)
-        with _on_device(device):
-            self.image = torch.empty(size, dtype=torch.uint8, device=device)
-            _lib.check(lib.rglru_hip_prepare(*(t.data_ptr() for t in operands), self.c, self.width, nb, code, vec_code,
-                                             self.image.data_ptr(), _stream_ptr(device)), "rglru_hip_prepare")
-
-
-def _check_fused_inputs(x: Tensor, w_a: Tensor, h0: Tensor | None, flags: Tensor | None) -> None:
-    if x.dim() != 3:
-        raise ValueError(f"hip RG-LRU expects [batch, sequence, width], got {tuple(x.shape)}")
-    B, T, W = x.shape
-    nb, bw, bw2 = w_a.shape
-    if bw != bw2 or nb * bw != W:
-        raise ValueError(f"gate weights {tuple(w_a.shape)} do not match width {W}")
-    if h0 is not None and h0.shape != (B, W):
-        raise ValueError(f"initial state must have shape ({B}, {W}), got {tuple(h0.shape)}")
-    if flags is not None and flags is not FIRST_TOKEN_RESET and flags.shape != (B, T):
-        raise ValueError(f"token flags must have shape ({B}, {T}), got {tuple(flags.shape)}")
-    if T == 0 or B == 0:
-        raise ValueError("hip RG-LRU does not accept empty batches or sequences")
-    _dtype_code(x.dtype)
-
-
-def _aligned(t: Tensor) -> Tensor:
-    """``t`` itself when its storage starts on a 16-byte boundary (what every fresh allocation does), else a
-    copy that does: a view at an odd offset costs one copy instead of sending the whole call to the portable
-    kernels, which are several times slower."""
-    return t if t.data_ptr() % 16 == 0 else t.clone(memory_format=torch.contiguous_format)
+        _dtype_code(dtype)
+        self.image = _lib.native().prepare(w_a, b_a, w_x, b_x, lam, self.c, dtype)
 
 
 def kernel_path(B: int, T: int, W: int, nb: int, dtype: torch.dtype, *tensors: Tensor) -> int:
@@ -285,133 +146,7 @@ def kernel_path(B: int, T: int, W: int, nb: int, dtype: torch.dtype, *tensors: T
     ``_lib.PATH_*``.  ``tensors``: the activation tensors of the call; one that is not 16-byte aligned
     sends the call to the portable kernels."""
     aligned = all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
-    path = _lib.load().rglru_hip_backward_path(B, T, W, nb, _dtype_code(dtype), 1 if aligned else 0)
-    if path < 0:
-        _lib.check(2, "rglru_hip_backward_path")
-    return path
-
-
-class _HipRGLRU(torch.autograd.Function):
-    """y, h_T = RG-LRU(x; W_a, b_a, W_x, b_x, Lambda) with a recomputing backward."""
-
-    @staticmethod
-    def forward(ctx, x, w_a, b_a, w_x, b_x, lam, h0, flags, c):
-        first_reset = flags is FIRST_TOKEN_RESET
-        _require_gpu("hip RG-LRU", x, w_a, b_a, w_x, b_x, lam, h0, None if first_reset else flags)
-        _check_fused_inputs(x, w_a, h0, flags)
-        lib = _lib.load()
-        x = _aligned(x.contiguous())
-        B, T, W = x.shape
-        nb = w_a.shape[0]
-        code = _dtype_code(x.dtype)
-        operands, vec_code = _parameter_operands(w_a, b_a, w_x, b_x, lam, x.dtype)
-        h0c = None if h0 is None else h0.detach().to(torch.float32).contiguous()
-        device = x.device
-        with _on_device(device):
-            y = torch.empty_like(x)
-            h_last = torch.empty(B, W, dtype=torch.float32, device=device)
-            image = torch.empty(_prep_bytes(W, nb, code), dtype=torch.uint8, device=device)
-            ws = torch.empty(lib.rglru_hip_workspace_bytes(B, T, W, nb), dtype=torch.uint8, device=device)
-            if kernel_path(B, T, W, nb, x.dtype, x) == _lib.PATH_PRE:
-                pre = torch.empty(nb, B * T, 2 * (W // nb), dtype=x.dtype, device=device)   # scratch of the call
-                _lib.check(lib.rglru_hip_prepare(*(t.data_ptr() for t in operands), float(c), W, nb, code, vec_code,
-                                                 image.data_ptr(), _stream_ptr(device)), "rglru_hip_prepare")
-                _lib.check(lib.rglru_hip_fwd_pre(x.data_ptr(), pre.data_ptr(), image.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                                 y.data_ptr(), h_last.data_ptr(), ws.data_ptr(), B, T, W, nb, code,
-                                                 _stream_ptr(device)), "rglru_hip_fwd_pre")
-                del pre
-            else:
-                # parameter conversion, workspace clearing and the forward kernel: two launches, or one where the
-                # forward kernel does all three (batch-rich shapes)
-                _lib.check(lib.rglru_hip_prepare_fwd(*(t.data_ptr() for t in operands), float(c), vec_code,
-                                                     image.data_ptr(), x.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                                     y.data_ptr(), h_last.data_ptr(), ws.data_ptr(), B, T, W, nb, code,
-                                                     _stream_ptr(device)), "rglru_hip_prepare_fwd")
-        ctx.save_for_backward(x, w_a, w_x, h0c, None if first_reset else flags, ws, image, y)
-        ctx.first_reset = first_reset
-        ctx.param_dtypes = (w_a.dtype, b_a.dtype, w_x.dtype, b_x.dtype, lam.dtype)
-        ctx.h0_dtype = None if h0 is None else h0.dtype
-        ctx.set_materialize_grads(False)      # an unused output arrives as None, not as a tensor of zeros
-        return y, h_last
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, dy, dh_last):
-        x, w_a, w_x, h0c, flags, ws, image, y = ctx.saved_tensors
-        if ctx.first_reset:
-            flags = FIRST_TOKEN_RESET
-        dx, dw_a, db_a, dw_x, db_x, dlam, dh0 = rglru_backward(
-            x, y, w_a, w_x, h0c, flags, ws, image, dy, dh_last, ctx.param_dtypes, ctx.needs_input_grad[6])
-        return (dx, dw_a, db_a, dw_x, db_x, dlam, None if dh0 is None else dh0.to(ctx.h0_dtype), None, None)
-
-
-def rglru_backward(x, y, w_a, w_x, h0c, flags, ws, image, dy, dh_last, param_dtypes, need_dh0):
-    """Backward pass of the RG-LRU on what its forward kept (the workspace with checkpoints and records, the
-    parameter image): returns (dx, dW_a, db_a, dW_x, db_x, dLambda, dh0 in fp32 or None), the parameter
-    gradients in the parameters' types."""
-    lib = _lib.load()
-    B, T, W = x.shape
-    nb, bw, _ = w_a.shape
-    code = _dtype_code(x.dtype)
-    device = x.device
-    dy = torch.zeros_like(x) if dy is None else _aligned(dy.to(x.dtype).contiguous())
-    dhl = None if dh_last is None else dh_last.to(torch.float32).contiguous()
-    # parameter gradients come back in the parameters' own type when all five share one the
-    # library writes (fp32 or bf16); otherwise in fp32, converted below
-    pd = param_dtypes
-    gdt = pd[0] if (len(set(pd)) == 1 and pd[0] in _DTYPE_CODES) else torch.float32
-    gcode = _DTYPE_CODES[gdt]
-    with _on_device(device):
-        dx = torch.empty_like(x)
-        db_a = torch.empty(nb, bw, dtype=gdt, device=device)
-        db_x = torch.empty(nb, bw, dtype=gdt, device=device)
-        dlam = torch.empty(W, dtype=gdt, device=device)
-        dh0 = torch.empty(B, W, dtype=torch.float32, device=device) if need_dh0 else None
-        # scratch of this call only (the workspace kept since forward holds just checkpoints and records)
-        scratch = torch.empty(lib.rglru_hip_bwd_scratch_bytes(B, T, W, nb, code), dtype=torch.uint8, device=device)
-        path = kernel_path(B, T, W, nb, x.dtype, x, y, dy, dx)
-        if path in (_lib.PATH_FAST_CHAIN, _lib.PATH_FAST_TILED):
-            # everything in hand-written kernels, including the two gate GEMMs
-            dw_a = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            dw_x = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            _lib.check(lib.rglru_hip_bwd_full(x.data_ptr(), y.data_ptr(), image.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                              dy.data_ptr(), _ptr(dhl), ws.data_ptr(), scratch.data_ptr(), dx.data_ptr(), dw_a.data_ptr(),
-                                              dw_x.data_ptr(), db_a.data_ptr(), db_x.data_ptr(), dlam.data_ptr(),
-                                              _ptr(dh0), B, T, W, nb, code, gcode, _stream_ptr(device)),
-                       "rglru_hip_bwd_full")
-        elif path == _lib.PATH_WIDE:
-            # blocks of 160 .. 384 channels: scan and gate math, then the two gate GEMMs, all hand-written
-            dw_a = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            dw_x = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            _lib.check(lib.rglru_hip_bwd_wide(x.data_ptr(), image.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                              dy.data_ptr(), _ptr(dhl), ws.data_ptr(), scratch.data_ptr(), dx.data_ptr(), dw_a.data_ptr(),
-                                              dw_x.data_ptr(), db_a.data_ptr(), db_x.data_ptr(), dlam.data_ptr(),
-                                              _ptr(dh0), B, T, W, nb, code, gcode, _stream_ptr(device)),
-                       "rglru_hip_bwd_wide")
-        elif path == _lib.PATH_PRE:
-            # bf16 blocks of 416 .. 512 channels: a GEMM kernel for the gate projections, the scan and all gate math
-            # in the scan kernel, then the two GEMM kernels of the gate gradients
-            dw_a = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            dw_x = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            pre = torch.empty(nb, B * T, 2 * bw, dtype=x.dtype, device=device)
-            du = torch.empty_like(pre)
-            _lib.check(lib.rglru_hip_bwd_pre(x.data_ptr(), pre.data_ptr(), image.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                             dy.data_ptr(), _ptr(dhl), ws.data_ptr(), scratch.data_ptr(), dx.data_ptr(),
-                                             du.data_ptr(), dw_a.data_ptr(), dw_x.data_ptr(), db_a.data_ptr(), db_x.data_ptr(),
-                                             dlam.data_ptr(), _ptr(dh0), B, T, W, nb, code, gcode, _stream_ptr(device)),
-                       "rglru_hip_bwd_pre")
-        else:
-            # any storage type, width and alignment: the scan kernel leaves the gradients at the gate
-            # pre-activations in du_a, du_x; two GEMM kernels of the library finish dW and dx
-            dw_a = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            dw_x = torch.empty(nb, bw, bw, dtype=gdt, device=device)
-            du_a = torch.empty_like(x)
-            du_x = torch.empty_like(x)
-            _lib.check(lib.rglru_hip_bwd(x.data_ptr(), image.data_ptr(), _ptr(h0c), _flags_ptr(flags),
-                                         dy.data_ptr(), _ptr(dhl), ws.data_ptr(), scratch.data_ptr(), dx.data_ptr(), du_a.data_ptr(),
-                                         du_x.data_ptr(), dw_a.data_ptr(), dw_x.data_ptr(), db_a.data_ptr(), db_x.data_ptr(),
-                                         dlam.data_ptr(), _ptr(dh0), B, T, W, nb, code, gcode, _stream_ptr(device)), "rglru_hip_bwd")
-    return dx, dw_a.to(pd[0]), db_a.to(pd[1]), dw_x.to(pd[2]), db_x.to(pd[3]), dlam.to(pd[4]), dh0
+    return _lib.native().kernel_path(B, T, W, nb, dtype, aligned)
 
 
 def hip_rglru(x: Tensor, w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor, lam: Tensor, c: float = 8.0,
@@ -424,29 +159,36 @@ def hip_rglru(x: Tensor, w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor, lam
     if first_token_reset:
         if reset_mask is not None or active_mask is not None:
             raise ValueError("first_token_reset replaces the masks; pass one or the other")
-        flags = FIRST_TOKEN_RESET
+        flags = None
     else:
         flags = pack_flags(reset_mask, active_mask)
-    return _HipRGLRU.apply(x, w_a, b_a, w_x, b_x, lam, h0, flags, c)
+    native = _lib.native()
+    # a misaligned view is copied onto a 16-byte boundary first, so the shape alone decides
+    regular = x.is_cuda and x.dim() == 3 and x.dtype in _DTYPE_CODES and x.numel() > 0 and x.size(2) % w_a.size(0) == 0
+    path = kernel_path(*x.shape, w_a.size(0), x.dtype) if regular else 0
+    return native.rglru(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_token_reset, c, path)
 
 
 def hip_rglru_step(x: Tensor, prep: PreparedParams, state: Tensor, flags: Tensor | None = None) -> Tensor:
     """One decode step: ``state`` [B, W] fp32 is updated in place; returns y [B, W] in x.dtype."""
-    _require_gpu("hip RG-LRU step", x, state, flags)
     if x.dim() != 2 or x.shape[1] != prep.width:
         raise ValueError(f"step expects x of shape [batch, {prep.width}], got {tuple(x.shape)}")
-    if state.shape != x.shape or state.dtype != torch.float32 or not state.is_contiguous():
-        raise ValueError("step expects a contiguous fp32 state of the same shape as x")
     if x.dtype != prep.dtype:
         raise TypeError(f"parameters were prepared for {prep.dtype}, got activations in {x.dtype}")
-    lib = _lib.load()
-    x = x.contiguous()
-    with _on_device(x.device):
-        y = torch.empty_like(x)
-        _lib.check(lib.rglru_hip_step(x.data_ptr(), prep.image.data_ptr(), state.data_ptr(), _ptr(flags),
-                                      y.data_ptr(), x.shape[0], prep.width, prep.blocks, _dtype_code(x.dtype),
-                                      _stream_ptr(x.device)), "rglru_hip_step")
-    return y
+    return _lib.native().rglru_step(x, prep.image, prep.blocks, state, flags)
+
+
+def hip_rglru_module_step(x: Tensor, prep: PreparedParams, state: Tensor | None, flags: Tensor | None) -> tuple[Tensor, Tensor]:
+    """One decode step of the layer: ``x`` [B, 1, W], ``state`` [B, W] or None (zeros) left untouched, ``flags``
+    [B, 1] or None.  Returns (y [B, 1, W], the new state [B, W] fp32)."""
+    return _lib.native().rglru_module_step(x, prep.image, prep.blocks, state, flags)
+
+
+def fingerprint(tensors) -> tuple:
+    """What tells whether any of ``tensors`` was replaced or written to in place: storage addresses and version
+    counters."""
+    return _lib.native().fingerprint(tensors) if _lib.available() else tuple(
+        v for t in tensors for v in (t.data_ptr(), t._version))
 
 
 def hip_rglru_steps(xs: Tensor, prep: PreparedParams, state: Tensor, flags: Tensor | None = None) -> Tensor:
@@ -462,17 +204,7 @@ def hip_rglru_steps(xs: Tensor, prep: PreparedParams, state: Tensor, flags: Tens
         raise ValueError("flags must be uint8 of shape [steps, batch]")
     if xs.dtype != prep.dtype:
         raise TypeError(f"parameters were prepared for {prep.dtype}, got activations in {xs.dtype}")
-    lib = _lib.load()
-    xs = xs.contiguous()
-    K, B, _ = xs.shape
-    with _on_device(xs.device):
-        ys = torch.empty_like(xs)
-        if K > 0 and B > 0:
-            _lib.check(lib.rglru_hip_steps(xs.data_ptr(), prep.image.data_ptr(), state.data_ptr(),
-                                           None if flags is None else flags.contiguous().data_ptr(), ys.data_ptr(),
-                                           K, B, prep.width, prep.blocks, _dtype_code(xs.dtype), _stream_ptr(xs.device)),
-                       "rglru_hip_steps")
-    return ys
+    return _lib.native().rglru_steps(xs, prep.image, prep.blocks, state, flags)
 
 
 # ----------------------------------------------------------------------------------------------
@@ -647,6 +379,10 @@ def _validate_hip_scan(device: torch.device) -> None:
 
 def hip_scan_is_usable(device: torch.device | str) -> bool:
     """Validate the HIP kernels once per device before ``scan_mode="auto"`` may use them."""
+    if isinstance(device, torch.device) and device.index is not None and device.type == "cuda":
+        known = _VALIDATED.get(device.index)               # asked on every call of a module: no lock, no device query
+        if known is not None:
+            return known
     resolved = torch.device(device)
     if resolved.type != "cuda" or not torch.cuda.is_available() or not hip_scan_available():
         return False

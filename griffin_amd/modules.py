@@ -96,8 +96,14 @@ class RG_LRU(nn.Module):
         )
 
     def _gate_parameters(self):
-        return (self.recurrence_gate.weight, self.recurrence_gate.bias, self.input_gate.weight,
-                self.input_gate.bias, self.Lambda)
+        try:
+            # nn.Module's attribute lookup costs as much as a launch over these seven names
+            gates = self._modules
+            r, i = gates["recurrence_gate"]._parameters, gates["input_gate"]._parameters
+            return r["weight"], r["bias"], i["weight"], i["bias"], self._parameters["Lambda"]
+        except KeyError:                                     # a parametrised or otherwise replaced parameter
+            return (self.recurrence_gate.weight, self.recurrence_gate.bias, self.input_gate.weight,
+                    self.input_gate.bias, self.Lambda)
 
     def _needs_grad(self, xt: Tensor, ht_minus_1: Tensor | None) -> bool:
         if not torch.is_grad_enabled():
@@ -109,7 +115,7 @@ class RG_LRU(nn.Module):
         """Kernel-side parameter image for inference, rebuilt when a parameter is replaced or updated
         in place (every in-place update bumps the tensor's version counter)."""
         params = self._gate_parameters()
-        key = (dtype, device, float(self.c)) + tuple((q.data_ptr(), q._version) for q in params)
+        key = (dtype, device, self.c, *hip_scan.fingerprint(params))
         if getattr(self, "_prep_key", None) != key:
             prep = hip_scan.PreparedParams(*params, self.c, dtype)
             if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
@@ -184,19 +190,14 @@ class RG_LRU(nn.Module):
             if steps == 1 and not self._needs_grad(xt, ht_minus_1):
                 # decode: the single-step kernel on a prepared parameter image kept between calls
                 prep = self._prepared(xt.dtype, xt.device)
-                state = (torch.zeros(batch, width, device=xt.device, dtype=torch.float32) if ht_minus_1 is None
-                         else ht_minus_1.to(torch.float32).clone(memory_format=torch.contiguous_format))
-                flags = hip_scan.pack_flags(reset_mask, active_mask)
-                y = hip_scan.hip_rglru_step(xt[:, 0], prep, state, None if flags is None else flags.reshape(batch))
-                y = y.unsqueeze(1)
+                y, state = hip_scan.hip_rglru_module_step(xt, prep, ht_minus_1, hip_scan.pack_flags(reset_mask, active_mask))
                 return (y, state) if return_state else y
             # the reset mask of the default positions (a document start at token 0 of every row, nothing else)
             # is known by identity: the kernels then need no per-token flags at all
             default = _DEFAULT_POSITIONS.get((batch, steps, xt.device))
             first_only = default is not None and reset_mask is default[1] and active_mask is None
             y, state = hip_scan.hip_rglru(
-                xt, self.recurrence_gate.weight, self.recurrence_gate.bias, self.input_gate.weight,
-                self.input_gate.bias, self.Lambda, self.c, ht_minus_1, None if first_only else reset_mask, active_mask,
+                xt, *self._gate_parameters(), self.c, ht_minus_1, None if first_only else reset_mask, active_mask,
                 first_token_reset=first_only,
             )
             return (y, state) if return_state else y
@@ -444,7 +445,7 @@ class RecurrentBlock(nn.Module):
         until a weight or bias changes (storage or version counter)."""
         layers = (self.linear_x, self.linear_y)
         tensors = [t for layer in layers for t in (layer.weight, layer.bias) if t is not None]
-        key = tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in tensors)
+        key = (*hip_scan.fingerprint(tensors), *((t.dtype, t.device) for t in tensors))
         cached = getattr(self, "_stacked_projection", None)
         if cached is None or cached[0] != key:
             if len(tensors) != 4 or (token.is_cuda and torch.cuda.is_current_stream_capturing()):
