@@ -14,7 +14,7 @@ RGLRU_BF16 = 1
 FLAG_RESET = 1
 FLAG_INACTIVE = 2
 CHUNK = 32
-ABI_VERSION = 19
+ABI_VERSION = 20
 PATH_PORTABLE, PATH_FAST_TILED, PATH_FAST_CHAIN, PATH_WIDE, PATH_PRE = range(5)
 PATH_NAMES = ("portable", "fast_tiled", "fast_chain", "wide", "pre")
 
@@ -54,6 +54,11 @@ _SIGNATURES = {
     "rglru_hip_conv_fwd": (ctypes.c_int, [_P] * 7 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_conv_scratch_bytes": (ctypes.c_size_t, [_I, _I, _I, _I]),
     "rglru_hip_conv_bwd": (ctypes.c_int, [_P] * 7 + [_I] + [_P] * 3 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "rglru_hip_conv_rows_bwd": (ctypes.c_int, [_P] * 8 + [_I] + [_P] * 3 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "rglru_hip_conv_carry": (ctypes.c_int, [_P, _I] + [_P] * 3 + [_I, _I, _I, _I, ctypes.c_int, _P]),
+    "rglru_hip_token_facts": (ctypes.c_int, [_P] * 9 + [_I, _I, _P]),
+    "rglru_hip_pack_flags": (ctypes.c_int, [_P] * 3 + [_I, _P]),
+    "rglru_hip_mask_rows": (ctypes.c_int, [_P] * 3 + [_I, _I, ctypes.c_int, _P]),
     "rglru_hip_conv_padded_scratch_bytes": (ctypes.c_size_t, [_I, _I]),
     "rglru_hip_conv_padded_fwd": (ctypes.c_int, [_P] * 9 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_conv_padded_bwd": (ctypes.c_int, [_P] * 12 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
@@ -67,6 +72,8 @@ _SIGNATURES = {
     "rglru_hip_rmsnorm_scratch_bytes": (ctypes.c_size_t, [_I, _I]),
     "rglru_hip_rmsnorm_bwd": (ctypes.c_int, [_P] * 7 + [_I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_decode_prepare": (ctypes.c_int, [_P, _I] + [_P] * 10 + [_I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
+    "rglru_hip_decode_linear": (ctypes.c_int, [_P, _I] + [_P] * 4 + [_I, _I, _I, ctypes.c_int, _P]),
+    "rglru_hip_decode_project": (ctypes.c_int, [_P, _I] + [_P] * 15 + [_I, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_block_fwd_path": (ctypes.c_int, [_I, _I, _I, ctypes.c_int]),
     "rglru_hip_block_flags": (ctypes.c_int, [_P, _P, _I, _P]),
     "rglru_hip_block_fwd": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _P, _I, ctypes.c_int] + [_P] * 9

@@ -1316,6 +1316,14 @@ int rglru_hip_conv_bwd(const void* u, const void* state, const void* taps, const
                        const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
                        int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
                        void* stream) {
+  return rglru_hip_conv_rows_bwd(u, state, taps, segment_pos, nullptr, dout, scratch, du, du_stride, dstate, dtaps, dbias, B, T, W,
+                                 K, dtype, vec_dtype, grad_dtype, stream);
+}
+
+int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
+                            const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
+                            int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
+                            void* stream) {
   int rc = conv_check("conv_bwd", B, T, W, K, dtype, vec_dtype);
   if (rc) return rc;
   if (du_stride == 0) du_stride = W;
@@ -1328,6 +1336,7 @@ int rglru_hip_conv_bwd(const void* u, const void* state, const void* taps, const
   memset(&a, 0, sizeof(a));
   a.u = u; a.state = state; a.taps = taps; a.segpos = (const long long*)segment_pos;
   a.dout = dout; a.du = du; a.dstate = dstate; a.partial = (float*)scratch; a.ld_du = du_stride;
+  a.rows = rows;
   a.B = (int)B; a.T = (int)T; a.W = (int)W; a.K = (int)K; a.vec_dtype = vec_dtype;
   const bool vec = conv_vector_ok(W, dtype, {u, state, dout, du, dstate}) && (du_stride * (dtype == RGLRU_BF16 ? 2 : 4)) % 16 == 0;
   a.nvec = (int)(vec ? W / (dtype == RGLRU_BF16 ? 8 : 4) : W);

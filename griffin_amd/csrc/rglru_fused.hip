@@ -399,6 +399,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int hidden = MASKED ? (int)((conv_fl >> (8 * i + 2)) & 3u) : 0;        // lags 4 - hidden .. 3 do not apply
+          const bool padding = MASKED && ((conv_fl >> (8 * i)) & RGLRU_FLAG_INACTIVE);   // takes no part: zero, like the padded convolution
           Frag out;
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
               const float with = fmaf((float)um[3 + i - lag][e], tap[lag][e], a);
               a = (MASKED && lag + hidden > 3) ? a : with;
             }
-            out[e] = (IO)a;
+            out[e] = (IO)(padding ? 0.f : a);
           }
           *reinterpret_cast<Frag*>(lds + (4 * rho + i) * LDSROW + bcv * Tr::HW) = out;
           buf_store_b128(__builtin_bit_cast(i32x4, out), rxo, bcol_ok ? (unsigned)(4 * rho + i) * row_bytes + bcol_bytes : kOutOfRange);

@@ -9,6 +9,8 @@
 // ValueError for shapes, TypeError for types.
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
@@ -27,6 +29,16 @@ using torch::autograd::AutogradContext;
 using torch::autograd::Variable;
 using torch::autograd::variable_list;
 using MaybeTensor = std::optional<Tensor>;
+
+// Whether a decode step of so many multiply-adds in its three projections takes the library's own kernels.  Against the BLAS
+// library they are faster up to about 16 rows of a 768 x 1024 block and up to three times slower beyond (GPU time of 512 rows,
+// 2560 -> 5120: 70 against 23 us in bf16), but a call of it costs the host 25 us: the line lies where our launches take
+// about as long as the host would (75 us at the rates the kernels reach, 1e8 multiply-adds a microsecond in bf16, 0.4e8 in
+// fp32); inside a captured graph, where host time is nothing, at the sizes where the kernels themselves are no slower.
+bool own_projections(double macs, at::ScalarType dtype) {
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < 1e8;
+  return macs < (dtype == at::kBFloat16 ? 7.5e9 : 3e9);
+}
 
 // ---- small helpers ---------------------------------------------------------------------------------------------
 
@@ -382,22 +394,21 @@ Tensor rglru_steps(const Tensor& xs_in, const Tensor& image, int64_t blocks, con
   return ys;
 }
 
-// One token per row of the bare layer: y and the new state, the old one untouched (x [B, 1, W]).  The kernel takes the
-// state in place, so the copy into the new buffer is the only other launch.
-std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x, const Tensor& image, int64_t blocks, const MaybeTensor& state_,
+// One token per row of the bare layer: y and the new state, the old one untouched (x [B, 1, W]).
+std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const MaybeTensor& state,
                                              const MaybeTensor& flags_) {
   Tensor flags = opt(flags_);
-  require_gpu("hip RG-LRU step", {&x, &flags});
-  c10::DeviceGuard guard(x.device());
-  const int64_t B = x.size(0), W = x.size(2);
-  Tensor h = fresh({B, W}, at::kFloat, x);
-  if (state_.has_value()) h.copy_(*state_);
-  else h.zero_();
-  Tensor xc = x.contiguous();
+  require_gpu("hip RG-LRU step", {&x_in, &flags});
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(x_in.device());
+  const int64_t B = x_in.size(0), W = x_in.size(2);
+  Tensor x = x_in.contiguous();
+  Tensor h = state.has_value() ? as(*state, at::kFloat) : at::zeros({B, W}, x.options().dtype(at::kFloat));
+  Tensor h_new = fresh({B, W}, at::kFloat, x);
   Tensor y = fresh({B, 1, W}, x.scalar_type(), x);
-  check(rglru_hip_step(ptr(xc), ptr(image), fptr(h), bptr(flags), ptr(y), B, W, blocks, code_of(x.scalar_type()),
-                       stream_of(x)), "rglru_hip_step");
-  return {y, h};
+  check(rglru_hip_step_gated(ptr(x), ptr(image), fptr(h), fptr(h_new), bptr(flags), nullptr, 0, ptr(y), B, W, blocks,
+                             code_of(x.scalar_type()), stream_of(x)), "rglru_hip_step_gated");
+  return {y, h_new};
 }
 
 // ---- scan-only operator: h_t = a_t h_{t-1} + z_t (griffin/triton_scan.py:207-276) --------------------------------
@@ -462,6 +473,74 @@ Tensor scan(const Tensor& a, const Tensor& z, const Tensor& h0) {
 
 // ---- causal depthwise convolution (griffin/griffin.py:474-510) ----------------------------------------------------
 
+// What an activity mask says about every token (rglru_hip_token_facts), and, once the host asks, whether all tokens are
+// active and whether the rows are right-padded.  The answer is written to host memory by the kernel: asking waits for that
+// kernel alone, not for work queued behind it.
+struct TokenFacts {
+  Tensor positions, flags, conv_positions, rows, last_position;
+  TokenFacts(const Tensor& active_in, const MaybeTensor& segment_pos, const MaybeTensor& prev_pos) : event_(at::kCUDA) {
+    require_gpu("token facts", {&active_in});
+    at::NoGradGuard no_grad;
+    c10::DeviceGuard guard(active_in.device());
+    Tensor active = active_in.contiguous();
+    TORCH_CHECK_VALUE(active.dim() == 2 && active.element_size() == 1, "active_mask must be a [batch, sequence] mask");
+    const int64_t B = active.size(0), T = active.size(1);
+    Tensor prev;
+    if (segment_pos.has_value()) positions = segment_pos->to(active.device(), at::kLong).contiguous();
+    if (prev_pos.has_value()) prev = prev_pos->to(active.device(), at::kLong).contiguous();
+    const bool given = positions.defined();
+    TORCH_CHECK_VALUE(!given || positions.sizes() == active.sizes(), "segment_pos must have the shape of active_mask");
+    TORCH_CHECK_VALUE(!prev.defined() || (prev.dim() == 1 && prev.size(0) == B), "Cached segment positions have an incompatible shape");
+    if (!given) positions = fresh({B, T}, at::kLong, active);
+    flags = fresh({B, T}, at::kByte, active);
+    conv_positions = fresh({B, T}, at::kLong, active);
+    rows = fresh({3, B}, at::kInt, active);
+    last_position = fresh({B}, at::kLong, active);
+    answer_ = at::empty({B}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    check(rglru_hip_token_facts(bptr(active), given ? iptr(positions) : nullptr, iptr(prev),
+                                given ? nullptr : static_cast<int64_t*>(positions.data_ptr()), static_cast<uint8_t*>(flags.data_ptr()),
+                                static_cast<int64_t*>(conv_positions.data_ptr()), static_cast<int32_t*>(rows.data_ptr()),
+                                static_cast<int64_t*>(last_position.data_ptr()), static_cast<uint32_t*>(answer_.data_ptr()), B, T,
+                                stream_of(active)), "rglru_hip_token_facts");
+    event_.record(c10::Stream(c10::Stream::UNSAFE, active.device(), c10::hip::getCurrentHIPStream(active.device().index()).id()));
+  }
+  TokenFacts(const TokenFacts&) = delete;
+  ~TokenFacts() { wait(); }                  // the kernel writes into memory that this object gives back
+  std::tuple<bool, bool> resolve() {
+    {
+      py::gil_scoped_release no_gil;
+      wait();
+    }
+    bool all_active = true, prefix = true;
+    const int32_t* a = static_cast<const int32_t*>(answer_.data_ptr());
+    for (int64_t b = 0; b < answer_.size(0); ++b) all_active &= (a[b] & 1) != 0, prefix &= (a[b] & 2) != 0;
+    return {all_active, prefix};
+  }
+
+ private:
+  void wait() {
+    if (!done_) event_.synchronize();
+    done_ = true;
+  }
+  Tensor answer_;
+  c10::Event event_;
+  bool done_ = false;
+};
+
+Tensor pack_flags(const MaybeTensor& reset_, const MaybeTensor& active_) {
+  at::NoGradGuard no_grad;
+  auto mask = [](const MaybeTensor& m) { return m.has_value() ? m->to(at::kBool).contiguous() : Tensor(); };
+  Tensor reset = mask(reset_), active = mask(active_);
+  const Tensor& like = reset.defined() ? reset : active;
+  require_gpu("hip RG-LRU", {&reset, &active});
+  c10::DeviceGuard guard(like.device());
+  Tensor flags = fresh(like.sizes(), at::kByte, like);
+  if (flags.numel() > 0)
+    check(rglru_hip_pack_flags(bptr(reset), bptr(active), static_cast<uint8_t*>(flags.data_ptr()), flags.numel(), stream_of(like)),
+          "rglru_hip_pack_flags");
+  return flags;
+}
+
 struct ConvMeta {  // types of the forward's arguments (kNone: absent)
   int64_t state, weight, bias;
 };
@@ -469,7 +548,8 @@ struct ConvMeta {  // types of the forward's arguments (kNone: absent)
 // Reverse mode of the dense convolution on contiguous operands.  `du_out`: where to write du instead of a new tensor --
 // [B, T, W] with unit stride along W and rows a common distance apart (a column range of a wider matrix).
 variable_list conv_backward(const Tensor& u, const Tensor& state, const Tensor& taps, const Tensor& pos, const Tensor& dout_in,
-                            ConvMeta meta, bool need_u, bool need_state, bool need_w, bool need_b, const Tensor& du_out) {
+                            ConvMeta meta, bool need_u, bool need_state, bool need_w, bool need_b, const Tensor& du_out,
+                            const Tensor& rows = Tensor()) {
   const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = taps.size(2);
   Tensor dout = as(dout_in, u.scalar_type());
   const auto gt = taps.scalar_type();
@@ -479,9 +559,9 @@ variable_list conv_backward(const Tensor& u, const Tensor& state, const Tensor& 
   if (need_w) dtaps = fresh({W, 1, K}, gt, u);
   if (need_b && meta.bias != kNone) dbias = fresh({W}, gt, u);
   Tensor scratch = bytes(rglru_hip_conv_scratch_bytes(B, T, W, K), u);
-  check(rglru_hip_conv_bwd(ptr(u), ptr(state), ptr(taps), iptr(pos), ptr(dout), ptr(scratch), ptr(du), du.stride(1), ptr(dstate),
-                           ptr(dtaps), ptr(dbias), B, T, W, K, code_of(u.scalar_type()), code_of(gt), code_of(gt), stream_of(u)),
-        "rglru_hip_conv_bwd");
+  check(rglru_hip_conv_rows_bwd(ptr(u), ptr(state), ptr(taps), iptr(pos), static_cast<const int32_t*>(ptr(rows)), ptr(dout),
+                                ptr(scratch), ptr(du), du.stride(1), ptr(dstate), ptr(dtaps), ptr(dbias), B, T, W, K,
+                                code_of(u.scalar_type()), code_of(gt), code_of(gt), stream_of(u)), "rglru_hip_conv_rows_bwd");
   if (dtaps.defined()) dtaps = dtaps.to(static_cast<at::ScalarType>(meta.weight));
   if (dbias.defined()) dbias = dbias.to(static_cast<at::ScalarType>(meta.bias));
   if (need_state && meta.state != kNone)
@@ -686,7 +766,7 @@ struct BlockResult {
 BlockResult block_forward_pass(const Tensor& u, const Tensor& v, const Tensor& conv_state, const Tensor& weight,
                                const Tensor& bias, const Tensor& segment_pos, const Tensor& flags, bool first_reset,
                                const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam,
-                               const Tensor& h0, double c, const Tensor& image, bool training) {
+                               const Tensor& h0, double c, const Tensor& image, const Tensor& rows, bool need_carry, bool training) {
   BlockResult r;
   c10::DeviceGuard guard(u.device());
   const int64_t B = u.size(0), T = u.size(1), W = u.size(2), K = weight.size(2), nb = w_a.size(0);
@@ -704,7 +784,7 @@ BlockResult block_forward_pass(const Tensor& u, const Tensor& v, const Tensor& c
   r.new_conv = fresh({B, K - 1, W}, dtype, u);
   r.h_last = fresh({B, W}, at::kFloat, u);
   void* stream = stream_of(u);
-  void* new_conv = K > 1 ? ptr(r.new_conv) : nullptr;
+  void* new_conv = K > 1 && !rows.defined() ? ptr(r.new_conv) : nullptr;   // of a padded row: not its last tokens, see below
   const uint8_t* fl = flags_ptr(r.flags, first_reset);
   if (training || !image.defined()) {
     Operands p(w_a, b_a, w_x, b_x, lam, dtype);
@@ -720,6 +800,9 @@ BlockResult block_forward_pass(const Tensor& u, const Tensor& v, const Tensor& c
                               code_of(r.taps.scalar_type()), ptr(image), fptr(r.h0), fl, ptr(r.x_conv), ptr(r.y), ptr(r.gated),
                               new_conv, fptr(r.h_last), ptr(ws), B, T, W, nb, code, stream), "rglru_hip_block_fwd");
   }
+  if (rows.defined() && need_carry && K > 1)
+    check(rglru_hip_conv_carry(ptr(r.u), r.u.stride(1), ptr(r.state), static_cast<const int32_t*>(ptr(rows)), ptr(r.new_conv), B, T, W, K,
+                               code, stream), "rglru_hip_conv_carry");
   return r;
 }
 
@@ -728,13 +811,14 @@ struct BlockForward : torch::autograd::Function<BlockForward> {
   static variable_list forward(AutogradContext* ctx, const Tensor& u, const Tensor& v, const MaybeTensor& conv_state_,
                                const Tensor& weight, const MaybeTensor& bias_, const Tensor& segment_pos,
                                const MaybeTensor& flags_, bool first_reset, const Tensor& w_a, const Tensor& b_a,
-                               const Tensor& w_x, const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_, double c) {
-    Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_);
+                               const Tensor& w_x, const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_, double c,
+                               const MaybeTensor& rows_, bool need_carry) {
+    Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_), rows = opt(rows_);
     note_arguments(ctx, {true, true, conv_state.defined(), true, bias.defined(), true, flags.defined(), true, true, true, true,
                          true, h0.defined()});
     BlockResult r = block_forward_pass(u, v, conv_state, weight, bias, segment_pos, flags, first_reset, w_a, b_a, w_x, b_x, lam,
-                                       h0, c, Tensor(), true);
-    ctx->save_for_backward({r.u, r.v, r.state, r.taps, r.pos, r.x_conv, r.y, r.h0, r.flags, r.kept});
+                                       h0, c, Tensor(), rows, need_carry, true);
+    ctx->save_for_backward({r.u, r.v, r.state, r.taps, r.pos, r.x_conv, r.y, r.h0, r.flags, r.kept, rows});
     auto t = types_of(w_a, b_a, w_x, b_x, lam);
     pack(ctx, {first_reset, w_a.size(0), type_or_none(h0), (int64_t)t[0], (int64_t)t[1], (int64_t)t[2], (int64_t)t[3], (int64_t)t[4],
                type_or_none(conv_state), type_or_none(weight), type_or_none(bias)});
@@ -778,11 +862,11 @@ struct BlockForward : torch::autograd::Function<BlockForward> {
                          {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)}, need(12));
       if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
       conv = conv_backward(u.contiguous(), state, taps, pos, g.dx, {m[8], m[9], m[10]}, need_u, need(2), need(3),
-                           need(4), du_out);
+                           need(4), du_out, s[10]);
       if (!need_v) dv = Tensor();
     }
     return once({conv[0], dv, conv[1], conv[2], conv[3], Tensor(), Tensor(), Tensor(), g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam,
-                 g.dh0, Tensor()});
+                 g.dh0, Tensor(), Tensor(), Tensor()});
   }
 };
 
@@ -790,8 +874,8 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& 
                                                  const Tensor& weight, const MaybeTensor& bias_, const Tensor& segment_pos,
                                                  const MaybeTensor& flags_, bool first_reset, const Tensor& w_a, const Tensor& b_a,
                                                  const Tensor& w_x, const Tensor& b_x, const Tensor& lam, const MaybeTensor& h0_,
-                                                 double c, const MaybeTensor& image_) {
-  Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_);
+                                                 double c, const MaybeTensor& image_, const MaybeTensor& rows_, bool need_carry) {
+  Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_), rows = opt(rows_);
   require_gpu("hip_block_forward", {&u, &v, &conv_state, &weight, &bias, &segment_pos, &w_a, &b_a, &w_x, &b_x, &lam, &h0});
   TORCH_CHECK_VALUE(u.dim() == 3 && u.sizes() == v.sizes() && u.scalar_type() == v.scalar_type(),
                     "hip_block_forward expects two [batch, sequence, width] tensors of one dtype");
@@ -802,12 +886,12 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& 
                     "flags must be a contiguous uint8 tensor of shape [batch, sequence]");
   if (wants_grad({&u, &v, &conv_state, &weight, &bias, &w_a, &b_a, &w_x, &b_x, &lam, &h0})) {
     auto out = BlockForward::apply(u, v, maybe(conv_state), weight, maybe(bias), segment_pos, maybe(flags), first_reset, w_a,
-                                   b_a, w_x, b_x, lam, maybe(h0), c);
+                                   b_a, w_x, b_x, lam, maybe(h0), c, maybe(rows), need_carry);
     return {out[0], out[1], out[2]};
   }
   at::NoGradGuard no_grad;
   BlockResult r = block_forward_pass(u, v, conv_state, weight, bias, segment_pos, flags, first_reset, w_a, b_a, w_x, b_x, lam, h0, c,
-                                     opt(image_), false);
+                                     opt(image_), rows, need_carry, false);
   return {r.gated, r.h_last, r.new_conv};
 }
 
@@ -850,6 +934,49 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> block_decode_step(const Tensor& u_in,
   check(rglru_hip_step_gated(x, ptr(image), fptr(h_in), fptr(h_out), flags, ptr(v), v.stride(0), ptr(out), B, W, blocks, code, stream),
         "rglru_hip_step_gated");
   return {out, h_out, new_conv, new_pos};
+}
+
+// The whole single-token step of the block around the RG-LRU (griffin/griffin.py:459-528 with T == 1, no autograd) in three
+// launches: projections + positions + convolution, RG-LRU step + output gate, output projection.  Nothing is returned
+// where the kernels do not take the operands (mixed types, unaligned rows, many rows): the caller then goes through the
+// BLAS library.
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
+    const Tensor& x_in, const Tensor& w_x, const MaybeTensor& b_x_, const Tensor& w_y, const MaybeTensor& b_y_, const Tensor& conv_w,
+    const MaybeTensor& conv_b_, const Tensor& w_o, const MaybeTensor& b_o_, const MaybeTensor& conv_state_, const MaybeTensor& prev_pos_,
+    const MaybeTensor& segment_pos_, const MaybeTensor& active_, const Tensor& image, int64_t blocks, const MaybeTensor& rnn_state_) {
+  Tensor b_x = opt(b_x_), b_y = opt(b_y_), conv_b = opt(conv_b_), b_o = opt(b_o_), conv_state = opt(conv_state_),
+         prev_pos = opt(prev_pos_), segment_pos = opt(segment_pos_), active = opt(active_), rnn_state = opt(rnn_state_);
+  const auto dtype = x_in.scalar_type();
+  const int64_t B = x_in.size(0), D = x_in.size(2), W = w_x.size(0), K = conv_w.size(2);
+  if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || w_o.size(0) != D || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
+  for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state})
+    if (t->defined() && (t->scalar_type() != dtype || !t->is_contiguous() || !t->is_cuda())) return std::nullopt;
+  for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &w_y, &w_o})
+    if (!is_aligned(*t)) return std::nullopt;
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(x_in.device());
+  const int code = code_of(dtype);
+  Tensor x = x_in.select(1, 0);
+  if (x.stride(1) != 1 || (x.stride(0) * x.element_size()) % 16 || !is_aligned(x)) x = aligned(x);
+  Tensor h_in = rnn_state.defined() ? as(rnn_state, at::kFloat) : at::zeros({B, W}, x.options().dtype(at::kFloat));
+  Tensor h_out = fresh({B, W}, at::kFloat, x);
+  Tensor new_conv = fresh({B, K - 1, W}, dtype, x);
+  Tensor new_pos = fresh({B}, at::kLong, x);
+  Tensor out = fresh({B, 1, D}, dtype, x);
+  // x after the convolution, the second branch, their product with the state, one flag byte per row
+  const size_t row_bytes = round_up(B * W * x.element_size());
+  Tensor scratch = bytes(3 * row_bytes + B, x);
+  char* sp = static_cast<char*>(scratch.data_ptr());
+  uint8_t* flags = reinterpret_cast<uint8_t*>(sp + 3 * row_bytes);
+  void* stream = stream_of(x);
+  check(rglru_hip_decode_project(ptr(x), x.stride(0), ptr(w_x), ptr(b_x), ptr(w_y), ptr(b_y), ptr(conv_state), ptr(conv_w), ptr(conv_b),
+                                 iptr(prev_pos), iptr(segment_pos), bptr(active), sp, sp + row_bytes, K > 1 ? ptr(new_conv) : nullptr,
+                                 static_cast<int64_t*>(new_pos.data_ptr()), flags, B, D, W, K, code, stream), "rglru_hip_decode_project");
+  check(rglru_hip_step_gated(sp, ptr(image), fptr(h_in), fptr(h_out), flags, sp + row_bytes, W, sp + 2 * row_bytes, B, W, blocks, code,
+                             stream), "rglru_hip_step_gated");
+  check(rglru_hip_decode_linear(sp + 2 * row_bytes, W, ptr(w_o), ptr(b_o), bptr(active), ptr(out), B, D, W, code, stream),
+        "rglru_hip_decode_linear");
+  return std::make_tuple(out, h_out, new_conv, new_pos);
 }
 
 // ---- Linear layers of the block (griffin/griffin.py:379-389) ------------------------------------------------------
@@ -897,33 +1024,53 @@ std::tuple<Tensor, Tensor> linear_parameter_grads(const Tensor& x, at::ScalarTyp
   return {dw, db};
 }
 
+// src with the rows of inactive tokens zeroed, in a new tensor or in place.
+Tensor masked_rows(const Tensor& src_in, const Tensor& active, bool in_place) {
+  c10::DeviceGuard guard(src_in.device());
+  Tensor src = src_in.contiguous();
+  Tensor dst = in_place ? src : fresh_like(src);
+  const int64_t D = src.size(-1);
+  if (src.numel() > 0)
+    check(rglru_hip_mask_rows(ptr(src), bptr(active), ptr(dst), src.numel() / D, D, code_of(src.scalar_type()), stream_of(src)),
+          "rglru_hip_mask_rows");
+  return dst;
+}
+
+// `active` (one byte per token): outputs of inactive tokens are zero, and so are the gradients that reach them.
 struct Linear : torch::autograd::Function<Linear> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const MaybeTensor& bias) {
-    ctx->save_for_backward({x, weight});
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const MaybeTensor& bias, const MaybeTensor& active) {
+    ctx->save_for_backward({x, weight, opt(active)});
     note_arguments(ctx, {true, true, bias.has_value()});
     pack(ctx, {type_or_none(opt(bias))});
-    return at::linear(x, weight, bias);
+    Tensor y = at::linear(x, weight, bias);
+    return active.has_value() ? masked_rows(y, *active, true) : y;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     auto s = ctx->get_saved_variables();
     Tensor dx, dw, db;
     {
       at::NoGradGuard no_grad;
-      const Tensor &x = s[0], &weight = s[1], &dy = grads[0];
+      const Tensor &x = s[0], &weight = s[1];
+      Tensor dy = s[2].defined() ? masked_rows(grads[0], s[2], false) : grads[0];
       c10::DeviceGuard guard(x.device());
       Needs need(ctx);
       if (need(0)) dx = at::matmul(dy, weight.to(dy.scalar_type()));
       std::tie(dw, db) = linear_parameter_grads(x, weight.scalar_type(), dy, need(1), need(2) ? unpack(ctx)[0] : kNone);
     }
-    return once({dx, dw, db});
+    return once({dx, dw, db, Tensor()});
   }
 };
 
-Tensor linear(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_) {
+Tensor linear(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& active_) {
   Tensor bias = opt(bias_);
   require_gpu("hip_linear", {&x, &weight, &bias});
   code_of(x.scalar_type());
-  return Linear::apply(x, weight, maybe(bias));
+  MaybeTensor active;
+  if (active_.has_value()) {
+    TORCH_CHECK_VALUE(active_->numel() == x.numel() / x.size(-1) && active_->element_size() == 1, "active: one byte for each row of x");
+    active = active_->contiguous();
+  }
+  return Linear::apply(x, weight, maybe(bias), active);
 }
 
 // The [rows, 2 W] matrix whose column halves `a` and `b` ([..., W] each) are, or an undefined tensor if they are not
@@ -1070,12 +1217,22 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(rglru_steps);
   EXPORT(rglru_module_step);
   EXPORT(scan);
+  EXPORT(pack_flags);
+  py::class_<TokenFacts>(m, "TokenFacts")
+      .def(py::init<const Tensor&, const MaybeTensor&, const MaybeTensor&>())
+      .def("resolve", &TokenFacts::resolve)
+      .def_readonly("positions", &TokenFacts::positions)
+      .def_readonly("flags", &TokenFacts::flags)
+      .def_readonly("conv_positions", &TokenFacts::conv_positions)
+      .def_readonly("rows", &TokenFacts::rows)
+      .def_readonly("last_position", &TokenFacts::last_position);
   EXPORT(causal_conv);
   EXPORT(causal_conv_padded);
   EXPORT(gelu_gate);
   EXPORT(block_flags);
   EXPORT(block_forward);
   EXPORT(block_decode_step);
+  EXPORT(block_step);
   EXPORT(sum_sets);
   EXPORT(stacked_halves);
   EXPORT(linear);

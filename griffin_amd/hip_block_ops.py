@@ -8,6 +8,8 @@ There is no CPU fallback here: the operator raises when the library or a GPU is 
 
 from __future__ import annotations
 
+from functools import lru_cache
+
 import torch
 from torch import Tensor
 
@@ -16,6 +18,7 @@ from . import _lib
 from .hip_scan import FIRST_TOKEN_RESET, _DTYPE_CODES, _dtype_code, _ptr, _stream_ptr
 
 
+@lru_cache(maxsize=None)
 def max_kernel_size() -> int:
     """Largest convolution kernel size the HIP kernels cover."""
     return int(_lib.load().rglru_hip_conv_max_kernel_size())
@@ -58,6 +61,7 @@ def hip_gelu_gate(h: Tensor, v: Tensor) -> Tensor:
     return _lib.native().gelu_gate(h, v)
 
 
+@lru_cache(maxsize=None)
 def hip_block_forward_covers(width: int, blocks: int, taps_count: int, dtype: torch.dtype) -> bool:
     """Whether ``hip_block_forward`` has a kernel for this shape (rglru_hip_block_fwd_path)."""
     if dtype not in _DTYPE_CODES or blocks <= 0 or width % blocks:
@@ -74,21 +78,23 @@ def hip_block_flags(segment_pos: Tensor) -> Tensor:
 
 def hip_block_forward(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: Tensor, bias: Tensor | None,
                       segment_pos: Tensor, flags: Tensor | None, w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor,
-                      lam: Tensor, h0: Tensor | None, c: float = 8.0, prep=None):
+                      lam: Tensor, h0: Tensor | None, c: float = 8.0, prep=None, rows: Tensor | None = None, need_state: bool = True):
     """``gelu_tanh(v) * RG_LRU(conv(u))`` for whole sequences with every token active, one forward launch.
 
     ``u``, ``v`` [B, T, W]: the block's two projections; ``conv_state`` [B, K-1, W] or None; ``weight``
     [W, 1, K], ``bias`` [W] of the depthwise ``nn.Conv1d`` (K <= 4); ``segment_pos`` [B, T]; ``flags``:
     ``hip_block_flags(segment_pos)`` if the caller has it already, ``hip_scan.FIRST_TOKEN_RESET`` when the
     positions are 0 .. T-1 in every row (no flag tensor is needed then), else None; the five RG-LRU parameters, ``h0`` [B, W] or None; ``prep``: a prepared parameter image to use
-    when no gradient is asked for.  Returns ``(gated [B, T, W], final state [B, W] fp32, new_conv_state
+    when no gradient is asked for.  For right-padded batches ``rows``, ``segment_pos`` and ``flags`` are the rows,
+    conv_positions and flags of ``token_facts``; the new convolution state then carries no gradient and is computed only
+    if ``need_state``.  Returns ``(gated [B, T, W], final state [B, W] fp32, new_conv_state
     [B, K-1, W])``; differentiable in u, v, the parameters, conv_state and h0.
     """
     first_reset = flags is FIRST_TOKEN_RESET
     gated, h_last, new_conv = _lib.native().block_forward(
         u, v, conv_state, weight, bias, segment_pos, None if first_reset else flags, first_reset, w_a, b_a, w_x, b_x, lam, h0,
-        c, None if prep is None else prep.image)
-    if torch.is_grad_enabled() and (u.requires_grad or (conv_state is not None and conv_state.requires_grad)):
+        c, None if prep is None else prep.image, rows, need_state)
+    if rows is None and torch.is_grad_enabled() and (u.requires_grad or (conv_state is not None and conv_state.requires_grad)):
         # the carried rows as a differentiable function of u and conv_state (the kernel's copy carries no gradient)
         history, steps = weight.size(2) - 1, u.size(1)
         if steps >= history:
@@ -114,6 +120,17 @@ def hip_block_decode_step(u: Tensor, v: Tensor, conv_state: Tensor | None, weigh
                                            prep.width, prep.blocks, prep.dtype, rnn_state)
 
 
+def hip_block_step(x: Tensor, linear_x, linear_y, conv, linear_out, conv_state: Tensor | None, prev_pos: Tensor | None,
+                   segment_pos: Tensor | None, active: Tensor | None, prep, rnn_state: Tensor | None):
+    """The block on one token per row, ``x`` [B, 1, D] (no autograd), in three launches: both projections with positions and
+    convolution, the RG-LRU step with the output gate, the output projection.  The four layers are those of the block, the
+    other arguments as for ``hip_block_decode_step``.  Returns ``(output [B, 1, D], rnn_state, conv_state, positions)``,
+    or None where the kernels do not take the operands."""
+    return _lib.native().block_step(x, linear_x.weight, linear_x.bias, linear_y.weight, linear_y.bias, conv.weight, conv.bias,
+                                    linear_out.weight, linear_out.bias, conv_state, prev_pos, segment_pos, active, prep.image,
+                                    prep.blocks, rnn_state)
+
+
 def _sum_sets(sets: Tensor) -> Tensor:
     """``sets.sum(0)`` for a contiguous [sets, ...] tensor on the GPU by a kernel of the library (one pass over the
     sets, 16-byte accesses; the generic reduction takes about three times as long for eight sets of a weight
@@ -129,10 +146,19 @@ def _stacked_halves(a: Tensor | None, b: Tensor | None) -> Tensor | None:
     return _lib.native().stacked_halves(a, b)
 
 
-def hip_linear(x: Tensor, weight: Tensor, bias: Tensor | None) -> Tensor:
+def hip_linear(x: Tensor, weight: Tensor, bias: Tensor | None, active: Tensor | None = None) -> Tensor:
     """``x @ weight.T + bias`` (griffin/griffin.py:379-389, the block's Linear layers) with the bias
-    gradient reduced by a kernel of this library; differentiable in all three arguments."""
-    return _lib.native().linear(x, weight, bias)
+    gradient reduced by a kernel of this library; differentiable in all three arguments.  ``active`` [...]: a mask of
+    the rows; those where it is False come out as zeros (griffin/griffin.py:522-523)."""
+    return _lib.native().linear(x, weight, bias, active)
+
+
+def token_facts(active_mask: Tensor, segment_pos: Tensor | None, previous_position: Tensor | None):
+    """What an activity mask [B, T] says about every token, in one launch: an object with ``positions`` [B, T] (given, or
+    previous + running count of active tokens), ``flags`` / ``conv_positions`` / ``rows`` for ``hip_block_forward``,
+    ``last_position`` [B], and ``resolve() -> (every token is active, every row is right-padded)``, which waits for that
+    launch but not for work queued behind it."""
+    return _lib.native().TokenFacts(active_mask, segment_pos, previous_position)
 
 
 def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None) -> tuple[Tensor, Tensor]:
@@ -141,6 +167,7 @@ def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Te
     return _lib.native().linear_pair(x, w1, b1, w2, b2)
 
 
+@lru_cache(maxsize=None)
 def rmsnorm_max_width(dtype: torch.dtype, aligned: bool = True) -> int:
     return int(_lib.load().rglru_hip_rmsnorm_max_width(_dtype_code(dtype), 1 if aligned else 0))
 

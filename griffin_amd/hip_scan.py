@@ -119,6 +119,8 @@ def pack_flags(reset_mask: Tensor | None, active_mask: Tensor | None) -> Tensor 
                 _PACKED_FLAGS.clear()
             _PACKED_FLAGS[id(reset_mask)] = (weakref.ref(reset_mask), reset_mask._version, flags)
         return flags
+    if active_mask is not None and active_mask.is_cuda and (reset_mask is None or reset_mask.is_cuda):
+        return _lib.native().pack_flags(reset_mask, active_mask)
     flags = None
     if reset_mask is not None:
         flags = reset_mask.to(torch.uint8)

@@ -158,9 +158,10 @@ class RG_LRU(nn.Module):
         batch, steps, width = xt.shape
         if width != self.rnn_width:
             raise ValueError(f"Expected width {self.rnn_width}, got {width}")
-        for name, mask in (("reset_mask", reset_mask), ("active_mask", active_mask)):
-            if mask is not None and mask.shape != (batch, steps):
-                raise ValueError(f"{name} must have shape ({batch}, {steps}), got {tuple(mask.shape)}")
+        if reset_mask is not None or active_mask is not None:
+            for name, mask in (("reset_mask", reset_mask), ("active_mask", active_mask)):
+                if mask is not None and mask.shape != (batch, steps):
+                    raise ValueError(f"{name} must have shape ({batch}, {steps}), got {tuple(mask.shape)}")
         if ht_minus_1 is not None and ht_minus_1.shape != (batch, width):
             raise ValueError(f"ht_minus_1 must have shape ({batch}, {width}), got {tuple(ht_minus_1.shape)}")
         state_dtype = torch.float32 if xt.dtype in (torch.float16, torch.bfloat16) else xt.dtype
@@ -397,11 +398,12 @@ class RecurrentBlock(nn.Module):
                 return False
         if self.linear_x.weight.dtype != x.dtype or self.linear_y.weight.dtype != x.dtype:
             return False
-        mode = self.rg_lru.scan_mode
-        if mode == "auto":
-            probe = x.new_empty(x.size(0), 1, self.rnn_width)
-            return self._hip_block_ops_covers(probe)
-        return mode in ("hip", "fused") and self.conv_kernel_size <= hip_block_ops.max_kernel_size()
+        rg_lru = self.rg_lru
+        if self.conv_kernel_size > hip_block_ops.max_kernel_size():
+            return False
+        if rg_lru.scan_mode == "auto":
+            return rg_lru.recurrence_gate.block_width <= 512 and hip_scan.hip_scan_is_usable(x.device)
+        return rg_lru.scan_mode in ("hip", "fused")
 
     def _hip_decode(self, x: Tensor, cache: RecurrentBlockCache | None, segment_pos: Tensor | None,
                     active_mask: Tensor | None, return_cache: bool):
@@ -427,6 +429,12 @@ class RecurrentBlock(nn.Module):
         active = None
         if active_mask is not None and not bool(active_mask.all()):
             active = active_mask[:, 0].to(torch.uint8).contiguous()
+        if not torch.is_autocast_enabled() and self._is_plain(self.linear_out):
+            done = hip_block_ops.hip_block_step(x, self.linear_x, self.linear_y, self.temporal_conv, self.linear_out, conv_state,
+                                                prev_pos, segment_pos, active, self.rg_lru._prepared(x.dtype, x.device), rnn_state)
+            if done is not None:
+                output, *state = done
+                return (output, RecurrentBlockCache(*state)) if return_cache else output
         projected, gate_input = self._decode_projections(x[:, 0])
         prep = self.rg_lru._prepared(projected.dtype, projected.device)
         gated, new_rnn_state, new_conv_state, new_pos = hip_block_ops.hip_block_decode_step(
@@ -472,6 +480,11 @@ class RecurrentBlock(nn.Module):
                 and self.rg_lru.scan_mode in ("hip", "fused", "auto") and x.numel() > 0
                 and (self.rg_lru.scan_mode != "auto" or hip_scan.hip_scan_is_usable(x.device)))
 
+    @staticmethod
+    def _is_plain(layer: nn.Module) -> bool:
+        """Nobody wrapped or hooked the Linear layer: calling it is a product with its weight and nothing else."""
+        return type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks
+
     def _dense_conv(self, projected: Tensor, conv_state: Tensor | None, segment_pos: Tensor, need_state: bool = True):
         """All-tokens-active path (griffin/griffin.py:476-487): taps are masked per document."""
         if self._hip_block_ops_covers(projected):
@@ -516,8 +529,14 @@ class RecurrentBlock(nn.Module):
         previous_position = None if cache is None else cache.segment_position
         if steps == 1 and self._hip_decode_covers(x, cache):
             return self._hip_decode(x, cache, segment_pos, active_mask, return_cache)
-        segment_pos = _resolve_segment_positions(
-            x, segment_pos, previous_position, None if everything_active else active_mask)
+        facts = None
+        if not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
+            # launched in front of the projections, so that its answer is there before they are done
+            facts = hip_block_ops.token_facts(active_mask, segment_pos, previous_position)
+            segment_pos = facts.positions
+        else:
+            segment_pos = _resolve_segment_positions(
+                x, segment_pos, previous_position, None if everything_active else active_mask)
 
         if self._linear_on_hip(self.linear_x, x) and self._linear_on_hip(self.linear_y, x):
             projected, gate_input = hip_block_ops.hip_linear_pair(
@@ -530,9 +549,14 @@ class RecurrentBlock(nn.Module):
         conv_state = (None if on_hip else self._empty_conv_state(projected)) if cache is None else cache.conv_state
         if conv_state is not None and conv_state.shape != (batch, self.conv_kernel_size - 1, self.rnn_width):
             raise ValueError("Recurrent convolution cache has an incompatible shape")
-        dense = everything_active or bool(active_mask.all())
+        right_padded = False
+        if facts is not None:
+            dense, right_padded = facts.resolve()
+        else:
+            dense = everything_active or bool(active_mask.all())
+        padded_launch = right_padded and not dense and on_hip and self._hip_block_forward_covers(projected, gate_input, cache)
         default = _DEFAULT_POSITIONS.get((batch, steps, x.device))
-        if dense and on_hip and self._hip_block_forward_covers(projected, gate_input, cache):
+        if padded_launch or (dense and on_hip and self._hip_block_forward_covers(projected, gate_input, cache)):
             # convolution, RG-LRU and output gate in one forward launch
             rnn_state = None if cache is None else cache.rnn_state
             needs_grad = torch.is_grad_enabled() and any(
@@ -540,10 +564,13 @@ class RecurrentBlock(nn.Module):
                 for t in (projected, gate_input, conv_state, rnn_state, self.temporal_conv.weight,
                           self.temporal_conv.bias, *self.rg_lru._gate_parameters()))
             gated, new_rnn_state, new_conv_state = hip_block_ops.hip_block_forward(
-                projected, gate_input, conv_state, self.temporal_conv.weight, self.temporal_conv.bias, segment_pos,
+                projected, gate_input, conv_state, self.temporal_conv.weight, self.temporal_conv.bias,
+                facts.conv_positions if padded_launch else segment_pos,
+                facts.flags if padded_launch else
                 hip_scan.FIRST_TOKEN_RESET if (cache is None and default is not None and segment_pos is default[0]) else None,
                 *self.rg_lru._gate_parameters(), rnn_state, self.rg_lru.c,
-                None if needs_grad else self.rg_lru._prepared(projected.dtype, projected.device))
+                None if needs_grad else self.rg_lru._prepared(projected.dtype, projected.device),
+                facts.rows if padded_launch else None, return_cache)
         else:
             if dense:
                 recurrent_in, new_conv_state = self._dense_conv(projected, conv_state, segment_pos, return_cache)
@@ -560,11 +587,17 @@ class RecurrentBlock(nn.Module):
                 gated = hip_block_ops.hip_gelu_gate(recurrent_out, gate_input)
             else:
                 gated = recurrent_out * F.gelu(gate_input, approximate="tanh")
-        output = self._linear(self.linear_out, gated)
-        if not everything_active:
-            output = output.masked_fill(~active_mask.unsqueeze(-1), 0.0)
+        if (facts is not None and not dense and gated.dtype in hip_scan.SUPPORTED_DTYPES and not torch.is_autocast_enabled()
+                and (self._linear_on_hip(self.linear_out, gated) or self._is_plain(self.linear_out))):
+            output = hip_block_ops.hip_linear(gated, self.linear_out.weight, self.linear_out.bias, active_mask)
+        else:
+            output = self._linear(self.linear_out, gated)
+            if not everything_active and not (facts is not None and dense):
+                output = output.masked_fill(~active_mask.unsqueeze(-1), 0.0)
         if return_cache:
-            if everything_active:
+            if facts is not None:
+                last_position = facts.last_position
+            elif everything_active:
                 last_position = segment_pos[:, -1].clone()   # every token is active: the last one's position
             else:
                 last_position = _last_active_position(segment_pos, active_mask, previous_position)

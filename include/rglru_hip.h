@@ -51,7 +51,7 @@
 extern "C" {
 #endif
 
-#define RGLRU_ABI_VERSION 19
+#define RGLRU_ABI_VERSION 20
 
 enum { RGLRU_F32 = 0, RGLRU_BF16 = 1 };
 
@@ -244,6 +244,30 @@ int rglru_hip_step(const void* x, const void* prep, float* h, const uint8_t* fla
 int rglru_hip_steps(const void* x, const void* prep, float* h, const uint8_t* flags, void* y,
                     int64_t K, int64_t B, int64_t W, int64_t nb, int dtype, void* stream);
 
+/* What an activity mask says about every token (griffin/griffin.py:309-358, :459-510), one launch.  active[B,T]: one byte per
+ * token; segment_pos[B,T] or NULL: then a token's position is prev_pos[b] (NULL: -1) plus the number of active tokens up to
+ * it.  Writes pos[B,T] (NULL to skip); flags[B,T] as rglru_hip_block_fwd takes them (reset at position 0, inactive, lags
+ * that reach in front of the document as the padded convolution counts them); conv_pos[B,T] (NULL to skip): the position
+ * rglru_hip_conv_rows_bwd needs, tokens since the document start or unbounded where none lies in this call; rows[3 B]: active
+ * tokens of the row, ordinal of its last document start (-1: none), 1 where its active tokens are its first ones;
+ * last_pos[B] (NULL to skip): position of the row's last active token, or prev_pos; host_facts[B] (NULL to skip; may be
+ * memory of the host): bit 0 = every token of the row is active, bit 1 = rows' third word. */
+int rglru_hip_token_facts(const uint8_t* active, const int64_t* segment_pos, const int64_t* prev_pos, int64_t* pos, uint8_t* flags,
+                          int64_t* conv_pos, int32_t* rows, int64_t* last_pos, uint32_t* host_facts, int64_t B, int64_t T,
+                          void* stream);
+
+/* RGLRU_FLAG_* bytes of n tokens from the masks of RG_LRU.forward (one byte per token, either may be NULL). */
+int rglru_hip_pack_flags(const uint8_t* reset, const uint8_t* active, uint8_t* flags, int64_t n, void* stream);
+
+/* dst[r, :] = active[r] ? src[r, :] : 0 over rows of D elements (griffin/griffin.py:522-523).  With dst == src only the rows
+ * that become zero are written. */
+int rglru_hip_mask_rows(const void* src, const uint8_t* active, void* dst, int64_t rows, int64_t D, int dtype, void* stream);
+
+/* The carried rows new_state[B,K-1,W] of the padded convolution (griffin/griffin.py:488-510) for rows whose active tokens are
+ * their first ones; `rows` from rglru_hip_token_facts. */
+int rglru_hip_conv_carry(const void* u, int64_t u_stride, const void* state, const int32_t* rows, void* new_state, int64_t B, int64_t T,
+                         int64_t W, int64_t K, int dtype, void* stream);
+
 /* Causal depthwise temporal convolution that feeds the RG-LRU inside the recurrent block, all
  * tokens active (griffin/griffin.py:474-487):
  *   out[b,t,c] = bias[c] + sum_{lag<K} taps[c][K-1-lag] * [segment_pos[b,t] >= lag] * padded[b,t-lag,c]
@@ -269,6 +293,12 @@ int rglru_hip_conv_bwd(const void* u, const void* state, const void* taps, const
                        const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
                        int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
                        void* stream);
+/* The same for right-padded batches: `rows` from rglru_hip_token_facts (every row's third word must be 1), segment_pos its
+ * conv_pos.  The gradient at a padded output is not read, that of a padded input is zero.  rows NULL: rglru_hip_conv_bwd. */
+int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
+                            const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
+                            int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
+                            void* stream);
 
 /* The same convolution over right-padded batches (griffin/griffin.py:488-510): tokens with
  * active[b,t] == 0 produce zeros and never enter the window of the K-1 previous ACTIVE inputs; an
@@ -352,12 +382,30 @@ int rglru_hip_step_gated(const void* x, const void* prep, const float* h_in, flo
                          const void* v, int64_t v_stride, void* out, int64_t B, int64_t W, int64_t nb, int dtype,
                          void* stream);
 
+/* Linear layer of a few rows (griffin/griffin.py:379-389 with one token per row): y[B, N] = x[B, K] w[N, K]^T + bias, fp32
+ * accumulation.  `x_stride`: elements between rows of x; w contiguous; bias in the storage type or NULL; `active` (one byte
+ * per row, or NULL): rows with a zero byte are written as zeros.  Rows of x and w must start on 16-byte boundaries.
+ * Made for up to a few hundred rows: latency, not throughput. */
+int rglru_hip_decode_linear(const void* x, int64_t x_stride, const void* w, const void* bias, const uint8_t* active, void* y,
+                            int64_t B, int64_t N, int64_t K, int dtype, void* stream);
+
+/* Both input projections of a single-token step and everything in front of the RG-LRU step, one launch:
+ * u = x w_x^T + b_x, v = x w_y^T + b_y ([B, W] each, x [B, D]), then what rglru_hip_decode_prepare does with u (same arguments
+ * and meaning; the taps, their bias and the carried rows are in the storage type here).  u itself is not written. */
+int rglru_hip_decode_project(const void* x, int64_t x_stride, const void* w_x, const void* b_x, const void* w_y, const void* b_y,
+                             const void* conv_state, const void* taps, const void* conv_bias, const int64_t* prev_pos,
+                             const int64_t* segment_pos, const uint8_t* active, void* x_conv, void* v, void* new_conv_state,
+                             int64_t* new_pos, uint8_t* flags, int64_t B, int64_t D, int64_t W, int64_t K, int dtype,
+                             void* stream);
+
+
 /* The recurrent block's forward between its projections in ONE launch (griffin/griffin.py:474-487, the
  * RG-LRU of :97-286, and :464, :520): x = causal depthwise convolution of u[B,T,W] (taps[W][K], K <= 4,
  * conv_bias[W] or NULL, both in vec_dtype; conv_state[B,K-1,W] or NULL = zeros in front of every row),
  * y = RG-LRU(x) and gated[B,T,W] = y * gelu_tanh(v[B,T,W]).  u and v may be rows of wider buffers
- * (u_stride, v_stride in elements, 0 = W).  Every token is active; the flag bytes carry, next to
- * RGLRU_FLAG_RESET, in bits 2-3 how many convolution lags reach in front of the token's document,
+ * (u_stride, v_stride in elements, 0 = W).  The flag bytes carry, next to
+ * RGLRU_FLAG_RESET and RGLRU_FLAG_INACTIVE (x_conv is zero there; only for rows whose active tokens are their first
+ * ones), in bits 2-3 how many convolution lags reach in front of the token's document,
  * 3 - min(segment_pos, 3) (rglru_hip_block_flags writes them from segment_pos[n]); flags NULL means no
  * document starts inside the rows and position >= K - 1 or an all-zero history at their beginning.
  * Optional outputs (NULL to skip): x_conv[B,T,W] and y[B,T,W] (what a backward pass needs),

@@ -747,3 +747,162 @@ def test_block_forward_argument_errors():
     assert lib.rglru_hip_block_fwd(*unaligned) != 0 and b"aligned" in lib.rglru_hip_last_error()
     wide = list(args); wide[20] = 640
     assert lib.rglru_hip_block_fwd(*wide) != 0
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 1e-2)])
+@pytest.mark.parametrize("rows,features,outputs", [(1, 8, 1), (16, 40, 17), (17, 104, 33), (33, 64, 16), (70, 1000, 2064), (129, 72, 4100)])
+def test_decode_linear_matches_fp64(rows, features, outputs, dtype, tol):
+    """The projections of a decode step at the edges of their tiles: row tiles of 16 to 64, column tiles of 16 and 32, a
+    contraction that ends inside a step, rows of a wider buffer, rows that do not take part."""
+    from griffin_amd import _lib
+    from griffin_amd.hip_block_ops import _dtype_code, _ptr, _stream_ptr
+
+    print("decode linear", rows, features, outputs, dtype, flush=True)
+    torch.manual_seed(rows)
+    wide = torch.randn(rows, features + 8, device="cuda", dtype=dtype)
+    x = wide[:, :features]
+    w = torch.randn(outputs, features, device="cuda", dtype=dtype) / features ** 0.5
+    bias = torch.randn(outputs, device="cuda", dtype=dtype)
+    active = (torch.arange(rows, device="cuda") % 3 != 1).to(torch.uint8)
+    y = torch.empty(rows, outputs, device="cuda", dtype=dtype)
+    _lib.check(_lib.load().rglru_hip_decode_linear(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), _ptr(active), _ptr(y), rows,
+                                                   outputs, features, _dtype_code(dtype), _stream_ptr(x.device)), "decode_linear")
+    want = (x.double() @ w.double().t() + bias.double()) * active.double()[:, None]
+    assert ((y.double() - want).norm() / want.norm()).item() < tol
+    assert torch.count_nonzero(y[active == 0]).item() == 0
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2e-2)])
+@pytest.mark.parametrize("batch,dim,width,blocks,taps", [(1, 64, 128, 2, 4), (16, 40, 96, 3, 3), (17, 96, 160, 1, 2), (70, 72, 136, 2, 4), (130, 64, 64, 2, 1)])
+def test_block_step_matches_the_library_route(batch, dim, width, blocks, taps, dtype, tol):
+    """One token per row through the three launches of ``hip_block_step`` against the same block with the projections of
+    the BLAS library and ``hip_block_decode_step`` (itself checked against the oracle), with inactive rows, document
+    starts and a cache, and without any of them."""
+    from griffin_amd import RecurrentBlock, RecurrentBlockCache, hip_block_ops
+
+    print("block step", batch, dim, width, blocks, taps, dtype, flush=True)
+    torch.manual_seed(batch)
+    block = RecurrentBlock(dim, width, conv_kernel_size=taps, gate_blocks=blocks, scan_mode="hip").cuda().to(dtype).eval()
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            if name.endswith("bias"):
+                p.normal_(std=0.3)
+        block.temporal_conv.weight.normal_(std=0.5)
+        x = torch.randn(batch, 1, dim, device="cuda", dtype=dtype)
+        cache = RecurrentBlockCache(torch.randn(batch, width, device="cuda"),
+                                    torch.randn(batch, taps - 1, width, device="cuda", dtype=dtype),
+                                    torch.arange(batch, device="cuda") % 5 - 1)
+        active = (torch.arange(batch, device="cuda") % 4 != 2)[:, None]
+        positions = (torch.arange(batch, device="cuda") % 3)[:, None]
+        calls = [dict(), dict(cache=cache), dict(cache=cache, segment_pos=positions)]
+        if batch > 2:
+            calls += [dict(cache=cache, active_mask=active), dict(cache=cache, segment_pos=positions, active_mask=active)]
+        real = hip_block_ops.hip_block_step
+        for call in calls:
+            got, got_cache = block(x, return_cache=True, **call)
+            hip_block_ops.hip_block_step = lambda *args: None
+            try:
+                want, want_cache = block(x, return_cache=True, **call)
+            finally:
+                hip_block_ops.hip_block_step = real
+            assert rel_err(got.float(), want.float()) < tol
+            assert rel_err(got_cache.rnn_state, want_cache.rnn_state) < tol
+            assert torch.equal(got_cache.segment_position, want_cache.segment_position)
+            if taps > 1:
+                assert rel_err(got_cache.conv_state.float(), want_cache.conv_state.float()) < tol
+
+
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 7), (2, 64), (4, 2047), (2, 2048), (3, 4100)])
+@pytest.mark.parametrize("given,carried", [(False, False), (False, True), (True, True)])
+def test_token_facts_match_the_elementwise_formulas(B, T, given, carried):
+    """Positions, flag bytes, convolution positions, row words and last positions of one launch against the running counts
+    they stand for, on rows that are whole, right-padded, empty and full of holes, over more than one pass of the kernel."""
+    from griffin_amd.hip_block_ops import token_facts
+
+    g = torch.Generator().manual_seed(B * 10000 + T)
+    active = torch.rand(B, T, generator=g) < 0.7
+    for b in range(B):
+        if b % 4 == 1:
+            active[b] = torch.arange(T) < max(T // 3, 1)
+        elif b % 4 == 2:
+            active[b] = False
+        elif b % 4 == 3:
+            active[b] = True
+    prev = torch.randint(-1, 5, (B,), generator=g) if carried else None
+    pos = torch.randint(0, 4, (B, T), generator=g) if given else None
+    facts = token_facts(active.cuda(), None if pos is None else pos.cuda(), None if prev is None else prev.cuda())
+    everything, prefix = facts.resolve()
+    start = torch.full((B,), -1) if prev is None else prev
+    want_pos = pos if given else start[:, None] + active.long().cumsum(1)
+    assert torch.equal(facts.positions.cpu(), want_pos)
+    want_last, rows = [], facts.rows.cpu()
+    flags, conv = facts.flags.cpu(), facts.conv_positions.cpu()
+    prefixes = []
+    for b in range(B):
+        order, doc, last = 0, -1, int(start[b])
+        for t in range(T):
+            a, p = bool(active[b, t]), int(want_pos[b, t])
+            if a and p == 0:
+                doc = order
+            f = int(flags[b, t])
+            assert (f & 1) == (p == 0) and ((f >> 1) & 1) == (not a)
+            if a:
+                hidden = 0 if doc < 0 else 3 - min(order - doc, 3)
+                assert (f >> 2) == hidden, (b, t)
+                assert int(conv[b, t]) == (1 << 30 if doc < 0 else order - doc)
+                last = p
+                order += 1
+        want_last.append(last)
+        prefixes.append(bool(active[b, :order].all()))
+        assert rows[:, b].tolist() == [order, doc, int(prefixes[-1])]
+    assert facts.last_position.tolist() == want_last
+    assert everything == bool(active.all()) and prefix == all(prefixes)
+
+
+@pytest.mark.parametrize("cfg", [(3, 70, 64, 128, 2, 4), (2, 129, 96, 256, 8, 3), (4, 64, 64, 192, 3, 2), (5, 33, 64, 64, 2, 1)])
+@pytest.mark.parametrize("packed,carried", [(False, False), (True, False), (False, True), (True, True)])
+def test_right_padded_block_in_one_launch_matches_the_separate_kernels(cfg, packed, carried):
+    """A right-padded bf16 batch through the one-launch forward (flags with padding, row table in the backward convolution)
+    against convolution, RG-LRU and gate as kernels of their own: output, cache and every gradient."""
+    from griffin_amd import RecurrentBlock, RecurrentBlockCache
+
+    B, T, D, W, blocks, taps = cfg
+    print("padded block", cfg, packed, carried, flush=True)
+    torch.manual_seed(T)
+    block = RecurrentBlock(D, W, conv_kernel_size=taps, gate_blocks=blocks, scan_mode="hip").cuda().bfloat16()
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            if name.endswith("bias"):
+                p.normal_(std=0.2)
+        block.temporal_conv.weight.normal_(std=0.5)
+    x = torch.randn(B, T, D, device="cuda").bfloat16().requires_grad_(True)
+    dy = torch.randn(B, T, D, device="cuda").bfloat16()
+    lengths = torch.tensor([T, 1, T // 2, 0, T - 1][:B], device="cuda")
+    token = torch.arange(T, device="cuda")
+    active = token[None] < lengths[:, None]
+    positions = (token[None] + 3 * torch.arange(B, device="cuda")[:, None]) % 19 if packed else None
+    cache = None
+    leaves = [x, *block.parameters()]
+    if carried:
+        cache = RecurrentBlockCache(torch.randn(B, W, device="cuda").requires_grad_(True),
+                                    torch.randn(B, taps - 1, W, device="cuda").bfloat16().requires_grad_(True),
+                                    torch.arange(B, device="cuda") + 1)
+        leaves += [cache.rnn_state] + ([cache.conv_state] if taps > 1 else [])
+    results = []
+    for covers in (True, False):
+        real = block._hip_block_forward_covers
+        if not covers:
+            block._hip_block_forward_covers = lambda *args: False
+        try:
+            out, new = block(x, cache, positions, active_mask=active, return_cache=True)
+        finally:
+            block._hip_block_forward_covers = real
+        results.append((out, new, torch.autograd.grad(out, leaves, dy)))
+    (a, na, ga), (b, nb, gb) = results
+    assert torch.count_nonzero(a[~active]).item() == 0
+    assert rel_err(a.float(), b.float()) < 1e-2
+    assert rel_err(na.rnn_state, nb.rnn_state) < 1e-2 and torch.equal(na.segment_position, nb.segment_position)
+    if taps > 1:
+        assert torch.equal(na.conv_state, nb.conv_state)
+    for i, (p, q) in enumerate(zip(ga, gb)):
+        assert rel_err(p.float(), q.float()) < BF16_TOL, i
