@@ -88,7 +88,7 @@ __global__ __launch_bounds__(kThreads) void step_kernel(FusedArgs p) {
   }
 }
 
-// Decode step for 16-bit storage and gate blocks of 32 to 384 channels in steps of 32, on 16 x 16 MFMA tiles: a wave
+// Decode step for 16-bit storage and gate blocks of 16 to 384 channels in steps of 16, on 16 x 16 MFMA tiles: a wave
 // owns 16 sequences x 16 channels, a lane 4 sequences of one channel.  The step is a chain of latencies
 // (launch, loads, products, gate math, stores), so the work is cut as fine as the matrix unit allows:
 // four elements of gate math per lane instead of sixteen, 8 KB of weights per wave instead of 16, x rows
@@ -115,7 +115,8 @@ __global__ __launch_bounds__(kThreads) void step16_kernel(FusedArgs p) {
   const IO* xr = (const IO*)p.x + (arow_ok ? arow : 0) * W + k * p.bw + 8 * q;
   Frag xa[NKS], fa[NKS], fx[NKS];
 #pragma unroll
-  for (int ks = 0; ks < NKS; ++ks) xa[ks] = *reinterpret_cast<const Frag*>(xr + 32 * ks);   // a row past the end reads row 0: its products are not used
+  for (int ks = 0; ks < NKS; ++ks)                         // a row past the end reads row 0: its products are not used
+    xa[ks] = *reinterpret_cast<const Frag*>(xr + (32 * ks + 8 * q < p.bw ? 32 * ks : 0));
   // B fragments: column n is output channel o, same K elements: rows of the two weight matrices
   const IO* wa = (const IO*)p.wg + ((long long)(0 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
   const IO* wx = (const IO*)p.wg + ((long long)(1 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
@@ -153,6 +154,8 @@ __global__ __launch_bounds__(kThreads) void step16_kernel(FusedArgs p) {
     gate[v] = (float)gate_raw[v];
     fls[v] = p.flags ? (unsigned)fl_raw[v] : 0u;
   }
+  // a block of an odd multiple of 16 channels ends inside the last K step: what was read in its place does not count
+  if (32 * (NKS - 1) + 8 * q >= p.bw) xa[NKS - 1] = Io<IO>::zero();
   f32x4v ua = {bias_a, bias_a, bias_a, bias_a}, ux = {bias_x, bias_x, bias_x, bias_x};
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks) {
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void steps16_kernel(FusedArgs p) {
     const long long tt = t < steps ? t : 0;                // a step past the end re-reads step 0
     const long long base = tt * step_elems;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + 32 * ks);
+    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + (32 * ks + 8 * q < p.bw ? 32 * ks : 0));
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       s.xv[v] = ((const IO*)p.x)[base + at[v]];
@@ -249,6 +252,7 @@ __global__ __launch_bounds__(kThreads) void steps16_kernel(FusedArgs p) {
     }
   };
   auto step = [&](In& s, int t) {
+    if (32 * (NKS - 1) + 8 * q >= p.bw) s.xa[NKS - 1] = Io<IO>::zero();      // see step16_kernel
     f32x4v ua = {bias_a, bias_a, bias_a, bias_a}, ux = {bias_x, bias_x, bias_x, bias_x};
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) {

@@ -123,15 +123,16 @@ RGLRU_DEVICE void wave_lds_fence() {
 }
 
 // Store a staged ROWS x 32 tile of 16-bit values: `r` covers the tile's rows (row stride
-// row_bytes), col_bytes is the byte offset of the wave's first channel inside a row.
+// row_bytes), col_bytes is the byte offset of the wave's first channel inside a row.  seg_ok: the lane's eight channels
+// belong to the block (a block that does not fill its last slab).
 template <int ROWS>
-RGLRU_DEVICE void stage_flush(const unsigned char* stage, rsrc_t r, unsigned row_bytes, unsigned col_bytes, int lane) {
+RGLRU_DEVICE void stage_flush(const unsigned char* stage, rsrc_t r, unsigned row_bytes, unsigned col_bytes, int lane, bool seg_ok = true) {
 #pragma unroll
   for (int i = 0; i < ROWS / 16; ++i) {
     const int row = 16 * i + (lane >> 2);
     const unsigned seg = (unsigned)(lane & 3) * 16u;
     i32x4 v = *reinterpret_cast<const i32x4*>(stage + WaveStage<ROWS>::row_offset(row) + seg);
-    buf_store_b128(v, r, (unsigned)row * row_bytes + col_bytes + seg);
+    buf_store_b128(v, r, seg_ok ? (unsigned)row * row_bytes + col_bytes + seg : kOutOfRange);
   }
 }
 

@@ -25,6 +25,7 @@ struct PrepArgs {
   void* wg; float* bias; float* sp; float* cs; float* dsp; void* w2t;
   int W, nb, bw, bwp, Wp, vec_dtype;
   int vec_ok;                          // 16-bit weights, unpadded blocks, 16-byte aligned: eight elements per thread
+  int rows_ok;                         // 16-bit weights whose rows are whole 16-byte vectors (blocks of a multiple of 8 channels)
   float c;
   uint4* clear; long long clear_n;     // optional: a workspace region to zero in the same launch
 };
@@ -217,7 +218,7 @@ RGLRU_DEVICE WaveId wave_identity(const FusedArgs& p, int block, bool scalar_wav
     w.slab = w.wave - blk * p.S;
     w.slab_ok = k < p.nb;
     w.k = w.slab_ok ? k : p.nb - 1;
-    w.tile_col = w.unit * p.bpu * p.bw; w.kb = blk * p.bw;
+    w.tile_col = w.unit * p.bpu * p.bw; w.kb = blk * p.bwp;
   } else {
     w.k = w.unit / p.groups;
     w.slab = (w.unit % p.groups) * kWaves + w.wave;
@@ -229,6 +230,15 @@ RGLRU_DEVICE WaveId wave_identity(const FusedArgs& p, int block, bool scalar_wav
   w.ch = w.k * p.bw + (w.ch_ok ? w.o : 0);
   w.kp = w.k * p.bwp + (w.slab_ok ? w.o : 0);
   return w;
+}
+
+// Channel behind column `col` of a unit's 128-wide tile, or -1.  Blocks take bwp columns of it each (their width rounded up
+// to whole 32-channel slabs); the columns a block does not fill hold zeros, and nothing is stored for them.
+template <bool PAD>
+RGLRU_DEVICE int tile_channel(const FusedArgs& p, int unit, int tile_col, int col) {
+  if constexpr (!PAD) return tile_col + col;
+  const int blk = col / p.bwp, c = col - blk * p.bwp, k = unit * p.bpu + blk;
+  return c < p.bw && blk < p.bpu && k < p.nb ? k * p.bw + c : -1;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -443,11 +453,22 @@ inline int held_groups(const Geometry& g, int dtype, int aligned) {
   return 0;
 }
 
-// K steps of 32 channels of the decode kernels on 16 x 16 tiles (gate blocks of 32 .. 384 channels in steps
-// of 32, 16-bit storage, aligned rows), or 0 for the portable decode kernels
+// K groups of the kernels for narrow blocks with register-held weights (2, 4, 6, 8: slabs of 32 channels), or 0.  A block
+// of any multiple of 8 channels up to 128 takes them, padded to whole slabs in LDS and registers (`padded`): per element
+// they are two to four times as fast as the portable kernels, which stream the weights and finish the gradients in GEMM
+// kernels of their own, and what padding wastes is at most a slab (RG-LRU forward + backward, B3 T1537 W768 with 48-wide
+// blocks: see narrow blocks in rglru_fused_bwd.hip).
+inline int narrow_groups(const Geometry& g, int dtype, int aligned) {
+  return dtype == RGLRU_BF16 && aligned && g.bw % 8 == 0 && g.bwp <= 128 ? (int)(g.bwp / 16) : 0;
+}
+// ... and whether it is the padded variant (96-wide blocks have no other: three slabs leave the unit's fourth wave idle)
+inline bool narrow_padded(const Geometry& g) { return g.bw != g.bwp || g.bwp == 96; }
+
+// K steps of 32 channels of the decode kernels on 16 x 16 tiles (gate blocks of 16 .. 384 channels in steps
+// of 16, 16-bit storage, aligned rows), or 0 for the portable decode kernels
 inline int step16_groups(const Geometry& g, int dtype, int aligned) {
-  if (dtype != RGLRU_BF16 || !aligned || g.bw != g.bwp || g.bw > 384) return 0;
-  return (int)(g.bw / 32);
+  if (dtype != RGLRU_BF16 || !aligned || g.bw % 16 || g.bw > 384) return 0;
+  return (int)(g.bwp / 32);
 }
 
 // ... and for the blocks wider than a workgroup's four slabs whose weights the forward and the
@@ -500,7 +521,7 @@ struct KernelTimer {
 // Narrow blocks of the kernels with register-held weights share a unit (see kPackedWidth).
 inline void pack_units(FusedArgs& a, const Geometry& g, int nkg) {
   if (nkg == 4 || nkg == 2) {
-    a.bpu = kPackedWidth / (int)g.bw;
+    a.bpu = kPackedWidth / (int)g.bwp;
     a.units = (int)((g.nb + a.bpu - 1) / a.bpu);
   }
 }
@@ -538,7 +559,7 @@ inline int pick_queues(long long B, int wg) {
 // Whether the forward runs one workgroup per chain (fwd_chain_kernel) instead of tiles with look-back:
 // 0 = by shape, 1 = never, 2 = whenever that kernel covers the shape (tests).
 inline std::atomic<int> g_chain_forward{0};
-inline bool fwd_chain_pays(int64_t B, int64_t T, int64_t W) {
+inline bool fwd_chain_pays(int64_t B, int64_t T, int64_t W) {    // W: channels with the padding of their blocks
   const int mode = g_chain_forward.load(std::memory_order_relaxed);
   if (mode == 1) return false;
   if (mode == 2) return true;

@@ -79,7 +79,7 @@ RGLRU_DEVICE void fwd_local(const FusedArgs& p, const WaveId& w, FwdTile<MT>& t,
 }
 
 // Stage 2: carry in, carry out and checkpoint, then the recurrence itself and the stores.
-template <typename IO, int MT, bool MASKED, bool STAGED, bool BLOCK = false>
+template <typename IO, int MT, bool MASKED, bool STAGED, bool BLOCK = false, bool PAD = false>
 RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTile<MT>& t, unsigned char* stage,
                                const CarryBatch<kFwdDepth>* first = nullptr, bool live = true,
                                const bf16x8* gate_rows = nullptr) {
@@ -131,6 +131,7 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
       if ((e & 15) == 15) BufIo<float>::store(h, rck, ck_off[e >> 4], 0u);
     }
     wave_lds_fence();
+    const bool seg_ok = !PAD || w.slab * 32 + (w.lane & 3) * 8 < p.bw;
     if constexpr (BLOCK) {
       // output gate at the store: a lane holds the same 8 channels of a row of y and of the gate input
       const rsrc_t rg = make_rsrc((const IO*)p.gated + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
@@ -140,7 +141,7 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
         const int row = 16 * i + (w.lane >> 2);
         const unsigned seg = (unsigned)(w.lane & 3) * 16u;
         const i32x4 raw = *reinterpret_cast<const i32x4*>(stage + WaveStage<TR>::row_offset(row) + seg);
-        const unsigned off = (unsigned)row * row_bytes + col_bytes + seg;
+        const unsigned off = seg_ok ? (unsigned)row * row_bytes + col_bytes + seg : kOutOfRange;
         buf_store_b128(raw, ry, off);                       // y itself: dropped unless the caller keeps it
         const bf16x8 hv = __builtin_bit_cast(bf16x8, raw);
         bf16x8 out;
@@ -149,7 +150,7 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
         buf_store_b128(__builtin_bit_cast(i32x4, out), rg, off);
       }
     } else {
-      stage_flush<TR>(stage, ry, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane);
+      stage_flush<TR>(stage, ry, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane, seg_ok);
     }
     wave_lds_fence();
   } else {
@@ -196,10 +197,12 @@ constexpr int fwd_lds_groups(int nkg, bool masked) {
 // consecutive rows of eight channels plus the three rows in front of them, convolves them (taps by lag
 // from LDS, lags masked per token through bits 2-3 of the flag bytes = 3 - min(position, 3)) and puts the
 // result where the plain kernel puts x; the store stage multiplies by gelu_tanh of the second projection.
-template <typename IO, int NKG, bool MASKED, bool BLOCK = false>
+// PAD: blocks of up to 128 channels that do not fill their slabs (see narrow_groups); masked variant only.
+template <typename IO, int NKG, bool MASKED, bool BLOCK = false, bool PAD = false>
 __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : (NKG == 4 || NKG == 2) ? RGLRU_NARROW_OCC : NKG > 8 ? fwd_wide_occ(NKG) : 2)) void fwd_kernel(FusedArgs p) {
   constexpr int MT = fwd_mt(NKG), TR = 32 * MT, EL = 16 * MT;
-  static_assert(!BLOCK || (sizeof(IO) == 2 && (NKG == 8 || NKG == 4 || NKG == 2)), "block forward: 16-bit storage, register-held weights");
+  static_assert(!BLOCK || (sizeof(IO) == 2 && (NKG == 8 || NKG == 6 || NKG == 4 || NKG == 2)), "block forward: 16-bit storage, register-held weights");
+  static_assert(!PAD || MASKED, "padded blocks run the masked variant");
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
   // NKG > 0: gate weights held in registers, pre-activations on MFMA.  Up to NKG = 8 (128 channels) a
@@ -224,9 +227,9 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
   if constexpr (BLOCK) {
     // read after the barrier that follows the first ticket
     for (int i = tid; i < 5 * KC; i += kThreads) {
-      const int j = i / KC, ch = w.tile_col + (i - j * KC);
+      const int j = i / KC, ch = tile_channel<PAD>(p, w.unit, w.tile_col, i - j * KC);
       float v = 0.f;
-      if (ch < p.W) {
+      if (ch >= 0 && ch < p.W) {
         if (j == 4) { if (p.conv_bias) v = p.conv_vec_dtype == RGLRU_BF16 ? (float)((const __bf16*)p.conv_bias)[ch] : ((const float*)p.conv_bias)[ch]; }
         else if (j < p.conv_k) {
           const long long at = (long long)ch * p.conv_k + (p.conv_k - 1 - j);     // the tap of lag j
@@ -271,8 +274,9 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
     static_assert(!BLOCK || (NV == 4 && VPR == 16), "block forward: four rows of a 128-channel tile per lane");
     const int rho = tid / VPR, bcv = tid - rho * VPR;
     const unsigned x_row_bytes = BLOCK ? (unsigned)p.ld_x * (unsigned)sizeof(IO) : row_bytes;
-    const bool bcol_ok = BLOCK && (x_col + bcv * Tr::HW < p.W);
-    const unsigned bcol_bytes = (unsigned)(x_col + bcv * Tr::HW) * (unsigned)sizeof(IO);
+    const int bcol = tile_channel<PAD>(p, w.unit, x_col, bcv * Tr::HW);
+    const bool bcol_ok = BLOCK && bcol >= 0 && bcol < p.W;
+    const unsigned bcol_bytes = (unsigned)(bcol_ok ? bcol : 0) * (unsigned)sizeof(IO);
     Frag halo[BLOCK ? 3 : 1];
     unsigned conv_fl = 0u;                               // flag bytes of the lane's four rows
 #pragma unroll
@@ -281,9 +285,10 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
       const int row = idx / VPR, cv = idx - row * VPR;
       if constexpr (BLOCK)
         pre_off[i] = bcol_ok ? (unsigned)(4 * rho + i + 3) * x_row_bytes + bcol_bytes : kOutOfRange;
-      else
-      pre_off[i] = (idx < TR * VPR) ? (unsigned)row * row_bytes + (unsigned)(x_col + cv * Tr::HW) * (unsigned)sizeof(IO)
-                                    : kOutOfRange;
+      else {
+        const int col = tile_channel<PAD>(p, w.unit, x_col, cv * Tr::HW);
+        pre_off[i] = (idx < TR * VPR && col >= 0) ? (unsigned)row * row_bytes + (unsigned)col * (unsigned)sizeof(IO) : kOutOfRange;
+      }
       if constexpr (GIVEN)
         u_off[i] = (idx < TR * VPR) ? (unsigned)row * u_row_bytes + (unsigned)(group_col + cv * Tr::HW) * (unsigned)sizeof(IO)
                                     : kOutOfRange;
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
 #pragma unroll
       for (int i = 0; i < TR / 16; ++i) gate_rows[i] = Io<__bf16>::zero();
     }
-    fwd_finalize<IO, MT, MASKED, sizeof(IO) == 2, BLOCK>(p, w, cur, stage, nullptr, false, gate_rows);
+    fwd_finalize<IO, MT, MASKED, sizeof(IO) == 2, BLOCK, PAD>(p, w, cur, stage, nullptr, false, gate_rows);
     while (tk < q.tiles) {
       cur.c = (int)((unsigned)tk / (unsigned)q.n_b);
       cur.b = q.first_b + (int)((unsigned)tk - (unsigned)cur.c * (unsigned)q.n_b) * p.queues;
@@ -479,7 +484,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
                                                    (unsigned)(w.k * p.bw + w.slab * 32) * 2u + (unsigned)(w.lane & 3) * 16u);
       }
       issue(tk_next);
-      fwd_finalize<IO, MT, MASKED, sizeof(IO) == 2, BLOCK>(p, w, cur, stage, &ahead, slab_ok, gate_rows);
+      fwd_finalize<IO, MT, MASKED, sizeof(IO) == 2, BLOCK, PAD>(p, w, cur, stage, &ahead, slab_ok, gate_rows);
       tk = tk_next;
     }
   } else {
@@ -532,13 +537,15 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
 // ------------------------------------------------------------------------------------------
 // PREP: the launch also does what prepare_kernel does (the parameter image for the backward kernels, the zeroed
 // workspace region) and takes its own weights, biases and decay constants straight from the caller's parameters.
-template <typename IO, int NKG, bool MASKED, bool PREP = false>
+// PAD: blocks that do not fill their slabs; the columns and channels past the block's width hold zeros and store nothing.
+template <typename IO, int NKG, bool MASKED, bool PREP = false, bool PAD = false>
 __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
-  static_assert(sizeof(IO) == 2 && (NKG == 8 || NKG == 4 || NKG == 2), "16-bit storage, gate blocks of 128, 64 or 32 channels");
+  static_assert(sizeof(IO) == 2 && (NKG == 8 || NKG == 6 || NKG == 4 || NKG == 2), "16-bit storage, gate blocks of one to four slabs");
   constexpr int TR = 32;
   constexpr int KC = NKG * Tr::KG;                         // block width = K range of the gate products
+  const int bw = PAD ? p.bw : KC;                          // ... of which so many channels exist
   constexpr int S = KC / 32;                               // slabs (chains) per block
   constexpr int LDSROW = KC + Tr::HW;
   constexpr int VPR = KC / Tr::HW;                         // 16-byte vectors per tile row
@@ -560,8 +567,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
   // wait for all memory operations into every hand-off).
   for (int i = tid; i < kChainWaves * 32; i += kChainWaves * 64) {
     unsigned long long entry = 0ull;
-    if (i >= (kChainWaves - 1) * 32 && chain_ok && p.h0)
-      entry = (unsigned long long)__float_as_uint(p.h0[(long long)b * p.W + k * KC + sl * 32 + (i - (kChainWaves - 1) * 32)]) << 32;
+    const int o = sl * 32 + i - (kChainWaves - 1) * 32;
+    if (i >= (kChainWaves - 1) * 32 && chain_ok && p.h0 && o < bw)
+      entry = (unsigned long long)__float_as_uint(p.h0[(long long)b * p.W + k * bw + o]) << 32;
     (&carry[0][0])[i] = entry;
   }
   // The chain kernels use no carry records and no tickets: all this pass needs from the workspace is a failure word
@@ -571,9 +579,10 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
   {
     for (int i = tid; i < 2 * 32 * VPR; i += kChainWaves * 64) {
       const int gate = i / (32 * VPR), o = (i / VPR) % 32, cv = i % VPR;
-      const IO* wg = PREP ? (const IO*)(gate ? p.prep.w_x : p.prep.w_a) + ((long long)k * p.bwp + sl * 32 + o) * p.bwp
+      const IO* wg = PREP ? (const IO*)(gate ? p.prep.w_x : p.prep.w_a) + ((long long)k * bw + sl * 32 + o) * bw
                           : (const IO*)p.wg + ((long long)(gate * p.nb + k) * p.bwp + sl * 32 + o) * p.bwp;
-      *reinterpret_cast<Frag*>(lds_w + (gate * 32 + o) * LDSROW + cv * Tr::HW) = *reinterpret_cast<const Frag*>(wg + cv * Tr::HW);
+      const bool there = !PAD || !PREP || (sl * 32 + o < bw && cv * Tr::HW < bw);      // the image is padded with zeros itself
+      *reinterpret_cast<Frag*>(lds_w + (gate * 32 + o) * LDSROW + cv * Tr::HW) = there ? *reinterpret_cast<const Frag*>(wg + cv * Tr::HW) : Tr::zero();
     }
   }
   __syncthreads();
@@ -599,8 +608,10 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
       if (tid < 32) prepare_channel(p.prep, k * p.bwp + sl * 32 + tid);
     }
   }
-  const int col0 = k * KC;                                 // first channel of the block
-  const int ch = col0 + sl * 32 + r;                       // the lane's channel
+  const int col0 = k * bw;                                 // first channel of the block
+  const bool ch_ok = !PAD || sl * 32 + r < bw;
+  const int ch = col0 + (ch_ok ? sl * 32 + r : 0);         // the lane's channel
+  const bool seg_ok = !PAD || sl * 32 + (lane & 3) * 8 < bw;   // ... and the eight it stores
   const long long W = p.W;
   IO* lds = lds_all[wave];
   unsigned char* stage = reinterpret_cast<unsigned char*>(lds);
@@ -610,8 +621,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
     nbx = -kLog2e * load_vec(p.prep.b_x, ch, p.prep.vec_dtype);
     sp = p.prep.c * log_sigmoid(load_vec(p.prep.lambda, ch, p.prep.vec_dtype)) * kLog2e;
   } else {
-    nba = -kLog2e * p.bias[ch]; nbx = -kLog2e * p.bias[p.Wp + ch];
-    sp = p.sp[ch];
+    const int kp = k * KC + sl * 32 + r;
+    nba = -kLog2e * p.bias[kp]; nbx = -kLog2e * p.bias[p.Wp + kp];
+    sp = p.sp[kp];
   }
   const int nC = (p.T + TR - 1) / TR;
   const unsigned row_bytes = (unsigned)p.W * 2u;
@@ -622,7 +634,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int idx = lane + 64 * i, row = idx / VPR, cv = idx - row * VPR;
-    pre_off[i] = (unsigned)row * row_bytes + (unsigned)(col0 + cv * Tr::HW) * 2u;
+    pre_off[i] = !PAD || cv * Tr::HW < bw ? (unsigned)row * row_bytes + (unsigned)(col0 + cv * Tr::HW) * 2u : kOutOfRange;
   }
   const IO* xb = (const IO*)p.x + (long long)b * p.T * W;
   auto issue = [&](int c) {                                // a tile past the end: empty extent, nothing is fetched
@@ -702,7 +714,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
     const float h_mid = fmaf(A_lo, h_in, H_lo);
     if (hf == 0) __hip_atomic_store(&carry[wave][r], ((unsigned long long)__float_as_uint(h_end) << 32) | (unsigned long long)(unsigned)(c + 1),
                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    BufIo<float>::store(h_end, rhl, (hf == 0 && c == nC - 1) ? ((unsigned)b * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
+    BufIo<float>::store(h_end, rhl, (hf == 0 && c == nC - 1 && ch_ok) ? ((unsigned)b * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
 
     float h = hf ? h_mid : h_in;
     const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
@@ -715,9 +727,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
       *reinterpret_cast<IO*>(my + e * WaveStage<TR>::kRowBytes) = (IO)h;
     }
     // checkpoint for the backward pass: the state after the lane's 16 tokens (slot = token / 16)
-    BufIo<float>::store(h, rck, ((unsigned)(2 * c + hf) * (unsigned)W + (unsigned)ch) * 4u, 0u);
+    BufIo<float>::store(h, rck, ch_ok ? ((unsigned)(2 * c + hf) * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
     wave_lds_fence();
-    stage_flush<TR>(stage, ry, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane);
+    stage_flush<TR>(stage, ry, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane, seg_ok);
     wave_lds_fence();
   }
   if (gave_up && lane == 0) atomicOr(p.fail, 1u);
@@ -778,6 +790,7 @@ static int build_prep_args(const void* w_a, const void* b_a, const void* w_x, co
   a.clear = (uint4*)clear; a.clear_n = (long long)(clear_bytes / 16);
   a.vec_ok = dtype == RGLRU_BF16 && g.bw == g.bwp && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0 &&
              (uintptr_t)a.wg % 16 == 0 && (uintptr_t)a.w2t % 16 == 0;
+  a.rows_ok = dtype == RGLRU_BF16 && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0;
   return RGLRU_OK;
 }
 
@@ -816,8 +829,7 @@ int rglru_hip_wide_path(int64_t W, int64_t nb, int dtype);
 
 int rglru_hip_block_fwd_path(int64_t W, int64_t nb, int64_t K, int dtype) {
   if (dtype != RGLRU_BF16 || W <= 0 || nb <= 0 || W % nb || K < 1 || K > 4) return 0;
-  const int64_t bw = W / nb;
-  return (bw == 32 || bw == 64 || bw == 128) ? 1 : 0;
+  return narrow_groups(make_geometry(W, nb), dtype, 1) ? 1 : 0;
 }
 
 size_t rglru_hip_bwd_scratch_bytes(int64_t B, int64_t T, int64_t W, int64_t nb, int dtype) {
@@ -860,7 +872,8 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   a.ticket = (unsigned*)(wb + L.f_ticket); a.fail = (unsigned*)(wb + L.fail);
   a.B = (int)B; a.T = (int)T; a.nC = (int)L.nC; a.ckpt_nC = 2 * (int)L.nC;
   a.aligned = is_aligned(x, W, g.bw, elem_size(dtype)) && ((uintptr_t)y % 16 == 0);
-  int nkg = held_groups(g, dtype, a.aligned);
+  int nkg = narrow_groups(g, dtype, a.aligned);
+  const bool narrow = nkg != 0, pad = narrow && narrow_padded(g);
   if (!nkg && !pre) nkg = wide_groups(g, dtype, a.aligned);
   if (pre) {
     if (!rglru_hip_pre_path(W, nb, dtype)) return fail(RGLRU_E_UNSUPPORTED, "fwd_pre: needs bf16 storage and gate blocks of a multiple of 32 channels");
@@ -873,7 +886,7 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   if (blk) {
     const int64_t xs = blk->x_stride ? blk->x_stride : W, vs = blk->v_stride ? blk->v_stride : W;
     if (!rglru_hip_block_fwd_path(W, nb, blk->K, dtype))
-      return fail(RGLRU_E_UNSUPPORTED, "block_fwd: needs bf16 storage, gate blocks of 32, 64 or 128 channels and 1 to 4 taps");
+      return fail(RGLRU_E_UNSUPPORTED, "block_fwd: needs bf16 storage, gate blocks of up to 128 channels (a multiple of 8) and 1 to 4 taps");
     if (blk->vec_dtype != RGLRU_F32 && blk->vec_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "block_fwd: unknown vector dtype %d", blk->vec_dtype);
     if (!blk->v || !blk->taps || !blk->gated) return fail(RGLRU_E_ARG, "block_fwd: null pointer");
     if (xs < W || vs < W) return fail(RGLRU_E_ARG, "block_fwd: a row stride is smaller than the width %lld", (long long)W);
@@ -889,7 +902,7 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   }
   // The tiled kernels need the forward records, tickets and failure word zeroed; the chain kernel needs the
   // failure word only and clears it itself.  (Every backward entry point that uses records clears its own.)
-  const bool chain = !blk && !pre && (nkg == 8 || nkg == 4 || nkg == 2) && fwd_chain_pays(B, T, W);
+  const bool chain = !blk && !pre && narrow && fwd_chain_pays(B, T, g.Wp);
   if (!cleared && !chain) {
     rc = launch_clear(wb, L.f_begin, L.f_end, s);
     if (rc) return rc;
@@ -897,7 +910,7 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   // fuse: the parameter conversion (and, for the tiled kernels, the clearing of the workspace region it names)
   // still has to happen.  The chain kernel converts by itself when the caller's weights can be read as 16-byte
   // vectors; else one launch first.
-  const bool fused_prepare = fuse && chain && fuse->vec_ok;
+  const bool fused_prepare = fuse && chain && fuse->rows_ok;
   if (fuse && !fused_prepare) {
     PrepArgs pa = *fuse;
     if (chain) { pa.clear = nullptr; pa.clear_n = 0; }
@@ -905,7 +918,7 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     if (rc) return rc;
   }
   if (chain) {
-    const int S = (int)(g.bw / 32);
+    const int S = (int)g.S;
     const dim3 grid((unsigned)(8 * ((B * nb + 7) / 8) * S));
     const int masked = (flags != nullptr) || (T % 32 != 0);
     if (fused_prepare) a.prep = *fuse;
@@ -915,6 +928,16 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     if (nkg == N) {                                                                                                    \
       if (fused_prepare) { if (masked) RGLRU_CHAIN_LAUNCH(N, true, true); else RGLRU_CHAIN_LAUNCH(N, false, true); }   \
       else { if (masked) RGLRU_CHAIN_LAUNCH(N, true, false); else RGLRU_CHAIN_LAUNCH(N, false, false); }               \
+    }
+    if (pad) {
+#define RGLRU_CHAIN_PAD(N)                                                                                             \
+      if (nkg == N) {                                                                                                  \
+        if (fused_prepare) hipLaunchKernelGGL((fwd_chain_kernel<__bf16, N, true, true, true>), grid, dim3(kChainWaves * 64), 0, s, a); \
+        else hipLaunchKernelGGL((fwd_chain_kernel<__bf16, N, true, false, true>), grid, dim3(kChainWaves * 64), 0, s, a); \
+      }
+      RGLRU_CHAIN_PAD(8) RGLRU_CHAIN_PAD(6) RGLRU_CHAIN_PAD(4) RGLRU_CHAIN_PAD(2)
+#undef RGLRU_CHAIN_PAD
+      return check_launch("fwd");
     }
     RGLRU_CHAIN_CASE(8) RGLRU_CHAIN_CASE(4) RGLRU_CHAIN_CASE(2)
 #undef RGLRU_CHAIN_CASE
@@ -937,7 +960,15 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     // the plain kernels with register-held weights of up to 128 channels know first_reset; the others take it
     // through the flag logic of their masked variant
     const int masked = (flags != nullptr) || (T % tile_tokens != 0) || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
-    if (blk) {
+    if (pad) {
+#define RGLRU_PAD_CASE(N)                                                                                              \
+      if (nkg == N) {                                                                                                  \
+        if (blk) hipLaunchKernelGGL((fwd_kernel<__bf16, N, true, true, true>), grid, dim3(kThreads), 0, s, a);         \
+        else hipLaunchKernelGGL((fwd_kernel<__bf16, N, true, false, true>), grid, dim3(kThreads), 0, s, a);            \
+      }
+      RGLRU_PAD_CASE(8) RGLRU_PAD_CASE(6) RGLRU_PAD_CASE(4) RGLRU_PAD_CASE(2)
+#undef RGLRU_PAD_CASE
+    } else if (blk) {
 #define RGLRU_BLOCK_CASE(N)                                                                                            \
       if (nkg == N) {                                                                                                  \
         if (masked) hipLaunchKernelGGL((fwd_kernel<__bf16, N, true, true>), grid, dim3(kThreads), 0, s, a);            \

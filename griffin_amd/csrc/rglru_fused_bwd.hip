@@ -534,7 +534,8 @@ constexpr int kDeltaDepth = RGLRU_DELTA_DEPTH;         // records a walk of the 
 #ifndef RGLRU_DELTA_OCC
 #define RGLRU_DELTA_OCC 2
 #endif
-template <typename IO, int NKG, bool MASKED, int MT>
+// PAD, in this kernel and the two behind it: blocks that do not fill their slabs (see narrow_groups), masked variant only.
+template <typename IO, int NKG, bool MASKED, int MT, bool PAD = false>
 __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd_delta_kernel(FusedArgs p) {
   constexpr int TR = 32 * MT, EL = 16 * MT;
   typedef Io<IO> Tr;
@@ -573,8 +574,10 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
   for (int i = 0; i < NV; ++i) {
     const int idx = tid + i * kThreads;
     const int row = idx / VPR, cv = idx - row * VPR;
-    pre_off[i] = (idx < TR * VPR) ? (unsigned)row * row_bytes + (unsigned)(w.tile_col + cv * Tr::HW) * 2u : kOutOfRange;
+    const int col = tile_channel<PAD>(p, w.unit, w.tile_col, cv * Tr::HW);
+    pre_off[i] = (idx < TR * VPR && col >= 0) ? (unsigned)row * row_bytes + (unsigned)col * 2u : kOutOfRange;
   }
+  const bool ch_ok = !PAD || w.ch_ok;
   auto decode = [&](unsigned tk, int& c, int& b) {
     const unsigned cr = tk / (unsigned)q.n_b;
     c = nCk - 1 - (int)cr;
@@ -660,12 +663,12 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     CarryChain chain;
     chain.rec = p.rec_a + (long long)b * p.nC * W + w.ch; chain.stride = W;
     const bool last_chunk = c == nCk - 1;
-    if (!last_chunk && hf == 0) carry_publish(chain, c, A_t, D_t, false);
-    float d_in = (last_chunk && p.dh_last) ? p.dh_last[(long long)b * W + w.ch] : 0.f;
-    if (!last_chunk) d_in = carry_lookback<kDeltaDepth>(chain, c, +1, nCk, 0.f, true, p.limit, p.fail);
+    if (!last_chunk && hf == 0 && ch_ok) carry_publish(chain, c, A_t, D_t, false);
+    float d_in = (last_chunk && p.dh_last && ch_ok) ? p.dh_last[(long long)b * W + w.ch] : 0.f;
+    if (!last_chunk) d_in = carry_lookback<kDeltaDepth>(chain, c, +1, nCk, 0.f, ch_ok, p.limit, p.fail);
     const float d_out = fmaf(A_t, d_in, D_t);
-    if (hf == 0) carry_publish(chain, c, 0.f, d_out, true);
-    if (hf == 0 && c == 0 && p.dh0) p.dh0[(long long)b * W + w.ch] = d_out;
+    if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
+    if (hf == 0 && c == 0 && p.dh0 && ch_ok) p.dh0[(long long)b * W + w.ch] = d_out;
 
     // delta of every token, through the wave's staging area, as 16-byte row segments
     carry = hf ? d_in : fmaf(A_hi, d_in, D_hi);
@@ -680,7 +683,7 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     {
       const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
       const rsrc_t rd = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane);
+      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane, !PAD || w.slab * 32 + (w.lane & 3) * 8 < p.bw);
     }
     wave_lds_fence();
     tk = tk_next;
@@ -691,13 +694,14 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
 // chain's 32-token tiles round robin from the last tile to the first, the recurrence gate's rows of the slab
 // sit in LDS, and the carry goes from tile c + 1 to tile c through LDS.  A wave stages its own x tile (the
 // block's K range) and its own 32 channels of dy; delta leaves through the x tile's area.
-template <typename IO, int NKG, bool MASKED>
+template <typename IO, int NKG, bool MASKED, bool PAD = false>
 __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(FusedArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
-  static_assert(sizeof(IO) == 2 && (NKG == 8 || NKG == 4 || NKG == 2), "16-bit storage, gate blocks of 128, 64 or 32 channels");
+  static_assert(sizeof(IO) == 2 && (NKG == 8 || NKG == 6 || NKG == 4 || NKG == 2), "16-bit storage, gate blocks of one to four slabs");
   constexpr int TR = 32;
   constexpr int KC = NKG * Tr::KG;
+  const int bw = PAD ? p.bw : KC;                          // channels of the block that exist
   constexpr int S = KC / 32;
   constexpr int LDSROW = KC + Tr::HW;
   constexpr int VPR = KC / Tr::HW;
@@ -725,14 +729,16 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
   }
   __syncthreads();
   if (!chain_ok) return;
-  const int col0 = k * KC;
-  const int ch = col0 + sl * 32 + r;
+  const int col0 = k * bw;
+  const bool ch_ok = !PAD || sl * 32 + r < bw;
+  const int ch = col0 + (ch_ok ? sl * 32 + r : 0), kp = k * KC + sl * 32 + r;
+  const bool seg_ok = !PAD || sl * 32 + (lane & 3) * 8 < bw;
   const long long W = p.W;
   IO* lds = lds_all[wave];
   IO* lds_dy = lds;                                        // dy takes the x tile's place once the gate products have read it
   unsigned char* stage = reinterpret_cast<unsigned char*>(lds);
-  const float nba = -kLog2e * p.bias[ch];
-  const float sp = p.sp[ch];
+  const float nba = -kLog2e * p.bias[kp];
+  const float sp = p.sp[kp];
   const int nC = (p.T + TR - 1) / TR;
   const unsigned row_bytes = (unsigned)p.W * 2u;
   const long long limit = p.limit < 0 ? -p.limit : p.limit;
@@ -742,12 +748,12 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int idx = lane + 64 * i, row = idx / VPR, cv = idx - row * VPR;
-    pre_off[i] = (unsigned)row * row_bytes + (unsigned)(col0 + cv * Tr::HW) * 2u;
+    pre_off[i] = !PAD || cv * Tr::HW < bw ? (unsigned)row * row_bytes + (unsigned)(col0 + cv * Tr::HW) * 2u : kOutOfRange;
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {                            // 32 rows x four 16-byte vectors
     const int idx = lane + 64 * i, row = idx >> 2, cv = idx & 3;
-    dy_off[i] = (unsigned)row * row_bytes + (unsigned)(col0 + sl * 32 + cv * Tr::HW) * 2u;
+    dy_off[i] = !PAD || sl * 32 + cv * Tr::HW < bw ? (unsigned)row * row_bytes + (unsigned)(col0 + sl * 32 + cv * Tr::HW) * 2u : kOutOfRange;
   }
   const IO* xb = (const IO*)p.x + (long long)b * p.T * W;
   const IO* dyb = (const IO*)p.dy + (long long)b * p.T * W;
@@ -765,7 +771,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
   const int next_wave = (wave + kChainWaves - 1) % kChainWaves;    // the wave of tile c + 1
   bool gave_up = false;
   // carry into the chain's last tile (used by its wave only): no memory operation inside the loop is conditional
-  const float d_first = p.dh_last ? p.dh_last[(long long)b * W + ch] : 0.f;
+  const float d_first = p.dh_last && ch_ok ? p.dh_last[(long long)b * W + ch] : 0.f;
   issue(nC - 1 - wave);
   {
     // the stores the loop's back edge has in flight behind the prefetched tiles (dh0, two delta segments),
@@ -841,7 +847,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
     const float d_out = fmaf(A_t, d_in, D_t);
     if (hf == 0) __hip_atomic_store(&carry[wave][r], ((unsigned long long)__float_as_uint(d_out) << 32) | (unsigned long long)(unsigned)(c + 1),
                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    BufIo<float>::store(d_out, rh0, (hf == 0 && c == 0) ? ((unsigned)b * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
+    BufIo<float>::store(d_out, rh0, (hf == 0 && c == 0 && ch_ok) ? ((unsigned)b * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
 
     // delta of every token, through the x tile's area, as 16-byte row segments
     run = hf ? d_in : fmaf(A_hi, d_in, D_hi);
@@ -857,7 +863,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
     {
       const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
       const rsrc_t rd = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane);
+      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane, seg_ok);
     }
     wave_lds_fence();
   }
@@ -885,7 +891,7 @@ constexpr int kGradThreads = 64 * kGradWaves;
 // each SIMD overlaps the two; neither role needs more than 256 registers (weights in one, weight
 // gradient accumulators in the other).  Exchange buffers and the x tile are double-buffered: one
 // barrier per tile.
-template <typename IO, int NKG, bool MASKED>
+template <typename IO, int NKG, bool MASKED, bool PAD = false>
 __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
@@ -910,11 +916,13 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
   const int units = (p.nb + BPU - 1) / BPU;
   const int unit = blockIdx.x % units, wg_in_unit = blockIdx.x / units, n_wg = gridDim.x / units;
   const int blk = slab / S, sl = slab - blk * S;           // the wave's block inside the unit, its slab inside the block
-  const bool slab_ok = unit * BPU + blk < p.nb;
+  const bool slab_ok = unit * BPU + blk < p.nb && blk < BPU;      // three slabs to a block: the fourth wave of a role has none
   const int k = slab_ok ? unit * BPU + blk : p.nb - 1;
   const int uo = slab * 32 + r;                            // channel inside the unit
-  const int unit_col = unit * TW;                          // first channel of the unit
-  const int ch = slab_ok ? unit_col + uo : 0;
+  const int bw = PAD ? p.bw : KC;                          // channels of a block that exist
+  const int slab_col = k * bw + sl * 32;                   // first channel of the wave's slab
+  const bool ch_ok = !PAD || sl * 32 + r < bw;
+  const int ch = slab_ok && ch_ok ? slab_col + r : 0, kp = slab_ok ? k * KC + sl * 32 + r : 0;
   const int kb = blk * KC;
   unsigned char* stage = stage_all + slab * WaveStage<TR>::kBytes;
   const long long W = p.W;
@@ -941,8 +949,8 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
       hw.load(wg + ((long long)(0 * p.nb + k) * p.bwp + o) * p.bwp + hf * Tr::HW,
               wg + ((long long)(1 * p.nb + k) * p.bwp + o) * p.bwp + hf * Tr::HW);
     }
-    const float nba = -kLog2e * p.bias[ch], nbx = -kLog2e * p.bias[p.Wp + ch];
-    const float sp = p.sp[ch], cs = p.cs[ch];
+    const float nba = -kLog2e * p.bias[kp], nbx = -kLog2e * p.bias[p.Wp + kp];
+    const float sp = p.sp[kp], cs = p.cs[kp];
     float sum_ba = 0.f, sum_bx = 0.f, sum_l = 0.f;
     // The lane's x, delta and h_{t-1} values (16 consecutive tokens of its channel) come from the matrix
     // unit: a 32 x 32 tile times the identity returns the tile in accumulator layout, which is that
@@ -969,9 +977,10 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
       const rsrc_t rh = make_rsrc((const IO*)p.y + ((long long)b * p.T + y_first) * W, (unsigned)(y_rows > 0 ? y_rows : 0) * row_bytes);
 #pragma unroll
       for (int q2 = 0; q2 < 2; ++q2) {
-        const unsigned col = (unsigned)(unit_col + slab * 32 + q2 * Tr::KG + hf * Tr::HW) * 2u;
-        pre_d[q2] = buf_load_frag<Frag>(rd, (unsigned)my_row * row_bytes + col);
-        pre_h[q2] = buf_load_frag<Frag>(rh, my_row >= shift ? (unsigned)(my_row - shift) * row_bytes + col : kOutOfRange);
+        const bool there = !PAD || sl * 32 + q2 * Tr::KG + hf * Tr::HW < bw;
+        const unsigned col = (unsigned)(slab_col + q2 * Tr::KG + hf * Tr::HW) * 2u;
+        pre_d[q2] = buf_load_frag<Frag>(rd, there ? (unsigned)my_row * row_bytes + col : kOutOfRange);
+        pre_h[q2] = buf_load_frag<Frag>(rh, my_row >= shift && there ? (unsigned)(my_row - shift) * row_bytes + col : kOutOfRange);
       }
     };
     // gate products of one tile: issued one iteration before their results are used, so the matrix
@@ -1002,7 +1011,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
         unsigned flbits = 0u;
         if constexpr (MASKED) flbits = flag_run(p, (long long)b * p.T + t0 + hf * 16, t0 + hf * 16);
         float h_first = 0.f;                             // h0 of the sequence, for the lane that owns token 0
-        if (c == 0 && hf == 0 && p.h0) h_first = p.h0[(long long)b * W + ch];
+        if (c == 0 && hf == 0 && p.h0 && ch_ok) h_first = p.h0[(long long)b * W + ch];
 
         const IO* tile_x = lds_x[xb];
         f32x16 xc, dc, hc, ua_next, ux_next;
@@ -1073,7 +1082,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
       // per-workgroup partial of the bias and Lambda gradients
       sum_ba += xhalf(sum_ba, hf); sum_bx += xhalf(sum_bx, hf); sum_l += xhalf(sum_l, hf);
       if (hf == 0) {
-        float* ps = p.partial + (long long)wg_in_unit * 3 * p.Wp + ch;
+        float* ps = p.partial + (long long)wg_in_unit * 3 * p.Wp + kp;
         ps[0] = sum_ba; ps[p.Wp] = sum_bx; ps[2 * p.Wp] = sum_l;
       }
     }
@@ -1096,6 +1105,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
         for (int v = 0; v < 16; ++v) dw[g][js][v] = 0.f;
     // x tiles: 32 rows x 16 vectors, two per thread of the four product waves
     const int gid = tid - 4 * 64;
+    const int x_col = tile_channel<PAD>(p, unit, unit * TW, (gid & 15) * Tr::HW);      // the same for both
     Frag pre_x[2];
     auto issue = [&](const Place& q) {
       const bool live = q.tile < n_tiles;
@@ -1106,7 +1116,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const int idx = gid + 256 * i, row = idx >> 4, cv = idx & 15;
-        pre_x[i] = buf_load_frag<Frag>(rx, (unsigned)row * row_bytes + (unsigned)(unit_col + cv * Tr::HW) * 2u);
+        pre_x[i] = buf_load_frag<Frag>(rx, x_col >= 0 ? (unsigned)row * row_bytes + (unsigned)x_col * 2u : kOutOfRange);
       }
     };
     auto store_x = [&](int buf) {
@@ -1173,7 +1183,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
         wave_lds_fence();
         const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
         const rsrc_t rdx = make_rsrc((const IO*)p.dx + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-        stage_flush<TR>(stage, rdx, row_bytes, (unsigned)(unit_col + slab * 32) * 2u, lane);
+        stage_flush<TR>(stage, rdx, row_bytes, (unsigned)slab_col * 2u, lane, !PAD || sl * 32 + (lane & 3) * 8 < bw);
         wave_lds_fence();
       }
       done = at;
@@ -1485,7 +1495,7 @@ struct FinishArgs {
   const float* partial; const float* dsp; void* db_a; void* db_x; void* dlambda;
   const float* dw_partial; void* dw_a; void* dw_x;
   int W, nb, bw, bwp, Wp, wg_per_unit, n_wg, vec_blocks, grad_dtype, dw_bf16;
-  int dw_vec;                                              // unpadded blocks of a multiple of 8 channels, 16-byte aligned gradients
+  int dw_vec;                                              // blocks of a multiple of 8 channels, 16-byte aligned gradients
 };
 
 __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
@@ -1517,12 +1527,17 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
     const long long i = i8 * 8;
     const int gate = (int)((i / per_gate) % 2);
     const long long k = i / (2 * per_gate);
-    const long long stride = (long long)p.nb * 2 * per_gate;
+    const long long stride = (long long)p.nb * 2 * p.bwp * p.bwp;
+    long long from = i;                                      // of the partials: blocks of bwp x bwp
+    if (p.bw != p.bwp) {
+      const int in_gate = (int)(i % per_gate), o = in_gate / p.bw;
+      from = ((k * 2 + gate) * p.bwp + o) * p.bwp + (in_gate - o * p.bw);
+    }
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
     if (p.dw_bf16) {
-      const __bf16* src16 = (const __bf16*)p.dw_partial + i;
+      const __bf16* src16 = (const __bf16*)p.dw_partial + from;
       int g = 0;
       for (; g + 7 < p.n_wg; g += 8) {                       // eight loads in flight per thread
         bf16x8 v[8];
@@ -1539,7 +1554,7 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
         for (int e = 0; e < 8; ++e) acc[e] += (float)v[e];
       }
     } else {
-      const float* src = p.dw_partial + i;
+      const float* src = p.dw_partial + from;
       int g = 0;
       for (; g + 3 < p.n_wg; g += 4) {
         f32x4 v[4][2];
@@ -1625,7 +1640,7 @@ static int gate_gemms_and_finish(const FusedArgs& a, const Geometry& g, const vo
   r.dw_partial = dw_partial; r.dw_a = dw_a; r.dw_x = dw_x;
   r.W = (int)g.W; r.nb = (int)g.nb; r.bw = (int)g.bw; r.bwp = (int)g.bwp; r.Wp = (int)g.Wp; r.wg_per_unit = a.wg_per_unit;
   r.n_wg = splits; r.vec_blocks = (int)((g.W + 15) / 16); r.grad_dtype = grad_dtype;
-  r.dw_vec = (g.bw == g.bwp && (uintptr_t)dw_a % 16 == 0 && (uintptr_t)dw_x % 16 == 0) ? 1 : 0;
+  r.dw_vec = (g.bw % 8 == 0 && (uintptr_t)dw_a % 16 == 0 && (uintptr_t)dw_x % 16 == 0) ? 1 : 0;
   const long long total = g.nb * g.bw * 2 * g.bw;
   hipLaunchKernelGGL(finish_kernel, dim3((unsigned)(r.vec_blocks + (total / 8 + 255) / 256)), dim3(256), 0, s, r);
   return check_launch("bwd finish");
@@ -1737,8 +1752,7 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
 
 int rglru_hip_fast_path(int64_t W, int64_t nb, int dtype) {
   if (dtype != RGLRU_BF16 || W <= 0 || nb <= 0 || W % nb) return 0;
-  const int64_t bw = W / nb;
-  return (bw == 32 || bw == 64 || bw == 128) ? 1 : 0;
+  return narrow_groups(make_geometry(W, nb), dtype, 1) ? 1 : 0;
 }
 
 // tokens per tile of the reverse-scan kernel: 32 * kDeltaMT
@@ -1757,7 +1771,7 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   rc = check_grad_dtype("bwd_full", grad_dtype);
   if (rc) return rc;
   if (!rglru_hip_fast_path(W, nb, dtype))
-    return fail(RGLRU_E_UNSUPPORTED, "bwd_full: needs 16-bit storage and gate blocks of 32, 64 or 128 channels");
+    return fail(RGLRU_E_UNSUPPORTED, "bwd_full: needs 16-bit storage and gate blocks of up to 128 channels, a multiple of 8");
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "bwd_full: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
   if (!x || !y || !prep || !dy || !ws || !scratch || !dx || !dw_a || !dw_x || !db_a || !db_x || !dlambda)
     return fail(RGLRU_E_ARG, "bwd_full: null pointer");
@@ -1785,7 +1799,8 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   a.partial = (float*)(sb + SL.partial); a.dw_partial = (float*)(sb + SL.dw_partial);
   a.B = (int)B; a.T = (int)T; a.nC = (int)((T + kChunk - 1) / kChunk); a.ckpt_nC = 2 * (int)L.nC;
   a.aligned = 1;
-  const int nkg = held_groups(g, dtype, 1);
+  const int nkg = narrow_groups(g, dtype, 1);
+  const bool pad = narrow_padded(g);
   pack_units(a, g, nkg);
 #ifndef RGLRU_DW_BF16
 #define RGLRU_DW_BF16 1
@@ -1799,17 +1814,20 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   a.queues = pick_queues(B, a.wg_per_unit);
   const bool masked = (flags != nullptr) || (T % (32 * kDeltaMT) != 0);
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
-  const bool chain_scan = fwd_chain_pays(B, T, W);
+  const bool chain_scan = fwd_chain_pays(B, T, g.Wp);
   if (chain_scan) {
     // enough chains to give every compute unit one of its own (see fwd_impl)
-    const dim3 cgrid((unsigned)(8 * ((B * nb + 7) / 8) * (g.bw / 32)));
+    const dim3 cgrid((unsigned)(8 * ((B * nb + 7) / 8) * g.S));
     const bool cmasked = (flags != nullptr) || (T % 32 != 0);
     KernelTimer timer(1, s);
 #define RGLRU_LAUNCH_DELTA_CHAIN(N)                                                                                  \
     if (cmasked) hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, true>), cgrid, dim3(kChainWaves * 64), 0, s, a); \
     else hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, false>), cgrid, dim3(kChainWaves * 64), 0, s, a)
-    if (nkg == 8) { RGLRU_LAUNCH_DELTA_CHAIN(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA_CHAIN(4); } else { RGLRU_LAUNCH_DELTA_CHAIN(2); }
+#define RGLRU_LAUNCH_DELTA_CHAIN_PAD(N) hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, true, true>), cgrid, dim3(kChainWaves * 64), 0, s, a)
+    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA_CHAIN_PAD(8); break; case 6: RGLRU_LAUNCH_DELTA_CHAIN_PAD(6); break; case 4: RGLRU_LAUNCH_DELTA_CHAIN_PAD(4); break; default: RGLRU_LAUNCH_DELTA_CHAIN_PAD(2); } }
+    else if (nkg == 8) { RGLRU_LAUNCH_DELTA_CHAIN(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA_CHAIN(4); } else { RGLRU_LAUNCH_DELTA_CHAIN(2); }
 #undef RGLRU_LAUNCH_DELTA_CHAIN
+#undef RGLRU_LAUNCH_DELTA_CHAIN_PAD
   } else {
     rc = launch_clear(wb, L.b_begin, L.b_end, s);        // records and tickets of this pass
     if (rc) return rc;
@@ -1817,8 +1835,11 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
 #define RGLRU_LAUNCH_DELTA(N)                                                                                        \
     if (masked) hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, true, kDeltaMT>), grid, dim3(kThreads), 0, s, a);      \
     else hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, false, kDeltaMT>), grid, dim3(kThreads), 0, s, a)
-    if (nkg == 8) { RGLRU_LAUNCH_DELTA(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA(4); } else { RGLRU_LAUNCH_DELTA(2); }
+#define RGLRU_LAUNCH_DELTA_PAD(N) hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, true, kDeltaMT, true>), grid, dim3(kThreads), 0, s, a)
+    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA_PAD(8); break; case 6: RGLRU_LAUNCH_DELTA_PAD(6); break; case 4: RGLRU_LAUNCH_DELTA_PAD(4); break; default: RGLRU_LAUNCH_DELTA_PAD(2); } }
+    else if (nkg == 8) { RGLRU_LAUNCH_DELTA(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA(4); } else { RGLRU_LAUNCH_DELTA(2); }
 #undef RGLRU_LAUNCH_DELTA
+#undef RGLRU_LAUNCH_DELTA_PAD
   }
   rc = check_launch("bwd_full scan");
   if (rc) return rc;
@@ -1833,8 +1854,11 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
 #define RGLRU_LAUNCH_GRAD(N)                                                                                          \
     if (masked_grad) hipLaunchKernelGGL((bwd_grad_kernel<__bf16, N, true>), grid2, dim3(kGradThreads), 0, s, a);         \
     else hipLaunchKernelGGL((bwd_grad_kernel<__bf16, N, false>), grid2, dim3(kGradThreads), 0, s, a)
-    if (nkg == 8) { RGLRU_LAUNCH_GRAD(8); } else if (nkg == 4) { RGLRU_LAUNCH_GRAD(4); } else { RGLRU_LAUNCH_GRAD(2); }
+#define RGLRU_LAUNCH_GRAD_PAD(N) hipLaunchKernelGGL((bwd_grad_kernel<__bf16, N, true, true>), grid2, dim3(kGradThreads), 0, s, a)
+    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_GRAD_PAD(8); break; case 6: RGLRU_LAUNCH_GRAD_PAD(6); break; case 4: RGLRU_LAUNCH_GRAD_PAD(4); break; default: RGLRU_LAUNCH_GRAD_PAD(2); } }
+    else if (nkg == 8) { RGLRU_LAUNCH_GRAD(8); } else if (nkg == 4) { RGLRU_LAUNCH_GRAD(4); } else { RGLRU_LAUNCH_GRAD(2); }
 #undef RGLRU_LAUNCH_GRAD
+#undef RGLRU_LAUNCH_GRAD_PAD
   }
   rc = check_launch("bwd_full gradients");
   if (rc) return rc;
@@ -1856,7 +1880,7 @@ int rglru_hip_wide_path(int64_t W, int64_t nb, int dtype) {
 
 int rglru_hip_backward_path(int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int aligned) {
   if (B <= 0 || T <= 0 || W <= 0 || nb <= 0 || W % nb || (dtype != RGLRU_F32 && dtype != RGLRU_BF16)) return -1;
-  if (aligned && rglru_hip_fast_path(W, nb, dtype)) return fwd_chain_pays(B, T, W) ? RGLRU_PATH_FAST_CHAIN : RGLRU_PATH_FAST_TILED;
+  if (aligned && rglru_hip_fast_path(W, nb, dtype)) return fwd_chain_pays(B, T, make_geometry(W, nb).Wp) ? RGLRU_PATH_FAST_CHAIN : RGLRU_PATH_FAST_TILED;
   if (aligned && rglru_hip_wide_path(W, nb, dtype)) return RGLRU_PATH_WIDE;
   if (aligned && rglru_hip_pre_path(W, nb, dtype)) return RGLRU_PATH_PRE;
   return RGLRU_PATH_PORTABLE;

@@ -869,3 +869,57 @@ def test_hip_graph_replays_match_eager_results():
             # the carry composition order of a look-back depends on timing: equal up to rounding
             assert rel_err(got.float(), want.float()) < 1e-2, (replay, name)
         assert rel_err(captured[0].float(), eager[0].float()) < 1e-6
+
+
+# ------------------------------------------------------------------ gate blocks that do not fill their 32-channel slabs
+@pytest.mark.parametrize("bw,nb", [(8, 3), (16, 5), (24, 4), (40, 3), (48, 16), (56, 1), (72, 2), (88, 3), (96, 3), (104, 2), (120, 3)])
+@pytest.mark.parametrize("B,T,masks,carried", [(2, 70, True, True), (1, 64, False, False), (3, 33, False, True)])
+def test_padded_narrow_blocks_match_oracle(bw, nb, B, T, masks, carried, kernel_choice):
+    """bf16 gate blocks of any multiple of 8 channels up to 128 run the register-held kernels with padded slabs: outputs,
+    final state and every gradient against the oracle, with the parameters (and their gradients) in bf16 and in fp32."""
+    from griffin_amd import _lib, hip_rglru
+    from griffin_amd.hip_scan import kernel_path
+
+    W = bw * nb
+    assert kernel_path(B, T, W, nb, torch.bfloat16) in (_lib.PATH_FAST_CHAIN, _lib.PATH_FAST_TILED)
+    _say("padded blocks", bw, nb, B, T, masks, carried, kernel_choice)
+    case = orc.make_case(B, T, W, nb, seed=bw, h0_std=0.5 if carried else 0.0, bias_std=0.5)
+    reset, active = _masks(B, T, masks)
+    dh_last = torch.randn(B, W, generator=torch.Generator().manual_seed(6)) if carried else None
+    y, h_last, grads = hip_run(case, torch.bfloat16, reset, active, dh_last)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, active, dh_last)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
+    # fp32 parameters holding the same values: fp32 gradients
+    leaves = [case[k].bfloat16().cuda() if k == "x" else case[k].bfloat16().float().cuda().requires_grad_(True) for k in PARAMS]
+    h0 = None if case.get("h0") is None else case["h0"].cuda()
+    y32, h32 = hip_rglru(*leaves, 8.0, h0, None if reset is None else reset.cuda(), None if active is None else active.cuda())
+    outs, ups = [y32], [case["dy"].bfloat16().cuda()]
+    if dh_last is not None:
+        outs.append(h32)
+        ups.append(dh_last.cuda())
+    for name, g in zip(PARAMS[1:], torch.autograd.grad(outs, leaves[1:], ups)):
+        assert g.dtype == torch.float32
+        errs[name + " fp32"] = rel_err(g, rgrads[name])
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
+
+
+@pytest.mark.parametrize("bw,nb,B", [(16, 3, 5), (48, 4, 17), (80, 2, 33), (144, 2, 3), (240, 1, 16)])
+def test_decode_of_blocks_that_end_inside_a_step(bw, nb, B):
+    """Decode steps of gate blocks of an odd multiple of 16 channels: the last 32-channel step of the products is half
+    empty.  One step at a time and all steps in one launch, against the oracle."""
+    from griffin_amd import PreparedParams, hip_rglru_step, hip_rglru_steps
+
+    steps, W = 5, bw * nb
+    case = orc.make_case(B, steps, W, nb, seed=bw, h0_std=0.5, bias_std=0.5)
+    params = [case[k].bfloat16() for k in PARAMS[1:]]
+    x = case["x"].bfloat16()
+    y, h_last, _ = oracle_run(case, torch.bfloat16)
+    prep = PreparedParams(*[t.cuda() for t in params], 8.0, torch.bfloat16)
+    state = case["h0"].cuda().contiguous()
+    rows = torch.stack([hip_rglru_step(x[:, t].cuda(), prep, state) for t in range(steps)], 1)
+    assert rel_err(rows.float(), y) < BF16_TOL and rel_err(state, h_last) < BF16_TOL
+    many = case["h0"].cuda().contiguous()
+    ys = hip_rglru_steps(x.transpose(0, 1).contiguous().cuda(), prep, many)
+    assert rel_err(many, state) < 1e-6 and rel_err(ys.transpose(0, 1).float(), rows.float()) < 1e-6
