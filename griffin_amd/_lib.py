@@ -14,7 +14,7 @@ RGLRU_BF16 = 1
 FLAG_RESET = 1
 FLAG_INACTIVE = 2
 CHUNK = 32
-ABI_VERSION = 20
+ABI_VERSION = 21
 PATH_PORTABLE, PATH_FAST_TILED, PATH_FAST_CHAIN, PATH_WIDE, PATH_PRE = range(5)
 PATH_NAMES = ("portable", "fast_tiled", "fast_chain", "wide", "pre")
 
@@ -71,6 +71,11 @@ _SIGNATURES = {
     "rglru_hip_rmsnorm_fwd": (ctypes.c_int, [_P, _P, _P, _P, _I, _I, ctypes.c_float, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_rmsnorm_scratch_bytes": (ctypes.c_size_t, [_I, _I]),
     "rglru_hip_rmsnorm_bwd": (ctypes.c_int, [_P] * 7 + [_I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "rglru_hip_linear_splits": (ctypes.c_int64, [ctypes.c_int, _I, _I, _I, ctypes.c_int, ctypes.c_int]),
+    "rglru_hip_linear": (ctypes.c_int, [ctypes.c_int, _P, _P, _I, _P, _P, _I] + [_P] * 5 + [_I, _P, _P, _I, _I, _I, ctypes.c_int, _P]),
+    "rglru_hip_sums": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P]),
+    "rglru_hip_block_bwd": (ctypes.c_int, [_P] * 15 + [_I] * 6 + [_P]),
+    "rglru_hip_block_finish": (ctypes.c_int, [_P] * 11 + [ctypes.c_int] + [_I] * 5 + [_P]),
     "rglru_hip_decode_prepare": (ctypes.c_int, [_P, _I] + [_P] * 10 + [_I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_decode_linear": (ctypes.c_int, [_P, _I] + [_P] * 4 + [_I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_decode_project": (ctypes.c_int, [_P, _I] + [_P] * 15 + [_I, _I, _I, _I, ctypes.c_int, _P]),

@@ -19,6 +19,7 @@
 
 #include "rglru_device.h"
 #include "rglru_host.h"
+#include "rglru_sums.h"
 
 namespace rglru {
 
@@ -413,34 +414,28 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvArgs p) {
   }
 }
 
-// Sums the per-run partials: one thread per (tap or bias, channel).
-struct ConvFinishArgs { const float* partial; void* dtaps; void* dbias; int W, K, slots, grad_dtype; };
-__global__ __launch_bounds__(256) void conv_finish_kernel(ConvFinishArgs p) {
-  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long long)(p.K + 1) * p.W) return;
-  const int j = (int)(i / p.W), c = (int)(i - (long long)j * p.W);
-  const float* src = p.partial + (long long)j * p.W + c;
-  const long long stride = (long long)(p.K + 1) * p.W;
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  int n = 0;
-  for (; n + 16 <= p.slots; n += 16) {                   // sixteen loads in flight: latency, not bytes, is what this kernel waits for
-    float v[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = src[(long long)(n + u) * stride];
-#pragma unroll
-    for (int u = 0; u < 16; u += 4) { s0 += v[u]; s1 += v[u + 1]; s2 += v[u + 2]; s3 += v[u + 3]; }
-  }
-  for (; n < p.slots; ++n) s0 += src[(long long)n * stride];
-  const float s = (s0 + s1) + (s2 + s3);
-  void* dst = j < p.K ? p.dtaps : p.dbias;
-  if (!dst) return;
-  const long long at = j < p.K ? (long long)c * p.K + j : c;
-  if (p.grad_dtype == RGLRU_BF16) ((__bf16*)dst)[at] = (__bf16)s; else ((float*)dst)[at] = s;
+static __global__ __launch_bounds__(256) void sum_job_kernel(SumJob j) {
+  __shared__ float red[8][32];
+  run_sum_job(j, (int)blockIdx.x, red);
 }
 
 // ------------------------------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------------------------------
+static int launch_sum_job(const char* who, SumJob j, void* stream) {
+  plan_sum_job(j);
+  hipLaunchKernelGGL(sum_job_kernel, dim3((unsigned)j.blocks), dim3(256), 0, (hipStream_t)stream, j);
+  return check_launch(who);
+}
+
+// Column sums of fp32 partial rows [slots][n].
+static SumJob column_sum_job(const float* partial, void* out, int64_t n, int64_t slots, int out_dtype) {
+  SumJob j;
+  memset(&j, 0, sizeof(j));
+  j.src = partial; j.dst = out; j.n = n; j.sets = (int)slots; j.dst_bf16 = out_dtype == RGLRU_BF16;
+  return j;
+}
+
 static int conv_check(const char* who, int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype) {
   if (dtype != RGLRU_F32 && dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "%s: dtype must be RGLRU_F32 or RGLRU_BF16, got %d", who, dtype);
   if (vec_dtype != RGLRU_F32 && vec_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "%s: unknown parameter dtype %d", who, vec_dtype);
@@ -1124,39 +1119,9 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(NormArgs p) {
   }
 }
 
-// Sums the per-workgroup partial rows: a workgroup owns 32 columns, eight threads share a column.
-struct NormFinishArgs { const float* partial; void* dg; int D, slots, grad_dtype; };
-__global__ __launch_bounds__(256) void rmsnorm_finish_kernel(NormFinishArgs p) {
-  __shared__ float red[8][32];
-  const int col = threadIdx.x & 31, share = threadIdx.x >> 5;
-  const int c = blockIdx.x * 32 + col;
-  float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-  if (c < p.D) {
-    // sixteen loads in flight per thread: the kernel is a chain of memory round trips, not of bytes
-    int n = share;
-    for (; n + 120 < p.slots; n += 128) {
-      float v[16];
-#pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = p.partial[(long long)(n + 8 * u) * p.D + c];
-#pragma unroll
-      for (int u = 0; u < 16; u += 4) { s0 += v[u]; s1 += v[u + 1]; s2 += v[u + 2]; s3 += v[u + 3]; }
-    }
-    for (; n < p.slots; n += 8) s0 += p.partial[(long long)n * p.D + c];
-  }
-  red[share][col] = (s0 + s1) + (s2 + s3);
-  __syncthreads();
-  if (share == 0 && c < p.D) {
-    float s = 0.f;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) s += red[q][col];
-    if (p.grad_dtype == RGLRU_BF16) ((__bf16*)p.dg)[c] = (__bf16)s; else ((float*)p.dg)[c] = s;
-  }
-}
-
 // Column sums of a [rows, D] matrix (the bias gradient of a Linear layer: db = sum over rows of dy).  A
 // workgroup owns 32 vectors of columns and a slot of rows; its 8 row lanes stride through the slot with all
-// their loads in flight, add up in LDS and leave one partial row per slot, which rmsnorm_finish_kernel
-// sums in fixed order.
+// their loads in flight, add up in LDS and leave one partial row per slot, which a sum job adds up in fixed order.
 constexpr int kColsumVecs = 32, kColsumLanes = 8, kColsumRowsPerLane = 8;
 struct ColsumArgs { const void* x; float* partial; long long rows; int D, nvec, vec_groups; };
 template <typename IO, int V>
@@ -1199,49 +1164,6 @@ __global__ __launch_bounds__(256) void colsum_kernel(ColsumArgs p) {
       for (int q = 0; q < kColsumLanes; ++q) sum += red[q][v][l];
       p.partial[slot * p.D + c] = sum;
     }
-  }
-}
-
-// Sum of `sets` arrays of n elements each, x[s * n + i] -> out[i]: what is left of a weight gradient whose
-// contraction over the tokens was split into a batch of shorter GEMMs.  A thread owns V consecutive elements and
-// asks for up to eight sets at once; fp32 accumulation in the order of the sets.
-struct SumSetsArgs { const void* x; void* out; long long n; int sets; };
-template <typename IO, int V>
-__global__ __launch_bounds__(256) void sum_sets_kernel(SumSetsArgs p) {
-  typedef typename ConvRow<IO, V>::Raw Raw;
-  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * V;
-  if (i >= p.n) return;
-  const IO* src = (const IO*)p.x + i;
-  float acc[V];
-#pragma unroll
-  for (int v = 0; v < V; ++v) acc[v] = 0.f;
-  for (int s0 = 0; s0 < p.sets; s0 += 8) {
-    Raw raw[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int s = s0 + q < p.sets ? s0 + q : p.sets - 1;   // a set past the last is asked again and not added
-      if constexpr (V == 1) raw[q] = (float)src[(long long)s * p.n];
-      else raw[q] = *reinterpret_cast<const Raw*>(src + (long long)s * p.n);
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      float v[V];
-      ConvRow<IO, V>::unpack(v, raw[q]);
-      if (s0 + q < p.sets) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) acc[e] += v[e];
-      }
-    }
-  }
-  IO* dst = (IO*)p.out + i;
-  if constexpr (V == 1) {
-    dst[0] = (IO)acc[0];
-  } else {
-    typedef IO Vec __attribute__((ext_vector_type(V)));
-    Vec o;
-#pragma unroll
-    for (int e = 0; e < V; ++e) o[e] = (IO)acc[e];
-    *reinterpret_cast<Vec*>(dst) = o;
   }
 }
 
@@ -1320,17 +1242,22 @@ int rglru_hip_conv_bwd(const void* u, const void* state, const void* taps, const
                                  K, dtype, vec_dtype, grad_dtype, stream);
 }
 
-int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
-                            const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
-                            int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
-                            void* stream) {
+}  // extern "C"
+
+int64_t rglru::conv_partial_sets(int64_t B, int64_t T) {
+  const int64_t runs = (T + kConvRunBwd - 1) / kConvRunBwd;
+  return B * ((runs + kConvBwdRuns - 1) / kConvBwdRuns);
+}
+
+int rglru::conv_bwd_partials(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
+                             const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate,
+                             int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, void* stream) {
   int rc = conv_check("conv_bwd", B, T, W, K, dtype, vec_dtype);
   if (rc) return rc;
   if (du_stride == 0) du_stride = W;
   if (du_stride < W) return fail(RGLRU_E_ARG, "conv_bwd: du_stride %lld is smaller than the width %lld", (long long)du_stride, (long long)W);
   rc = conv_check("conv_bwd", B, T, du_stride, K, dtype, vec_dtype);      // the strided rows obey the same per-sequence limit
   if (rc) return rc;
-  if (grad_dtype != RGLRU_F32 && grad_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "conv_bwd: unknown gradient dtype %d", grad_dtype);
   if (!u || !taps || !segment_pos || !dout || !scratch || !du) return fail(RGLRU_E_ARG, "conv_bwd: null pointer");
   ConvArgs a;
   memset(&a, 0, sizeof(a));
@@ -1347,17 +1274,19 @@ int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, 
   dim3 grid((unsigned)(B * run_groups * vec_groups));
   hipStream_t s = (hipStream_t)stream;
   RGLRU_CONV_DISPATCH(conv_bwd_kernel, dtype, vec, grid, s, a);
-  rc = check_launch("conv_bwd");
-  if (rc) return rc;
-  if (dtaps || dbias) {
-    ConvFinishArgs f;
-    f.partial = a.partial; f.dtaps = dtaps; f.dbias = dbias; f.W = (int)W; f.K = (int)K;
-    f.slots = (int)(B * run_groups); f.grad_dtype = grad_dtype;
-    const long long n = (long long)(K + 1) * W;
-    hipLaunchKernelGGL(conv_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, f);
-    rc = check_launch("conv_bwd finish");
-  }
-  return rc;
+  return check_launch("conv_bwd");
+}
+
+extern "C" {
+
+int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
+                            const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate, void* dtaps, void* dbias,
+                            int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
+                            void* stream) {
+  if (grad_dtype != RGLRU_F32 && grad_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "conv_bwd: unknown gradient dtype %d", grad_dtype);
+  const int rc = conv_bwd_partials(u, state, taps, segment_pos, rows, dout, scratch, du, du_stride, dstate, B, T, W, K, dtype, vec_dtype, stream);
+  if (rc || (!dtaps && !dbias)) return rc;
+  return launch_sum_job("conv_bwd finish", conv_sum_job((const float*)scratch, dtaps, dbias, W, K, conv_partial_sets(B, T), grad_dtype), stream);
 }
 
 // Host-side view of the index (see padded_index): the positions of prefix rows and the per-row words.
@@ -1407,12 +1336,7 @@ int rglru_hip_conv_padded_bwd(const void* u, const void* state, const void* taps
     if (rc) return rc;
   }
   if (dtaps || dbias) {
-    ConvFinishArgs f;
-    f.partial = a.partial; f.dtaps = dtaps; f.dbias = dbias; f.W = (int)W; f.K = (int)K;
-    f.slots = (int)(B * run_groups); f.grad_dtype = grad_dtype;
-    const long long n = (long long)(K + 1) * W;
-    hipLaunchKernelGGL(conv_finish_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, f);
-    rc = check_launch("conv_padded_bwd finish");
+    rc = launch_sum_job("conv_padded_bwd finish", conv_sum_job(a.partial, dtaps, dbias, W, K, B * run_groups, grad_dtype), stream);
   }
   return rc;
 }
@@ -1593,10 +1517,7 @@ int rglru_hip_rmsnorm_bwd(const void* x, const void* g, const float* inv, const 
   }
   rc = check_launch("rmsnorm_bwd");
   if (rc || !dg) return rc;
-  NormFinishArgs f;
-  f.partial = a.partial; f.dg = dg; f.D = (int)D; f.slots = blocks; f.grad_dtype = grad_dtype;
-  hipLaunchKernelGGL(rmsnorm_finish_kernel, dim3((unsigned)((D + 31) / 32)), dim3(256), 0, s, f);
-  return check_launch("rmsnorm_bwd finish");
+  return launch_sum_job("rmsnorm_bwd finish", column_sum_job(a.partial, dg, D, blocks, grad_dtype), stream);
 }
 
 static long long colsum_slots(int64_t rows) {
@@ -1608,22 +1529,10 @@ int rglru_hip_sum_sets(const void* x, void* out, int64_t sets, int64_t n, int dt
   if (dtype != RGLRU_F32 && dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "sum_sets: dtype must be RGLRU_F32 or RGLRU_BF16, got %d", dtype);
   if (sets <= 0 || n <= 0) return fail(RGLRU_E_ARG, "sum_sets: sets and n must be positive (got %lld, %lld)", (long long)sets, (long long)n);
   if (sets >= (1 << 20) || n >= (1ll << 38)) return fail(RGLRU_E_UNSUPPORTED, "sum_sets: problem too large");
-  const bool vec = conv_vector_ok(n, dtype, {x, out});
-  const int V = vec ? (dtype == RGLRU_BF16 ? 8 : 4) : 1;
-  SumSetsArgs a;
-  a.x = x; a.out = out; a.n = n; a.sets = (int)sets;
-  const long long blocks = ((n + V - 1) / V + 255) / 256;
-  if (blocks >= (1ll << 31)) return fail(RGLRU_E_UNSUPPORTED, "sum_sets: problem too large");
-  dim3 grid((unsigned)blocks);
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == RGLRU_BF16) {
-    if (vec) hipLaunchKernelGGL((sum_sets_kernel<__bf16, 8>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((sum_sets_kernel<__bf16, 1>), grid, dim3(256), 0, s, a);
-  } else {
-    if (vec) hipLaunchKernelGGL((sum_sets_kernel<float, 4>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((sum_sets_kernel<float, 1>), grid, dim3(256), 0, s, a);
-  }
-  return check_launch("sum_sets");
+  SumJob j;
+  memset(&j, 0, sizeof(j));
+  j.src = x; j.dst = out; j.n = n; j.sets = (int)sets; j.src_bf16 = j.dst_bf16 = dtype == RGLRU_BF16;
+  return launch_sum_job("sum_sets", j, stream);
 }
 
 size_t rglru_hip_colsum_scratch_bytes(int64_t rows, int64_t D) {
@@ -1633,7 +1542,7 @@ size_t rglru_hip_colsum_scratch_bytes(int64_t rows, int64_t D) {
 
 int rglru_hip_colsum(const void* x, void* scratch, void* out, int64_t rows, int64_t D, int dtype, int out_dtype,
                      void* stream) {
-  if (!x || !scratch || !out) return fail(RGLRU_E_ARG, "colsum: null pointer");
+  if (!x || !scratch) return fail(RGLRU_E_ARG, "colsum: null pointer");
   if (dtype != RGLRU_F32 && dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "colsum: dtype must be RGLRU_F32 or RGLRU_BF16, got %d", dtype);
   if (out_dtype != RGLRU_F32 && out_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "colsum: unknown output dtype %d", out_dtype);
   if (rows <= 0 || D <= 0) return fail(RGLRU_E_ARG, "colsum: rows and D must be positive (got %lld, %lld)", (long long)rows, (long long)D);
@@ -1656,10 +1565,7 @@ int rglru_hip_colsum(const void* x, void* scratch, void* out, int64_t rows, int6
   }
   int rc = check_launch("colsum");
   if (rc) return rc;
-  NormFinishArgs f;
-  f.partial = a.partial; f.dg = out; f.D = (int)D; f.slots = (int)slots; f.grad_dtype = out_dtype;
-  hipLaunchKernelGGL(rmsnorm_finish_kernel, dim3((unsigned)((D + 31) / 32)), dim3(256), 0, s, f);
-  return check_launch("colsum finish");
+  return out ? launch_sum_job("colsum finish", column_sum_job(a.partial, out, D, slots, out_dtype), stream) : RGLRU_OK;
 }
 
 }  // extern "C"

@@ -3,6 +3,7 @@
 // entry points.  The forward kernels and the conventions shared with them are in rglru_fused.hip / .h.
 
 #include "rglru_fused.h"
+#include "rglru_sums.h"
 
 namespace rglru {
 
@@ -1498,9 +1499,8 @@ struct FinishArgs {
   int dw_vec;                                              // blocks of a multiple of 8 channels, 16-byte aligned gradients
 };
 
-__global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
-  __shared__ float part_sum[3][16][16];
-  if ((int)blockIdx.x >= p.vec_blocks) {
+RGLRU_DEVICE void gate_finish(const FinishArgs& p, int block, float (&part_sum)[3][16][16]) {
+  if (block >= p.vec_blocks) {
     // eight consecutive input channels j of one (block, gate, output channel o) per thread: the partials are laid
     // out like the gradients, so this is a streaming sum in a fixed order with 16-byte accesses (dw_vec: the
     // block width equals the padded width)
@@ -1508,7 +1508,7 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
     if (!p.dw_vec) {
       // any width, any alignment: eight elements of the unpadded gradients per thread, one at a time
       const long long total = (long long)p.nb * 2 * per_gate;
-      const long long first = ((long long)(blockIdx.x - p.vec_blocks) * blockDim.x + threadIdx.x) * 8;
+      const long long first = ((long long)(block - p.vec_blocks) * blockDim.x + threadIdx.x) * 8;
       const long long stride = (long long)p.nb * 2 * p.bwp * p.bwp;
       for (long long i = first; i < first + 8 && i < total; ++i) {
         const int j = (int)(i % p.bw), o = (int)((i / p.bw) % p.bw);
@@ -1522,7 +1522,7 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
       return;
     }
     const long long total8 = (long long)p.nb * 2 * per_gate / 8;
-    const long long i8 = (long long)(blockIdx.x - p.vec_blocks) * blockDim.x + threadIdx.x;
+    const long long i8 = (long long)(block - p.vec_blocks) * blockDim.x + threadIdx.x;
     if (i8 >= total8) return;
     const long long i = i8 * 8;
     const int gate = (int)((i / per_gate) % 2);
@@ -1590,7 +1590,7 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
   // 16 channels per workgroup; sixteen threads per channel each sum a share of the per-workgroup
   // partials (independent loads), combined through LDS in a fixed order
   const int cl = threadIdx.x & 15, share = threadIdx.x >> 4;
-  const int ch = blockIdx.x * 16 + cl;
+  const int ch = block * 16 + cl;
   float sa = 0.f, sx = 0.f, sl = 0.f;
   int kp = 0;
   if (ch < p.W) {
@@ -1611,6 +1611,28 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
     store_vec(p.db_a, ch, sa, p.grad_dtype);
     store_vec(p.db_x, ch, sx, p.grad_dtype);
     store_vec(p.dlambda, ch, sl * p.dsp[kp], p.grad_dtype);
+  }
+}
+
+__global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
+  __shared__ float part_sum[3][16][16];
+  gate_finish(p, (int)blockIdx.x, part_sum);
+}
+
+// All last sums of a block's backward pass in one launch: the gates' (the first gate_blocks workgroups), then up to five jobs.
+// Six launches of 4 to 6 us each took as long as they have steps (B8 T2048 W1024: 41 us together).
+constexpr int kBlockJobs = 5;
+struct BlockFinishArgs { FinishArgs gates; SumJob job[kBlockJobs]; int gate_blocks, jobs; };
+__global__ __launch_bounds__(256) void block_finish_kernel(BlockFinishArgs p) {
+  __shared__ union { float gates[3][16][16]; float sums[8][32]; } lds;
+  int block = (int)blockIdx.x;
+  if (block < p.gate_blocks) { gate_finish(p.gates, block, lds.gates); return; }
+  block -= p.gate_blocks;
+#pragma unroll
+  for (int i = 0; i < kBlockJobs; ++i) {
+    if (i >= p.jobs) return;
+    if (block < p.job[i].blocks) { run_sum_job(p.job[i], block, lds.sums); return; }
+    block -= p.job[i].blocks;
   }
 }
 
@@ -1761,11 +1783,35 @@ int rglru_hip_fast_path(int64_t W, int64_t nb, int dtype) {
 #endif
 constexpr int kDeltaMT = RGLRU_DELTA_MT;
 
-int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const float* h0,
-                       const uint8_t* flags, const void* dy, const float* dh_last, void* ws, void* scratch,
-                       void* dx, void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda,
-                       float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
-                       void* stream) {
+// Workgroups per unit of the gradient kernel (one per compute unit), which are also the sets its partial sums come in.
+static int grad_workgroups(int64_t B, int64_t T, int units) {
+  int n_wg = num_compute_units() / units; if (n_wg < 1) n_wg = 1; if (n_wg > kGemmWgPerUnit) n_wg = kGemmWgPerUnit;
+  const long long tiles = B * ((T + 31) / 32);
+  return n_wg > tiles ? (int)tiles : n_wg;
+}
+
+// Last sums of the fast backward; returns the workgroups they take.
+static int fast_finish_args(const Geometry& g, const void* prep, const char* scratch, int64_t B, int64_t T, int dtype, int grad_dtype,
+                            void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda, FinishArgs& r) {
+  const ScratchLayout SL = make_scratch_layout(B, T, g, kScratchFast);
+  FusedArgs a;
+  memset(&a, 0, sizeof(a));
+  a.units = (int)g.units;
+  pack_units(a, g, narrow_groups(g, dtype, 1));
+  memset(&r, 0, sizeof(r));
+  r.partial = (const float*)(scratch + SL.partial); r.dsp = finish_dsp(g, prep, dtype); r.db_a = db_a; r.db_x = db_x; r.dlambda = dlambda;
+  r.dw_partial = (const float*)(scratch + SL.dw_partial); r.dw_a = dw_a; r.dw_x = dw_x;
+  r.W = (int)g.W; r.nb = (int)g.nb; r.bw = (int)g.bw; r.bwp = (int)g.bwp; r.Wp = (int)g.Wp;
+  r.n_wg = r.wg_per_unit = grad_workgroups(B, T, a.units);
+  r.vec_blocks = (int)((g.W + 15) / 16); r.grad_dtype = grad_dtype; r.dw_bf16 = grad_dtype == RGLRU_BF16; r.dw_vec = 1;
+  return r.vec_blocks + (int)((g.nb * g.bw * 2 * g.bw / 8 + 255) / 256);
+}
+
+// The two kernels of the fast backward; their partial sums stay in `scratch`.
+static int bwd_full_kernels(const void* x, const void* y, const void* prep, const float* h0,
+                            const uint8_t* flags, const void* dy, const float* dh_last, void* ws, void* scratch,
+                            void* dx, float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
+                            void* stream) {
   int rc = check_geometry("bwd_full", W, nb, dtype);
   if (rc) return rc;
   rc = check_grad_dtype("bwd_full", grad_dtype);
@@ -1773,15 +1819,13 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   if (!rglru_hip_fast_path(W, nb, dtype))
     return fail(RGLRU_E_UNSUPPORTED, "bwd_full: needs 16-bit storage and gate blocks of up to 128 channels, a multiple of 8");
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "bwd_full: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
-  if (!x || !y || !prep || !dy || !ws || !scratch || !dx || !dw_a || !dw_x || !db_a || !db_x || !dlambda)
-    return fail(RGLRU_E_ARG, "bwd_full: null pointer");
+  if (!x || !y || !prep || !dy || !ws || !scratch || !dx) return fail(RGLRU_E_ARG, "bwd_full: null pointer");
   rc = check_extents("bwd_full", B, T, W);
   if (rc) return rc;
   Geometry g = make_geometry(W, nb);
   if (!is_aligned(x, W, g.bw, 2) || !is_aligned(y, W, g.bw, 2) || !is_aligned(dy, W, g.bw, 2) || !is_aligned(dx, W, g.bw, 2))
     return fail(RGLRU_E_UNSUPPORTED, "bwd_full: x, y, dy and dx must be 16-byte aligned");
-  if ((uintptr_t)dw_a % 16 || (uintptr_t)dw_x % 16 || (uintptr_t)scratch % 16)
-    return fail(RGLRU_E_UNSUPPORTED, "bwd_full: dw_a, dw_x and scratch must be 16-byte aligned");
+  if ((uintptr_t)scratch % 16) return fail(RGLRU_E_UNSUPPORTED, "bwd_full: scratch must be 16-byte aligned");
   WorkLayout L = make_work_layout(B, T, g);
   hipStream_t s = (hipStream_t)stream;
   char* wb = (char*)ws;
@@ -1802,12 +1846,9 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   const int nkg = narrow_groups(g, dtype, 1);
   const bool pad = narrow_padded(g);
   pack_units(a, g, nkg);
-#ifndef RGLRU_DW_BF16
-#define RGLRU_DW_BF16 1
-#endif
   // 16-bit weight gradients asked for: the per-workgroup sums (fp32 in registers over a workgroup's share of
   // the tokens) cross memory as bf16 too, which halves what the finish kernel reads back
-  a.dw_bf16 = (RGLRU_DW_BF16 && grad_dtype == RGLRU_BF16) ? 1 : 0;
+  a.dw_bf16 = grad_dtype == RGLRU_BF16 ? 1 : 0;
   // reverse scan: delta[B, T, W] (and dh0)
   const long long chunks = (T + 32 * kDeltaMT - 1) / (32 * kDeltaMT);
   a.wg_per_unit = pick_wg_per_unit(a.units, B * chunks, kDeltaMT == 1 ? 4 : RGLRU_DELTA_OCC, L.max_wg);
@@ -1844,9 +1885,7 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   rc = check_launch("bwd_full scan");
   if (rc) return rc;
   // gradients: one workgroup per compute unit, the same units
-  int n_wg = num_compute_units() / a.units; if (n_wg < 1) n_wg = 1; if (n_wg > kGemmWgPerUnit) n_wg = kGemmWgPerUnit;
-  const long long grad_tiles = B * ((T + 31) / 32);
-  if (n_wg > grad_tiles) n_wg = (int)grad_tiles;
+  const int n_wg = grad_workgroups(B, T, a.units);
   const bool masked_grad = (flags != nullptr) || (T % 32 != 0);
   dim3 grid2((unsigned)(n_wg * a.units));
   {
@@ -1860,17 +1899,92 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
 #undef RGLRU_LAUNCH_GRAD
 #undef RGLRU_LAUNCH_GRAD_PAD
   }
-  rc = check_launch("bwd_full gradients");
+  return check_launch("bwd_full gradients");
+}
+
+int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const float* h0,
+                       const uint8_t* flags, const void* dy, const float* dh_last, void* ws, void* scratch,
+                       void* dx, void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda,
+                       float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
+                       void* stream) {
+  int rc = check_grad_dtype("bwd_full", grad_dtype);
+  if (rc) return rc;
+  if (!dw_a || !dw_x || !db_a || !db_x || !dlambda) return fail(RGLRU_E_ARG, "bwd_full: null pointer");
+  if ((uintptr_t)dw_a % 16 || (uintptr_t)dw_x % 16) return fail(RGLRU_E_UNSUPPORTED, "bwd_full: dw_a and dw_x must be 16-byte aligned");
+  rc = bwd_full_kernels(x, y, prep, h0, flags, dy, dh_last, ws, scratch, dx, dh0, B, T, W, nb, dtype, grad_dtype, stream);
   if (rc) return rc;
   FinishArgs r;
-  memset(&r, 0, sizeof(r));
-  r.partial = a.partial; r.dsp = finish_dsp(g, prep, dtype); r.db_a = db_a; r.db_x = db_x; r.dlambda = dlambda;
-  r.dw_partial = a.dw_partial; r.dw_a = dw_a; r.dw_x = dw_x;
-  r.W = (int)W; r.nb = (int)nb; r.bw = (int)g.bw; r.bwp = (int)g.bwp; r.Wp = (int)g.Wp; r.wg_per_unit = n_wg;
-  r.n_wg = n_wg; r.vec_blocks = (int)((W + 15) / 16); r.grad_dtype = grad_dtype; r.dw_bf16 = a.dw_bf16; r.dw_vec = 1;
-  const long long total = nb * g.bw * 2 * g.bw;
-  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)(r.vec_blocks + (total / 8 + 255) / 256)), dim3(256), 0, s, r);
+  const int blocks = fast_finish_args(make_geometry(W, nb), prep, (const char*)scratch, B, T, dtype, grad_dtype, dw_a, dw_x, db_a, db_x, dlambda, r);
+  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, r);
   return check_launch("bwd_full finish");
+}
+
+int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
+                        const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
+                        void* gate_scratch, void* conv_scratch, void* du, void* dv, int64_t d_stride,
+                        int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream) {
+  if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "block_bwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
+  // the gradient at y takes the place of the one at y * gelu(v), the one at the convolution's output the place of that
+  int rc = rglru_hip_gelu_gate_bwd(dgated, y, v, dgated, dv, B * T * W, W, d_stride, RGLRU_BF16, stream);
+  if (rc) return rc;
+  rc = bwd_full_kernels(x_conv, y, prep, nullptr, flags, dgated, nullptr, ws, gate_scratch, dgated, nullptr, B, T, W, nb, RGLRU_BF16,
+                        RGLRU_BF16, stream);
+  if (rc) return rc;
+  return conv_bwd_partials(u, nullptr, taps, positions, rows, dgated, conv_scratch, du, d_stride, nullptr, B, T, W, K, RGLRU_BF16,
+                           RGLRU_BF16, stream);
+}
+
+// The caller's sums as jobs behind those already there.
+static int add_sums(BlockFinishArgs& p, const rglru_sum* sums, int n_sums, int dst_dtype, long long& blocks) {
+  for (int i = 0; i < n_sums; ++i) {
+    if (!sums[i].dst) continue;
+    if (!sums[i].src || sums[i].sets <= 0 || sums[i].n <= 0 || sums[i].sets >= (1 << 20) || sums[i].n >= (1ll << 38)) return fail(RGLRU_E_ARG, "sums: bad sum %d", i);
+    if (p.jobs == kBlockJobs) return fail(RGLRU_E_ARG, "sums: too many");
+    SumJob j;
+    memset(&j, 0, sizeof(j));
+    j.src = sums[i].src; j.dst = sums[i].dst; j.n = sums[i].n; j.sets = (int)sums[i].sets;
+    j.src_bf16 = sums[i].src_dtype == RGLRU_BF16; j.dst_bf16 = dst_dtype == RGLRU_BF16;
+    plan_sum_job(j);
+    blocks += j.blocks;
+    p.job[p.jobs++] = j;
+  }
+  return blocks >= (1ll << 31) ? fail(RGLRU_E_UNSUPPORTED, "sums: too large") : RGLRU_OK;
+}
+
+int rglru_hip_sums(const rglru_sum* sums, int n_sums, int dst_dtype, void* stream) {
+  if (dst_dtype != RGLRU_F32 && dst_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "sums: unknown result dtype %d", dst_dtype);
+  BlockFinishArgs p;
+  memset(&p, 0, sizeof(p));
+  long long blocks = 0;
+  const int rc = add_sums(p, sums, n_sums, dst_dtype, blocks);
+  if (rc || blocks == 0) return rc;
+  hipLaunchKernelGGL(block_finish_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
+  return check_launch("sums");
+}
+
+int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, void* dw_a, void* dw_x,
+                           void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, const rglru_sum* sums, int n_sums,
+                           int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream) {
+  int rc = check_geometry("block_finish", W, nb, RGLRU_BF16);
+  if (rc) return rc;
+  if (!prep || !gate_scratch || !conv_scratch || !dw_a || !dw_x || !db_a || !db_x || !dlambda) return fail(RGLRU_E_ARG, "block_finish: null pointer");
+  if ((uintptr_t)dw_a % 16 || (uintptr_t)dw_x % 16) return fail(RGLRU_E_UNSUPPORTED, "block_finish: dw_a and dw_x must be 16-byte aligned");
+  if (n_sums < 0 || n_sums >= kBlockJobs) return fail(RGLRU_E_ARG, "block_finish: up to %d sums, got %d", kBlockJobs - 1, n_sums);
+  BlockFinishArgs p;
+  memset(&p, 0, sizeof(p));
+  p.gate_blocks = fast_finish_args(make_geometry(W, nb), prep, (const char*)gate_scratch, B, T, RGLRU_BF16, RGLRU_BF16, dw_a, dw_x, db_a,
+                                   db_x, dlambda, p.gates);
+  long long blocks = p.gate_blocks;
+  if (dtaps || dbias) {
+    SumJob j = conv_sum_job((const float*)conv_scratch, dtaps, dbias, W, K, conv_partial_sets(B, T), RGLRU_BF16);
+    plan_sum_job(j);
+    blocks += j.blocks;
+    p.job[p.jobs++] = j;
+  }
+  rc = add_sums(p, sums, n_sums, RGLRU_BF16, blocks);
+  if (rc) return rc;
+  hipLaunchKernelGGL(block_finish_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);
+  return check_launch("block_finish");
 }
 
 int rglru_hip_wide_path(int64_t W, int64_t nb, int dtype) {

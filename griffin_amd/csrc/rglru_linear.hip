@@ -1,0 +1,352 @@
+// Matrix products of the recurrent block's Linear layers (griffin/griffin.py:379-389 and their reverse mode) on the matrix
+// unit, as kernels of this library:
+//
+//   forward      C_i[m, n] = sum_k X[m, k] W_i[n, k] + b_i[n]         one or two weights on one input
+//   input grad   C[m, n]   = sum_i sum_k A_i[m, k] W_i[k, n]          one or two products into one result
+//   weight grad  C_i[m, n] = sum_k A_i[k, m] X[k, n]                  contraction over the tokens, split over workgroups;
+//                            the column sums of A_i (the bias gradient) come with it
+//
+// Why not the BLAS library alone: a call of it costs the host 17 us, seven calls of it are a third of the host time of a
+// training step of the block, which is what bounds such a step up to several thousand tokens; and it takes no row mask and
+// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 59 us against 70 us, 735 TFLOP/s,
+// here; the split weight gradient of the same 52 us against 91 us), so callers choose by the size of the product.
+//
+// A workgroup of four waves owns a BM x BN tile of C; K is walked in slices of 128 bytes.  A slice of both operands goes
+// through registers (requested one slice ahead) into one of two LDS buffers, one barrier a slice.  An operand that lies in
+// memory with its contraction index contiguous is read from LDS as 16-byte rows (row stride 144 bytes: no bank conflicts);
+// one that lies the other way round is read with the transposing LDS loads (16-bit types), or element by element (fp32).
+// Edges of M, N and K are masked through the offsets of buffer loads, so any size works as long as rows are whole 16-byte
+// vectors.
+#include <hip/hip_runtime.h>
+
+#include <cstring>
+
+#include "rglru_device.h"
+#include "rglru_host.h"
+
+namespace rglru {
+
+struct LinearArgs {
+  const void* a[2]; const void* b[2]; const void* bias[2]; void* c[2];
+  const unsigned char* active;       // one byte per token, or null: inactive rows of the result are zero (weight gradient: rows of A count as zero)
+  float* partial;                    // [split][problem][M][N] instead of c where the contraction is split
+  float* colsum;                     // weight gradient: [split][problem][M] column sums of A, or null
+  long long lda, ldb, ldc;           // elements between rows in memory
+  int M, N, K;                       // of one problem; K of one segment (input gradient)
+  int tiles_m, tiles_n, problems, segments, splits, k_per_split, total;
+};
+
+// Tile of one operand: ROWS rows of the result's index (m or n) x BK of the contraction index.  T: in memory (and in LDS) a row
+// is one contraction index, else one result index.
+template <typename IO, bool T, int ROWS, int THREADS>
+struct OperandTile {
+  typedef Io<IO> Tr;
+  typedef typename Tr::Frag Frag;
+  static constexpr int HW = Tr::HW, BK = 8 * HW;                              // 128 bytes
+  static constexpr int kLines = T ? BK : ROWS, kLineElems = T ? ROWS : BK;    // memory rows of the tile, elements of each
+  // 16-bit transposed rows: 64 bytes more than a multiple of 128, so that the four rows of a transposing read fall on
+  // different banks; fp32: the two halves of a wave read rows four apart, half the banks away
+  static constexpr int kStride = T ? (sizeof(IO) == 2 ? ROWS + 32 : ROWS + 8) : BK + HW;
+  static constexpr int kElems = kLines * kStride;
+  static constexpr int VPR = kLineElems / HW, NV = kLines * VPR / THREADS;
+  static_assert(kLines * VPR % THREADS == 0, "whole vectors per thread");
+  Frag v[NV];
+  unsigned off[NV];                  // lane offsets in bytes, kOutOfRange past the last result index
+  unsigned live;                     // masked weight gradient: bit i = the token of vector i takes part
+
+  RGLRU_DEVICE void setup(int tid, long long ld, int limit) {               // limit: result indices left in the tile
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * THREADS, line = idx / VPR, cv = idx - line * VPR;
+      const int index = T ? cv * HW : line;
+      off[i] = index < limit ? (unsigned)((long long)line * ld * (int)sizeof(IO)) + (unsigned)(cv * HW) * (unsigned)sizeof(IO) : kOutOfRange;
+    }
+    live = ~0u;
+  }
+  // base: first element of the slice (uniform); k_left: contraction indices left
+  RGLRU_DEVICE void request(const IO* base, long long ld, int k_left, int limit, int tid, const unsigned char* active = nullptr) {
+    const int lines = T ? (k_left < BK ? (k_left < 0 ? 0 : k_left) : BK) : (limit < ROWS ? limit : ROWS);
+    const rsrc_t r = make_rsrc(base, k_left > 0 ? (unsigned)((long long)lines * ld) * (unsigned)sizeof(IO) : 0u);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      unsigned o = off[i];
+      if constexpr (!T) {
+        const int cv = (tid + i * THREADS) % VPR;
+        if (cv * HW >= k_left) o = kOutOfRange;
+      }
+      v[i] = buf_load_frag<Frag>(r, o);
+    }
+    if (T && active) {
+      const rsrc_t ra = make_rsrc(active, (unsigned)lines);
+      live = 0u;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        live |= (__builtin_amdgcn_raw_buffer_load_b8(ra, (unsigned)((tid + i * THREADS) / VPR), 0, 0) & 0xff) ? 1u << i : 0u;
+    }
+  }
+  RGLRU_DEVICE void deposit(IO* lds, int tid, bool masked = false) const {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * THREADS, line = idx / VPR, cv = idx - line * VPR;
+      Frag f = v[i];
+      if (T && masked && !((live >> i) & 1u)) f = Tr::zero();
+      *reinterpret_cast<Frag*>(lds + line * kStride + cv * HW) = f;
+    }
+  }
+  // fragment of 32 result indices from `first`, K group kg
+  static RGLRU_DEVICE Frag fragment(const IO* lds, int first, int kg, int lane) {
+    const int r = lane & 31, hf = lane >> 5;
+    if constexpr (!T) {
+      return *reinterpret_cast<const Frag*>(lds + (first + r) * kStride + kg * Tr::KG + hf * HW);
+    } else if constexpr (sizeof(IO) == 2) {
+      return lds_transposed_frag(lds, kStride, kg * Tr::KG, first, lane);
+    } else {
+      Frag f;
+#pragma unroll
+      for (int i = 0; i < HW; ++i) f[i] = lds[(kg * Tr::KG + hf * HW + i) * kStride + first + r];
+      return f;
+    }
+  }
+};
+
+constexpr int kLinearThreads = 256;
+
+template <typename IO, bool TA, bool TB, int BM, int BN>
+__global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
+  typedef Io<IO> Tr;
+  typedef typename Tr::Frag Frag;
+  typedef OperandTile<IO, TA, BM, kLinearThreads> TileA;
+  typedef OperandTile<IO, TB, BN, kLinearThreads> TileB;
+  constexpr int BK = TileA::BK, KGS = BK / Tr::KG;
+  constexpr int MI = BM / 64, NI = BN / 64;                  // 32 x 32 accumulator tiles of a wave (2 x 2 waves)
+  constexpr int kStageRow = BN / 2 + Tr::HW;                 // epilogue: the wave's half tile, row by row
+  constexpr int kStage = 4 * (BM / 2) * kStageRow;
+  constexpr int kBuffers = 2 * (TileA::kElems + TileB::kElems);
+  __shared__ __attribute__((aligned(16))) IO lds[kBuffers > kStage ? kBuffers : kStage];
+
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+  // Workgroups go to the eight XCDs round-robin; each XCD gets a contiguous run of tiles (columns fastest), so that
+  // the rows they share come from memory once and the weights stay in its L2.
+  const int per_xcd = (p.total + 7) >> 3;
+  int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= p.total) return;
+  const int tn = t % p.tiles_n; t /= p.tiles_n;
+  const int problem = t % p.problems; t /= p.problems;
+  const int tm = t % p.tiles_m;
+  const int split = t / p.tiles_m;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int m_left = p.M - m0, n_left = p.N - n0;
+  const int k_begin = split * p.k_per_split;
+  const int k_end = (k_begin + p.k_per_split) < p.K ? (k_begin + p.k_per_split) : p.K;
+  const int slices = (k_end - k_begin + BK - 1) / BK;
+  const int total_slices = slices * p.segments;
+  // one input, two weights (forward); two gradients, one input (weight gradient); both change with the segment (input gradient)
+  const bool masked = TA && p.active != nullptr;
+
+  TileA ta;
+  TileB tb;
+  ta.setup(tid, p.lda, m_left);
+  tb.setup(tid, p.ldb, n_left);
+  auto request = [&](int s) {
+    const int seg = s >= slices ? 1 : 0;
+    const int k = k_begin + (s - seg * slices) * BK;
+    const IO* a = (const IO*)p.a[p.segments > 1 ? seg : (TA ? problem : 0)];
+    const IO* b = (const IO*)p.b[p.segments > 1 ? seg : (TA ? 0 : problem)];
+    const int left = s < total_slices ? k_end - k : 0;
+    const long long ks = s < total_slices ? k : 0;
+    ta.request(a + (TA ? ks * p.lda + m0 : m0 * p.lda + ks), p.lda, left, m_left, tid, masked ? p.active + ks : nullptr);
+    tb.request(b + (TB ? ks * p.ldb + n0 : n0 * p.ldb + ks), p.ldb, left, n_left, tid);
+  };
+  constexpr int kBuffer = TileA::kElems + TileB::kElems;
+
+  f32x16 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  float sum[MI];                                             // column sums of A over the lane's share of K
+#pragma unroll
+  for (int i = 0; i < MI; ++i) sum[i] = 0.f;
+  const bool sums = TA && p.colsum && tn == 0 && wn == 0;
+
+  request(0);
+  ta.deposit(lds, tid, masked);
+  tb.deposit(lds + TileA::kElems, tid);
+  request(1);
+  __syncthreads();
+  for (int s = 0; s < total_slices; ++s) {
+    const IO* cur = lds + (s & 1) * kBuffer;
+    IO* nxt = lds + ((s & 1) ^ 1) * kBuffer;
+    ta.deposit(nxt, tid, masked);
+    tb.deposit(nxt + TileA::kElems, tid);
+    request(s + 2);
+#pragma unroll
+    for (int kg = 0; kg < KGS; ++kg) {
+      Frag fa[MI], fb[NI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) fa[i] = TileA::fragment(cur, wm * (BM / 2) + 32 * i, kg, lane);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) fb[j] = TileB::fragment(cur + TileA::kElems, wn * (BN / 2) + 32 * j, kg, lane);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) Tr::mma(acc[i][j], fa[i], fb[j]);
+      if (sums) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int e = 0; e < Tr::HW; ++e) sum[i] += (float)fa[i][e];
+      }
+    }
+    __syncthreads();
+  }
+
+  if (sums) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const float both = sum[i] + xhalf(sum[i], hf);
+      const int m = wm * (BM / 2) + 32 * i + r;
+      if (hf == 0 && m < m_left) p.colsum[((long long)split * p.problems + problem) * p.M + m0 + m] = both;
+    }
+  }
+  const int col0 = wn * (BN / 2), row0 = wm * (BM / 2);
+  if (p.partial) {
+    float* part = p.partial + (((long long)split * p.problems + problem) * p.M + m0) * p.N + n0;
+    const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.N) * 4u);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int n = col0 + 32 * j + r;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = row0 + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
+          BufIo<float>::store(acc[i][j][v], rc, n < n_left ? ((unsigned)m * (unsigned)p.N + (unsigned)n) * 4u : kOutOfRange, 0u);
+        }
+    }
+    return;
+  }
+  // result in the storage type: through LDS (the slices have been read), then 16-byte vectors of rows
+  float bias[NI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const int n = col0 + 32 * j + r;
+    bias[j] = (p.bias[problem] && n < n_left) ? (float)((const IO*)p.bias[problem])[n0 + n] : 0.f;
+  }
+  IO* stage = lds + wave * (BM / 2) * kStageRow;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int m = 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
+        stage[m * kStageRow + 32 * j + r] = (IO)(acc[i][j][v] + bias[j]);
+      }
+  wave_lds_fence();
+  const rsrc_t rc = make_rsrc((IO*)p.c[problem] + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
+  constexpr int VPR = (BN / 2) / Tr::HW, ROWS = 64 / VPR;
+#pragma unroll
+  for (int q = 0; q < (BM / 2) / ROWS; ++q) {
+    const int m = q * ROWS + lane / VPR, cv = lane % VPR;
+    Frag f = *reinterpret_cast<const Frag*>(stage + m * kStageRow + cv * Tr::HW);
+    const int row = row0 + m, n = col0 + cv * Tr::HW;
+    if (!TA && p.active && row < m_left && !p.active[m0 + row]) f = Tr::zero();
+    buf_store_b128(__builtin_bit_cast(i32x4, f), rc,
+                   n < n_left && row < m_left ? ((unsigned)row * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange);
+  }
+}
+
+// How a product is cut up.  Tiles of 128 x 128 where they give every compute unit one, else 64 x 64 (four times the workgroups
+// at half the reuse): at 2331 x 1024 x 768 in bf16 two forward products take 20 us either way (304 large tiles), one of
+// 2331 x 768 x 1024 12 us in small tiles and 18 us in 114 large ones.  A weight gradient contracts over the tokens, so its
+// tiles are few and its contraction long: it is split over workgroups until there are about two to a compute unit, at
+// least four slices each and at most eight splits (every split costs a pass over the result in fp32; 2331 tokens,
+// 768 x 1024: 67 us whole, 24 us in four, 19 us in eight).
+struct LinearPlan { bool large; int splits; };
+static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
+  auto tiles = [&](int64_t edge) { return ((M + edge - 1) / edge) * ((N + edge - 1) / edge) * problems; };
+  const int64_t units = num_compute_units();
+  LinearPlan p = {tiles(128) >= units, 1};
+  if (kind != RGLRU_LINEAR_WEIGHT_GRAD) return p;
+  const int64_t slices = (K + (dtype == RGLRU_BF16 ? 63 : 31)) / (dtype == RGLRU_BF16 ? 64 : 32);
+  auto splits = [&](int64_t t) {
+    int64_t s = (2 * units + t - 1) / t;
+    if (s > slices / 4) s = slices / 4;
+    return s > 8 ? (int64_t)8 : s < 1 ? (int64_t)1 : s;
+  };
+  p.large = tiles(128) * splits(tiles(128)) >= units;
+  p.splits = (int)splits(tiles(p.large ? 128 : 64));
+  return p;
+}
+
+template <typename IO, bool TA, bool TB>
+static void linear_launch(LinearArgs& a, bool large, hipStream_t s) {
+  const int edge = large ? 128 : 64;
+  a.tiles_m = (a.M + edge - 1) / edge;
+  a.tiles_n = (a.N + edge - 1) / edge;
+  a.total = a.tiles_m * a.tiles_n * a.problems * a.splits;
+  const dim3 grid((unsigned)(8 * ((a.total + 7) / 8)));
+  if (large) hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 128, 128>), grid, dim3(kLinearThreads), 0, s, a);
+  else hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 64, 64>), grid, dim3(kLinearThreads), 0, s, a);
+}
+
+}  // namespace rglru
+
+using namespace rglru;
+
+extern "C" {
+
+int64_t rglru_hip_linear_splits(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return linear_plan(kind, M, N, K, problems, dtype).splits;
+}
+
+int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
+                     const void* bias0, const void* bias1, const uint8_t* active, void* c0, void* c1, int64_t ldc,
+                     float* partial, float* colsum, int64_t M, int64_t N, int64_t K, int dtype, void* stream) {
+  if (dtype != RGLRU_F32 && dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "linear: dtype must be RGLRU_F32 or RGLRU_BF16, got %d", dtype);
+  if (kind < RGLRU_LINEAR_FORWARD || kind > RGLRU_LINEAR_WEIGHT_GRAD) return fail(RGLRU_E_ARG, "linear: unknown kind %d", kind);
+  if (M <= 0 || N <= 0 || K <= 0) return fail(RGLRU_E_ARG, "linear: empty product %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
+  LinearArgs a;
+  memset(&a, 0, sizeof(a));
+  a.a[0] = a0; a.a[1] = a1; a.b[0] = b0; a.b[1] = b1; a.bias[0] = bias0; a.bias[1] = bias1; a.c[0] = c0; a.c[1] = c1;
+  a.active = active; a.colsum = colsum; a.lda = lda; a.ldb = ldb; a.ldc = ldc;
+  a.problems = kind == RGLRU_LINEAR_FORWARD ? (b1 ? 2 : 1) : kind == RGLRU_LINEAR_WEIGHT_GRAD ? (a1 ? 2 : 1) : 1;
+  a.segments = kind == RGLRU_LINEAR_INPUT_GRAD && a1 ? 2 : 1;
+  const LinearPlan plan = linear_plan(kind, M, N, K, a.problems, dtype);
+  a.splits = plan.splits;
+  if (plan.splits > 1) a.partial = partial;
+  if (!a0 || !b0 || (a.segments == 2 && !b1) || (plan.splits > 1 ? !partial : (!c0 || (a.problems == 2 && !c1)))) return fail(RGLRU_E_ARG, "linear: null pointer");
+  const int64_t es = dtype == RGLRU_BF16 ? 2 : 4, vec = 16 / es;
+  const bool ta = kind == RGLRU_LINEAR_WEIGHT_GRAD, tb = kind != RGLRU_LINEAR_FORWARD;
+  // rows of whole 16-byte vectors on a 16-byte boundary: what every load and store of the kernel is
+  const void* ptrs[] = {a0, a1, b0, b1, a.partial ? nullptr : c0, a.partial ? nullptr : c1};
+  for (const void* q : ptrs) if ((uintptr_t)q % 16) return fail(RGLRU_E_UNSUPPORTED, "linear: operands must be 16-byte aligned");
+  if ((lda % vec) || (ldb % vec) || (!a.partial && ldc % vec) || (ta ? M : K) % vec || N % vec || (!tb && K % vec))
+    return fail(RGLRU_E_UNSUPPORTED, "linear: rows must be whole 16-byte vectors");
+  if (lda < (ta ? M : K) || ldb < (tb ? N : K) || (!a.partial && ldc < N)) return fail(RGLRU_E_ARG, "linear: a row stride is smaller than the row");
+  if (M >= (1ll << 30) || N >= (1ll << 24) || K >= (1ll << 30) || lda >= (1 << 22) || ldb >= (1 << 22) || ldc >= (1 << 22) ||
+      ((M + 63) / 64) * ((N + 63) / 64) * a.problems * a.splits >= (1ll << 30))
+    return fail(RGLRU_E_UNSUPPORTED, "linear: product too large");
+  a.M = (int)M; a.N = (int)N; a.K = (int)K;
+  const int64_t bk = dtype == RGLRU_BF16 ? 64 : 32;
+  a.k_per_split = (int)(((K + a.splits - 1) / a.splits + bk - 1) / bk * bk);
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == RGLRU_BF16) {
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, plan.large, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<__bf16, false, true>(a, plan.large, s);
+    else linear_launch<__bf16, true, true>(a, plan.large, s);
+  } else {
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, plan.large, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, plan.large, s);
+    else linear_launch<float, true, true>(a, plan.large, s);
+  }
+  return check_launch("linear");
+}
+
+}  // extern "C"

@@ -7,6 +7,7 @@
 //
 // Errors follow the reference's operator module (griffin/triton_scan.py:213-224): RuntimeError for a missing GPU,
 // ValueError for shapes, TypeError for types.
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
@@ -82,6 +83,28 @@ Tensor fresh_like(const Tensor& t) { return fresh(t.sizes(), t.scalar_type(), t)
 Tensor bytes(size_t n, const Tensor& like) { return fresh({static_cast<int64_t>(n)}, at::kByte, like); }
 
 size_t round_up(size_t n) { return (n + 255) & ~size_t(255); }
+
+// A contiguous tensor over part of a buffer's storage, `at` bytes in.  An allocation (and its release) costs the host a
+// microsecond and more; a tensor over memory that is there, a fraction of one.
+Tensor part(const Tensor& buffer, size_t at, at::IntArrayRef size, at::ScalarType dtype) {
+  Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(buffer.storage()), c10::DispatchKeySet(c10::DispatchKey::CUDA),
+                                                      c10::scalarTypeToTypeMeta(dtype));
+  t.unsafeGetTensorImpl()->set_storage_offset(static_cast<int64_t>(at / c10::elementSize(dtype)));
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(size);
+  return t;
+}
+
+// Tensors that live as long as each other, as parts of one allocation: first their sizes, then the memory, then the tensors
+// in the same order.
+struct Parts {
+  std::vector<size_t> offsets;
+  size_t total = 0, next = 0;
+  Tensor buffer;
+  void add(size_t n) { offsets.push_back(total), total += round_up(n); }
+  void allocate(const Tensor& like) { buffer = bytes(total, like); }
+  char* raw() { return static_cast<char*>(buffer.data_ptr()) + offsets[next++]; }
+  Tensor take(at::IntArrayRef size, at::ScalarType dtype) { return part(buffer, offsets[next++], size, dtype); }
+};
 
 // Contiguous and on a 16-byte boundary (what every fresh allocation is): a view at an odd offset costs one copy
 // instead of sending the whole call to the portable kernels, which are several times slower.
@@ -244,11 +267,14 @@ ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Te
   if (!known(gt)) gt = at::kFloat;
   const int gcode = code_of(gt);
   g.dx = fresh_like(x);
-  g.dw_a = fresh({nb, bw, bw}, gt, x);
-  g.dw_x = fresh({nb, bw, bw}, gt, x);
-  g.db_a = fresh({nb, bw}, gt, x);
-  g.db_x = fresh({nb, bw}, gt, x);
-  g.dlam = fresh({W}, gt, x);
+  {
+    const size_t gs = c10::elementSize(gt);
+    Parts parts;
+    parts.add(W * bw * gs), parts.add(W * bw * gs), parts.add(W * gs), parts.add(W * gs), parts.add(W * gs);
+    parts.allocate(x);
+    g.dw_a = parts.take({nb, bw, bw}, gt), g.dw_x = parts.take({nb, bw, bw}, gt);
+    g.db_a = parts.take({nb, bw}, gt), g.db_x = parts.take({nb, bw}, gt), g.dlam = parts.take({W}, gt);
+  }
   if (need_dh0) g.dh0 = fresh({B, W}, at::kFloat, x);
   void* stream = stream_of(x);
   const uint8_t* fl = flags_ptr(flags, first_reset);
@@ -991,6 +1017,65 @@ Tensor sum_sets(const Tensor& sets) {
   return out;
 }
 
+// Whether products of `macs` multiply-adds each (tokens x width x model width) run on the library's own kernels.  The BLAS
+// library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us, a step of
+// the block has seven, and below the line the step is over before the host has issued it: in bf16 about 8192 tokens of
+// 768 -> 1024.  Inside a captured graph host time is nothing: there the line lies where the kernels take equally long.
+bool own_products(double macs, at::ScalarType dtype) {
+  if (!known(dtype)) return false;
+  const bool bf16 = dtype == at::kBFloat16;
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < (bf16 ? 2e9 : 4e8);
+  return macs < (bf16 ? 6e9 : 9e8);
+}
+
+// Contiguous rows of whole 16-byte vectors, as rglru_hip_linear takes them.
+bool vector_rows(const Tensor& t) {
+  return t.is_contiguous() && (t.size(-1) * t.element_size()) % 16 == 0 && is_aligned(t);
+}
+
+// Whether the library takes y = x w^T + b (and its gradients) for these operands.
+bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b) {
+  const auto dtype = x.scalar_type();
+  return w.dim() == 2 && x.size(-1) == w.size(1) && w.scalar_type() == dtype && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
+         x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype) && vector_rows(w) && vector_rows(x) &&
+         (w.size(0) * x.element_size()) % 16 == 0 && !at::autocast::is_autocast_enabled(at::kCUDA);
+}
+
+void linear_forward(const Tensor& x, const Tensor& w0, const Tensor& b0, const Tensor& w1, const Tensor& b1, const Tensor& active, void* y0,
+                    void* y1) {
+  const int64_t K = x.size(-1), N = w0.size(0);
+  check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, ptr(x), nullptr, K, ptr(w0), ptr(w1), K, ptr(b0), ptr(b1), bptr(active), y0, y1, N,
+                         nullptr, nullptr, x.numel() / K, N, K, code_of(x.scalar_type()), stream_of(x)), "rglru_hip_linear");
+}
+
+// Weight and bias gradients of one or two Linear layers on one input x [rows, K]: dy_i [rows, N], rows `ld` elements apart.
+struct WeightGrad {
+  int64_t splits, sets_bytes, sums_bytes, N, K, problems;
+  WeightGrad(int64_t rows, int64_t n, int64_t k, int64_t n_problems, at::ScalarType dtype) : N(n), K(k), problems(n_problems) {
+    splits = rglru_hip_linear_splits(RGLRU_LINEAR_WEIGHT_GRAD, N, K, rows, problems, code_of(dtype));
+    sets_bytes = splits > 1 ? splits * problems * N * K * 4 : 0;
+    sums_bytes = splits * problems * N * 4;
+  }
+  // dw (problems x N x K, contiguous) is written here where nothing is left to add up
+  void run(const void* dy0, const void* dy1, int64_t ld, const void* x, const uint8_t* active, void* dw, void* sets, void* sums,
+           int64_t rows, at::ScalarType dtype, void* stream) const {
+    char* second = problems == 2 ? static_cast<char*>(dw) + N * K * c10::elementSize(dtype) : nullptr;
+    check(rglru_hip_linear(RGLRU_LINEAR_WEIGHT_GRAD, dy0, dy1, ld, x, nullptr, K, nullptr, nullptr, active, dw, second, K,
+                           static_cast<float*>(sets), static_cast<float*>(sums), N, K, rows, code_of(dtype), stream), "rglru_hip_linear");
+  }
+  rglru_sum weight_sum(void* sets, void* dw) const { return {sets, splits > 1 ? dw : nullptr, splits, problems * N * K, RGLRU_F32}; }
+  rglru_sum bias_sum(void* sums, void* db) const { return {sums, db, splits, problems * N, RGLRU_F32}; }
+};
+
+// dW = dy^T x contracts over all tokens: one GEMM of the BLAS library with K = rows runs at a fraction of the rate of the same
+// work as a batch of GEMMs with K = 2048 whose results are added (100 us against 43 us for 16384 x 1024 x 768 in bf16), so
+// long contractions are split into this many.
+int64_t contraction_chunks(int64_t rows) {
+  int64_t chunks = rows % 2048 == 0 ? rows / 2048 : 1;
+  while (chunks > 16 && chunks % 2 == 0) chunks /= 2;
+  return chunks;
+}
+
 // (dW, db) of y = x W^T + b for the incoming dy; bias_type kNone skips db.
 std::tuple<Tensor, Tensor> linear_parameter_grads(const Tensor& x, at::ScalarType weight_type, const Tensor& dy, bool need_w, int64_t bias_type) {
   Tensor dy2 = dy.reshape({-1, dy.size(-1)});
@@ -998,11 +1083,7 @@ std::tuple<Tensor, Tensor> linear_parameter_grads(const Tensor& x, at::ScalarTyp
   const int64_t rows = dy2.size(0), width = dy2.size(1);
   if (need_w) {
     Tensor x2 = x.reshape({-1, x.size(-1)}).to(dy.scalar_type());
-    // dW = dy^T x contracts over all tokens: one GEMM with K = rows runs at a fraction of the rate of the same work as
-    // a batch of GEMMs with K = 2048 whose results are added (100 us against 43 us for 16384 x 1024 x 768 in bf16 on
-    // this library), so long contractions are split
-    int64_t chunks = (rows % 2048 == 0 && dy2.is_contiguous() && x2.is_contiguous()) ? rows / 2048 : 1;
-    while (chunks > 16 && chunks % 2 == 0) chunks /= 2;
+    const int64_t chunks = dy2.is_contiguous() && x2.is_contiguous() ? contraction_chunks(rows) : 1;
     if (chunks > 1) {
       const int64_t per = rows / chunks;
       dw = sum_sets(at::bmm(dy2.view({chunks, per, width}).transpose(1, 2), x2.view({chunks, per, x2.size(1)})));
@@ -1042,8 +1123,19 @@ struct Linear : torch::autograd::Function<Linear> {
     ctx->save_for_backward({x, weight, opt(active)});
     note_arguments(ctx, {true, true, bias.has_value()});
     pack(ctx, {type_or_none(opt(bias))});
-    Tensor y = at::linear(x, weight, bias);
-    return active.has_value() ? masked_rows(y, *active, true) : y;
+    return values(x, weight, opt(bias), opt(active));
+  }
+  static Tensor values(const Tensor& x, const Tensor& weight, const Tensor& bias, const Tensor& active) {
+    if (own_linear(x, weight, bias)) {
+      c10::DeviceGuard guard(x.device());
+      at::DimVector size(x.sizes());
+      size.back() = weight.size(0);
+      Tensor y = fresh(size, x.scalar_type(), x);
+      linear_forward(x, weight, bias, Tensor(), Tensor(), active, ptr(y), nullptr);
+      return y;
+    }
+    Tensor y = at::linear(x, weight, maybe(bias));
+    return active.defined() ? masked_rows(y, active, true) : y;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     auto s = ctx->get_saved_variables();
@@ -1051,13 +1143,45 @@ struct Linear : torch::autograd::Function<Linear> {
     {
       at::NoGradGuard no_grad;
       const Tensor &x = s[0], &weight = s[1];
-      Tensor dy = s[2].defined() ? masked_rows(grads[0], s[2], false) : grads[0];
       c10::DeviceGuard guard(x.device());
       Needs need(ctx);
+      const int64_t bias_type = unpack(ctx)[0];
+      if (own_linear(x, weight, Tensor()) && grads[0].scalar_type() == x.scalar_type() && (bias_type == kNone || bias_type == (int64_t)x.scalar_type())) {
+        std::tie(dx, dw, db) = own_backward(x, weight, grads[0], s[2], need(0), need(1), need(2));
+        return once({dx, dw, db, Tensor()});
+      }
+      Tensor dy = s[2].defined() ? masked_rows(grads[0], s[2], false) : grads[0];
       if (need(0)) dx = at::matmul(dy, weight.to(dy.scalar_type()));
-      std::tie(dw, db) = linear_parameter_grads(x, weight.scalar_type(), dy, need(1), need(2) ? unpack(ctx)[0] : kNone);
+      std::tie(dw, db) = linear_parameter_grads(x, weight.scalar_type(), dy, need(1), need(2) ? bias_type : kNone);
     }
     return once({dx, dw, db, Tensor()});
+  }
+  static std::tuple<Tensor, Tensor, Tensor> own_backward(const Tensor& x, const Tensor& weight, const Tensor& dy_in, const Tensor& active,
+                                                         bool need_x, bool need_w, bool need_b) {
+    const auto dtype = x.scalar_type();
+    Tensor dy = aligned(dy_in), dx, dw, db;
+    const int64_t K = x.size(-1), N = weight.size(0), rows = x.numel() / K;
+    void* stream = stream_of(x);
+    if (need_x) {
+      dx = fresh_like(x);
+      check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, ptr(dy), nullptr, N, ptr(weight), nullptr, K, nullptr, nullptr, bptr(active), ptr(dx), nullptr,
+                             K, nullptr, nullptr, rows, K, N, code_of(dtype), stream), "rglru_hip_linear");
+    }
+    if (need_w || need_b) {
+      const WeightGrad wg(rows, N, K, 1, dtype);
+      Parts out, scratch;
+      out.add(N * K * x.element_size()), out.add(N * x.element_size());
+      scratch.add(wg.sets_bytes), scratch.add(wg.sums_bytes);
+      out.allocate(x), scratch.allocate(x);
+      dw = out.take({N, K}, dtype), db = out.take({N}, dtype);
+      char *sets = scratch.raw(), *sums = scratch.raw();
+      wg.run(ptr(dy), nullptr, N, ptr(x), bptr(active), ptr(dw), sets, sums, rows, dtype, stream);
+      const rglru_sum jobs[] = {wg.weight_sum(sets, ptr(dw)), wg.bias_sum(sums, ptr(db))};
+      check(rglru_hip_sums(jobs, 2, code_of(dtype), stream), "rglru_hip_sums");
+      if (!need_w) dw = Tensor();
+      if (!need_b) db = Tensor();
+    }
+    return {dx, dw, db};
   }
 };
 
@@ -1098,7 +1222,20 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
     note_arguments(ctx, {true, true, b1.has_value(), true, b2.has_value()});
     pack(ctx, {type_or_none(opt(b1)), type_or_none(opt(b2))});
     ctx->set_materialize_grads(false);
-    return {at::linear(x, w1, b1), at::linear(x, w2, b2)};
+    auto [u, v] = values(x, w1, opt(b1), w2, opt(b2));
+    return {u, v};
+  }
+  static bool own(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
+    return own_linear(x, w1, b1) && own_linear(x, w2, b2) && w1.sizes() == w2.sizes() && b1.defined() == b2.defined();
+  }
+  static std::tuple<Tensor, Tensor> values(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
+    if (!own(x, w1, b1, w2, b2)) return {at::linear(x, w1, maybe(b1)), at::linear(x, w2, maybe(b2))};
+    c10::DeviceGuard guard(x.device());
+    at::DimVector size(x.sizes());
+    size.back() = w1.size(0);
+    Tensor u = fresh(size, x.scalar_type(), x), v = fresh(size, x.scalar_type(), x);
+    linear_forward(x, w1, b1, w2, b2, Tensor(), ptr(u), ptr(v));
+    return {u, v};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     auto s = ctx->get_saved_variables();
@@ -1111,7 +1248,39 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
       at::NoGradGuard no_grad;
       c10::DeviceGuard guard(x.device());
       Tensor both = stacked_halves(grads[0], grads[1]);
-      if (both.defined() && w1.scalar_type() == w2.scalar_type() && w1.sizes() == w2.sizes() && need_w1 == need_w2 &&
+      const auto dtype = x.scalar_type();
+      auto usual = [&](int64_t t) { return t == kNone || t == (int64_t)dtype; };
+      if (grads[0].defined() && grads[1].defined() && grads[0].scalar_type() == dtype && grads[1].scalar_type() == dtype &&
+          own(x, w1, Tensor(), w2, Tensor()) && usual(m[0]) && usual(m[1])) {
+        Tensor g0 = grads[0], g1 = grads[1];
+        const int64_t N = w1.size(0), K = w1.size(1), rows = x.numel() / K;
+        const int64_t ld = both.defined() ? 2 * N : N;
+        if (!both.defined() || !is_aligned(g0)) g0 = aligned(g0), g1 = aligned(g1);
+        void* stream = stream_of(x);
+        const int code = code_of(dtype);
+        if (need_x) {
+          dx = fresh_like(x);
+          check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, ptr(g0), ptr(g1), ld, ptr(w1), ptr(w2), K, nullptr, nullptr, nullptr, ptr(dx), nullptr,
+                                 K, nullptr, nullptr, rows, K, N, code, stream), "rglru_hip_linear");
+        }
+        if (need_w1 || need_w2 || need_b1 || need_b2) {
+          const WeightGrad wg(rows, N, K, 2, dtype);
+          Parts out, scratch;
+          out.add(2 * N * K * x.element_size()), out.add(2 * N * x.element_size());
+          scratch.add(wg.sets_bytes), scratch.add(wg.sums_bytes);
+          out.allocate(x), scratch.allocate(x);
+          Tensor dw = out.take({2, N, K}, dtype), db = out.take({2, N}, dtype);
+          char *sets = scratch.raw(), *sums = scratch.raw();
+          wg.run(ptr(g0), ptr(g1), ld, ptr(x), nullptr, ptr(dw), sets, sums, rows, dtype, stream);
+          const rglru_sum jobs[] = {wg.weight_sum(sets, ptr(dw)), wg.bias_sum(sums, ptr(db))};
+          check(rglru_hip_sums(jobs, 2, code, stream), "rglru_hip_sums");
+          const size_t at_b = round_up(2 * N * K * x.element_size()), row = N * x.element_size();
+          if (need_w1) dw1 = part(out.buffer, 0, {N, K}, dtype);
+          if (need_w2) dw2 = part(out.buffer, N * K * x.element_size(), {N, K}, dtype);
+          if (need_b1) db1 = part(out.buffer, at_b, {N}, dtype);
+          if (need_b2) db2 = part(out.buffer, at_b + row, {N}, dtype);
+        }
+      } else if (both.defined() && w1.scalar_type() == w2.scalar_type() && w1.sizes() == w2.sizes() && need_w1 == need_w2 &&
           need_b1 == need_b2 && m[0] == m[1]) {
         // The halves of one matrix (the block's backward writes them so): one GEMM for dx against the stacked weights,
         // one for both weight gradients, one column sum.  At 16384 rows, 768 -> 2 x 1024: 49 against 65 us (dx), 60
@@ -1140,12 +1309,199 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
   }
 };
 
+// The values alone, without a graph.
+std::tuple<Tensor, Tensor> linear_pair_values(const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2, const MaybeTensor& b2) {
+  at::NoGradGuard no_grad;
+  return LinearPair::values(x, w1, opt(b1), w2, opt(b2));
+}
+
 std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const MaybeTensor& b1_, const Tensor& w2, const MaybeTensor& b2_) {
   Tensor b1 = opt(b1_), b2 = opt(b2_);
   require_gpu("hip_linear_pair", {&x, &w1, &b1, &w2, &b2});
   code_of(x.scalar_type());
   auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2));
   return {out[0], out[1]};
+}
+
+// ---- the whole block in training (griffin/griffin.py:459-528 without cache) ----------------------------------------
+
+// One node for projections, convolution, RG-LRU, output gate and output projection, so that a step costs the host one pass
+// of the engine, three allocations each way and the launches; the last sums of all parameter gradients are one launch.  bf16
+// throughout, every row a document from its beginning or right-padded (rows, active).
+struct BlockTrain : torch::autograd::Function<BlockTrain> {
+  static constexpr at::ScalarType kType = at::kBFloat16;
+  enum { X, WX, BX, WY, BY, CW, CB, WA, BA, WI, BI, LAM, WO, BO, kTensors };
+
+  // what the forward keeps: x_conv, y, gated, then the parameter image with the workspace; u and v in front where it made them
+  struct Saved {
+    size_t tensor_bytes;
+    char* at;
+    Saved(const Tensor& buffer, int64_t M, int64_t W) : tensor_bytes(round_up(M * W * 2)), at(static_cast<char*>(buffer.data_ptr())) {}
+    char* operator[](int i) const { return at + i * tensor_bytes; }
+  };
+
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& wx, const Tensor& bx, const Tensor& wy, const Tensor& by,
+                        const Tensor& cw, const Tensor& cb, const Tensor& wa, const Tensor& ba, const Tensor& wi, const Tensor& bi,
+                        const Tensor& lam, const Tensor& wo, const Tensor& bo, const Tensor& pos, const MaybeTensor& flags_,
+                        const MaybeTensor& rows_, const MaybeTensor& active_, const MaybeTensor& u_, const MaybeTensor& v_, bool first_reset,
+                        double c) {
+    Tensor flags = opt(flags_), rows = opt(rows_), active = opt(active_), u = opt(u_), v = opt(v_);
+    c10::DeviceGuard guard(x.device());
+    const int64_t B = x.size(0), T = x.size(1), D = x.size(2), W = wx.size(0), K = cw.size(2), nb = wa.size(0), M = B * T;
+    void* stream = stream_of(x);
+    const size_t image_bytes = round_up(prep_bytes(W, nb, RGLRU_BF16));
+    const size_t tensor_bytes = round_up(M * W * 2);
+    const int own = u.defined() ? 3 : 5;
+    Tensor buffer = bytes(own * tensor_bytes + image_bytes + rglru_hip_workspace_bytes(B, T, W, nb), x);
+    Saved s(buffer, M, W);
+    if (!first_reset && !flags.defined()) flags = block_flags(pos);
+    if (!u.defined()) {
+      if (own_linear(x, wx, bx)) {
+        linear_forward(x, wx, bx, wy, by, Tensor(), s[3], s[4]);
+      } else {
+        Tensor x2 = x.view({M, D});
+        Tensor out_u = part(buffer, 3 * tensor_bytes, {M, W}, kType), out_v = part(buffer, 4 * tensor_bytes, {M, W}, kType);
+        at::addmm_out(out_u, bx, x2, wx.t());
+        at::addmm_out(out_v, by, x2, wy.t());
+      }
+    }
+    void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
+    char *image = s[own], *ws = image + image_bytes;
+    check(rglru_hip_prepare_block_fwd(ptr(wa), ptr(ba), ptr(wi), ptr(bi), ptr(lam), static_cast<float>(c), RGLRU_BF16, image, up, W, vp, W,
+                                      nullptr, ptr(cw), ptr(cb), K, nullptr, flags_ptr(flags, first_reset), s[0], s[1], s[2], nullptr,
+                                      nullptr, ws, B, T, W, nb, RGLRU_BF16, stream), "rglru_hip_prepare_block_fwd");
+    Tensor out;
+    if (own_linear(x, wx, bx)) {
+      out = fresh_like(x);
+      check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, s[2], nullptr, W, ptr(wo), nullptr, W, ptr(bo), nullptr, bptr(active), ptr(out), nullptr, D,
+                             nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
+    } else {
+      out = at::linear(part(buffer, 2 * tensor_bytes, {B, T, W}, kType), wo, bo);
+      if (active.defined()) masked_rows(out, active, true);
+    }
+    ctx->save_for_backward({x, wx, wy, wo, cw, pos, flags, rows, active, u, v, buffer});
+    pack(ctx, {first_reset, nb});
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    auto saved = ctx->get_saved_variables();
+    auto m = unpack(ctx);
+    const Tensor &x = saved[0], &wx = saved[1], &wy = saved[2], &wo = saved[3], &cw = saved[4], &pos = saved[5], &flags = saved[6],
+                 &rows = saved[7], &active = saved[8], &u = saved[9], &v = saved[10], &buffer = saved[11];
+    const bool first_reset = m[0];
+    const int64_t nb = m[1];
+    variable_list g(22);
+    {
+      at::NoGradGuard no_grad;
+      c10::DeviceGuard guard(x.device());
+      const int64_t B = x.size(0), T = x.size(1), D = x.size(2), W = wx.size(0), K = cw.size(2), bw = W / nb, M = B * T;
+      void* stream = stream_of(x);
+      Saved s(buffer, M, W);
+      void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
+      char *image = s[u.defined() ? 3 : 5], *ws = image + round_up(prep_bytes(W, nb, RGLRU_BF16));
+      Tensor dy = aligned(grads[0].to(kType));
+      const bool own = own_linear(x, wx, Tensor());
+      if (!own && active.defined()) dy = masked_rows(dy, active, false);
+
+      // parameter gradients: parts of one allocation
+      Parts out;
+      for (int64_t n : {2 * W * D, 2 * W, W * K, W, W * bw, W, W * bw, W, W, D * W, D}) out.add(n * 2);
+      out.allocate(x);
+      Tensor dw_pair = out.take({2, W, D}, kType), db_pair = out.take({2, W}, kType);
+      g[CW] = out.take({W, 1, K}, kType), g[CB] = out.take({W}, kType);
+      g[WA] = out.take({nb, bw, bw}, kType), g[BA] = out.take({nb, bw}, kType), g[WI] = out.take({nb, bw, bw}, kType), g[BI] = out.take({nb, bw}, kType);
+      g[LAM] = out.take({W}, kType);
+      g[WO] = out.take({D, W}, kType), g[BO] = out.take({D}, kType);
+      g[WX] = part(out.buffer, out.offsets[0], {W, D}, kType), g[WY] = part(out.buffer, out.offsets[0] + W * D * 2, {W, D}, kType);
+      g[BX] = part(out.buffer, out.offsets[1], {W}, kType), g[BY] = part(out.buffer, out.offsets[1] + W * 2, {W}, kType);
+
+      const WeightGrad go(M, D, W, 1, kType), gp(M, W, D, 2, kType);
+      const size_t column_bytes_o = rglru_hip_colsum_scratch_bytes(M, D), column_bytes_p = rglru_hip_colsum_scratch_bytes(M, 2 * W);
+      Parts scratch;
+      scratch.add(M * W * 2), scratch.add(2 * M * W * 2);
+      scratch.add(rglru_hip_bwd_scratch_bytes(B, T, W, nb, RGLRU_BF16)), scratch.add(rglru_hip_conv_scratch_bytes(B, T, W, K));
+      scratch.add(own ? go.sets_bytes : 0), scratch.add(own ? go.sums_bytes : column_bytes_o);
+      scratch.add(own ? gp.sets_bytes : 0), scratch.add(own ? gp.sums_bytes : column_bytes_p);
+      scratch.allocate(x);
+      char *dgated = scratch.raw(), *du = scratch.raw(), *gate_scratch = scratch.raw(), *conv_scratch = scratch.raw(), *sets_o = scratch.raw(),
+           *sums_o = scratch.raw(), *sets_p = scratch.raw(), *sums_p = scratch.raw();
+      char* dv = du + W * 2;                               // the halves of one [M, 2 W] matrix
+      rglru_sum sums[4];
+      Tensor held_o, held_p;                               // results of the BLAS library that the last launch reads
+
+      // output projection
+      if (own) {
+        go.run(ptr(dy), nullptr, D, s[2], bptr(active), ptr(g[WO]), sets_o, sums_o, M, kType, stream);
+        check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, ptr(dy), nullptr, D, ptr(wo), nullptr, W, nullptr, nullptr, bptr(active), dgated, nullptr, W,
+                               nullptr, nullptr, M, W, D, RGLRU_BF16, stream), "rglru_hip_linear");
+        sums[0] = go.weight_sum(sets_o, ptr(g[WO])), sums[1] = go.bias_sum(sums_o, ptr(g[BO]));
+      } else {
+        Tensor dy2 = dy.view({M, D});
+        Tensor dg = part(scratch.buffer, scratch.offsets[0], {M, W}, kType);
+        at::mm_out(dg, dy2, wo);
+        held_o = contraction(dy2, part(buffer, 2 * s.tensor_bytes, {M, W}, kType));
+        check(rglru_hip_colsum(ptr(dy), sums_o, nullptr, M, D, RGLRU_BF16, RGLRU_BF16, stream), "rglru_hip_colsum");
+        sums[0] = {ptr(held_o), ptr(g[WO]), held_o.size(0), D * W, RGLRU_BF16};
+        sums[1] = {sums_o, ptr(g[BO]), int64_t(column_bytes_o / (4 * D)), D, RGLRU_F32};
+      }
+      check(rglru_hip_block_bwd(dgated, s[1], up, vp, s[0], image, ptr(cw), iptr(pos), static_cast<const int32_t*>(ptr(rows)),
+                                flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, du, dv, 2 * W, B, T, W, nb, K, stream),
+            "rglru_hip_block_bwd");
+      // input projections
+      const bool need_x = ctx->needs_input_grad(0);
+      if (own) {
+        if (need_x) {
+          g[X] = fresh_like(x);
+          check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, du, dv, 2 * W, ptr(wx), ptr(wy), D, nullptr, nullptr, nullptr, ptr(g[X]), nullptr, D,
+                                 nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
+        }
+        gp.run(du, dv, 2 * W, ptr(x), nullptr, ptr(dw_pair), sets_p, sums_p, M, kType, stream);
+        sums[2] = gp.weight_sum(sets_p, ptr(dw_pair)), sums[3] = gp.bias_sum(sums_p, ptr(db_pair));
+      } else {
+        Tensor both = part(scratch.buffer, scratch.offsets[1], {M, 2 * W}, kType);
+        if (need_x) g[X] = at::mm(both, at::cat({wx, wy})).view(x.sizes());
+        held_p = contraction(both, x.view({M, D}));
+        check(rglru_hip_colsum(du, sums_p, nullptr, M, 2 * W, RGLRU_BF16, RGLRU_BF16, stream), "rglru_hip_colsum");
+        sums[2] = {ptr(held_p), ptr(dw_pair), held_p.size(0), 2 * W * D, RGLRU_BF16};
+        sums[3] = {sums_p, ptr(db_pair), int64_t(column_bytes_p / (8 * W)), 2 * W, RGLRU_F32};
+      }
+      check(rglru_hip_block_finish(image, gate_scratch, conv_scratch, ptr(g[WA]), ptr(g[WI]), ptr(g[BA]), ptr(g[BI]), ptr(g[LAM]), ptr(g[CW]),
+                                   ptr(g[CB]), sums, 4, B, T, W, nb, K, stream), "rglru_hip_block_finish");
+      for (int i = 1; i < kTensors; ++i)
+        if (!ctx->needs_input_grad(i)) g[i] = Tensor();
+    }
+    return once(std::move(g));
+  }
+
+  // a^T b over the rows, as the partial products [chunks, columns of a, columns of b] of the BLAS library
+  static Tensor contraction(const Tensor& a, const Tensor& b) {
+    const int64_t rows = a.size(0), chunks = contraction_chunks(rows), per = rows / chunks;
+    if (chunks == 1) return at::mm(a.t(), b).unsqueeze(0);
+    return at::bmm(a.view({chunks, per, a.size(1)}).transpose(1, 2), b.view({chunks, per, b.size(1)}));
+  }
+};
+
+// Nothing is returned where the node does not take the operands; the caller then goes layer by layer.
+MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const MaybeTensor& flags, const MaybeTensor& rows,
+                        const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
+  typedef BlockTrain N;
+  const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
+  for (const Tensor& t : p)
+    if (t.scalar_type() != N::kType || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
+  // p: the node's tensors behind x
+  const Tensor &wx = p[N::WX - 1], &wy = p[N::WY - 1], &wo = p[N::WO - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
+  const int64_t W = wx.size(0);
+  if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 || wx.dim() != 2 || wx.size(1) != D || wy.sizes() != wx.sizes() ||
+      wo.dim() != 2 || wo.size(0) != D || wo.size(1) != W || cw.dim() != 3 || cw.size(0) != W || wa.dim() != 3 || wa.size(0) * wa.size(1) != W ||
+      (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
+    return std::nullopt;
+  MaybeTensor live;
+  if (active.has_value()) live = active->contiguous();
+  Tensor positions = pos.to(at::kLong).contiguous();
+  auto contiguous = [](const MaybeTensor& t) { return t.has_value() ? MaybeTensor(aligned(*t)) : t; };
+  return BlockTrain::apply(x, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11], p[12], positions, flags, rows, live,
+                           contiguous(u), contiguous(v), first_reset, c);
 }
 
 // ---- RMSNorm (griffin/griffin.py:68-80) ---------------------------------------------------------------------------
@@ -1237,6 +1593,8 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(stacked_halves);
   EXPORT(linear);
   EXPORT(linear_pair);
+  EXPORT(linear_pair_values);
+  EXPORT(block_train);
   EXPORT(rmsnorm);
 #undef EXPORT
 }

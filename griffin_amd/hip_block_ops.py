@@ -78,7 +78,7 @@ def hip_block_flags(segment_pos: Tensor) -> Tensor:
 
 def hip_block_forward(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: Tensor, bias: Tensor | None,
                       segment_pos: Tensor, flags: Tensor | None, w_a: Tensor, b_a: Tensor, w_x: Tensor, b_x: Tensor,
-                      lam: Tensor, h0: Tensor | None, c: float = 8.0, prep=None, rows: Tensor | None = None, need_state: bool = True):
+                      lam: Tensor, h0: Tensor | None, c: float = 8.0, prep=None, rows: Tensor | None = None, need_state: bool = True, around=None):
     """``gelu_tanh(v) * RG_LRU(conv(u))`` for whole sequences with every token active, one forward launch.
 
     ``u``, ``v`` [B, T, W]: the block's two projections; ``conv_state`` [B, K-1, W] or None; ``weight``
@@ -89,8 +89,17 @@ def hip_block_forward(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: T
     conv_positions and flags of ``token_facts``; the new convolution state then carries no gradient and is computed only
     if ``need_state``.  Returns ``(gated [B, T, W], final state [B, W] fp32, new_conv_state
     [B, K-1, W])``; differentiable in u, v, the parameters, conv_state and h0.
+
+    ``around``: (x [B, T, D], the weights and biases of linear_x, linear_y and linear_out, activity mask or None) puts the Linear
+    layers into the operator: the whole block of a training step without cache, one node of the graph.  u and v are then None,
+    or the projections of x if the caller has them already (``hip_linear_pair_values``).  Returns ``(output [B, T, D], None,
+    None)``; the output is None where the node does not take the operands (the caller then goes layer by layer).
     """
     first_reset = flags is FIRST_TOKEN_RESET
+    if around is not None:
+        x, w_u, b_u, w_v, b_v, w_o, b_o, active = around
+        return _lib.native().block_train(x, (w_u, b_u, w_v, b_v, weight, bias, w_a, b_a, w_x, b_x, lam, w_o, b_o), segment_pos,
+                                         None if first_reset else flags, rows, active, u, v, first_reset, c), None, None
     gated, h_last, new_conv = _lib.native().block_forward(
         u, v, conv_state, weight, bias, segment_pos, None if first_reset else flags, first_reset, w_a, b_a, w_x, b_x, lam, h0,
         c, None if prep is None else prep.image, rows, need_state)
@@ -165,6 +174,11 @@ def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Te
     """``(x @ w1.T + b1, x @ w2.T + b2)``: two ``hip_linear`` calls whose backward passes share the input
     gradient (the second GEMM accumulates into the first one's result)."""
     return _lib.native().linear_pair(x, w1, b1, w2, b2)
+
+
+def hip_linear_pair_values(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None) -> tuple[Tensor, Tensor]:
+    """The values of ``hip_linear_pair`` without a graph behind them."""
+    return _lib.native().linear_pair_values(x, w1, b1, w2, b2)
 
 
 @lru_cache(maxsize=None)

@@ -485,6 +485,62 @@ class RecurrentBlock(nn.Module):
         """Nobody wrapped or hooked the Linear layer: calling it is a product with its weight and nothing else."""
         return type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks
 
+    @staticmethod
+    def _unhooked(layer: nn.Module) -> bool:
+        return not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
+
+    def _training_parameters(self, x: Tensor):
+        """The block's parameters (linear_x, linear_y, convolution, gates, Lambda, linear_out) where one operator may stand for the
+        whole block: training in bf16 on the HIP path, nobody wrapped, hooked or replaced a layer; else None."""
+        if not torch.is_grad_enabled() or x.dtype != torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.is_autocast_enabled():
+            return None
+        lru = self.rg_lru
+        if lru.scan_mode not in ("auto", "hip", "fused") or type(lru) is not RG_LRU:
+            return None
+        try:
+            layers = self._modules
+            lx, ly, conv, lo = layers["linear_x"], layers["linear_y"], layers["temporal_conv"], layers["linear_out"]
+            if not (type(lx) is type(ly) is type(lo) is nn.Linear and type(conv) is nn.Conv1d
+                    and all(self._unhooked(m) for m in (lx, ly, conv, lo, lru))):
+                return None
+            parameters = [m._parameters[name] for m in (lx, ly, conv) for name in ("weight", "bias")]
+            parameters += lru._gate_parameters()
+            parameters += [lo._parameters["weight"], lo._parameters["bias"]]
+        except KeyError:                                     # a parametrised or otherwise replaced parameter
+            return None
+        if any(p is None or p.dtype != torch.bfloat16 for p in parameters):
+            return None
+        if not (x.requires_grad or any(p.requires_grad for p in parameters)):
+            return None
+        if not hip_block_ops.hip_block_forward_covers(self.rnn_width, parameters[6].shape[0], self.conv_kernel_size, x.dtype):
+            return None
+        if lru.scan_mode == "auto" and not hip_scan.hip_scan_is_usable(x.device):
+            return None
+        return parameters
+
+    def _train_whole(self, x: Tensor, parameters, segment_pos: Tensor | None, active_mask: Tensor | None) -> Tensor | None:
+        """The block as one operator (``around`` of hip_block_ops.hip_block_forward), or None where that does not take the
+        operands."""
+        w_u, b_u, w_v, b_v, taps, conv_bias, w_a, b_a, w_x, b_x, lam, w_o, b_o = parameters
+        u = v = rows = flags = live = None
+        if active_mask is None:
+            if segment_pos is None:
+                flags = hip_scan.FIRST_TOKEN_RESET
+            positions = _resolve_segment_positions(x, segment_pos)
+        else:
+            facts = hip_block_ops.token_facts(active_mask, segment_pos, None)
+            # queued before the facts are asked for: the answer arrives while the projections run
+            u, v = hip_block_ops.hip_linear_pair_values(x, w_u, b_u, w_v, b_v)
+            dense, right_padded = facts.resolve()
+            if dense:
+                positions = facts.positions
+            elif right_padded:
+                positions, flags, rows, live = facts.conv_positions, facts.flags, facts.rows, active_mask
+            else:
+                return None
+        return hip_block_ops.hip_block_forward(u, v, None, taps, conv_bias, positions, flags, w_a, b_a, w_x, b_x, lam, None,
+                                               self.rg_lru.c, None, rows, False, (x, w_u, b_u, w_v, b_v, w_o, b_o, live))[0]
+
     def _dense_conv(self, projected: Tensor, conv_state: Tensor | None, segment_pos: Tensor, need_state: bool = True):
         """All-tokens-active path (griffin/griffin.py:476-487): taps are masked per document."""
         if self._hip_block_ops_covers(projected):
@@ -529,6 +585,12 @@ class RecurrentBlock(nn.Module):
         previous_position = None if cache is None else cache.segment_position
         if steps == 1 and self._hip_decode_covers(x, cache):
             return self._hip_decode(x, cache, segment_pos, active_mask, return_cache)
+        if cache is None and not return_cache and steps > 0:
+            parameters = self._training_parameters(x)
+            if parameters is not None:
+                output = self._train_whole(x, parameters, segment_pos, active_mask)
+                if output is not None:
+                    return output
         facts = None
         if not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
             # launched in front of the projections, so that its answer is there before they are done

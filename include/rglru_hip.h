@@ -51,7 +51,7 @@
 extern "C" {
 #endif
 
-#define RGLRU_ABI_VERSION 20
+#define RGLRU_ABI_VERSION 21
 
 enum { RGLRU_F32 = 0, RGLRU_BF16 = 1 };
 
@@ -350,7 +350,8 @@ int rglru_hip_rmsnorm_bwd(const void* x, const void* g, const float* inv, const 
 /* Column sums of x[rows, D] (dtype) into out[D] (out_dtype), fp32 accumulation in a fixed order: the
  * bias gradient of the block's three Linear layers (griffin/griffin.py:379-389; autograd of
  * `nn.Linear`: db = sum over tokens of dy), which the caller's BLAS library leaves to a generic reduction.
- * `scratch` holds rglru_hip_colsum_scratch_bytes(rows, D) bytes. */
+ * `scratch` holds rglru_hip_colsum_scratch_bytes(rows, D) bytes: partial sums [sets][D] in fp32, sets = bytes / (4 D).
+ * out NULL: they are left for rglru_hip_block_finish to add up. */
 size_t rglru_hip_colsum_scratch_bytes(int64_t rows, int64_t D);
 int rglru_hip_colsum(const void* x, void* scratch, void* out, int64_t rows, int64_t D, int dtype, int out_dtype,
                      void* stream);
@@ -360,6 +361,43 @@ int rglru_hip_colsum(const void* x, void* scratch, void* out, int64_t rows, int6
  * dW = dy^T x) where the caller splits the contraction over all tokens into a batch of shorter GEMMs of its BLAS
  * library and has their results added. */
 int rglru_hip_sum_sets(const void* x, void* out, int64_t sets, int64_t n, int dtype, void* stream);
+
+/* Products of the block's Linear layers (griffin/griffin.py:379-389) on the matrix unit, fp32 accumulation, all matrices in
+ * `dtype`, their rows whole 16-byte vectors on 16-byte boundaries, lda / ldb / ldc elements apart:
+ *   RGLRU_LINEAR_FORWARD      c_i[M, N] = a0[M, K] b_i[N, K]^T + bias_i[N]     i = 0, and 1 where b1 is given; biases may be NULL
+ *   RGLRU_LINEAR_INPUT_GRAD   c0[M, N]  = a0[M, K] b0[K, N] + a1[M, K] b1[K, N]     a1 NULL: the first product alone
+ *   RGLRU_LINEAR_WEIGHT_GRAD  c_i[M, N] = a_i[K, M]^T b0[K, N]                 i = 0, and 1 where a1 is given
+ * `active`: one byte per token or NULL; the results of inactive tokens (rows of c) are zero, and in a weight gradient the
+ * inactive rows of a count as zero.  A weight gradient whose rglru_hip_linear_splits (problems: 1 or 2) is above one
+ * leaves fp32 sums partial[splits][problems][M][N] instead of c; colsum[splits][problems][M] (or NULL) receives the column
+ * sums of a_i over each split's rows, the gradient of the biases. */
+enum { RGLRU_LINEAR_FORWARD = 0, RGLRU_LINEAR_INPUT_GRAD = 1, RGLRU_LINEAR_WEIGHT_GRAD = 2 };
+int64_t rglru_hip_linear_splits(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype);
+int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
+                     const void* bias0, const void* bias1, const uint8_t* active, void* c0, void* c1, int64_t ldc,
+                     float* partial, float* colsum, int64_t M, int64_t N, int64_t K, int dtype, void* stream);
+
+/* Reverse mode of what rglru_hip_prepare_block_fwd does between the projections (griffin/griffin.py:474-520), up to the last
+ * sums of the parameter gradients, which rglru_hip_block_finish does for the whole block in one launch.
+ * `dgated`[B,T,W]: the gradient at the gated output on entry, scratch afterwards; y, v, x_conv: as that call wrote or read
+ * them; u: the first projection, contiguous; positions / rows as for rglru_hip_conv_rows_bwd.  Writes du and dv, rows
+ * `d_stride` elements apart (W, or 2 W for the halves of one matrix).  gate_scratch: rglru_hip_bwd_scratch_bytes, conv_scratch:
+ * rglru_hip_conv_scratch_bytes; both hold the partial sums until rglru_hip_block_finish.  bf16 storage, parameters and
+ * gradients; no carried state.  Only where rglru_hip_fast_path() is 1. */
+int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
+                        const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
+                        void* gate_scratch, void* conv_scratch, void* du, void* dv, int64_t d_stride,
+                        int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
+
+/* dst[i] = sum over s < sets of src[s * n + i] (src_dtype), fp32 accumulation in a fixed order; up to five in one launch, all
+ * with results in dst_dtype.  dst NULL: skipped. */
+typedef struct { const void* src; void* dst; int64_t sets, n; int src_dtype; } rglru_sum;
+int rglru_hip_sums(const rglru_sum* sums, int n_sums, int dst_dtype, void* stream);
+/* The parameter gradients (bf16) of the block from the partial sums of rglru_hip_block_bwd, and up to four further sums
+ * (weight and bias gradients of the projections), in one launch.  dtaps, dbias, and any dst may be NULL. */
+int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, void* dw_a, void* dw_x,
+                           void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, const rglru_sum* sums, int n_sums,
+                           int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
 
 /* Single-token step of the recurrent block (griffin/griffin.py:459-528 with one token per row) in
  * two launches around the caller's three Linear layers:

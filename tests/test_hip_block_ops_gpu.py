@@ -906,3 +906,90 @@ def test_right_padded_block_in_one_launch_matches_the_separate_kernels(cfg, pack
         assert torch.equal(na.conv_state, nb.conv_state)
     for i, (p, q) in enumerate(zip(ga, gb)):
         assert rel_err(p.float(), q.float()) < BF16_TOL, i
+
+
+# ----------------------------------------------------------------------------------------------
+# matrix products of the Linear layers (C ABI: rglru_hip_linear) and the block as one training operator
+# ----------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 72, 64), (65, 64, 136), (64, 128, 40), (700, 200, 328), (2050, 2056, 72), (1100, 136, 2304)])
+def test_linear_products_match_fp64(M, N, K, dtype):
+    """All three kinds at edges of tiles, slices and splits, one and two products a launch, with and without masked rows."""
+    from griffin_amd import _lib
+
+    lib = _lib.load()
+    code = _lib.RGLRU_BF16 if dtype == torch.bfloat16 else _lib.RGLRU_F32
+    _say("products", M, N, K, dtype)
+    gen = torch.Generator().manual_seed(7)
+    make = lambda *shape: torch.randn(*shape, generator=gen).to(dtype).cuda()
+    x, w0, w1, b0, b1 = make(M, K), make(N, K), make(N, K), make(N), make(N)
+    dy = make(M, 2 * N)                                          # the halves of one matrix: rows 2 N apart
+    keep = torch.rand(M, generator=gen).cuda() < 0.7
+    active = keep.to(torch.uint8)
+    at = lambda t: None if t is None else t.data_ptr()
+    stream = torch.cuda.current_stream().cuda_stream
+    tol = 2e-5 if dtype == torch.float32 else 1e-2
+
+    def product(kind, a0, a1, lda, b0_, b1_, ldb, bias0, bias1, act, c0, c1, ldc, partial, sums, m, n, k):
+        _lib.check(lib.rglru_hip_linear(kind, at(a0), at(a1), lda, at(b0_), at(b1_), ldb, at(bias0), at(bias1), at(act), at(c0), at(c1), ldc,
+                                        at(partial), at(sums), m, n, k, code, stream), "linear")
+
+    def compare(got, want, name):
+        torch.cuda.synchronize()
+        assert rel_err(got.double().cpu(), want.cpu()) < tol, name
+
+    f = lambda t: t.double()
+    y0, y1 = make(M, N), make(M, N)
+    product(0, x, None, K, w0, w1, K, b0, b1, active, y0, y1, N, None, None, M, N, K)
+    compare(y0, (f(x) @ f(w0).t() + f(b0)) * keep[:, None], "first of two")
+    compare(y1, (f(x) @ f(w1).t() + f(b1)) * keep[:, None], "second of two")
+    product(0, x, None, K, w0, None, K, None, None, None, y0, None, N, None, None, M, N, K)
+    compare(y0, f(x) @ f(w0).t(), "one, no bias")
+    dx = make(M, K)
+    product(1, dy, dy[:, N:], 2 * N, w0, w1, K, None, None, active, dx, None, K, None, None, M, K, N)
+    compare(dx, (f(dy) @ torch.cat((f(w0), f(w1)))) * keep[:, None], "input gradient of two")
+    for pair in (1, 2):
+        splits = lib.rglru_hip_linear_splits(2, N, K, M, pair, code)
+        dw = torch.full((splits, pair, N, K), float("nan"), device="cuda", dtype=torch.float32 if splits > 1 else dtype)
+        sums = torch.full((splits, pair, N), float("nan"), device="cuda")
+        product(2, dy, dy[:, N:] if pair == 2 else None, 2 * N, x, None, K, None, None, active, dw[0, 0], dw[0, 1] if pair == 2 else None, K,
+                dw if splits > 1 else None, sums, N, K, M)
+        live = f(dy)[:, :pair * N] * keep[:, None]
+        compare(dw.double().sum(0).view(pair * N, K), live.t() @ f(x), "weight gradient")
+        compare(sums.double().sum(0).view(-1), live.sum(0), "column sums")
+
+
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("B,T,D,W,nb", [(2, 1, 64, 96, 3), (3, 37, 72, 128, 2), (2, 333, 192, 256, 16), (2, 4097, 768, 1024, 16), (4, 2048, 1536, 2048, 16)])
+def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded):
+    """The node that covers the whole block (own products and, for the long ones, those of the BLAS library) against the same
+    block taken layer by layer, which is what a call that returns a cache does."""
+    from griffin_amd import RecurrentBlock
+
+    _say("block as one operator", B, T, D, W, nb, padded)
+    torch.manual_seed(5)
+    block = RecurrentBlock(D, W, gate_blocks=nb, scan_mode="hip").cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            if name.endswith("bias"):
+                p.normal_(std=0.1)
+    x = torch.randn(B, T, D, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn_like(x)
+    active = None
+    if padded:
+        lengths = torch.linspace(max(1, T // 5), T, B, device="cuda").long()
+        active = torch.arange(T, device="cuda")[None] < lengths[:, None]
+    names, leaves = zip(*([("x", x)] + list(block.named_parameters())))
+    nodes = []
+    whole = block(x, active_mask=active)
+    nodes.append(type(whole.grad_fn).__name__ + str(whole.grad_fn.name()))
+    assert "BlockTrain" in nodes[0]
+    got = torch.autograd.grad(whole, leaves, dy)
+    layered, _ = block(x, active_mask=active, return_cache=True)
+    want = torch.autograd.grad(layered, leaves, dy)
+    torch.cuda.synchronize()
+    assert rel_err(whole.float(), layered.float()) < 1e-2
+    for name, g, w in zip(names, got, want):
+        err = float((g.float() - w.float()).norm() / w.float().norm().clamp_min(1e-30))
+        _say("  d%s rel error: %.2e" % (name, err))
+        assert err < 1e-2, name
