@@ -86,6 +86,8 @@ _SIGNATURES = {
     "rglru_hip_prepare_block_fwd": (ctypes.c_int, [_P] * 5 + [ctypes.c_float, ctypes.c_int, _P]
                                     + [_P, _I, _P, _I, _P, _P, _P, _I] + [_P] * 8
                                     + [_I, _I, _I, _I, ctypes.c_int, _P]),
+    "rglru_hip_block_infer": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _P, _I, ctypes.c_int] + [_P] * 10
+                              + [_I, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_step_gated": (ctypes.c_int, [_P] * 6 + [_I, _P] + [_I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_set_spin_limit": (ctypes.c_int64, [_I]),
     "rglru_hip_set_reproducible": (ctypes.c_int, [ctypes.c_int]),

@@ -392,6 +392,20 @@ py::tuple fingerprint(const std::vector<Tensor>& tensors) {
   return out;
 }
 
+// The same, kept on this side and compared here: a decode loop asks every step.
+struct Stamp {
+  std::vector<std::pair<const void*, int64_t>> seen;
+  explicit Stamp(const std::vector<Tensor>& tensors) {
+    for (const Tensor& t : tensors) seen.emplace_back(t.data_ptr(), static_cast<int64_t>(t._version()));
+  }
+  bool matches(const std::vector<Tensor>& tensors) const {
+    if (tensors.size() != seen.size()) return false;
+    for (size_t i = 0; i < seen.size(); ++i)
+      if (tensors[i].data_ptr() != seen[i].first || static_cast<int64_t>(tensors[i]._version()) != seen[i].second) return false;
+    return true;
+  }
+};
+
 // ---- decode steps ----------------------------------------------------------------------------------------------
 
 Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
@@ -982,12 +996,13 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(x_in.device());
   const int code = code_of(dtype);
-  Tensor x = x_in.select(1, 0);
-  if (x.stride(1) != 1 || (x.stride(0) * x.element_size()) % 16 || !is_aligned(x)) x = aligned(x);
+  Tensor x = x_in;
+  if (x.stride(2) != 1 || (x.stride(0) * x.element_size()) % 16 || !is_aligned(x)) x = aligned(x);
   Tensor h_in = rnn_state.defined() ? as(rnn_state, at::kFloat) : at::zeros({B, W}, x.options().dtype(at::kFloat));
-  Tensor h_out = fresh({B, W}, at::kFloat, x);
-  Tensor new_conv = fresh({B, K - 1, W}, dtype, x);
-  Tensor new_pos = fresh({B}, at::kLong, x);
+  Parts cache;                                             // what the next step reads: the three live as long as each other
+  cache.add(B * W * 4), cache.add(B * (K - 1) * W * x.element_size()), cache.add(B * 8);
+  cache.allocate(x);
+  Tensor h_out = cache.take({B, W}, at::kFloat), new_conv = cache.take({B, K - 1, W}, dtype), new_pos = cache.take({B}, at::kLong);
   Tensor out = fresh({B, 1, D}, dtype, x);
   // x after the convolution, the second branch, their product with the state, one flag byte per row
   const size_t row_bytes = round_up(B * W * x.element_size());
@@ -1194,6 +1209,10 @@ Tensor linear(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, c
     TORCH_CHECK_VALUE(active_->numel() == x.numel() / x.size(-1) && active_->element_size() == 1, "active: one byte for each row of x");
     active = active_->contiguous();
   }
+  if (!wants_grad({&x, &weight, &bias})) {
+    at::NoGradGuard no_grad;
+    return Linear::values(x, weight, bias, opt(active));
+  }
   return Linear::apply(x, weight, maybe(bias), active);
 }
 
@@ -1319,6 +1338,7 @@ std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const 
   Tensor b1 = opt(b1_), b2 = opt(b2_);
   require_gpu("hip_linear_pair", {&x, &w1, &b1, &w2, &b2});
   code_of(x.scalar_type());
+  if (!wants_grad({&x, &w1, &b1, &w2, &b2})) return linear_pair_values(x, w1, b1_, w2, b2_);
   auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2));
   return {out[0], out[1]};
 }
@@ -1504,15 +1524,83 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
                            contiguous(u), contiguous(v), first_reset, c);
 }
 
+// The whole block over sequences without gradients (griffin/griffin.py:459-528): projections, positions, convolution, RG-LRU
+// and gate, output projection in four launches.  Every token active: positions follow prev_pos (or are segment_pos);
+// right-padded: flags, rows, active and the projections u, v as the caller has them from TokenFacts.  Returns (output, final
+// state, convolution state, last position); nothing where the kernels do not take the operands.
+std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
+    const Tensor& x, const std::vector<Tensor>& p, const Tensor& image, const MaybeTensor& conv_state_, const MaybeTensor& rnn_state_,
+    const MaybeTensor& prev_pos_, const MaybeTensor& segment_pos_, const MaybeTensor& flags_, const MaybeTensor& rows_, const MaybeTensor& active_,
+    const MaybeTensor& u_, const MaybeTensor& v_, bool need_carry) {
+  typedef BlockTrain N;
+  const auto dtype = x.scalar_type();
+  const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
+  for (const Tensor& t : p)
+    if (t.scalar_type() != dtype || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
+  const Tensor &wx = p[N::WX - 1], &bx = p[N::BX - 1], &wy = p[N::WY - 1], &by = p[N::BY - 1], &cw = p[N::CW - 1], &cb = p[N::CB - 1],
+               &wa = p[N::WA - 1], &wo = p[N::WO - 1], &bo = p[N::BO - 1];
+  const int64_t W = wx.size(0), K = cw.size(2), nb = wa.size(0), M = B * T;
+  if (!vector_rows(x) || W % 8 || wx.dim() != 2 || wx.size(1) != D || wy.sizes() != wx.sizes() || wo.dim() != 2 || wo.size(0) != D ||
+      wo.size(1) != W || cw.size(0) != W || !rglru_hip_block_fwd_path(W, nb, K, code_of(dtype)))
+    return std::nullopt;
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(x.device());
+  const int code = code_of(dtype);
+  void* stream = stream_of(x);
+  Tensor u = opt(u_), v = opt(v_), flags = opt(flags_), rows = opt(rows_), active = opt(active_), prev = opt(prev_pos_), seg = opt(segment_pos_);
+  Tensor state = K == 1 ? Tensor() : as(opt(conv_state_), dtype), h0 = as(opt(rnn_state_), at::kFloat);
+  if (prev.defined()) prev = prev.to(at::kLong).contiguous();
+  if (seg.defined()) seg = seg.to(at::kLong).contiguous();
+  const bool own = own_linear(x, wx, bx);
+  Parts s;
+  const size_t row_bytes = M * W * x.element_size();
+  s.add(row_bytes), s.add(own && !u.defined() ? row_bytes : 0), s.add(own && !u.defined() ? row_bytes : 0);
+  s.add(rglru_hip_workspace_bytes(B, T, W, nb)), s.add(M);
+  s.allocate(x);
+  char *gated = s.raw(), *up = s.raw(), *vp = s.raw(), *ws = s.raw();
+  uint8_t* flag_bytes = reinterpret_cast<uint8_t*>(s.raw());
+  if (u.defined()) {
+    u = aligned(u), v = aligned(v);
+  } else if (own) {
+    linear_forward(x, wx, bx, wy, by, Tensor(), up, vp);
+  } else {
+    u = at::linear(x, wx, bx), v = at::linear(x, wy, by);
+  }
+  if (u.defined()) up = static_cast<char*>(ptr(u)), vp = static_cast<char*>(ptr(v));
+  Tensor h_last = fresh({B, W}, at::kFloat, x), new_conv = fresh({B, K - 1, W}, dtype, x), last;
+  if (!flags.defined()) {
+    last = fresh({B}, at::kLong, x);
+    check(rglru_hip_block_infer(up, W, vp, W, ptr(state), ptr(cw), ptr(cb), K, code, ptr(image), fptr(h0), iptr(prev), iptr(seg), flag_bytes, gated,
+                                K > 1 ? ptr(new_conv) : nullptr, fptr(h_last), static_cast<int64_t*>(last.data_ptr()), ws, B, T, W, nb, code, stream),
+          "rglru_hip_block_infer");
+  } else {
+    check(rglru_hip_block_fwd(up, W, vp, W, ptr(state), ptr(cw), ptr(cb), K, code, ptr(image), fptr(h0), bptr(flags), nullptr, nullptr, gated,
+                              nullptr, fptr(h_last), ws, B, T, W, nb, code, stream), "rglru_hip_block_fwd");
+    if (need_carry && K > 1)
+      check(rglru_hip_conv_carry(up, W, ptr(state), static_cast<const int32_t*>(ptr(rows)), ptr(new_conv), B, T, W, K, code, stream),
+            "rglru_hip_conv_carry");
+  }
+  Tensor out, live = active.defined() ? active.contiguous() : active;
+  if (own) {
+    out = fresh_like(x);
+    check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, gated, nullptr, W, ptr(wo), nullptr, W, ptr(bo), nullptr, bptr(live), ptr(out), nullptr, D, nullptr,
+                           nullptr, M, D, W, code, stream), "rglru_hip_linear");
+  } else {
+    out = at::linear(part(s.buffer, 0, {B, T, W}, dtype), wo, bo);
+    if (live.defined()) masked_rows(out, live, true);
+  }
+  return std::make_tuple(out, h_last, new_conv, last);
+}
+
 // ---- RMSNorm (griffin/griffin.py:68-80) ---------------------------------------------------------------------------
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> rmsnorm_forward(const Tensor& x_in, const Tensor& g, double eps) {
+std::tuple<Tensor, Tensor, Tensor, Tensor> rmsnorm_forward(const Tensor& x_in, const Tensor& g, double eps, bool need_inv) {
   c10::DeviceGuard guard(x_in.device());
   Tensor x = x_in.contiguous();
   Tensor scale = operand(g, x.scalar_type());
   const int64_t D = x.size(-1), rows = x.numel() / D;
   Tensor y = fresh_like(x);
-  Tensor inv = fresh({rows}, at::kFloat, x);
+  Tensor inv = need_inv ? fresh({rows}, at::kFloat, x) : Tensor();
   if (rows > 0)
     check(rglru_hip_rmsnorm_fwd(ptr(x), ptr(scale), ptr(y), fptr(inv), rows, D, static_cast<float>(eps), code_of(x.scalar_type()),
                                 code_of(scale.scalar_type()), stream_of(x)), "rglru_hip_rmsnorm_fwd");
@@ -1521,7 +1609,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> rmsnorm_forward(const Tensor& x_in, c
 
 struct RmsNorm : torch::autograd::Function<RmsNorm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor& g, double eps) {
-    auto [x, scale, y, inv] = rmsnorm_forward(x_in, g, eps);
+    auto [x, scale, y, inv] = rmsnorm_forward(x_in, g, eps, true);
     ctx->save_for_backward({x, scale, inv});
     pack(ctx, {type_or_none(g)});
     return y;
@@ -1558,7 +1646,7 @@ Tensor rmsnorm(const Tensor& x, const Tensor& g, double eps) {
   code_of(x.scalar_type());
   if (wants_grad({&x, &g})) return RmsNorm::apply(x, g, eps);
   at::NoGradGuard no_grad;
-  return std::get<2>(rmsnorm_forward(x, g, eps));
+  return std::get<2>(rmsnorm_forward(x, g, eps, false));
 }
 
 }  // namespace
@@ -1568,6 +1656,7 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(kernel_path);
   EXPORT(prepare);
   EXPORT(fingerprint);
+  py::class_<Stamp>(m, "Stamp").def(py::init<const std::vector<Tensor>&>()).def("matches", &Stamp::matches);
   EXPORT(rglru);
   EXPORT(rglru_step);
   EXPORT(rglru_steps);
@@ -1595,6 +1684,7 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(linear_pair);
   EXPORT(linear_pair_values);
   EXPORT(block_train);
+  EXPORT(block_infer);
   EXPORT(rmsnorm);
 #undef EXPORT
 }

@@ -135,9 +135,26 @@ def hip_block_step(x: Tensor, linear_x, linear_y, conv, linear_out, conv_state: 
     convolution, the RG-LRU step with the output gate, the output projection.  The four layers are those of the block, the
     other arguments as for ``hip_block_decode_step``.  Returns ``(output [B, 1, D], rnn_state, conv_state, positions)``,
     or None where the kernels do not take the operands."""
-    return _lib.native().block_step(x, linear_x.weight, linear_x.bias, linear_y.weight, linear_y.bias, conv.weight, conv.bias,
-                                    linear_out.weight, linear_out.bias, conv_state, prev_pos, segment_pos, active, prep.image,
-                                    prep.blocks, rnn_state)
+    # nn.Module's attribute lookup costs half a microsecond a name
+    px, py, pc, po = linear_x._parameters, linear_y._parameters, conv._parameters, linear_out._parameters
+    try:
+        operands = (px["weight"], px["bias"], py["weight"], py["bias"], pc["weight"], pc["bias"], po["weight"], po["bias"])
+    except KeyError:                                         # a parametrised or otherwise replaced parameter
+        operands = (linear_x.weight, linear_x.bias, linear_y.weight, linear_y.bias, conv.weight, conv.bias, linear_out.weight,
+                    linear_out.bias)
+    return _lib.native().block_step(x, *operands, conv_state, prev_pos, segment_pos, active, prep.image, prep.blocks, rnn_state)
+
+
+def hip_block_infer(x: Tensor, parameters, prep, conv_state: Tensor | None, rnn_state: Tensor | None, prev_pos: Tensor | None,
+                    segment_pos: Tensor | None, flags: Tensor | None, rows: Tensor | None, active: Tensor | None, u: Tensor | None,
+                    v: Tensor | None, need_state: bool):
+    """The whole recurrent block over sequences without gradients (griffin/griffin.py:459-528), four launches.  ``parameters``:
+    weights and biases of linear_x, linear_y and the convolution, the five of the RG-LRU, weight and bias of linear_out; ``prep`` the
+    image of the RG-LRU's.  Every token active: positions follow ``prev_pos`` [B] or are ``segment_pos`` [B, T].  Right-padded:
+    ``flags`` and ``rows`` of ``token_facts``, ``active`` the mask.  ``u``, ``v``: the projections if the caller has them.  Returns
+    ``(output, final state, convolution state, last position or None)``, or None where the kernels do not take the operands."""
+    return _lib.native().block_infer(x, parameters, prep.image, conv_state, rnn_state, prev_pos, segment_pos, flags, rows, active, u, v,
+                                     need_state)
 
 
 def _sum_sets(sets: Tensor) -> Tensor:

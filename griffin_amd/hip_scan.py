@@ -139,6 +139,7 @@ class PreparedParams:
         self.blocks = nb
         self.dtype = dtype
         self.c = float(c)
+        self.device = w_a.device
         _dtype_code(dtype)
         self.image = _lib.native().prepare(w_a, b_a, w_x, b_x, lam, self.c, dtype)
 
@@ -191,6 +192,11 @@ def fingerprint(tensors) -> tuple:
     counters."""
     return _lib.native().fingerprint(tensors) if _lib.available() else tuple(
         v for t in tensors for v in (t.data_ptr(), t._version))
+
+
+def parameter_stamp(tensors):
+    """The same as an object with ``matches(tensors)``, for callers that ask often."""
+    return _lib.native().Stamp(tensors)
 
 
 def hip_rglru_steps(xs: Tensor, prep: PreparedParams, state: Tensor, flags: Tensor | None = None) -> Tensor:

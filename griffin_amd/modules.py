@@ -91,7 +91,7 @@ class RG_LRU(nn.Module):
     def _hip_covers(self, xt: Tensor) -> bool:
         return (
             xt.dtype in hip_scan.SUPPORTED_DTYPES
-            and self.recurrence_gate.block_width <= 512
+            and self._modules["recurrence_gate"].block_width <= 512
             and xt.numel() > 0
         )
 
@@ -115,14 +115,17 @@ class RG_LRU(nn.Module):
         """Kernel-side parameter image for inference, rebuilt when a parameter is replaced or updated
         in place (every in-place update bumps the tensor's version counter)."""
         params = self._gate_parameters()
-        key = (dtype, device, self.c, *hip_scan.fingerprint(params))
-        if getattr(self, "_prep_key", None) != key:
-            prep = hip_scan.PreparedParams(*params, self.c, dtype)
-            if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
-                return prep                                  # allocated by the graph being captured: this call only
-            self._prep = prep
-            self._prep_key = key
-        return self._prep
+        held = self.__dict__
+        prep, stamp = held.get("_prep"), held.get("_prep_key")
+        if (prep is not None and stamp is not None and prep.dtype is dtype and prep.device == device and prep.c == self.c
+                and stamp.matches(params)):
+            return prep
+        prep = hip_scan.PreparedParams(*params, self.c, dtype)
+        if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            return prep                                      # allocated by the graph being captured: this call only
+        self._prep = prep
+        self._prep_key = hip_scan.parameter_stamp(params)
+        return prep
 
     def invalidate_caches(self) -> None:
         """Forget the kernel-side parameter image.  It is rebuilt by itself when a parameter is replaced or
@@ -164,13 +167,14 @@ class RG_LRU(nn.Module):
                     raise ValueError(f"{name} must have shape ({batch}, {steps}), got {tuple(mask.shape)}")
         if ht_minus_1 is not None and ht_minus_1.shape != (batch, width):
             raise ValueError(f"ht_minus_1 must have shape ({batch}, {width}), got {tuple(ht_minus_1.shape)}")
+        device = xt.device
         state_dtype = torch.float32 if xt.dtype in (torch.float16, torch.bfloat16) else xt.dtype
         if reset_mask is not None:
             reset_mask = reset_mask.to(device=xt.device, dtype=torch.bool)
         if active_mask is not None:
             active_mask = active_mask.to(device=xt.device, dtype=torch.bool)
-        if ht_minus_1 is not None:
-            ht_minus_1 = ht_minus_1.to(device=xt.device, dtype=state_dtype)
+        if ht_minus_1 is not None and (ht_minus_1.dtype is not state_dtype or ht_minus_1.device != device):
+            ht_minus_1 = ht_minus_1.to(device=device, dtype=state_dtype)
 
         mode = self.scan_mode
         if mode not in SCAN_MODES:
@@ -180,7 +184,7 @@ class RG_LRU(nn.Module):
             mode == "auto"
             and xt.is_cuda
             and self._hip_covers(xt)
-            and hip_scan.hip_scan_is_usable(xt.device)
+            and hip_scan.hip_scan_is_usable(device)
         )
         if explicit_hip or auto_hip:
             if explicit_hip and not xt.is_cuda:
@@ -190,7 +194,7 @@ class RG_LRU(nn.Module):
                 )
             if steps == 1 and not self._needs_grad(xt, ht_minus_1):
                 # decode: the single-step kernel on a prepared parameter image kept between calls
-                prep = self._prepared(xt.dtype, xt.device)
+                prep = self._prepared(xt.dtype, device)
                 y, state = hip_scan.hip_rglru_module_step(xt, prep, ht_minus_1, hip_scan.pack_flags(reset_mask, active_mask))
                 return (y, state) if return_state else y
             # the reset mask of the default positions (a document start at token 0 of every row, nothing else)
@@ -313,6 +317,9 @@ class RMSNorm(nn.Module):
         return normalized * (1.0 + self.g)
 
 
+_BLOCK_LAYERS = ("linear_x", "linear_y", "temporal_conv", "linear_out", "rg_lru")
+
+
 class RecurrentBlock(nn.Module):
     """Linear -> causal depthwise conv -> RG-LRU, gated by GeLU(Linear), then Linear out
     (griffin/griffin.py:361-529).  The RG-LRU inside honours ``scan_mode`` unchanged."""
@@ -396,13 +403,14 @@ class RecurrentBlock(nn.Module):
                 tensors += [cache.rnn_state, cache.conv_state]
             if any(t.requires_grad for t in tensors):
                 return False
-        if self.linear_x.weight.dtype != x.dtype or self.linear_y.weight.dtype != x.dtype:
+        layers = self._modules
+        if layers["linear_x"].weight.dtype != x.dtype or layers["linear_y"].weight.dtype != x.dtype:
             return False
-        rg_lru = self.rg_lru
+        rg_lru = layers["rg_lru"]
         if self.conv_kernel_size > hip_block_ops.max_kernel_size():
             return False
         if rg_lru.scan_mode == "auto":
-            return rg_lru.recurrence_gate.block_width <= 512 and hip_scan.hip_scan_is_usable(x.device)
+            return rg_lru._modules["recurrence_gate"].block_width <= 512 and hip_scan.hip_scan_is_usable(x.device)
         return rg_lru.scan_mode in ("hip", "fused")
 
     def _hip_decode(self, x: Tensor, cache: RecurrentBlockCache | None, segment_pos: Tensor | None,
@@ -425,13 +433,16 @@ class RecurrentBlock(nn.Module):
                 raise ValueError("Cached segment positions have an incompatible shape")
             if rnn_state is not None and rnn_state.shape != (batch, width):
                 raise ValueError(f"ht_minus_1 must have shape ({batch}, {width}), got {tuple(rnn_state.shape)}")
-            prev_pos = prev_pos.to(device=x.device, dtype=torch.long).contiguous()
+            if prev_pos.dtype is not torch.long or prev_pos.device != x.device or not prev_pos.is_contiguous():
+                prev_pos = prev_pos.to(device=x.device, dtype=torch.long).contiguous()
         active = None
         if active_mask is not None and not bool(active_mask.all()):
             active = active_mask[:, 0].to(torch.uint8).contiguous()
-        if not torch.is_autocast_enabled() and self._is_plain(self.linear_out):
-            done = hip_block_ops.hip_block_step(x, self.linear_x, self.linear_y, self.temporal_conv, self.linear_out, conv_state,
-                                                prev_pos, segment_pos, active, self.rg_lru._prepared(x.dtype, x.device), rnn_state)
+        layers = self._modules
+        if not torch.is_autocast_enabled() and self._is_plain(layers["linear_out"]):
+            done = hip_block_ops.hip_block_step(x, layers["linear_x"], layers["linear_y"], layers["temporal_conv"], layers["linear_out"],
+                                                conv_state, prev_pos, segment_pos, active, layers["rg_lru"]._prepared(x.dtype, x.device),
+                                                rnn_state)
             if done is not None:
                 output, *state = done
                 return (output, RecurrentBlockCache(*state)) if return_cache else output
@@ -470,9 +481,15 @@ class RecurrentBlock(nn.Module):
     def _linear(self, layer: nn.Linear, x: Tensor) -> Tensor:
         """A Linear layer of the block; in training on the HIP path its bias gradient is summed by a
         kernel of the library instead of a generic reduction (the GEMMs are the BLAS library's either way)."""
-        if self._linear_on_hip(layer, x):
+        if self._linear_on_hip(layer, x) or self._inference_on_hip(layer, x):
             return hip_block_ops.hip_linear(x, layer.weight, layer.bias)
         return layer(x)
+
+    def _inference_on_hip(self, layer: nn.Linear, x: Tensor) -> bool:
+        """Without gradients: short products run on the library's kernels, which cost the host less than a call of the BLAS
+        library (hip_linear chooses)."""
+        return (not torch.is_grad_enabled() and not torch.is_autocast_enabled() and x.is_cuda and x.numel() > 0 and self._is_plain(layer)
+                and x.dtype in hip_scan.SUPPORTED_DTYPES and layer.weight.dtype == x.dtype and self._hip_block_ops_covers(x))
 
     def _linear_on_hip(self, layer: nn.Linear, x: Tensor) -> bool:
         return (torch.is_grad_enabled() and layer.bias is not None and layer.bias.requires_grad
@@ -485,38 +502,73 @@ class RecurrentBlock(nn.Module):
         """Nobody wrapped or hooked the Linear layer: calling it is a product with its weight and nothing else."""
         return type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks
 
-    @staticmethod
-    def _unhooked(layer: nn.Module) -> bool:
-        return not (layer._forward_hooks or layer._forward_pre_hooks or layer._backward_hooks or layer._backward_pre_hooks)
-
-    def _training_parameters(self, x: Tensor):
+    def _whole_parameters(self, x: Tensor):
         """The block's parameters (linear_x, linear_y, convolution, gates, Lambda, linear_out) where one operator may stand for the
-        whole block: training in bf16 on the HIP path, nobody wrapped, hooked or replaced a layer; else None."""
-        if not torch.is_grad_enabled() or x.dtype != torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.is_autocast_enabled():
+        whole block: bf16 on the HIP path, nobody wrapped, hooked or replaced a layer; else None."""
+        if x.dtype is not torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.is_autocast_enabled():
             return None
-        lru = self.rg_lru
-        if lru.scan_mode not in ("auto", "hip", "fused") or type(lru) is not RG_LRU:
+        layers = self._modules
+        lx, ly, conv, lo, lru = (layers[name] for name in _BLOCK_LAYERS)
+        if not (type(lx) is type(ly) is type(lo) is nn.Linear and type(conv) is nn.Conv1d and type(lru) is RG_LRU):
             return None
-        try:
-            layers = self._modules
-            lx, ly, conv, lo = layers["linear_x"], layers["linear_y"], layers["temporal_conv"], layers["linear_out"]
-            if not (type(lx) is type(ly) is type(lo) is nn.Linear and type(conv) is nn.Conv1d
-                    and all(self._unhooked(m) for m in (lx, ly, conv, lo, lru))):
+        mode = lru.scan_mode
+        if mode not in ("auto", "hip", "fused"):
+            return None
+        for m in (lx, ly, conv, lo, lru):
+            if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
                 return None
-            parameters = [m._parameters[name] for m in (lx, ly, conv) for name in ("weight", "bias")]
-            parameters += lru._gate_parameters()
-            parameters += [lo._parameters["weight"], lo._parameters["bias"]]
+        try:
+            px, py, pc, po = lx._parameters, ly._parameters, conv._parameters, lo._parameters
+            parameters = (px["weight"], px["bias"], py["weight"], py["bias"], pc["weight"], pc["bias"], *lru._gate_parameters(),
+                          po["weight"], po["bias"])
         except KeyError:                                     # a parametrised or otherwise replaced parameter
             return None
-        if any(p is None or p.dtype != torch.bfloat16 for p in parameters):
+        for p in parameters:
+            if p is None or p.dtype is not torch.bfloat16:
+                return None
+        if not hip_block_ops.hip_block_forward_covers(self.rnn_width, parameters[6].shape[0], self.conv_kernel_size, torch.bfloat16):
             return None
-        if not (x.requires_grad or any(p.requires_grad for p in parameters)):
-            return None
-        if not hip_block_ops.hip_block_forward_covers(self.rnn_width, parameters[6].shape[0], self.conv_kernel_size, x.dtype):
-            return None
-        if lru.scan_mode == "auto" and not hip_scan.hip_scan_is_usable(x.device):
+        if mode == "auto" and not hip_scan.hip_scan_is_usable(x.device):
             return None
         return parameters
+
+    def _infer_whole(self, x: Tensor, parameters, cache: RecurrentBlockCache | None, segment_pos: Tensor | None, active_mask: Tensor | None,
+                     return_cache: bool):
+        """The block over sequences without gradients in one call of the library, or None where that does not take the
+        operands (or an operand has the wrong shape: the general path reports it)."""
+        batch, steps = x.shape[:2]
+        device = x.device
+        conv_state = rnn_state = previous = None
+        if cache is not None:
+            conv_state, rnn_state, previous = cache.conv_state, cache.rnn_state, cache.segment_position
+            if (conv_state.shape != (batch, self.conv_kernel_size - 1, self.rnn_width) or previous.shape != (batch,)
+                    or (rnn_state is not None and rnn_state.shape != (batch, self.rnn_width))):
+                return None
+        for t in (conv_state, rnn_state, previous, segment_pos):
+            if t is not None and t.device != device:
+                return None
+        if segment_pos is not None and segment_pos.shape != (batch, steps):
+            return None
+        u = v = flags = rows = live = facts = None
+        if active_mask is not None:
+            facts = hip_block_ops.token_facts(active_mask, segment_pos, previous)
+            # queued before the facts are asked for: the answer arrives while the projections run
+            u, v = hip_block_ops.hip_linear_pair_values(x, *parameters[:4])
+            dense, right_padded = facts.resolve()
+            if dense:
+                segment_pos = facts.positions
+            elif right_padded:
+                flags, rows, live = facts.flags, facts.rows, active_mask
+            else:
+                return None
+        done = hip_block_ops.hip_block_infer(x, parameters, self._modules["rg_lru"]._prepared(x.dtype, device), conv_state, rnn_state, previous,
+                                             segment_pos, flags, rows, live, u, v, return_cache)
+        if done is None:
+            return None
+        output, new_rnn_state, new_conv_state, last_position = done
+        if not return_cache:
+            return output
+        return output, RecurrentBlockCache(new_rnn_state, new_conv_state, last_position if facts is None else facts.last_position)
 
     def _train_whole(self, x: Tensor, parameters, segment_pos: Tensor | None, active_mask: Tensor | None) -> Tensor | None:
         """The block as one operator (``around`` of hip_block_ops.hip_block_forward), or None where that does not take the
@@ -585,12 +637,16 @@ class RecurrentBlock(nn.Module):
         previous_position = None if cache is None else cache.segment_position
         if steps == 1 and self._hip_decode_covers(x, cache):
             return self._hip_decode(x, cache, segment_pos, active_mask, return_cache)
-        if cache is None and not return_cache and steps > 0:
-            parameters = self._training_parameters(x)
-            if parameters is not None:
-                output = self._train_whole(x, parameters, segment_pos, active_mask)
-                if output is not None:
-                    return output
+        parameters = self._whole_parameters(x) if steps > 0 else None
+        if parameters is not None:
+            result = None
+            carried = () if cache is None else (cache.rnn_state, cache.conv_state)
+            if not torch.is_grad_enabled() or not any(t is not None and t.requires_grad for t in (x, *parameters, *carried)):
+                result = self._infer_whole(x, parameters, cache, segment_pos, active_mask, return_cache)
+            elif cache is None and not return_cache:
+                result = self._train_whole(x, parameters, segment_pos, active_mask)
+            if result is not None:
+                return result
         facts = None
         if not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
             # launched in front of the projections, so that its answer is there before they are done
@@ -600,7 +656,8 @@ class RecurrentBlock(nn.Module):
             segment_pos = _resolve_segment_positions(
                 x, segment_pos, previous_position, None if everything_active else active_mask)
 
-        if self._linear_on_hip(self.linear_x, x) and self._linear_on_hip(self.linear_y, x):
+        if (self._linear_on_hip(self.linear_x, x) and self._linear_on_hip(self.linear_y, x)) or (
+                self._inference_on_hip(self.linear_x, x) and self._inference_on_hip(self.linear_y, x)):
             projected, gate_input = hip_block_ops.hip_linear_pair(
                 x, self.linear_x.weight, self.linear_x.bias, self.linear_y.weight, self.linear_y.bias)
         else:

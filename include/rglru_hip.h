@@ -468,6 +468,15 @@ int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_
                                 void* x_conv, void* y, void* gated, void* new_conv_state, float* h_last, void* ws,
                                 int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
 
+/* rglru_hip_block_fwd for inference with every token active, positions included, in two launches: token t of row b stands at
+ * segment_pos[b, t], or at prev_pos[b] + 1 + t where segment_pos is NULL (prev_pos NULL: at t, every row a document from its
+ * beginning).  flag_bytes: B * T bytes of scratch.  last_pos[B] (or NULL) receives the position of each row's last token. */
+int rglru_hip_block_infer(const void* u, int64_t u_stride, const void* v, int64_t v_stride,
+                          const void* conv_state, const void* taps, const void* conv_bias, int64_t K, int vec_dtype,
+                          const void* prep, const float* h0, const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes,
+                          void* gated, void* new_conv_state, float* h_last, int64_t* last_pos, void* ws,
+                          int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
+
 /* Test hook: number of polls a wave may spend waiting for a neighbouring chunk's carry before it
  * gives up, records the failure in the workspace and finishes with unspecified results.  The
  * default is large enough never to trigger in normal operation.  Returns the previous value. */

@@ -993,3 +993,45 @@ def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, p
         err = float((g.float() - w.float()).norm() / w.float().norm().clamp_min(1e-30))
         _say("  d%s rel error: %.2e" % (name, err))
         assert err < 1e-2, name
+
+
+@pytest.mark.parametrize("tokens", ["all", "positions", "padded"])
+@pytest.mark.parametrize("B,T,D,W,nb,carried", [(2, 2, 64, 96, 3, True), (3, 77, 72, 128, 2, True), (1, 1000, 192, 256, 16, False), (3, 2777, 1536, 2048, 16, True)])
+def test_block_inference_in_one_call_matches_layer_by_layer(B, T, D, W, nb, carried, tokens):
+    """Output and cache of the inference call that covers the whole block against the same block with one launch per layer
+    (a forward hook on a layer takes it there)."""
+    from griffin_amd import RecurrentBlock, RecurrentBlockCache, hip_block_ops
+
+    _say("block inference", B, T, D, W, nb, carried, tokens)
+    torch.manual_seed(6)
+    block = RecurrentBlock(D, W, gate_blocks=nb, scan_mode="hip").cuda().to(torch.bfloat16).eval()
+    x = torch.randn(B, T, D, device="cuda", dtype=torch.bfloat16)
+    cache = None
+    if carried:
+        cache = RecurrentBlockCache(torch.randn(B, W, device="cuda"), torch.randn(B, 3, W, device="cuda", dtype=torch.bfloat16),
+                                    torch.tensor([99, 0, -1][:B], device="cuda"))
+    kwargs = {}
+    if tokens == "positions":
+        position = torch.arange(T, device="cuda").repeat(B, 1)
+        position[:, T // 2:] -= T // 2
+        kwargs["segment_pos"] = position
+    elif tokens == "padded":
+        lengths = torch.linspace(max(1, T // 5), T, B, device="cuda").long()
+        kwargs["active_mask"] = torch.arange(T, device="cuda")[None] < lengths[:, None]
+    calls, real = [], hip_block_ops.hip_block_infer
+    hip_block_ops.hip_block_infer = lambda *args: calls.append(1) or real(*args)
+    try:
+        with torch.no_grad():
+            got, got_cache = block(x, cache, return_cache=True, **kwargs)
+            assert calls
+            handle = block.temporal_conv.register_forward_hook(lambda *args: None)
+            want, want_cache = block(x, cache, return_cache=True, **kwargs)
+            handle.remove()
+    finally:
+        hip_block_ops.hip_block_infer = real
+    torch.cuda.synchronize()
+    assert len(calls) == 1
+    assert rel_err(got.float(), want.float()) < 1e-2
+    assert rel_err(got_cache.rnn_state, want_cache.rnn_state) < 1e-2
+    assert torch.equal(got_cache.segment_position, want_cache.segment_position)
+    assert rel_err(got_cache.conv_state.float(), want_cache.conv_state.float()) < 1e-2
