@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kThreads) void step_kernel(FusedArgs p) {
     if (w.slab_ok) gate_mfma_held<IO, MT, NKG>(lds, hw, 0, w.slab, w.r, hf, bias_a, bias_x, ua[0], ux[0], xv);
   } else {
     load_state();
-    gate_tile_generic<IO, MT>(p, (const IO*)p.x, row0, p.B, w.k, w.slab, w.slab_ok, w_a_row, w_x_row,
+    gate_tile_generic<IO, MT>(p, (const IO*)p.x, row0, p.B, w.k, 0, w.slab, w.slab_ok, w_a_row, w_x_row,
                               bias_a, bias_x, lds, ua, ux, xv);
   }
   if (!w.ch_ok) return;
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kThreads) void steps_kernel(FusedArgs p) {
       if (w.slab_ok) gate_mfma_held<IO, MT, NKG>(lds, hw, 0, w.slab, w.r, hf, bias_a, bias_x, ua[0], ux[0], xv);
       __syncthreads();                                   // the tile is overwritten at the top of the next step
     } else {
-      gate_tile_generic<IO, MT>(p, (const IO*)p.x + (long long)k * step_elems, row0, p.B, w.k, w.slab, w.slab_ok,
+      gate_tile_generic<IO, MT>(p, (const IO*)p.x + (long long)k * step_elems, row0, p.B, w.k, 0, w.slab, w.slab_ok,
                                 w_a_row, w_x_row, bias_a, bias_x, lds, ua, ux, xv);
     }
     if (w.ch_ok) {

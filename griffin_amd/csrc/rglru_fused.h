@@ -266,9 +266,11 @@ RGLRU_DEVICE typename Io<IO>::Frag load_x_frag(const FusedArgs& p, const IO* xma
 // memory, K staged through LDS in slices of KCMAX).  On return ua/ux hold W x + b for the wave's
 // slab (register v of tile mt <-> local row hf*16*MT + 16*mt + v) and xv the matching x values.
 // Every thread of the workgroup must call this (it contains barriers).
+// Narrow blocks are packed like those of the kernels with register-held weights (p.bpu > 1: the tile holds the unit's blocks side
+// by side, `first_k` the first of them, and the wave's block starts at column kb), so that all four waves have a slab.
 template <typename IO, int MT>
 RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long long row0, long long rows_total,
-                                    int k, int slab, bool slab_ok, const IO* w_a_row, const IO* w_x_row,
+                                    int first_k, int kb, int slab, bool slab_ok, const IO* w_a_row, const IO* w_x_row,
                                     float bias_a, float bias_x, IO* lds,
                                     f32x16 (&ua)[MT], f32x16 (&ux)[MT], float (&xv)[16 * MT]) {
   typedef Io<IO> Tr;
@@ -284,13 +286,14 @@ RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long lon
 #pragma unroll
   for (int e = 0; e < 16 * MT; ++e) xv[e] = 0.f;
 
-  for (int kc0 = 0; kc0 < p.bwp; kc0 += KCMAX) {
+  for (int kc0 = 0; kc0 < p.bwp; kc0 += KCMAX) {           // one slice when blocks are packed: they are narrow
     const int kcw = (p.bwp - kc0) < KCMAX ? (p.bwp - kc0) : KCMAX;
-    const int vecs = kcw / HW;
-    for (int idx = tid; idx < TR * vecs; idx += kThreads) {
-      const int row = idx / vecs, cv = idx - row * vecs;
-      Frag v = load_x_frag<IO>(p, xmat, row0 + row, rows_total, k, kc0 + cv * HW);
-      *reinterpret_cast<Frag*>(lds + row * LDSROW + cv * HW) = v;
+    const int vecs = kcw / HW, per_row = vecs * p.bpu;
+    for (int idx = tid; idx < TR * per_row; idx += kThreads) {
+      const int row = idx / per_row, at = idx - row * per_row, blk = at / vecs, cv = at - blk * vecs;
+      const bool there = first_k + blk < p.nb;
+      Frag v = load_x_frag<IO>(p, xmat, there ? row0 + row : rows_total, rows_total, first_k + blk, kc0 + cv * HW);
+      *reinterpret_cast<Frag*>(lds + row * LDSROW + blk * kcw + cv * HW) = v;
     }
     __syncthreads();
     if (slab_ok) {
@@ -299,7 +302,7 @@ RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long lon
         Frag fx = *reinterpret_cast<const Frag*>(w_x_row + kc0 + kk);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          Frag xa = *reinterpret_cast<const Frag*>(lds + tile_row<MT>(mt, r) * LDSROW + kk + hf * HW);
+          Frag xa = *reinterpret_cast<const Frag*>(lds + tile_row<MT>(mt, r) * LDSROW + kb + kk + hf * HW);
           Tr::mma(ua[mt], xa, fa);
           Tr::mma(ux[mt], xa, fx);
         }
@@ -307,7 +310,7 @@ RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long lon
       const int own = slab * 32 - kc0;                    // first column of this wave's slab in the slice
       if (own >= 0 && own < kcw) {
 #pragma unroll
-        for (int e = 0; e < 16 * MT; ++e) xv[e] = (float)lds[(hf * 16 * MT + e) * LDSROW + own + r];
+        for (int e = 0; e < 16 * MT; ++e) xv[e] = (float)lds[(hf * 16 * MT + e) * LDSROW + kb + own + r];
       }
     }
     __syncthreads();
@@ -443,16 +446,6 @@ inline int is_aligned(const void* ptr, int64_t W, int64_t bw, size_t es) {
   return ((uintptr_t)ptr % 16 == 0) && ((W * (int64_t)es) % 16 == 0) && ((bw * (int64_t)es) % 16 == 0);
 }
 
-// number of register-held K groups for this block width, or 0 for the streaming variant
-inline int held_groups(const Geometry& g, int dtype, int aligned) {
-  if (dtype == RGLRU_BF16 && aligned && g.bw == g.bwp) {
-    if (g.bwp == 128) return 8;
-    if (g.bwp == 64) return 4;
-    if (g.bwp == 32) return 2;
-  }
-  return 0;
-}
-
 // K groups of the kernels for narrow blocks with register-held weights (2, 4, 6, 8: slabs of 32 channels), or 0.  A block
 // of any multiple of 8 channels up to 128 takes them, padded to whole slabs in LDS and registers (`padded`): per element
 // they are two to four times as fast as the portable kernels, which stream the weights and finish the gradients in GEMM
@@ -518,9 +511,10 @@ struct KernelTimer {
   ~KernelTimer() { if (slot) { (void)hipEventRecord(slot->stop, stream); slot->armed = true; } }
 };
 
-// Narrow blocks of the kernels with register-held weights share a unit (see kPackedWidth).
+// Narrow blocks share a unit (see kPackedWidth), in the kernels with register-held weights and in the portable ones (nkg 0):
+// without that a 64-wide block leaves two of a workgroup's four waves without a slab.
 inline void pack_units(FusedArgs& a, const Geometry& g, int nkg) {
-  if (nkg == 4 || nkg == 2) {
+  if (nkg == 4 || nkg == 2 || (nkg == 0 && g.S <= 2)) {
     a.bpu = kPackedWidth / (int)g.bwp;
     a.units = (int)((g.nb + a.bpu - 1) / a.bpu);
   }

@@ -496,7 +496,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
       const int c = (int)(tk / q.n_b), b = q.first_b + (int)(tk - (long long)c * q.n_b) * p.queues;
       f32x16 ua[MT], ux[MT];
       float xv[EL];
-      gate_tile_generic<IO, MT>(p, x + (long long)b * p.T * W, (long long)c * TR, p.T, w.k, w.slab, w.slab_ok,
+      gate_tile_generic<IO, MT>(p, x + (long long)b * p.T * W, (long long)c * TR, p.T, p.bpu > 1 ? w.unit * p.bpu : w.k, w.kb, w.slab, w.slab_ok,
                                 w_a_row, w_x_row, 0.0f, 0.0f, lds, ua, ux, xv);
       if (w.slab_ok) {
         const long long trow = (long long)b * p.T + c * TR + hf * EL;
@@ -903,7 +903,7 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     if (!a.aligned || (uintptr_t)pre % 16) return fail(RGLRU_E_UNSUPPORTED, "fwd_pre: x, pre and y must be 16-byte aligned");
     a.pre = pre; a.rows_total = B * T;
     nkg = -1;
-    rc = launch_gate_pre_gemm(x, a.wg, const_cast<void*>(pre), B * T, g, s);
+    rc = gate_pre_product(x, a.wg, const_cast<void*>(pre), B * T, g, s);
     if (rc) return rc;
   }
   if (blk) {

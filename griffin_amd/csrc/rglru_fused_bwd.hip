@@ -12,13 +12,11 @@ namespace rglru {
 // first.  Emits the direct input gradient, the gradients at both gate pre-activations and
 // per-workgroup partial sums for the bias and Lambda gradients.
 // ------------------------------------------------------------------------------------------
-template <typename IO, int NKG>
-__global__ __launch_bounds__(kThreads, (NKG == 0 ? 2 : 1)) void bwd_kernel(FusedArgs p) {
+template <typename IO>
+__global__ __launch_bounds__(kThreads, 2) void bwd_kernel(FusedArgs p) {
   constexpr int MT = 1, TR = 32, EL = 16;
   typedef Io<IO> Tr;
-  typedef typename Tr::Frag Frag;
-  constexpr int KC = NKG > 0 ? NKG * Tr::KG : Tr::KCMAX;
-  constexpr int LDSROW = KC + Tr::HW;
+  constexpr int LDSROW = Tr::KCMAX + Tr::HW;
   __shared__ __attribute__((aligned(16))) IO lds[TR * LDSROW];
   __shared__ unsigned s_ticket;
 
@@ -27,8 +25,6 @@ __global__ __launch_bounds__(kThreads, (NKG == 0 ? 2 : 1)) void bwd_kernel(Fused
   const IO* wg = (const IO*)p.wg;
   const IO* w_a_row = wg + ((long long)(0 * p.nb + w.k) * p.bwp + (w.slab_ok ? w.o : 0)) * p.bwp + hf * Tr::HW;
   const IO* w_x_row = wg + ((long long)(1 * p.nb + w.k) * p.bwp + (w.slab_ok ? w.o : 0)) * p.bwp + hf * Tr::HW;
-  HeldWeights<IO, NKG> hw;
-  hw.load(w_a_row, w_x_row);
   const float nba = -kLog2e * p.bias[w.kp], nbx = -kLog2e * p.bias[p.Wp + w.kp];   // biases as the sigmoids take them
   const float sp = w.ch_ok ? p.sp[w.kp] : 0.f;
   const float cs = w.ch_ok ? p.cs[w.kp] : 0.f;
@@ -50,20 +46,8 @@ __global__ __launch_bounds__(kThreads, (NKG == 0 ? 2 : 1)) void bwd_kernel(Fused
 
     f32x16 ua[MT], ux[MT];
     float xv[EL];
-    if constexpr (NKG > 0) {
-      constexpr int VPR = KC / Tr::HW;
-      for (int idx = tid; idx < TR * VPR; idx += kThreads) {
-        const int row = idx / VPR, cv = idx - row * VPR;
-        Frag v = load_x_frag<IO>(p, x + (long long)b * p.T * W, (long long)t0 + row, p.T, w.k, cv * Tr::HW);
-        *reinterpret_cast<Frag*>(lds + row * LDSROW + cv * Tr::HW) = v;
-      }
-      __syncthreads();
-      if (w.slab_ok) gate_mfma_held<IO, MT, NKG>(lds, hw, 0, w.slab, w.r, hf, 0.0f, 0.0f, ua[0], ux[0], xv);
-      __syncthreads();
-    } else {
-      gate_tile_generic<IO, MT>(p, x + (long long)b * p.T * W, t0, p.T, w.k, w.slab, w.slab_ok, w_a_row, w_x_row,
-                                0.0f, 0.0f, lds, ua, ux, xv);
-    }
+    gate_tile_generic<IO, MT>(p, x + (long long)b * p.T * W, t0, p.T, p.bpu > 1 ? w.unit * p.bpu : w.k, w.kb, w.slab, w.slab_ok, w_a_row, w_x_row,
+                              0.0f, 0.0f, lds, ua, ux, xv);
     if (!w.slab_ok) continue;
 
     const long long trow = (long long)b * p.T + t0 + hf * EL;
@@ -1490,7 +1474,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gate_grad_wide_kernel(FusedAr
 
 // Last launch of a backward pass: sums the per-workgroup partial results and writes the parameter
 // gradients in the caller's type.  Workgroups [0, vec_blocks) own 16 channels each of db_a, db_x and
-// dLambda; the rest (backward paths with their own weight-gradient GEMM) own 2048 elements each of the two weight
+// dLambda; the rest own 2048 elements each (256 where rows are no whole vectors) of the two weight
 // gradients, dW_gate[k][o][j] = sum over workgroups of the partials [wg][k][gate][o][j].
 struct FinishArgs {
   const float* partial; const float* dsp; void* db_a; void* db_x; void* dlambda;
@@ -1506,19 +1490,19 @@ RGLRU_DEVICE void gate_finish(const FinishArgs& p, int block, float (&part_sum)[
     // block width equals the padded width)
     const long long per_gate = (long long)p.bw * p.bw;
     if (!p.dw_vec) {
-      // any width, any alignment: eight elements of the unpadded gradients per thread, one at a time
-      const long long total = (long long)p.nb * 2 * per_gate;
-      const long long first = ((long long)(block - p.vec_blocks) * blockDim.x + threadIdx.x) * 8;
+      // any width, any alignment: one element of the unpadded gradients per thread (eight of them one after the other took
+      // 48 us for eight blocks of 85 channels)
+      const long long i = (long long)(block - p.vec_blocks) * blockDim.x + threadIdx.x;
+      if (i >= (long long)p.nb * 2 * per_gate) return;
       const long long stride = (long long)p.nb * 2 * p.bwp * p.bwp;
-      for (long long i = first; i < first + 8 && i < total; ++i) {
-        const int j = (int)(i % p.bw), o = (int)((i / p.bw) % p.bw);
-        const int gate = (int)((i / per_gate) % 2);
-        const long long k = i / (2 * per_gate);
-        const float* src = p.dw_partial + (((k * 2 + gate) * p.bwp + o) * p.bwp + j);
-        float sum = 0.f;
-        for (int g = 0; g < p.n_wg; ++g) sum += src[(long long)g * stride];
-        store_vec(gate ? p.dw_x : p.dw_a, (k * p.bw + o) * p.bw + j, sum, p.grad_dtype);
-      }
+      const long long k = i / (2 * per_gate);
+      const unsigned rem = (unsigned)(i - k * 2 * per_gate), gate = rem >= (unsigned)per_gate, in_gate = rem - gate * (unsigned)per_gate;
+      const unsigned o = in_gate / (unsigned)p.bw, j = in_gate - o * (unsigned)p.bw;
+      const float* src = p.dw_partial + (((k * 2 + gate) * p.bwp + o) * p.bwp + j);
+      float sum = 0.f;
+#pragma unroll 8
+      for (int g = 0; g < p.n_wg; ++g) sum += src[(long long)g * stride];
+      store_vec(gate ? p.dw_x : p.dw_a, (k * p.bw + o) * p.bw + j, sum, p.grad_dtype);
       return;
     }
     const long long total8 = (long long)p.nb * 2 * per_gate / 8;
@@ -1654,7 +1638,7 @@ static int gate_gemms_and_finish(const FusedArgs& a, const Geometry& g, const vo
   const ScratchLayout SL = make_scratch_layout(B, T, g, kScratchPlain);
   const int splits = gate_dw_splits(B * T, g);
   float* dw_partial = (float*)(scratch + SL.dw_partial);
-  int rc = launch_gate_gemms(x, du_a, du_x, du_ld, du_blk, a.w2t, dx, dw_partial, B * T, g, dtype, splits, s);
+  int rc = launch_gate_gemms(x, du_a, du_x, du_ld, du_blk, a.wg, a.w2t, dx, dw_partial, B * T, g, dtype, splits, s);
   if (rc) return rc;
   FinishArgs r;
   memset(&r, 0, sizeof(r));
@@ -1664,7 +1648,7 @@ static int gate_gemms_and_finish(const FusedArgs& a, const Geometry& g, const vo
   r.n_wg = splits; r.vec_blocks = (int)((g.W + 15) / 16); r.grad_dtype = grad_dtype;
   r.dw_vec = (g.bw % 8 == 0 && (uintptr_t)dw_a % 16 == 0 && (uintptr_t)dw_x % 16 == 0) ? 1 : 0;
   const long long total = g.nb * g.bw * 2 * g.bw;
-  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)(r.vec_blocks + (total / 8 + 255) / 256)), dim3(256), 0, s, r);
+  hipLaunchKernelGGL(finish_kernel, dim3((unsigned)(r.vec_blocks + (total / (r.dw_vec ? 8 : 1) + 255) / 256)), dim3(256), 0, s, r);
   return check_launch("bwd finish");
 }
 
@@ -1708,7 +1692,7 @@ int rglru_hip_bwd_pre(const void* x, void* pre, const void* prep, const float* h
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
   rc = launch_clear(wb, L.b_begin, L.b_end, s);          // records and tickets of this pass
   if (rc) return rc;
-  rc = launch_gate_pre_gemm(x, a.wg, pre, B * T, g, s);  // the gate projections again
+  rc = gate_pre_product(x, a.wg, pre, B * T, g, s);  // the gate projections again
   if (rc) return rc;
   {
     KernelTimer timer(1, s);
@@ -1757,6 +1741,7 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
   a.partial = (float*)((char*)scratch + make_scratch_layout(B, T, g, kScratchPlain).partial);
   a.B = (int)B; a.T = (int)T; a.nC = (int)((T + kChunk - 1) / kChunk); a.ckpt_nC = 2 * (int)L.nC; a.nCf = (int)L.nCf;
   a.aligned = is_aligned(x, W, g.bw, elem_size(dtype));
+  pack_units(a, g, 0);
   a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 2, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
@@ -1764,7 +1749,8 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
   if (rc) return rc;
   {
     KernelTimer timer(1, s);
-    RGLRU_DISPATCH(bwd_kernel, grid, s, a, dtype, held_groups(g, dtype, a.aligned));
+    if (dtype == RGLRU_BF16) hipLaunchKernelGGL(bwd_kernel<__bf16>, grid, dim3(kThreads), 0, s, a);
+    else hipLaunchKernelGGL(bwd_kernel<float>, grid, dim3(kThreads), 0, s, a);
   }
   rc = check_launch("bwd");
   if (rc) return rc;

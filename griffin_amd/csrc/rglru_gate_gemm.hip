@@ -16,6 +16,8 @@
 //     gathers its tokens one by one, and a wave-wide load is two rows of 32 consecutive channels: coalesced
 //     without any transposition.  The token axis is split over workgroups; every split writes a partial
 //     set [k][gate][o][j] that finish_kernel sums in a fixed order.
+// Blocks whose rows are whole 16-byte vectors run as batches of the dense products of rglru_linear.hip instead (slices of both
+// operands through LDS, requested ahead); the kernels here are for the others.
 // Any width up to 512 per block: rows and columns outside the block and tokens outside the tensor are
 // masked through the offsets of buffer loads (they read as zero) and stores (dropped).
 #include <hip/hip_runtime.h>
@@ -29,8 +31,8 @@
 namespace rglru {
 
 struct GateGemmArgs {
-  const void* x; const void* du_a; const void* du_x; const void* w2t; const void* wg;
-  void* dx; float* dw_partial; void* pre;
+  const void* x; const void* du_a; const void* du_x; const void* w2t;
+  void* dx; float* dw_partial;
   long long N;                    // tokens, B * T
   long long tokens_per_split;     // dW: tokens of one split (a multiple of the K group)
   long long du_ld, du_blk;        // du_g[n][k][o] sits at du_g + k * du_blk + n * du_ld + o (elements)
@@ -207,57 +209,6 @@ __global__ __launch_bounds__(kThreads) void gate_dw_gemm_kernel(GateGemmArgs p) 
     }
 }
 
-// Gate pre-activations without the bias for the bf16 block widths whose scan kernels take them as an operand
-// (multiples of 32 with no register-held variant): pre[k][n][g bw + o] = sum_j x[n, k bw + j] W_g[k][o][j].
-// A wave owns 32 tokens and walks the 2 bw / 32 output tiles kGemmJG at a time; both operands are 16 contiguous
-// bytes per lane (x rows; rows of the image's [gate][k][o][j] copy).
-__global__ __launch_bounds__(kThreads) void gate_pre_gemm_kernel(GateGemmArgs p) {
-  typedef Io<__bf16> Tr;
-  typedef Tr::Frag Frag;
-  constexpr int KG = Tr::KG, HW = Tr::HW;
-  const int lane = threadIdx.x & 63, r = lane & 31, hf = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int k = blockIdx.y;
-  const long long n0 = ((long long)blockIdx.x * kWaves + wave) * 32;
-  if (n0 >= p.N) return;
-  const int rows = (int)((p.N - n0) < 32 ? (p.N - n0) : 32);
-  const unsigned row_bytes = (unsigned)p.W * 2u, out_row_bytes = 4u * (unsigned)p.bw;
-  const rsrc_t rx = make_rsrc((const __bf16*)p.x + n0 * p.W, (unsigned)rows * row_bytes);
-  const rsrc_t rp = make_rsrc((__bf16*)p.pre + ((long long)k * p.N + n0) * (2 * p.bw), (unsigned)rows * out_row_bytes);
-  const __bf16* wg = (const __bf16*)p.wg;
-  const int T32 = p.bw / 32, OT = 2 * T32, NKG = p.bw / KG;
-  for (int ot0 = 0; ot0 < OT; ot0 += kGemmJG) {
-    f32x16 acc[kGemmJG];
-#pragma unroll
-    for (int jj = 0; jj < kGemmJG; ++jj)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[jj][v] = 0.f;
-    for (int kg = 0; kg < NKG; ++kg) {
-      const Frag fa = buf_load_frag<Frag>(rx, (unsigned)r * row_bytes + (unsigned)(k * p.bw + kg * KG + hf * HW) * 2u);
-#pragma unroll
-      for (int jj = 0; jj < kGemmJG; ++jj) {
-        const int ot = ot0 + jj;
-        if (ot < OT) {                                         // wave-uniform
-          const int g = ot / T32, o = (ot - g * T32) * 32 + r;
-          const Frag fb = *reinterpret_cast<const Frag*>(wg + ((long long)(g * p.nb + k) * p.bwp + o) * p.bwp + kg * KG + hf * HW);
-          Tr::mma(acc[jj], fa, fb);
-        }
-      }
-    }
-#pragma unroll
-    for (int jj = 0; jj < kGemmJG; ++jj) {
-      const int ot = ot0 + jj;
-      if (ot < OT) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = 8 * (v >> 2) + 4 * hf + (v & 3);
-          BufIo<__bf16>::store((__bf16)acc[jj][v], rp, (unsigned)m * out_row_bytes + (unsigned)(ot * 32 + r) * 2u, 0u);
-        }
-      }
-    }
-  }
-}
-
 // Partial sets of the weight-gradient GEMM for B * T = N tokens: enough splits of the token axis to give every
 // compute unit of a 256-unit part a workgroup, at least 64 tokens per split, at most kGemmWgPerUnit sets.
 int gate_dw_splits(long long N, const Geometry& g) {
@@ -271,19 +222,14 @@ int gate_dw_splits(long long N, const Geometry& g) {
   return (int)s;
 }
 
-int launch_gate_pre_gemm(const void* x, const void* wg, void* pre, long long N, const Geometry& g, hipStream_t s) {
-  GateGemmArgs a;
-  memset(&a, 0, sizeof(a));
-  a.x = x; a.wg = wg; a.pre = pre;
-  a.N = N; a.W = (int)g.W; a.nb = (int)g.nb; a.bw = (int)g.bw; a.bwp = (int)g.bwp;
-  const dim3 grid((unsigned)((N + 32 * kWaves - 1) / (32 * kWaves)), (unsigned)g.nb);
-  hipLaunchKernelGGL(gate_pre_gemm_kernel, grid, dim3(kThreads), 0, s, a);
-  return check_launch("gate pre-activation GEMM");
-}
-
 int launch_gate_gemms(const void* x, const void* du_a, const void* du_x, long long du_ld, long long du_blk,
-                      const void* w2t, void* dx, float* dw_partial, long long N, const Geometry& g, int dtype,
+                      const void* wg, const void* w2t, void* dx, float* dw_partial, long long N, const Geometry& g, int dtype,
                       int n_split, hipStream_t s) {
+  // B4 T1024 W1024 in fp32 (64-wide blocks): 27 + 56 us in the kernels of this file, latency of the operands' loads
+  if (gate_products_cover(g, dtype, {x, du_a, du_x, wg, dx}, {g.W, du_ld}) && du_blk % (dtype == RGLRU_BF16 ? 8 : 4) == 0) {
+    const int rc = gate_input_grad(du_a, du_x, du_ld, du_blk, wg, dx, N, g, dtype, s);
+    return rc ? rc : gate_weight_grad(du_a, du_x, du_ld, du_blk, x, dw_partial, n_split, N, g, dtype, s);
+  }
   GateGemmArgs a;
   memset(&a, 0, sizeof(a));
   a.x = x; a.du_a = du_a; a.du_x = du_x; a.w2t = w2t; a.dx = dx; a.dw_partial = dw_partial;

@@ -7,6 +7,7 @@
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/rglru_hip.h"
 
@@ -27,12 +28,22 @@ static __global__ void clear_words_kernel(unsigned* p, long long n) {
 }
 
 struct Geometry;
-// The block-diagonal GEMMs of the gate projections and their gradients (rglru_gate_gemm.hip).
+// The block-diagonal GEMMs of the gate projections and their gradients (rglru_gate_gemm.hip; as batches of the dense products
+// of rglru_linear.hip where a block's rows are whole 16-byte vectors).
 int gate_dw_splits(long long N, const Geometry& g);
-int launch_gate_pre_gemm(const void* x, const void* wg, void* pre, long long N, const Geometry& g, hipStream_t s);
 int launch_gate_gemms(const void* x, const void* du_a, const void* du_x, long long du_ld, long long du_blk,
-                      const void* w2t, void* dx, float* dw_partial, long long N, const Geometry& g, int dtype,
+                      const void* wg, const void* w2t, void* dx, float* dw_partial, long long N, const Geometry& g, int dtype,
                       int n_split, hipStream_t s);
+
+bool gate_products_cover(const Geometry& g, int dtype, std::initializer_list<const void*> tensors, std::initializer_list<long long> strides);
+// pre[k][n][g bw + o] = sum_j x[n, k bw + j] W_g[k][o][j] (bf16)
+int gate_pre_product(const void* x, const void* wg, void* pre, long long N, const Geometry& g, hipStream_t s);
+// dx[n, k bw + j] += sum over gates and o of du_g[n, k, o] W_g[k][o][j];  du_g[n, k, o] at du_g + k du_blk + n du_ld + o
+int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, long long N,
+                    const Geometry& g, int dtype, hipStream_t s);
+// partial[split][k][g][o][j] (blocks of bwp x bwp, the padding is not written) = sum over the split's n of du_g[n, k, o] x[n, k bw + j]
+int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* x, float* partial, int splits,
+                     long long N, const Geometry& g, int dtype, hipStream_t s);
 
 // The same for two ranges in one launch.
 static __global__ void clear_two_kernel(unsigned* p0, long long n0, unsigned* p1, long long n1) {

@@ -20,13 +20,19 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <initializer_list>
 
 #include "rglru_device.h"
 #include "rglru_host.h"
+#include "rglru_layout.h"
 
 namespace rglru {
 
 struct LinearArgs {
+  // `batch` equal problem sets side by side, operands a_step, b_step and c_step elements on: the gate blocks of the RG-LRU
+  long long a_step, b_step, c_step;
+  int batch, accumulate;             // accumulate: c += product, rounded once
+  int partial_ld;                    // partial: [split][batch][problem][partial_ld][partial_ld] where set, else [split][problem][M][N]
   const void* a[2]; const void* b[2]; const void* bias[2]; void* c[2];
   const unsigned char* active;       // one byte per token, or null: inactive rows of the result are zero (weight gradient: rows of A count as zero)
   float* partial;                    // [split][problem][M][N] instead of c where the contraction is split
@@ -134,8 +140,9 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   if ((int)(blockIdx.x >> 3) >= per_xcd || t >= p.total) return;
   const int tn = t % p.tiles_n; t /= p.tiles_n;
   const int problem = t % p.problems; t /= p.problems;
-  const int tm = t % p.tiles_m;
-  const int split = t / p.tiles_m;
+  const int tm = t % p.tiles_m; t /= p.tiles_m;
+  const int item = t % p.batch;
+  const int split = t / p.batch;
   const int m0 = tm * BM, n0 = tn * BN;
   const int m_left = p.M - m0, n_left = p.N - n0;
   const int k_begin = split * p.k_per_split;
@@ -152,8 +159,8 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   auto request = [&](int s) {
     const int seg = s >= slices ? 1 : 0;
     const int k = k_begin + (s - seg * slices) * BK;
-    const IO* a = (const IO*)p.a[p.segments > 1 ? seg : (TA ? problem : 0)];
-    const IO* b = (const IO*)p.b[p.segments > 1 ? seg : (TA ? 0 : problem)];
+    const IO* a = (const IO*)p.a[p.segments > 1 ? seg : (TA ? problem : 0)] + item * p.a_step;
+    const IO* b = (const IO*)p.b[p.segments > 1 ? seg : (TA ? 0 : problem)] + item * p.b_step;
     const int left = s < total_slices ? k_end - k : 0;
     const long long ks = s < total_slices ? k : 0;
     ta.request(a + (TA ? ks * p.lda + m0 : m0 * p.lda + ks), p.lda, left, m_left, tid, masked ? p.active + ks : nullptr);
@@ -168,6 +175,20 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  if (p.accumulate) {
+    const rsrc_t rc = make_rsrc((const IO*)p.c[problem] + item * p.c_step + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      const int n = wn * (BN / 2) + 32 * j + r;
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int m = wm * (BM / 2) + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
+          acc[i][j][v] = BufIo<IO>::load(rc, n < n_left ? ((unsigned)m * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange, 0u);
+        }
+    }
+  }
   float sum[MI];                                             // column sums of A over the lane's share of K
 #pragma unroll
   for (int i = 0; i < MI; ++i) sum[i] = 0.f;
@@ -215,8 +236,9 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   }
   const int col0 = wn * (BN / 2), row0 = wm * (BM / 2);
   if (p.partial) {
-    float* part = p.partial + (((long long)split * p.problems + problem) * p.M + m0) * p.N + n0;
-    const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.N) * 4u);
+    const int ld = p.partial_ld ? p.partial_ld : p.N, rows = p.partial_ld ? p.partial_ld : p.M;
+    float* part = p.partial + ((((long long)split * p.batch + item) * p.problems + problem) * rows + m0) * ld + n0;
+    const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * ld) * 4u);
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int n = col0 + 32 * j + r;
@@ -225,7 +247,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const int m = row0 + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
-          BufIo<float>::store(acc[i][j][v], rc, n < n_left ? ((unsigned)m * (unsigned)p.N + (unsigned)n) * 4u : kOutOfRange, 0u);
+          BufIo<float>::store(acc[i][j][v], rc, n < n_left ? ((unsigned)m * (unsigned)ld + (unsigned)n) * 4u : kOutOfRange, 0u);
         }
     }
     return;
@@ -248,7 +270,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
         stage[m * kStageRow + 32 * j + r] = (IO)(acc[i][j][v] + bias[j]);
       }
   wave_lds_fence();
-  const rsrc_t rc = make_rsrc((IO*)p.c[problem] + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
+  const rsrc_t rc = make_rsrc((IO*)p.c[problem] + item * p.c_step + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
   constexpr int VPR = (BN / 2) / Tr::HW, ROWS = 64 / VPR;
 #pragma unroll
   for (int q = 0; q < (BM / 2) / ROWS; ++q) {
@@ -256,8 +278,8 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     Frag f = *reinterpret_cast<const Frag*>(stage + m * kStageRow + cv * Tr::HW);
     const int row = row0 + m, n = col0 + cv * Tr::HW;
     if (!TA && p.active && row < m_left && !p.active[m0 + row]) f = Tr::zero();
-    buf_store_b128(__builtin_bit_cast(i32x4, f), rc,
-                   n < n_left && row < m_left ? ((unsigned)row * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange);
+    const unsigned off = n < n_left && row < m_left ? ((unsigned)row * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange;
+    buf_store_b128(__builtin_bit_cast(i32x4, f), rc, off);
   }
 }
 
@@ -289,10 +311,76 @@ static void linear_launch(LinearArgs& a, bool large, hipStream_t s) {
   const int edge = large ? 128 : 64;
   a.tiles_m = (a.M + edge - 1) / edge;
   a.tiles_n = (a.N + edge - 1) / edge;
-  a.total = a.tiles_m * a.tiles_n * a.problems * a.splits;
+  a.total = a.tiles_m * a.tiles_n * a.problems * a.batch * a.splits;
   const dim3 grid((unsigned)(8 * ((a.total + 7) / 8)));
   if (large) hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 128, 128>), grid, dim3(kLinearThreads), 0, s, a);
   else hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 64, 64>), grid, dim3(kLinearThreads), 0, s, a);
+}
+
+static void linear_launch(LinearArgs& a, int kind, bool large, int dtype, hipStream_t s) {
+  if (dtype == RGLRU_BF16) {
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, large, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<__bf16, false, true>(a, large, s);
+    else linear_launch<__bf16, true, true>(a, large, s);
+  } else {
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, large, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, large, s);
+    else linear_launch<float, true, true>(a, large, s);
+  }
+}
+
+// ---- the gate blocks' products (griffin/griffin.py:149-154 and their reverse mode) as batches ----------------------
+// For the configurations whose scan kernels leave the gradients at the gate pre-activations in memory.  Tiles of 128 where
+// the block is wider than 64 channels and there are enough of them.
+static bool batch_large(const Geometry& g, long long tokens_or_width, int problems) {
+  return g.bw > 64 && ((tokens_or_width + 127) / 128) * ((g.bw + 127) / 128) * g.nb * problems >= num_compute_units();
+}
+
+bool gate_products_cover(const Geometry& g, int dtype, std::initializer_list<const void*> tensors, std::initializer_list<long long> strides) {
+  const int vec = dtype == RGLRU_BF16 ? 8 : 4;
+  if (g.bw % vec || g.W % vec) return false;
+  for (const void* q : tensors) if ((uintptr_t)q % 16) return false;
+  for (long long v : strides) if (v % vec || v >= (1 << 22)) return false;
+  return true;
+}
+
+int gate_pre_product(const void* x, const void* wg, void* pre, long long N, const Geometry& g, hipStream_t s) {
+  LinearArgs a;
+  memset(&a, 0, sizeof(a));
+  const long long gate = g.nb * g.bwp * g.bwp;
+  a.a[0] = x; a.b[0] = wg; a.b[1] = (const __bf16*)wg + gate; a.c[0] = pre; a.c[1] = (__bf16*)pre + g.bw;
+  a.lda = g.W; a.ldb = g.bwp; a.ldc = 2 * g.bw; a.a_step = g.bw; a.b_step = g.bwp * g.bwp; a.c_step = N * 2 * g.bw;
+  a.batch = (int)g.nb; a.problems = 2; a.segments = 1; a.splits = 1;
+  a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
+  linear_launch(a, RGLRU_LINEAR_FORWARD, batch_large(g, N, 2), RGLRU_BF16, s);
+  return check_launch("gate pre-activations");
+}
+
+int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, long long N,
+                    const Geometry& g, int dtype, hipStream_t s) {
+  LinearArgs a;
+  memset(&a, 0, sizeof(a));
+  const long long gate = g.nb * g.bwp * g.bwp;
+  a.a[0] = du_a; a.a[1] = du_x; a.b[0] = wg; a.b[1] = (const char*)wg + gate * (dtype == RGLRU_BF16 ? 2 : 4); a.c[0] = dx;
+  a.lda = du_ld; a.ldb = g.bwp; a.ldc = g.W; a.a_step = du_blk; a.b_step = g.bwp * g.bwp; a.c_step = g.bw;
+  a.batch = (int)g.nb; a.problems = 1; a.segments = 2; a.splits = 1; a.accumulate = 1;
+  a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
+  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, batch_large(g, N, 1), dtype, s);
+  return check_launch("gate input gradient");
+}
+
+int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* x, float* partial, int splits,
+                     long long N, const Geometry& g, int dtype, hipStream_t s) {
+  LinearArgs a;
+  memset(&a, 0, sizeof(a));
+  a.a[0] = du_a; a.a[1] = du_x; a.b[0] = x; a.partial = partial; a.partial_ld = (int)g.bwp;
+  a.lda = du_ld; a.ldb = g.W; a.a_step = du_blk; a.b_step = g.bw;
+  a.batch = (int)g.nb; a.problems = 2; a.segments = 1; a.splits = splits;
+  a.M = a.N = (int)g.bw; a.K = (int)N;
+  const long long bk = dtype == RGLRU_BF16 ? 64 : 32;
+  a.k_per_split = (int)(((N + splits - 1) / splits + bk - 1) / bk * bk);
+  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, batch_large(g, g.bw, 2 * splits), dtype, s);
+  return check_launch("gate weight gradients");
 }
 
 }  // namespace rglru
@@ -315,7 +403,7 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
   LinearArgs a;
   memset(&a, 0, sizeof(a));
   a.a[0] = a0; a.a[1] = a1; a.b[0] = b0; a.b[1] = b1; a.bias[0] = bias0; a.bias[1] = bias1; a.c[0] = c0; a.c[1] = c1;
-  a.active = active; a.colsum = colsum; a.lda = lda; a.ldb = ldb; a.ldc = ldc;
+  a.batch = 1; a.active = active; a.colsum = colsum; a.lda = lda; a.ldb = ldb; a.ldc = ldc;
   a.problems = kind == RGLRU_LINEAR_FORWARD ? (b1 ? 2 : 1) : kind == RGLRU_LINEAR_WEIGHT_GRAD ? (a1 ? 2 : 1) : 1;
   a.segments = kind == RGLRU_LINEAR_INPUT_GRAD && a1 ? 2 : 1;
   const LinearPlan plan = linear_plan(kind, M, N, K, a.problems, dtype);
@@ -337,15 +425,7 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
   const int64_t bk = dtype == RGLRU_BF16 ? 64 : 32;
   a.k_per_split = (int)(((K + a.splits - 1) / a.splits + bk - 1) / bk * bk);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == RGLRU_BF16) {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, plan.large, s);
-    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<__bf16, false, true>(a, plan.large, s);
-    else linear_launch<__bf16, true, true>(a, plan.large, s);
-  } else {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, plan.large, s);
-    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, plan.large, s);
-    else linear_launch<float, true, true>(a, plan.large, s);
-  }
+  linear_launch(a, kind, plan.large, dtype, s);
   return check_launch("linear");
 }
 

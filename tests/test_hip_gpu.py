@@ -923,3 +923,22 @@ def test_decode_of_blocks_that_end_inside_a_step(bw, nb, B):
     many = case["h0"].cuda().contiguous()
     ys = hip_rglru_steps(x.transpose(0, 1).contiguous().cuda(), prep, many)
     assert rel_err(many, state) < 1e-6 and rel_err(ys.transpose(0, 1).float(), rows.float()) < 1e-6
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, FP32_TOL), (torch.bfloat16, BF16_TOL)])
+@pytest.mark.parametrize("bw,nb", [(7, 5), (21, 8), (32, 3), (36, 7), (64, 3), (68, 2), (130, 2), (152, 3)])
+def test_portable_kernels_pack_narrow_blocks(bw, nb, dtype, tol):
+    """Blocks the portable kernels take: several to a workgroup up to 64 channels (the last workgroup's share not full), gate
+    gradients as batches of dense products where rows are whole vectors, element by element elsewhere; ragged lengths and masks."""
+    B, T, W = 3, 77, bw * nb
+    print("portable", bw, nb, dtype, flush=True)
+    case = orc.make_case(B, T, W, nb, seed=bw + nb, h0_std=0.5, bias_std=0.3)
+    reset = torch.zeros(B, T, dtype=torch.bool)
+    reset[:, 40] = True
+    active = torch.ones(B, T, dtype=torch.bool)
+    active[1, -9:] = False
+    y, h_last, grads = hip_run(case, dtype, reset, active, None)
+    ry, rh, rgrads = oracle_run(case, dtype, reset, active, None)
+    assert rel_err(y.float(), ry) < tol and rel_err(h_last, rh) < tol
+    for name in rgrads:
+        assert rel_err(grads[name].float(), rgrads[name]) < tol, name
