@@ -16,6 +16,9 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <atomic>
 #include <optional>
 #include <string>
 #include <tuple>
@@ -392,17 +395,26 @@ py::tuple fingerprint(const std::vector<Tensor>& tensors) {
   return out;
 }
 
-// The same, kept on this side and compared here: a decode loop asks every step.
+// What a prepared parameter image was made from, compared on this side: a decode loop asks every step.
 struct Stamp {
   std::vector<std::pair<const void*, int64_t>> seen;
-  explicit Stamp(const std::vector<Tensor>& tensors) {
+  Tensor image;
+  int64_t blocks;
+  double c;
+  at::ScalarType dtype;
+  Stamp(const std::vector<Tensor>& tensors, const Tensor& img, int64_t nb, double decay, at::ScalarType type)
+      : image(img), blocks(nb), c(decay), dtype(type) {
     for (const Tensor& t : tensors) seen.emplace_back(t.data_ptr(), static_cast<int64_t>(t._version()));
   }
-  bool matches(const std::vector<Tensor>& tensors) const {
-    if (tensors.size() != seen.size()) return false;
-    for (size_t i = 0; i < seen.size(); ++i)
+  template <typename Tensors>
+  bool holds(const Tensors& tensors, size_t n, double decay, at::ScalarType type) const {
+    if (n != seen.size() || c != decay || dtype != type) return false;
+    for (size_t i = 0; i < n; ++i)
       if (tensors[i].data_ptr() != seen[i].first || static_cast<int64_t>(tensors[i]._version()) != seen[i].second) return false;
     return true;
+  }
+  bool matches(const std::vector<Tensor>& tensors, double decay, at::ScalarType type, c10::Device device) const {
+    return image.device() == device && holds(tensors, tensors.size(), decay, type);
   }
 };
 
@@ -1018,6 +1030,122 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
   check(rglru_hip_decode_linear(sp + 2 * row_bytes, W, ptr(w_o), ptr(b_o), bptr(active), ptr(out), B, D, W, code, stream),
         "rglru_hip_decode_linear");
   return std::make_tuple(out, h_out, new_conv, new_pos);
+}
+
+// ---- single-token calls of the modules ----------------------------------------------------------------------------
+// What a module's forward does around a decode step -- look up its parameters, check shapes, types and the prepared image --
+// costs the interpreter more than the step's launches take (layer: 5 of 9 us, block: 8 of 18).  These read the module's own
+// dictionaries and do it here.  None: not the plain case, the module's Python code goes on (and reports what is wrong).
+
+std::atomic<uint64_t> usable_devices{0};                   // GPUs whose one-time self-test has passed
+void mark_usable(int64_t device, bool usable) {
+  if (device < 0 || device >= 64) return;
+  if (usable) usable_devices |= uint64_t(1) << device; else usable_devices &= ~(uint64_t(1) << device);
+}
+
+// Members of an nn.Module as its instance dictionary holds them (borrowed references; null where missing).
+struct Members {
+  PyObject* dict;
+  explicit Members(PyObject* module) : dict(nullptr) {
+    PyObject** d = module != nullptr ? _PyObject_GetDictPtr(module) : nullptr;
+    if (d != nullptr) dict = *d;
+  }
+  PyObject* at(const char* name) const { return dict != nullptr ? PyDict_GetItemString(dict, name) : nullptr; }
+  static PyObject* in(PyObject* d, const char* name) { return d != nullptr && PyDict_Check(d) ? PyDict_GetItemString(d, name) : nullptr; }
+  PyObject* module(const char* name) const { return in(at("_modules"), name); }
+  bool parameter(const char* name, Tensor& t) const {
+    PyObject* p = in(at("_parameters"), name);
+    if (p == nullptr || !THPVariable_Check(p)) return false;
+    t = THPVariable_Unpack(p);
+    return true;
+  }
+  double number(const char* name, double otherwise) const {
+    PyObject* v = at(name);
+    return v == nullptr ? otherwise : PyFloat_Check(v) ? PyFloat_AS_DOUBLE(v) : PyLong_Check(v) ? PyLong_AsDouble(v) : otherwise;
+  }
+  bool hooked() const {
+    for (const char* name : {"_forward_hooks", "_forward_pre_hooks"}) {
+      PyObject* h = at(name);
+      if (h == nullptr || PyObject_Length(h) != 0) return true;
+    }
+    return false;
+  }
+};
+
+bool usable_mode(const Members& lru, c10::Device device) {
+  PyObject* mode = lru.at("scan_mode");
+  if (mode == nullptr || !PyUnicode_Check(mode)) return false;
+  if (PyUnicode_CompareWithASCIIString(mode, "auto") == 0) return (usable_devices.load(std::memory_order_relaxed) >> device.index()) & 1;
+  return PyUnicode_CompareWithASCIIString(mode, "hip") == 0 || PyUnicode_CompareWithASCIIString(mode, "fused") == 0;
+}
+
+// The prepared image an RG_LRU module keeps, if it is that of its parameters as they are now.
+const Stamp* current_stamp(const Members& lru, at::ScalarType dtype, c10::Device device) {
+  PyObject* held = lru.at("_prep_key");
+  if (held == nullptr || held == Py_None || !py::isinstance<Stamp>(held)) return nullptr;
+  const Members r(lru.module("recurrence_gate")), i(lru.module("input_gate"));
+  std::array<Tensor, 5> p;
+  if (!r.parameter("weight", p[0]) || !r.parameter("bias", p[1]) || !i.parameter("weight", p[2]) || !i.parameter("bias", p[3]) ||
+      !lru.parameter("Lambda", p[4]))
+    return nullptr;
+  const Stamp* s = py::handle(held).cast<const Stamp*>();
+  return s->image.device() == device && s->holds(p, p.size(), lru.number("c", 0.0), dtype) ? s : nullptr;
+}
+
+// RG_LRU on one token per row without masks: (y, state).
+py::object lru_decode(py::handle module, const Tensor& x, const MaybeTensor& state) {
+  if (at::GradMode::is_enabled() || x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0) return py::none();
+  const Members lru(module.ptr());
+  if (x.size(2) != (int64_t)lru.number("rnn_width", -1) || !usable_mode(lru, x.device())) return py::none();
+  if (state.has_value() && (state->dim() != 2 || state->size(0) != x.size(0) || state->size(1) != x.size(2) || state->scalar_type() != at::kFloat ||
+                            state->device() != x.device()))
+    return py::none();
+  const Stamp* s = current_stamp(lru, x.scalar_type(), x.device());
+  if (s == nullptr) return py::none();
+  auto [y, h] = rglru_module_step(x, s->image, s->blocks, state, std::nullopt);
+  return py::make_tuple(y, h);
+}
+
+// RecurrentBlock on one token per row, every row active, positions carried on: (output, rnn_state, conv_state, positions).
+py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py::handle linear_type) {
+  if (at::GradMode::is_enabled() || x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0 ||
+      at::autocast::is_autocast_enabled(at::kCUDA))
+    return py::none();
+  const Members block(module.ptr());
+  PyObject* layers[4] = {block.module("linear_x"), block.module("linear_y"), block.module("linear_out"), block.module("temporal_conv")};
+  for (int i = 0; i < 3; ++i)
+    if (layers[i] == nullptr || (PyObject*)Py_TYPE(layers[i]) != linear_type.ptr()) return py::none();
+  const Members lx(layers[0]), ly(layers[1]), lo(layers[2]), conv(layers[3]), lru(block.module("rg_lru"));
+  if (lx.hooked() || ly.hooked() || lo.hooked() || !usable_mode(lru, x.device())) return py::none();
+  Tensor wx, bx, wy, by, cw, cb, wo, bo;
+  if (!lx.parameter("weight", wx) || !lx.parameter("bias", bx) || !ly.parameter("weight", wy) || !ly.parameter("bias", by) ||
+      !conv.parameter("weight", cw) || !conv.parameter("bias", cb) || !lo.parameter("weight", wo) || !lo.parameter("bias", bo))
+    return py::none();
+  const int64_t B = x.size(0), W = (int64_t)block.number("rnn_width", -1), K = (int64_t)block.number("conv_kernel_size", -1);
+  if (wx.dim() != 2 || wx.size(0) != W || wx.size(1) != x.size(2) || wy.sizes() != wx.sizes() || wo.dim() != 2 || wo.size(1) != W ||
+      cw.dim() != 3 || cw.size(2) != K || wx.scalar_type() != x.scalar_type())
+    return py::none();
+  MaybeTensor conv_state, prev, rnn;
+  if (!cache.is_none()) {
+    auto field = [&](const char* name, MaybeTensor& t) {
+      py::object v = py::reinterpret_steal<py::object>(PyObject_GetAttrString(cache.ptr(), name));
+      if (!v) { PyErr_Clear(); return false; }
+      if (v.is_none()) return true;
+      if (!THPVariable_Check(v.ptr())) return false;
+      t = THPVariable_Unpack(v.ptr());
+      return t->device() == x.device();
+    };
+    if (!field("conv_state", conv_state) || !field("segment_position", prev) || !field("rnn_state", rnn)) return py::none();
+    if (!conv_state || !prev || conv_state->dim() != 3 || conv_state->size(0) != B || conv_state->size(1) != K - 1 || conv_state->size(2) != W ||
+        prev->dim() != 1 || prev->size(0) != B || prev->scalar_type() != at::kLong || !prev->is_contiguous())
+      return py::none();
+    if (rnn && (rnn->dim() != 2 || rnn->size(0) != B || rnn->size(1) != W)) return py::none();
+  }
+  const Stamp* s = current_stamp(lru, x.scalar_type(), x.device());
+  if (s == nullptr) return py::none();
+  auto done = block_step(x, wx, bx, wy, by, cw, cb, wo, bo, conv_state, prev, std::nullopt, std::nullopt, s->image, s->blocks, rnn);
+  if (!done.has_value()) return py::none();
+  return py::cast(*done);
 }
 
 // ---- Linear layers of the block (griffin/griffin.py:379-389) ------------------------------------------------------
@@ -1649,6 +1777,19 @@ Tensor rmsnorm(const Tensor& x, const Tensor& g, double eps) {
   return std::get<2>(rmsnorm_forward(x, g, eps, false));
 }
 
+// RMSNorm.forward where the kernels take x.
+py::object norm_forward(py::handle module, const Tensor& x) {
+  if (!x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0 || x.dim() < 1 || !((usable_devices.load(std::memory_order_relaxed) >> x.device().index()) & 1))
+    return py::none();
+  const Members norm(module.ptr());
+  Tensor g;
+  if (!norm.parameter("g", g) || g.dim() != 1 || g.size(0) != x.size(-1) || !g.is_cuda()) return py::none();
+  const bool bf16 = x.scalar_type() == at::kBFloat16;
+  const int code = code_of(x.scalar_type());
+  if (x.size(-1) > rglru_hip_rmsnorm_max_width(code, x.size(-1) % (bf16 ? 8 : 4) == 0)) return py::none();
+  return py::cast(rmsnorm(x, g, norm.number("eps", 1e-6)));
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
@@ -1656,7 +1797,13 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(kernel_path);
   EXPORT(prepare);
   EXPORT(fingerprint);
-  py::class_<Stamp>(m, "Stamp").def(py::init<const std::vector<Tensor>&>()).def("matches", &Stamp::matches);
+  py::class_<Stamp>(m, "Stamp")
+      .def(py::init<const std::vector<Tensor>&, const Tensor&, int64_t, double, at::ScalarType>())
+      .def("matches", &Stamp::matches);
+  EXPORT(mark_usable);
+  EXPORT(lru_decode);
+  EXPORT(block_decode);
+  EXPORT(norm_forward);
   EXPORT(rglru);
   EXPORT(rglru_step);
   EXPORT(rglru_steps);

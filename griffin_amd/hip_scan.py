@@ -139,7 +139,6 @@ class PreparedParams:
         self.blocks = nb
         self.dtype = dtype
         self.c = float(c)
-        self.device = w_a.device
         _dtype_code(dtype)
         self.image = _lib.native().prepare(w_a, b_a, w_x, b_x, lam, self.c, dtype)
 
@@ -194,9 +193,9 @@ def fingerprint(tensors) -> tuple:
         v for t in tensors for v in (t.data_ptr(), t._version))
 
 
-def parameter_stamp(tensors):
-    """The same as an object with ``matches(tensors)``, for callers that ask often."""
-    return _lib.native().Stamp(tensors)
+def parameter_stamp(tensors, prep: PreparedParams):
+    """What ``prep`` was made from, as an object with ``matches(tensors, c, dtype, device)``, for callers that ask often."""
+    return _lib.native().Stamp(tensors, prep.image, prep.blocks, prep.c, prep.dtype)
 
 
 def hip_rglru_steps(xs: Tensor, prep: PreparedParams, state: Tensor, flags: Tensor | None = None) -> Tensor:
@@ -411,4 +410,5 @@ def hip_scan_is_usable(device: torch.device | str) -> bool:
             )
         else:
             _VALIDATED[index] = True
+        _lib.native().mark_usable(index, _VALIDATED[index])
         return _VALIDATED[index]

@@ -20,7 +20,7 @@ from torch import Tensor
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import hip_block_ops, hip_scan, portable
+from . import _lib, hip_block_ops, hip_scan, portable
 
 ScanMode = Literal["auto", "sequential", "associative", "hip", "fused"]
 SCAN_MODES = ("auto", "sequential", "associative", "hip", "fused")
@@ -117,14 +117,13 @@ class RG_LRU(nn.Module):
         params = self._gate_parameters()
         held = self.__dict__
         prep, stamp = held.get("_prep"), held.get("_prep_key")
-        if (prep is not None and stamp is not None and prep.dtype is dtype and prep.device == device and prep.c == self.c
-                and stamp.matches(params)):
+        if prep is not None and stamp is not None and stamp.matches(params, self.c, dtype, device):
             return prep
         prep = hip_scan.PreparedParams(*params, self.c, dtype)
         if device.type == "cuda" and torch.cuda.is_current_stream_capturing():
             return prep                                      # allocated by the graph being captured: this call only
         self._prep = prep
-        self._prep_key = hip_scan.parameter_stamp(params)
+        self._prep_key = hip_scan.parameter_stamp(params, prep)
         return prep
 
     def invalidate_caches(self) -> None:
@@ -156,6 +155,11 @@ class RG_LRU(nn.Module):
         active_mask: Tensor | None = None,
         return_state: bool = False,
     ):
+        native = _lib._native_module
+        if native is not None and reset_mask is None and active_mask is None and type(self) is RG_LRU and not torch.is_grad_enabled():
+            done = native.lru_decode(self, xt, ht_minus_1)   # one token per row, nothing unusual
+            if done is not None:
+                return done if return_state else done[0]
         if xt.dim() != 3:
             raise ValueError(f"RG_LRU expects [batch, sequence, width], got {tuple(xt.shape)}")
         batch, steps, width = xt.shape
@@ -311,6 +315,11 @@ class RMSNorm(nn.Module):
         return x.size(-1) <= hip_block_ops.rmsnorm_max_width(x.dtype, aligned)
 
     def forward(self, x: Tensor) -> Tensor:
+        native = _lib._native_module
+        if native is not None:
+            done = native.norm_forward(self, x)
+            if done is not None:
+                return done
         if self._hip_covers(x):
             return hip_block_ops.hip_rmsnorm(x, self.g, self.eps)
         normalized = x * torch.rsqrt(x.pow(2).mean(dim=-1, keepdim=True) + self.eps)
@@ -626,6 +635,12 @@ class RecurrentBlock(nn.Module):
 
     def forward(self, x: Tensor, cache: RecurrentBlockCache | None = None, segment_pos: Tensor | None = None,
                 *, active_mask: Tensor | None = None, return_cache: bool = False):
+        native = _lib._native_module
+        if native is not None and segment_pos is None and active_mask is None and type(self) is RecurrentBlock and not torch.is_grad_enabled():
+            done = native.block_decode(self, x, cache, nn.Linear)    # one token per row, nothing unusual
+            if done is not None:
+                output, rnn_state, conv_state, position = done
+                return (output, RecurrentBlockCache(rnn_state, conv_state, position)) if return_cache else output
         if x.dim() != 3:
             raise ValueError(f"RecurrentBlock expects [batch, sequence, width], got {tuple(x.shape)}")
         batch, steps = x.shape[:2]
