@@ -74,8 +74,9 @@ _SIGNATURES = {
     "rglru_hip_linear_splits": (ctypes.c_int64, [ctypes.c_int, _I, _I, _I, ctypes.c_int, ctypes.c_int]),
     "rglru_hip_linear": (ctypes.c_int, [ctypes.c_int, _P, _P, _I, _P, _P, _I] + [_P] * 5 + [_I, _P, _P, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_sums": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P]),
-    "rglru_hip_block_bwd": (ctypes.c_int, [_P] * 15 + [_I] * 6 + [_P]),
-    "rglru_hip_block_finish": (ctypes.c_int, [_P] * 11 + [ctypes.c_int] + [_I] * 5 + [_P]),
+    "rglru_hip_block_sums_bytes": (ctypes.c_size_t, [_I, _I, _I, _I]),
+    "rglru_hip_block_bwd": (ctypes.c_int, [_P] * 16 + [_I] * 6 + [_P]),
+    "rglru_hip_block_finish": (ctypes.c_int, [_P] * 14 + [ctypes.c_int] + [_I] * 5 + [_P]),
     "rglru_hip_decode_prepare": (ctypes.c_int, [_P, _I] + [_P] * 10 + [_I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_decode_linear": (ctypes.c_int, [_P, _I] + [_P] * 4 + [_I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_decode_project": (ctypes.c_int, [_P, _I] + [_P] * 15 + [_I, _I, _I, _I, ctypes.c_int, _P]),
@@ -84,7 +85,7 @@ _SIGNATURES = {
     "rglru_hip_block_fwd": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _P, _I, ctypes.c_int] + [_P] * 9
                             + [_I, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_prepare_block_fwd": (ctypes.c_int, [_P] * 5 + [ctypes.c_float, ctypes.c_int, _P]
-                                    + [_P, _I, _P, _I, _P, _P, _P, _I] + [_P] * 8
+                                    + [_P, _I, _P, _I, _P, _P, _P, _I] + [_P] * 8 + [_P] * 3 + [_I]
                                     + [_I, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_block_infer": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _P, _I, ctypes.c_int] + [_P] * 10
                               + [_I, _I, _I, _I, ctypes.c_int, _P]),

@@ -42,6 +42,7 @@ struct ConvArgs {
   // arbitrary masks).  Null: every row has T tokens.
   const int* rows;
   int B, T, W, K, nvec, runs, vec_dtype;
+  int sum_du;                                               // backward: the partials hold the column sums of du too (row K + 1)
 };
 
 // Tokens of row b these kernels work on (inputs past them read as zero), or -1 where the row is not theirs.
@@ -270,10 +271,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_fwd_kernel(ConvArgs p) {
 // Backward: du, the gradient at the carried state (optional) and partial sums of the tap and bias
 // gradients.  A workgroup covers kConvBwdVecs channel vectors and kConvBwdRuns consecutive runs of
 // one sequence and adds the sums of its runs up in LDS:
-//   partial[((b * run_groups + run_group) * (K + 1) + j) * W + c],  j = K for the bias.
+//   partial[((b * run_groups + run_group) * (K + 1) + j) * W + c],  j = K for the bias (rows of K + 2 with sum_du).
 template <typename IO, int V, int K>
 __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvArgs p) {
-  __shared__ float red[kConvBwdRuns][(K + 1) * V][kConvBwdVecs + 1];
+  __shared__ float red[kConvBwdRuns][(K + 2) * V][kConvBwdVecs + 1];
   const int vec_groups = (p.nvec + kConvBwdVecs - 1) / kConvBwdVecs;
   const int run_groups = (p.runs + kConvBwdRuns - 1) / kConvBwdRuns;
   const int vg = blockIdx.x % vec_groups;
@@ -304,10 +305,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvArgs p) {
   float dwin[K][V];                                        // dwin[j] = dout row t + j
   long long spw[K];
   float uwin[K > 1 ? K - 1 : 1][V];                        // uwin[j] = padded row t - 1 - j
-  float acc_tap[K][V], acc_bias[V];
+  float acc_tap[K][V], acc_bias[V], acc_du[V];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    acc_bias[v] = 0.f;
+    acc_bias[v] = 0.f; acc_du[v] = 0.f;
 #pragma unroll
     for (int j = 0; j < K; ++j) acc_tap[j][v] = 0.f;
   }
@@ -343,6 +344,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvArgs p) {
         for (int lag = 0; lag < K; ++lag)
           if (spw[lag] >= lag) a = fmaf(dwin[lag][v], tap[K - 1 - lag][v], a);
         g[v] = a;
+        acc_du[v] += a;
         // parameter gradients of output t
         const float d = dwin[0][v];
         acc_bias[v] += d;
@@ -398,10 +400,11 @@ __global__ __launch_bounds__(kConvThreads) void conv_bwd_kernel(ConvArgs p) {
 #pragma unroll
     for (int v = 0; v < V; ++v) red[lane_run][j * V + v][lane_vec] = acc_tap[j][v];
 #pragma unroll
-  for (int v = 0; v < V; ++v) red[lane_run][K * V + v][lane_vec] = acc_bias[v];
+  for (int v = 0; v < V; ++v) { red[lane_run][K * V + v][lane_vec] = acc_bias[v]; red[lane_run][(K + 1) * V + v][lane_vec] = acc_du[v]; }
   __syncthreads();
-  float* part = p.partial + ((long long)(b * run_groups + rgp) * (K + 1)) * p.W;
-  for (int idx = threadIdx.x; idx < (K + 1) * V * kConvBwdVecs; idx += kConvThreads) {
+  const int sums = K + 1 + p.sum_du;
+  float* part = p.partial + ((long long)(b * run_groups + rgp) * sums) * p.W;
+  for (int idx = threadIdx.x; idx < sums * V * kConvBwdVecs; idx += kConvThreads) {
     const int row = idx / kConvBwdVecs, lv = idx - row * kConvBwdVecs;   // row = j * V + v
     const int j = row / V, v = row - j * V;
     const int ch = (vg * kConvBwdVecs + lv) * V + v;
@@ -1231,7 +1234,7 @@ size_t rglru_hip_conv_scratch_bytes(int64_t B, int64_t T, int64_t W, int64_t K) 
   if (B <= 0 || T <= 0 || W <= 0 || K < 1 || K > kConvMaxTaps) return 0;
   const int64_t runs = (T + kConvRunBwd - 1) / kConvRunBwd;
   const int64_t run_groups = (runs + kConvBwdRuns - 1) / kConvBwdRuns;
-  return (size_t)(B * run_groups * (K + 1) * W * 4);
+  return (size_t)(B * run_groups * (K + 2) * W * 4);
 }
 
 int rglru_hip_conv_bwd(const void* u, const void* state, const void* taps, const int64_t* segment_pos,
@@ -1251,7 +1254,7 @@ int64_t rglru::conv_partial_sets(int64_t B, int64_t T) {
 
 int rglru::conv_bwd_partials(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
                              const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate,
-                             int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, void* stream) {
+                             int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, bool sum_du, void* stream) {
   int rc = conv_check("conv_bwd", B, T, W, K, dtype, vec_dtype);
   if (rc) return rc;
   if (du_stride == 0) du_stride = W;
@@ -1263,7 +1266,7 @@ int rglru::conv_bwd_partials(const void* u, const void* state, const void* taps,
   memset(&a, 0, sizeof(a));
   a.u = u; a.state = state; a.taps = taps; a.segpos = (const long long*)segment_pos;
   a.dout = dout; a.du = du; a.dstate = dstate; a.partial = (float*)scratch; a.ld_du = du_stride;
-  a.rows = rows;
+  a.rows = rows; a.sum_du = sum_du;
   a.B = (int)B; a.T = (int)T; a.W = (int)W; a.K = (int)K; a.vec_dtype = vec_dtype;
   const bool vec = conv_vector_ok(W, dtype, {u, state, dout, du, dstate}) && (du_stride * (dtype == RGLRU_BF16 ? 2 : 4)) % 16 == 0;
   a.nvec = (int)(vec ? W / (dtype == RGLRU_BF16 ? 8 : 4) : W);
@@ -1284,7 +1287,7 @@ int rglru_hip_conv_rows_bwd(const void* u, const void* state, const void* taps, 
                             int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, int grad_dtype,
                             void* stream) {
   if (grad_dtype != RGLRU_F32 && grad_dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "conv_bwd: unknown gradient dtype %d", grad_dtype);
-  const int rc = conv_bwd_partials(u, state, taps, segment_pos, rows, dout, scratch, du, du_stride, dstate, B, T, W, K, dtype, vec_dtype, stream);
+  const int rc = conv_bwd_partials(u, state, taps, segment_pos, rows, dout, scratch, du, du_stride, dstate, B, T, W, K, dtype, vec_dtype, false, stream);
   if (rc || (!dtaps && !dbias)) return rc;
   return launch_sum_job("conv_bwd finish", conv_sum_job((const float*)scratch, dtaps, dbias, W, K, conv_partial_sets(B, T), grad_dtype), stream);
 }

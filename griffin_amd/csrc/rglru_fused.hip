@@ -811,6 +811,7 @@ static int build_prep_args(const void* w_a, const void* b_a, const void* w_x, co
   a.w2t = pb + pl.w2t;
   a.W = (int)W; a.nb = (int)nb; a.bw = (int)g.bw; a.bwp = (int)g.bwp; a.Wp = (int)g.Wp; a.c = c;
   a.clear = (uint4*)clear; a.clear_n = (long long)(clear_bytes / 16);
+  a.stack_from[0] = a.stack_from[1] = nullptr; a.stack_to = nullptr; a.stack_n = 0;
   a.vec_ok = dtype == RGLRU_BF16 && g.bw == g.bwp && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0 &&
              (uintptr_t)a.wg % 16 == 0 && (uintptr_t)a.w2t % 16 == 0;
   a.rows_ok = dtype == RGLRU_BF16 && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0;
@@ -821,6 +822,7 @@ static int launch_prepare(const PrepArgs& a, int dtype, void* stream) {
   const long long cells = (long long)a.nb * a.bwp * a.bwp;
   long long total = a.vec_ok ? 4 * cells / 8 + a.Wp : 4 * cells + a.Wp;
   if (a.clear_n > total) total = a.clear_n;
+  if (2 * a.stack_n > total) total = 2 * a.stack_n;
   int blocks = (int)((total + 255) / 256); if (blocks > 2048) blocks = 2048;
   hipStream_t s = (hipStream_t)stream;
   if (dtype == RGLRU_BF16) hipLaunchKernelGGL(prepare_kernel<__bf16>, dim3(blocks), dim3(256), 0, s, a);
@@ -1119,13 +1121,20 @@ int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_
                                 const void* conv_state, const void* taps, const void* conv_bias, int64_t K,
                                 const float* h0, const uint8_t* flags,
                                 void* x_conv, void* y, void* gated, void* new_conv_state, float* h_last, void* ws,
+                                const void* stack0, const void* stack1, void* stacked, int64_t stack_bytes,
                                 int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream) {
   int rc = check_geometry("prepare_block_fwd", W, nb, dtype);
   if (rc) return rc;
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "prepare_block_fwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
   if (!ws) return fail(RGLRU_E_ARG, "prepare_block_fwd: null pointer");
   const WorkLayout L = make_work_layout(B, T, make_geometry(W, nb));
-  rc = prepare_impl(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, L.f_end - L.f_begin, stream);
+  if (stack_bytes < 0 || stack_bytes % 16 || (stack_bytes && (!stack0 || !stack1 || !stacked || (uintptr_t)stack0 % 16 || (uintptr_t)stack1 % 16 || (uintptr_t)stacked % 16)))
+    return fail(RGLRU_E_ARG, "prepare_block_fwd: the arrays to stack must be whole 16-byte vectors on 16-byte boundaries");
+  PrepArgs pa;
+  rc = build_prep_args(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, L.f_end - L.f_begin, pa);
+  if (rc) return rc;
+  pa.stack_from[0] = (const uint4*)stack0; pa.stack_from[1] = (const uint4*)stack1; pa.stack_to = (uint4*)stacked; pa.stack_n = stack_bytes / 16;
+  rc = launch_prepare(pa, dtype, stream);
   if (rc) return rc;
   const BlockFwd blk = {v, u_stride, v_stride, conv_state, taps, conv_bias, K, vec_dtype, x_conv, gated, new_conv_state};
   return fwd_impl(u, prep, h0, flags, y, h_last, ws, B, T, W, nb, dtype, true, stream, nullptr, &blk);

@@ -519,8 +519,27 @@ constexpr int kDeltaDepth = RGLRU_DELTA_DEPTH;         // records a walk of the 
 #ifndef RGLRU_DELTA_OCC
 #define RGLRU_DELTA_OCC 2
 #endif
+// Reverse mode of the output gate out = h gelu_tanh(v) on eight values (griffin/griffin.py:464, :520): d at out becomes the gradient
+// at h, the gradient at v is returned; `sums` adds that up.
+RGLRU_DEVICE bf16x8 gate_backward(bf16x8& d, const bf16x8& h, const bf16x8& v, float (&sums)[8]) {
+  bf16x8 dv;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const GeluParts g = gelu_tanh_parts((float)v[e]);
+    const float de = (float)d[e];
+    d[e] = (__bf16)(de * g.gelu);
+    const float dve = (de * (float)h[e]) * g.dgelu;
+    sums[e] += dve;
+    dv[e] = (__bf16)dve;
+    if (e & 1) __builtin_amdgcn_sched_barrier(0);            // two elements at a time: the registers are needed for the tile
+  }
+  return dv;
+}
+
+// GATED, in the two scan kernels: the output gate's reverse mode on the way in.  As a kernel of its own it read y, v and the
+// gradient and wrote two gradients, one of which the scan read back: 31 us next to the scan's 31 us at B8 T2048 W1024.
 // PAD, in this kernel and the two behind it: blocks that do not fill their slabs (see narrow_groups), masked variant only.
-template <typename IO, int NKG, bool MASKED, int MT, bool PAD = false>
+template <typename IO, int NKG, bool MASKED, int MT, bool PAD = false, bool GATED = false>
 __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd_delta_kernel(FusedArgs p) {
   constexpr int TR = 32 * MT, EL = 16 * MT;
   typedef Io<IO> Tr;
@@ -553,15 +572,20 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
 
   constexpr int VPR = TW / Tr::HW;
   constexpr int NV = (TR * VPR + kThreads - 1) / kThreads;
-  Frag pre_x[NV], pre_dy[NV];
+  Frag pre_x[NV], pre_dy[NV], pre_h[GATED ? NV : 1], pre_v[GATED ? NV : 1];
   unsigned pre_off[NV];
+  const int my_col = tile_channel<PAD>(p, w.unit, w.tile_col, (tid % VPR) * Tr::HW);    // the same for all vectors of a thread
+  static_assert(kThreads % VPR == 0, "a thread's vectors lie below each other");
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int idx = tid + i * kThreads;
-    const int row = idx / VPR, cv = idx - row * VPR;
-    const int col = tile_channel<PAD>(p, w.unit, w.tile_col, cv * Tr::HW);
-    pre_off[i] = (idx < TR * VPR && col >= 0) ? (unsigned)row * row_bytes + (unsigned)col * 2u : kOutOfRange;
+    const int idx = tid + i * kThreads, row = idx / VPR;
+    pre_off[i] = (idx < TR * VPR && my_col >= 0) ? (unsigned)row * row_bytes + (unsigned)my_col * 2u : kOutOfRange;
   }
+  const unsigned v_row_bytes = (unsigned)p.ld_gate * 2u, dv_row_bytes = (unsigned)p.ld_dv * 2u;
+  const bool my_col_ok = my_col >= 0 && my_col < p.W;      // the last unit of a block count that does not fill it
+  float dv_sum[GATED ? 8 : 1];
+#pragma unroll
+  for (int e = 0; e < (GATED ? 8 : 1); ++e) dv_sum[e] = 0.f;
   const bool ch_ok = !PAD || w.ch_ok;
   auto decode = [&](unsigned tk, int& c, int& b) {
     const unsigned cr = tk / (unsigned)q.n_b;
@@ -579,6 +603,16 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     const rsrc_t rdy = make_rsrc(dy + first, (unsigned)rows * row_bytes);
 #pragma unroll
     for (int i = 0; i < NV; ++i) { pre_x[i] = buf_load_frag<Frag>(rx, pre_off[i]); pre_dy[i] = buf_load_frag<Frag>(rdy, pre_off[i]); }
+    if constexpr (GATED) {
+      const rsrc_t rh = make_rsrc((const IO*)p.y + first, (unsigned)rows * row_bytes);
+      const rsrc_t rv = make_rsrc((const IO*)p.gate_v + ((long long)b * p.T + (long long)c * TR) * p.ld_gate, (unsigned)rows * v_row_bytes);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const unsigned off_v = (unsigned)((tid + i * kThreads) / VPR) * v_row_bytes + (unsigned)my_col * 2u;
+        pre_h[i] = buf_load_frag<Frag>(rh, pre_off[i]);
+        pre_v[i] = buf_load_frag<Frag>(rv, my_col_ok ? off_v : kOutOfRange);
+      }
+    }
   };
 
   if (tid == 0) s_ticket[0] = atomicAdd(q.counter, 1u);
@@ -600,6 +634,14 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     for (int i = 0; i < NV; ++i) {
       const int idx = tid + i * kThreads;
       const int row = idx / VPR, cv = idx - row * VPR;
+      if constexpr (GATED) {
+        // rows past the sequence's end: the gradient reads as zero there, and the store is dropped
+        const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+        const rsrc_t rdv = make_rsrc((const IO*)p.dv + ((long long)b * p.T + t0) * p.ld_dv, (unsigned)(rows - 1) * dv_row_bytes + row_bytes);
+        const Frag dv = gate_backward(pre_dy[i], pre_h[i], pre_v[i], dv_sum);
+        buf_store_b128(__builtin_bit_cast(i32x4, dv), rdv, my_col_ok && idx < TR * VPR && row < rows ? (unsigned)row * dv_row_bytes + (unsigned)my_col * 2u : kOutOfRange);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       if (idx < TR * VPR) {
         *reinterpret_cast<Frag*>(lds_x + row * LDSROW + cv * Tr::HW) = pre_x[i];
         *reinterpret_cast<Frag*>(lds_dy + row * LDSROW + cv * Tr::HW) = pre_dy[i];
@@ -673,18 +715,38 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     wave_lds_fence();
     tk = tk_next;
   }
+  if constexpr (GATED) {
+    // column sums of dv over the workgroup's tiles: the threads of a column vector meet in LDS
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(lds_x);
+    static_assert(sizeof(lds_x) >= kThreads * 9 * sizeof(float), "nine words a thread: no bank conflicts");
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[tid * 9 + e] = dv_sum[e];
+    __syncthreads();
+    if (tid < VPR && my_col_ok) {
+      float* part = p.dv_partial + (long long)w.wg_in_unit * p.W + my_col;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float sum = 0.f;
+        for (int q = tid; q < kThreads; q += VPR) sum += red[q * 9 + e];
+        part[e] = sum;
+      }
+    }
+  }
 }
 
 // The reverse scan with one workgroup per chain, the counterpart of fwd_chain_kernel: sixteen waves take the
 // chain's 32-token tiles round robin from the last tile to the first, the recurrence gate's rows of the slab
 // sit in LDS, and the carry goes from tile c + 1 to tile c through LDS.  A wave stages its own x tile (the
 // block's K range) and its own 32 channels of dy; delta leaves through the x tile's area.
-template <typename IO, int NKG, bool MASKED, bool PAD = false>
-__global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(FusedArgs p) {
+// Waves of its workgroup: sixteen leave 128 registers each; with the output gate's operands in flight too that is not enough.
+constexpr int delta_chain_waves(bool gated) { return gated ? 12 : kChainWaves; }
+template <typename IO, int NKG, bool MASKED, bool PAD = false, bool GATED = false>
+__global__ __launch_bounds__(delta_chain_waves(GATED) * 64, 1) void bwd_delta_chain_kernel(FusedArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
   static_assert(sizeof(IO) == 2 && (NKG == 8 || NKG == 6 || NKG == 4 || NKG == 2), "16-bit storage, gate blocks of one to four slabs");
-  constexpr int TR = 32;
+  constexpr int TR = 32, WAVES = delta_chain_waves(GATED);
   constexpr int KC = NKG * Tr::KG;
   const int bw = PAD ? p.bw : KC;                          // channels of the block that exist
   constexpr int S = KC / 32;
@@ -693,9 +755,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
   constexpr int NV = TR * VPR / 64;
   constexpr int DYROW = 32 + Tr::HW;                       // the wave's 32 channels of dy, padded
   static_assert(TR * LDSROW * (int)sizeof(IO) >= WaveStage<TR>::kBytes, "the staging area lies over the x tile");
-  __shared__ __attribute__((aligned(16))) IO lds_all[kChainWaves][TR * LDSROW];
+  __shared__ __attribute__((aligned(16))) IO lds_all[WAVES][TR * LDSROW];
   __shared__ __attribute__((aligned(16))) IO lds_w[32 * LDSROW];                    // [output channel][K], recurrence gate
-  __shared__ __attribute__((aligned(8))) unsigned long long carry[kChainWaves][32];
+  __shared__ __attribute__((aligned(8))) unsigned long long carry[WAVES][32];
 
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -703,10 +765,10 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
   const int sl = slot % S, u = (slot / S) * 8 + xcd;
   const bool chain_ok = u < p.B * p.nb;
   const int b = chain_ok ? u / p.nb : 0, k = chain_ok ? u - b * p.nb : 0;
-  for (int i = tid; i < kChainWaves * 32; i += kChainWaves * 64) (&carry[0][0])[i] = 0ull;
+  for (int i = tid; i < WAVES * 32; i += WAVES * 64) (&carry[0][0])[i] = 0ull;
   {
     const IO* wg = (const IO*)p.wg;
-    for (int i = tid; i < 32 * VPR; i += kChainWaves * 64) {
+    for (int i = tid; i < 32 * VPR; i += WAVES * 64) {
       const int o = i / VPR, cv = i % VPR;
       *reinterpret_cast<Frag*>(lds_w + o * LDSROW + cv * Tr::HW) =
           *reinterpret_cast<const Frag*>(wg + ((long long)(0 * p.nb + k) * p.bwp + sl * 32 + o) * p.bwp + cv * Tr::HW);
@@ -728,7 +790,12 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
   const unsigned row_bytes = (unsigned)p.W * 2u;
   const long long limit = p.limit < 0 ? -p.limit : p.limit;
 
-  Frag pre[NV], pre_dy[2];
+  Frag pre[NV], pre_dy[2], pre_h[GATED ? 2 : 1], pre_v[GATED ? 2 : 1];
+  float dv_sum[GATED ? 8 : 1];
+#pragma unroll
+  for (int e = 0; e < (GATED ? 8 : 1); ++e) dv_sum[e] = 0.f;
+  const unsigned v_row_bytes = (unsigned)p.ld_gate * 2u, dv_row_bytes = (unsigned)p.ld_dv * 2u;
+  const unsigned gate_col = (unsigned)(col0 + sl * 32 + (lane & 3) * Tr::HW) * 2u;
   unsigned pre_off[NV], dy_off[2];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -752,12 +819,26 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
 #pragma unroll
     for (int i = 0; i < 2; ++i) pre_dy[i] = buf_load_frag<Frag>(rdy, dy_off[i]);
   };
+  auto issue_gate = [&](int c) {                           // the output gate's operands of a tile, likewise
+    if constexpr (GATED) {
+      const int rows = c < 0 ? 0 : ((p.T - c * TR) < TR ? (p.T - c * TR) : TR);
+      const long long row0 = (long long)b * p.T + (c < 0 ? 0 : c) * TR;
+      const rsrc_t rh = make_rsrc((const IO*)p.y + row0 * W, (unsigned)rows * row_bytes);
+      const rsrc_t rv = make_rsrc((const IO*)p.gate_v + row0 * p.ld_gate, (unsigned)rows * v_row_bytes);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        pre_h[i] = buf_load_frag<Frag>(rh, dy_off[i]);
+        pre_v[i] = buf_load_frag<Frag>(rv, seg_ok ? (unsigned)((lane + 64 * i) >> 2) * v_row_bytes + gate_col : kOutOfRange);
+      }
+    }
+  };
   const rsrc_t rh0 = make_rsrc(p.dh0, p.dh0 ? (unsigned)p.B * (unsigned)W * 4u : 0u);
-  const int next_wave = (wave + kChainWaves - 1) % kChainWaves;    // the wave of tile c + 1
+  const int next_wave = (wave + WAVES - 1) % WAVES;    // the wave of tile c + 1
   bool gave_up = false;
   // carry into the chain's last tile (used by its wave only): no memory operation inside the loop is conditional
   const float d_first = p.dh_last && ch_ok ? p.dh_last[(long long)b * W + ch] : 0.f;
   issue(nC - 1 - wave);
+  issue_gate(nC - 1 - wave);
   {
     // the stores the loop's back edge has in flight behind the prefetched tiles (dh0, two delta segments),
     // dropped through their offsets, in front of its entry (see fwd_chain_kernel)
@@ -766,10 +847,22 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
     buf_store_b128(nothing, rh0, kOutOfRange);
     buf_store_b128(nothing, rh0, kOutOfRange + 16u);
   }
-  for (int c = nC - 1 - wave; c >= 0; c -= kChainWaves) {
+  for (int c = nC - 1 - wave; c >= 0; c -= WAVES) {
     const int t0 = c * TR;
     unsigned flbits = 0u;
     if constexpr (MASKED) flbits = flag_run(p, (long long)b * p.T + t0 + hf * 16, t0 + hf * 16);
+    if constexpr (GATED) {
+      // first of all, one fragment after the other: what it needs in registers is free again for the rest of the tile
+      const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;    // past them the gradient reads as zero and the store is dropped
+      const rsrc_t rdv = make_rsrc((const IO*)p.dv + ((long long)b * p.T + t0) * p.ld_dv, (unsigned)(rows - 1) * dv_row_bytes + row_bytes);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int row = (lane + 64 * i) >> 2;
+        const Frag dv = gate_backward(pre_dy[i], pre_h[i], pre_v[i], dv_sum);
+        buf_store_b128(__builtin_bit_cast(i32x4, dv), rdv, seg_ok && row < rows ? (unsigned)row * dv_row_bytes + gate_col : kOutOfRange);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = lane + 64 * i, row = idx / VPR, cv = idx - row * VPR;
@@ -795,7 +888,8 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
       for (int kg = 0; kg < NKG; ++kg) Tr::mma(ua, xa[kg], *reinterpret_cast<const Frag*>(wrow + kg * Tr::KG));
     }
     wave_lds_fence();
-    issue(c - kChainWaves);
+    issue(c - WAVES);
+    issue_gate(c - WAVES);
     float a[16], gy[16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
@@ -853,6 +947,26 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void bwd_delta_chain_kernel(Fu
     wave_lds_fence();
   }
   if (gave_up && lane == 0) atomicOr(p.fail, 1u);
+  if constexpr (GATED) {
+    // column sums of dv over the sequence: rows of a wave by shuffles, the waves through LDS (the weights are not needed any more)
+    float* red = reinterpret_cast<float*>(lds_w);
+    static_assert(sizeof(lds_w) >= WAVES * 32 * sizeof(float), "one word per wave and channel");
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float sum = dv_sum[e];
+#pragma unroll
+      for (int m = 4; m < 64; m <<= 1) sum += __shfl_xor(sum, m);
+      if (lane < 4) red[wave * 32 + lane * 8 + e] = sum;
+    }
+    __syncthreads();
+    if (tid < 32 && (!PAD || sl * 32 + tid < bw)) {
+      float sum = 0.f;
+#pragma unroll
+      for (int q = 0; q < WAVES; ++q) sum += red[q * 32 + tid];
+      p.dv_partial[(long long)b * W + col0 + sl * 32 + tid] = sum;
+    }
+  }
 }
 
 constexpr int kGradWaves = 8;                            // waves per workgroup of the gradient kernel
@@ -1603,9 +1717,9 @@ __global__ __launch_bounds__(256) void finish_kernel(FinishArgs p) {
   gate_finish(p, (int)blockIdx.x, part_sum);
 }
 
-// All last sums of a block's backward pass in one launch: the gates' (the first gate_blocks workgroups), then up to five jobs.
+// All last sums of a block's backward pass in one launch: the gates' (the first gate_blocks workgroups), then up to six jobs.
 // Six launches of 4 to 6 us each took as long as they have steps (B8 T2048 W1024: 41 us together).
-constexpr int kBlockJobs = 5;
+constexpr int kBlockJobs = 6;
 struct BlockFinishArgs { FinishArgs gates; SumJob job[kBlockJobs]; int gate_blocks, jobs; };
 __global__ __launch_bounds__(256) void block_finish_kernel(BlockFinishArgs p) {
   __shared__ union { float gates[3][16][16]; float sums[8][32]; } lds;
@@ -1794,10 +1908,11 @@ static int fast_finish_args(const Geometry& g, const void* prep, const char* scr
 }
 
 // The two kernels of the fast backward; their partial sums stay in `scratch`.
+struct GateBwd { const void* v; void* dv; int64_t d_stride; float* dv_partial; };
 static int bwd_full_kernels(const void* x, const void* y, const void* prep, const float* h0,
                             const uint8_t* flags, const void* dy, const float* dh_last, void* ws, void* scratch,
                             void* dx, float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
-                            void* stream) {
+                            void* stream, const GateBwd* gate = nullptr) {
   int rc = check_geometry("bwd_full", W, nb, dtype);
   if (rc) return rc;
   rc = check_grad_dtype("bwd_full", grad_dtype);
@@ -1829,6 +1944,7 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
   a.partial = (float*)(sb + SL.partial); a.dw_partial = (float*)(sb + SL.dw_partial);
   a.B = (int)B; a.T = (int)T; a.nC = (int)((T + kChunk - 1) / kChunk); a.ckpt_nC = 2 * (int)L.nC;
   a.aligned = 1;
+  if (gate) { a.gate_v = gate->v; a.ld_gate = W; a.dv = gate->dv; a.ld_dv = gate->d_stride; a.dv_partial = gate->dv_partial; }
   const int nkg = narrow_groups(g, dtype, 1);
   const bool pad = narrow_padded(g);
   pack_units(a, g, nkg);
@@ -1847,26 +1963,28 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
     const dim3 cgrid((unsigned)(8 * ((B * nb + 7) / 8) * g.S));
     const bool cmasked = (flags != nullptr) || (T % 32 != 0);
     KernelTimer timer(1, s);
-#define RGLRU_LAUNCH_DELTA_CHAIN(N)                                                                                  \
-    if (cmasked) hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, true>), cgrid, dim3(kChainWaves * 64), 0, s, a); \
-    else hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, false>), cgrid, dim3(kChainWaves * 64), 0, s, a)
-#define RGLRU_LAUNCH_DELTA_CHAIN_PAD(N) hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, true, true>), cgrid, dim3(kChainWaves * 64), 0, s, a)
-    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA_CHAIN_PAD(8); break; case 6: RGLRU_LAUNCH_DELTA_CHAIN_PAD(6); break; case 4: RGLRU_LAUNCH_DELTA_CHAIN_PAD(4); break; default: RGLRU_LAUNCH_DELTA_CHAIN_PAD(2); } }
-    else if (nkg == 8) { RGLRU_LAUNCH_DELTA_CHAIN(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA_CHAIN(4); } else { RGLRU_LAUNCH_DELTA_CHAIN(2); }
+#define RGLRU_LAUNCH_DELTA_CHAIN(N, M, P)                                                                            \
+    do {                                                                                                             \
+      if (gate) hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, M, P, true>), cgrid, dim3(delta_chain_waves(true) * 64), 0, s, a); \
+      else hipLaunchKernelGGL((bwd_delta_chain_kernel<__bf16, N, M, P, false>), cgrid, dim3(kChainWaves * 64), 0, s, a);     \
+    } while (0)
+    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA_CHAIN(8, true, true); break; case 6: RGLRU_LAUNCH_DELTA_CHAIN(6, true, true); break; case 4: RGLRU_LAUNCH_DELTA_CHAIN(4, true, true); break; default: RGLRU_LAUNCH_DELTA_CHAIN(2, true, true); } }
+    else if (cmasked) { if (nkg == 8) RGLRU_LAUNCH_DELTA_CHAIN(8, true, false); else if (nkg == 4) RGLRU_LAUNCH_DELTA_CHAIN(4, true, false); else RGLRU_LAUNCH_DELTA_CHAIN(2, true, false); }
+    else { if (nkg == 8) RGLRU_LAUNCH_DELTA_CHAIN(8, false, false); else if (nkg == 4) RGLRU_LAUNCH_DELTA_CHAIN(4, false, false); else RGLRU_LAUNCH_DELTA_CHAIN(2, false, false); }
 #undef RGLRU_LAUNCH_DELTA_CHAIN
-#undef RGLRU_LAUNCH_DELTA_CHAIN_PAD
   } else {
     rc = launch_clear(wb, L.b_begin, L.b_end, s);        // records and tickets of this pass
     if (rc) return rc;
     KernelTimer timer(1, s);
-#define RGLRU_LAUNCH_DELTA(N)                                                                                        \
-    if (masked) hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, true, kDeltaMT>), grid, dim3(kThreads), 0, s, a);      \
-    else hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, false, kDeltaMT>), grid, dim3(kThreads), 0, s, a)
-#define RGLRU_LAUNCH_DELTA_PAD(N) hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, true, kDeltaMT, true>), grid, dim3(kThreads), 0, s, a)
-    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA_PAD(8); break; case 6: RGLRU_LAUNCH_DELTA_PAD(6); break; case 4: RGLRU_LAUNCH_DELTA_PAD(4); break; default: RGLRU_LAUNCH_DELTA_PAD(2); } }
-    else if (nkg == 8) { RGLRU_LAUNCH_DELTA(8); } else if (nkg == 4) { RGLRU_LAUNCH_DELTA(4); } else { RGLRU_LAUNCH_DELTA(2); }
+#define RGLRU_LAUNCH_DELTA(N, M, P)                                                                                  \
+    do {                                                                                                             \
+      if (gate) hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, M, kDeltaMT, P, true>), grid, dim3(kThreads), 0, s, a); \
+      else hipLaunchKernelGGL((bwd_delta_kernel<__bf16, N, M, kDeltaMT, P, false>), grid, dim3(kThreads), 0, s, a);     \
+    } while (0)
+    if (pad) { switch (nkg) { case 8: RGLRU_LAUNCH_DELTA(8, true, true); break; case 6: RGLRU_LAUNCH_DELTA(6, true, true); break; case 4: RGLRU_LAUNCH_DELTA(4, true, true); break; default: RGLRU_LAUNCH_DELTA(2, true, true); } }
+    else if (masked) { if (nkg == 8) RGLRU_LAUNCH_DELTA(8, true, false); else if (nkg == 4) RGLRU_LAUNCH_DELTA(4, true, false); else RGLRU_LAUNCH_DELTA(2, true, false); }
+    else { if (nkg == 8) RGLRU_LAUNCH_DELTA(8, false, false); else if (nkg == 4) RGLRU_LAUNCH_DELTA(4, false, false); else RGLRU_LAUNCH_DELTA(2, false, false); }
 #undef RGLRU_LAUNCH_DELTA
-#undef RGLRU_LAUNCH_DELTA_PAD
   }
   rc = check_launch("bwd_full scan");
   if (rc) return rc;
@@ -1905,19 +2023,36 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   return check_launch("bwd_full finish");
 }
 
+// Partial rows in which the gated reverse scan leaves the column sums of dv (see bwd_full_kernels).
+static int64_t gate_sum_sets(int64_t B, int64_t T, const Geometry& g) {
+  if (fwd_chain_pays(B, T, g.Wp)) return B;
+  FusedArgs a;
+  memset(&a, 0, sizeof(a));
+  a.units = (int)g.units;
+  pack_units(a, g, narrow_groups(g, RGLRU_BF16, 1));
+  return pick_wg_per_unit(a.units, B * ((T + 32 * kDeltaMT - 1) / (32 * kDeltaMT)), kDeltaMT == 1 ? 4 : RGLRU_DELTA_OCC, make_work_layout(B, T, g).max_wg);
+}
+
+size_t rglru_hip_block_sums_bytes(int64_t B, int64_t T, int64_t W, int64_t nb) {
+  if (B <= 0 || T <= 0 || W <= 0 || nb <= 0 || W % nb) return 0;
+  return (size_t)(gate_sum_sets(B, T, make_geometry(W, nb)) * W * 4);
+}
+
 int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
                         const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
-                        void* gate_scratch, void* conv_scratch, void* du, void* dv, int64_t d_stride,
+                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride,
                         int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream) {
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "block_bwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
-  // the gradient at y takes the place of the one at y * gelu(v), the one at the convolution's output the place of that
-  int rc = rglru_hip_gelu_gate_bwd(dgated, y, v, dgated, dv, B * T * W, W, d_stride, RGLRU_BF16, stream);
-  if (rc) return rc;
-  rc = bwd_full_kernels(x_conv, y, prep, nullptr, flags, dgated, nullptr, ws, gate_scratch, dgated, nullptr, B, T, W, nb, RGLRU_BF16,
-                        RGLRU_BF16, stream);
+  if (!dgated || !v || !dv || !sums_scratch) return fail(RGLRU_E_ARG, "block_bwd: null pointer");
+  if ((uintptr_t)v % 16 || (uintptr_t)dv % 16 || (d_stride * 2) % 16 || d_stride < W || d_stride >= (1 << 22))
+    return fail(RGLRU_E_UNSUPPORTED, "block_bwd: v and dv must be rows of whole 16-byte vectors");
+  // the gradient at the convolution's output takes the place of the one at y * gelu(v)
+  const GateBwd gate = {v, dv, d_stride, (float*)sums_scratch};
+  const int rc = bwd_full_kernels(x_conv, y, prep, nullptr, flags, dgated, nullptr, ws, gate_scratch, dgated, nullptr, B, T, W, nb, RGLRU_BF16,
+                                  RGLRU_BF16, stream, &gate);
   if (rc) return rc;
   return conv_bwd_partials(u, nullptr, taps, positions, rows, dgated, conv_scratch, du, d_stride, nullptr, B, T, W, K, RGLRU_BF16,
-                           RGLRU_BF16, stream);
+                           RGLRU_BF16, true, stream);
 }
 
 // The caller's sums as jobs behind those already there.
@@ -1948,25 +2083,28 @@ int rglru_hip_sums(const rglru_sum* sums, int n_sums, int dst_dtype, void* strea
   return check_launch("sums");
 }
 
-int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, void* dw_a, void* dw_x,
-                           void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, const rglru_sum* sums, int n_sums,
+int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, const void* sums_scratch, void* dw_a,
+                           void* dw_x, void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, void* du_sums, void* dv_sums,
+                           const rglru_sum* sums, int n_sums,
                            int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream) {
   int rc = check_geometry("block_finish", W, nb, RGLRU_BF16);
   if (rc) return rc;
-  if (!prep || !gate_scratch || !conv_scratch || !dw_a || !dw_x || !db_a || !db_x || !dlambda) return fail(RGLRU_E_ARG, "block_finish: null pointer");
+  if (!prep || !gate_scratch || !conv_scratch || !sums_scratch || !dw_a || !dw_x || !db_a || !db_x || !dlambda || !du_sums || !dv_sums)
+    return fail(RGLRU_E_ARG, "block_finish: null pointer");
   if ((uintptr_t)dw_a % 16 || (uintptr_t)dw_x % 16) return fail(RGLRU_E_UNSUPPORTED, "block_finish: dw_a and dw_x must be 16-byte aligned");
-  if (n_sums < 0 || n_sums >= kBlockJobs) return fail(RGLRU_E_ARG, "block_finish: up to %d sums, got %d", kBlockJobs - 1, n_sums);
+  if (n_sums < 0 || n_sums > kBlockJobs - 2) return fail(RGLRU_E_ARG, "block_finish: up to %d sums, got %d", kBlockJobs - 2, n_sums);
   BlockFinishArgs p;
   memset(&p, 0, sizeof(p));
   p.gate_blocks = fast_finish_args(make_geometry(W, nb), prep, (const char*)gate_scratch, B, T, RGLRU_BF16, RGLRU_BF16, dw_a, dw_x, db_a,
                                    db_x, dlambda, p.gates);
   long long blocks = p.gate_blocks;
-  if (dtaps || dbias) {
-    SumJob j = conv_sum_job((const float*)conv_scratch, dtaps, dbias, W, K, conv_partial_sets(B, T), RGLRU_BF16);
-    plan_sum_job(j);
-    blocks += j.blocks;
-    p.job[p.jobs++] = j;
-  }
+  SumJob conv = conv_sum_job((const float*)conv_scratch, dtaps, dbias, W, K, conv_partial_sets(B, T), RGLRU_BF16, du_sums);
+  plan_sum_job(conv);
+  p.job[p.jobs++] = conv;
+  blocks += conv.blocks;
+  const rglru_sum gate = {sums_scratch, dv_sums, gate_sum_sets(B, T, make_geometry(W, nb)), W, RGLRU_F32};
+  rc = add_sums(p, &gate, 1, RGLRU_BF16, blocks);
+  if (rc) return rc;
   rc = add_sums(p, sums, n_sums, RGLRU_BF16, blocks);
   if (rc) return rc;
   hipLaunchKernelGGL(block_finish_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, p);

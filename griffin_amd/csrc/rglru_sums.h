@@ -16,8 +16,8 @@ struct SumJob {
   const void* src; void* dst;
   long long n;                       // elements of a set; set s starts at src + s * n
   int sets, src_bf16, dst_bf16;
-  int taps, width;                   // convolution: n = (taps + 1) * width, element j * width + c goes to dst[c * taps + j] ...
-  void* dst_bias;                    // ... and the last `width` ones to dst_bias[c]; either may be null
+  int taps, width;                   // convolution: n = (taps + 1 or 2) * width, element j * width + c goes to dst[c * taps + j], ...
+  void* dst_bias; void* dst_du;      // ... those of j = taps to dst_bias[c] and of j = taps + 1 to dst_du[c]; any may be null
   int vec;                           // elements per thread of the streaming form (8 or 1), 0: the column form
   int blocks;                        // workgroups of 256 threads
 };
@@ -120,14 +120,16 @@ RGLRU_DEVICE void run_sum_job(const SumJob& j, int block, float (&red)[8][32]) {
   if (!j.taps) { sum_job_store(j, j.dst, c, s); return; }
   const int t = (int)(c / j.width), ch = (int)(c - (long long)t * j.width);
   if (t < j.taps) { if (j.dst) sum_job_store(j, j.dst, (long long)ch * j.taps + t, s); }
-  else if (j.dst_bias) sum_job_store(j, j.dst_bias, ch, s);
+  else if (void* dst = t == j.taps ? j.dst_bias : j.dst_du) sum_job_store(j, dst, ch, s);
 }
 
-// A convolution's tap and bias gradients from the per-run partials [slots][K + 1][W].
-inline SumJob conv_sum_job(const float* partial, void* dtaps, void* dbias, int64_t W, int64_t K, int64_t slots, int grad_dtype) {
+// A convolution's tap and bias gradients from the per-run partials [slots][K + 1][W] (K + 2 rows with the column
+// sums of du).
+inline SumJob conv_sum_job(const float* partial, void* dtaps, void* dbias, int64_t W, int64_t K, int64_t slots, int grad_dtype,
+                           void* du_sums = nullptr) {
   SumJob j;
   memset(&j, 0, sizeof(j));
-  j.src = partial; j.dst = dtaps; j.dst_bias = dbias; j.n = (K + 1) * W; j.sets = (int)slots; j.dst_bf16 = grad_dtype == RGLRU_BF16;
+  j.src = partial; j.dst = dtaps; j.dst_bias = dbias; j.dst_du = du_sums; j.n = (K + (du_sums ? 2 : 1)) * W; j.sets = (int)slots; j.dst_bf16 = grad_dtype == RGLRU_BF16;
   j.taps = (int)K; j.width = (int)W;
   return j;
 }
@@ -136,6 +138,6 @@ inline SumJob conv_sum_job(const float* partial, void* dtaps, void* dbias, int64
 int64_t conv_partial_sets(int64_t B, int64_t T);
 int conv_bwd_partials(const void* u, const void* state, const void* taps, const int64_t* segment_pos, const int32_t* rows,
                       const void* dout, void* scratch, void* du, int64_t du_stride, void* dstate,
-                      int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, void* stream);
+                      int64_t B, int64_t T, int64_t W, int64_t K, int dtype, int vec_dtype, bool sum_du, void* stream);
 
 }  // namespace rglru

@@ -845,7 +845,7 @@ BlockResult block_forward_pass(const Tensor& u, const Tensor& v, const Tensor& c
     check(rglru_hip_prepare_block_fwd(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), p.vec,
                                       kept.image, ptr(r.u), r.u.stride(1), ptr(r.v), r.v.stride(1), ptr(r.state), ptr(r.taps),
                                       ptr(b), K, fptr(r.h0), fl, ptr(r.x_conv), ptr(r.y), ptr(r.gated), new_conv,
-                                      fptr(r.h_last), kept.ws, B, T, W, nb, code, stream), "rglru_hip_prepare_block_fwd");
+                                      fptr(r.h_last), kept.ws, nullptr, nullptr, nullptr, 0, B, T, W, nb, code, stream), "rglru_hip_prepare_block_fwd");
   } else {
     Tensor ws = bytes(rglru_hip_workspace_bytes(B, T, W, nb), u);
     check(rglru_hip_block_fwd(ptr(r.u), r.u.stride(1), ptr(r.v), r.v.stride(1), ptr(r.state), ptr(r.taps), ptr(b), K,
@@ -1500,11 +1500,13 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     const size_t image_bytes = round_up(prep_bytes(W, nb, RGLRU_BF16));
     const size_t tensor_bytes = round_up(M * W * 2);
     const int own = u.defined() ? 3 : 5;
-    Tensor buffer = bytes(own * tensor_bytes + image_bytes + rglru_hip_workspace_bytes(B, T, W, nb), x);
+    const size_t ws_bytes = round_up(rglru_hip_workspace_bytes(B, T, W, nb));
+    const bool stack = !own_linear(x, wx, bx);               // the weights stacked for the backward's GEMM of the BLAS library
+    Tensor buffer = bytes(own * tensor_bytes + image_bytes + ws_bytes + (stack ? 2 * W * D * 2 : 0), x);
     Saved s(buffer, M, W);
     if (!first_reset && !flags.defined()) flags = block_flags(pos);
     if (!u.defined()) {
-      if (own_linear(x, wx, bx)) {
+      if (!stack) {
         linear_forward(x, wx, bx, wy, by, Tensor(), s[3], s[4]);
       } else {
         Tensor x2 = x.view({M, D});
@@ -1517,9 +1519,10 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     char *image = s[own], *ws = image + image_bytes;
     check(rglru_hip_prepare_block_fwd(ptr(wa), ptr(ba), ptr(wi), ptr(bi), ptr(lam), static_cast<float>(c), RGLRU_BF16, image, up, W, vp, W,
                                       nullptr, ptr(cw), ptr(cb), K, nullptr, flags_ptr(flags, first_reset), s[0], s[1], s[2], nullptr,
-                                      nullptr, ws, B, T, W, nb, RGLRU_BF16, stream), "rglru_hip_prepare_block_fwd");
+                                      nullptr, ws, ptr(wx), ptr(wy), ws + ws_bytes, stack ? W * D * 2 : 0, B, T, W, nb, RGLRU_BF16, stream),
+          "rglru_hip_prepare_block_fwd");
     Tensor out;
-    if (own_linear(x, wx, bx)) {
+    if (!stack) {
       out = fresh_like(x);
       check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, s[2], nullptr, W, ptr(wo), nullptr, W, ptr(bo), nullptr, bptr(active), ptr(out), nullptr, D,
                              nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
@@ -1528,7 +1531,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       if (active.defined()) masked_rows(out, active, true);
     }
     ctx->save_for_backward({x, wx, wy, wo, cw, pos, flags, rows, active, u, v, buffer});
-    pack(ctx, {first_reset, nb});
+    pack(ctx, {first_reset, nb, stack});
     return out;
   }
 
@@ -1549,14 +1552,15 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
       char *image = s[u.defined() ? 3 : 5], *ws = image + round_up(prep_bytes(W, nb, RGLRU_BF16));
       Tensor dy = aligned(grads[0].to(kType));
-      const bool own = own_linear(x, wx, Tensor());
+      const bool own = !m[2];
       if (!own && active.defined()) dy = masked_rows(dy, active, false);
 
       // parameter gradients: parts of one allocation
       Parts out;
       for (int64_t n : {2 * W * D, 2 * W, W * K, W, W * bw, W, W * bw, W, W, D * W, D}) out.add(n * 2);
       out.allocate(x);
-      Tensor dw_pair = out.take({2, W, D}, kType), db_pair = out.take({2, W}, kType);
+      Tensor dw_pair = out.take({2, W, D}, kType);
+      out.next++;                                          // the two bias gradients: g[BX], g[BY]
       g[CW] = out.take({W, 1, K}, kType), g[CB] = out.take({W}, kType);
       g[WA] = out.take({nb, bw, bw}, kType), g[BA] = out.take({nb, bw}, kType), g[WI] = out.take({nb, bw, bw}, kType), g[BI] = out.take({nb, bw}, kType);
       g[LAM] = out.take({W}, kType);
@@ -1565,17 +1569,17 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       g[BX] = part(out.buffer, out.offsets[1], {W}, kType), g[BY] = part(out.buffer, out.offsets[1] + W * 2, {W}, kType);
 
       const WeightGrad go(M, D, W, 1, kType), gp(M, W, D, 2, kType);
-      const size_t column_bytes_o = rglru_hip_colsum_scratch_bytes(M, D), column_bytes_p = rglru_hip_colsum_scratch_bytes(M, 2 * W);
+      const size_t column_bytes_o = rglru_hip_colsum_scratch_bytes(M, D);
       Parts scratch;
       scratch.add(M * W * 2), scratch.add(2 * M * W * 2);
       scratch.add(rglru_hip_bwd_scratch_bytes(B, T, W, nb, RGLRU_BF16)), scratch.add(rglru_hip_conv_scratch_bytes(B, T, W, K));
       scratch.add(own ? go.sets_bytes : 0), scratch.add(own ? go.sums_bytes : column_bytes_o);
-      scratch.add(own ? gp.sets_bytes : 0), scratch.add(own ? gp.sums_bytes : column_bytes_p);
+      scratch.add(own ? gp.sets_bytes : 0), scratch.add(rglru_hip_block_sums_bytes(B, T, W, nb));
       scratch.allocate(x);
       char *dgated = scratch.raw(), *du = scratch.raw(), *gate_scratch = scratch.raw(), *conv_scratch = scratch.raw(), *sets_o = scratch.raw(),
            *sums_o = scratch.raw(), *sets_p = scratch.raw(), *sums_p = scratch.raw();
       char* dv = du + W * 2;                               // the halves of one [M, 2 W] matrix
-      rglru_sum sums[4];
+      rglru_sum sums[3];
       Tensor held_o, held_p;                               // results of the BLAS library that the last launch reads
 
       // output projection
@@ -1594,7 +1598,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
         sums[1] = {sums_o, ptr(g[BO]), int64_t(column_bytes_o / (4 * D)), D, RGLRU_F32};
       }
       check(rglru_hip_block_bwd(dgated, s[1], up, vp, s[0], image, ptr(cw), iptr(pos), static_cast<const int32_t*>(ptr(rows)),
-                                flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, du, dv, 2 * W, B, T, W, nb, K, stream),
+                                flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, sums_p, du, dv, 2 * W, B, T, W, nb, K, stream),
             "rglru_hip_block_bwd");
       // input projections
       const bool need_x = ctx->needs_input_grad(0);
@@ -1604,18 +1608,17 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
           check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, du, dv, 2 * W, ptr(wx), ptr(wy), D, nullptr, nullptr, nullptr, ptr(g[X]), nullptr, D,
                                  nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
         }
-        gp.run(du, dv, 2 * W, ptr(x), nullptr, ptr(dw_pair), sets_p, sums_p, M, kType, stream);
-        sums[2] = gp.weight_sum(sets_p, ptr(dw_pair)), sums[3] = gp.bias_sum(sums_p, ptr(db_pair));
+        gp.run(du, dv, 2 * W, ptr(x), nullptr, ptr(dw_pair), sets_p, nullptr, M, kType, stream);
+        sums[2] = gp.weight_sum(sets_p, ptr(dw_pair));
       } else {
         Tensor both = part(scratch.buffer, scratch.offsets[1], {M, 2 * W}, kType);
-        if (need_x) g[X] = at::mm(both, at::cat({wx, wy})).view(x.sizes());
+        const size_t stacked = static_cast<size_t>(ws - s.at) + round_up(rglru_hip_workspace_bytes(B, T, W, nb));
+        if (need_x) g[X] = at::mm(both, part(buffer, stacked, {2 * W, D}, kType)).view(x.sizes());
         held_p = contraction(both, x.view({M, D}));
-        check(rglru_hip_colsum(du, sums_p, nullptr, M, 2 * W, RGLRU_BF16, RGLRU_BF16, stream), "rglru_hip_colsum");
         sums[2] = {ptr(held_p), ptr(dw_pair), held_p.size(0), 2 * W * D, RGLRU_BF16};
-        sums[3] = {sums_p, ptr(db_pair), int64_t(column_bytes_p / (8 * W)), 2 * W, RGLRU_F32};
       }
-      check(rglru_hip_block_finish(image, gate_scratch, conv_scratch, ptr(g[WA]), ptr(g[WI]), ptr(g[BA]), ptr(g[BI]), ptr(g[LAM]), ptr(g[CW]),
-                                   ptr(g[CB]), sums, 4, B, T, W, nb, K, stream), "rglru_hip_block_finish");
+      check(rglru_hip_block_finish(image, gate_scratch, conv_scratch, sums_p, ptr(g[WA]), ptr(g[WI]), ptr(g[BA]), ptr(g[BI]), ptr(g[LAM]),
+                                   ptr(g[CW]), ptr(g[CB]), ptr(g[BX]), ptr(g[BY]), sums, 3, B, T, W, nb, K, stream), "rglru_hip_block_finish");
       for (int i = 1; i < kTensors; ++i)
         if (!ctx->needs_input_grad(i)) g[i] = Tensor();
     }

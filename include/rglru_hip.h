@@ -380,24 +380,26 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
 /* Reverse mode of what rglru_hip_prepare_block_fwd does between the projections (griffin/griffin.py:474-520), up to the last
  * sums of the parameter gradients, which rglru_hip_block_finish does for the whole block in one launch.
  * `dgated`[B,T,W]: the gradient at the gated output on entry, scratch afterwards; y, v, x_conv: as that call wrote or read
- * them; u: the first projection, contiguous; positions / rows as for rglru_hip_conv_rows_bwd.  Writes du and dv, rows
- * `d_stride` elements apart (W, or 2 W for the halves of one matrix).  gate_scratch: rglru_hip_bwd_scratch_bytes, conv_scratch:
- * rglru_hip_conv_scratch_bytes; both hold the partial sums until rglru_hip_block_finish.  bf16 storage, parameters and
- * gradients; no carried state.  Only where rglru_hip_fast_path() is 1. */
+ * them (contiguous); u: the first projection, contiguous; positions / rows as for rglru_hip_conv_rows_bwd.  Writes du and dv,
+ * rows `d_stride` elements apart (W, or 2 W for the halves of one matrix).  gate_scratch: rglru_hip_bwd_scratch_bytes,
+ * conv_scratch: rglru_hip_conv_scratch_bytes, sums_scratch: rglru_hip_block_sums_bytes; they hold the partial sums until
+ * rglru_hip_block_finish.  bf16 storage, parameters and gradients; no carried state.  Only where rglru_hip_fast_path() is 1. */
+size_t rglru_hip_block_sums_bytes(int64_t B, int64_t T, int64_t W, int64_t nb);
 int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
                         const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
-                        void* gate_scratch, void* conv_scratch, void* du, void* dv, int64_t d_stride,
+                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride,
                         int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
 
 /* dst[i] = sum over s < sets of src[s * n + i] (src_dtype), fp32 accumulation in a fixed order; up to five in one launch, all
  * with results in dst_dtype.  dst NULL: skipped. */
 typedef struct { const void* src; void* dst; int64_t sets, n; int src_dtype; } rglru_sum;
 int rglru_hip_sums(const rglru_sum* sums, int n_sums, int dst_dtype, void* stream);
-/* The parameter gradients (bf16) of the block from the partial sums of rglru_hip_block_bwd, and up to four further sums
- * (weight and bias gradients of the projections), in one launch.  dtaps, dbias, and any dst may be NULL. */
-int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, void* dw_a, void* dw_x,
-                           void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, const rglru_sum* sums, int n_sums,
-                           int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
+/* The parameter gradients (bf16) of the block from the partial sums of rglru_hip_block_bwd -- du_sums[W] and dv_sums[W] are the
+ * gradients of the projections' biases -- and up to four further sums (weight gradients, output bias), in one launch.  dtaps,
+ * dbias, and any dst may be NULL. */
+int rglru_hip_block_finish(const void* prep, const void* gate_scratch, const void* conv_scratch, const void* sums_scratch, void* dw_a,
+                           void* dw_x, void* db_a, void* db_x, void* dlambda, void* dtaps, void* dbias, void* du_sums, void* dv_sums,
+                           const rglru_sum* sums, int n_sums, int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
 
 /* Single-token step of the recurrent block (griffin/griffin.py:459-528 with one token per row) in
  * two launches around the caller's three Linear layers:
@@ -452,7 +454,9 @@ int rglru_hip_decode_project(const void* x, int64_t x_stride, const void* w_x, c
  * rglru_hip_block_fwd_path() returns 1 (bf16 storage, gate blocks of 32, 64 or 128 channels, 16-byte
  * aligned rows); otherwise RGLRU_E_UNSUPPORTED, and the caller runs rglru_hip_conv_fwd, rglru_hip_fwd and
  * rglru_hip_gelu_gate_fwd one after the other.  rglru_hip_prepare_block_fwd is rglru_hip_prepare +
- * rglru_hip_block_fwd in two launches (as rglru_hip_prepare_fwd). */
+ * rglru_hip_block_fwd in two launches (as rglru_hip_prepare_fwd); with stack_bytes > 0 the first of them also copies stack0 and
+ * stack1 (so many bytes each) one behind the other to `stacked`: the two projections' weights as the one matrix that their
+ * input gradient's GEMM takes. */
 int rglru_hip_block_fwd_path(int64_t W, int64_t nb, int64_t K, int dtype);
 int rglru_hip_block_flags(const int64_t* segment_pos, uint8_t* flags, int64_t n, void* stream);
 int rglru_hip_block_fwd(const void* u, int64_t u_stride, const void* v, int64_t v_stride,
@@ -466,6 +470,7 @@ int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_
                                 const void* conv_state, const void* taps, const void* conv_bias, int64_t K,
                                 const float* h0, const uint8_t* flags,
                                 void* x_conv, void* y, void* gated, void* new_conv_state, float* h_last, void* ws,
+                                const void* stack0, const void* stack1, void* stacked, int64_t stack_bytes,
                                 int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
 
 /* rglru_hip_block_fwd for inference with every token active, positions included, in two launches: token t of row b stands at
