@@ -240,9 +240,10 @@ RGLRU_DEVICE WaveId wave_identity(const FusedArgs& p, int block, bool scalar_wav
 
 // Channel behind column `col` of a unit's 128-wide tile, or -1.  Blocks take bwp columns of it each (their width rounded up
 // to whole 32-channel slabs); the columns a block does not fill hold zeros, and nothing is stored for them.
-template <bool PAD>
+template <bool PAD, bool WIDE = false>
 RGLRU_DEVICE int tile_channel(const FusedArgs& p, int unit, int tile_col, int col) {
   if constexpr (!PAD) return tile_col + col;
+  if constexpr (WIDE) return col < p.bw ? tile_col + col : -1;       // the tile is one block
   const int blk = col / p.bwp, c = col - blk * p.bwp, k = unit * p.bpu + blk;
   return c < p.bw && blk < p.bpu && k < p.nb ? k * p.bw + c : -1;
 }
@@ -473,10 +474,11 @@ inline int step16_groups(const Geometry& g, int dtype, int aligned) {
 // ... and for the blocks wider than a workgroup's four slabs whose weights the forward and the
 // gate-gradient kernels hold in registers: K groups of the padded width (whole 32-channel slabs), or 0.  A block of any multiple
 // of 8 channels takes them (`padded` as above): at B8 T1000 W1216 (152 channels) the portable kernels took 274 us, forward and
-// backward.
+// backward, these 187.
 inline int wide_groups(const Geometry& g, int dtype, int aligned) {
   return dtype == RGLRU_BF16 && aligned && g.bw % 8 == 0 && g.bwp > 128 && g.bwp <= 384 ? (int)(g.bwp / 16) : 0;
 }
+inline bool wide_padded(const Geometry& g) { return g.bw != g.bwp; }
 
 #define RGLRU_DISPATCH(KERNEL, grid, stream, args, dtype, nkg)                                         \
   do {                                                                                                 \

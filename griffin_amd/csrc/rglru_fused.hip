@@ -197,7 +197,7 @@ constexpr int fwd_lds_groups(int nkg, bool masked) {
 // consecutive rows of eight channels plus the three rows in front of them, convolves them (taps by lag
 // from LDS, lags masked per token through bits 2-3 of the flag bytes = 3 - min(position, 3)) and puts the
 // result where the plain kernel puts x; the store stage multiplies by gelu_tanh of the second projection.
-// PAD: blocks of up to 128 channels that do not fill their slabs (see narrow_groups); masked variant only.
+// PAD: blocks that do not fill their slabs (see narrow_groups, wide_groups); masked variant only.
 template <typename IO, int NKG, bool MASKED, bool BLOCK = false, bool PAD = false>
 __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : (NKG == 4 || NKG == 2) ? RGLRU_NARROW_OCC : NKG > 8 ? fwd_wide_occ(NKG) : 2)) void fwd_kernel(FusedArgs p) {
   constexpr int MT = fwd_mt(NKG), TR = 32 * MT, EL = 16 * MT;
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
       if constexpr (BLOCK)
         pre_off[i] = bcol_ok ? (unsigned)(4 * rho + i + 3) * x_row_bytes + bcol_bytes : kOutOfRange;
       else {
-        const int col = tile_channel<PAD>(p, w.unit, x_col, cv * Tr::HW);
+        const int col = tile_channel<PAD, (NKG > 8)>(p, w.unit, x_col, cv * Tr::HW);
         pre_off[i] = (idx < TR * VPR && col >= 0) ? (unsigned)row * row_bytes + (unsigned)col * (unsigned)sizeof(IO) : kOutOfRange;
       }
       if constexpr (GIVEN)
@@ -898,8 +898,9 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   a.B = (int)B; a.T = (int)T; a.nC = (int)L.nC; a.ckpt_nC = 2 * (int)L.nC;
   a.aligned = is_aligned(x, W, g.bw, elem_size(dtype)) && ((uintptr_t)y % 16 == 0);
   int nkg = narrow_groups(g, dtype, a.aligned);
-  const bool narrow = nkg != 0, pad = narrow && narrow_padded(g);
+  const bool narrow = nkg != 0;
   if (!nkg && !pre) nkg = wide_groups(g, dtype, a.aligned);
+  const bool pad = narrow ? narrow_padded(g) : nkg > 8 && wide_padded(g);
   if (pre) {
     if (!rglru_hip_pre_path(W, nb, dtype)) return fail(RGLRU_E_UNSUPPORTED, "fwd_pre: needs bf16 storage and gate blocks of a multiple of 32 channels");
     if (!a.aligned || (uintptr_t)pre % 16) return fail(RGLRU_E_UNSUPPORTED, "fwd_pre: x, pre and y must be 16-byte aligned");
@@ -993,6 +994,9 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
       }
       RGLRU_PAD_CASE(8) RGLRU_PAD_CASE(6) RGLRU_PAD_CASE(4) RGLRU_PAD_CASE(2)
 #undef RGLRU_PAD_CASE
+#define RGLRU_PAD_WIDE(N) if (nkg == N) hipLaunchKernelGGL((fwd_kernel<__bf16, N, true, false, true>), grid, dim3(kThreads), 0, s, a);
+      RGLRU_PAD_WIDE(10) RGLRU_PAD_WIDE(12) RGLRU_PAD_WIDE(14) RGLRU_PAD_WIDE(16) RGLRU_PAD_WIDE(18) RGLRU_PAD_WIDE(20) RGLRU_PAD_WIDE(22) RGLRU_PAD_WIDE(24)
+#undef RGLRU_PAD_WIDE
     } else if (blk) {
 #define RGLRU_BLOCK_CASE(N)                                                                                            \
       if (nkg == N) {                                                                                                  \

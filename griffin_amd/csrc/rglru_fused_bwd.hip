@@ -155,7 +155,8 @@ template <int ROWS> struct PairStage {                  // ROWS x 32 channels x 
   static RGLRU_DEVICE unsigned row_offset(int row) { return (unsigned)row * kRowBytes + (row >= ROWS / 2 ? 128u : 0u); }
 };
 
-template <typename IO, int NKG, bool MASKED>
+// PAD: wide blocks that do not fill their slabs: columns past the block's width read as zero, their lanes store and publish nothing.
+template <typename IO, int NKG, bool MASKED, bool PAD = false>
 __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(FusedArgs p) {
   constexpr int MT = 1, TR = 32, EL = 16;
   typedef Io<IO> Tr;
@@ -209,6 +210,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
   }
   const float nba = -kLog2e * p.bias[w.kp], nbx = -kLog2e * p.bias[p.Wp + w.kp];   // biases as the sigmoids take them
   const float sp = p.sp[w.kp], cs = p.cs[w.kp];
+  const bool ch_ok = !PAD || w.ch_ok;
   const IO* x = (const IO*)p.x;
   const IO* dy = (const IO*)p.dy;
   const long long W = p.W;
@@ -232,7 +234,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
   for (int i = 0; i < NV; ++i) {
     const int idx = tid + i * kThreads;
     const int row = idx / VPR, cv = idx - row * VPR;
-    pre_off[i] = (idx < TR * VPR) ? (unsigned)row * row_bytes + (unsigned)(x_col + cv * Tr::HW) * 2u : kOutOfRange;
+    pre_off[i] = (idx < TR * VPR && (!PAD || cv * Tr::HW < p.bw)) ? (unsigned)row * row_bytes + (unsigned)(x_col + cv * Tr::HW) * 2u : kOutOfRange;
     if constexpr (GIVEN)
       u_off[i] = (idx < TR * VPR) ? (unsigned)row * u_row_bytes + (unsigned)(group_col + cv * Tr::HW) * 2u : kOutOfRange;
   }
@@ -398,7 +400,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
     const long long seq = (long long)b * p.nC * W + w.ch;
     chain.rec = p.rec_a + seq; chain.stride = W;
     const bool last_chunk = c == p.nC - 1;
-    if (!last_chunk && hf == 0) carry_publish(chain, c, A_t, D_t, false);
+    if (!last_chunk && hf == 0 && ch_ok) carry_publish(chain, c, A_t, D_t, false);
 
     // input gate and g = sqrt(1 - a^2)
 #pragma unroll
@@ -410,13 +412,13 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
       gi[e] = ie; g[e] = ge;
     }
     float d_in = (last_chunk && p.dh_last) ? p.dh_last[(long long)b * W + w.ch] : 0.f;
-    if (!last_chunk) d_in = carry_lookback(chain, c, +1, p.nC, 0.f, true, p.limit, p.fail);
+    if (!last_chunk) d_in = carry_lookback(chain, c, +1, p.nC, 0.f, ch_ok, p.limit, p.fail);
     // the next tile's loads go out behind the look-back: loads return in issue order, so requested in front of it
     // they would put their latency into every round trip of the walk
     issue(tk_next);
     const float d_out = fmaf(A_t, d_in, D_t);
-    if (hf == 0) carry_publish(chain, c, 0.f, d_out, true);
-    if (hf == 0 && c == 0 && p.dh0) p.dh0[(long long)b * W + w.ch] = d_out;
+    if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
+    if (hf == 0 && c == 0 && p.dh0 && ch_ok) p.dh0[(long long)b * W + w.ch] = d_out;
 
     // delta_t in place of dy_t (reverse), then one forward pass that carries h_{t-1} along
     carry = hf ? d_in : fmaf(A_hi, d_in, D_hi);
@@ -464,7 +466,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
     {
       const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
       const rsrc_t rdx = make_rsrc((const IO*)p.dx + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage_dx, rdx, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane);
+      stage_flush<TR>(stage_dx, rdx, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane, !PAD || w.slab * 32 + (w.lane & 3) * 8 < p.bw);
       if constexpr (GIVEN) {
         IO* dbase = (IO*)p.du_a + ((long long)w.k * p.rows_total + (long long)b * p.T + t0) * (2 * p.bw);
         const rsrc_t rdu = make_rsrc(dbase, (unsigned)rows * u_row_bytes);
@@ -479,7 +481,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
         const int row = 8 * i + (w.lane >> 3);
         const unsigned seg = (unsigned)(w.lane & 7) * 16u;
         i32x4 v = *reinterpret_cast<const i32x4*>(stage_du + PairStage<TR>::row_offset(row) + seg);
-        buf_store_b128(v, rdu, (unsigned)row * du_row_bytes + du_col + seg);
+        buf_store_b128(v, rdu, !PAD || w.slab * 32 + (w.lane & 7) * 4 < p.bw ? (unsigned)row * du_row_bytes + du_col + seg : kOutOfRange);
       }
       }
     }
@@ -1350,7 +1352,7 @@ template <int NKG> struct GateGradWideLds {
   static constexpr int kBuffers = kDouble ? 2 : 1;
 };
 
-template <typename IO, int NKG>
+template <typename IO, int NKG, bool PAD = false>
 __global__ __launch_bounds__(kGradThreads, 1) void gate_grad_wide_kernel(FusedArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
@@ -1421,11 +1423,11 @@ __global__ __launch_bounds__(kGradThreads, 1) void gate_grad_wide_kernel(FusedAr
   for (int i = 0; i < NV_DU; ++i) {
     const int idx = tid + i * kGradThreads;
     const int row = idx / VPR_DU, cv = idx - row * VPR_DU;
-    du_off[i] = idx < TR * VPR_DU ? (unsigned)row * 2u * row_bytes + (unsigned)(2 * k * p.bw + cv * Tr::HW) * 2u : kOutOfRange;
+    du_off[i] = idx < TR * VPR_DU && (!PAD || cv * Tr::HW < 2 * p.bw) ? (unsigned)row * 2u * row_bytes + (unsigned)(2 * k * p.bw + cv * Tr::HW) * 2u : kOutOfRange;
   }
   {
     const int row = tid / VPR_X, cv = tid - row * VPR_X;
-    x_off = (tid < TR * VPR_X && jg * JW + cv * Tr::HW < KC) ? (unsigned)row * row_bytes + (unsigned)(unit_col + cv * Tr::HW) * 2u : kOutOfRange;
+    x_off = (tid < TR * VPR_X && jg * JW + cv * Tr::HW < (PAD ? p.bw : KC)) ? (unsigned)row * row_bytes + (unsigned)(unit_col + cv * Tr::HW) * 2u : kOutOfRange;
   }
   auto issue = [&](Pre& s, long long tile) {
     // a tile past the end keeps valid addresses but an empty extent: nothing is fetched
@@ -1554,7 +1556,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void gate_grad_wide_kernel(FusedAr
       const int frow = ((lane >> 4) & 1) * 16 + 4 * q + ((lane >> 2) & 3);
       const unsigned seg = (unsigned)(lane & 3) * 16u;
       const i32x4 v = *reinterpret_cast<const i32x4*>(stage + WaveStage<TR>::row_offset(frow) + seg);
-      buf_store_b128(v, rdx, (lane < 32 && slab_ok) ? (unsigned)frow * row_bytes + (unsigned)(k * p.bw + j0) * 2u + seg : kOutOfRange);
+      buf_store_b128(v, rdx, (lane < 32 && slab_ok && (!PAD || j0 + (lane & 3) * 8 < p.bw)) ? (unsigned)frow * row_bytes + (unsigned)(k * p.bw + j0) * 2u + seg : kOutOfRange);
       wave_lds_fence();
     }
     if (DB) buf ^= 1;
@@ -2134,7 +2136,7 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   rc = check_grad_dtype("bwd_wide", grad_dtype);
   if (rc) return rc;
   if (!rglru_hip_wide_path(W, nb, dtype))
-    return fail(RGLRU_E_UNSUPPORTED, "bwd_wide: needs 16-bit storage and gate blocks of 160 to 384 channels in steps of 32");
+    return fail(RGLRU_E_UNSUPPORTED, "bwd_wide: needs 16-bit storage and gate blocks of 129 to 384 channels, a multiple of 8");
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "bwd_wide: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
   if (!x || !prep || !dy || !ws || !scratch || !dx || !dw_a || !dw_x || !db_a || !db_x || !dlambda)
     return fail(RGLRU_E_ARG, "bwd_wide: null pointer");
@@ -2163,6 +2165,7 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   a.B = (int)B; a.T = (int)T; a.nC = (int)((T + kChunk - 1) / kChunk); a.ckpt_nC = 2 * (int)L.nC; a.nCf = (int)L.nCf;
   a.aligned = 1;
   const int nkg = wide_groups(g, dtype, 1);
+  const bool pad = wide_padded(g);
   // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums
   a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 1, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
@@ -2175,7 +2178,8 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
     KernelTimer timer(1, s);
 #define RGLRU_LAUNCH_WIDE_SCAN(N)                                                                                    \
     case N:                                                                                                          \
-      if (masked) hipLaunchKernelGGL((bwd_scan_kernel<__bf16, N, true>), grid, dim3(kThreads), 0, s, a);              \
+      if (pad) hipLaunchKernelGGL((bwd_scan_kernel<__bf16, N, true, true>), grid, dim3(kThreads), 0, s, a);           \
+      else if (masked) hipLaunchKernelGGL((bwd_scan_kernel<__bf16, N, true>), grid, dim3(kThreads), 0, s, a);         \
       else hipLaunchKernelGGL((bwd_scan_kernel<__bf16, N, false>), grid, dim3(kThreads), 0, s, a);                     \
       break
     switch (nkg) {
@@ -2198,16 +2202,16 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   dim3 grid2((unsigned)(8 * ((grad_pairs + 7) / 8) * ((g.S + 1) / 2)));
   {
     KernelTimer timer(3, s);
+#define RGLRU_LAUNCH_WIDE_GRAD(N)                                                                                     \
+    case N:                                                                                                          \
+      if (pad) hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, N, true>), grid2, dim3(kGradThreads), 0, s, a);      \
+      else hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, N>), grid2, dim3(kGradThreads), 0, s, a);                \
+      break
     switch (nkg) {
-      case 10: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 10>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 12: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 12>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 14: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 14>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 16: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 16>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 18: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 18>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 20: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 20>), grid2, dim3(kGradThreads), 0, s, a); break;
-      case 22: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 22>), grid2, dim3(kGradThreads), 0, s, a); break;
-      default: hipLaunchKernelGGL((gate_grad_wide_kernel<__bf16, 24>), grid2, dim3(kGradThreads), 0, s, a); break;
+      RGLRU_LAUNCH_WIDE_GRAD(10); RGLRU_LAUNCH_WIDE_GRAD(12); RGLRU_LAUNCH_WIDE_GRAD(14); RGLRU_LAUNCH_WIDE_GRAD(16);
+      RGLRU_LAUNCH_WIDE_GRAD(18); RGLRU_LAUNCH_WIDE_GRAD(20); RGLRU_LAUNCH_WIDE_GRAD(22); RGLRU_LAUNCH_WIDE_GRAD(24);
     }
+#undef RGLRU_LAUNCH_WIDE_GRAD
   }
   rc = check_launch("bwd_wide gate gradients");
   if (rc) return rc;

@@ -103,7 +103,7 @@ int gate_dw_splits(long long N, const Geometry& g);
 // Scratch of one backward call; nothing in it outlives the call, its contents on entry do not matter.
 //   partial     [maxWg][3][Wp]  per-workgroup sums for db_a, db_x, dLambda
 //   delta       fast backward (blocks of 32, 64, 128 channels): [B][T][W] 16-bit, dL/dh_t after the
-//               reverse scan; wide backward (blocks of 160 .. 384 channels): [B][T][nb][2 bw] 16-bit,
+//               reverse scan; wide backward (blocks of 129 .. 384 channels): [B][T][nb][2 bw] 16-bit,
 //               the gradients at the gate pre-activations as pairs (element 2 o + gate)
 //   dw_partial  [sets][nb][2][bwp][bwp] per-workgroup weight-gradient sums, sets = kGemmWgPerUnit (fast),
 //               kWideWgPerUnit (wide) or gate_dw_splits (the other paths); fp32, or bf16 in the fast backward

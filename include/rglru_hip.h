@@ -10,7 +10,7 @@
  *   griffin/triton_scan.py:246-271  _FusedRGLRUScan.backward  rglru_hip_scan_bwd
  *   griffin/griffin.py:237-289      RG_LRU.forward (gates + scan, T > 1)   rglru_hip_prepare + rglru_hip_fwd
  *   autograd of griffin/griffin.py:237-289                                   rglru_hip_bwd_full (blocks of 32/64/128 channels),
- *                                                                            rglru_hip_bwd_wide (160 .. 384), rglru_hip_bwd (any)
+ *                                                                            rglru_hip_bwd_wide (129 .. 384), rglru_hip_bwd (any)
  *   the same for bf16 blocks of 416 .. 512 channels (gate projections of griffin/griffin.py:149-154 as a GEMM kernel of their own)   rglru_hip_fwd_pre, rglru_hip_bwd_pre
  *   griffin/griffin.py:279-284 with T == 1 (decode step, carried state)     rglru_hip_step, rglru_hip_steps (K steps a launch)
  *   (no counterpart: forward for callers that cannot allocate)              rglru_hip_fwd_static
@@ -183,7 +183,7 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
                        float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
                        void* stream);
 
-/* Complete backward for gate blocks of 160 to 384 channels in steps of 32 (rglru_hip_wide_path(W, nb,
+/* Complete backward for gate blocks of 129 to 384 channels, a multiple of 8 (rglru_hip_wide_path(W, nb,
  * dtype) != 0: 16-bit storage; griffin/griffin.py:149-154 at those widths and its autograd).  For these
  * widths rglru_hip_fwd and rglru_hip_prepare_fwd hold a block's weights in the registers of several
  * workgroups (four 32-channel slabs each), and this entry point is the matching backward: same inputs

@@ -942,3 +942,25 @@ def test_portable_kernels_pack_narrow_blocks(bw, nb, dtype, tol):
     assert rel_err(y.float(), ry) < tol and rel_err(h_last, rh) < tol
     for name in rgrads:
         assert rel_err(grads[name].float(), rgrads[name]) < tol, name
+
+
+@pytest.mark.parametrize("bw,nb", [(136, 2), (152, 3), (168, 1), (216, 2), (248, 1), (264, 2), (312, 1), (344, 1), (376, 2)])
+@pytest.mark.parametrize("B,T,masks,carried", [(2, 70, True, True), (1, 64, False, False), (3, 33, False, True)])
+def test_padded_wide_blocks_match_oracle(bw, nb, B, T, masks, carried):
+    """bf16 gate blocks of any multiple of 8 channels between 128 and 384 run the wide kernels with a last slab that is not
+    full: outputs, final state and every gradient against the oracle."""
+    from griffin_amd import _lib
+    from griffin_amd.hip_scan import kernel_path
+
+    W = bw * nb
+    assert kernel_path(B, T, W, nb, torch.bfloat16) == _lib.PATH_WIDE
+    _say("padded wide blocks", bw, nb, B, T, masks, carried)
+    case = orc.make_case(B, T, W, nb, seed=bw, h0_std=0.5 if carried else 0.0, bias_std=0.5)
+    reset, active = _masks(B, T, masks)
+    dh_last = torch.randn(B, W, generator=torch.Generator().manual_seed(6)) if carried else None
+    y, h_last, grads = hip_run(case, torch.bfloat16, reset, active, dh_last)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, active, dh_last)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
