@@ -399,9 +399,10 @@ py::tuple fingerprint(const std::vector<Tensor>& tensors) {
 struct Stamp {
   std::vector<std::pair<const void*, int64_t>> seen;
   Tensor image;
-  int64_t blocks;
-  double c;
-  at::ScalarType dtype;
+  int64_t blocks = 0;
+  double c = 0.0;
+  at::ScalarType dtype = at::kFloat;
+  Stamp() = default;
   Stamp(const std::vector<Tensor>& tensors, const Tensor& img, int64_t nb, double decay, at::ScalarType type)
       : image(img), blocks(nb), c(decay), dtype(type) {
     for (const Tensor& t : tensors) seen.emplace_back(t.data_ptr(), static_cast<int64_t>(t._version()));
@@ -414,11 +415,51 @@ struct Stamp {
     return true;
   }
   bool matches(const std::vector<Tensor>& tensors, double decay, at::ScalarType type, c10::Device device) const {
-    return image.device() == device && holds(tensors, tensors.size(), decay, type);
+    return image.defined() && image.device() == device && holds(tensors, tensors.size(), decay, type);
   }
 };
 
 // ---- decode steps ----------------------------------------------------------------------------------------------
+
+// The ends of the autograd graph at a module's parameters, held between training steps.  A leaf keeps its accumulation node only
+// by a weak reference, so the node dies with every graph and is made again by the next forward: with the five parameters of the
+// RG-LRU 9 us of the 114 us that the host takes for a training step (width 256; the device needs 30).  A node made under
+// another stream or for another shape of the parameter is not kept: a new one is made as if none had been there.
+struct Leaves {
+  typedef std::shared_ptr<torch::autograd::Node> NodePtr;
+  std::vector<NodePtr> nodes;
+  std::optional<c10::Stream> stream;
+  static bool ends(const Tensor& t) { return t.defined() && t.requires_grad() && t.is_leaf(); }
+  static bool current(const NodePtr& node, const Tensor& t) {
+    if (!ends(t)) return node == nullptr;
+    return node != nullptr && node == torch::autograd::impl::try_get_grad_accumulator(t) && node->input_metadata(0).is_same_shape(t);
+  }
+  // under the interpreter's lock; every change of `nodes` is one step, so another thread may come in where a node's end lets it
+  void hold(const std::vector<Tensor>& tensors) {
+    const c10::Stream now = c10::hip::getCurrentHIPStream(tensors[0].device().index()).unwrap();
+    bool same = nodes.size() == tensors.size() && stream == now;
+    for (size_t i = 0; same && i < tensors.size(); ++i) same = current(nodes[i], tensors[i]);
+    if (same) return;
+    std::vector<NodePtr>().swap(nodes);
+    std::vector<NodePtr> fresh;
+    for (const Tensor& t : tensors) fresh.push_back(ends(t) ? torch::autograd::impl::grad_accumulator(t) : nullptr);
+    stream = now;
+    nodes.swap(fresh);
+  }
+};
+
+// Hold the leaves `tensors` of a module in its instance dictionary.
+void hold_leaves(const py::dict& members, const std::vector<Tensor>& tensors) {
+  if (!at::GradMode::is_enabled() || tensors.empty() || !tensors[0].is_cuda()) return;
+  PyObject* held = PyDict_GetItemString(members.ptr(), "_leaves");
+  if (held == nullptr || !py::isinstance<Leaves>(held)) {
+    py::object made = py::cast(new Leaves(), py::return_value_policy::take_ownership);
+    members["_leaves"] = made;
+    made.cast<Leaves*>()->hold(tensors);
+  } else {
+    py::handle(held).cast<Leaves*>()->hold(tensors);
+  }
+}
 
 Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
   Tensor flags = opt(flags_);
@@ -1089,7 +1130,7 @@ const Stamp* current_stamp(const Members& lru, at::ScalarType dtype, c10::Device
       !lru.parameter("Lambda", p[4]))
     return nullptr;
   const Stamp* s = py::handle(held).cast<const Stamp*>();
-  return s->image.device() == device && s->holds(p, p.size(), lru.number("c", 0.0), dtype) ? s : nullptr;
+  return s->image.defined() && s->image.device() == device && s->holds(p, p.size(), lru.number("c", 0.0), dtype) ? s : nullptr;
 }
 
 // RG_LRU on one token per row without masks: (y, state).
@@ -1790,6 +1831,7 @@ py::object norm_forward(py::handle module, const Tensor& x) {
   const bool bf16 = x.scalar_type() == at::kBFloat16;
   const int code = code_of(x.scalar_type());
   if (x.size(-1) > rglru_hip_rmsnorm_max_width(code, x.size(-1) % (bf16 ? 8 : 4) == 0)) return py::none();
+  if (g.requires_grad() && at::GradMode::is_enabled()) hold_leaves(py::reinterpret_borrow<py::dict>(norm.dict), {g});
   return py::cast(rmsnorm(x, g, norm.number("eps", 1e-6)));
 }
 
@@ -1802,7 +1844,12 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(fingerprint);
   py::class_<Stamp>(m, "Stamp")
       .def(py::init<const std::vector<Tensor>&, const Tensor&, int64_t, double, at::ScalarType>())
-      .def("matches", &Stamp::matches);
+      .def("matches", &Stamp::matches)
+      // a copy of a module starts without what is kept for the original
+      .def(py::pickle([](const Stamp&) { return py::tuple(); }, [](const py::tuple&) { return Stamp(); }));
+  py::class_<Leaves>(m, "Leaves")
+      .def(py::pickle([](const Leaves&) { return py::tuple(); }, [](const py::tuple&) { return Leaves(); }));
+  m.def("hold_leaves", &hold_leaves);
   EXPORT(mark_usable);
   EXPORT(lru_decode);
   EXPORT(block_decode);

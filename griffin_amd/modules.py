@@ -133,6 +133,7 @@ class RG_LRU(nn.Module):
         ``load_state_dict`` call it."""
         self._prep = None
         self._prep_key = None
+        self._leaves = None
 
     def _apply(self, fn, *args, **kwargs):
         self.invalidate_caches()
@@ -205,8 +206,11 @@ class RG_LRU(nn.Module):
             # is known by identity: the kernels then need no per-token flags at all
             default = _DEFAULT_POSITIONS.get((batch, steps, xt.device))
             first_only = default is not None and reset_mask is default[1] and active_mask is None
+            parameters = self._gate_parameters()
+            if torch.is_grad_enabled():
+                _lib.native().hold_leaves(self.__dict__, parameters)
             y, state = hip_scan.hip_rglru(
-                xt, *self._gate_parameters(), self.c, ht_minus_1, None if first_only else reset_mask, active_mask,
+                xt, *parameters, self.c, ht_minus_1, None if first_only else reset_mask, active_mask,
                 first_token_reset=first_only,
             )
             return (y, state) if return_state else y
@@ -306,6 +310,10 @@ class RMSNorm(nn.Module):
         self.eps = eps
         self.g = nn.Parameter(torch.zeros(dim))
 
+    def _apply(self, fn, *args, **kwargs):
+        self._leaves = None
+        return super()._apply(fn, *args, **kwargs)
+
     def _hip_covers(self, x: Tensor) -> bool:
         if not x.is_cuda or x.dtype not in hip_scan.SUPPORTED_DTYPES or x.numel() == 0:
             return False
@@ -364,10 +372,12 @@ class RecurrentBlock(nn.Module):
         bypass the version counter (``p.data.copy_()``) need this call.  ``module.to()``, ``train()``/``eval()``
         and ``load_state_dict`` call it."""
         self._stacked_projection = None
+        self._leaves = None
         self.rg_lru.invalidate_caches()
 
     def _apply(self, fn, *args, **kwargs):
         self._stacked_projection = None
+        self._leaves = None
         return super()._apply(fn, *args, **kwargs)
 
     def train(self, mode: bool = True):
@@ -511,6 +521,16 @@ class RecurrentBlock(nn.Module):
         """Nobody wrapped or hooked the Linear layer: calling it is a product with its weight and nothing else."""
         return type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks
 
+    def _own_parameters(self):
+        """linear_x, linear_y, convolution, gates, Lambda, linear_out, or None where one is parametrised or otherwise replaced."""
+        layers = self._modules
+        try:
+            px, py, pc, po = (layers[name]._parameters for name in ("linear_x", "linear_y", "temporal_conv", "linear_out"))
+            return (px["weight"], px["bias"], py["weight"], py["bias"], pc["weight"], pc["bias"], *layers["rg_lru"]._gate_parameters(),
+                    po["weight"], po["bias"])
+        except (KeyError, AttributeError):
+            return None
+
     def _whole_parameters(self, x: Tensor):
         """The block's parameters (linear_x, linear_y, convolution, gates, Lambda, linear_out) where one operator may stand for the
         whole block: bf16 on the HIP path, nobody wrapped, hooked or replaced a layer; else None."""
@@ -526,11 +546,8 @@ class RecurrentBlock(nn.Module):
         for m in (lx, ly, conv, lo, lru):
             if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
                 return None
-        try:
-            px, py, pc, po = lx._parameters, ly._parameters, conv._parameters, lo._parameters
-            parameters = (px["weight"], px["bias"], py["weight"], py["bias"], pc["weight"], pc["bias"], *lru._gate_parameters(),
-                          po["weight"], po["bias"])
-        except KeyError:                                     # a parametrised or otherwise replaced parameter
+        parameters = self._own_parameters()
+        if parameters is None:
             return None
         for p in parameters:
             if p is None or p.dtype is not torch.bfloat16:
@@ -659,9 +676,14 @@ class RecurrentBlock(nn.Module):
             if not torch.is_grad_enabled() or not any(t is not None and t.requires_grad for t in (x, *parameters, *carried)):
                 result = self._infer_whole(x, parameters, cache, segment_pos, active_mask, return_cache)
             elif cache is None and not return_cache:
+                _lib.native().hold_leaves(self.__dict__, parameters)
                 result = self._train_whole(x, parameters, segment_pos, active_mask)
             if result is not None:
                 return result
+        elif torch.is_grad_enabled() and self._hip_block_ops_covers(x):
+            held = self._own_parameters()
+            if held is not None:
+                _lib.native().hold_leaves(self.__dict__, [p for p in held if p is not None])
         facts = None
         if not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
             # launched in front of the projections, so that its answer is there before they are done

@@ -848,3 +848,54 @@ def test_random_prefill_and_decode_like_the_cpu_block():
         if not max(errs.values()) < tol:
             failures.append((index, kind, {k: "%.2e" % v for k, v in errs.items() if not v < tol}))
     assert not failures, failures
+
+
+def test_leaves_held_between_steps_follow_the_parameters():
+    """Gradients reach the parameters as they are now: after a step on another stream, with a parameter replaced, resized in
+    place or frozen, after ``.to()``, and in a deep copy or an unpickled copy of a module that has trained and decoded."""
+    import io
+
+    from griffin_amd import RG_LRU
+
+    torch.manual_seed(3)
+    layer = RG_LRU(64, gate_blocks=4).cuda()
+    x = torch.randn(2, 9, 64, device="cuda")
+
+    def grads(m):
+        m.zero_grad(set_to_none=True)
+        m(x.to(m.Lambda.dtype)).float().square().sum().backward()
+        return [None if p.grad is None else p.grad.clone() for p in m.parameters()]
+
+    want = grads(layer)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = grads(layer)
+    torch.cuda.current_stream().wait_stream(side)
+    assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(want, got))
+    layer.Lambda = torch.nn.Parameter(layer.Lambda.detach().clone())
+    got = grads(layer)
+    assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(want, got))
+    layer.Lambda.requires_grad_(False)
+    got = grads(layer)
+    assert layer.Lambda.grad is None and sum(g is not None for g in got) == 4
+    layer.Lambda.requires_grad_(True)
+    with torch.no_grad():
+        layer(x[:, :1])                                      # the decode image of the parameters
+    stored = io.BytesIO()
+    torch.save(layer, stored)
+    stored.seek(0)
+    for other in (copy.deepcopy(layer), torch.load(stored, weights_only=False)):
+        got = grads(other)
+        assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(want, got))
+        with torch.no_grad():
+            assert torch.equal(other(x[:, :1]), layer(x[:, :1]))
+    wider = RG_LRU(128, gate_blocks=4).cuda()
+    for own, new in zip(layer.parameters(), wider.parameters()):
+        own.data = new.data.clone()                          # the same tensors at another size
+    for m in (layer.recurrence_gate, layer.input_gate):
+        m.block_width, m.width = wider.recurrence_gate.block_width, 128
+    layer.rnn_width, x = 128, torch.randn(2, 9, 128, device="cuda")
+    assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(grads(wider), grads(layer)))
+    half = layer.to(torch.bfloat16)
+    assert all(g.dtype == torch.bfloat16 and torch.isfinite(g.float()).all() for g in grads(half))
