@@ -14,7 +14,7 @@ RGLRU_BF16 = 1
 FLAG_RESET = 1
 FLAG_INACTIVE = 2
 CHUNK = 32
-ABI_VERSION = 21
+ABI_VERSION = 22
 PATH_PORTABLE, PATH_FAST_TILED, PATH_FAST_CHAIN, PATH_WIDE, PATH_PRE = range(5)
 PATH_NAMES = ("portable", "fast_tiled", "fast_chain", "wide", "pre")
 
@@ -75,7 +75,7 @@ _SIGNATURES = {
     "rglru_hip_linear": (ctypes.c_int, [ctypes.c_int, _P, _P, _I, _P, _P, _I] + [_P] * 5 + [_I, _P, _P, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_sums": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_block_sums_bytes": (ctypes.c_size_t, [_I, _I, _I, _I]),
-    "rglru_hip_block_bwd": (ctypes.c_int, [_P] * 16 + [_I] * 6 + [_P]),
+    "rglru_hip_block_bwd": (ctypes.c_int, [_P] * 16 + [_I, ctypes.c_int] + [_I] * 5 + [_P]),
     "rglru_hip_block_finish": (ctypes.c_int, [_P] * 14 + [ctypes.c_int] + [_I] * 5 + [_P]),
     "rglru_hip_decode_prepare": (ctypes.c_int, [_P, _I] + [_P] * 10 + [_I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_decode_linear": (ctypes.c_int, [_P, _I] + [_P] * 4 + [_I, _I, _I, ctypes.c_int, _P]),

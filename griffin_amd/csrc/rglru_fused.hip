@@ -1070,6 +1070,8 @@ int rglru_hip_prepare_fwd(const void* w_a, const void* b_a, const void* w_x, con
                           const void* x, const float* h0, const uint8_t* flags,
                           void* y, float* h_last, void* ws,
                           int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream) {
+  const bool both = dtype & RGLRU_BACKWARD_CLEAR;         // also the records and tickets of the backward pass
+  dtype &= ~RGLRU_BACKWARD_CLEAR;
   int rc = check_geometry("prepare_fwd", W, nb, dtype);
   if (rc) return rc;
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "prepare_fwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
@@ -1078,7 +1080,7 @@ int rglru_hip_prepare_fwd(const void* w_a, const void* b_a, const void* w_x, con
   // of its own in front of the forward kernel, or part of the forward launch where that kernel can do it (fwd_impl).
   const WorkLayout L = make_work_layout(B, T, make_geometry(W, nb));
   PrepArgs pa;
-  rc = build_prep_args(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, L.f_end - L.f_begin, pa);
+  rc = build_prep_args(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, (both ? L.b_end : L.f_end) - L.f_begin, pa);
   if (rc) return rc;
   return fwd_impl(x, prep, h0, flags, y, h_last, ws, B, T, W, nb, dtype, true, stream, nullptr, nullptr, &pa);
 }
@@ -1127,6 +1129,8 @@ int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_
                                 void* x_conv, void* y, void* gated, void* new_conv_state, float* h_last, void* ws,
                                 const void* stack0, const void* stack1, void* stacked, int64_t stack_bytes,
                                 int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream) {
+  const bool both = dtype & RGLRU_BACKWARD_CLEAR;         // also the records and tickets of the backward pass
+  dtype &= ~RGLRU_BACKWARD_CLEAR;
   int rc = check_geometry("prepare_block_fwd", W, nb, dtype);
   if (rc) return rc;
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "prepare_block_fwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
@@ -1135,7 +1139,7 @@ int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_
   if (stack_bytes < 0 || stack_bytes % 16 || (stack_bytes && (!stack0 || !stack1 || !stacked || (uintptr_t)stack0 % 16 || (uintptr_t)stack1 % 16 || (uintptr_t)stacked % 16)))
     return fail(RGLRU_E_ARG, "prepare_block_fwd: the arrays to stack must be whole 16-byte vectors on 16-byte boundaries");
   PrepArgs pa;
-  rc = build_prep_args(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, L.f_end - L.f_begin, pa);
+  rc = build_prep_args(w_a, b_a, w_x, b_x, lambda, c, W, nb, dtype, vec_dtype, prep, (char*)ws + L.f_begin, (both ? L.b_end : L.f_end) - L.f_begin, pa);
   if (rc) return rc;
   pa.stack_from[0] = (const uint4*)stack0; pa.stack_from[1] = (const uint4*)stack1; pa.stack_to = (uint4*)stacked; pa.stack_n = stack_bytes / 16;
   rc = launch_prepare(pa, dtype, stream);

@@ -1832,6 +1832,8 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
                   void* dx, void* du_a, void* du_x, void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda,
                   float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
                   void* stream) {
+  const bool ws_clear = grad_dtype & RGLRU_BACKWARD_CLEAR;
+  grad_dtype &= ~RGLRU_BACKWARD_CLEAR;
   int rc = check_geometry("bwd", W, nb, dtype);
   if (rc) return rc;
   rc = check_grad_dtype("bwd", grad_dtype);
@@ -1861,8 +1863,7 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
   a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 2, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
-  rc = launch_clear(wb, L.b_begin, L.b_end, s);          // records and tickets of this pass
-  if (rc) return rc;
+  if (!ws_clear && (rc = launch_clear(wb, L.b_begin, L.b_end, s)) != 0) return rc;   // records and tickets of this pass
   {
     KernelTimer timer(1, s);
     if (dtype == RGLRU_BF16) hipLaunchKernelGGL(bwd_kernel<__bf16>, grid, dim3(kThreads), 0, s, a);
@@ -1913,7 +1914,7 @@ static int fast_finish_args(const Geometry& g, const void* prep, const char* scr
 struct GateBwd { const void* v; void* dv; int64_t d_stride; float* dv_partial; };
 static int bwd_full_kernels(const void* x, const void* y, const void* prep, const float* h0,
                             const uint8_t* flags, const void* dy, const float* dh_last, void* ws, void* scratch,
-                            void* dx, float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
+                            void* dx, float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype, bool ws_clear,
                             void* stream, const GateBwd* gate = nullptr) {
   int rc = check_geometry("bwd_full", W, nb, dtype);
   if (rc) return rc;
@@ -1975,8 +1976,7 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
     else { if (nkg == 8) RGLRU_LAUNCH_DELTA_CHAIN(8, false, false); else if (nkg == 4) RGLRU_LAUNCH_DELTA_CHAIN(4, false, false); else RGLRU_LAUNCH_DELTA_CHAIN(2, false, false); }
 #undef RGLRU_LAUNCH_DELTA_CHAIN
   } else {
-    rc = launch_clear(wb, L.b_begin, L.b_end, s);        // records and tickets of this pass
-    if (rc) return rc;
+    if (!ws_clear && (rc = launch_clear(wb, L.b_begin, L.b_end, s)) != 0) return rc;   // records and tickets of this pass
     KernelTimer timer(1, s);
 #define RGLRU_LAUNCH_DELTA(N, M, P)                                                                                  \
     do {                                                                                                             \
@@ -2013,11 +2013,13 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
                        void* dx, void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda,
                        float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
                        void* stream) {
+  const bool ws_clear = grad_dtype & RGLRU_BACKWARD_CLEAR;
+  grad_dtype &= ~RGLRU_BACKWARD_CLEAR;
   int rc = check_grad_dtype("bwd_full", grad_dtype);
   if (rc) return rc;
   if (!dw_a || !dw_x || !db_a || !db_x || !dlambda) return fail(RGLRU_E_ARG, "bwd_full: null pointer");
   if ((uintptr_t)dw_a % 16 || (uintptr_t)dw_x % 16) return fail(RGLRU_E_UNSUPPORTED, "bwd_full: dw_a and dw_x must be 16-byte aligned");
-  rc = bwd_full_kernels(x, y, prep, h0, flags, dy, dh_last, ws, scratch, dx, dh0, B, T, W, nb, dtype, grad_dtype, stream);
+  rc = bwd_full_kernels(x, y, prep, h0, flags, dy, dh_last, ws, scratch, dx, dh0, B, T, W, nb, dtype, grad_dtype, ws_clear, stream);
   if (rc) return rc;
   FinishArgs r;
   const int blocks = fast_finish_args(make_geometry(W, nb), prep, (const char*)scratch, B, T, dtype, grad_dtype, dw_a, dw_x, db_a, db_x, dlambda, r);
@@ -2042,7 +2044,7 @@ size_t rglru_hip_block_sums_bytes(int64_t B, int64_t T, int64_t W, int64_t nb) {
 
 int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
                         const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
-                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride,
+                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride, int ws_clear,
                         int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream) {
   if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "block_bwd: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
   if (!dgated || !v || !dv || !sums_scratch) return fail(RGLRU_E_ARG, "block_bwd: null pointer");
@@ -2051,7 +2053,7 @@ int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* 
   // the gradient at the convolution's output takes the place of the one at y * gelu(v)
   const GateBwd gate = {v, dv, d_stride, (float*)sums_scratch};
   const int rc = bwd_full_kernels(x_conv, y, prep, nullptr, flags, dgated, nullptr, ws, gate_scratch, dgated, nullptr, B, T, W, nb, RGLRU_BF16,
-                                  RGLRU_BF16, stream, &gate);
+                                  RGLRU_BF16, ws_clear != 0, stream, &gate);
   if (rc) return rc;
   return conv_bwd_partials(u, nullptr, taps, positions, rows, dgated, conv_scratch, du, d_stride, nullptr, B, T, W, K, RGLRU_BF16,
                            RGLRU_BF16, true, stream);
@@ -2131,6 +2133,8 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
                        void* dx, void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda,
                        float* dh0, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int grad_dtype,
                        void* stream) {
+  const bool ws_clear = grad_dtype & RGLRU_BACKWARD_CLEAR;
+  grad_dtype &= ~RGLRU_BACKWARD_CLEAR;
   int rc = check_geometry("bwd_wide", W, nb, dtype);
   if (rc) return rc;
   rc = check_grad_dtype("bwd_wide", grad_dtype);
@@ -2172,8 +2176,7 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   const bool masked = (flags != nullptr) || a.first_reset || (T % kChunk != 0);
   a.xcd_map = 1;
   dim3 grid((unsigned)(8 * (((long long)nb * a.wg_per_unit + 7) / 8) * a.groups));
-  rc = launch_clear(wb, L.b_begin, L.b_end, s);          // records and tickets of this pass
-  if (rc) return rc;
+  if (!ws_clear && (rc = launch_clear(wb, L.b_begin, L.b_end, s)) != 0) return rc;   // records and tickets of this pass
   {
     KernelTimer timer(1, s);
 #define RGLRU_LAUNCH_WIDE_SCAN(N)                                                                                    \

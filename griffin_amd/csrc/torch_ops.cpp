@@ -216,7 +216,8 @@ struct ForwardResult {
 };
 
 ForwardResult rglru_forward(const Tensor& x_in, const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x,
-                            const Tensor& lam, const Tensor& h0_in, const Tensor& flags, bool first_reset, double c, int64_t path) {
+                            const Tensor& lam, const Tensor& h0_in, const Tensor& flags, bool first_reset, double c, int64_t path,
+                            bool clear_backward = false) {
   ForwardResult r;
   c10::DeviceGuard guard(x_in.device());
   r.x = aligned(x_in);
@@ -240,8 +241,8 @@ ForwardResult rglru_forward(const Tensor& x_in, const Tensor& w_a, const Tensor&
     // parameter conversion, workspace clearing and the forward kernel: two launches, or one where the forward kernel
     // does all three (batch-rich shapes)
     check(rglru_hip_prepare_fwd(ptr(p.w_a), ptr(p.b_a), ptr(p.w_x), ptr(p.b_x), ptr(p.lam), static_cast<float>(c), p.vec,
-                                kept.image, ptr(r.x), fptr(r.h0), fl, ptr(r.y), fptr(r.h_last), kept.ws, B, T, W, nb, code,
-                                stream), "rglru_hip_prepare_fwd");
+                                kept.image, ptr(r.x), fptr(r.h0), fl, ptr(r.y), fptr(r.h_last), kept.ws, B, T, W, nb,
+                                code | (clear_backward ? RGLRU_BACKWARD_CLEAR : 0), stream), "rglru_hip_prepare_fwd");
   }
   return r;
 }
@@ -254,7 +255,7 @@ struct ParamGrads {
 // (w_a, b_a, w_x, b_x, lam).
 ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Tensor& h0, const Tensor& flags, bool first_reset,
                           const Tensor& held, const Tensor& dy_in, const Tensor& dh_last_in,
-                          const std::array<at::ScalarType, 5>& types, bool need_dh0) {
+                          const std::array<at::ScalarType, 5>& types, bool need_dh0, bool ws_clear) {
   ParamGrads g;
   c10::DeviceGuard guard(x.device());
   const int64_t B = x.size(0), T = x.size(1), W = x.size(2), bw = W / nb;
@@ -268,7 +269,7 @@ ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Te
   for (auto t : types)
     if (t != gt) gt = at::kFloat;
   if (!known(gt)) gt = at::kFloat;
-  const int gcode = code_of(gt);
+  const int gcode = code_of(gt) | (ws_clear ? RGLRU_BACKWARD_CLEAR : 0);
   g.dx = fresh_like(x);
   {
     const size_t gs = c10::elementSize(gt);
@@ -300,7 +301,7 @@ ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Te
   } else if (path == RGLRU_PATH_PRE) {
     check(rglru_hip_bwd_pre(ptr(x), more, kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx),
                             more + 2 * tensor_bytes, ptr(g.dw_a), ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam),
-                            fptr(g.dh0), B, T, W, nb, code, gcode, stream), "rglru_hip_bwd_pre");
+                            fptr(g.dh0), B, T, W, nb, code, code_of(gt), stream), "rglru_hip_bwd_pre");
   } else {
     check(rglru_hip_bwd(ptr(x), kept.image, fptr(h0), fl, ptr(dy), fptr(dh_last), kept.ws, sp, ptr(g.dx), more,
                         more + tensor_bytes, ptr(g.dw_a), ptr(g.dw_x), ptr(g.db_a), ptr(g.db_x), ptr(g.dlam), fptr(g.dh0), B,
@@ -347,7 +348,11 @@ struct RGLRU : torch::autograd::Function<RGLRU> {
                                double c, int64_t path) {
     Tensor h0 = opt(h0_), flags = opt(flags_);
     note_arguments(ctx, {true, true, true, true, true, true, h0.defined()});
-    ForwardResult r = rglru_forward(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_reset, c, path);
+    // the tiled kernels' records: the forward's clearing launch covers the backward's as well, for the first backward call over
+    // this forward (a repeated one clears them itself)
+    const bool clears = path != RGLRU_PATH_FAST_CHAIN && path != RGLRU_PATH_PRE;
+    ForwardResult r = rglru_forward(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_reset, c, path, clears);
+    if (clears) ctx->saved_data["clear"] = true;
     ctx->save_for_backward({r.x, r.h0, flags, r.kept, r.y});
     auto t = types_of(w_a, b_a, w_x, b_x, lam);
     pack(ctx, {first_reset, w_a.size(0), type_or_none(h0), (int64_t)t[0], (int64_t)t[1], (int64_t)t[2], (int64_t)t[3], (int64_t)t[4]});
@@ -362,7 +367,7 @@ struct RGLRU : torch::autograd::Function<RGLRU> {
       at::NoGradGuard no_grad;
       g = rglru_backward(saved[0], saved[4], m[1], saved[1], saved[2], m[0], saved[3], grads[0], grads[1],
                          {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)},
-                         Needs(ctx)(6));
+                         Needs(ctx)(6), ctx->saved_data.erase("clear") != 0);
       if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
     }
     return once({g.dx, g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam, g.dh0, Tensor(), Tensor(), Tensor(), Tensor()});
@@ -952,7 +957,7 @@ struct BlockForward : torch::autograd::Function<BlockForward> {
                                       stream_of(y)), "rglru_hip_gelu_gate_bwd");
       }
       g = rglru_backward(x_conv, y, m[1], h0, flags, m[0], kept, dy, grads[1],
-                         {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)}, need(12));
+                         {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)}, need(12), false);
       if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
       conv = conv_backward(u.contiguous(), state, taps, pos, g.dx, {m[8], m[9], m[10]}, need_u, need(2), need(3),
                            need(4), du_out, s[10]);
@@ -1558,9 +1563,12 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     }
     void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
     char *image = s[own], *ws = image + image_bytes;
+    const bool clears = kernel_path(B, T, W, nb, kType, true) != RGLRU_PATH_FAST_CHAIN;   // as in RGLRU
+    if (clears) ctx->saved_data["clear"] = true;
     check(rglru_hip_prepare_block_fwd(ptr(wa), ptr(ba), ptr(wi), ptr(bi), ptr(lam), static_cast<float>(c), RGLRU_BF16, image, up, W, vp, W,
                                       nullptr, ptr(cw), ptr(cb), K, nullptr, flags_ptr(flags, first_reset), s[0], s[1], s[2], nullptr,
-                                      nullptr, ws, ptr(wx), ptr(wy), ws + ws_bytes, stack ? W * D * 2 : 0, B, T, W, nb, RGLRU_BF16, stream),
+                                      nullptr, ws, ptr(wx), ptr(wy), ws + ws_bytes, stack ? W * D * 2 : 0, B, T, W, nb,
+                                      RGLRU_BF16 | (clears ? RGLRU_BACKWARD_CLEAR : 0), stream),
           "rglru_hip_prepare_block_fwd");
     Tensor out;
     if (!stack) {
@@ -1639,7 +1647,8 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
         sums[1] = {sums_o, ptr(g[BO]), int64_t(column_bytes_o / (4 * D)), D, RGLRU_F32};
       }
       check(rglru_hip_block_bwd(dgated, s[1], up, vp, s[0], image, ptr(cw), iptr(pos), static_cast<const int32_t*>(ptr(rows)),
-                                flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, sums_p, du, dv, 2 * W, B, T, W, nb, K, stream),
+                                flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, sums_p, du, dv, 2 * W,
+                                ctx->saved_data.erase("clear") != 0, B, T, W, nb, K, stream),
             "rglru_hip_block_bwd");
       // input projections
       const bool need_x = ctx->needs_input_grad(0);

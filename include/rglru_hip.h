@@ -51,7 +51,7 @@
 extern "C" {
 #endif
 
-#define RGLRU_ABI_VERSION 21
+#define RGLRU_ABI_VERSION 22
 
 enum { RGLRU_F32 = 0, RGLRU_BF16 = 1 };
 
@@ -69,6 +69,12 @@ enum {
  * passes when every row holds one document from its beginning (griffin/griffin.py:309-338 without cache).  The
  * kernels then need no per-token flags; rglru_hip_block_fwd also takes the rows' convolution history as empty. */
 #define RGLRU_FLAGS_FIRST_RESET ((const uint8_t*)(uintptr_t)1)
+/* Or'ed into the `dtype` of rglru_hip_prepare_fwd or rglru_hip_prepare_block_fwd: the launch that clears the forward's part of
+ * the workspace clears the backward's part as well.  Or'ed into the `grad_dtype` of rglru_hip_bwd, rglru_hip_bwd_full or
+ * rglru_hip_bwd_wide: the workspace comes from such a forward call that ran the tiled kernels (rglru_hip_backward_path is not
+ * RGLRU_PATH_FAST_CHAIN or RGLRU_PATH_PRE, or the block's forward) and no backward call has used it since; the backward call
+ * then needs no clearing launch of its own. */
+#define RGLRU_BACKWARD_CLEAR 0x100
 /* Bits 2-3 of a flag byte are read by rglru_hip_block_fwd only (convolution lags that reach in front of the
  * token's document); every other entry point ignores them. */
 #define RGLRU_FLAG_CONV_SHIFT 2
@@ -383,11 +389,11 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
  * them (contiguous); u: the first projection, contiguous; positions / rows as for rglru_hip_conv_rows_bwd.  Writes du and dv,
  * rows `d_stride` elements apart (W, or 2 W for the halves of one matrix).  gate_scratch: rglru_hip_bwd_scratch_bytes,
  * conv_scratch: rglru_hip_conv_scratch_bytes, sums_scratch: rglru_hip_block_sums_bytes; they hold the partial sums until
- * rglru_hip_block_finish.  bf16 storage, parameters and gradients; no carried state.  Only where rglru_hip_fast_path() is 1. */
+ * rglru_hip_block_finish.  ws_clear: as RGLRU_BACKWARD_CLEAR says.  bf16 storage, parameters and gradients; no carried state.  Only where rglru_hip_fast_path() is 1. */
 size_t rglru_hip_block_sums_bytes(int64_t B, int64_t T, int64_t W, int64_t nb);
 int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,
                         const void* taps, const int64_t* positions, const int32_t* rows, const uint8_t* flags, void* ws,
-                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride,
+                        void* gate_scratch, void* conv_scratch, void* sums_scratch, void* du, void* dv, int64_t d_stride, int ws_clear,
                         int64_t B, int64_t T, int64_t W, int64_t nb, int64_t K, void* stream);
 
 /* dst[i] = sum over s < sets of src[s * n + i] (src_dtype), fp32 accumulation in a fixed order; up to five in one launch, all
