@@ -275,6 +275,9 @@ RGLRU_DEVICE typename Io<IO>::Frag load_x_frag(const FusedArgs& p, const IO* xma
 // Every thread of the workgroup must call this (it contains barriers).
 // Narrow blocks are packed like those of the kernels with register-held weights (p.bpu > 1: the tile holds the unit's blocks side
 // by side, `first_k` the first of them, and the wave's block starts at column kb), so that all four waves have a slab.
+// Bound by the latency of its loads: all vectors of a slice are requested before the first is used (through a descriptor that
+// ends with the rows, so no load sits in a branch), and the weights of 32 input channels while the 32 before them are
+// multiplied.
 template <typename IO, int MT>
 RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long long row0, long long rows_total,
                                     int first_k, int kb, int slab, bool slab_ok, const IO* w_a_row, const IO* w_x_row,
@@ -285,6 +288,8 @@ RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long lon
   constexpr int TR = 32 * MT;
   constexpr int KG = Tr::KG, HW = Tr::HW, KCMAX = Tr::KCMAX;
   constexpr int LDSROW = KCMAX + HW;
+  constexpr int NV = TR * (KCMAX / HW) / kThreads;         // vectors a thread loads of a slice, at most
+  constexpr int GK = 32 / KG;                              // K groups of 32 input channels
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
@@ -293,25 +298,66 @@ RGLRU_DEVICE void gate_tile_generic(const FusedArgs& p, const IO* xmat, long lon
 #pragma unroll
   for (int e = 0; e < 16 * MT; ++e) xv[e] = 0.f;
 
-  for (int kc0 = 0; kc0 < p.bwp; kc0 += KCMAX) {           // one slice when blocks are packed: they are narrow
+  const unsigned row_bytes = (unsigned)p.W * (unsigned)sizeof(IO);
+  const long long left = rows_total - row0;
+  const rsrc_t rx = make_rsrc(xmat + row0 * p.W, left <= 0 ? 0u : (unsigned)(left < TR ? left : TR) * row_bytes);
+  Frag xin[NV];
+  auto request = [&](int kc0) {
     const int kcw = (p.bwp - kc0) < KCMAX ? (p.bwp - kc0) : KCMAX;
     const int vecs = kcw / HW, per_row = vecs * p.bpu;
-    for (int idx = tid; idx < TR * per_row; idx += kThreads) {
-      const int row = idx / per_row, at = idx - row * per_row, blk = at / vecs, cv = at - blk * vecs;
-      const bool there = first_k + blk < p.nb;
-      Frag v = load_x_frag<IO>(p, xmat, there ? row0 + row : rows_total, rows_total, first_k + blk, kc0 + cv * HW);
-      *reinterpret_cast<Frag*>(lds + row * LDSROW + blk * kcw + cv * HW) = v;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kThreads;
+      const int row = idx / per_row, at = idx - row * per_row, blk = at / vecs, col = kc0 + (at - blk * vecs) * HW;
+      const bool there = row < TR && first_k + blk < p.nb;
+      const unsigned off = (unsigned)row * row_bytes + (unsigned)((first_k + blk) * p.bw + col) * (unsigned)sizeof(IO);
+      if (p.aligned) {                                     // a vector lies wholly inside or outside its block
+        xin[i] = buf_load_frag<Frag>(rx, there && col < p.bw ? off : kOutOfRange);
+      } else {
+#pragma unroll
+        for (int e = 0; e < HW; ++e)
+          xin[i][e] = (IO)BufIo<IO>::load(rx, there && col + e < p.bw ? off + (unsigned)(e * sizeof(IO)) : kOutOfRange, 0u);
+      }
+    }
+  };
+  Frag fa[2][GK], fx[2][GK];
+  auto weights = [&](int set, int col) {                   // past the end: the last 32 channels again
+    const int c = col < p.bwp ? col : p.bwp - 32;
+#pragma unroll
+    for (int g = 0; g < GK; ++g) {
+      fa[set][g] = *reinterpret_cast<const Frag*>(w_a_row + c + g * KG);
+      fx[set][g] = *reinterpret_cast<const Frag*>(w_x_row + c + g * KG);
+    }
+  };
+  weights(0, 0);
+  for (int kc0 = 0; kc0 < p.bwp; kc0 += KCMAX) {           // one slice when blocks are packed: they are narrow
+    const int kcw = (p.bwp - kc0) < KCMAX ? (p.bwp - kc0) : KCMAX;
+    const int per_row = kcw / HW * p.bpu;
+    request(kc0);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kThreads;
+      const int row = idx / per_row, at = idx - row * per_row;   // the packed blocks' columns lie side by side
+      if (row < TR) *reinterpret_cast<Frag*>(lds + row * LDSROW + at * HW) = xin[i];
     }
     __syncthreads();
     if (slab_ok) {
-      for (int kk = 0; kk < kcw; kk += KG) {
-        Frag fa = *reinterpret_cast<const Frag*>(w_a_row + kc0 + kk);
-        Frag fx = *reinterpret_cast<const Frag*>(w_x_row + kc0 + kk);
+      auto multiply = [&](int set, int kk) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          Frag xa = *reinterpret_cast<const Frag*>(lds + tile_row<MT>(mt, r) * LDSROW + kb + kk + hf * HW);
-          Tr::mma(ua[mt], xa, fa);
-          Tr::mma(ux[mt], xa, fx);
+        for (int g = 0; g < GK; ++g)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            const Frag xa = *reinterpret_cast<const Frag*>(lds + tile_row<MT>(mt, r) * LDSROW + kb + kk + g * KG + hf * HW);
+            Tr::mma(ua[mt], xa, fa[set][g]);
+            Tr::mma(ux[mt], xa, fx[set][g]);
+          }
+      };
+      for (int kk = 0; kk < kcw; kk += 64) {               // a slice but the last is a multiple of 64 wide: set 0 starts each
+        weights(1, kc0 + kk + 32);
+        multiply(0, kk);
+        if (kk + 32 < kcw) {
+          weights(0, kc0 + kk + 64);
+          multiply(1, kk + 32);
         }
       }
       const int own = slab * 32 - kc0;                    // first column of this wave's slab in the slice
@@ -378,11 +424,6 @@ RGLRU_DEVICE void gate_mfma_held(const IO* lds, const HeldWeights<IO, NKG, LDSG>
   for (int e = 0; e < 16; ++e) xv[e] = (float)lds[(hf * 16 * MT + 16 * mt + e) * LDSROW + kb + slab * 32 + r];
 }
 
-RGLRU_DEVICE unsigned token_flag(const FusedArgs& p, long long token_row, bool inside) {
-  if (!inside) return RGLRU_FLAG_INACTIVE;
-  return p.flags ? (unsigned)p.flags[token_row] & 3u : 0u;   // bits 2-3 belong to the block forward's convolution
-}
-
 // Flags of a lane's run of 16 consecutive tokens, two bits per token (token e at bits 2e, 2e + 1);
 // tokens past the end of the sequence read as inactive.  When the sequence length is a multiple of
 // 16 and the flag array is 16-byte aligned (flags_vec), a run is wholly inside or outside the
@@ -401,9 +442,17 @@ RGLRU_DEVICE unsigned flag_run(const FusedArgs& p, long long token_row, int t_fi
     const uint4 w = *reinterpret_cast<const uint4*>(p.flags + token_row);
     return pack_flag_bytes(w.x) | (pack_flag_bytes(w.y) << 8) | (pack_flag_bytes(w.z) << 16) | (pack_flag_bytes(w.w) << 24) | first;
   }
-  unsigned bits = first;
+  // any length and alignment: sixteen byte loads in flight together, those past the end dropped by their offset
+  const int n = p.T - t_first;
+  unsigned bits = first | (n >= 16 ? 0u : n <= 0 ? 0xAAAAAAAAu : 0xAAAAAAAAu << (2 * n));
+  if (p.flags) {
+    const rsrc_t rf = make_rsrc(p.flags, (unsigned)p.B * (unsigned)p.T);
+    unsigned f[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) bits |= token_flag(p, token_row + e, t_first + e < p.T) << (2 * e);
+    for (int e = 0; e < 16; ++e) f[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b8(rf, e < n ? (unsigned)token_row + (unsigned)e : kOutOfRange, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) bits |= (f[e] & 3u) << (2 * e);   // bits 2-3 belong to the block forward's convolution
+  }
   return bits;
 }
 

@@ -30,8 +30,8 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_kernel(FusedArgs p) {
   const float cs = w.ch_ok ? p.cs[w.kp] : 0.f;
   const IO* x = (const IO*)p.x;
   const IO* dy = (const IO*)p.dy;
-  IO* dx = (IO*)p.dx; IO* dua = (IO*)p.du_a; IO* dux = (IO*)p.du_x;
   const long long W = p.W;
+  const unsigned row_bytes = (unsigned)p.W * (unsigned)sizeof(IO);
   float sum_ba = 0.f, sum_bx = 0.f, sum_l = 0.f;
   const Queue q = make_queue(p, w.unit, w.wg_in_unit, p.nC);
 
@@ -44,38 +44,41 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_kernel(FusedArgs p) {
     const int c = p.nC - 1 - cr;
     const int t0 = c * TR;
 
+    // requested in front of the gate products, which hide their latency; rows past the end read as zero
+    const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+    const long long first = ((long long)b * p.T + t0) * W;
+    const unsigned voff = w.ch_ok ? (unsigned)(hf * EL) * row_bytes + (unsigned)w.ch * (unsigned)sizeof(IO) : kOutOfRange;
+    const rsrc_t rdy = make_rsrc(dy + first, (unsigned)rows * row_bytes);
+    float gy[EL];
+#pragma unroll
+    for (int e = 0; e < EL; ++e) gy[e] = BufIo<IO>::load(rdy, voff == kOutOfRange ? kOutOfRange : voff + (unsigned)e * row_bytes, 0u);
+    const unsigned flbits = flag_run(p, (long long)b * p.T + t0 + hf * EL, t0 + hf * EL);   // two flag bits per local step
+    float h_start = 0.f;                                 // from the checkpoint in front of the lane's 16 tokens
+    if (w.ch_ok) {
+      if (c == 0 && hf == 0) h_start = p.h0 ? p.h0[(long long)b * W + w.ch] : 0.f;
+      else h_start = p.ckpt[((long long)b * p.ckpt_nC + (2 * c - 1 + hf)) * W + w.ch];
+    }
     f32x16 ua[MT], ux[MT];
     float xv[EL];
     gate_tile_generic<IO, MT>(p, x + (long long)b * p.T * W, t0, p.T, p.bpu > 1 ? w.unit * p.bpu : w.k, w.kb, w.slab, w.slab_ok, w_a_row, w_x_row,
                               0.0f, 0.0f, lds, ua, ux, xv);
     if (!w.slab_ok) continue;
 
-    const long long trow = (long long)b * p.T + t0 + hf * EL;
     // kept per local step: both gates, the decay, the input scale and dy; z = g i x is recomputed
     // where it is needed (two workgroups per compute unit need the registers)
-    float r[EL], gi[EL], a[EL], g[EL], gy[EL];
-    unsigned flbits = 0u;                                // two flag bits per local step
+    float r[EL], gi[EL], a[EL], g[EL];
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
-      const bool in = t0 + hf * EL + e < p.T;
-      const unsigned fl = token_flag(p, trow + e, in) | ((p.first_reset && t0 + hf * EL + e == 0) ? RGLRU_FLAG_RESET : 0u);
-      flbits |= fl << (2 * e);
-      GateOut go = gate_forward<Precise<IO>::value, true>(ua[0][e], ux[0][e], xv[e], sp, fl, nba, nbx);
+      const GateOut go = gate_forward_run<Precise<IO>::value>(ua[0][e], ux[0][e], xv[e], sp, flbits, e, nba, nbx);
       r[e] = go.r; gi[e] = go.i; a[e] = go.a; g[e] = go.g;
-      gy[e] = (in && w.ch_ok) ? (float)dy[(trow + e) * W + w.ch] : 0.f;
     }
-    // forward recomputation of h_{t-1} from the checkpoint in front of the lane's 16 tokens
+    // forward recomputation of h_{t-1}
     float A = 1.f;
 #pragma unroll
     for (int e = 0; e < EL; ++e) A *= a[e];
     const float A_o = xhalf(A, hf);
     const float A_lo = hf ? A_o : A;
     const float A_hi = hf ? A : A_o;
-    float h_start = 0.f;
-    if (w.ch_ok) {
-      if (c == 0 && hf == 0) h_start = p.h0 ? p.h0[(long long)b * W + w.ch] : 0.f;
-      else h_start = p.ckpt[((long long)b * p.ckpt_nC + (2 * c - 1 + hf)) * W + w.ch];
-    }
     float h = h_start;
     float hp[EL];
 #pragma unroll
@@ -104,6 +107,9 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_kernel(FusedArgs p) {
     if (w.ch_ok && hf == 0) carry_publish(chain, c, 0.f, d_out, true);
     if (c == 0 && p.dh0 && w.ch_ok && hf == 0) p.dh0[(long long)b * W + w.ch] = d_out;
 
+    const rsrc_t rdx = make_rsrc((const IO*)p.dx + first, (unsigned)rows * row_bytes);
+    const rsrc_t rdua = make_rsrc((const IO*)p.du_a + first, (unsigned)rows * row_bytes);
+    const rsrc_t rdux = make_rsrc((const IO*)p.du_x + first, (unsigned)rows * row_bytes);
     carry = hf ? d_in : fmaf(A_hi, d_in, D_hi);
 #pragma unroll
     for (int e = EL - 1; e >= 0; --e) {
@@ -126,10 +132,10 @@ __global__ __launch_bounds__(kThreads, 2) void bwd_kernel(FusedArgs p) {
       if (ina) { dl = 0.f; va = 0.f; vx = 0.f; dxd = 0.f; }
       sum_l = fmaf(dl, r[e], sum_l);
       sum_ba += va; sum_bx += vx;
-      if (w.ch_ok && (t0 + hf * EL + e < p.T)) {
-        const long long at = (trow + e) * W + w.ch;
-        dx[at] = (IO)dxd; dua[at] = (IO)va; dux[at] = (IO)vx;
-      }
+      const unsigned at = voff == kOutOfRange ? kOutOfRange : voff + (unsigned)e * row_bytes;
+      BufIo<IO>::store((IO)dxd, rdx, at, 0u);
+      BufIo<IO>::store((IO)va, rdua, at, 0u);
+      BufIo<IO>::store((IO)vx, rdux, at, 0u);
     }
   }
   // per-workgroup partial sums (every slot is written, so the buffer needs no clearing)
