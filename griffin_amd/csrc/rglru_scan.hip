@@ -77,6 +77,7 @@ __global__ __launch_bounds__(kThreads) void scan_fwd_kernel(ScanArgs p) {
   unsigned tk = 0;
   if (lane == 0) tk = atomicAdd(p.ticket + chain_id, 1u);
   tk = __builtin_amdgcn_readfirstlane(tk);
+  if (tk >= (unsigned)p.nC) return;                        // only where the workspace was not clear: there is no such chunk
   const int c = (int)tk;
   const int b = chain_id / p.groups, grp = chain_id - b * p.groups;
   const int ch = grp * 64 + lane;
@@ -126,6 +127,7 @@ __global__ __launch_bounds__(kThreads) void scan_bwd_kernel(ScanArgs p) {
   unsigned tk = 0;
   if (lane == 0) tk = atomicAdd(p.ticket + chain_id, 1u);
   tk = __builtin_amdgcn_readfirstlane(tk);
+  if (tk >= (unsigned)p.nC) return;                  // as in the forward kernel
   const int c = p.nC - 1 - (int)tk;                  // the chain runs from the last chunk to the first
   const int b = chain_id / p.groups, grp = chain_id - b * p.groups;
   const int ch = grp * 64 + lane;
@@ -274,6 +276,7 @@ __global__ __launch_bounds__(kVecThreads, 2) void scan_vec_kernel(ScanArgs p) {
   const int chain_id = (int)(blockIdx.x % chains);
   if (threadIdx.x == 0) s_ticket = atomicAdd(p.ticket + chain_id, 1u);
   __syncthreads();
+  if (s_ticket >= (unsigned)nR) return;                  // only where the workspace was not clear: there is no such run
   const int tk = (int)s_ticket;
   const int c = FORWARD ? tk : nR - 1 - tk;              // chain order: first run first / last run first
   const int b = chain_id / groups4, grp = chain_id - b * groups4;

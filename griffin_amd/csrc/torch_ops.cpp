@@ -13,6 +13,7 @@
 #include <c10/core/Event.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
@@ -325,6 +326,29 @@ std::vector<int64_t> unpack(AutogradContext* ctx) { return ctx->saved_data["meta
 at::ScalarType type_at(const std::vector<int64_t>& m, size_t i) { return static_cast<at::ScalarType>(m[i]); }
 constexpr int64_t kNone = -1;
 
+// The capture that the current stream of t's device records into (0: none), or kNone where the runtime does not say.
+int64_t capture_of(const Tensor& t) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream_of(t)), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();
+    return kNone;
+  }
+  return status == hipStreamCaptureStatusNone ? 0 : status == hipStreamCaptureStatusActive ? static_cast<int64_t>(id) + 1 : kNone;
+}
+
+// The forward's clearing launch covers what the first backward pass over it needs clear (a repeated pass clears that itself).
+// That holds where both run, or both are recorded, together: a graph that holds the backward alone is replayed without
+// the forward, and one that holds the forward alone does its clearing at another time than the backward.
+void note_cleared(AutogradContext* ctx, const Tensor& t) { ctx->saved_data["clear"] = capture_of(t); }
+bool take_cleared(AutogradContext* ctx, const Tensor& t) {
+  auto noted = ctx->saved_data.find("clear");
+  if (noted == ctx->saved_data.end()) return false;
+  const int64_t capture = noted->second.toInt();
+  ctx->saved_data.erase(noted);
+  return capture != kNone && capture == capture_of(t);
+}
+
 // Whether the gradient of tensor argument i of a Function's forward is asked for.  The node has an edge only for the
 // arguments that were there, so an optional argument in front shifts the ones behind it: forward notes which were.
 void note_arguments(AutogradContext* ctx, std::initializer_list<bool> present) {
@@ -348,11 +372,9 @@ struct RGLRU : torch::autograd::Function<RGLRU> {
                                double c, int64_t path) {
     Tensor h0 = opt(h0_), flags = opt(flags_);
     note_arguments(ctx, {true, true, true, true, true, true, h0.defined()});
-    // the tiled kernels' records: the forward's clearing launch covers the backward's as well, for the first backward call over
-    // this forward (a repeated one clears them itself)
-    const bool clears = path != RGLRU_PATH_FAST_CHAIN && path != RGLRU_PATH_PRE;
+    const bool clears = path != RGLRU_PATH_FAST_CHAIN && path != RGLRU_PATH_PRE;   // the kernels that use records
     ForwardResult r = rglru_forward(x, w_a, b_a, w_x, b_x, lam, h0, flags, first_reset, c, path, clears);
-    if (clears) ctx->saved_data["clear"] = true;
+    if (clears) note_cleared(ctx, r.x);
     ctx->save_for_backward({r.x, r.h0, flags, r.kept, r.y});
     auto t = types_of(w_a, b_a, w_x, b_x, lam);
     pack(ctx, {first_reset, w_a.size(0), type_or_none(h0), (int64_t)t[0], (int64_t)t[1], (int64_t)t[2], (int64_t)t[3], (int64_t)t[4]});
@@ -367,7 +389,7 @@ struct RGLRU : torch::autograd::Function<RGLRU> {
       at::NoGradGuard no_grad;
       g = rglru_backward(saved[0], saved[4], m[1], saved[1], saved[2], m[0], saved[3], grads[0], grads[1],
                          {type_at(m, 3), type_at(m, 4), type_at(m, 5), type_at(m, 6), type_at(m, 7)},
-                         Needs(ctx)(6), ctx->saved_data.erase("clear") != 0);
+                         Needs(ctx)(6), take_cleared(ctx, saved[0]));
       if (g.dh0.defined() && type_at(m, 2) != at::kFloat) g.dh0 = g.dh0.to(type_at(m, 2));
     }
     return once({g.dx, g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam, g.dh0, Tensor(), Tensor(), Tensor(), Tensor()});
@@ -527,9 +549,7 @@ struct Scan : torch::autograd::Function<Scan> {
     Tensor a = a_in.contiguous(), h0 = h0_in.contiguous(), ws;
     Tensor out = scan_forward(a, z.contiguous(), h0, &ws);
     ctx->save_for_backward({a, h0, out});
-    // the forward call has cleared the backward part of the workspace too: the first backward call over this forward
-    // finds it clear (a repeated one clears its part itself)
-    if (ws.defined()) ctx->saved_data["ws"] = ws;
+    if (ws.defined()) ctx->saved_data["ws"] = ws, note_cleared(ctx, a);
     return out;
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
@@ -545,10 +565,9 @@ struct Scan : torch::autograd::Function<Scan> {
       if (a.numel() == 0) {
         dh0.zero_();
       } else {
-        auto held = ctx->saved_data.find("ws");
-        const bool clear = held != ctx->saved_data.end();
-        Tensor ws = clear ? held->second.toTensor() : bytes(rglru_hip_scan_workspace_bytes(B, T, W), a);
-        if (clear) ctx->saved_data.erase(held);
+        const bool clear = take_cleared(ctx, a);
+        Tensor ws = clear ? ctx->saved_data["ws"].toTensor() : bytes(rglru_hip_scan_workspace_bytes(B, T, W), a);
+        ctx->saved_data.erase("ws");
         check(rglru_hip_scan_bwd(fptr(a), fptr(h0), fptr(out), fptr(dh), fptr(da), fptr(dz), fptr(dh0), ptr(ws), clear ? 1 : 0, B,
                                  T, W, stream_of(a)), "rglru_hip_scan_bwd");
       }
@@ -1564,7 +1583,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
     char *image = s[own], *ws = image + image_bytes;
     const bool clears = kernel_path(B, T, W, nb, kType, true) != RGLRU_PATH_FAST_CHAIN;   // as in RGLRU
-    if (clears) ctx->saved_data["clear"] = true;
+    if (clears) note_cleared(ctx, x);
     check(rglru_hip_prepare_block_fwd(ptr(wa), ptr(ba), ptr(wi), ptr(bi), ptr(lam), static_cast<float>(c), RGLRU_BF16, image, up, W, vp, W,
                                       nullptr, ptr(cw), ptr(cb), K, nullptr, flags_ptr(flags, first_reset), s[0], s[1], s[2], nullptr,
                                       nullptr, ws, ptr(wx), ptr(wy), ws + ws_bytes, stack ? W * D * 2 : 0, B, T, W, nb,
@@ -1648,7 +1667,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       }
       check(rglru_hip_block_bwd(dgated, s[1], up, vp, s[0], image, ptr(cw), iptr(pos), static_cast<const int32_t*>(ptr(rows)),
                                 flags_ptr(flags, first_reset), ws, gate_scratch, conv_scratch, sums_p, du, dv, 2 * W,
-                                ctx->saved_data.erase("clear") != 0, B, T, W, nb, K, stream),
+                                take_cleared(ctx, x), B, T, W, nb, K, stream),
             "rglru_hip_block_bwd");
       // input projections
       const bool need_x = ctx->needs_input_grad(0);

@@ -1,6 +1,8 @@
 """GPU parity tests: the HIP kernels, called through the C ABI, against the CPU oracle."""
 
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -869,6 +871,15 @@ def test_hip_graph_replays_match_eager_results():
             # the carry composition order of a look-back depends on timing: equal up to rounding
             assert rel_err(got.float(), want.float()) < 1e-2, (replay, name)
         assert rel_err(captured[0].float(), eager[0].float()) < 1e-6
+
+
+def test_captured_backward_repeats():
+    """A HIP graph that holds a backward pass without its forward clears what that pass needs clear: every replay gives the
+    gradients of its upstream gradient (the forward's clearing covers a backward pass of the same capture only)."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-m", "tests.capture_child"], cwd=root, capture_output=True, text=True, timeout=100)
+    _say(run.stdout + run.stderr[-2000:])
+    assert run.returncode == 0
 
 
 # ------------------------------------------------------------------ gate blocks that do not fill their 32-channel slabs
