@@ -14,6 +14,7 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
@@ -64,9 +65,24 @@ int code_of(at::ScalarType t) {
   return t == at::kBFloat16 ? RGLRU_BF16 : RGLRU_F32;
 }
 
+// Forward-mode tangents: none of the operators carries one on, so a dual tensor is refused (also where no gradient is asked
+// for and no autograd function would notice it).  A tangent lives only inside an entered level, which is one question.
+bool dual_level() { return torch::autograd::ForwardADLevel::try_get_by_idx(0) != nullptr; }
+bool is_dual(const Tensor& t) { return t.defined() && t._fw_grad(0).defined(); }
+void refuse_tangent(const char* name, const Tensor& t) {
+  TORCH_CHECK_NOT_IMPLEMENTED(!is_dual(t), name, " has no forward-mode derivative; it takes no dual tensors");
+}
+template <typename Tensors>
+void refuse_tangents(const char* name, const Tensors& tensors) {
+  if (!dual_level()) return;
+  for (const Tensor& t : tensors) refuse_tangent(name, t);
+}
+
 void require_gpu(const char* name, std::initializer_list<const Tensor*> tensors) {
   for (const Tensor* t : tensors)
     TORCH_CHECK(!t->defined() || t->is_cuda(), name, " requires CUDA/HIP tensors, got a ", t->device().type(), " tensor");
+  if (!dual_level()) return;
+  for (const Tensor* t : tensors) refuse_tangent(name, *t);
 }
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -178,6 +194,7 @@ Tensor prepare(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Te
                at::ScalarType dtype) {
   const int64_t nb = w_a.size(0), W = nb * w_a.size(1);
   const int code = code_of(dtype);
+  refuse_tangents("hip RG-LRU", std::array<Tensor, 5>{w_a, b_a, w_x, b_x, lam});
   c10::DeviceGuard guard(w_a.device());
   at::NoGradGuard no_grad;
   Operands p(w_a, b_a, w_x, b_x, lam, dtype);
@@ -414,6 +431,7 @@ std::tuple<Tensor, Tensor> rglru(const Tensor& x, const Tensor& w_a, const Tenso
 // Storage addresses and version counters of some tensors, one after the other: unchanged while nobody replaced one or
 // wrote to it through PyTorch.
 py::tuple fingerprint(const std::vector<Tensor>& tensors) {
+  refuse_tangents("the recurrent block", tensors);            // what is kept under a fingerprint carries none
   py::tuple out(2 * tensors.size());
   for (size_t i = 0; i < tensors.size(); ++i) {
     out[2 * i] = reinterpret_cast<uintptr_t>(tensors[i].data_ptr());
@@ -436,7 +454,7 @@ struct Stamp {
   }
   template <typename Tensors>
   bool holds(const Tensors& tensors, size_t n, double decay, at::ScalarType type) const {
-    if (n != seen.size() || c != decay || dtype != type) return false;
+    if (n != seen.size() || c != decay || dtype != type || dual_level()) return false;   // a dual tensor shares its primal's memory
     for (size_t i = 0; i < n; ++i)
       if (tensors[i].data_ptr() != seen[i].first || static_cast<int64_t>(tensors[i]._version()) != seen[i].second) return false;
     return true;
@@ -517,8 +535,8 @@ Tensor rglru_steps(const Tensor& xs_in, const Tensor& image, int64_t blocks, con
 // One token per row of the bare layer: y and the new state, the old one untouched (x [B, 1, W]).
 std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const MaybeTensor& state,
                                              const MaybeTensor& flags_) {
-  Tensor flags = opt(flags_);
-  require_gpu("hip RG-LRU step", {&x_in, &flags});
+  Tensor flags = opt(flags_), carried = opt(state);
+  require_gpu("hip RG-LRU step", {&x_in, &flags, &carried});
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(x_in.device());
   const int64_t B = x_in.size(0), W = x_in.size(2);
@@ -1064,6 +1082,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
   Tensor b_x = opt(b_x_), b_y = opt(b_y_), conv_b = opt(conv_b_), b_o = opt(b_o_), conv_state = opt(conv_state_),
          prev_pos = opt(prev_pos_), segment_pos = opt(segment_pos_), active = opt(active_), rnn_state = opt(rnn_state_);
   const auto dtype = x_in.scalar_type();
+  refuse_tangents("hip_block_step", std::initializer_list<Tensor>{x_in, w_x, b_x, w_y, b_y, conv_w, conv_b, w_o, b_o, conv_state, rnn_state});
   const int64_t B = x_in.size(0), D = x_in.size(2), W = w_x.size(0), K = conv_w.size(2);
   if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || w_o.size(0) != D || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state})
@@ -1523,6 +1542,7 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
 
 // The values alone, without a graph.
 std::tuple<Tensor, Tensor> linear_pair_values(const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2, const MaybeTensor& b2) {
+  refuse_tangents("hip_linear_pair", std::initializer_list<Tensor>{x, w1, opt(b1), w2, opt(b2)});
   at::NoGradGuard no_grad;
   return LinearPair::values(x, w1, opt(b1), w2, opt(b2));
 }
@@ -1707,6 +1727,8 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
                         const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
   typedef BlockTrain N;
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
+  refuse_tangents("the recurrent block", p);
+  refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(u), opt(v)});
   for (const Tensor& t : p)
     if (t.scalar_type() != N::kType || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
   // p: the node's tensors behind x
@@ -1735,6 +1757,8 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
   typedef BlockTrain N;
   const auto dtype = x.scalar_type();
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
+  refuse_tangents("the recurrent block", p);
+  refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(conv_state_), opt(rnn_state_), opt(u_), opt(v_)});
   for (const Tensor& t : p)
     if (t.scalar_type() != dtype || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
   const Tensor &wx = p[N::WX - 1], &bx = p[N::BX - 1], &wy = p[N::WY - 1], &by = p[N::BY - 1], &cw = p[N::CW - 1], &cb = p[N::CB - 1],

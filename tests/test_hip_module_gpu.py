@@ -899,3 +899,57 @@ def test_leaves_held_between_steps_follow_the_parameters():
     assert all(torch.allclose(a, b, rtol=1e-5, atol=1e-6) for a, b in zip(grads(wider), grads(layer)))
     half = layer.to(torch.bfloat16)
     assert all(g.dtype == torch.bfloat16 and torch.isfinite(g.float()).all() for g in grads(half))
+
+
+@pytest.mark.parametrize("grad", [False, True], ids=["no_grad", "frozen"])
+def test_forward_mode_is_refused(grad):
+    """No operator has a forward-mode derivative: a dual tensor is an error on every path, also where no reverse-mode
+    gradient is asked for (parameters frozen, or under no_grad) and dropping the tangent would read as a zero derivative."""
+    import torch.autograd.forward_ad as fwd
+
+    from griffin_amd import RG_LRU, RMSNorm, RecurrentBlock, hip_block_ops, hip_rglru, hip_rglru_scan
+
+    torch.manual_seed(0)
+    bf = torch.bfloat16
+
+    def rand(*shape, dtype=torch.float32):
+        return torch.randn(*shape, device="cuda", dtype=dtype)
+
+    layer, norm, block = RG_LRU(64, gate_blocks=2), RMSNorm(64), RecurrentBlock(64, 128, gate_blocks=2)
+    for m in (layer, norm, block):
+        m.cuda().to(bf).requires_grad_(False)
+    x, token, state = rand(2, 9, 64, dtype=bf), rand(2, 1, 64, dtype=bf), rand(2, 64)
+    mask = torch.ones(2, 9, dtype=torch.bool, device="cuda")
+    mask[1, 5:] = False
+    with torch.no_grad():
+        for m in (layer, block):
+            m(x), m(token)                                   # images and default positions are there, as in a running program
+    w, b = rand(32, 64, dtype=bf), rand(32, dtype=bf)
+    a, z, h = torch.rand(2, 9, 64, device="cuda"), rand(2, 9, 64), rand(2, 64)
+    calls = {
+        "rglru": (x, lambda t: hip_rglru(t, *layer._gate_parameters(), 8.0)),
+        "rglru Lambda": (layer.Lambda.detach(), lambda t: hip_rglru(x, *layer._gate_parameters()[:4], t, 8.0)),
+        "scan": (a, lambda t: hip_rglru_scan(t, z, h)),
+        "scan state": (h, lambda t: hip_rglru_scan(a, z, t)),
+        "norm": (x, lambda t: hip_block_ops.hip_rmsnorm(t, norm.g)),
+        "norm scale": (norm.g.detach(), lambda t: hip_block_ops.hip_rmsnorm(x, t)),
+        "linear": (w, lambda t: hip_block_ops.hip_linear(x, t, b)),
+        "linear pair": (x, lambda t: hip_block_ops.hip_linear_pair(t, w, b, w, b)),
+        "gate": (x, lambda t: hip_block_ops.hip_gelu_gate(t, x)),
+        "layer": (x, layer),
+        "layer decode": (token, layer),
+        "layer decode state": (state, lambda t: layer(token, t)),
+        "RMSNorm": (x, norm),
+        "block": (x, block),
+        "block padded": (x, lambda t: block(t, active_mask=mask)),
+        "block decode": (token, block),
+        "block weight": (block.linear_out.weight.detach(), lambda t: torch.func.functional_call(block, {"linear_out.weight": t}, (x,))),
+        "block decode weight": (block.rg_lru.Lambda.detach(), lambda t: torch.func.functional_call(block, {"rg_lru.Lambda": t}, (token,))),
+    }
+    with torch.set_grad_enabled(grad), fwd.dual_level():
+        for name, (primal, call) in calls.items():
+            _say("forward mode", name)
+            with pytest.raises(NotImplementedError):
+                call(fwd.make_dual(primal, torch.ones_like(primal)))
+    with torch.no_grad():
+        assert all(torch.isfinite(m(x).float()).all() for m in (layer, norm, block))
