@@ -617,6 +617,9 @@ struct TokenFacts {
     require_gpu("token facts", {&active_in});
     at::NoGradGuard no_grad;
     c10::DeviceGuard guard(active_in.device());
+    // before anything is launched: a graph that held the kernel would write to the host memory on every replay
+    TORCH_CHECK(c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None,
+                "an activity mask is answered on the host, which a stream that is being captured does not allow");
     Tensor active = active_in.contiguous();
     TORCH_CHECK_VALUE(active.dim() == 2 && active.element_size() == 1, "active_mask must be a [batch, sequence] mask");
     const int64_t B = active.size(0), T = active.size(1);
@@ -637,10 +640,23 @@ struct TokenFacts {
                                 static_cast<int64_t*>(conv_positions.data_ptr()), static_cast<int32_t*>(rows.data_ptr()),
                                 static_cast<int64_t*>(last_position.data_ptr()), static_cast<uint32_t*>(answer_.data_ptr()), B, T,
                                 stream_of(active)), "rglru_hip_token_facts");
-    event_.record(c10::Stream(c10::Stream::UNSAFE, active.device(), c10::hip::getCurrentHIPStream(active.device().index()).id()));
+    try {
+      event_.record(c10::Stream(c10::Stream::UNSAFE, active.device(), c10::hip::getCurrentHIPStream(active.device().index()).id()));
+    } catch (...) {
+      abandon();
+      throw;
+    }
   }
   TokenFacts(const TokenFacts&) = delete;
-  ~TokenFacts() { wait(); }                  // the kernel writes into memory that this object gives back
+  // the kernel writes into memory that this object gives back, so its end is waited for; where that fails (an error is
+  // pending on the device, and resolve() has reported it) the memory is not given back
+  ~TokenFacts() {
+    try {
+      wait();
+    } catch (...) {
+      abandon();
+    }
+  }
   std::tuple<bool, bool> resolve() {
     {
       py::gil_scoped_release no_gil;
@@ -657,6 +673,7 @@ struct TokenFacts {
     if (!done_) event_.synchronize();
     done_ = true;
   }
+  void abandon() { new Tensor(std::move(answer_)); }
   Tensor answer_;
   c10::Event event_;
   bool done_ = false;

@@ -1,4 +1,4 @@
-"""Graph captures for test_captured_backward_repeats, in a process of their own: a program captures on its own streams, and
+"""Graph captures for test_captured_backward_repeats and test_masked_block_under_capture_is_an_error, in a process of their own: a program captures on its own streams, and
 what a capture leaves behind stays out of the other tests.  Prints a line for each case, ends with status 1 after a mismatch."""
 
 import sys
@@ -76,11 +76,42 @@ def captured_backward(make, dtype, shape, tol):
     return worst, worst < tol
 
 
-if __name__ == "__main__":
+def captured_mask():
+    """Which kernels a masked block runs is decided on the host: under capture that is a RuntimeError before anything is
+    launched, the process goes on, and the same call outside the capture is what it was."""
+    from griffin_amd import RecurrentBlock
+
+    ok = True
+    for dtype in (torch.bfloat16, torch.float32):
+        torch.manual_seed(5)
+        block = RecurrentBlock(64, 128, gate_blocks=2, scan_mode="hip").to(dtype).cuda()
+        x = torch.randn(2, 40, 64).to(dtype).cuda()
+        mask = torch.ones(2, 40, dtype=torch.bool, device="cuda")
+        mask[1, 17:] = False
+        for train in (False, True):
+            with torch.set_grad_enabled(train):
+                want = block(x, active_mask=mask).detach()
+                torch.cuda.synchronize()
+                try:
+                    with torch.cuda.graph(torch.cuda.CUDAGraph()):
+                        block(x, active_mask=mask)
+                    ok = False
+                except RuntimeError as error:
+                    print("  refused:", str(error).splitlines()[0], flush=True)
+                torch.cuda.synchronize()
+                ok &= rel_err(block(x, active_mask=mask).float(), want.float()) < 1e-2
+    return ok
+
+
+def captured_backwards():
     ok = True
     for name, make, dtype, shape, tol in CASES:
         print("captured backward", name, shape, flush=True)
         worst, good = captured_backward(make, dtype, shape, tol)
         print("  worst", "%.2e" % worst, flush=True)
         ok &= good
-    sys.exit(0 if ok else 1)
+    return ok
+
+
+if __name__ == "__main__":
+    sys.exit(0 if {"backward": captured_backwards, "mask": captured_mask}[sys.argv[1]]() else 1)

@@ -873,13 +873,22 @@ def test_hip_graph_replays_match_eager_results():
         assert rel_err(captured[0].float(), eager[0].float()) < 1e-6
 
 
+def _captures(what):
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-m", "tests.capture_child", what], cwd=root, capture_output=True, text=True, timeout=100)
+    _say(run.stdout + run.stderr[-2000:])
+    return run.returncode
+
+
 def test_captured_backward_repeats():
     """A HIP graph that holds a backward pass without its forward clears what that pass needs clear: every replay gives the
     gradients of its upstream gradient (the forward's clearing covers a backward pass of the same capture only)."""
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    run = subprocess.run([sys.executable, "-m", "tests.capture_child"], cwd=root, capture_output=True, text=True, timeout=100)
-    _say(run.stdout + run.stderr[-2000:])
-    assert run.returncode == 0
+    assert _captures("backward") == 0
+
+
+def test_masked_block_under_capture_is_an_error():
+    """... and not the end of the process."""
+    assert _captures("mask") == 0
 
 
 # ------------------------------------------------------------------ gate blocks that do not fill their 32-channel slabs
