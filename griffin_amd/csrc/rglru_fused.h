@@ -164,7 +164,7 @@ struct FusedArgs {
   int bpu;                                                // gate blocks per unit (packed narrow blocks), else 1
   long long rows_total;                                   // B * T, the row count of one block of `pre`
   int nC, nCf, ckpt_nC, wg_per_unit, aligned, full_slabs, queues, flags_vec;
-  int dw_bf16;                                            // fast backward: per-workgroup weight-gradient sums stored as bf16
+  int dw_bf16;                                            // fast backward: per-workgroup weight-gradient sums stored as bf16 (unpadded blocks)
   int xcd_map;                                            // wide blocks: the workgroups that share a block's x tiles sit on one XCD
   int first_reset;                                        // token 0 of every sequence carries RGLRU_FLAG_RESET (and flags is null)
   unsigned bw_magic;                                      // decode step: ceil(2^32 / bw), channel / bw as a multiply-high (channel < 2^16)
@@ -503,15 +503,16 @@ inline int is_aligned(const void* ptr, int64_t W, int64_t bw, size_t es) {
 }
 
 // K groups of the kernels for narrow blocks with register-held weights (2, 4, 6, 8: slabs of 32 channels), or 0.  A block
-// of any multiple of 8 channels up to 128 takes them, padded to whole slabs in LDS and registers (`padded`): per element
-// they are two to four times as fast as the portable kernels, which stream the weights and finish the gradients in GEMM
-// kernels of their own, and what padding wastes is at most a slab (RG-LRU forward + backward, B3 T1537 W768 with 48-wide
-// blocks: see narrow blocks in rglru_fused_bwd.hip).
+// of any multiple of 8 channels up to 128 takes them, padded to whole slabs in LDS and registers (narrow_padded), although an
+// 8-wide block then computes on four times its channels: the portable kernels stream the weights and finish the gradients in
+// GEMM kernels of their own.  Forward + backward (forward alone) in us, portable -> padded, width 768:
+//   B8 T2048   8-wide blocks 531 -> 310 (100 -> 69), 16: 273 -> 168 (57 -> 46), 40: 222 -> 155, 48: 183 -> 119, 96: 217 -> 115, 120: 173 -> 111
+//   B1 T8192   8: 292 -> 180 (62 -> 50), 16: 165 -> 112 (37 -> 33), 40: 142 -> 111, 48: 118 -> 90, 72: 142 -> 110
+//   B2 T256    forward alone 12.6-18.0 -> 7.9-8.6 (forward + backward is bound by the host)
 inline int narrow_groups(const Geometry& g, int dtype, int aligned) {
+  if (narrow_padded(g) && g.W >= (1 << 22)) return 0;     // 64 rows of fp32 past the reach of a lane's offset
   return dtype == RGLRU_BF16 && aligned && g.bw % 8 == 0 && g.bwp <= 128 ? (int)(g.bwp / 16) : 0;
 }
-// ... and whether it is the padded variant (96-wide blocks have no other: three slabs leave the unit's fourth wave idle)
-inline bool narrow_padded(const Geometry& g) { return g.bw != g.bwp || g.bwp == 96; }
 
 // K steps of 32 channels of the decode kernels on 16 x 16 tiles (gate blocks of 16 .. 384 channels in steps
 // of 16, 16-bit storage, aligned rows), or 0 for the portable decode kernels

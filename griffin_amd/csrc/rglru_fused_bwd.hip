@@ -508,12 +508,12 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
 //   bwd_delta_kernel   the reverse scan  delta_t = dy_t + a_{t+1} delta_{t+1}  (and dh0 = a_0 delta_0).
 //                      It recomputes only the decay a_t (the recurrence gate: half of the gate
 //                      products, one sigmoid, one exp2 per element), runs the chunked scan with the
-//                      carry protocol in the reverse direction and writes delta in the storage type.
+//                      carry protocol in the reverse direction and writes delta in the storage type (PAD: in fp32).
 //   bwd_grad_kernel    everything else, which has no dependency between tokens once delta is known:
 //                      both gates again, the gradient at every element, and the two block-diagonal
 //                      GEMMs (input gradient and weight gradients) straight from registers and LDS,
 //                      so the gradients at the gate pre-activations never leave the chip.  The state
-//                      in front of a token, h_{t-1}, is the forward output y_{t-1} as stored.
+//                      in front of a token, h_{t-1}, is the forward output y_{t-1} as stored (PAD: recomputed in fp32).
 //
 // The scan kernel is light (few registers, many waves per SIMD hide the look-back); the heavy
 // kernel has no chains, no tickets and no carries, so its tiles are known in advance and can be
@@ -544,9 +544,18 @@ RGLRU_DEVICE bf16x8 gate_backward(bf16x8& d, const bf16x8& h, const bf16x8& v, f
   return dv;
 }
 
+// Keeps what is computed from v inside the loop that it stands in: the offsets of a tile's rows, hoisted out of it, take a
+// register each and push the scan kernels into scratch memory (140 bytes a lane instead of 48).
+RGLRU_DEVICE void hold_in_loop(unsigned& v) { asm volatile("" : "+v"(v)); }
+
 // GATED, in the two scan kernels: the output gate's reverse mode on the way in.  As a kernel of its own it read y, v and the
 // gradient and wrote two gradients, one of which the scan read back: 31 us next to the scan's 31 us at B8 T2048 W1024.
-// PAD, in this kernel and the two behind it: blocks that do not fill their slabs (see narrow_groups), masked variant only.
+// PAD, in this kernel and the two behind it: blocks that do not fill their slabs (see narrow_groups), masked variant only.  Before
+// these kernels took such blocks the portable ones did, which keep delta and h_{t-1} in fp32 registers and the weight-gradient sums
+// in fp32: so delta crosses memory in fp32 here, the gradient kernel recomputes h from the forward's checkpoints, and its
+// sums leave in fp32 whatever the gradients' type (unpadded blocks: 16-bit delta, y as stored, sums in the gradients' type).  That
+// is two bytes an element more and a chain of sixteen multiply-adds: at B8 T2048 W768, 48-wide blocks, the reverse scan takes 31.2 us
+// (28.7 with 16 bits), the gradient kernel 58.5 (50.6), the last sums 6.0 (4.3).
 template <typename IO, int NKG, bool MASKED, int MT, bool PAD = false, bool GATED = false>
 __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd_delta_kernel(FusedArgs p) {
   constexpr int TR = 32 * MT, EL = 16 * MT;
@@ -557,12 +566,12 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
   static_assert(sizeof(IO) == 2 && NKG > 0, "fast backward is for 16-bit storage and register-held weights");
   __shared__ __attribute__((aligned(16))) IO lds_x[TR * LDSROW];
   __shared__ __attribute__((aligned(16))) IO lds_dy[TR * LDSROW];
-  __shared__ __attribute__((aligned(16))) unsigned char stage_all[kWaves * WaveStage<TR>::kBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char stage_all[PAD ? 16 : kWaves * WaveStage<TR>::kBytes];
   __shared__ unsigned s_ticket[2];
 
   const WaveId w = wave_identity(p, blockIdx.x);
   const int hf = w.hf, tid = threadIdx.x;
-  unsigned char* stage = stage_all + w.wave * WaveStage<TR>::kBytes;
+  unsigned char* stage = PAD ? stage_all : stage_all + w.wave * WaveStage<TR>::kBytes;
   const IO* wg = (const IO*)p.wg;
   const IO* w_a_row = wg + ((long long)(0 * p.nb + w.k) * p.bwp + (w.slab_ok ? w.o : 0)) * p.bwp + hf * Tr::HW;
   Frag wa[NKG];
@@ -705,22 +714,33 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
     if (hf == 0 && c == 0 && p.dh0 && ch_ok) p.dh0[(long long)b * W + w.ch] = d_out;
 
-    // delta of every token, through the wave's staging area, as 16-byte row segments
     carry = hf ? d_in : fmaf(A_hi, d_in, D_hi);
-    unsigned char* my = stage + WaveStage<TR>::row_offset(hf * EL) + w.r * 2;
+    const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+    if constexpr (PAD) {
+      // delta in fp32: a half-wave's store is a 128-byte row segment as it is
+      const rsrc_t rd = make_rsrc((const float*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * (2u * row_bytes));
+      unsigned off = ch_ok ? (unsigned)(hf * EL) * (2u * row_bytes) + (unsigned)w.ch * 4u : kOutOfRange;
+      hold_in_loop(off);
 #pragma unroll
-    for (int e = EL - 1; e >= 0; --e) {
-      const float d = gy[e] + carry;
-      carry = a[e] * d;
-      *reinterpret_cast<IO*>(my + e * WaveStage<TR>::kRowBytes) = (IO)d;
-    }
-    wave_lds_fence();
-    {
-      const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+      for (int e = EL - 1; e >= 0; --e) {
+        const float d = gy[e] + carry;
+        carry = a[e] * d;
+        BufIo<float>::store(d, rd, off + (unsigned)e * (2u * row_bytes), 0u);   // past kOutOfRange: dropped too
+      }
+    } else {
+      // delta of every token, through the wave's staging area, as 16-byte row segments
+      unsigned char* my = stage + WaveStage<TR>::row_offset(hf * EL) + w.r * 2;
+#pragma unroll
+      for (int e = EL - 1; e >= 0; --e) {
+        const float d = gy[e] + carry;
+        carry = a[e] * d;
+        *reinterpret_cast<IO*>(my + e * WaveStage<TR>::kRowBytes) = (IO)d;
+      }
+      wave_lds_fence();
       const rsrc_t rd = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane, !PAD || w.slab * 32 + (w.lane & 3) * 8 < p.bw);
+      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane);
+      wave_lds_fence();
     }
-    wave_lds_fence();
     tk = tk_next;
   }
   if constexpr (GATED) {
@@ -851,9 +871,14 @@ __global__ __launch_bounds__(delta_chain_waves(GATED) * 64, 1) void bwd_delta_ch
     // the stores the loop's back edge has in flight behind the prefetched tiles (dh0, two delta segments),
     // dropped through their offsets, in front of its entry (see fwd_chain_kernel)
     BufIo<float>::store(0.f, rh0, kOutOfRange, 0u);
-    const i32x4 nothing = {0, 0, 0, 0};
-    buf_store_b128(nothing, rh0, kOutOfRange);
-    buf_store_b128(nothing, rh0, kOutOfRange + 16u);
+    if constexpr (PAD) {                                   // ... or sixteen words of delta
+#pragma unroll
+      for (int e = 0; e < 16; ++e) BufIo<float>::store(0.f, rh0, kOutOfRange + 4u * (unsigned)(e + 1), 0u);
+    } else {
+      const i32x4 nothing = {0, 0, 0, 0};
+      buf_store_b128(nothing, rh0, kOutOfRange);
+      buf_store_b128(nothing, rh0, kOutOfRange + 16u);
+    }
   }
   for (int c = nC - 1 - wave; c >= 0; c -= WAVES) {
     const int t0 = c * TR;
@@ -936,23 +961,34 @@ __global__ __launch_bounds__(delta_chain_waves(GATED) * 64, 1) void bwd_delta_ch
                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     BufIo<float>::store(d_out, rh0, (hf == 0 && c == 0 && ch_ok) ? ((unsigned)b * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
 
-    // delta of every token, through the x tile's area, as 16-byte row segments
     run = hf ? d_in : fmaf(A_hi, d_in, D_hi);
-    wave_lds_fence();                                      // dy has been read: its area becomes the staging area
-    unsigned char* my = stage + WaveStage<TR>::row_offset(hf * 16) + r * 2;
+    wave_lds_fence();                                      // dy has been read: its area is free
+    const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+    if constexpr (PAD) {
+      // delta in fp32: a half-wave's store is a 128-byte row segment as it is
+      const rsrc_t rd = make_rsrc((const float*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * (2u * row_bytes));
+      unsigned off = ch_ok ? (unsigned)(hf * 16) * (2u * row_bytes) + (unsigned)ch * 4u : kOutOfRange;
+      hold_in_loop(off);
 #pragma unroll
-    for (int e = 15; e >= 0; --e) {
-      const float d = gy[e] + run;
-      run = a[e] * d;
-      *reinterpret_cast<IO*>(my + e * WaveStage<TR>::kRowBytes) = (IO)d;
-    }
-    wave_lds_fence();
-    {
-      const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
+      for (int e = 15; e >= 0; --e) {
+        const float d = gy[e] + run;
+        run = a[e] * d;
+        BufIo<float>::store(d, rd, off + (unsigned)e * (2u * row_bytes), 0u);   // past kOutOfRange: dropped too
+      }
+    } else {
+      // delta of every token, through the x tile's area, as 16-byte row segments
+      unsigned char* my = stage + WaveStage<TR>::row_offset(hf * 16) + r * 2;
+#pragma unroll
+      for (int e = 15; e >= 0; --e) {
+        const float d = gy[e] + run;
+        run = a[e] * d;
+        *reinterpret_cast<IO*>(my + e * WaveStage<TR>::kRowBytes) = (IO)d;
+      }
+      wave_lds_fence();
       const rsrc_t rd = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane, seg_ok);
+      stage_flush<TR>(stage, rd, row_bytes, (unsigned)(col0 + sl * 32) * 2u, lane);
+      wave_lds_fence();
     }
-    wave_lds_fence();
   }
   if (gave_up && lane == 0) atomicOr(p.fail, 1u);
   if constexpr (GATED) {
@@ -1068,13 +1104,26 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
     for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int i = 0; i < Tr::HW; ++i) ident[q][i] = (IO)((16 * q + 8 * hf + i == r) ? 1.0f : 0.0f);
-    Frag pre_d[2], pre_h[2];
+    // PAD: delta is fp32 and comes as it lies in the accumulator, the state in front of the lane's run from its checkpoint.
+    Frag pre_d[PAD ? 1 : 2], pre_h[PAD ? 1 : 2];
+    float pre_delta[PAD ? 16 : 1], pre_state = 0.f;
     const int my_row = tile_row<1>(0, r);
     auto issue = [&](const Place& q) {
       const bool live = q.tile < n_tiles;
       const int b = live ? q.b : 0, c = live ? q.c : 0;
       const int t0 = c * TR;
       const int rows = !live ? 0 : ((p.T - t0) < TR ? (p.T - t0) : TR);
+      if constexpr (PAD) {
+        const rsrc_t rd = make_rsrc((const float*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * (2u * row_bytes));
+        unsigned off = ch_ok ? (unsigned)(hf * 16) * (2u * row_bytes) + (unsigned)ch * 4u : kOutOfRange;
+        hold_in_loop(off);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) pre_delta[e] = BufIo<float>::load(rd, off + (unsigned)e * (2u * row_bytes), 0u);
+        const rsrc_t rs = make_rsrc(p.ckpt + (long long)b * p.ckpt_nC * W, live ? (unsigned)p.ckpt_nC * (unsigned)W * 4u : 0u);
+        const int run = 2 * c + hf;                        // in front of token 0: h0, further down
+        pre_state = BufIo<float>::load(rs, ch_ok && run > 0 ? ((unsigned)(run - 1) * (unsigned)W + (unsigned)ch) * 4u : kOutOfRange, 0u);
+        return;
+      }
       const rsrc_t rd = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
       // the state in front of token t is the output row t - 1; tile row i wants y row t0 - 1 + i.  The
       // row in front of the sequence's first token does not exist (h0 takes its place further down).
@@ -1083,11 +1132,10 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
       const int y_rows = !live ? 0 : (t0 + rows - 1 - y_first);
       const rsrc_t rh = make_rsrc((const IO*)p.y + ((long long)b * p.T + y_first) * W, (unsigned)(y_rows > 0 ? y_rows : 0) * row_bytes);
 #pragma unroll
-      for (int q2 = 0; q2 < 2; ++q2) {
-        const bool there = !PAD || sl * 32 + q2 * Tr::KG + hf * Tr::HW < bw;
+      for (int q2 = 0; q2 < (PAD ? 1 : 2); ++q2) {
         const unsigned col = (unsigned)(slab_col + q2 * Tr::KG + hf * Tr::HW) * 2u;
-        pre_d[q2] = buf_load_frag<Frag>(rd, there ? (unsigned)my_row * row_bytes + col : kOutOfRange);
-        pre_h[q2] = buf_load_frag<Frag>(rh, my_row >= shift && there ? (unsigned)(my_row - shift) * row_bytes + col : kOutOfRange);
+        pre_d[q2] = buf_load_frag<Frag>(rd, (unsigned)my_row * row_bytes + col);
+        pre_h[q2] = buf_load_frag<Frag>(rh, my_row >= shift ? (unsigned)(my_row - shift) * row_bytes + col : kOutOfRange);
       }
     };
     // gate products of one tile: issued one iteration before their results are used, so the matrix
@@ -1123,12 +1171,15 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
         const IO* tile_x = lds_x[xb];
         f32x16 xc, dc, hc, ua_next, ux_next;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) { xc[v] = 0.0f; dc[v] = 0.0f; hc[v] = 0.0f; }
+        for (int v = 0; v < 16; ++v) { xc[v] = 0.0f; dc[v] = PAD ? pre_delta[PAD ? v : 0] : 0.0f; hc[v] = 0.0f; }
+        float h = c == 0 && hf == 0 ? h_first : pre_state;   // PAD: the state in front of the token at hand
         const IO* xrow = tile_x + my_row * ROW + hf * Tr::HW;
 #pragma unroll
         for (int q2 = 0; q2 < 2; ++q2) {
-          Tr::mma(dc, pre_d[q2], ident[q2]);
-          Tr::mma(hc, pre_h[q2], ident[q2]);
+          if constexpr (!PAD) {
+            Tr::mma(dc, pre_d[q2], ident[q2]);
+            Tr::mma(hc, pre_h[q2], ident[q2]);
+          }
           Tr::mma(xc, *reinterpret_cast<const Frag*>(xrow + slab * 32 + q2 * Tr::KG), ident[q2]);
         }
         gate_products(lds_x[xn], ua_next, ux_next);
@@ -1147,7 +1198,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
           const int tok = hf * 16 + v;
           const float xe = xc[v];
           const float d = dc[v];
-          const float hp = hc[v];
+          const float hp = PAD ? h : hc[v];
           const float re = sigmoid_fast(ua[v], nba), ie = sigmoid_fast(ux[v], nbx);
           float l2 = re * sp;
           if constexpr (MASKED) l2 = masked_log2_decay_run(l2, flbits, v);
@@ -1160,6 +1211,7 @@ __global__ __launch_bounds__(kGradThreads, 1) void bwd_grad_kernel(FusedArgs p) 
           const float c1 = ge * ie;
           const float dxd = d * c1;
           const float ze = c1 * xe;
+          if constexpr (PAD) h = fmaf(ae, h, ze);
           const float q2 = (ie * xe) * __builtin_amdgcn_rsqf(fmaxf(g2, 0.25f * 1e-6f));
           float dl = (ae * d) * fmaf(-ae, q2, hp);
           // A reset token has a = 2^-126, which already switches dl off; a padded one has g = 0, which
@@ -1899,6 +1951,10 @@ static int grad_workgroups(int64_t B, int64_t T, int units) {
   return n_wg > tiles ? (int)tiles : n_wg;
 }
 
+// 16-bit weight gradients asked for: the per-workgroup sums (fp32 in registers over a workgroup's share of the tokens) of
+// unpadded blocks cross memory as bf16 too, which halves what the finish kernel reads back.
+static int sums_bf16(const Geometry& g, int grad_dtype) { return grad_dtype == RGLRU_BF16 && !narrow_padded(g); }
+
 // Last sums of the fast backward; returns the workgroups they take.
 static int fast_finish_args(const Geometry& g, const void* prep, const char* scratch, int64_t B, int64_t T, int dtype, int grad_dtype,
                             void* dw_a, void* dw_x, void* db_a, void* db_x, void* dlambda, FinishArgs& r) {
@@ -1912,7 +1968,7 @@ static int fast_finish_args(const Geometry& g, const void* prep, const char* scr
   r.dw_partial = (const float*)(scratch + SL.dw_partial); r.dw_a = dw_a; r.dw_x = dw_x;
   r.W = (int)g.W; r.nb = (int)g.nb; r.bw = (int)g.bw; r.bwp = (int)g.bwp; r.Wp = (int)g.Wp;
   r.n_wg = r.wg_per_unit = grad_workgroups(B, T, a.units);
-  r.vec_blocks = (int)((g.W + 15) / 16); r.grad_dtype = grad_dtype; r.dw_bf16 = grad_dtype == RGLRU_BF16; r.dw_vec = 1;
+  r.vec_blocks = (int)((g.W + 15) / 16); r.grad_dtype = grad_dtype; r.dw_bf16 = sums_bf16(g, grad_dtype); r.dw_vec = 1;
   return r.vec_blocks + (int)((g.nb * g.bw * 2 * g.bw / 8 + 255) / 256);
 }
 
@@ -1957,9 +2013,7 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
   const int nkg = narrow_groups(g, dtype, 1);
   const bool pad = narrow_padded(g);
   pack_units(a, g, nkg);
-  // 16-bit weight gradients asked for: the per-workgroup sums (fp32 in registers over a workgroup's share of
-  // the tokens) cross memory as bf16 too, which halves what the finish kernel reads back
-  a.dw_bf16 = grad_dtype == RGLRU_BF16 ? 1 : 0;
+  a.dw_bf16 = sums_bf16(g, grad_dtype);
   // reverse scan: delta[B, T, W] (and dh0)
   const long long chunks = (T + 32 * kDeltaMT - 1) / (32 * kDeltaMT);
   a.wg_per_unit = pick_wg_per_unit(a.units, B * chunks, kDeltaMT == 1 ? 4 : RGLRU_DELTA_OCC, L.max_wg);

@@ -26,6 +26,10 @@ inline Geometry make_geometry(int64_t W, int64_t nb) {
   return g;
 }
 
+// Whether the kernels for blocks of up to 128 channels run their padded variant (96-wide blocks have no other: three slabs
+// leave the unit's fourth wave idle).
+inline bool narrow_padded(const Geometry& g) { return g.bw != g.bwp || g.bwp == 96; }
+
 // Prepared parameter image.
 //   wg    [2][nb][bwp][bwp]  storage type, zero padded: gate weights, row = output channel
 //   bias  [2][Wp]            fp32
@@ -102,12 +106,12 @@ int gate_dw_splits(long long N, const Geometry& g);
 
 // Scratch of one backward call; nothing in it outlives the call, its contents on entry do not matter.
 //   partial     [maxWg][3][Wp]  per-workgroup sums for db_a, db_x, dLambda
-//   delta       fast backward (blocks of 32, 64, 128 channels): [B][T][W] 16-bit, dL/dh_t after the
-//               reverse scan; wide backward (blocks of 129 .. 384 channels): [B][T][nb][2 bw] 16-bit,
+//   delta       fast backward (blocks of up to 128 channels): [B][T][W] 16-bit (padded blocks: fp32), dL/dh_t after
+//               the reverse scan; wide backward (blocks of 129 .. 384 channels): [B][T][nb][2 bw] 16-bit,
 //               the gradients at the gate pre-activations as pairs (element 2 o + gate)
 //   dw_partial  [sets][nb][2][bwp][bwp] per-workgroup weight-gradient sums, sets = kGemmWgPerUnit (fast),
 //               kWideWgPerUnit (wide) or gate_dw_splits (the other paths); fp32, or bf16 in the fast backward
-//               when 16-bit gradients are asked for (sized for fp32 either way)
+//               of unpadded blocks when 16-bit gradients are asked for (sized for fp32 either way)
 enum ScratchKind { kScratchPlain = 0, kScratchFast = 1, kScratchWide = 2 };
 struct ScratchLayout {
   size_t partial, delta, dw_partial, total;
@@ -118,7 +122,7 @@ inline ScratchLayout make_scratch_layout(int64_t B, int64_t T, const Geometry& g
   size_t off = 0;
   auto take = [&](int64_t bytes) { size_t at = off; off += (size_t)round_up(bytes, 256); return at; };
   s.partial = take((int64_t)256 * 3 * g.Wp * 4);
-  s.delta = take(kind == kScratchFast ? B * T * g.W * 2 : kind == kScratchWide ? B * T * g.W * 4 : 0);
+  s.delta = take(kind == kScratchFast ? B * T * g.W * (narrow_padded(g) ? 4 : 2) : kind == kScratchWide ? B * T * g.W * 4 : 0);
   const int64_t sets = kind == kScratchFast ? kGemmWgPerUnit : kind == kScratchWide ? kWideWgPerUnit : gate_dw_splits(B * T, g);
   s.dw_partial = take(sets * g.nb * g.bwp * 2 * g.bwp * 4);
   s.total = off;

@@ -964,6 +964,42 @@ def test_portable_kernels_pack_narrow_blocks(bw, nb, dtype, tol):
         assert rel_err(grads[name].float(), rgrads[name]) < tol, name
 
 
+@pytest.mark.parametrize("bw,nb", [(8, 3), (24, 4), (48, 16), (72, 2), (96, 3), (120, 2)])
+@pytest.mark.parametrize("B,T,masks", [(2, 200, True), (1, 96, False)])
+def test_padded_narrow_blocks_keep_fp32_inside_the_backward(bw, nb, B, T, masks, kernel_choice):
+    """What the portable kernels, which such blocks had before, hold in fp32 stays so: dL/dh, the state in front of a token and
+    the partial sums of the weight gradients.  The bias, Lambda and initial-state gradients are sums of fp32 products of
+    these: 32-bit rounding of a few dozen operations an element (fast sigmoid and exp2 among them, about 1e-6 each) stays below
+    1e-4 of the largest entry, one 16-bit rounding of dL/dh or h alone (2^-9 an element) does not.  Weight gradients
+    asked for in bf16 are those in fp32 rounded once, which 16-bit partial sums are not."""
+    from griffin_amd import hip_rglru, set_reproducible
+
+    _say("fp32 inside", bw, nb, B, T, masks, kernel_choice)
+    case = orc.make_case(B, T, bw * nb, nb, seed=bw + 1, h0_std=0.5, bias_std=0.5)
+    for k in (*PARAMS, "dy"):
+        case[k] = case[k].bfloat16().float()
+    reset, active = _masks(B, T, masks)
+    dh_last = torch.randn(B, bw * nb, generator=torch.Generator().manual_seed(6))
+    _, _, want = oracle_run(case, torch.float64, reset, active, dh_last.double())
+
+    def run(dtype):
+        leaves = [case[k].to(torch.bfloat16 if k == "x" else dtype).cuda().requires_grad_(True) for k in PARAMS]
+        leaves.append(case["h0"].float().cuda().requires_grad_(True))
+        y, h = hip_rglru(*leaves[:6], 8.0, leaves[6], None if reset is None else reset.cuda(), None if active is None else active.cuda())
+        return dict(zip((*PARAMS, "h0"), torch.autograd.grad([y, h], leaves, [case["dy"].bfloat16().cuda(), dh_last.cuda()])))
+
+    was = set_reproducible(True)
+    try:
+        got, got16 = run(torch.float32), run(torch.bfloat16)
+    finally:
+        set_reproducible(was)
+    errs = {name: rel_err(got[name], want[name]) for name in ("b_a", "b_x", "lam", "h0")}
+    _say("  ", {k: "%.1e" % v for k, v in errs.items()})
+    assert max(errs.values()) < 1e-4, errs
+    for name in ("w_a", "w_x"):
+        assert torch.equal(got16[name], got[name].bfloat16()), name
+
+
 @pytest.mark.parametrize("bw,nb", [(136, 2), (152, 3), (168, 1), (216, 2), (248, 1), (264, 2), (312, 1), (344, 1), (376, 2)])
 @pytest.mark.parametrize("B,T,masks,carried", [(2, 70, True, True), (1, 64, False, False), (3, 33, False, True)])
 def test_padded_wide_blocks_match_oracle(bw, nb, B, T, masks, carried):
