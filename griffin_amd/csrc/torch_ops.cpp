@@ -190,8 +190,18 @@ int64_t kernel_path(int64_t B, int64_t T, int64_t W, int64_t nb, at::ScalarType 
   return path;
 }
 
+// The kernels read as many elements as the first gate's weights say: the other four parameters have to have them.
+void check_gates(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam) {
+  TORCH_CHECK_VALUE(w_a.dim() == 3 && w_a.size(1) == w_a.size(2) && w_x.sizes() == w_a.sizes(), "gate weights must both have shape [blocks, width, width], got ",
+                    w_a.sizes(), " and ", w_x.sizes());
+  const int64_t W = w_a.size(0) * w_a.size(1);
+  TORCH_CHECK_VALUE(b_a.numel() == W && b_x.numel() == W && lam.numel() == W, "gate biases and Lambda must have ", W, " elements, got ", b_a.numel(),
+                    ", ", b_x.numel(), " and ", lam.numel());
+}
+
 Tensor prepare(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam, double c,
                at::ScalarType dtype) {
+  check_gates(w_a, b_a, w_x, b_x, lam);
   const int64_t nb = w_a.size(0), W = nb * w_a.size(1);
   const int code = code_of(dtype);
   refuse_tangents("hip RG-LRU", std::array<Tensor, 5>{w_a, b_a, w_x, b_x, lam});
@@ -419,6 +429,7 @@ std::tuple<Tensor, Tensor> rglru(const Tensor& x, const Tensor& w_a, const Tenso
   Tensor h0 = opt(h0_), flags = opt(flags_);
   require_gpu("hip RG-LRU", {&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0, &flags});
   check_fused(x, w_a, h0, flags);
+  check_gates(w_a, b_a, w_x, b_x, lam);
   if (wants_grad({&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0})) {
     auto out = RGLRU::apply(x, w_a, b_a, w_x, b_x, lam, maybe(h0), maybe(flags), first_reset, c, path);
     return {out[0], out[1]};
@@ -506,11 +517,19 @@ void hold_leaves(const py::dict& members, const std::vector<Tensor>& tensors) {
   }
 }
 
+// One flag byte for each of so many tokens, as the kernels read them.
+Tensor token_bytes(const Tensor& flags, int64_t tokens) {
+  if (!flags.defined()) return flags;
+  TORCH_CHECK_VALUE(flags.numel() == tokens && flags.element_size() == 1, "expected one byte for each of ", tokens, " tokens, got ", flags.sizes());
+  return flags.contiguous();
+}
+
 Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
   Tensor flags = opt(flags_);
   require_gpu("hip RG-LRU step", {&x_in, &state, &flags});
   TORCH_CHECK_VALUE(state.sizes() == x_in.sizes() && state.scalar_type() == at::kFloat && state.is_contiguous(),
                     "step expects a contiguous fp32 state of the same shape as x");
+  flags = token_bytes(flags, x_in.size(0));
   c10::DeviceGuard guard(x_in.device());
   Tensor x = x_in.contiguous();
   Tensor y = fresh_like(x);
@@ -540,6 +559,8 @@ std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x_in, const Tensor& i
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(x_in.device());
   const int64_t B = x_in.size(0), W = x_in.size(2);
+  flags = token_bytes(flags, B);
+  TORCH_CHECK_VALUE(!state.has_value() || (state->dim() == 2 && state->size(0) == B && state->size(1) == W), "the state must have shape (", B, ", ", W, ")");
   Tensor x = x_in.contiguous();
   Tensor h = state.has_value() ? as(*state, at::kFloat) : at::zeros({B, W}, x.options().dtype(at::kFloat));
   Tensor h_new = fresh({B, W}, at::kFloat, x);
@@ -1032,7 +1053,9 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& 
   TORCH_CHECK_VALUE(u.dim() == 3 && u.sizes() == v.sizes() && u.scalar_type() == v.scalar_type(),
                     "hip_block_forward expects two [batch, sequence, width] tensors of one dtype");
   const int64_t B = u.size(0), T = u.size(1), W = u.size(2);
-  check_conv("hip_block_forward", u, conv_state, weight, Tensor(), segment_pos);
+  check_conv("hip_block_forward", u, conv_state, weight, bias, segment_pos);
+  check_gates(w_a, b_a, w_x, b_x, lam);
+  TORCH_CHECK_VALUE(w_a.size(0) * w_a.size(1) == W, "gate weights ", w_a.sizes(), " do not match width ", W);
   TORCH_CHECK_VALUE(!h0.defined() || (h0.dim() == 2 && h0.size(0) == B && h0.size(1) == W), "initial state must have shape (", B, ", ", W, ")");
   TORCH_CHECK_VALUE(!flags.defined() || (flags.dim() == 2 && flags.size(0) == B && flags.size(1) == T && flags.scalar_type() == at::kByte && flags.is_contiguous()),
                     "flags must be a contiguous uint8 tensor of shape [batch, sequence]");
@@ -1060,6 +1083,15 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> block_decode_step(const Tensor& u_in,
                     "hip_block_decode_step expects two [batch, width] tensors of one dtype");
   const int64_t B = u_in.size(0), W = u_in.size(1), K = weight.size(2);
   TORCH_CHECK_VALUE(W == width && u_in.scalar_type() == prep_dtype, "the prepared RG-LRU parameters do not match the activations");
+  TORCH_CHECK_VALUE(weight.dim() == 3 && weight.size(0) == W && weight.size(1) == 1, "weight must be that of a depthwise Conv1d: [width, 1, kernel_size]");
+  TORCH_CHECK_VALUE(!bias.defined() || (bias.dim() == 1 && bias.size(0) == W), "bias must have shape [width]");
+  TORCH_CHECK_VALUE(!conv_state.defined() || (conv_state.dim() == 3 && conv_state.size(0) == B && conv_state.size(1) == K - 1 && conv_state.size(2) == W),
+                    "state must have shape [batch, kernel_size - 1, width]");
+  TORCH_CHECK_VALUE(!rnn_state.defined() || (rnn_state.dim() == 2 && rnn_state.size(0) == B && rnn_state.size(1) == W), "the state must have shape (",
+                    B, ", ", W, ")");
+  for (const Tensor* t : {&prev_pos, &segment_pos})
+    TORCH_CHECK_VALUE(!t->defined() || (t->numel() == B && t->scalar_type() == at::kLong && t->is_contiguous()), "positions must be ", B, " contiguous integers");
+  active = token_bytes(active, B);
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(u_in.device());
   const auto dtype = u_in.scalar_type();
@@ -1088,6 +1120,24 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> block_decode_step(const Tensor& u_in,
   return {out, h_out, new_conv, new_pos};
 }
 
+// A vector of n elements, or absent.
+bool has(const Tensor& t, int64_t n) { return !t.defined() || (t.dim() == 1 && t.size(0) == n); }
+
+// Whether the Linear layers and the convolution of a block belong together: [W, D] twice, [W, 1, K], [D, W], with biases to match.
+bool block_shapes(int64_t D, const Tensor& w_x, const Tensor& b_x, const Tensor& w_y, const Tensor& b_y, const Tensor& conv_w, const Tensor& conv_b,
+                  const Tensor& w_o, const Tensor& b_o) {
+  if (w_x.dim() != 2 || w_x.size(1) != D || w_y.sizes() != w_x.sizes() || w_o.dim() != 2 || conv_w.dim() != 3) return false;
+  const int64_t W = w_x.size(0);
+  return has(b_x, W) && has(b_y, W) && conv_w.size(0) == W && conv_w.size(1) == 1 && conv_w.size(2) >= 1 && has(conv_b, W) && w_o.size(0) == D &&
+         w_o.size(1) == W && has(b_o, D);
+}
+
+// ... and the carried state of B rows.
+bool state_shapes(int64_t B, int64_t W, int64_t K, const Tensor& conv_state, const Tensor& rnn_state, const Tensor& positions) {
+  if (conv_state.defined() && (conv_state.dim() != 3 || conv_state.size(0) != B || conv_state.size(1) != K - 1 || conv_state.size(2) != W)) return false;
+  return (!rnn_state.defined() || (rnn_state.dim() == 2 && rnn_state.size(0) == B && rnn_state.size(1) == W)) && has(positions, B);
+}
+
 // The whole single-token step of the block around the RG-LRU (griffin/griffin.py:459-528 with T == 1, no autograd) in three
 // launches: projections + positions + convolution, RG-LRU step + output gate, output projection.  Nothing is returned
 // where the kernels do not take the operands (mixed types, unaligned rows, many rows): the caller then goes through the
@@ -1100,8 +1150,11 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
          prev_pos = opt(prev_pos_), segment_pos = opt(segment_pos_), active = opt(active_), rnn_state = opt(rnn_state_);
   const auto dtype = x_in.scalar_type();
   refuse_tangents("hip_block_step", std::initializer_list<Tensor>{x_in, w_x, b_x, w_y, b_y, conv_w, conv_b, w_o, b_o, conv_state, rnn_state});
+  if (!block_shapes(x_in.size(2), w_x, b_x, w_y, b_y, conv_w, conv_b, w_o, b_o)) return std::nullopt;
   const int64_t B = x_in.size(0), D = x_in.size(2), W = w_x.size(0), K = conv_w.size(2);
-  if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || w_o.size(0) != D || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
+  if (!state_shapes(B, W, K, conv_state, rnn_state, prev_pos) || !has(segment_pos, B)) return std::nullopt;
+  active = token_bytes(active, B);
+  if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state})
     if (t->defined() && (t->scalar_type() != dtype || !t->is_contiguous() || !t->is_cuda())) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &w_y, &w_o})
@@ -1223,9 +1276,7 @@ py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py
       !conv.parameter("weight", cw) || !conv.parameter("bias", cb) || !lo.parameter("weight", wo) || !lo.parameter("bias", bo))
     return py::none();
   const int64_t B = x.size(0), W = (int64_t)block.number("rnn_width", -1), K = (int64_t)block.number("conv_kernel_size", -1);
-  if (wx.dim() != 2 || wx.size(0) != W || wx.size(1) != x.size(2) || wy.sizes() != wx.sizes() || wo.dim() != 2 || wo.size(1) != W ||
-      cw.dim() != 3 || cw.size(2) != K || wx.scalar_type() != x.scalar_type())
-    return py::none();
+  if (wx.dim() != 2 || wx.size(0) != W || cw.dim() != 3 || cw.size(2) != K || wx.scalar_type() != x.scalar_type()) return py::none();
   MaybeTensor conv_state, prev, rnn;
   if (!cache.is_none()) {
     auto field = [&](const char* name, MaybeTensor& t) {
@@ -1237,10 +1288,8 @@ py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py
       return t->device() == x.device();
     };
     if (!field("conv_state", conv_state) || !field("segment_position", prev) || !field("rnn_state", rnn)) return py::none();
-    if (!conv_state || !prev || conv_state->dim() != 3 || conv_state->size(0) != B || conv_state->size(1) != K - 1 || conv_state->size(2) != W ||
-        prev->dim() != 1 || prev->size(0) != B || prev->scalar_type() != at::kLong || !prev->is_contiguous())
-      return py::none();
-    if (rnn && (rnn->dim() != 2 || rnn->size(0) != B || rnn->size(1) != W)) return py::none();
+    if (!conv_state || !prev || !state_shapes(B, W, K, *conv_state, opt(rnn), *prev) || prev->scalar_type() != at::kLong || !prev->is_contiguous())
+      return py::none();                                   // the module's Python code reports a wrong shape
   }
   const Stamp* s = current_stamp(lru, x.scalar_type(), x.device());
   if (s == nullptr) return py::none();
@@ -1280,7 +1329,7 @@ bool vector_rows(const Tensor& t) {
 // Whether the library takes y = x w^T + b (and its gradients) for these operands.
 bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b) {
   const auto dtype = x.scalar_type();
-  return w.dim() == 2 && x.size(-1) == w.size(1) && w.scalar_type() == dtype && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
+  return w.dim() == 2 && x.size(-1) == w.size(1) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
          x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype) && vector_rows(w) && vector_rows(x) &&
          (w.size(0) * x.element_size()) % 16 == 0 && !at::autocast::is_autocast_enabled(at::kCUDA);
 }
@@ -1739,6 +1788,30 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
   }
 };
 
+// Whether the thirteen parameters p of a block (BlockTrain's tensors behind x) belong together and to inputs of model width D.
+bool block_parameters(int64_t D, const std::vector<Tensor>& p) {
+  typedef BlockTrain N;
+  if (p.size() != N::kTensors - 1) return false;
+  const Tensor &wa = p[N::WA - 1], &wi = p[N::WI - 1];
+  if (!block_shapes(D, p[N::WX - 1], p[N::BX - 1], p[N::WY - 1], p[N::BY - 1], p[N::CW - 1], p[N::CB - 1], p[N::WO - 1], p[N::BO - 1])) return false;
+  const int64_t W = p[N::WX - 1].size(0);
+  if (wa.dim() != 3 || wa.size(1) != wa.size(2) || wa.size(0) * wa.size(1) != W || wi.sizes() != wa.sizes()) return false;
+  for (int i : {N::BA, N::BI, N::LAM})
+    if (p[i - 1].numel() != W) return false;
+  return true;
+}
+
+// ... and whether the per-token operands have the shape of [B, T] tokens.
+bool token_shapes(int64_t B, int64_t T, int64_t W, const Tensor& pos, const Tensor& flags, const Tensor& rows, const Tensor& active, const Tensor& u,
+                  const Tensor& v) {
+  auto tokens = [&](const Tensor& t) { return t.dim() == 2 && t.size(0) == B && t.size(1) == T; };
+  auto width = [&](const Tensor& t) { return t.dim() == 3 && t.size(0) == B && t.size(1) == T && t.size(2) == W; };
+  return (!pos.defined() || tokens(pos)) && (!flags.defined() || (tokens(flags) && flags.element_size() == 1 && flags.is_contiguous())) &&
+         (!rows.defined() || (rows.numel() == 3 * B && rows.scalar_type() == at::kInt && rows.is_contiguous())) &&
+         (!active.defined() || (tokens(active) && active.element_size() == 1)) && u.defined() == v.defined() &&
+         (!u.defined() || (width(u) && width(v) && u.scalar_type() == v.scalar_type()));
+}
+
 // Nothing is returned where the node does not take the operands; the caller then goes layer by layer.
 MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const MaybeTensor& flags, const MaybeTensor& rows,
                         const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
@@ -1748,12 +1821,12 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
   refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(u), opt(v)});
   for (const Tensor& t : p)
     if (t.scalar_type() != N::kType || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
+  if (!block_parameters(D, p)) return std::nullopt;
   // p: the node's tensors behind x
-  const Tensor &wx = p[N::WX - 1], &wy = p[N::WY - 1], &wo = p[N::WO - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
+  const Tensor &wx = p[N::WX - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
   const int64_t W = wx.size(0);
-  if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 || wx.dim() != 2 || wx.size(1) != D || wy.sizes() != wx.sizes() ||
-      wo.dim() != 2 || wo.size(0) != D || wo.size(1) != W || cw.dim() != 3 || cw.size(0) != W || wa.dim() != 3 || wa.size(0) * wa.size(1) != W ||
-      (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
+  if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 || !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), opt(v)) ||
+      (u.has_value() && u->scalar_type() != N::kType) || (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
     return std::nullopt;
   MaybeTensor live;
   if (active.has_value()) live = active->contiguous();
@@ -1778,11 +1851,12 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
   refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(conv_state_), opt(rnn_state_), opt(u_), opt(v_)});
   for (const Tensor& t : p)
     if (t.scalar_type() != dtype || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
+  if (!block_parameters(D, p)) return std::nullopt;
   const Tensor &wx = p[N::WX - 1], &bx = p[N::BX - 1], &wy = p[N::WY - 1], &by = p[N::BY - 1], &cw = p[N::CW - 1], &cb = p[N::CB - 1],
                &wa = p[N::WA - 1], &wo = p[N::WO - 1], &bo = p[N::BO - 1];
   const int64_t W = wx.size(0), K = cw.size(2), nb = wa.size(0), M = B * T;
-  if (!vector_rows(x) || W % 8 || wx.dim() != 2 || wx.size(1) != D || wy.sizes() != wx.sizes() || wo.dim() != 2 || wo.size(0) != D ||
-      wo.size(1) != W || cw.size(0) != W || !rglru_hip_block_fwd_path(W, nb, K, code_of(dtype)))
+  if (!vector_rows(x) || W % 8 || !token_shapes(B, T, W, opt(segment_pos_), opt(flags_), opt(rows_), opt(active_), opt(u_), opt(v_)) ||
+      (u_.has_value() && u_->scalar_type() != dtype) || !state_shapes(B, W, K, opt(conv_state_), opt(rnn_state_), opt(prev_pos_)) || !rglru_hip_block_fwd_path(W, nb, K, code_of(dtype)))
     return std::nullopt;
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(x.device());

@@ -953,3 +953,46 @@ def test_forward_mode_is_refused(grad):
                 call(fwd.make_dual(primal, torch.ones_like(primal)))
     with torch.no_grad():
         assert all(torch.isfinite(m(x).float()).all() for m in (layer, norm, block))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("what", ["layer", "block"])
+def test_parameters_of_the_wrong_length_are_refused(what, dtype):
+    """A parameter that is shorter than its layer is an error on every path (a kernel that took its length from another
+    operand would read past its end), and the message is raised before anything runs."""
+    from griffin_amd import RG_LRU, RecurrentBlock
+
+    torch.manual_seed(0)
+    D, W = 64, 128
+    make = (lambda: RG_LRU(W, gate_blocks=2)) if what == "layer" else (lambda: RecurrentBlock(D, W, gate_blocks=2))
+    features = W if what == "layer" else D
+    x = torch.randn(3, 9, features, device="cuda", dtype=dtype)
+    mask = torch.ones(3, 9, dtype=torch.bool, device="cuda")
+    mask[1, 4:] = False
+    for name, _ in make().named_parameters():
+        module = make().cuda().to(dtype)
+        owner, leaf = name.rpartition(".")[::2]
+        owner = module.get_submodule(owner)
+        short = getattr(owner, leaf).detach()
+        for batch, masks in ((x, {}), (x[:, :1], {}), (x, {"active_mask": mask})):
+            with torch.no_grad():
+                module(batch, **masks)                       # what the module keeps is that of the whole parameter
+        setattr(owner, leaf, torch.nn.Parameter(short[: short.shape[0] // 2].clone()))
+        _say("short parameter", what, dtype, name)
+        for grad in (True, False):
+            for batch, masks in ((x, {}), (x[:, :1], {}), (x, {"active_mask": mask})):
+                with torch.set_grad_enabled(grad), pytest.raises((ValueError, RuntimeError)):
+                    module(batch, **masks)
+
+
+def test_a_short_bias_of_a_linear_layer_is_refused():
+    from griffin_amd.hip_block_ops import hip_linear, hip_linear_pair
+
+    x, w = torch.randn(5, 64, device="cuda"), torch.randn(32, 64, device="cuda")
+    for grad in (False, True):
+        b, good = torch.randn(16, device="cuda", requires_grad=grad), torch.randn(32, device="cuda")
+        with pytest.raises(RuntimeError):
+            hip_linear(x, w, b)
+        for pair in ((b, good), (good, b)):
+            with pytest.raises(RuntimeError):
+                hip_linear_pair(x, w, pair[0], w, pair[1])
