@@ -85,6 +85,13 @@ void require_gpu(const char* name, std::initializer_list<const Tensor*> tensors)
   for (const Tensor* t : tensors) refuse_tangent(name, *t);
 }
 
+// The kernels take addresses: an operand on another GPU than x's is an error, as it is for PyTorch's own operators.
+bool on_device_of(const Tensor& x, const Tensor& t) { return !t.defined() || t.device() == x.device(); }
+void require_device_of(const char* name, const Tensor& x, std::initializer_list<const Tensor*> tensors) {
+  for (const Tensor* t : tensors)
+    TORCH_CHECK(on_device_of(x, *t), name, " expects all tensors on the same device, found ", x.device(), " and ", t->device());
+}
+
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -202,6 +209,7 @@ void check_gates(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const 
 Tensor prepare(const Tensor& w_a, const Tensor& b_a, const Tensor& w_x, const Tensor& b_x, const Tensor& lam, double c,
                at::ScalarType dtype) {
   check_gates(w_a, b_a, w_x, b_x, lam);
+  require_device_of("hip RG-LRU", w_a, {&b_a, &w_x, &b_x, &lam});
   const int64_t nb = w_a.size(0), W = nb * w_a.size(1);
   const int code = code_of(dtype);
   refuse_tangents("hip RG-LRU", std::array<Tensor, 5>{w_a, b_a, w_x, b_x, lam});
@@ -428,6 +436,7 @@ std::tuple<Tensor, Tensor> rglru(const Tensor& x, const Tensor& w_a, const Tenso
                                  double c, int64_t path) {
   Tensor h0 = opt(h0_), flags = opt(flags_);
   require_gpu("hip RG-LRU", {&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0, &flags});
+  require_device_of("hip RG-LRU", x, {&w_a, &b_a, &w_x, &b_x, &lam, &h0, &flags});
   check_fused(x, w_a, h0, flags);
   check_gates(w_a, b_a, w_x, b_x, lam);
   if (wants_grad({&x, &w_a, &b_a, &w_x, &b_x, &lam, &h0})) {
@@ -527,6 +536,7 @@ Tensor token_bytes(const Tensor& flags, int64_t tokens) {
 Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
   Tensor flags = opt(flags_);
   require_gpu("hip RG-LRU step", {&x_in, &state, &flags});
+  require_device_of("hip RG-LRU step", x_in, {&image, &state, &flags});
   TORCH_CHECK_VALUE(state.sizes() == x_in.sizes() && state.scalar_type() == at::kFloat && state.is_contiguous(),
                     "step expects a contiguous fp32 state of the same shape as x");
   flags = token_bytes(flags, x_in.size(0));
@@ -541,6 +551,7 @@ Tensor rglru_step(const Tensor& x_in, const Tensor& image, int64_t blocks, const
 Tensor rglru_steps(const Tensor& xs_in, const Tensor& image, int64_t blocks, const Tensor& state, const MaybeTensor& flags_) {
   Tensor flags = opt(flags_);
   require_gpu("hip RG-LRU steps", {&xs_in, &state, &flags});
+  require_device_of("hip RG-LRU steps", xs_in, {&image, &state, &flags});
   c10::DeviceGuard guard(xs_in.device());
   Tensor xs = xs_in.contiguous();
   Tensor ys = fresh_like(xs);
@@ -556,6 +567,7 @@ std::tuple<Tensor, Tensor> rglru_module_step(const Tensor& x_in, const Tensor& i
                                              const MaybeTensor& flags_) {
   Tensor flags = opt(flags_), carried = opt(state);
   require_gpu("hip RG-LRU step", {&x_in, &flags, &carried});
+  require_device_of("hip RG-LRU step", x_in, {&image, &flags, &carried});
   at::NoGradGuard no_grad;
   c10::DeviceGuard guard(x_in.device());
   const int64_t B = x_in.size(0), W = x_in.size(2);
@@ -617,6 +629,7 @@ struct Scan : torch::autograd::Function<Scan> {
 
 Tensor scan(const Tensor& a, const Tensor& z, const Tensor& h0) {
   require_gpu("hip_rglru_scan", {&a, &z, &h0});
+  require_device_of("hip_rglru_scan", a, {&z, &h0});
   TORCH_CHECK_VALUE(a.dim() == 3 && a.sizes() == z.sizes(), "decay and current_input must share shape [batch, sequence, width]");
   TORCH_CHECK_VALUE(h0.dim() == 2 && h0.size(0) == a.size(0) && h0.size(1) == a.size(2), "initial_state must have shape [batch, width]");
   TORCH_CHECK_TYPE(a.scalar_type() == at::kFloat && z.scalar_type() == at::kFloat, "hip_rglru_scan expects fp32 decay and normalized input");
@@ -706,6 +719,7 @@ Tensor pack_flags(const MaybeTensor& reset_, const MaybeTensor& active_) {
   Tensor reset = mask(reset_), active = mask(active_);
   const Tensor& like = reset.defined() ? reset : active;
   require_gpu("hip RG-LRU", {&reset, &active});
+  require_device_of("hip RG-LRU", like, {&reset, &active});
   c10::DeviceGuard guard(like.device());
   Tensor flags = fresh(like.sizes(), at::kByte, like);
   if (flags.numel() > 0)
@@ -801,6 +815,7 @@ struct CausalConv : torch::autograd::Function<CausalConv> {
 Tensor causal_conv(const Tensor& u, const MaybeTensor& state_, const Tensor& weight, const MaybeTensor& bias_, const Tensor& pos) {
   Tensor state = opt(state_), bias = opt(bias_);
   require_gpu("hip_causal_conv", {&u, &state, &weight, &bias, &pos});
+  require_device_of("hip_causal_conv", u, {&state, &weight, &bias});
   check_conv("hip_causal_conv", u, state, weight, bias, pos);
   return CausalConv::apply(u, maybe(state), weight, maybe(bias), pos);
 }
@@ -866,6 +881,7 @@ std::tuple<Tensor, Tensor> causal_conv_padded(const Tensor& u, const MaybeTensor
                                               const MaybeTensor& bias_, const Tensor& pos, const Tensor& active) {
   Tensor state = opt(state_), bias = opt(bias_);
   require_gpu("hip_causal_conv_padded", {&u, &state, &weight, &bias, &pos, &active});
+  require_device_of("hip_causal_conv_padded", u, {&state, &weight, &bias});
   check_conv("hip_causal_conv_padded", u, state, weight, bias, pos);
   TORCH_CHECK_VALUE(active.sizes() == pos.sizes(), "segment_pos and active_mask must have shape [batch, sequence]");
   auto out = CausalConvPadded::apply(u, maybe(state), weight, maybe(bias), pos, active);
@@ -904,6 +920,7 @@ struct GeluGate : torch::autograd::Function<GeluGate> {
 
 Tensor gelu_gate(const Tensor& h, const Tensor& v) {
   require_gpu("hip_gelu_gate", {&h, &v});
+  require_device_of("hip_gelu_gate", h, {&v});
   TORCH_CHECK_VALUE(h.sizes() == v.sizes(), "hip_gelu_gate expects equal shapes, got ", h.sizes(), " and ", v.sizes());
   TORCH_CHECK_TYPE(h.scalar_type() == v.scalar_type(), "hip_gelu_gate expects equal dtypes, got ", h.scalar_type(), " and ", v.scalar_type());
   code_of(h.scalar_type());
@@ -1050,6 +1067,8 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& 
                                                  double c, const MaybeTensor& image_, const MaybeTensor& rows_, bool need_carry) {
   Tensor conv_state = opt(conv_state_), bias = opt(bias_), flags = opt(flags_), h0 = opt(h0_), rows = opt(rows_);
   require_gpu("hip_block_forward", {&u, &v, &conv_state, &weight, &bias, &segment_pos, &w_a, &b_a, &w_x, &b_x, &lam, &h0});
+  const Tensor image = opt(image_);
+  require_device_of("hip_block_forward", u, {&v, &conv_state, &weight, &bias, &flags, &w_a, &b_a, &w_x, &b_x, &lam, &h0, &rows, &image});
   TORCH_CHECK_VALUE(u.dim() == 3 && u.sizes() == v.sizes() && u.scalar_type() == v.scalar_type(),
                     "hip_block_forward expects two [batch, sequence, width] tensors of one dtype");
   const int64_t B = u.size(0), T = u.size(1), W = u.size(2);
@@ -1066,7 +1085,7 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Tensor& u, const Tensor& 
   }
   at::NoGradGuard no_grad;
   BlockResult r = block_forward_pass(u, v, conv_state, weight, bias, segment_pos, flags, first_reset, w_a, b_a, w_x, b_x, lam, h0, c,
-                                     opt(image_), rows, need_carry, false);
+                                     image, rows, need_carry, false);
   return {r.gated, r.h_last, r.new_conv};
 }
 
@@ -1079,6 +1098,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> block_decode_step(const Tensor& u_in,
   Tensor conv_state = opt(conv_state_), bias = opt(bias_), prev_pos = opt(prev_pos_), segment_pos = opt(segment_pos_),
          active = opt(active_), rnn_state = opt(rnn_state_);
   require_gpu("hip_block_decode_step", {&u_in, &v_in, &conv_state, &weight, &bias, &prev_pos, &segment_pos, &active, &rnn_state});
+  require_device_of("hip_block_decode_step", u_in, {&v_in, &conv_state, &weight, &bias, &prev_pos, &segment_pos, &active, &image, &rnn_state});
   TORCH_CHECK_VALUE(u_in.dim() == 2 && u_in.sizes() == v_in.sizes() && u_in.scalar_type() == v_in.scalar_type(),
                     "hip_block_decode_step expects two [batch, width] tensors of one dtype");
   const int64_t B = u_in.size(0), W = u_in.size(1), K = weight.size(2);
@@ -1153,10 +1173,13 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
   if (!block_shapes(x_in.size(2), w_x, b_x, w_y, b_y, conv_w, conv_b, w_o, b_o)) return std::nullopt;
   const int64_t B = x_in.size(0), D = x_in.size(2), W = w_x.size(0), K = conv_w.size(2);
   if (!state_shapes(B, W, K, conv_state, rnn_state, prev_pos) || !has(segment_pos, B)) return std::nullopt;
+  for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state, &prev_pos, &segment_pos,
+                                                              &active, &image, &rnn_state})
+    if (!on_device_of(x_in, *t)) return std::nullopt;
   active = token_bytes(active, B);
   if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state})
-    if (t->defined() && (t->scalar_type() != dtype || !t->is_contiguous() || !t->is_cuda())) return std::nullopt;
+    if (t->defined() && (t->scalar_type() != dtype || !t->is_contiguous())) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &w_y, &w_o})
     if (!is_aligned(*t)) return std::nullopt;
   at::NoGradGuard no_grad;
@@ -1329,7 +1352,7 @@ bool vector_rows(const Tensor& t) {
 // Whether the library takes y = x w^T + b (and its gradients) for these operands.
 bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b) {
   const auto dtype = x.scalar_type();
-  return w.dim() == 2 && x.size(-1) == w.size(1) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
+  return w.dim() == 2 && x.size(-1) == w.size(1) && on_device_of(x, w) && on_device_of(x, b) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
          x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype) && vector_rows(w) && vector_rows(x) &&
          (w.size(0) * x.element_size()) % 16 == 0 && !at::autocast::is_autocast_enabled(at::kCUDA);
 }
@@ -1481,6 +1504,8 @@ struct Linear : torch::autograd::Function<Linear> {
 Tensor linear(const Tensor& x, const Tensor& weight, const MaybeTensor& bias_, const MaybeTensor& active_) {
   Tensor bias = opt(bias_);
   require_gpu("hip_linear", {&x, &weight, &bias});
+  const Tensor mask = opt(active_);
+  require_device_of("hip_linear", x, {&weight, &bias, &mask});
   code_of(x.scalar_type());
   MaybeTensor active;
   if (active_.has_value()) {
@@ -1608,7 +1633,9 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
 
 // The values alone, without a graph.
 std::tuple<Tensor, Tensor> linear_pair_values(const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2, const MaybeTensor& b2) {
-  refuse_tangents("hip_linear_pair", std::initializer_list<Tensor>{x, w1, opt(b1), w2, opt(b2)});
+  const Tensor bias1 = opt(b1), bias2 = opt(b2);
+  refuse_tangents("hip_linear_pair", std::initializer_list<Tensor>{x, w1, bias1, w2, bias2});
+  require_device_of("hip_linear_pair", x, {&w1, &bias1, &w2, &bias2});
   at::NoGradGuard no_grad;
   return LinearPair::values(x, w1, opt(b1), w2, opt(b2));
 }
@@ -1616,6 +1643,7 @@ std::tuple<Tensor, Tensor> linear_pair_values(const Tensor& x, const Tensor& w1,
 std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const MaybeTensor& b1_, const Tensor& w2, const MaybeTensor& b2_) {
   Tensor b1 = opt(b1_), b2 = opt(b2_);
   require_gpu("hip_linear_pair", {&x, &w1, &b1, &w2, &b2});
+  require_device_of("hip_linear_pair", x, {&w1, &b1, &w2, &b2});
   code_of(x.scalar_type());
   if (!wants_grad({&x, &w1, &b1, &w2, &b2})) return linear_pair_values(x, w1, b1_, w2, b2_);
   auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2));
@@ -1819,9 +1847,13 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
   refuse_tangents("the recurrent block", p);
   refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(u), opt(v)});
+  if (!block_parameters(D, p) || !on_device_of(x, pos)) return std::nullopt;
   for (const Tensor& t : p)
-    if (t.scalar_type() != N::kType || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
-  if (!block_parameters(D, p)) return std::nullopt;
+    if (!on_device_of(x, t)) return std::nullopt;
+  for (const MaybeTensor* t : {&flags, &rows, &active, &u, &v})
+    if (t->has_value() && !on_device_of(x, **t)) return std::nullopt;
+  for (const Tensor& t : p)
+    if (t.scalar_type() != N::kType || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
   // p: the node's tensors behind x
   const Tensor &wx = p[N::WX - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
   const int64_t W = wx.size(0);
@@ -1849,9 +1881,13 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
   refuse_tangents("the recurrent block", p);
   refuse_tangents("the recurrent block", std::initializer_list<Tensor>{x, opt(conv_state_), opt(rnn_state_), opt(u_), opt(v_)});
+  if (!block_parameters(D, p) || !on_device_of(x, image)) return std::nullopt;
   for (const Tensor& t : p)
-    if (t.scalar_type() != dtype || !t.is_cuda() || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
-  if (!block_parameters(D, p)) return std::nullopt;
+    if (!on_device_of(x, t)) return std::nullopt;
+  for (const MaybeTensor* t : {&conv_state_, &rnn_state_, &prev_pos_, &segment_pos_, &flags_, &rows_, &active_, &u_, &v_})
+    if (t->has_value() && !on_device_of(x, **t)) return std::nullopt;
+  for (const Tensor& t : p)
+    if (t.scalar_type() != dtype || !t.is_contiguous() || !is_aligned(t)) return std::nullopt;
   const Tensor &wx = p[N::WX - 1], &bx = p[N::BX - 1], &wy = p[N::WY - 1], &by = p[N::BY - 1], &cw = p[N::CW - 1], &cb = p[N::CB - 1],
                &wa = p[N::WA - 1], &wo = p[N::WO - 1], &bo = p[N::BO - 1];
   const int64_t W = wx.size(0), K = cw.size(2), nb = wa.size(0), M = B * T;
@@ -1956,6 +1992,7 @@ struct RmsNorm : torch::autograd::Function<RmsNorm> {
 
 Tensor rmsnorm(const Tensor& x, const Tensor& g, double eps) {
   require_gpu("hip_rmsnorm", {&x, &g});
+  require_device_of("hip_rmsnorm", x, {&g});
   TORCH_CHECK_VALUE(g.dim() == 1 && x.dim() >= 1 && x.size(-1) == g.numel(), "hip_rmsnorm expects a scale of shape [",
                     x.dim() >= 1 ? x.size(-1) : 0, "], got ", g.sizes());
   code_of(x.scalar_type());
@@ -1970,7 +2007,7 @@ py::object norm_forward(py::handle module, const Tensor& x) {
     return py::none();
   const Members norm(module.ptr());
   Tensor g;
-  if (!norm.parameter("g", g) || g.dim() != 1 || g.size(0) != x.size(-1) || !g.is_cuda()) return py::none();
+  if (!norm.parameter("g", g) || g.dim() != 1 || g.size(0) != x.size(-1) || !on_device_of(x, g)) return py::none();
   const bool bf16 = x.scalar_type() == at::kBFloat16;
   const int code = code_of(x.scalar_type());
   if (x.size(-1) > rglru_hip_rmsnorm_max_width(code, x.size(-1) % (bf16 ? 8 : 4) == 0)) return py::none();

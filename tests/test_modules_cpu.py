@@ -378,3 +378,73 @@ def test_stacked_halves_are_recognised_only_when_they_are_one_matrix():
     offset = torch.zeros(5 + 2 * 3 * 8)[5:].view(2, 3, 8)                 # a storage offset carries over
     got = _stacked_halves(offset[..., :4], offset[..., 4:])
     assert got is not None and got.storage_offset() == 5
+
+
+def test_operands_on_different_gpus_are_refused():
+    """The kernels take addresses, so an operand on another GPU is an error before anything is launched, or (the calls that may
+    decline) sends the caller to the general path, which reports it.  Fake tensors stand in for the second GPU."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from griffin_amd import _lib
+
+    native = _lib.native()
+    B, T, W, D, nb, K = 2, 6, 32, 16, 2, 4
+    f32, bf, byte = torch.float32, torch.bfloat16, torch.uint8
+
+    with FakeTensorMode():
+        def t(*shape, dtype=f32):
+            return torch.empty(*shape, device="cuda:0", dtype=dtype)
+
+        def block(dtype):
+            return [t(*s, dtype=dtype) for s in ((W, D), (W,), (W, D), (W,), (W, 1, K), (W,), (nb, W // nb, W // nb), (nb, W // nb),
+                                                 (nb, W // nb, W // nb), (nb, W // nb), (W,), (D, W), (D,))]
+
+        x, gates, pos = t(B, T, W), block(f32)[6:11], t(B, T, dtype=torch.long)
+        image, state = t(64, dtype=byte), t(B, W)
+        taps, bias, conv_state = t(W, 1, K), t(W), t(B, K - 1, W)
+        # operator, its operands by position, and those of them that have to be on x's device
+        raising = {
+            "rglru": ([x, *gates, state, t(B, T, dtype=byte), False, 8.0, 0], range(1, 8)),
+            "prepare": ([*gates, 8.0, f32], range(1, 5)),
+            "rglru_step": ([t(B, W), image, nb, state, t(B, dtype=byte)], (1, 3, 4)),
+            "rglru_steps": ([x, image, nb, state, None], (1, 3)),
+            "rglru_module_step": ([t(B, 1, W), image, nb, state, t(B, 1, dtype=byte)], (1, 3, 4)),
+            "scan": ([x, t(B, T, W), state], (1, 2)),
+            "causal_conv": ([x, conv_state, taps, bias, pos], (1, 2, 3)),
+            "causal_conv_padded": ([x, conv_state, taps, bias, pos, t(B, T, dtype=byte)], (1, 2, 3)),
+            "gelu_gate": ([x, t(B, T, W)], (1,)),
+            "block_forward": ([x, t(B, T, W), conv_state, taps, bias, pos, t(B, T, dtype=byte), False, *gates, state, 8.0, image, None, True],
+                              (1, 2, 3, 4, 6, 8, 9, 10, 11, 12, 13, 15)),
+            "block_decode_step": ([t(B, W), t(B, W), conv_state, taps, bias, t(B, dtype=torch.long), None, None, image, W, nb, f32, state],
+                                  (1, 2, 3, 4, 5, 8, 12)),
+            "linear": ([x, t(D, W), t(D), t(B, T, dtype=byte)], (1, 2, 3)),
+            "linear_pair": ([x, t(D, W), t(D), t(D, W), t(D)], (1, 2, 3, 4)),
+            "linear_pair_values": ([x, t(D, W), t(D), t(D, W), t(D)], (1, 2, 3, 4)),
+            "rmsnorm": ([x, t(W), 1e-6], (1,)),
+            "pack_flags": ([t(B, T, dtype=torch.bool), t(B, T, dtype=torch.bool)], (1,)),
+        }
+        for name, (args, places) in raising.items():
+            for at in places:
+                moved = list(args)
+                moved[at] = moved[at].to("cuda:1")
+                with pytest.raises(RuntimeError, match="same device"):
+                    getattr(native, name)(*moved)
+        xs = t(B, T, D, dtype=bf)
+        for name, args, places in (
+            ("block_train", [xs, block(bf), pos, t(B, T, dtype=byte), None, t(B, T, dtype=byte), None, None, False, 8.0], (2, 3, 5)),
+            ("block_infer", [xs, block(bf), image, conv_state.to(bf), state, t(B, dtype=torch.long), None, None, None, None, None, None, True], (2, 3, 4, 5)),
+        ):
+            for at in places:
+                moved = list(args)
+                moved[at] = moved[at].to("cuda:1")
+                assert getattr(native, name)(*moved) is None
+            for i in range(13):
+                p = block(bf)
+                p[i] = p[i].to("cuda:1")
+                assert getattr(native, name)(args[0], p, *args[2:]) is None
+        p = block(bf)
+        step = [t(B, 1, D, dtype=bf), *p[:6], *p[11:], conv_state.to(bf), t(B, dtype=torch.long), None, None, image, nb, state]
+        for at in (*range(1, 11), 13, 15):
+            moved = list(step)
+            moved[at] = moved[at].to("cuda:1")
+            assert native.block_step(*moved) is None
