@@ -1236,9 +1236,16 @@ struct Members {
     t = THPVariable_Unpack(p);
     return true;
   }
-  double number(const char* name, double otherwise) const {
+  // a plain number; anything else (an array scalar, a tensor, no such attribute) is left to the module's Python code
+  std::optional<double> number(const char* name) const {
     PyObject* v = at(name);
-    return v == nullptr ? otherwise : PyFloat_Check(v) ? PyFloat_AS_DOUBLE(v) : PyLong_Check(v) ? PyLong_AsDouble(v) : otherwise;
+    if (v == nullptr || !(PyFloat_Check(v) || PyLong_Check(v))) return std::nullopt;
+    const double d = PyFloat_AsDouble(v);
+    if (d == -1.0 && PyErr_Occurred()) {
+      PyErr_Clear();
+      return std::nullopt;
+    }
+    return d;
   }
   bool hooked() const {
     for (const char* name : {"_forward_hooks", "_forward_pre_hooks"}) {
@@ -1266,14 +1273,15 @@ const Stamp* current_stamp(const Members& lru, at::ScalarType dtype, c10::Device
       !lru.parameter("Lambda", p[4]))
     return nullptr;
   const Stamp* s = py::handle(held).cast<const Stamp*>();
-  return s->image.defined() && s->image.device() == device && s->holds(p, p.size(), lru.number("c", 0.0), dtype) ? s : nullptr;
+  const auto c = lru.number("c");
+  return c && s->image.defined() && s->image.device() == device && s->holds(p, p.size(), *c, dtype) ? s : nullptr;
 }
 
 // RG_LRU on one token per row without masks: (y, state).
 py::object lru_decode(py::handle module, const Tensor& x, const MaybeTensor& state) {
   if (at::GradMode::is_enabled() || x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0) return py::none();
   const Members lru(module.ptr());
-  if (x.size(2) != (int64_t)lru.number("rnn_width", -1) || !usable_mode(lru, x.device())) return py::none();
+  if (lru.number("rnn_width") != double(x.size(2)) || !usable_mode(lru, x.device())) return py::none();
   if (state.has_value() && (state->dim() != 2 || state->size(0) != x.size(0) || state->size(1) != x.size(2) || state->scalar_type() != at::kFloat ||
                             state->device() != x.device()))
     return py::none();
@@ -1298,7 +1306,9 @@ py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py
   if (!lx.parameter("weight", wx) || !lx.parameter("bias", bx) || !ly.parameter("weight", wy) || !ly.parameter("bias", by) ||
       !conv.parameter("weight", cw) || !conv.parameter("bias", cb) || !lo.parameter("weight", wo) || !lo.parameter("bias", bo))
     return py::none();
-  const int64_t B = x.size(0), W = (int64_t)block.number("rnn_width", -1), K = (int64_t)block.number("conv_kernel_size", -1);
+  const auto width = block.number("rnn_width"), taps = block.number("conv_kernel_size");
+  if (!width || !taps) return py::none();
+  const int64_t B = x.size(0), W = (int64_t)*width, K = (int64_t)*taps;
   if (wx.dim() != 2 || wx.size(0) != W || cw.dim() != 3 || cw.size(2) != K || wx.scalar_type() != x.scalar_type()) return py::none();
   MaybeTensor conv_state, prev, rnn;
   if (!cache.is_none()) {
@@ -2011,8 +2021,10 @@ py::object norm_forward(py::handle module, const Tensor& x) {
   const bool bf16 = x.scalar_type() == at::kBFloat16;
   const int code = code_of(x.scalar_type());
   if (x.size(-1) > rglru_hip_rmsnorm_max_width(code, x.size(-1) % (bf16 ? 8 : 4) == 0)) return py::none();
+  const auto eps = norm.number("eps");
+  if (!eps) return py::none();
   if (g.requires_grad() && at::GradMode::is_enabled()) hold_leaves(py::reinterpret_borrow<py::dict>(norm.dict), {g});
-  return py::cast(rmsnorm(x, g, norm.number("eps", 1e-6)));
+  return py::cast(rmsnorm(x, g, *eps));
 }
 
 }  // namespace

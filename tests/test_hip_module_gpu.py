@@ -2,6 +2,7 @@
 
 import copy
 
+import numpy as np
 import pytest
 import torch
 
@@ -996,3 +997,24 @@ def test_a_short_bias_of_a_linear_layer_is_refused():
         for pair in ((b, good), (good, b)):
             with pytest.raises(RuntimeError):
                 hip_linear_pair(x, w, pair[0], w, pair[1])
+
+
+def test_rmsnorm_takes_eps_as_it_is():
+    """An eps that is no plain number is not replaced by another one: array scalars and tensors count, a text is an error."""
+    from griffin_amd import RMSNorm
+
+    norm = RMSNorm(64, eps=0.5).cuda()
+    x = torch.randn(3, 64, device="cuda")
+    want = norm(x)
+    assert rel_err(want, x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 0.5)) < FP32_TOL
+    for eps in (np.float32(0.5), np.float64(0.5), torch.tensor(0.5)):
+        norm.eps = eps
+        assert torch.equal(norm(x), want), type(eps)
+    norm.eps = 1                                             # an integer is a number
+    assert rel_err(norm(x), x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1.0)) < FP32_TOL
+    norm.eps = "small"
+    with pytest.raises(TypeError):
+        norm(x)
+    del norm.eps
+    with pytest.raises(AttributeError):
+        norm(x)
