@@ -1247,7 +1247,9 @@ struct Members {
     }
     return d;
   }
+  // calling the layer does more than its class's forward: hooks, or a forward of its own
   bool hooked() const {
+    if (at("forward") != nullptr) return true;
     for (const char* name : {"_forward_hooks", "_forward_pre_hooks"}) {
       PyObject* h = at(name);
       if (h == nullptr || PyObject_Length(h) != 0) return true;

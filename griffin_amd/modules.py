@@ -19,8 +19,14 @@ import torch
 from torch import Tensor
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _nn_module
 
 from . import _lib, hip_block_ops, hip_scan, portable
+
+# What makes the call of a layer more than its class's forward: hooks for all modules, a forward patched into nn.Linear.
+_HOOKS_BEFORE, _HOOKS_AFTER = _nn_module._global_forward_pre_hooks, _nn_module._global_forward_hooks
+_HOOKS_BACKWARD = (_nn_module._global_backward_pre_hooks, _nn_module._global_backward_hooks)
+_LINEAR_FORWARD = nn.Linear.forward
 
 ScanMode = Literal["auto", "sequential", "associative", "hip", "fused"]
 SCAN_MODES = ("auto", "sequential", "associative", "hip", "fused")
@@ -518,8 +524,9 @@ class RecurrentBlock(nn.Module):
 
     @staticmethod
     def _is_plain(layer: nn.Module) -> bool:
-        """Nobody wrapped or hooked the Linear layer: calling it is a product with its weight and nothing else."""
-        return type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks
+        """Nobody wrapped, patched or hooked the Linear layer: calling it is a product with its weight and nothing else."""
+        return (type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks and "forward" not in layer.__dict__
+                and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD)
 
     def _own_parameters(self):
         """linear_x, linear_y, convolution, gates, Lambda, linear_out, or None where one is parametrised or otherwise replaced."""
@@ -533,7 +540,7 @@ class RecurrentBlock(nn.Module):
 
     def _whole_parameters(self, x: Tensor):
         """The block's parameters (linear_x, linear_y, convolution, gates, Lambda, linear_out) where one operator may stand for the
-        whole block: bf16 on the HIP path, nobody wrapped, hooked or replaced a layer; else None."""
+        whole block: bf16 on the HIP path, nobody wrapped, patched, hooked or replaced a layer; else None."""
         if x.dtype is not torch.bfloat16 or not x.is_cuda or x.numel() == 0 or torch.is_autocast_enabled():
             return None
         layers = self._modules
@@ -544,8 +551,10 @@ class RecurrentBlock(nn.Module):
         if mode not in ("auto", "hip", "fused"):
             return None
         for m in (lx, ly, conv, lo, lru):
-            if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or "forward" in m.__dict__:
                 return None
+        if _HOOKS_BEFORE or _HOOKS_AFTER or any(_HOOKS_BACKWARD) or nn.Linear.forward is not _LINEAR_FORWARD:
+            return None
         parameters = self._own_parameters()
         if parameters is None:
             return None
@@ -653,7 +662,8 @@ class RecurrentBlock(nn.Module):
     def forward(self, x: Tensor, cache: RecurrentBlockCache | None = None, segment_pos: Tensor | None = None,
                 *, active_mask: Tensor | None = None, return_cache: bool = False):
         native = _lib._native_module
-        if native is not None and segment_pos is None and active_mask is None and type(self) is RecurrentBlock and not torch.is_grad_enabled():
+        if (native is not None and segment_pos is None and active_mask is None and type(self) is RecurrentBlock and not torch.is_grad_enabled()
+                and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD):
             done = native.block_decode(self, x, cache, nn.Linear)    # one token per row, nothing unusual
             if done is not None:
                 output, rnn_state, conv_state, position = done

@@ -1018,3 +1018,46 @@ def test_rmsnorm_takes_eps_as_it_is():
     del norm.eps
     with pytest.raises(AttributeError):
         norm(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("how", ["global hook", "global pre-hook", "own forward", "class forward"])
+def test_hooked_and_patched_linear_layers_are_called(how, dtype, monkeypatch):
+    """Without gradients a block calls linear_out, and over whole sequences linear_x and linear_y, as modules wherever that is
+    more than their product: hooks for all modules, a forward patched into the layer or into nn.Linear."""
+    from torch.nn.modules import module as nn_module
+
+    from griffin_amd import RecurrentBlock
+
+    torch.manual_seed(0)
+    block = RecurrentBlock(64, 128, gate_blocks=2).to(dtype).cuda()
+    x = torch.randn(2, 9, 64, device="cuda", dtype=dtype)
+    mask = torch.ones(2, 9, dtype=torch.bool, device="cuda")
+    mask[1, 5:] = False
+    calls = {"prefill": (x, {}), "padded": (x, {"active_mask": mask}), "decode": (x[:, :1], {})}
+    names = {block.linear_x: "x", block.linear_y: "y", block.linear_out: "out"}
+    with torch.no_grad():
+        want = {k: block(t, **kw) for k, (t, kw) in calls.items()}
+        want = {k: block(t, **kw) for k, (t, kw) in calls.items()}      # the decode image is there
+        seen = []
+        handle = None
+        if how == "global hook":
+            handle = nn_module.register_module_forward_hook(lambda m, args, out: seen.append(names.get(m)))
+        elif how == "global pre-hook":
+            handle = nn_module.register_module_forward_pre_hook(lambda m, args: seen.append(names.get(m)))
+        elif how == "own forward":
+            for layer in names:
+                layer.forward = (lambda t, layer=layer: (seen.append(names[layer]), torch.nn.Linear.forward(layer, t))[1])
+        else:
+            plain = torch.nn.Linear.forward
+            monkeypatch.setattr(torch.nn.Linear, "forward", lambda self, t: (seen.append(names.get(self)), plain(self, t))[1])
+        try:
+            for kind, (t, kw) in calls.items():
+                del seen[:]
+                got = block(t, **kw)
+                expected = {"out"} if kind == "decode" else {"x", "y", "out"}
+                assert expected <= set(seen), (kind, seen)
+                assert rel_err(got.float(), want[kind].float()) < (FP32_TOL if dtype == torch.float32 else BF16_TOL)
+        finally:
+            if handle is not None:
+                handle.remove()
