@@ -1234,7 +1234,7 @@ struct Members {
     PyObject* p = in(at("_parameters"), name);
     if (p == nullptr || !THPVariable_Check(p)) return false;
     t = THPVariable_Unpack(p);
-    return true;
+    return !t.key_set().has(c10::DispatchKey::Python);        // a tensor that dispatches itself (quantised weights) has no plain memory
   }
   // a plain number; anything else (an array scalar, a tensor, no such attribute) is left to the module's Python code
   std::optional<double> number(const char* name) const {

@@ -27,6 +27,7 @@ from . import _lib, hip_block_ops, hip_scan, portable
 _HOOKS_BEFORE, _HOOKS_AFTER = _nn_module._global_forward_pre_hooks, _nn_module._global_forward_hooks
 _HOOKS_BACKWARD = (_nn_module._global_backward_pre_hooks, _nn_module._global_backward_hooks)
 _LINEAR_FORWARD = nn.Linear.forward
+_PLAIN_TENSORS = (nn.Parameter, Tensor)                      # and no subclass that stands for something else (quantised weights)
 
 ScanMode = Literal["auto", "sequential", "associative", "hip", "fused"]
 SCAN_MODES = ("auto", "sequential", "associative", "hip", "fused")
@@ -526,7 +527,8 @@ class RecurrentBlock(nn.Module):
     def _is_plain(layer: nn.Module) -> bool:
         """Nobody wrapped, patched or hooked the Linear layer: calling it is a product with its weight and nothing else."""
         return (type(layer) is nn.Linear and not layer._forward_hooks and not layer._forward_pre_hooks and "forward" not in layer.__dict__
-                and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD)
+                and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD
+                and all(p is None or type(p) in _PLAIN_TENSORS for p in layer._parameters.values()))
 
     def _own_parameters(self):
         """linear_x, linear_y, convolution, gates, Lambda, linear_out, or None where one is parametrised or otherwise replaced."""
@@ -559,7 +561,7 @@ class RecurrentBlock(nn.Module):
         if parameters is None:
             return None
         for p in parameters:
-            if p is None or p.dtype is not torch.bfloat16:
+            if p is None or p.dtype is not torch.bfloat16 or type(p) not in _PLAIN_TENSORS:
                 return None
         if not hip_block_ops.hip_block_forward_covers(self.rnn_width, parameters[6].shape[0], self.conv_kernel_size, torch.bfloat16):
             return None

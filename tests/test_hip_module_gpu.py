@@ -1061,3 +1061,40 @@ def test_hooked_and_patched_linear_layers_are_called(how, dtype, monkeypatch):
         finally:
             if handle is not None:
                 handle.remove()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_weights_that_dispatch_themselves_are_multiplied_by_pytorch(dtype):
+    """A weight that is a tensor subclass without memory of its own (quantised weights are such) goes through PyTorch's product in
+    a block without gradients, as it does in a plain nn.Linear."""
+    from torch.utils._pytree import tree_map
+
+    from griffin_amd import RecurrentBlock
+
+    class Wrapped(torch.Tensor):
+        @staticmethod
+        def __new__(cls, inner):
+            return torch.Tensor._make_wrapper_subclass(cls, inner.shape, dtype=inner.dtype, device=inner.device)
+
+        def __init__(self, inner):
+            self.inner = inner
+
+        __torch_function__ = torch._C._disabled_torch_function_impl
+
+        @classmethod
+        def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+            out = func(*tree_map(lambda t: t.inner if isinstance(t, cls) else t, args), **(kwargs or {}))
+            return cls(out) if func is torch.ops.aten.detach.default else out
+
+    torch.manual_seed(0)
+    block = RecurrentBlock(64, 128, gate_blocks=2).to(dtype).cuda().requires_grad_(False)
+    x = torch.randn(2, 9, 64, device="cuda", dtype=dtype)
+    mask = torch.ones(2, 9, dtype=torch.bool, device="cuda")
+    mask[1, 5:] = False
+    calls = [(x, {}), (x, {"active_mask": mask}), (x[:, :1], {})]
+    with torch.no_grad():
+        want = [block(t, **kw) for t, kw in calls]
+        want = [block(t, **kw) for t, kw in calls]
+        block.linear_out.weight = torch.nn.Parameter(Wrapped(block.linear_out.weight.detach()), requires_grad=False)
+        for (t, kw), expected in zip(calls, want):
+            assert rel_err(block(t, **kw).float(), expected.float()) < (FP32_TOL if dtype == torch.float32 else BF16_TOL)
