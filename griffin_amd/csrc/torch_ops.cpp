@@ -1550,13 +1550,15 @@ Tensor stacked_halves(const Tensor& a, const Tensor& b) {
 // Two Linear layers on one input (the block's two branches).  Their input gradients are one GEMM that accumulates into
 // the other's result instead of two results and an addition.
 struct LinearPair : torch::autograd::Function<LinearPair> {
+  typedef std::tuple<Tensor, Tensor> Values;
+  // `known`: the values, where the caller has them already
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2,
-                               const MaybeTensor& b2) {
+                               const MaybeTensor& b2, const Values* known) {
     ctx->save_for_backward({x, w1, w2});
     note_arguments(ctx, {true, true, b1.has_value(), true, b2.has_value()});
     pack(ctx, {type_or_none(opt(b1)), type_or_none(opt(b2))});
     ctx->set_materialize_grads(false);
-    auto [u, v] = values(x, w1, opt(b1), w2, opt(b2));
+    auto [u, v] = known != nullptr ? *known : values(x, w1, opt(b1), w2, opt(b2));
     return {u, v};
   }
   static bool own(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
@@ -1639,7 +1641,7 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
         if (grads[1].defined()) std::tie(dw2, db2) = linear_parameter_grads(x, w2.scalar_type(), grads[1], need_w2, need_b2 ? m[1] : kNone);
       }
     }
-    return once({dx, dw1, db1, dw2, db2});
+    return once({dx, dw1, db1, dw2, db2, Tensor()});
   }
 };
 
@@ -1652,13 +1654,21 @@ std::tuple<Tensor, Tensor> linear_pair_values(const Tensor& x, const Tensor& w1,
   return LinearPair::values(x, w1, opt(b1), w2, opt(b2));
 }
 
-std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const MaybeTensor& b1_, const Tensor& w2, const MaybeTensor& b2_) {
+std::tuple<Tensor, Tensor> linear_pair(const Tensor& x, const Tensor& w1, const MaybeTensor& b1_, const Tensor& w2, const MaybeTensor& b2_,
+                                       const MaybeTensor& u, const MaybeTensor& v) {
   Tensor b1 = opt(b1_), b2 = opt(b2_);
   require_gpu("hip_linear_pair", {&x, &w1, &b1, &w2, &b2});
   require_device_of("hip_linear_pair", x, {&w1, &b1, &w2, &b2});
   code_of(x.scalar_type());
-  if (!wants_grad({&x, &w1, &b1, &w2, &b2})) return linear_pair_values(x, w1, b1_, w2, b2_);
-  auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2));
+  TORCH_CHECK_VALUE(u.has_value() == v.has_value(), "hip_linear_pair expects both values or neither");
+  const bool known = u.has_value();
+  if (known)
+    for (const auto& [y, w] : {std::tie(*u, w1), std::tie(*v, w2)})
+      TORCH_CHECK_VALUE(!y.requires_grad() && y.numel() * x.size(-1) == x.numel() * w.size(0) && y.size(-1) == w.size(0) && y.scalar_type() == x.scalar_type(),
+                        "hip_linear_pair: these are not the values of the two products");
+  if (!wants_grad({&x, &w1, &b1, &w2, &b2})) return known ? std::make_tuple(*u, *v) : linear_pair_values(x, w1, b1_, w2, b2_);
+  const LinearPair::Values values = known ? std::make_tuple(*u, *v) : LinearPair::Values();
+  auto out = LinearPair::apply(x, w1, maybe(b1), w2, maybe(b2), known ? &values : nullptr);
   return {out[0], out[1]};
 }
 

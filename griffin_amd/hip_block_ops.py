@@ -187,10 +187,13 @@ def token_facts(active_mask: Tensor, segment_pos: Tensor | None, previous_positi
     return _lib.native().TokenFacts(active_mask, segment_pos, previous_position)
 
 
-def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None) -> tuple[Tensor, Tensor]:
+def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None,
+                    values: tuple[Tensor, Tensor] | None = None) -> tuple[Tensor, Tensor]:
     """``(x @ w1.T + b1, x @ w2.T + b2)``: two ``hip_linear`` calls whose backward passes share the input
-    gradient (the second GEMM accumulates into the first one's result)."""
-    return _lib.native().linear_pair(x, w1, b1, w2, b2)
+    gradient (the second GEMM accumulates into the first one's result).  ``values``: the two results of
+    ``hip_linear_pair_values`` on the same operands, which then only get their graph."""
+    u, v = (None, None) if values is None else values
+    return _lib.native().linear_pair(x, w1, b1, w2, b2, u, v)
 
 
 def hip_linear_pair_values(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None) -> tuple[Tensor, Tensor]:

@@ -571,8 +571,9 @@ class RecurrentBlock(nn.Module):
 
     def _infer_whole(self, x: Tensor, parameters, cache: RecurrentBlockCache | None, segment_pos: Tensor | None, active_mask: Tensor | None,
                      return_cache: bool):
-        """The block over sequences without gradients in one call of the library, or None where that does not take the
-        operands (or an operand has the wrong shape: the general path reports it)."""
+        """The block over sequences without gradients in one call of the library: (result, token facts, projections).  The result is
+        None where that does not take the operands (or an operand has the wrong shape: the general path reports it); the
+        other two are what the general path need not do again, or None."""
         batch, steps = x.shape[:2]
         device = x.device
         conv_state = rnn_state = previous = None
@@ -580,12 +581,12 @@ class RecurrentBlock(nn.Module):
             conv_state, rnn_state, previous = cache.conv_state, cache.rnn_state, cache.segment_position
             if (conv_state.shape != (batch, self.conv_kernel_size - 1, self.rnn_width) or previous.shape != (batch,)
                     or (rnn_state is not None and rnn_state.shape != (batch, self.rnn_width))):
-                return None
+                return None, None, None
         for t in (conv_state, rnn_state, previous, segment_pos):
             if t is not None and t.device != device:
-                return None
+                return None, None, None
         if segment_pos is not None and segment_pos.shape != (batch, steps):
-            return None
+            return None, None, None
         u = v = flags = rows = live = facts = None
         if active_mask is not None:
             facts = hip_block_ops.token_facts(active_mask, segment_pos, previous)
@@ -597,21 +598,21 @@ class RecurrentBlock(nn.Module):
             elif right_padded:
                 flags, rows, live = facts.flags, facts.rows, active_mask
             else:
-                return None
+                return None, facts, (u, v)
         done = hip_block_ops.hip_block_infer(x, parameters, self._modules["rg_lru"]._prepared(x.dtype, device), conv_state, rnn_state, previous,
                                              segment_pos, flags, rows, live, u, v, return_cache)
         if done is None:
-            return None
+            return None, facts, None if u is None else (u, v)
         output, new_rnn_state, new_conv_state, last_position = done
         if not return_cache:
-            return output
-        return output, RecurrentBlockCache(new_rnn_state, new_conv_state, last_position if facts is None else facts.last_position)
+            return output, None, None
+        return (output, RecurrentBlockCache(new_rnn_state, new_conv_state, last_position if facts is None else facts.last_position)), None, None
 
-    def _train_whole(self, x: Tensor, parameters, segment_pos: Tensor | None, active_mask: Tensor | None) -> Tensor | None:
-        """The block as one operator (``around`` of hip_block_ops.hip_block_forward), or None where that does not take the
-        operands."""
+    def _train_whole(self, x: Tensor, parameters, segment_pos: Tensor | None, active_mask: Tensor | None):
+        """The block as one operator (``around`` of hip_block_ops.hip_block_forward): (result, token facts, projections), as
+        _infer_whole returns them."""
         w_u, b_u, w_v, b_v, taps, conv_bias, w_a, b_a, w_x, b_x, lam, w_o, b_o = parameters
-        u = v = rows = flags = live = None
+        u = v = rows = flags = live = facts = None
         if active_mask is None:
             if segment_pos is None:
                 flags = hip_scan.FIRST_TOKEN_RESET
@@ -626,9 +627,10 @@ class RecurrentBlock(nn.Module):
             elif right_padded:
                 positions, flags, rows, live = facts.conv_positions, facts.flags, facts.rows, active_mask
             else:
-                return None
-        return hip_block_ops.hip_block_forward(u, v, None, taps, conv_bias, positions, flags, w_a, b_a, w_x, b_x, lam, None,
+                return None, facts, (u, v)
+        done = hip_block_ops.hip_block_forward(u, v, None, taps, conv_bias, positions, flags, w_a, b_a, w_x, b_x, lam, None,
                                                self.rg_lru.c, None, rows, False, (x, w_u, b_u, w_v, b_v, w_o, b_o, live))[0]
+        return done, facts, None if u is None else (u, v)
 
     def _dense_conv(self, projected: Tensor, conv_state: Tensor | None, segment_pos: Tensor, need_state: bool = True):
         """All-tokens-active path (griffin/griffin.py:476-487): taps are masked per document."""
@@ -682,22 +684,24 @@ class RecurrentBlock(nn.Module):
         if steps == 1 and self._hip_decode_covers(x, cache):
             return self._hip_decode(x, cache, segment_pos, active_mask, return_cache)
         parameters = self._whole_parameters(x) if steps > 0 else None
+        facts = projections = None
         if parameters is not None:
             result = None
             carried = () if cache is None else (cache.rnn_state, cache.conv_state)
             if not torch.is_grad_enabled() or not any(t is not None and t.requires_grad for t in (x, *parameters, *carried)):
-                result = self._infer_whole(x, parameters, cache, segment_pos, active_mask, return_cache)
+                result, facts, projections = self._infer_whole(x, parameters, cache, segment_pos, active_mask, return_cache)
             elif cache is None and not return_cache:
                 _lib.native().hold_leaves(self.__dict__, parameters)
-                result = self._train_whole(x, parameters, segment_pos, active_mask)
+                result, facts, projections = self._train_whole(x, parameters, segment_pos, active_mask)
             if result is not None:
                 return result
         elif torch.is_grad_enabled() and self._hip_block_ops_covers(x):
             held = self._own_parameters()
             if held is not None:
                 _lib.native().hold_leaves(self.__dict__, [p for p in held if p is not None])
-        facts = None
-        if not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
+        if facts is not None:
+            segment_pos = facts.positions
+        elif not everything_active and x.is_cuda and steps > 0 and self._hip_block_ops_covers(x):
             # launched in front of the projections, so that its answer is there before they are done
             facts = hip_block_ops.token_facts(active_mask, segment_pos, previous_position)
             segment_pos = facts.positions
@@ -705,10 +709,12 @@ class RecurrentBlock(nn.Module):
             segment_pos = _resolve_segment_positions(
                 x, segment_pos, previous_position, None if everything_active else active_mask)
 
-        if (self._linear_on_hip(self.linear_x, x) and self._linear_on_hip(self.linear_y, x)) or (
+        if projections is not None and not torch.is_grad_enabled():
+            projected, gate_input = projections
+        elif projections is not None or (self._linear_on_hip(self.linear_x, x) and self._linear_on_hip(self.linear_y, x)) or (
                 self._inference_on_hip(self.linear_x, x) and self._inference_on_hip(self.linear_y, x)):
             projected, gate_input = hip_block_ops.hip_linear_pair(
-                x, self.linear_x.weight, self.linear_x.bias, self.linear_y.weight, self.linear_y.bias)
+                x, self.linear_x.weight, self.linear_x.bias, self.linear_y.weight, self.linear_y.bias, projections)
         else:
             gate_input = self._linear(self.linear_y, x)
             projected = self._linear(self.linear_x, x)

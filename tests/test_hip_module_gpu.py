@@ -1098,3 +1098,57 @@ def test_weights_that_dispatch_themselves_are_multiplied_by_pytorch(dtype):
         block.linear_out.weight = torch.nn.Parameter(Wrapped(block.linear_out.weight.detach()), requires_grad=False)
         for (t, kw), expected in zip(calls, want):
             assert rel_err(block(t, **kw).float(), expected.float()) < (FP32_TOL if dtype == torch.float32 else BF16_TOL)
+
+
+@pytest.mark.parametrize("mask_kind", ["left", "holes", "right", "dense"])
+@pytest.mark.parametrize("train", [False, True])
+def test_masked_block_does_nothing_twice(train, mask_kind, monkeypatch):
+    """One look at the mask and one pair of input projections, whichever path the mask then leads to; results and gradients are
+    those of the general path on its own."""
+    from griffin_amd import RecurrentBlock, hip_block_ops, set_reproducible
+
+    torch.manual_seed(0)
+    block = RecurrentBlock(64, 128, gate_blocks=2).bfloat16().cuda()
+    x = torch.randn(3, 41, 64, device="cuda", dtype=torch.bfloat16, requires_grad=train)
+    mask = torch.ones(3, 41, dtype=torch.bool, device="cuda")
+    if mask_kind == "left":
+        mask[1, :7] = False
+    elif mask_kind == "holes":
+        mask[0, 5:9] = False
+        mask[2, 30] = False
+    elif mask_kind == "right":
+        mask[1, 20:] = False
+    dy = torch.randn_like(x)
+    count = {}
+
+    def spy(name):
+        plain = getattr(hip_block_ops, name)
+
+        def call(*args, **kwargs):
+            # a pair that only gives known values their graph computes nothing
+            known = name == "hip_linear_pair" and len(args) > 5 and args[5] is not None
+            count[name] = count.get(name, 0) + (not known)
+            return plain(*args, **kwargs)
+        monkeypatch.setattr(hip_block_ops, name, call)
+
+    def run():
+        with torch.set_grad_enabled(train):
+            y = block(x, active_mask=mask)
+        return (y.detach(), *torch.autograd.grad(y, [x, *block.parameters()], dy)) if train else (y,)
+
+    was = set_reproducible(True)
+    try:
+        for name in ("token_facts", "hip_linear_pair_values", "hip_linear_pair"):
+            spy(name)
+        got = run()
+        assert count.pop("token_facts") == 1
+        assert sum(count.values()) <= 1, count
+        monkeypatch.setattr(RecurrentBlock, "_whole_parameters", lambda self, x: None)
+        want = run()
+    finally:
+        set_reproducible(was)
+    for name, a, b in zip(("y", "x", *(n for n, _ in block.named_parameters())), got, want):
+        if mask_kind in ("left", "holes"):                   # the same path from here on
+            assert torch.equal(a, b), name
+        else:
+            assert rel_err(a.float(), b.float()) < BF16_TOL, name

@@ -418,7 +418,7 @@ def test_operands_on_different_gpus_are_refused():
             "block_decode_step": ([t(B, W), t(B, W), conv_state, taps, bias, t(B, dtype=torch.long), None, None, image, W, nb, f32, state],
                                   (1, 2, 3, 4, 5, 8, 12)),
             "linear": ([x, t(D, W), t(D), t(B, T, dtype=byte)], (1, 2, 3)),
-            "linear_pair": ([x, t(D, W), t(D), t(D, W), t(D)], (1, 2, 3, 4)),
+            "linear_pair": ([x, t(D, W), t(D), t(D, W), t(D), None, None], (1, 2, 3, 4)),
             "linear_pair_values": ([x, t(D, W), t(D), t(D, W), t(D)], (1, 2, 3, 4)),
             "rmsnorm": ([x, t(W), 1e-6], (1,)),
             "pack_flags": ([t(B, T, dtype=torch.bool), t(B, T, dtype=torch.bool)], (1,)),
