@@ -72,7 +72,39 @@ class BlockDiagonalLinear(nn.Module):
         return portable.block_diagonal_project(x, self.weight, self.bias)
 
 
-class RG_LRU(nn.Module):
+class _HoldsLeaves(nn.Module):
+    """A module whose training steps hold the ends of the autograd graph at its parameters (csrc/torch_ops.cpp, Leaves).  An end
+    keeps its parameter and that one's gradient alive, so it is dropped where parameters are replaced (assigned, loaded,
+    converted), between training and evaluation, and by every forward pass without gradients.  What it cannot see, a parameter
+    assigned to a layer inside, lasts until the next of these or the next training step."""
+
+    def __setattr__(self, name, value):
+        if isinstance(value, (nn.Parameter, nn.Module)):
+            self.__dict__["_leaves"] = None
+        super().__setattr__(name, value)
+
+    def __delattr__(self, name):
+        self.__dict__["_leaves"] = None
+        super().__delattr__(name)
+
+    def _drop_leaves_without_gradients(self):
+        if not torch.is_grad_enabled() and self.__dict__.get("_leaves") is not None:
+            self.__dict__["_leaves"] = None
+
+    def _apply(self, fn, *args, **kwargs):
+        self.__dict__["_leaves"] = None
+        return super()._apply(fn, *args, **kwargs)
+
+    def train(self, mode: bool = True):
+        self.__dict__["_leaves"] = None
+        return super().train(mode)
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        self.__dict__["_leaves"] = None
+        return super()._load_from_state_dict(*args, **kwargs)
+
+
+class RG_LRU(_HoldsLeaves):
     """Real-Gated Linear Recurrent Unit (griffin/griffin.py:157-306) with a HIP scan backend."""
 
     def __init__(self, rnn_width: int, c: float = 8.0, gate_blocks: int = 16, scan_mode: ScanMode = "auto"):
@@ -163,6 +195,7 @@ class RG_LRU(nn.Module):
         active_mask: Tensor | None = None,
         return_state: bool = False,
     ):
+        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if native is not None and reset_mask is None and active_mask is None and type(self) is RG_LRU and not torch.is_grad_enabled():
             done = native.lru_decode(self, xt, ht_minus_1)   # one token per row, nothing unusual
@@ -307,7 +340,7 @@ def _last_active_position(segment_pos: Tensor, active_mask: Tensor, previous_pos
     return torch.where(last >= 0, picked, fallback)
 
 
-class RMSNorm(nn.Module):
+class RMSNorm(_HoldsLeaves):
     """Root-mean-square normalisation with a learned per-channel scale (griffin/griffin.py:68-80), the
     layer in front of the recurrent block.  GPU tensors the HIP library covers go through its kernels
     (after the same per-device self-test as ``scan_mode="auto"``); everything else through PyTorch."""
@@ -316,10 +349,6 @@ class RMSNorm(nn.Module):
         super().__init__()
         self.eps = eps
         self.g = nn.Parameter(torch.zeros(dim))
-
-    def _apply(self, fn, *args, **kwargs):
-        self._leaves = None
-        return super()._apply(fn, *args, **kwargs)
 
     def _hip_covers(self, x: Tensor) -> bool:
         if not x.is_cuda or x.dtype not in hip_scan.SUPPORTED_DTYPES or x.numel() == 0:
@@ -330,6 +359,7 @@ class RMSNorm(nn.Module):
         return x.size(-1) <= hip_block_ops.rmsnorm_max_width(x.dtype, aligned)
 
     def forward(self, x: Tensor) -> Tensor:
+        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if native is not None:
             done = native.norm_forward(self, x)
@@ -344,7 +374,7 @@ class RMSNorm(nn.Module):
 _BLOCK_LAYERS = ("linear_x", "linear_y", "temporal_conv", "linear_out", "rg_lru")
 
 
-class RecurrentBlock(nn.Module):
+class RecurrentBlock(_HoldsLeaves):
     """Linear -> causal depthwise conv -> RG-LRU, gated by GeLU(Linear), then Linear out
     (griffin/griffin.py:361-529).  The RG-LRU inside honours ``scan_mode`` unchanged."""
 
@@ -384,7 +414,6 @@ class RecurrentBlock(nn.Module):
 
     def _apply(self, fn, *args, **kwargs):
         self._stacked_projection = None
-        self._leaves = None
         return super()._apply(fn, *args, **kwargs)
 
     def train(self, mode: bool = True):
@@ -665,6 +694,7 @@ class RecurrentBlock(nn.Module):
 
     def forward(self, x: Tensor, cache: RecurrentBlockCache | None = None, segment_pos: Tensor | None = None,
                 *, active_mask: Tensor | None = None, return_cache: bool = False):
+        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if (native is not None and segment_pos is None and active_mask is None and type(self) is RecurrentBlock and not torch.is_grad_enabled()
                 and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD):

@@ -1152,3 +1152,47 @@ def test_masked_block_does_nothing_twice(train, mask_kind, monkeypatch):
             assert torch.equal(a, b), name
         else:
             assert rel_err(a.float(), b.float()) < BF16_TOL, name
+
+
+@pytest.mark.parametrize("how", ["assign", "load", "to", "eval", "inference"])
+@pytest.mark.parametrize("what", ["norm", "layer", "block", "block fp32"])
+def test_replaced_parameters_are_not_kept_alive(what, how):
+    """The graph ends that a module holds between training steps do not outlive a replaced parameter: at once where the module
+    itself sees it replaced (assigned, loaded, converted), else with eval() or the next forward without gradients."""
+    import gc
+    import weakref
+
+    from griffin_amd import RG_LRU, RMSNorm, RecurrentBlock
+
+    dtype = torch.bfloat16 if what == "block" else torch.float32
+    module = {"norm": lambda: RMSNorm(64), "layer": lambda: RG_LRU(64, gate_blocks=2)}.get(what, lambda: RecurrentBlock(64, 128, gate_blocks=2))()
+    module.cuda().to(dtype)
+    x = torch.randn(2, 9, 64, device="cuda", dtype=dtype)
+    module(x).float().sum().backward()
+    assert module.__dict__.get("_leaves") is not None
+    old = [weakref.ref(p) for p in module.parameters()]
+    if how == "assign":
+        for name, p in list(module._parameters.items()):
+            setattr(module, name, torch.nn.Parameter(torch.randn_like(p)))
+        for name, m in list(module.named_children()):
+            setattr(module, name, copy.deepcopy(m))
+    elif how == "load":
+        module.load_state_dict({k: torch.randn_like(v) for k, v in module.state_dict().items()}, assign=True)
+    elif how == "to":
+        torch.__future__.set_overwrite_module_params_on_conversion(True)
+        try:
+            module.to(torch.float16)
+        finally:
+            torch.__future__.set_overwrite_module_params_on_conversion(False)
+    else:
+        for m in module.modules():
+            for name, p in list(m._parameters.items()):
+                setattr(m, name, torch.nn.Parameter(torch.randn_like(p)))
+        if how == "eval":
+            module.eval()
+        else:
+            with torch.no_grad():
+                module(x)
+    p = m = None
+    gc.collect()
+    assert all(ref() is None for ref in old)
