@@ -1229,6 +1229,11 @@ struct Members {
   }
   PyObject* at(const char* name) const { return dict != nullptr ? PyDict_GetItemString(dict, name) : nullptr; }
   static PyObject* in(PyObject* d, const char* name) { return d != nullptr && PyDict_Check(d) ? PyDict_GetItemString(d, name) : nullptr; }
+  // a pass without gradients: the graph ends held for training keep nothing alive meanwhile
+  void drop_leaves() const {
+    PyObject* held = at("_leaves");
+    if (held != nullptr && held != Py_None) PyDict_SetItemString(dict, "_leaves", Py_None);
+  }
   PyObject* module(const char* name) const { return in(at("_modules"), name); }
   bool parameter(const char* name, Tensor& t) const {
     PyObject* p = in(at("_parameters"), name);
@@ -1281,8 +1286,10 @@ const Stamp* current_stamp(const Members& lru, at::ScalarType dtype, c10::Device
 
 // RG_LRU on one token per row without masks: (y, state).
 py::object lru_decode(py::handle module, const Tensor& x, const MaybeTensor& state) {
-  if (at::GradMode::is_enabled() || x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0) return py::none();
+  if (at::GradMode::is_enabled()) return py::none();
   const Members lru(module.ptr());
+  lru.drop_leaves();
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0) return py::none();
   if (lru.number("rnn_width") != double(x.size(2)) || !usable_mode(lru, x.device())) return py::none();
   if (state.has_value() && (state->dim() != 2 || state->size(0) != x.size(0) || state->size(1) != x.size(2) || state->scalar_type() != at::kFloat ||
                             state->device() != x.device()))
@@ -1295,10 +1302,11 @@ py::object lru_decode(py::handle module, const Tensor& x, const MaybeTensor& sta
 
 // RecurrentBlock on one token per row, every row active, positions carried on: (output, rnn_state, conv_state, positions).
 py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py::handle linear_type) {
-  if (at::GradMode::is_enabled() || x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0 ||
-      at::autocast::is_autocast_enabled(at::kCUDA))
-    return py::none();
+  if (at::GradMode::is_enabled()) return py::none();
   const Members block(module.ptr());
+  block.drop_leaves();
+  if (x.dim() != 3 || x.size(1) != 1 || !x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0 || at::autocast::is_autocast_enabled(at::kCUDA))
+    return py::none();
   PyObject* layers[4] = {block.module("linear_x"), block.module("linear_y"), block.module("linear_out"), block.module("temporal_conv")};
   for (int i = 0; i < 3; ++i)
     if (layers[i] == nullptr || (PyObject*)Py_TYPE(layers[i]) != linear_type.ptr()) return py::none();
@@ -2028,6 +2036,7 @@ py::object norm_forward(py::handle module, const Tensor& x) {
   if (!x.is_cuda() || !known(x.scalar_type()) || x.numel() == 0 || x.dim() < 1 || !((usable_devices.load(std::memory_order_relaxed) >> x.device().index()) & 1))
     return py::none();
   const Members norm(module.ptr());
+  if (!at::GradMode::is_enabled()) norm.drop_leaves();
   Tensor g;
   if (!norm.parameter("g", g) || g.dim() != 1 || g.size(0) != x.size(-1) || !on_device_of(x, g)) return py::none();
   const bool bf16 = x.scalar_type() == at::kBFloat16;

@@ -87,10 +87,6 @@ class _HoldsLeaves(nn.Module):
         self.__dict__["_leaves"] = None
         super().__delattr__(name)
 
-    def _drop_leaves_without_gradients(self):
-        if not torch.is_grad_enabled() and self.__dict__.get("_leaves") is not None:
-            self.__dict__["_leaves"] = None
-
     def _apply(self, fn, *args, **kwargs):
         self.__dict__["_leaves"] = None
         return super()._apply(fn, *args, **kwargs)
@@ -195,7 +191,6 @@ class RG_LRU(_HoldsLeaves):
         active_mask: Tensor | None = None,
         return_state: bool = False,
     ):
-        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if native is not None and reset_mask is None and active_mask is None and type(self) is RG_LRU and not torch.is_grad_enabled():
             done = native.lru_decode(self, xt, ht_minus_1)   # one token per row, nothing unusual
@@ -237,6 +232,8 @@ class RG_LRU(_HoldsLeaves):
                     f'scan_mode="{mode}" requires CUDA/HIP tensors and the RG-LRU HIP library; '
                     f"got a {xt.device.type} tensor"
                 )
+            if not torch.is_grad_enabled():
+                self.__dict__["_leaves"] = None
             if steps == 1 and not self._needs_grad(xt, ht_minus_1):
                 # decode: the single-step kernel on a prepared parameter image kept between calls
                 prep = self._prepared(xt.dtype, device)
@@ -359,7 +356,6 @@ class RMSNorm(_HoldsLeaves):
         return x.size(-1) <= hip_block_ops.rmsnorm_max_width(x.dtype, aligned)
 
     def forward(self, x: Tensor) -> Tensor:
-        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if native is not None:
             done = native.norm_forward(self, x)
@@ -694,7 +690,6 @@ class RecurrentBlock(_HoldsLeaves):
 
     def forward(self, x: Tensor, cache: RecurrentBlockCache | None = None, segment_pos: Tensor | None = None,
                 *, active_mask: Tensor | None = None, return_cache: bool = False):
-        self._drop_leaves_without_gradients()
         native = _lib._native_module
         if (native is not None and segment_pos is None and active_mask is None and type(self) is RecurrentBlock and not torch.is_grad_enabled()
                 and not _HOOKS_BEFORE and not _HOOKS_AFTER and nn.Linear.forward is _LINEAR_FORWARD):
@@ -711,6 +706,8 @@ class RecurrentBlock(_HoldsLeaves):
                 raise ValueError("active_mask must match the input [batch, sequence] dimensions")
             active_mask = active_mask.to(device=x.device, dtype=torch.bool)
         previous_position = None if cache is None else cache.segment_position
+        if not torch.is_grad_enabled():
+            self.__dict__["_leaves"] = None
         if steps == 1 and self._hip_decode_covers(x, cache):
             return self._hip_decode(x, cache, segment_pos, active_mask, return_cache)
         parameters = self._whole_parameters(x) if steps > 0 else None
