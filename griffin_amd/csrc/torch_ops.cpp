@@ -3,7 +3,7 @@
 // Why native: a training step of a small layer is a handful of launches of 3-10 us, and the same glue in Python
 // (autograd.Function, one torch.empty per buffer, ctypes calls of twenty arguments) kept the host busy for 190 us of
 // a 50 us step and 790 us of a 560 us block step.  Here an operator costs its allocations and launches.
-// Buffers that live and die together are parts of one allocation.
+// Scratch buffers that live and die together are parts of one allocation.
 //
 // Errors follow the reference's operator module (griffin/triton_scan.py:213-224): RuntimeError for a missing GPU,
 // ValueError for shapes, TypeError for types.
@@ -121,8 +121,9 @@ Tensor part(const Tensor& buffer, size_t at, at::IntArrayRef size, at::ScalarTyp
   return t;
 }
 
-// Tensors that live as long as each other, as parts of one allocation: first their sizes, then the memory, then the tensors
-// in the same order.
+// Scratch areas that live as long as each other, as parts of one allocation: first their sizes, then the memory, then the
+// addresses in the same order.  What a caller gets to keep is not such a part: keeping or saving one would keep or save all.
+// Carried state is tensors of their own; gradients share memory with their like at most (see take_gates).
 struct Parts {
   std::vector<size_t> offsets;
   size_t total = 0, next = 0;
@@ -130,7 +131,6 @@ struct Parts {
   void add(size_t n) { offsets.push_back(total), total += round_up(n); }
   void allocate(const Tensor& like) { buffer = bytes(total, like); }
   char* raw() { return static_cast<char*>(buffer.data_ptr()) + offsets[next++]; }
-  Tensor take(at::IntArrayRef size, at::ScalarType dtype) { return part(buffer, offsets[next++], size, dtype); }
 };
 
 // Contiguous and on a 16-byte boundary (what every fresh allocation is): a view at an odd offset costs one copy
@@ -287,6 +287,18 @@ struct ParamGrads {
   Tensor dx, dw_a, db_a, dw_x, db_x, dlam, dh0;
 };
 
+// The gates' gradients, the two weights in one allocation and the three vectors in another: memory that the backward's thread
+// allocates and the caller's frees costs the host 2 to 3 us (layer B2 T256 W256 fp32: 91 us a step with all five in one, 94 so,
+// 103 with five allocations).
+void take_gates(int64_t nb, int64_t bw, at::ScalarType dtype, const Tensor& like, Tensor& dw_a, Tensor& db_a, Tensor& dw_x, Tensor& db_x,
+                Tensor& dlam) {
+  const int64_t W = nb * bw;
+  const size_t es = c10::elementSize(dtype), weight = round_up(W * bw * es), vector = round_up(W * es);
+  Tensor weights = bytes(2 * weight, like), vectors = bytes(3 * vector, like);
+  dw_a = part(weights, 0, {nb, bw, bw}, dtype), dw_x = part(weights, weight, {nb, bw, bw}, dtype);
+  db_a = part(vectors, 0, {nb, bw}, dtype), db_x = part(vectors, vector, {nb, bw}, dtype), dlam = part(vectors, 2 * vector, {W}, dtype);
+}
+
 // Backward pass of the RG-LRU on what its forward kept; the parameter gradients come back in the parameters' types
 // (w_a, b_a, w_x, b_x, lam).
 ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Tensor& h0, const Tensor& flags, bool first_reset,
@@ -307,14 +319,7 @@ ParamGrads rglru_backward(const Tensor& x, const Tensor& y, int64_t nb, const Te
   if (!known(gt)) gt = at::kFloat;
   const int gcode = code_of(gt) | (ws_clear ? RGLRU_BACKWARD_CLEAR : 0);
   g.dx = fresh_like(x);
-  {
-    const size_t gs = c10::elementSize(gt);
-    Parts parts;
-    parts.add(W * bw * gs), parts.add(W * bw * gs), parts.add(W * gs), parts.add(W * gs), parts.add(W * gs);
-    parts.allocate(x);
-    g.dw_a = parts.take({nb, bw, bw}, gt), g.dw_x = parts.take({nb, bw, bw}, gt);
-    g.db_a = parts.take({nb, bw}, gt), g.db_x = parts.take({nb, bw}, gt), g.dlam = parts.take({W}, gt);
-  }
+  take_gates(nb, bw, gt, x, g.dw_a, g.db_a, g.dw_x, g.db_x, g.dlam);
   if (need_dh0) g.dh0 = fresh({B, W}, at::kFloat, x);
   void* stream = stream_of(x);
   const uint8_t* fl = flags_ptr(flags, first_reset);
@@ -1188,10 +1193,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
   Tensor x = x_in;
   if (x.stride(2) != 1 || (x.stride(0) * x.element_size()) % 16 || !is_aligned(x)) x = aligned(x);
   Tensor h_in = rnn_state.defined() ? as(rnn_state, at::kFloat) : at::zeros({B, W}, x.options().dtype(at::kFloat));
-  Parts cache;                                             // what the next step reads: the three live as long as each other
-  cache.add(B * W * 4), cache.add(B * (K - 1) * W * x.element_size()), cache.add(B * 8);
-  cache.allocate(x);
-  Tensor h_out = cache.take({B, W}, at::kFloat), new_conv = cache.take({B, K - 1, W}, dtype), new_pos = cache.take({B}, at::kLong);
+  Tensor h_out = fresh({B, W}, at::kFloat, x), new_conv = fresh({B, K - 1, W}, dtype, x), new_pos = fresh({B}, at::kLong, x);
   Tensor out = fresh({B, 1, D}, dtype, x);
   // x after the convolution, the second branch, their product with the state, one flag byte per row
   const size_t row_bytes = round_up(B * W * x.element_size());
@@ -1505,11 +1507,10 @@ struct Linear : torch::autograd::Function<Linear> {
     }
     if (need_w || need_b) {
       const WeightGrad wg(rows, N, K, 1, dtype);
-      Parts out, scratch;
-      out.add(N * K * x.element_size()), out.add(N * x.element_size());
+      Parts scratch;
       scratch.add(wg.sets_bytes), scratch.add(wg.sums_bytes);
-      out.allocate(x), scratch.allocate(x);
-      dw = out.take({N, K}, dtype), db = out.take({N}, dtype);
+      scratch.allocate(x);
+      dw = fresh({N, K}, dtype, x), db = fresh({N}, dtype, x);
       char *sets = scratch.raw(), *sums = scratch.raw();
       wg.run(ptr(dy), nullptr, N, ptr(x), bptr(active), ptr(dw), sets, sums, rows, dtype, stream);
       const rglru_sum jobs[] = {wg.weight_sum(sets, ptr(dw)), wg.bias_sum(sums, ptr(db))};
@@ -1609,20 +1610,18 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
         }
         if (need_w1 || need_w2 || need_b1 || need_b2) {
           const WeightGrad wg(rows, N, K, 2, dtype);
-          Parts out, scratch;
-          out.add(2 * N * K * x.element_size()), out.add(2 * N * x.element_size());
+          Parts scratch;
           scratch.add(wg.sets_bytes), scratch.add(wg.sums_bytes);
-          out.allocate(x), scratch.allocate(x);
-          Tensor dw = out.take({2, N, K}, dtype), db = out.take({2, N}, dtype);
+          scratch.allocate(x);
+          Tensor dw = fresh({2, N, K}, dtype, x), db = fresh({2, N}, dtype, x);      // the halves of one sum
           char *sets = scratch.raw(), *sums = scratch.raw();
           wg.run(ptr(g0), ptr(g1), ld, ptr(x), nullptr, ptr(dw), sets, sums, rows, dtype, stream);
           const rglru_sum jobs[] = {wg.weight_sum(sets, ptr(dw)), wg.bias_sum(sums, ptr(db))};
           check(rglru_hip_sums(jobs, 2, code, stream), "rglru_hip_sums");
-          const size_t at_b = round_up(2 * N * K * x.element_size()), row = N * x.element_size();
-          if (need_w1) dw1 = part(out.buffer, 0, {N, K}, dtype);
-          if (need_w2) dw2 = part(out.buffer, N * K * x.element_size(), {N, K}, dtype);
-          if (need_b1) db1 = part(out.buffer, at_b, {N}, dtype);
-          if (need_b2) db2 = part(out.buffer, at_b + row, {N}, dtype);
+          if (need_w1) dw1 = part(dw, 0, {N, K}, dtype);
+          if (need_w2) dw2 = part(dw, N * K * x.element_size(), {N, K}, dtype);
+          if (need_b1) db1 = part(db, 0, {N}, dtype);
+          if (need_b2) db2 = part(db, N * x.element_size(), {N}, dtype);
         }
       } else if (both.defined() && w1.scalar_type() == w2.scalar_type() && w1.sizes() == w2.sizes() && need_w1 == need_w2 &&
           need_b1 == need_b2 && m[0] == m[1]) {
@@ -1767,18 +1766,13 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       const bool own = !m[2];
       if (!own && active.defined()) dy = masked_rows(dy, active, false);
 
-      // parameter gradients: parts of one allocation
-      Parts out;
-      for (int64_t n : {2 * W * D, 2 * W, W * K, W, W * bw, W, W * bw, W, W, D * W, D}) out.add(n * 2);
-      out.allocate(x);
-      Tensor dw_pair = out.take({2, W, D}, kType);
-      out.next++;                                          // the two bias gradients: g[BX], g[BY]
-      g[CW] = out.take({W, 1, K}, kType), g[CB] = out.take({W}, kType);
-      g[WA] = out.take({nb, bw, bw}, kType), g[BA] = out.take({nb, bw}, kType), g[WI] = out.take({nb, bw, bw}, kType), g[BI] = out.take({nb, bw}, kType);
-      g[LAM] = out.take({W}, kType);
-      g[WO] = out.take({D, W}, kType), g[BO] = out.take({D}, kType);
-      g[WX] = part(out.buffer, out.offsets[0], {W, D}, kType), g[WY] = part(out.buffer, out.offsets[0] + W * D * 2, {W, D}, kType);
-      g[BX] = part(out.buffer, out.offsets[1], {W}, kType), g[BY] = part(out.buffer, out.offsets[1] + W * 2, {W}, kType);
+      // parameter gradients; those of the two input projections are the halves of one sum each
+      Tensor dw_pair = fresh({2, W, D}, kType, x), db_pair = fresh({2, W}, kType, x);
+      g[WX] = part(dw_pair, 0, {W, D}, kType), g[WY] = part(dw_pair, W * D * 2, {W, D}, kType);
+      g[BX] = part(db_pair, 0, {W}, kType), g[BY] = part(db_pair, W * 2, {W}, kType);
+      g[CW] = fresh({W, 1, K}, kType, x), g[CB] = fresh({W}, kType, x);
+      take_gates(nb, bw, kType, x, g[WA], g[BA], g[WI], g[BI], g[LAM]);
+      g[WO] = fresh({D, W}, kType, x), g[BO] = fresh({D}, kType, x);
 
       const WeightGrad go(M, D, W, 1, kType), gp(M, W, D, 2, kType);
       const size_t column_bytes_o = rglru_hip_colsum_scratch_bytes(M, D);

@@ -1196,3 +1196,31 @@ def test_replaced_parameters_are_not_kept_alive(what, how):
     p = m = None
     gc.collect()
     assert all(ref() is None for ref in old)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_results_have_memory_of_their_own(dtype):
+    """Gradients and carried state are not views of one buffer: keeping or saving one keeps or saves that one, or with it at most
+    its like (the weights of the two gates and of the two input projections, the three vectors of the RG-LRU)."""
+    from griffin_amd import RG_LRU, RecurrentBlock
+
+    torch.manual_seed(0)
+    layer, block = RG_LRU(128, gate_blocks=2).cuda().to(dtype), RecurrentBlock(64, 128, gate_blocks=2).cuda().to(dtype)
+
+    def own(tensors, times=1):
+        return all(t.untyped_storage().nbytes() <= times * (-(-t.numel() * t.element_size() // 256) * 256) for t in tensors)
+
+    for module, features in ((layer, 128), (block, 64)):
+        x = torch.randn(2, 9, features, device="cuda", dtype=dtype, requires_grad=True)
+        module(x).float().square().sum().backward()
+        assert own([x.grad, *(p.grad for p in module.parameters())], 3)
+        with torch.no_grad():
+            cache = None
+            for _ in range(3):
+                token = torch.randn(2, 1, features, device="cuda", dtype=dtype)
+                if module is layer:
+                    _, cache = module(token, cache, return_state=True)
+                    assert own([cache])
+                else:
+                    _, cache = module(token, cache, return_cache=True)
+                    assert own([cache.rnn_state, cache.conv_state, cache.segment_position])
