@@ -36,14 +36,16 @@ using torch::autograd::Variable;
 using torch::autograd::variable_list;
 using MaybeTensor = std::optional<Tensor>;
 
-// Whether a decode step of so many multiply-adds in its three projections takes the library's own kernels.  Against the BLAS
-// library they are faster up to about 16 rows of a 768 x 1024 block and up to three times slower beyond (GPU time of 512 rows,
-// 2560 -> 5120: 70 against 23 us in bf16), but a call of it costs the host 25 us: the line lies where our launches take
-// about as long as the host would (75 us at the rates the kernels reach, 1e8 multiply-adds a microsecond in bf16, 0.4e8 in
-// fp32); inside a captured graph, where host time is nothing, at the sizes where the kernels themselves are no slower.
+// Whether a decode step of so many multiply-adds in its three projections takes the library's own kernels.  A call of the BLAS
+// library costs the host 17 to 25 us, so a block's step through it takes 90 us however few rows it has, in a stack of blocks too
+// (nothing waits between them); its kernels are the faster ones beyond about 16 rows of a 768 x 1024 block.  The line lies where
+// both ways take equally long per layer in a stack of eight, alone or with an MLP of three products behind each block
+// (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS, alone / with MLPs): bf16 2560 -> 2560 at 2.5e9 77 : 89 / 173 : 184,
+// at 5.0e9 107 : 89 / 221 : 185, 768 -> 1024 at 1.2e9 46 : 90 / 119 : 184; fp32 2560 at 6.3e8 87 : 89 / 170 : 185, at 1.3e9
+// 120 : 89 / 227 : 184.  Inside a captured graph, where host time is nothing, it lies where the kernels themselves are no slower.
 bool own_projections(double macs, at::ScalarType dtype) {
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < 1e8;
-  return macs < (dtype == at::kBFloat16 ? 7.5e9 : 3e9);
+  return macs < (dtype == at::kBFloat16 ? 3e9 : 9e8);
 }
 
 // ---- small helpers ---------------------------------------------------------------------------------------------
@@ -1356,14 +1358,17 @@ Tensor sum_sets(const Tensor& sets) {
 }
 
 // Whether products of `macs` multiply-adds each (tokens x width x model width) run on the library's own kernels.  The BLAS
-// library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us, a step of
-// the block has seven, and below the line the step is over before the host has issued it: in bf16 about 8192 tokens of
-// 768 -> 1024.  Inside a captured graph host time is nothing: there the line lies where the kernels take equally long.
+// library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us and a
+// training step of the block has seven.  The line lies where both ways take equally long per layer in a stack of eight blocks,
+// alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
+// alone / with MLPs).  bf16, training 768 -> 1024: at 3.2e9 259 : 309 / 702 : 701, at 6.4e9 390 : 349 / 1091 : 1044; prefill: 66 : 91 / 161 : 181 and
+// 104 : 98 / 273 : 269.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
+// host time is nothing: there the line lies where the kernels take equally long.
 bool own_products(double macs, at::ScalarType dtype) {
   if (!known(dtype)) return false;
   const bool bf16 = dtype == at::kBFloat16;
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < (bf16 ? 2e9 : 4e8);
-  return macs < (bf16 ? 6e9 : 9e8);
+  return macs < (bf16 ? 4e9 : 9e8);
 }
 
 // Contiguous rows of whole 16-byte vectors, as rglru_hip_linear takes them.
