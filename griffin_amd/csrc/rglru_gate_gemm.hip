@@ -1,6 +1,6 @@
 // The two block-diagonal GEMMs of the gate gradients (griffin/griffin.py:149-154 under autograd) for the
 // configurations whose backward kernel leaves the gradients at the gate pre-activations in memory
-// (rglru_hip_bwd: fp32 storage, block widths that are no multiple of 32, unaligned tensors, bf16 blocks
+// (rglru_hip_bwd: fp32 storage, block widths that are no multiple of 8, unaligned tensors, bf16 blocks
 // wider than 384 channels):
 //
 //     dx[n, k bw + j] += sum_o du_a[n, k bw + o] W_a[k][o][j] + du_x[n, k bw + o] W_x[k][o][j]

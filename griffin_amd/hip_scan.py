@@ -38,7 +38,7 @@ def set_reproducible(enable: bool) -> bool:
 
 
 def set_chain_forward(mode: int) -> int:
-    """Choice of the forward kernel for bf16 storage and gate blocks of 32, 64 or 128 channels
+    """Choice of the forward kernel for bf16 storage and gate blocks of up to 128 channels, a multiple of 8
     (rglru_hip_set_chain_forward): 0 = by shape (default), 1 = always tiles with a look-back between
     workgroups, 2 = one workgroup per chain whenever that kernel covers the shape.  Returns the previous mode."""
     return int(_lib.load().rglru_hip_set_chain_forward(int(mode)))

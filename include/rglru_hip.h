@@ -9,11 +9,15 @@
  *   griffin/triton_scan.py:207-244  _FusedRGLRUScan.forward   rglru_hip_scan_fwd
  *   griffin/triton_scan.py:246-271  _FusedRGLRUScan.backward  rglru_hip_scan_bwd
  *   griffin/griffin.py:237-289      RG_LRU.forward (gates + scan, T > 1)   rglru_hip_prepare + rglru_hip_fwd
- *   autograd of griffin/griffin.py:237-289                                   rglru_hip_bwd_full (blocks of 32/64/128 channels),
+ *   autograd of griffin/griffin.py:237-289                                   rglru_hip_bwd_full (blocks of 8 .. 128 channels),
  *                                                                            rglru_hip_bwd_wide (129 .. 384), rglru_hip_bwd (any)
  *   the same for bf16 blocks of 416 .. 512 channels (gate projections of griffin/griffin.py:149-154 as a GEMM kernel of their own)   rglru_hip_fwd_pre, rglru_hip_bwd_pre
  *   griffin/griffin.py:279-284 with T == 1 (decode step, carried state)     rglru_hip_step, rglru_hip_steps (K steps a launch)
  *   (no counterpart: forward for callers that cannot allocate)              rglru_hip_fwd_static
+ *   griffin/griffin.py:379-389 and autograd   the block's Linear layers      rglru_hip_linear, rglru_hip_sums
+ *   griffin/griffin.py:379-389, :474-487 with T == 1   the same for a decode step, with its convolution   rglru_hip_decode_project, rglru_hip_decode_linear
+ *   griffin/griffin.py:309-358, :488-510   what an activity mask says about the tokens   rglru_hip_token_facts, rglru_hip_pack_flags, rglru_hip_mask_rows
+ *   autograd of griffin/griffin.py:464-520   reverse scan with the output gate, convolution, last sums   rglru_hip_block_bwd, rglru_hip_block_finish
  *   griffin/griffin.py:474-487      causal depthwise convolution of the caller   rglru_hip_conv_fwd
  *   autograd of griffin/griffin.py:474-487                                   rglru_hip_conv_bwd
  *   griffin/griffin.py:488-510      the same over right-padded batches and its autograd   rglru_hip_conv_padded_fwd, _bwd
@@ -51,7 +55,7 @@
 extern "C" {
 #endif
 
-#define RGLRU_ABI_VERSION 22
+#define RGLRU_ABI_VERSION 23
 
 enum { RGLRU_F32 = 0, RGLRU_BF16 = 1 };
 
@@ -73,7 +77,7 @@ enum {
  * the workspace clears the backward's part as well.  Or'ed into the `grad_dtype` of rglru_hip_bwd, rglru_hip_bwd_full or
  * rglru_hip_bwd_wide: the workspace comes from such a forward call that ran the tiled kernels (rglru_hip_backward_path is not
  * RGLRU_PATH_FAST_CHAIN or RGLRU_PATH_PRE, or the block's forward) and no backward call has used it since; the backward call
- * then needs no clearing launch of its own. */
+ * then needs no clearing launch of its own.  In a captured graph: only where the same graph holds that forward call. */
 #define RGLRU_BACKWARD_CLEAR 0x100
 /* Bits 2-3 of a flag byte are read by rglru_hip_block_fwd only (convolution lags that reach in front of the
  * token's document); every other entry point ignores them. */
@@ -97,7 +101,8 @@ int rglru_hip_max_block_width(void);
  * use it concurrently.  The forward call clears both parts in its one clearing launch, so a training step pays
  * for one such launch: pass ws_fresh != 0 to the FIRST backward call that is given the workspace of its forward
  * call; ws_fresh == 0 (any other workspace, or a repeated backward call) makes the backward call clear its part
- * itself.  Nothing but that is carried from forward to backward in `ws`. */
+ * itself.  A backward call that is captured into a graph without its forward call needs ws_fresh == 0: the graph is
+ * replayed on what the replay before it left.  Nothing but that is carried from forward to backward in `ws`. */
 size_t rglru_hip_scan_workspace_bytes(int64_t B, int64_t T, int64_t W);
 int rglru_hip_scan_fwd(const float* a, const float* z, const float* h0, float* h, void* ws,
                        int64_t B, int64_t T, int64_t W, void* stream);
@@ -160,7 +165,7 @@ int rglru_hip_prepare_fwd(const void* w_a, const void* b_a, const void* w_x, con
                           void* y, float* h_last, void* ws,
                           int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
 
-/* Backward of rglru_hip_fwd for any configuration (fp32 storage, block widths that are no multiple of 32,
+/* Backward of rglru_hip_fwd for any configuration (fp32 storage, block widths that are no multiple of 8,
  * unaligned tensors).  Recomputes the gates and the decay from x (nothing but the chunk checkpoints in `ws`
  * is kept from forward).  dy[B,T,W] (dtype); dh_last[B,W] fp32 or NULL.  Outputs, all complete: dx[B,T,W]
  * (dtype), dw_a, dw_x [nb,bw,bw], db_a, db_x [nb*bw] and dlambda [W] (grad_dtype), dh0 [B,W] (fp32, may be
@@ -174,9 +179,11 @@ int rglru_hip_bwd(const void* x, const void* prep, const float* h0,
                   void* stream);
 
 /* Complete backward for the fast configurations (rglru_hip_fast_path(W, nb, dtype) != 0: 16-bit
- * storage, gate blocks of 32, 64 or 128 channels, 16-byte aligned tensors).  Same inputs as
- * rglru_hip_bwd plus y[B,T,W], the output of the forward call as it was stored (the state in front of
- * token t is read from row t - 1 of it; the checkpoints in `ws` are not used).  dx[B,T,W] is the full
+ * storage, gate blocks of any multiple of 8 channels up to 128, 16-byte aligned tensors).  Same inputs as
+ * rglru_hip_bwd plus y[B,T,W], the output of the forward call as it was stored.  Blocks of 32, 64 and 128 channels:
+ * the state in front of token t is read from row t - 1 of y, dL/dh_t crosses `scratch` in the storage type and the
+ * per-workgroup weight-gradient sums in grad_dtype.  The others (padded to whole 32-channel slabs, and 96): the state is
+ * recomputed from the checkpoints in `ws`, dL/dh_t and the sums are fp32, as in rglru_hip_bwd.  dx[B,T,W] is the full
  * input gradient and dw_a, dw_x [nb,bw,bw] (grad_dtype) the weight gradients.  Two hand-written
  * kernels: the reverse scan for dL/dh_t, which recomputes only the decay, then one kernel that
  * recomputes both gates and forms every gradient including the two block-diagonal GEMMs, so the
@@ -457,7 +464,7 @@ int rglru_hip_decode_project(const void* x, int64_t x_stride, const void* w_x, c
  * Optional outputs (NULL to skip): x_conv[B,T,W] and y[B,T,W] (what a backward pass needs),
  * new_conv_state[B,K-1,W], h_last[B,W].  No output may overlap an input (a tile reads the three rows of u in
  * front of it while its neighbour writes).  ws as for rglru_hip_fwd.  Only where
- * rglru_hip_block_fwd_path() returns 1 (bf16 storage, gate blocks of 32, 64 or 128 channels, 16-byte
+ * rglru_hip_block_fwd_path() returns 1 (bf16 storage, gate blocks of any multiple of 8 channels up to 128, 16-byte
  * aligned rows); otherwise RGLRU_E_UNSUPPORTED, and the caller runs rglru_hip_conv_fwd, rglru_hip_fwd and
  * rglru_hip_gelu_gate_fwd one after the other.  rglru_hip_prepare_block_fwd is rglru_hip_prepare +
  * rglru_hip_block_fwd in two launches (as rglru_hip_prepare_fwd); with stack_bytes > 0 the first of them also copies stack0 and
@@ -501,7 +508,7 @@ int64_t rglru_hip_set_spin_limit(int64_t polls);
  * composition follows the ticket order).  The chain becomes one memory round trip per chunk: slower,
  * mostly for long sequences.  Applies to launches made after the call; returns the previous setting. */
 int rglru_hip_set_reproducible(int enable);
-/* Which forward kernel rglru_hip_fwd uses for bf16 storage and gate blocks of 32, 64 or 128 channels (no
+/* Which forward kernel rglru_hip_fwd uses for bf16 storage and gate blocks of up to 128 channels, a multiple of 8 (no
  * counterpart in the reference).  0 (default): by shape -- the library estimates the time of both kernel pairs
  * from the number of (sequence, 32-channel slab) chains, the compute units and the sequence length and takes
  * the faster: one workgroup walks a whole chain (no exchange between workgroups, bit-reproducible) for small
