@@ -325,10 +325,13 @@ def secondary_workload(args):
             rewind()
             graph.replay()
             torch.cuda.synchronize()
-            agree = bool((out_g.float() - eager_out.float()).abs().max().item()
-                         <= 1e-6 * max(eager_out.float().abs().max().item(), 1.0))
+            # eager steps take their products from the library's kernels, captured ones at this size from the BLAS library:
+            # equal up to the bf16 rounding of the projections
+            worst = (out_g.float() - eager_out.float()).abs().max().item() / max(eager_out.float().abs().max().item(), 1e-30)
+            agree = bool(worst < 2e-2)
             ms_graph = _timed(graph.replay, max(args.steps // 10, 1), 1) / steps
-            extra = {"us_per_step_eager": ms * 1e3, "us_per_step_graph64": ms_graph * 1e3, "graph_matches_eager": agree}
+            extra = {"us_per_step_eager": ms * 1e3, "us_per_step_graph64": ms_graph * 1e3, "graph_matches_eager": agree,
+                     "graph_vs_eager_max_rel_err": worst}
             ms = ms_graph
         metric, tokens = "RecurrentBlock decode tokens/s", B
         workload = f"RecurrentBlock({D}, {W}) decode B{B} bf16, {steps} steps after a T128 prefill (one HIP graph of the {steps} steps)"

@@ -43,8 +43,9 @@ using MaybeTensor = std::optional<Tensor>;
 // (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS, alone / with MLPs): bf16 2560 -> 2560 at 2.5e9 77 : 89 / 173 : 184,
 // at 5.0e9 107 : 89 / 221 : 185, 768 -> 1024 at 1.2e9 46 : 90 / 119 : 184; fp32 2560 at 6.3e8 87 : 89 / 170 : 185, at 1.3e9
 // 120 : 89 / 227 : 184.  Inside a captured graph, where host time is nothing, it lies where the kernels themselves are no slower.
+bool own_projections_captured(double macs) { return macs < 1e8; }
 bool own_projections(double macs, at::ScalarType dtype) {
-  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < 1e8;
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return own_projections_captured(macs);
   return macs < (dtype == at::kBFloat16 ? 3e9 : 9e8);
 }
 
@@ -1338,6 +1339,11 @@ py::object block_decode(py::handle module, const Tensor& x, py::handle cache, py
     if (!conv_state || !prev || !state_shapes(B, W, K, *conv_state, opt(rnn), *prev) || prev->scalar_type() != at::kLong || !prev->is_contiguous())
       return py::none();                                   // the module's Python code reports a wrong shape
   }
+  if (!own_projections_captured(3.0 * B * W * x.size(2))) {
+    // the module's Python code leaves the stacked projection that a capture of this step would go through
+    PyObject* stacked = block.at("_stacked_projection");
+    if (stacked == nullptr || stacked == Py_None) return py::none();
+  }
   const Stamp* s = current_stamp(lru, x.scalar_type(), x.device());
   if (s == nullptr) return py::none();
   auto done = block_step(x, wx, bx, wy, by, cw, cb, wo, bo, conv_state, prev, std::nullopt, std::nullopt, s->image, s->blocks, rnn);
@@ -2087,6 +2093,7 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(block_forward);
   EXPORT(block_decode_step);
   EXPORT(block_step);
+  EXPORT(own_projections_captured);
   EXPORT(sum_sets);
   EXPORT(stacked_halves);
   EXPORT(linear);

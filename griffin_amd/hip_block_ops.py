@@ -145,6 +145,12 @@ def hip_block_step(x: Tensor, linear_x, linear_y, conv, linear_out, conv_state: 
     return _lib.native().block_step(x, *operands, conv_state, prev_pos, segment_pos, active, prep.image, prep.blocks, rnn_state)
 
 
+def hip_block_step_captured(batch: int, width: int, dim: int) -> bool:
+    """Whether ``hip_block_step`` takes so many rows inside a graph capture, where the line to the BLAS library's products lies
+    lower than outside (host time is nothing in a graph)."""
+    return _lib.native().own_projections_captured(3.0 * batch * width * dim)
+
+
 def hip_block_infer(x: Tensor, parameters, prep, conv_state: Tensor | None, rnn_state: Tensor | None, prev_pos: Tensor | None,
                     segment_pos: Tensor | None, flags: Tensor | None, rows: Tensor | None, active: Tensor | None, u: Tensor | None,
                     v: Tensor | None, need_state: bool):

@@ -490,6 +490,8 @@ class RecurrentBlock(_HoldsLeaves):
         if active_mask is not None and not bool(active_mask.all()):
             active = active_mask[:, 0].to(torch.uint8).contiguous()
         layers = self._modules
+        if not hip_block_ops.hip_block_step_captured(batch, width, x.size(2)) and not torch.cuda.is_current_stream_capturing():
+            self._stack_projections()                        # a capture of this step goes through it and cannot make it
         if not torch.is_autocast_enabled() and self._is_plain(layers["linear_out"]):
             done = hip_block_ops.hip_block_step(x, layers["linear_x"], layers["linear_y"], layers["temporal_conv"], layers["linear_out"],
                                                 conv_state, prev_pos, segment_pos, active, layers["rg_lru"]._prepared(x.dtype, x.device),
@@ -511,23 +513,29 @@ class RecurrentBlock(_HoldsLeaves):
 
     def _decode_projections(self, token: Tensor):
         """``linear_x`` and ``linear_y`` of one token per row as ONE GEMM against the two weights stacked
-        (the decode kernels take the halves of its output as strided rows).  The stacked copy is kept
-        until a weight or bias changes (storage or version counter)."""
-        layers = (self.linear_x, self.linear_y)
-        tensors = [t for layer in layers for t in (layer.weight, layer.bias) if t is not None]
+        (the decode kernels take the halves of its output as strided rows)."""
+        stacked = self._stack_projections()
+        if stacked is None:
+            return self.linear_x(token), self.linear_y(token)
+        both = torch.nn.functional.linear(token, *stacked)
+        return both[:, :self.rnn_width], both[:, self.rnn_width:]
+
+    def _stack_projections(self):
+        """Weight and bias of ``linear_x`` above those of ``linear_y``, kept until one of them changes (storage or version
+        counter).  None where a bias is missing, and during a graph capture where they are not there: nothing allocated
+        then may outlive it."""
+        tensors = [t for layer in (self.linear_x, self.linear_y) for t in (layer.weight, layer.bias) if t is not None]
         key = (*hip_scan.fingerprint(tensors), *((t.dtype, t.device) for t in tensors))
         cached = getattr(self, "_stacked_projection", None)
         if cached is None or cached[0] != key:
-            if len(tensors) != 4 or (token.is_cuda and torch.cuda.is_current_stream_capturing()):
-                # nothing allocated during a graph capture may outlive it: two GEMMs this time
-                return self.linear_x(token), self.linear_y(token)
+            if len(tensors) != 4 or (tensors[0].is_cuda and torch.cuda.is_current_stream_capturing()):
+                return None
             with torch.no_grad():
                 weight = torch.cat([self.linear_x.weight, self.linear_y.weight], 0).contiguous()
                 bias = torch.cat([self.linear_x.bias, self.linear_y.bias], 0).contiguous()
             cached = (key, weight, bias)
             self._stacked_projection = cached
-        both = torch.nn.functional.linear(token, cached[1], cached[2])
-        return both[:, :self.rnn_width], both[:, self.rnn_width:]
+        return cached[1:]
 
     def _linear(self, layer: nn.Linear, x: Tensor) -> Tensor:
         """A Linear layer of the block; in training on the HIP path its bias gradient is summed by a

@@ -1224,3 +1224,24 @@ def test_results_have_memory_of_their_own(dtype):
                 else:
                     _, cache = module(token, cache, return_cache=True)
                     assert own([cache.rnn_state, cache.conv_state, cache.segment_position])
+
+
+def test_decode_leaves_the_stacked_projection_for_a_capture():
+    """Eager steps of many rows run on the library's own products, captured ones go through one product with both projections'
+    weights stacked, which a capture cannot make: the eager step in front of it leaves it, and renews it after an update."""
+    from griffin_amd import RecurrentBlock
+
+    torch.manual_seed(0)
+    block = RecurrentBlock(768, 1024).bfloat16().cuda()
+    x = torch.randn(64, 1, 768, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad():
+        block(x[:2])
+        assert getattr(block, "_stacked_projection", None) is None      # few rows: own products either way
+        want = block(x)
+        first = block._stacked_projection
+        assert torch.equal(first[1], torch.cat([block.linear_x.weight, block.linear_y.weight]))
+        assert torch.equal(block(x), want)
+        block.linear_y.weight.mul_(0.5)
+        block.rg_lru.Lambda.mul_(1.0)
+        block(x)
+        assert torch.equal(block._stacked_projection[1], torch.cat([block.linear_x.weight, block.linear_y.weight]))
