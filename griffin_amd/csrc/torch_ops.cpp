@@ -1367,14 +1367,15 @@ Tensor sum_sets(const Tensor& sets) {
 // library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us and a
 // training step of the block has seven.  The line lies where both ways take equally long per layer in a stack of eight blocks,
 // alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
-// alone / with MLPs).  bf16, training 768 -> 1024: at 3.2e9 259 : 309 / 702 : 701, at 6.4e9 390 : 349 / 1091 : 1044; prefill: 66 : 91 / 161 : 181 and
-// 104 : 98 / 273 : 269.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
+// alone / with MLPs).  bf16, training 768 -> 1024: at 3.0e9 269 : 316 / 716 : 728, at 6.0e9 401 : 440 / 1106 : 1150, at 1.3e10 651 : 532 / 1847 : 1703;
+// 2560 -> 2560 at 4.5e9 373 : 384 / 963 : 952, at 6.0e9 431 : 419 / 1121 : 1108; prefill 768 -> 1024 at 6.0e9 109 : 105 / 299 : 296, 2560 at 4.5e9
+// 120 : 129 / 266 : 254.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
 // host time is nothing: there the line lies where the kernels take equally long.
 bool own_products(double macs, at::ScalarType dtype) {
   if (!known(dtype)) return false;
   const bool bf16 = dtype == at::kBFloat16;
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < (bf16 ? 2e9 : 4e8);
-  return macs < (bf16 ? 4e9 : 9e8);
+  return macs < (bf16 ? 6e9 : 9e8);
 }
 
 // Contiguous rows of whole 16-byte vectors, as rglru_hip_linear takes them.
