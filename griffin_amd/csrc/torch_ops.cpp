@@ -36,17 +36,19 @@ using torch::autograd::Variable;
 using torch::autograd::variable_list;
 using MaybeTensor = std::optional<Tensor>;
 
-// Whether a decode step of so many multiply-adds in its three projections takes the library's own kernels.  A call of the BLAS
-// library costs the host 17 to 25 us, so a block's step through it takes 90 us however few rows it has, in a stack of blocks too
-// (nothing waits between them); its kernels are the faster ones beyond about 16 rows of a 768 x 1024 block.  The line lies where
-// both ways take equally long per layer in a stack of eight, alone or with an MLP of three products behind each block
-// (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS, alone / with MLPs): bf16 2560 -> 2560 at 2.5e9 77 : 89 / 173 : 184,
-// at 5.0e9 107 : 89 / 221 : 185, 768 -> 1024 at 1.2e9 46 : 90 / 119 : 184; fp32 2560 at 6.3e8 87 : 89 / 170 : 185, at 1.3e9
-// 120 : 89 / 227 : 184.  Inside a captured graph, where host time is nothing, it lies where the kernels themselves are no slower.
+// Whether a decode step of `rows` rows, so many multiply-adds in its three projections, takes the library's own kernels.  A call
+// of the BLAS library costs the host 17 to 25 us, so a block's step through it takes 90 us however few rows it has, in a stack
+// of blocks too (nothing waits between them); its kernels are the faster ones beyond about 16 rows of a 768 x 1024 block.  The
+// line lies where our kernels take the 60 us that are left next to the step's other launches, at the rate they reach: with up to 64
+// rows (one tile of rows: every weight is used once) 31e6 multiply-adds a us in bf16 and 13e6 in fp32, with more 50e6 and 24e6.
+// Per layer in a stack of eight, alone / with an MLP of three products behind each block, us own : BLAS
+// (profiles/block_products_own_vs_blas_in_stacks.txt): bf16 2560 -> 2560 64 rows 64 : 91 / 134 : 200, 128 rows 77 : 89 / 173 : 184, 256 rows 107 : 89 /
+// 221 : 185; fp32 768 -> 1024 512 rows 70 : 100 / 150 : 172, 2560 32 rows 87 : 89 / 170 : 185, 64 rows 120 : 89 / 227 : 184, 128 rows 142 : 115 /
+// 351 : 323.  Inside a captured graph, where host time is nothing, it lies where the kernels themselves are no slower.
 bool own_projections_captured(double macs) { return macs < 1e8; }
-bool own_projections(double macs, at::ScalarType dtype) {
+bool own_projections(int64_t rows, double macs, at::ScalarType dtype) {
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return own_projections_captured(macs);
-  return macs < (dtype == at::kBFloat16 ? 3e9 : 9e8);
+  return macs < (dtype == at::kBFloat16 ? (rows > 64 ? 3e9 : 1.9e9) : (rows > 64 ? 1.45e9 : 8e8));
 }
 
 // ---- small helpers ---------------------------------------------------------------------------------------------
@@ -1185,7 +1187,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_step(
                                                               &active, &image, &rnn_state})
     if (!on_device_of(x_in, *t)) return std::nullopt;
   active = token_bytes(active, B);
-  if (K > 4 || B >= (1 << 16) || !own_projections(3.0 * B * W * D, dtype) || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
+  if (K > 4 || B >= (1 << 16) || !own_projections(B, 3.0 * B * W * D, dtype) || (D * x_in.element_size()) % 16 || (W * x_in.element_size()) % 16) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &b_x, &w_y, &b_y, &conv_w, &conv_b, &w_o, &b_o, &conv_state})
     if (t->defined() && (t->scalar_type() != dtype || !t->is_contiguous())) return std::nullopt;
   for (const Tensor* t : std::initializer_list<const Tensor*>{&w_x, &w_y, &w_o})
