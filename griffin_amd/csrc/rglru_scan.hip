@@ -417,6 +417,7 @@ int64_t rglru_hip_set_spin_limit(int64_t polls) {
   return (int64_t)g_spin_limit.exchange((long long)polls);
 }
 
+int rglru_hip_reproducible(void) { return g_reproducible.load(std::memory_order_relaxed); }
 int rglru_hip_set_reproducible(int enable) { return g_reproducible.exchange(enable ? 1 : 0); }
 
 size_t rglru_hip_scan_workspace_bytes(int64_t B, int64_t T, int64_t W) {

@@ -1898,6 +1898,8 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
   if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 || !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), opt(v)) ||
       (u.has_value() && u->scalar_type() != N::kType) || (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
     return std::nullopt;
+  // the gated reverse scan in tiles adds the gradient of linear_y's bias up in the order of its tickets
+  if (rglru_hip_reproducible() && kernel_path(B, T, W, wa.size(0), N::kType, true) != RGLRU_PATH_FAST_CHAIN) return std::nullopt;
   MaybeTensor live;
   if (active.has_value()) live = active->contiguous();
   Tensor positions = pos.to(at::kLong).contiguous();

@@ -508,6 +508,10 @@ int64_t rglru_hip_set_spin_limit(int64_t polls);
  * composition follows the ticket order).  The chain becomes one memory round trip per chunk: slower,
  * mostly for long sequences.  Applies to launches made after the call; returns the previous setting. */
 int rglru_hip_set_reproducible(int enable);
+/* The setting as it is.  rglru_hip_block_bwd does not honour it where the tiled kernels run (rglru_hip_backward_path is not
+ * RGLRU_PATH_FAST_CHAIN): the column sums of dv follow the tickets there; rglru_hip_gelu_gate_bwd, rglru_hip_bwd_full and
+ * rglru_hip_conv_rows_bwd one after the other do. */
+int rglru_hip_reproducible(void);
 /* Which forward kernel rglru_hip_fwd uses for bf16 storage and gate blocks of up to 128 channels, a multiple of 8 (no
  * counterpart in the reference).  0 (default): by shape -- the library estimates the time of both kernel pairs
  * from the number of (sequence, 32-channel slab) chains, the compute units and the sequence length and takes

@@ -1245,3 +1245,42 @@ def test_decode_leaves_the_stacked_projection_for_a_capture():
         block.rg_lru.Lambda.mul_(1.0)
         block(x)
         assert torch.equal(block._stacked_projection[1], torch.cat([block.linear_x.weight, block.linear_y.weight]))
+
+
+@pytest.mark.parametrize("dtype,blocks", [(torch.bfloat16, 4), (torch.bfloat16, 16), (torch.bfloat16, 5)])
+@pytest.mark.parametrize("kind", ["default", "packed", "right-padded", "left-padded"])
+def test_reproducible_mode_repeats_the_block_bit_for_bit(dtype, blocks, kind):
+    """With set_reproducible(True) a training step of the block repeats bit for bit: output and every gradient, the biases' too
+    (sums over the tokens have a fixed order then)."""
+    from griffin_amd import RecurrentBlock, set_reproducible
+
+    torch.manual_seed(0)
+    B, T, D, W = 3, 1500, 64, 240 if blocks == 5 else 256
+    block = RecurrentBlock(D, W, gate_blocks=blocks).to(dtype).cuda()
+    x = torch.randn(B, T, D, device="cuda", dtype=dtype, requires_grad=True)
+    dy = torch.randn_like(x)
+    mask = torch.ones(B, T, dtype=torch.bool, device="cuda")
+    kwargs = {}
+    if kind == "packed":
+        kwargs["segment_pos"] = (torch.arange(T, device="cuda") % 333).expand(B, T).contiguous()
+    elif kind == "right-padded":
+        mask[1, 700:] = False
+        kwargs["active_mask"] = mask
+    elif kind == "left-padded":
+        mask[2, :99] = False
+        kwargs["active_mask"] = mask
+
+    def run():
+        y = block(x, **kwargs)
+        out = [y.detach(), *torch.autograd.grad(y, [x, *block.parameters()], dy)]
+        torch.cuda.synchronize()
+        return out
+
+    was = set_reproducible(True)
+    try:
+        runs = [run() for _ in range(6)]
+    finally:
+        set_reproducible(was)
+    for other in runs[1:]:
+        for name, a, b in zip(("y", "x", *(n for n, _ in block.named_parameters())), runs[0], other):
+            assert torch.equal(a, b), name
