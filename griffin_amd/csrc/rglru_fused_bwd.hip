@@ -2087,9 +2087,9 @@ int rglru_hip_bwd_full(const void* x, const void* y, const void* prep, const flo
   return check_launch("bwd_full finish");
 }
 
-// Partial rows in which the gated reverse scan leaves the column sums of dv (see bwd_full_kernels).
-static int64_t gate_sum_sets(int64_t B, int64_t T, const Geometry& g) {
-  if (fwd_chain_pays(B, T, g.Wp)) return B;
+// Partial rows in which the gated reverse scan leaves the column sums of dv (see bwd_full_kernels): one a sequence in the chain
+// kernel, one a workgroup of the unit in tiles.
+static int64_t gate_sum_sets_tiled(int64_t B, int64_t T, const Geometry& g) {
   FusedArgs a;
   memset(&a, 0, sizeof(a));
   a.units = (int)g.units;
@@ -2097,9 +2097,12 @@ static int64_t gate_sum_sets(int64_t B, int64_t T, const Geometry& g) {
   return pick_wg_per_unit(a.units, B * ((T + 32 * kDeltaMT - 1) / (32 * kDeltaMT)), kDeltaMT == 1 ? 4 : RGLRU_DELTA_OCC, make_work_layout(B, T, g).max_wg);
 }
 
+static int64_t gate_sum_sets(int64_t B, int64_t T, const Geometry& g) { return fwd_chain_pays(B, T, g.Wp) ? B : gate_sum_sets_tiled(B, T, g); }
+
+// Room for either kernel: rglru_hip_set_chain_forward may be called between this and the launch.
 size_t rglru_hip_block_sums_bytes(int64_t B, int64_t T, int64_t W, int64_t nb) {
   if (B <= 0 || T <= 0 || W <= 0 || nb <= 0 || W % nb) return 0;
-  return (size_t)(gate_sum_sets(B, T, make_geometry(W, nb)) * W * 4);
+  return (size_t)(std::max(B, gate_sum_sets_tiled(B, T, make_geometry(W, nb))) * W * 4);
 }
 
 int rglru_hip_block_bwd(void* dgated, const void* y, const void* u, const void* v, const void* x_conv, const void* prep,

@@ -134,3 +134,20 @@ def test_block_forward_queries_and_errors_without_a_gpu(lib):
     # the sentinel for "every row starts a document" is not a flag array of the decode steps
     assert lib.rglru_hip_step(fake, fake, fake, ctypes.c_void_p(1), fake, 4, 64, 2, _lib.RGLRU_BF16, None) == 1
     assert b"FIRST_RESET" in lib.rglru_hip_last_error()
+
+
+def test_scratch_sizes_do_not_depend_on_the_kernel_choice():
+    """A buffer sized before rglru_hip_set_chain_forward is called still holds what the launch after it writes."""
+    lib = _lib.load()
+    sizes = {"bwd": lib.rglru_hip_bwd_scratch_bytes, "block sums": lib.rglru_hip_block_sums_bytes, "workspace": lib.rglru_hip_workspace_bytes}
+    was = lib.rglru_hip_set_chain_forward(0)
+    try:
+        for B, T, W, nb in [(1, 4096, 256, 4), (8, 2048, 1024, 16), (3, 700, 768, 16), (300, 64, 256, 2), (64, 1, 64, 2)]:
+            got = []
+            for mode in (0, 1, 2):
+                lib.rglru_hip_set_chain_forward(mode)
+                got.append([fn(B, T, W, nb, *((_lib.RGLRU_BF16,) if name == "bwd" else ())) for name, fn in sizes.items()])
+            assert got[0] == got[1] == got[2], (B, T, W, nb, got)
+            assert got[0][1] >= B * W * 4                    # one row a sequence in the chain kernel
+    finally:
+        lib.rglru_hip_set_chain_forward(was)
