@@ -1385,10 +1385,14 @@ bool vector_rows(const Tensor& t) {
   return t.is_contiguous() && (t.size(-1) * t.element_size()) % 16 == 0 && is_aligned(t);
 }
 
+// A tensor that dispatches itself (a subclass with __torch_dispatch__: quantised or distributed weights, wrapped inputs) has no
+// memory for a kernel to read; PyTorch's product takes it.
+bool plain(const Tensor& t) { return !t.defined() || !t.key_set().has(c10::DispatchKey::Python); }
+
 // Whether the library takes y = x w^T + b (and its gradients) for these operands.
 bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b) {
   const auto dtype = x.scalar_type();
-  return w.dim() == 2 && x.size(-1) == w.size(1) && on_device_of(x, w) && on_device_of(x, b) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
+  return plain(x) && plain(w) && plain(b) && w.dim() == 2 && x.size(-1) == w.size(1) && on_device_of(x, w) && on_device_of(x, b) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
          x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype) && vector_rows(w) && vector_rows(x) &&
          (w.size(0) * x.element_size()) % 16 == 0 && !at::autocast::is_autocast_enabled(at::kCUDA);
 }

@@ -1070,6 +1070,7 @@ def test_weights_that_dispatch_themselves_are_multiplied_by_pytorch(dtype):
     from torch.utils._pytree import tree_map
 
     from griffin_amd import RecurrentBlock
+    from griffin_amd.hip_block_ops import hip_linear, hip_linear_pair
 
     class Wrapped(torch.Tensor):
         @staticmethod
@@ -1098,6 +1099,11 @@ def test_weights_that_dispatch_themselves_are_multiplied_by_pytorch(dtype):
         block.linear_out.weight = torch.nn.Parameter(Wrapped(block.linear_out.weight.detach()), requires_grad=False)
         for (t, kw), expected in zip(calls, want):
             assert rel_err(block(t, **kw).float(), expected.float()) < (FP32_TOL if dtype == torch.float32 else BF16_TOL)
+        w, b = torch.randn(32, 64, device="cuda", dtype=dtype), torch.randn(32, device="cuda", dtype=dtype)
+        for args in ((x, Wrapped(w), b), (x, w, Wrapped(b))):        # the operators themselves
+            assert torch.equal(hip_linear(*args), torch.nn.functional.linear(x, w, b))
+        u, v = hip_linear_pair(x, Wrapped(w), b, w, b)
+        assert rel_err(u.float(), v.float()) < (FP32_TOL if dtype == torch.float32 else BF16_TOL)
 
 
 @pytest.mark.parametrize("mask_kind", ["left", "holes", "right", "dense"])
