@@ -1,4 +1,5 @@
-"""Graph captures for test_captured_backward_repeats and test_masked_block_under_capture_is_an_error, in a process of their own: a program captures on its own streams, and
+"""Graph captures for test_captured_backward_repeats, test_graphed_modules_train and
+test_masked_block_under_capture_is_an_error, in a process of their own: a program captures on its own streams, and
 what a capture leaves behind stays out of the other tests.  Prints a line for each case, ends with status 1 after a mismatch."""
 
 import sys
@@ -76,6 +77,37 @@ def captured_backward(make, dtype, shape, tol):
     return worst, worst < tol
 
 
+def graphed_modules():
+    """torch.cuda.make_graphed_callables: forward and backward in graphs of their own, replayed as a training loop does."""
+    from griffin_amd import RG_LRU, RecurrentBlock
+
+    ok = True
+    for name, make, shape, dtype, tol in (("layer", lambda: RG_LRU(96, gate_blocks=3), (2, 70, 96), torch.float32, 1e-5),
+                                          ("layer", lambda: RG_LRU(256, gate_blocks=2), (2, 200, 256), torch.bfloat16, 2e-2),
+                                          ("block", lambda: RecurrentBlock(64, 256, gate_blocks=2), (2, 200, 64), torch.bfloat16, 2e-2)):
+        print("graphed module", name, shape, flush=True)
+        torch.manual_seed(7)
+        plain = make().to(dtype).cuda()
+        graphed = make().to(dtype).cuda()
+        graphed.load_state_dict(plain.state_dict())
+        graphed = torch.cuda.make_graphed_callables(graphed, (torch.randn(*shape, device="cuda", dtype=dtype, requires_grad=True),))
+        worst = 0.0
+        for _ in range(3):
+            x, dy = (torch.randn(*shape, device="cuda", dtype=dtype) for _ in range(2))
+            results = []
+            for module in (plain, graphed):
+                module.zero_grad(set_to_none=True)
+                leaf = x.clone().requires_grad_(True)
+                y = module(leaf)
+                y.backward(dy)
+                torch.cuda.synchronize()
+                results.append([y.detach().clone(), leaf.grad.clone(), *(p.grad.clone() for p in module.parameters())])
+            worst = max([worst] + [rel_err(b.float(), a.float()) for a, b in zip(*results)])
+        print("  worst", "%.2e" % worst, flush=True)
+        ok &= worst < tol
+    return ok
+
+
 def captured_mask():
     """Which kernels a masked block runs is decided on the host: under capture that is a RuntimeError before anything is
     launched, the process goes on, and the same call outside the capture is what it was."""
@@ -114,4 +146,4 @@ def captured_backwards():
 
 
 if __name__ == "__main__":
-    sys.exit(0 if {"backward": captured_backwards, "mask": captured_mask}[sys.argv[1]]() else 1)
+    sys.exit(0 if {"backward": captured_backwards, "modules": graphed_modules, "mask": captured_mask}[sys.argv[1]]() else 1)

@@ -886,6 +886,11 @@ def test_captured_backward_repeats():
     assert _captures("backward") == 0
 
 
+def test_graphed_modules_train():
+    """Modules whose forward and backward are captured apart (torch.cuda.make_graphed_callables) train like eager ones."""
+    assert _captures("modules") == 0
+
+
 def test_masked_block_under_capture_is_an_error():
     """... and not the end of the process."""
     assert _captures("mask") == 0
