@@ -122,6 +122,13 @@ RGLRU_DEVICE void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Workgroup barrier that orders LDS accesses only: __syncthreads also waits for every global store in flight.
+RGLRU_DEVICE void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Store a staged ROWS x 32 tile of 16-bit values: `r` covers the tile's rows (row stride
 // row_bytes), col_bytes is the byte offset of the wave's first channel inside a row.  seg_ok: the lane's eight channels
 // belong to the block (a block that does not fill its last slab).

@@ -161,9 +161,26 @@ template <int ROWS> struct PairStage {                  // ROWS x 32 channels x 
   static RGLRU_DEVICE unsigned row_offset(int row) { return (unsigned)row * kRowBytes + (row >= ROWS / 2 ? 128u : 0u); }
 };
 
+// Keeps what is computed from v inside the loop that it stands in: the offsets of a tile's rows, hoisted out of it, take a
+// register each and push the scan kernels into scratch memory (140 bytes a lane instead of 48).
+RGLRU_DEVICE void hold_in_loop(unsigned& v) { asm volatile("" : "+v"(v)); }
+
+// Blocks wider than four slabs: what the reverse scan spends its time on is latency -- the loads of a tile, the barriers, the
+// walk along the records, the gate math's dependent transcendentals (a wave alone on its SIMD issues a vector instruction every 5 to
+// 6.6 clocks, two waves together every 2.5 to 4.4).  So two workgroups share a compute unit, which leaves a wave 256 registers:
+// up to 96 for the weights of twelve K groups, the others' (8 KB each) in LDS, where the outputs are staged over the x and dy
+// tiles.  A wave keeps per token r, a, the input gate's pre-activation, x and dy; the rest is computed behind the
+// look-back, two tokens at a time.  Forward state, ticket and tile of the next pass are requested in front of this pass's stores.
+// Until then a compute unit had one workgroup of four waves with 300 to 430 registers each.  Reverse scan, us, before -> now:
+//   320-wide blocks: B1 T32768 508 -> 420, B16 T2048 458 -> 321; 160-wide blocks: B8 T2048 W2560 270 -> 185.
+// Without the look-back the first would take 314, without the memory behind the stores 370 (timing builds).  Blocks of 352 and 384
+// channels need 264 and more registers this way and stay with one workgroup.
+constexpr int bwd_wide_occ(int nkg) { return nkg <= 20 ? 2 : 1; }
+constexpr int bwd_lds_groups(int nkg) { return bwd_wide_occ(nkg) == 2 && nkg > 12 ? (nkg - 12 > 6 ? 6 : nkg - 12) : 0; }
+
 // PAD: wide blocks that do not fill their slabs: columns past the block's width read as zero, their lanes store and publish nothing.
 template <typename IO, int NKG, bool MASKED, bool PAD = false>
-__global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(FusedArgs p) {
+__global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void bwd_scan_kernel(FusedArgs p) {
   constexpr int MT = 1, TR = 32, EL = 16;
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
@@ -179,41 +196,35 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
   constexpr int LDSROW = TW + Tr::HW;
   constexpr int DYROW = kPackedWidth + Tr::HW;
   static_assert(sizeof(IO) == 2 && NKG != 0, "fast backward is for 16-bit storage");
-  __shared__ __attribute__((aligned(16))) IO lds_x[TR * LDSROW];
-  __shared__ __attribute__((aligned(16))) IO lds_dy[TR * DYROW];
+  constexpr bool SHARED = WIDE && bwd_wide_occ(NKG) == 2;
+  constexpr int kDuStage = GIVEN ? 2 * WaveStage<TR>::kBytes : PairStage<TR>::kBytes;
+  constexpr int kTileBytes = 2 * TR * (LDSROW + DYROW), kStageBytes = kWaves * (WaveStage<TR>::kBytes + kDuStage);
+  // SHARED: the outputs are staged over the x and dy tiles once the whole workgroup is done with them
+  __shared__ __attribute__((aligned(16))) unsigned char lds_all[SHARED ? (kTileBytes > kStageBytes ? kTileBytes : kStageBytes) : kTileBytes + kStageBytes];
+  IO* const lds_x = reinterpret_cast<IO*>(lds_all);
+  IO* const lds_dy = lds_x + TR * LDSROW;
+  unsigned char* const stage_dx_all = lds_all + (SHARED ? 0 : kTileBytes);
+  unsigned char* const stage_du_all = stage_dx_all + kWaves * WaveStage<TR>::kBytes;
   __shared__ __attribute__((aligned(16))) IO lds_pre[GIVEN ? 2 * TR * LDSROW : Tr::HW];
-  __shared__ __attribute__((aligned(16))) unsigned char stage_dx_all[kWaves * WaveStage<TR>::kBytes];
-  __shared__ __attribute__((aligned(16))) unsigned char stage_du_all[kWaves * (GIVEN ? 2 * WaveStage<TR>::kBytes : PairStage<TR>::kBytes)];
   __shared__ unsigned s_ticket[2];
-  // With 128- and 64-channel blocks the weight registers (64, 32) push the kernel into spilling; the
-  // input gate's weights then live in LDS instead (each wave's 32 rows, read as B fragments per tile).
-  constexpr bool XLDS = (NKG == 8 || NKG == 4);
-  constexpr int WROW = KC + Tr::HW;
-  __shared__ __attribute__((aligned(16))) IO lds_wx[XLDS ? 32 * kWaves * WROW : Tr::HW];
 
   const WaveId w = wave_identity(p, blockIdx.x);
   if (w.wg_in_unit >= p.wg_per_unit) return;             // only with xcd_map: the grid's last round is not full
   const int hf = w.hf, tid = threadIdx.x;
   unsigned char* stage_dx = stage_dx_all + w.wave * WaveStage<TR>::kBytes;
-  unsigned char* stage_du = stage_du_all + w.wave * (GIVEN ? 2 * WaveStage<TR>::kBytes : PairStage<TR>::kBytes);
+  unsigned char* stage_du = stage_du_all + w.wave * kDuStage;
   const IO* wg = (const IO*)p.wg;
   const int o_safe = w.slab_ok ? w.o : 0;
   const IO* w_a_row = wg + ((long long)(0 * p.nb + w.k) * p.bwp + o_safe) * p.bwp + hf * Tr::HW;
   const IO* w_x_row = wg + ((long long)(1 * p.nb + w.k) * p.bwp + o_safe) * p.bwp + hf * Tr::HW;
-  HeldWeights<IO, NKG> hw;
-  if constexpr (XLDS) {
-#pragma unroll
-    for (int kg = 0; kg < NKG; ++kg) hw.a[kg] = *reinterpret_cast<const Frag*>(w_a_row + kg * Tr::KG);
-    // each wave copies the 32 rows of W_x of its own slab (the waves of a packed unit belong to different blocks)
-    const IO* src = wg + ((long long)(1 * p.nb + w.k) * p.bwp + (w.slab_ok ? w.slab * 32 : 0)) * p.bwp;
-    for (int idx = w.lane; idx < 32 * (KC / Tr::HW); idx += 64) {
-      const int row = idx / (KC / Tr::HW), v = idx - row * (KC / Tr::HW);
-      *reinterpret_cast<Frag*>(lds_wx + (w.wave * 32 + row) * WROW + v * Tr::HW) = *reinterpret_cast<const Frag*>(src + (long long)row * p.bwp + v * Tr::HW);
-    }
-    __syncthreads();
-  } else if constexpr (!GIVEN) {
-    hw.load(w_a_row, w_x_row);
+  constexpr int LDSG = WIDE ? bwd_lds_groups(NKG) : 0;
+  Frag* spill = nullptr;
+  if constexpr (LDSG > 0) {
+    __shared__ __attribute__((aligned(16))) Frag lds_hw[kWaves * 2 * LDSG * 64];
+    spill = lds_hw + w.wave * (2 * LDSG * 64);
   }
+  HeldWeights<IO, NKG, LDSG> hw;
+  hw.load(w_a_row, w_x_row, spill, w.lane);
   const float nba = -kLog2e * p.bias[w.kp], nbx = -kLog2e * p.bias[p.Wp + w.kp];   // biases as the sigmoids take them
   const float sp = p.sp[w.kp], cs = p.cs[w.kp];
   const bool ch_ok = !PAD || w.ch_ok;
@@ -224,34 +235,26 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
   float sum_ba = 0.f, sum_bx = 0.f, sum_l = 0.f;
   const Queue q = make_queue(p, w.unit, w.wg_in_unit, p.nC);
 
-  constexpr int VPR = TW / Tr::HW;
-  constexpr int NV = (TR * VPR + kThreads - 1) / kThreads;
-  constexpr int VPR_DY = kPackedWidth / Tr::HW;
-  constexpr int NV_DY = (TR * VPR_DY + kThreads - 1) / kThreads;
+  // A pass of the workgroup loads whole rows: RP rows of VPR vectors, so that the vectors of a lane lie at a fixed distance
+  // and one offset (memory and LDS) per lane serves them all.
+  constexpr int VPR = TW / Tr::HW, RP = kThreads / VPR, NV = (TR + RP - 1) / RP;
+  constexpr int VPR_DY = kPackedWidth / Tr::HW, RP_DY = kThreads / VPR_DY, NV_DY = TR / RP_DY;
+  static_assert(RP_DY * VPR_DY == kThreads && NV_DY * RP_DY == TR, "a pass over the dy tile fills the workgroup");
   Frag pre_x[NV], pre_dy[NV_DY], pre_ua[GIVEN ? NV : 1], pre_ux[GIVEN ? NV : 1];
-  unsigned pre_off[NV], dy_off[NV_DY], u_off[GIVEN ? NV : 1];
   // GIVEN: the tiles hold the 128 channels of this workgroup's four slabs
   const int group_col = (GIVEN || WIDE) ? (w.unit % p.groups) * kPackedWidth : 0;
   const int x_col = GIVEN ? w.k * p.bw + group_col : w.tile_col;
   const int dy_col = WIDE ? w.k * p.bw + group_col : x_col;
   const int own_col = WIDE ? group_col : 0;              // the dy tile's first column inside the x tile
   const unsigned u_row_bytes = 4u * (unsigned)p.bw;      // a row of `pre` and of du: two halves of bw 16-bit values
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int idx = tid + i * kThreads;
-    const int row = idx / VPR, cv = idx - row * VPR;
-    pre_off[i] = (idx < TR * VPR && (!PAD || cv * Tr::HW < p.bw)) ? (unsigned)row * row_bytes + (unsigned)(x_col + cv * Tr::HW) * 2u : kOutOfRange;
-    if constexpr (GIVEN)
-      u_off[i] = (idx < TR * VPR) ? (unsigned)row * u_row_bytes + (unsigned)(group_col + cv * Tr::HW) * 2u : kOutOfRange;
-  }
-#pragma unroll
-  for (int i = 0; i < NV_DY; ++i) {
-    const int idx = tid + i * kThreads;
-    const int row = idx / VPR_DY, cv = idx - row * VPR_DY;
-    // a wide block's last group may reach past the block: those columns belong to a wave without a slab
-    const bool in = idx < TR * VPR_DY && (!WIDE || own_col + cv * Tr::HW < p.bw);
-    dy_off[i] = in ? (unsigned)row * row_bytes + (unsigned)(dy_col + cv * Tr::HW) * 2u : kOutOfRange;
-  }
+  const int x_row = tid / VPR, x_cv = tid - x_row * VPR, dy_row = tid / VPR_DY, dy_cv = tid - dy_row * VPR_DY;
+  // offsets past every extent stay there when the distances of a lane's vectors are added; rows past the tile are past its extent
+  const unsigned pre_off = (x_row < RP && (!PAD || x_cv * Tr::HW < p.bw)) ? (unsigned)x_row * row_bytes + (unsigned)(x_col + x_cv * Tr::HW) * 2u : kOutOfRange;
+  const unsigned u_off = x_row < RP ? (unsigned)x_row * u_row_bytes + (unsigned)(group_col + x_cv * Tr::HW) * 2u : kOutOfRange;
+  // a wide block's last group may reach past the block: those columns belong to a wave without a slab
+  const unsigned dy_off = (!WIDE || own_col + dy_cv * Tr::HW < p.bw) ? (unsigned)dy_row * row_bytes + (unsigned)(dy_col + dy_cv * Tr::HW) * 2u : kOutOfRange;
+  IO* const x_at = lds_x + x_row * LDSROW + x_cv * Tr::HW;
+  IO* const dy_at = lds_dy + dy_row * DYROW + dy_cv * Tr::HW;
   auto decode = [&](unsigned tk, int& c, int& b) {
     const unsigned cr = tk / (unsigned)q.n_b;
     c = p.nC - 1 - (int)cr;
@@ -266,25 +269,58 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
     const long long first = ((long long)b * p.T + (long long)c * TR) * W;
     const rsrc_t rx = make_rsrc(x + first, (unsigned)rows * row_bytes);
     const rsrc_t rdy = make_rsrc(dy + first, (unsigned)rows * row_bytes);
+    unsigned xo = pre_off, dyo = dy_off;
+    hold_in_loop(xo); hold_in_loop(dyo);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) pre_x[i] = buf_load_frag<Frag>(rx, pre_off[i]);
+    for (int i = 0; i < NV; ++i) pre_x[i] = buf_load_frag<Frag>(rx, xo + (unsigned)(i * RP) * row_bytes);
 #pragma unroll
-    for (int i = 0; i < NV_DY; ++i) pre_dy[i] = buf_load_frag<Frag>(rdy, dy_off[i]);
+    for (int i = 0; i < NV_DY; ++i) pre_dy[i] = buf_load_frag<Frag>(rdy, dyo + (unsigned)(i * RP_DY) * row_bytes);
     if constexpr (GIVEN) {
       const IO* ubase = (const IO*)p.pre + ((long long)w.k * p.rows_total + (long long)b * p.T + (long long)c * TR) * (2 * p.bw);
       const rsrc_t ru = make_rsrc(ubase, (unsigned)rows * u_row_bytes);
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        pre_ua[i] = buf_load_frag<Frag>(ru, u_off[i]);
-        pre_ux[i] = buf_load_frag<Frag>(ru, u_off[i] == kOutOfRange ? kOutOfRange : u_off[i] + 2u * (unsigned)p.bw);
+        pre_ua[i] = buf_load_frag<Frag>(ru, u_off + (unsigned)(i * RP) * u_row_bytes);
+        pre_ux[i] = buf_load_frag<Frag>(ru, u_off + (unsigned)(i * RP) * u_row_bytes + 2u * (unsigned)p.bw);
       }
     }
   };
+  // the next ticket: one atomic instruction for the workgroup, live in its first lane only (atomicAdd would combine the lanes'
+  // operations first and wait for the result on the spot)
+  auto request_ticket = [&]() {
+    return (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, make_rsrc(q.counter, 4u), tid == 0 ? 0u : kOutOfRange, 0, 0);
+  };
+  // state in front of the lane's 16 tokens of the tile behind ticket tk: a checkpoint of the forward, or the initial state
+  // (two loads of which the offset drops one, and their sum)
+  float h_ckpt, h_init;
+  auto request_state = [&](unsigned tk) {
+    int c, b;
+    decode((long long)tk < q.tiles ? tk : 0u, c, b);
+    const int slot = 2 * c - 1 + hf;
+    const rsrc_t rck = make_rsrc(p.ckpt + (long long)b * p.ckpt_nC * W, (unsigned)p.ckpt_nC * row_bytes * 2u);
+    const rsrc_t rh0 = make_rsrc(p.h0, p.h0 ? (unsigned)p.B * row_bytes * 2u : 0u);
+    h_ckpt = BufIo<float>::load(rck, slot >= 0 ? ((unsigned)slot * (unsigned)p.W + (unsigned)w.ch) * 4u : kOutOfRange, 0u);
+    h_init = BufIo<float>::load(rh0, slot < 0 ? ((unsigned)b * (unsigned)p.W + (unsigned)w.ch) * 4u : kOutOfRange, 0u);
+  };
+  auto deposit = [&]() {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (x_row < RP && x_row + i * RP < TR) {
+        *reinterpret_cast<Frag*>(x_at + i * RP * LDSROW) = pre_x[i];
+        if constexpr (GIVEN) {
+          *reinterpret_cast<Frag*>(lds_pre + (x_at - lds_x) + i * RP * LDSROW) = pre_ua[i];
+          *reinterpret_cast<Frag*>(lds_pre + (x_at - lds_x) + (TR + i * RP) * LDSROW) = pre_ux[i];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV_DY; ++i) *reinterpret_cast<Frag*>(dy_at + i * RP_DY * DYROW) = pre_dy[i];
+  };
 
   // A pass of the loop ends with six 16-byte stores behind the loads of the next tile.  The wait for those loads at
-  // the top of the loop counts operations in issue order and must hold on every path into the loop, so the paths
-  // that store nothing (the first pass, a wave without a slab) issue six stores that their offset drops: the wait
-  // then leaves six operations in flight instead of draining the stores of the tile just finished.
+  // the top of the loop counts operations in issue order and must hold on every path into the loop, so the first
+  // pass is entered behind six stores that their offset drops: the wait then leaves six operations in flight
+  // instead of draining the stores of the tile just finished.
   auto six_dropped_stores = [&]() {
     const rsrc_t nowhere = make_rsrc(p.dx, 0u);
     const i32x4 nothing = {0, 0, 0, 0};
@@ -296,86 +332,63 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
   unsigned tk = s_ticket[0];
   int par = 0;
   issue(tk);
+  if (!w.slab_ok) {                                      // a wave without a slab only helps with the loads (wave 0 always has one)
+    while ((long long)tk < q.tiles) {
+      if constexpr (SHARED) lds_barrier();
+      deposit();
+      __syncthreads();
+      __syncthreads();
+      par ^= 1;
+      tk = s_ticket[par];
+      issue(tk);
+    }
+    return;
+  }
+  // The first records of a walk are requested as soon as the tile's own map is out where a sequence has at most two workgroups on
+  // it: the tile behind is then long finished (B16 T2048 W2560, 320-wide blocks: 321 against 343 us).  With more of them on one
+  // chain it is not, and the early look only comes back empty (B1 T32768: 458 against 420 us).
+  const unsigned ahead_lane = ch_ok && p.wg_per_unit <= 2 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
+  // Everything that the next tile needs early -- its tile, the state in front of it, the ticket after it -- is requested in front
+  // of the stores of this one: the counter that loads are waited for with counts in issue order, so whatever is requested
+  // behind the stores is waited for together with them.
+  request_state(tk);
+  unsigned next_raw = request_ticket();
   six_dropped_stores();
   while ((long long)tk < q.tiles) {
     int c, b;
     decode(tk, c, b);
     const int t0 = c * TR;
     const long long trow = (long long)b * p.T + t0 + hf * EL;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + i * kThreads;
-      const int row = idx / VPR, cv = idx - row * VPR;
-      if (idx < TR * VPR) {
-        *reinterpret_cast<Frag*>(lds_x + row * LDSROW + cv * Tr::HW) = pre_x[i];
-        if constexpr (GIVEN) {
-          *reinterpret_cast<Frag*>(lds_pre + row * LDSROW + cv * Tr::HW) = pre_ua[i];
-          *reinterpret_cast<Frag*>(lds_pre + (TR + row) * LDSROW + cv * Tr::HW) = pre_ux[i];
-        }
-      }
+    if constexpr (SHARED) {
+      __builtin_amdgcn_s_setprio(1);
+      lds_barrier();                                     // the stages of the tile before have been read
     }
-#pragma unroll
-    for (int i = 0; i < NV_DY; ++i) {
-      const int idx = tid + i * kThreads;
-      const int row = idx / VPR_DY, cv = idx - row * VPR_DY;
-      if (idx < TR * VPR_DY) *reinterpret_cast<Frag*>(lds_dy + row * DYROW + cv * Tr::HW) = pre_dy[i];
-    }
-    // the next ticket, the token flags (two bits per local step) and the state at the start of the chunk (forward
-    // checkpoint) are requested once the tile is in LDS: in front of it their latency would sit in the wait above
-    // (one atomic instruction for the workgroup, live in its first lane only: atomicAdd would combine the lanes'
-    // operations first and wait for the result on the spot)
-    const unsigned next_raw = (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, make_rsrc(q.counter, 4u), tid == 0 ? 0u : kOutOfRange, 0, 0);
-    unsigned flbits = 0u;
+    deposit();
+    unsigned flbits = 0u;                                // the token flags (two bits per local step)
     if constexpr (MASKED) flbits = flag_run(p, trow, t0 + hf * EL);
-    float h_start = 0.f;                                 // state in front of this lane's 16 tokens
-    if (c == 0 && hf == 0) { if (p.h0) h_start = p.h0[(long long)b * W + w.ch]; }
-    else h_start = p.ckpt[((long long)b * p.ckpt_nC + (2 * c - 1 + hf)) * W + w.ch];
+    const float h_start = h_ckpt + h_init;               // state in front of this lane's 16 tokens
     __syncthreads();
     f32x16 ua, ux;
     float xv[EL], gy[EL];
-    if (w.slab_ok) {
-      if constexpr (GIVEN) {
-        const int col = w.wave * 32 + w.r;
+    if constexpr (GIVEN) {
+      const int col = w.wave * 32 + w.r;
 #pragma unroll
-        for (int e = 0; e < EL; ++e) {
-          const int at = (hf * EL + e) * LDSROW + col;
-          xv[e] = (float)lds_x[at];
-          gy[e] = (float)lds_dy[(hf * EL + e) * DYROW + col];
-          ua[e] = (float)lds_pre[at];
-          ux[e] = (float)lds_pre[TR * LDSROW + at];
-        }
-      } else if constexpr (XLDS) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) { ua[v] = 0.0f; ux[v] = 0.0f; }     // the biases enter inside the sigmoids
-        const int kb = NKG >= 8 ? 0 : w.kb;
-        const IO* xrow = lds_x + tile_row<MT>(0, w.r) * LDSROW + kb + hf * Tr::HW;
-        const IO* brow = lds_wx + (w.wave * 32 + w.r) * WROW + hf * Tr::HW;
-#pragma unroll
-        for (int kg = 0; kg < NKG; ++kg) {
-          const Frag xa = *reinterpret_cast<const Frag*>(xrow + kg * Tr::KG);
-          Tr::mma(ua, xa, hw.a[kg]);
-          Tr::mma(ux, xa, *reinterpret_cast<const Frag*>(brow + kg * Tr::KG));
-        }
-#pragma unroll
-        for (int e = 0; e < EL; ++e) xv[e] = (float)lds_x[(hf * EL + e) * LDSROW + kb + w.slab * 32 + w.r];
-      } else {
-        gate_mfma_held<IO, MT, NKG, TW>(lds_x, hw, 0, w.slab, w.r, hf, 0.0f, 0.0f, ua, ux, xv, w.kb);
+      for (int e = 0; e < EL; ++e) {
+        const int at = (hf * EL + e) * LDSROW + col;
+        xv[e] = (float)lds_x[at];
+        gy[e] = (float)lds_dy[(hf * EL + e) * DYROW + col];
+        ua[e] = (float)lds_pre[at];
+        ux[e] = (float)lds_pre[TR * LDSROW + at];
       }
-      if constexpr (!GIVEN) {
+    } else {
+      gate_mfma_held<IO, MT, NKG, TW, LDSG>(lds_x, hw, 0, w.slab, w.r, hf, 0.0f, 0.0f, ua, ux, xv, w.kb, spill, w.lane);
 #pragma unroll
-        for (int e = 0; e < EL; ++e) gy[e] = (float)lds_dy[(hf * EL + e) * DYROW + (NKG >= 8 ? 0 : w.kb) + w.slab * 32 - own_col + w.r];
-      }
+      for (int e = 0; e < EL; ++e) gy[e] = (float)lds_dy[(hf * EL + e) * DYROW + w.slab * 32 - own_col + w.r];
     }
     if (tid == 0) s_ticket[par ^ 1] = next_raw;
     __syncthreads();
     par ^= 1;
     const unsigned tk_next = s_ticket[par];
-    if (!w.slab_ok) {                                    // a wave without a slab only helps with the loads
-      issue(tk_next);
-      six_dropped_stores();
-      tk = tk_next;
-      continue;
-    }
 
     // Gate recomputation in two steps.  The chunk's reverse map needs only the decay a_t (and dy),
     // so the recurrence gate comes first and the map is published before the rest of the gate math:
@@ -407,8 +420,12 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
     chain.rec = p.rec_a + seq; chain.stride = W;
     const bool last_chunk = c == p.nC - 1;
     if (!last_chunk && hf == 0 && ch_ok) carry_publish(chain, c, A_t, D_t, false);
+    CarryBatch<kDepth> ahead;
+    if constexpr (SHARED)
+      carry_prefetch<kDepth>(make_rsrc(p.rec_a + (long long)b * p.nC * W, (unsigned)p.nC * 4u * row_bytes), ahead_lane, 4u * row_bytes, c, +1, p.nC, ahead);
 
     // input gate and g = sqrt(1 - a^2)
+    if constexpr (!SHARED) {
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
       const float ie = sigmoid_fast(ux[e], nbx);
@@ -417,13 +434,16 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
       const float ge = __builtin_amdgcn_sqrtf(one_minus_a2<false>(l2, a[e]));
       gi[e] = ie; g[e] = ge;
     }
+    }
     float d_in = (last_chunk && p.dh_last) ? p.dh_last[(long long)b * W + w.ch] : 0.f;
-    if (!last_chunk) d_in = carry_lookback(chain, c, +1, p.nC, 0.f, ch_ok, p.limit, p.fail);
+    if (!last_chunk) d_in = SHARED ? carry_lookback_from<kDepth>(ahead, chain, c, +1, p.nC, 0.f, ch_ok, p.limit, p.fail)
+                                   : carry_lookback(chain, c, +1, p.nC, 0.f, ch_ok, p.limit, p.fail);
     // the next tile's loads go out behind the look-back: loads return in issue order, so requested in front of it
     // they would put their latency into every round trip of the walk
-    issue(tk_next);
+    if constexpr (!SHARED) { issue(tk_next); request_state(tk_next); next_raw = request_ticket(); }
     const float d_out = fmaf(A_t, d_in, D_t);
     if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
+    if constexpr (SHARED) __builtin_amdgcn_s_setprio(0);
     if (hf == 0 && c == 0 && p.dh0 && ch_ok) p.dh0[(long long)b * W + w.ch] = d_out;
 
     // delta_t in place of dy_t (reverse), then one forward pass that carries h_{t-1} along
@@ -442,14 +462,30 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
       const float xe = xv[e];
       // the factors below do not depend on delta; tying them to it keeps the compiler from computing
       // all of them before the look-back, where they would only occupy registers
-      float ge = g[e], ie = gi[e], re = r[e];
-      asm volatile("" : "+v"(ge), "+v"(ie), "+v"(re) : "v"(d));
+      float ge, ie, re = r[e];
+      if constexpr (SHARED) {
+        float ue = ux[e];
+        asm volatile("" : "+v"(ue), "+v"(re) : "v"(d));
+        ie = sigmoid_fast(ue, nbx);
+        float l2 = re * sp;
+        if constexpr (MASKED) {
+          unsigned fl = flbits;
+          asm volatile("" : "+v"(fl));
+          l2 = masked_log2_decay_run(l2, fl, e);                             // gives g = 1 / g = 0
+        }
+        ge = __builtin_amdgcn_sqrtf(one_minus_a2<false>(l2, a[e]));
+      } else {
+        ge = g[e]; ie = gi[e];
+        asm volatile("" : "+v"(ge), "+v"(ie), "+v"(re) : "v"(d));
+      }
       const float c1 = ge * ie;
       const float dxd = d * c1;
       const float ze = c1 * xe;
       // 2 q with q = i x / sqrt(max(4 g^2, 1e-6)): the factors 4 and 2 cancel exactly (powers of two)
       const float q2 = (ie * xe) * __builtin_amdgcn_rsqf(fmaxf(ge * ge, 0.25f * 1e-6f));
-      float dl = (a[e] * d) * fmaf(-a[e], q2, h);
+      float ae = a[e];
+      if constexpr (SHARED) asm volatile("" : "+v"(ae));     // a d again, not kept from the reverse recurrence
+      float dl = (ae * d) * fmaf(-ae, q2, h);
       // A reset token has a = 2^-126, which already switches dl off; a padded one has g = 0, which
       // zeroes dxd, vx and z, but its bounded-sqrt term would leak into dl.
       if constexpr (MASKED) { if ((flbits >> (2 * e)) & 2u) dl = 0.f; }
@@ -467,27 +503,31 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? 1 : 2)) void bwd_scan_kernel(F
         io2 pair; pair[0] = (IO)va; pair[1] = (IO)vx;
         *reinterpret_cast<io2*>(my_du + e * PairStage<TR>::kRowBytes) = pair;
       }
+      if constexpr (SHARED) { if (e & 1) __builtin_amdgcn_sched_barrier(0); }
     }
+    if constexpr (SHARED) { issue(tk_next); request_state(tk_next); next_raw = request_ticket(); }
     wave_lds_fence();
     {
+      unsigned fl_lane = (unsigned)w.lane;               // the offsets of the stores: a register each if they stayed between tiles
+      hold_in_loop(fl_lane);
       const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
       const rsrc_t rdx = make_rsrc((const IO*)p.dx + ((long long)b * p.T + t0) * W, (unsigned)rows * row_bytes);
-      stage_flush<TR>(stage_dx, rdx, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, w.lane, !PAD || w.slab * 32 + (w.lane & 3) * 8 < p.bw);
+      stage_flush<TR>(stage_dx, rdx, row_bytes, (unsigned)(w.k * p.bw + w.slab * 32) * 2u, (int)fl_lane, !PAD || w.slab * 32 + (int)(fl_lane & 3) * 8 < p.bw);
       if constexpr (GIVEN) {
         IO* dbase = (IO*)p.du_a + ((long long)w.k * p.rows_total + (long long)b * p.T + t0) * (2 * p.bw);
         const rsrc_t rdu = make_rsrc(dbase, (unsigned)rows * u_row_bytes);
-        stage_flush<TR>(stage_du, rdu, u_row_bytes, (unsigned)(w.slab * 32) * 2u, w.lane);
-        stage_flush<TR>(stage_du + WaveStage<TR>::kBytes, rdu, u_row_bytes, (unsigned)(p.bw + w.slab * 32) * 2u, w.lane);
+        stage_flush<TR>(stage_du, rdu, u_row_bytes, (unsigned)(w.slab * 32) * 2u, (int)fl_lane);
+        stage_flush<TR>(stage_du + WaveStage<TR>::kBytes, rdu, u_row_bytes, (unsigned)(p.bw + w.slab * 32) * 2u, (int)fl_lane);
       } else {
       const unsigned du_row_bytes = 2u * row_bytes;
       const rsrc_t rdu = make_rsrc((const IO*)p.du_a + ((long long)b * p.T + t0) * 2 * W, (unsigned)rows * du_row_bytes);
       const unsigned du_col = (unsigned)(w.k * 2 * p.bw + w.slab * 64) * 2u;
 #pragma unroll
       for (int i = 0; i < TR / 8; ++i) {
-        const int row = 8 * i + (w.lane >> 3);
-        const unsigned seg = (unsigned)(w.lane & 7) * 16u;
+        const int row = 8 * i + (int)(fl_lane >> 3);
+        const unsigned seg = (fl_lane & 7) * 16u;
         i32x4 v = *reinterpret_cast<const i32x4*>(stage_du + PairStage<TR>::row_offset(row) + seg);
-        buf_store_b128(v, rdu, !PAD || w.slab * 32 + (w.lane & 7) * 4 < p.bw ? (unsigned)row * du_row_bytes + du_col + seg : kOutOfRange);
+        buf_store_b128(v, rdu, !PAD || w.slab * 32 + (int)(fl_lane & 7) * 4 < p.bw ? (unsigned)row * du_row_bytes + du_col + seg : kOutOfRange);
       }
       }
     }
@@ -543,10 +583,6 @@ RGLRU_DEVICE bf16x8 gate_backward(bf16x8& d, const bf16x8& h, const bf16x8& v, f
   }
   return dv;
 }
-
-// Keeps what is computed from v inside the loop that it stands in: the offsets of a tile's rows, hoisted out of it, take a
-// register each and push the scan kernels into scratch memory (140 bytes a lane instead of 48).
-RGLRU_DEVICE void hold_in_loop(unsigned& v) { asm volatile("" : "+v"(v)); }
 
 // GATED, in the two scan kernels: the output gate's reverse mode on the way in.  As a kernel of its own it read y, v and the
 // gradient and wrote two gradients, one of which the scan read back: 31 us next to the scan's 31 us at B8 T2048 W1024.
@@ -2234,7 +2270,7 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   const int nkg = wide_groups(g, dtype, 1);
   const bool pad = wide_padded(g);
   // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums
-  a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 1, L.max_wg);
+  a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, bwd_wide_occ(nkg), L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
   const bool masked = (flags != nullptr) || a.first_reset || (T % kChunk != 0);
   a.xcd_map = 1;
