@@ -105,6 +105,7 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
     const unsigned uW = (unsigned)W, ch = (unsigned)w.ch;
     const bool lower = ch_ok && hf == 0;
     rec_store_buf(seq_records(p, b), lower ? ((unsigned)c * uW + ch) * 8u : kOutOfRange, 0.f, h_end);
+    __builtin_amdgcn_s_setprio(0);
     const rsrc_t rhl = make_rsrc(p.h_last, p.h_last ? (unsigned)p.B * uW * 4u : 0u);
     BufIo<float>::store(h_end, rhl, (lower && c == p.nCf - 1) ? ((unsigned)b * uW + ch) * 4u : kOutOfRange, 0u);
   }
@@ -349,7 +350,11 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
     const bool slab_ok = (NKG == 8) ? true : w.slab_ok;
     const rsrc_t rticket = make_rsrc(q.counter, 4u);
     const unsigned rec_stride = (unsigned)W * 8u;
-    const unsigned rec_lane = (slab_ok && w.ch_ok) ? (unsigned)w.ch * 8u : kOutOfRange;
+    // The first records of a walk are requested behind the tile's own map, across the barrier and the next tile's loads, where a
+    // sequence has at most two workgroups on it.  With more of them the chunk in front is not out yet and the early look comes back
+    // empty; so does one at the top of the tile, the place it had before.  Forward alone, us, with the priority above: B16 T2048
+    // W2560 238 -> 228, the block's forward at B8 T2048 W1024 53 -> 49 (16 gate blocks), B1 T32768 W2560 294 (315 when it looked).
+    const unsigned rec_lane = (slab_ok && w.ch_ok) && p.wg_per_unit <= 2 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
     // A dead finalize in front of the loop: the loop is entered with the same memory operations in
     // flight as its back edge has, so the waits at its top are exact instead of worst case.
     bf16x8 gate_rows[BLOCK ? TR / 16 : 1];               // the lane's vectors of the second projection
@@ -368,10 +373,9 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
       for (int mt = 0; mt < MT; ++mt) flbits[mt] = MASKED ? flag_run(p, trow + 16 * mt, cur.c * TR + hf * EL + 16 * mt) : 0u;
       // next ticket: one instruction for the whole workgroup, live only in its first lane
       const unsigned next_raw = (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, rticket, tid == 0 ? 0u : kOutOfRange, 0, 0);
-      // records this tile will need: requested now, used after its gate math
-      CarryBatch<kFwdDepth> ahead;
-      carry_prefetch<kFwdDepth>(make_rsrc(p.rec_a + (long long)cur.b * p.nCf * W, (unsigned)p.nCf * rec_stride), rec_lane,
-                       rec_stride, cur.c, -1, -1, ahead);
+      // From here until its carry is out, the tile is what other workgroups wait for: its waves go before those of the
+      // workgroup that shares their SIMDs and is storing (forward alone, us: B256 T2048 W1024 831 -> 808, B8 T2048 W2560 109 -> 106).
+      __builtin_amdgcn_s_setprio(1);
       if constexpr (BLOCK) {
         const int t0 = cur.c * TR;
         const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
@@ -468,6 +472,9 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
         }
       }
       fwd_local<MT, MASKED>(p, w, cur, slab_ok);
+      CarryBatch<kFwdDepth> ahead;
+      carry_prefetch<kFwdDepth>(make_rsrc(p.rec_a + (long long)cur.b * p.nCf * W, (unsigned)p.nCf * rec_stride), rec_lane,
+                       rec_stride, cur.c, -1, -1, ahead);
       if (tid == 0) s_ticket[par ^ 1] = next_raw;
       __syncthreads();
       par ^= 1;
