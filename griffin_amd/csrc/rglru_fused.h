@@ -606,6 +606,12 @@ inline int pick_queues(long long B, int wg) {
 }
 
 
+// rglru_fwd_rows.hip: the forward of batches large enough that every workgroup can own whole sequences (16-bit storage, blocks of
+// up to 128 channels).
+int fwd_rows_tile(int nkg);
+int fwd_rows_per_cu(int nkg);
+int launch_fwd_rows(const FusedArgs& a, int nkg, bool pad, hipStream_t s);
+
 // Whether the forward runs one workgroup per chain (fwd_chain_kernel) instead of tiles with look-back:
 // 0 = by shape, 1 = never, 2 = whenever that kernel covers the shape (tests).
 inline std::atomic<int> g_chain_forward{0};

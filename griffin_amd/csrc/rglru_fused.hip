@@ -878,6 +878,19 @@ struct BlockFwd {
 };
 
 
+// Workgroups per unit of the kernel whose workgroups own whole sequences (rglru_fwd_rows.hip), or 0 where the tiled kernel is the
+// better one.  It needs a sequence for every workgroup that fits the chip, and rounds of sequences that are mostly full, or the
+// last round idles: forward at T512 W1024 in 128-wide blocks, us, tiled -> rows, 64 workgroups a unit: 64 sequences 53 -> 49, 96 (two
+// rounds, three quarters full) 74 -> 66, 129 111 -> 108, 80 63 -> 64, 65 54 -> 61; 48 sequences 44 -> 47.  Tiles with flags cost the tiled
+// kernel a third more and this one only where a flag is: B96 T700 W1024 packed 141 -> 104.
+static int fwd_row_workgroups(int64_t B, const Geometry& g, int nkg, bool flags) {
+  FusedArgs a;
+  a.units = (int)g.units;
+  pack_units(a, g, nkg);
+  const int64_t slots = pick_wg_per_unit(a.units, 1ll << 40, fwd_rows_per_cu(nkg), 1 << 20), rounds = (B + slots - 1) / slots;
+  return B >= slots && 100 * B >= (flags ? 60 : 75) * slots * rounds ? (int)slots : 0;
+}
+
 static int fwd_impl(const void* x, const void* prep, const float* h0, const uint8_t* flags,
                     void* y, float* h_last, void* ws,
                     int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, bool cleared, void* stream,
@@ -936,7 +949,8 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   // The tiled kernels need the forward records, tickets and failure word zeroed; the chain kernel needs the
   // failure word only and clears it itself.  (Every backward entry point that uses records clears its own.)
   const bool chain = !blk && !pre && narrow && fwd_chain_pays(B, T, g.Wp);
-  if (!cleared && !chain) {
+  const int row_wg = blk || pre || !narrow || chain ? 0 : fwd_row_workgroups(B, g, nkg, flags != nullptr);
+  if (!cleared && !chain && !row_wg) {
     rc = launch_clear(wb, L.f_begin, L.f_end, s);
     if (rc) return rc;
   }
@@ -946,7 +960,9 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   const bool fused_prepare = fuse && chain && fuse->rows_ok;
   if (fuse && !fused_prepare) {
     PrepArgs pa = *fuse;
+    const long long own = (long long)(L.f_end - L.f_begin) / 16;    // this pass's region; the backward's may follow it
     if (chain) { pa.clear = nullptr; pa.clear_n = 0; }
+    else if (row_wg) { pa.clear_n = pa.clear_n > own ? pa.clear_n - own : 0; pa.clear = pa.clear_n ? pa.clear + own : nullptr; }
     rc = launch_prepare(pa, dtype, stream);
     if (rc) return rc;
   }
@@ -978,6 +994,12 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     return check_launch("fwd");
   }
   pack_units(a, g, nkg);
+  if (row_wg) {
+    a.nCf = (int)((T + fwd_rows_tile(nkg) - 1) / fwd_rows_tile(nkg));
+    a.wg_per_unit = row_wg;
+    KernelTimer timer(0, s);
+    return launch_fwd_rows(a, nkg, pad, s);
+  }
   const int tile_tokens = 32 * fwd_mt(nkg);
   a.nCf = (int)((T + tile_tokens - 1) / tile_tokens);
   // without weights in registers three workgroups fit a compute unit

@@ -1043,3 +1043,28 @@ def test_wide_backward_with_few_and_many_workgroups_on_a_sequence(bw, B, T, mask
     errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
     for name, err in errs.items():
         assert err < BF16_TOL, (name, err)
+
+
+@pytest.mark.parametrize("bw,nb,B", [(128, 1, 512), (128, 1, 600), (88, 1, 512), (64, 2, 768), (64, 3, 390), (40, 2, 770), (32, 4, 768), (8, 1, 768)])
+@pytest.mark.parametrize("T,masks,with_h0", [(64, False, False), (70, True, True), (33, False, True), (1, False, True)])
+def test_forward_of_batches_that_fill_the_chip_with_sequences(bw, nb, B, T, masks, with_h0):
+    """Batches with a sequence for every workgroup run the forward whose workgroups own whole sequences: full and ragged tiles,
+    flags in some tiles, a second round of sequences, packed and padded blocks, a last unit that is not full; outputs, final state
+    and the gradients that the backward computes from its checkpoints."""
+    from griffin_amd import set_chain_forward
+
+    W = bw * nb
+    _say("sequences per workgroup", bw, nb, B, T, masks, with_h0)
+    case = orc.make_case(B, T, W, nb, seed=bw + T, h0_std=0.5 if with_h0 else 0.0, bias_std=0.5)
+    reset, active = _masks(B, T, masks)
+    dh_last = torch.randn(B, W, generator=torch.Generator().manual_seed(6)) if with_h0 else None
+    was = set_chain_forward(1)
+    try:
+        y, h_last, grads = hip_run(case, torch.bfloat16, reset, active, dh_last)
+    finally:
+        set_chain_forward(was)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, active, dh_last)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
