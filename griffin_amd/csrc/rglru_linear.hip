@@ -17,6 +17,12 @@
 // one that lies the other way round is read with the transposing LDS loads (16-bit types), or element by element (fp32).
 // Edges of M, N and K are masked through the offsets of buffer loads, so any size works as long as rows are whole 16-byte
 // vectors.
+// What bounds it: neither the matrix unit nor memory.  With the products or the loads taken out (timing builds) two products of
+// 2331 x 1024 x 768 in bf16 take the same 20 us: 3.7 us until the first slice is there, 6 us for one slice and the result, then
+// 0.9 us a slice, of which the LDS writes (13.8 clocks a KB on a compute unit, reads 4.3) and the barrier are most; 304 tiles leave
+// 48 compute units with two.  us before -> with the order of a slice below, operand pointers outside the loop and results staged
+// four columns at a time: 2331 x 2 x 1024 x 768 21.3 -> 20.2, x 768 x 1024 13.1 -> 11.6; 800 tokens, both 23.6 -> 19.8;
+// gate gradients of B4 T1024 W1024 in fp32 39.5 -> 37.  More slices in flight (3, 4 or 6) and tiles of 128 x 64: no gain.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -46,6 +52,7 @@ struct LinearArgs {
 // is one contraction index, else one result index.
 template <typename IO, bool T, int ROWS, int THREADS>
 struct OperandTile {
+  static constexpr int RING = 2;     // slices on their way from memory
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
   static constexpr int HW = Tr::HW, BK = 8 * HW;                              // 128 bytes
@@ -56,9 +63,9 @@ struct OperandTile {
   static constexpr int kElems = kLines * kStride;
   static constexpr int VPR = kLineElems / HW, NV = kLines * VPR / THREADS;
   static_assert(kLines * VPR % THREADS == 0, "whole vectors per thread");
-  Frag v[NV];
+  Frag v[RING][NV];
   unsigned off[NV];                  // lane offsets in bytes, kOutOfRange past the last result index
-  unsigned live;                     // masked weight gradient: bit i = the token of vector i takes part
+  unsigned live[RING];               // masked weight gradient: bit i = the token of vector i takes part
 
   RGLRU_DEVICE void setup(int tid, long long ld, int limit) {               // limit: result indices left in the tile
 #pragma unroll
@@ -67,10 +74,10 @@ struct OperandTile {
       const int index = T ? cv * HW : line;
       off[i] = index < limit ? (unsigned)((long long)line * ld * (int)sizeof(IO)) + (unsigned)(cv * HW) * (unsigned)sizeof(IO) : kOutOfRange;
     }
-    live = ~0u;
+    live[0] = live[1] = ~0u;
   }
-  // base: first element of the slice (uniform); k_left: contraction indices left
-  RGLRU_DEVICE void request(const IO* base, long long ld, int k_left, int limit, int tid, const unsigned char* active = nullptr) {
+  // q: slot of the ring; base: first element of the slice (uniform); k_left: contraction indices left
+  RGLRU_DEVICE void request(int q, const IO* base, long long ld, int k_left, int limit, int tid, const unsigned char* active = nullptr) {
     const int lines = T ? (k_left < BK ? (k_left < 0 ? 0 : k_left) : BK) : (limit < ROWS ? limit : ROWS);
     const rsrc_t r = make_rsrc(base, k_left > 0 ? (unsigned)((long long)lines * ld) * (unsigned)sizeof(IO) : 0u);
 #pragma unroll
@@ -80,22 +87,22 @@ struct OperandTile {
         const int cv = (tid + i * THREADS) % VPR;
         if (cv * HW >= k_left) o = kOutOfRange;
       }
-      v[i] = buf_load_frag<Frag>(r, o);
+      v[q][i] = buf_load_frag<Frag>(r, o);
     }
     if (T && active) {
       const rsrc_t ra = make_rsrc(active, (unsigned)lines);
-      live = 0u;
+      live[q] = 0u;
 #pragma unroll
       for (int i = 0; i < NV; ++i)
-        live |= (__builtin_amdgcn_raw_buffer_load_b8(ra, (unsigned)((tid + i * THREADS) / VPR), 0, 0) & 0xff) ? 1u << i : 0u;
+        live[q] |= (__builtin_amdgcn_raw_buffer_load_b8(ra, (unsigned)((tid + i * THREADS) / VPR), 0, 0) & 0xff) ? 1u << i : 0u;
     }
   }
-  RGLRU_DEVICE void deposit(IO* lds, int tid, bool masked = false) const {
+  RGLRU_DEVICE void deposit(int q, IO* lds, int tid, bool masked = false) const {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = tid + i * THREADS, line = idx / VPR, cv = idx - line * VPR;
-      Frag f = v[i];
-      if (T && masked && !((live >> i) & 1u)) f = Tr::zero();
+      Frag f = v[q][i];
+      if (T && masked && !((live[q] >> i) & 1u)) f = Tr::zero();
       *reinterpret_cast<Frag*>(lds + line * kStride + cv * HW) = f;
     }
   }
@@ -116,6 +123,13 @@ struct OperandTile {
 };
 
 constexpr int kLinearThreads = 256;
+
+// Four consecutive elements (N is a multiple of a 16-byte vector, so they lie wholly inside or outside a row).
+template <typename IO> RGLRU_DEVICE auto buf_load_four(rsrc_t r, unsigned voff) {
+  typedef IO io4 __attribute__((ext_vector_type(4)));
+  if constexpr (sizeof(IO) == 2) return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
+  else return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
+}
 
 template <typename IO, bool TA, bool TB, int BM, int BN>
 __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
@@ -156,15 +170,22 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   TileB tb;
   ta.setup(tid, p.lda, m_left);
   tb.setup(tid, p.ldb, n_left);
-  auto request = [&](int s) {
-    const int seg = s >= slices ? 1 : 0;
-    const int k = k_begin + (s - seg * slices) * BK;
-    const IO* a = (const IO*)p.a[p.segments > 1 ? seg : (TA ? problem : 0)] + item * p.a_step;
-    const IO* b = (const IO*)p.b[p.segments > 1 ? seg : (TA ? 0 : problem)] + item * p.b_step;
+  // the segments' operands, read from the arguments once: inside the loop that would be a scalar load and a wait for it a slice
+  const IO* const a_first = (const IO*)p.a[p.segments > 1 ? 0 : (TA ? problem : 0)] + item * p.a_step;
+  const IO* const b_first = (const IO*)p.b[p.segments > 1 ? 0 : (TA ? 0 : problem)] + item * p.b_step;
+  const IO* const a_second = p.segments > 1 ? (const IO*)p.a[1] + item * p.a_step : a_first;
+  const IO* const b_second = p.segments > 1 ? (const IO*)p.b[1] + item * p.b_step : b_first;
+  const unsigned char* const active = masked ? p.active : nullptr;
+  const long long lda = p.lda, ldb = p.ldb;
+  auto request = [&](int q, int s) {
+    const bool second = s >= slices;
+    const int k = k_begin + (s - (second ? slices : 0)) * BK;
+    const IO* a = second ? a_second : a_first;
+    const IO* b = second ? b_second : b_first;
     const int left = s < total_slices ? k_end - k : 0;
     const long long ks = s < total_slices ? k : 0;
-    ta.request(a + (TA ? ks * p.lda + m0 : m0 * p.lda + ks), p.lda, left, m_left, tid, masked ? p.active + ks : nullptr);
-    tb.request(b + (TB ? ks * p.ldb + n0 : n0 * p.ldb + ks), p.ldb, left, n_left, tid);
+    ta.request(q, a + (TA ? ks * lda + m0 : m0 * lda + ks), lda, left, m_left, tid, masked ? active + ks : nullptr);
+    tb.request(q, b + (TB ? ks * ldb + n0 : n0 * ldb + ks), ldb, left, n_left, tid);
   };
   constexpr int kBuffer = TileA::kElems + TileB::kElems;
 
@@ -175,38 +196,39 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+  // The weights are the products' first operand, so an accumulator's lane has ONE row of the result (m = r) and runs of four
+  // columns (n = 8 (v / 4) + 4 hf + v % 4): what is loaded, staged and stored below are vectors of four.
+  typedef IO io4 __attribute__((ext_vector_type(4)));
   if (p.accumulate) {
     const rsrc_t rc = make_rsrc((const IO*)p.c[problem] + item * p.c_step + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int n = wn * (BN / 2) + 32 * j + r;
+    for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = wm * (BM / 2) + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
-          acc[i][j][v] = BufIo<IO>::load(rc, n < n_left ? ((unsigned)m * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange, 0u);
+        for (int g = 0; g < 4; ++g) {
+          const int n = wn * (BN / 2) + 32 * j + 8 * g + 4 * hf, m = wm * (BM / 2) + 32 * i + r;
+          const io4 c = buf_load_four<IO>(rc, n < n_left ? ((unsigned)m * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)c[e];
         }
-    }
   }
   float sum[MI];                                             // column sums of A over the lane's share of K
 #pragma unroll
   for (int i = 0; i < MI; ++i) sum[i] = 0.f;
   const bool sums = TA && p.colsum && tn == 0 && wn == 0;
 
-  request(0);
-  ta.deposit(lds, tid, masked);
-  tb.deposit(lds + TileA::kElems, tid);
-  request(1);
+  request(0, 0);
+  request(1, 1);
+  ta.deposit(0, lds, tid, masked);
+  tb.deposit(0, lds + TileA::kElems, tid);
   __syncthreads();
-  for (int s = 0; s < total_slices; ++s) {
-    const IO* cur = lds + (s & 1) * kBuffer;
-    IO* nxt = lds + ((s & 1) ^ 1) * kBuffer;
-    ta.deposit(nxt, tid, masked);
-    tb.deposit(nxt + TileA::kElems, tid);
-    request(s + 2);
+  // Slice s is multiplied out of one buffer while slice s + 1 goes from registers to the other and slice s + 2 is requested.  The
+  // order inside a slice: requests first (left to itself the compiler sinks them to the end, where they cover nothing), then half of
+  // the products, whose LDS reads would otherwise queue behind the writes, then the writes, then the other half.
+  auto multiply = [&](const IO* cur, int from) {
 #pragma unroll
-    for (int kg = 0; kg < KGS; ++kg) {
+    for (int kg = from; kg < from + KGS / 2; ++kg) {
       Frag fa[MI], fb[NI];
 #pragma unroll
       for (int i = 0; i < MI; ++i) fa[i] = TileA::fragment(cur, wm * (BM / 2) + 32 * i, kg, lane);
@@ -215,7 +237,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) Tr::mma(acc[i][j], fa[i], fb[j]);
+        for (int j = 0; j < NI; ++j) Tr::mma(acc[i][j], fb[j], fa[i]);
       if (sums) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -223,7 +245,22 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
           for (int e = 0; e < Tr::HW; ++e) sum[i] += (float)fa[i][e];
       }
     }
-    __syncthreads();
+  };
+  for (int s0 = 0; s0 < total_slices; s0 += 2) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {                            // the parity names buffer and slot
+      const int s = s0 + u;
+      if (s >= total_slices) break;
+      const IO* cur = lds + u * kBuffer;
+      IO* nxt = lds + (u ^ 1) * kBuffer;
+      request(u, s + 2);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(cur, 0);
+      ta.deposit(u ^ 1, nxt, tid, masked);
+      tb.deposit(u ^ 1, nxt + TileA::kElems, tid);
+      multiply(cur, KGS / 2);
+      __syncthreads();
+    }
   }
 
   if (sums) {
@@ -239,36 +276,49 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     const int ld = p.partial_ld ? p.partial_ld : p.N, rows = p.partial_ld ? p.partial_ld : p.M;
     float* part = p.partial + ((((long long)split * p.batch + item) * p.problems + problem) * rows + m0) * ld + n0;
     const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * ld) * 4u);
+    // through LDS like the result: stored from the accumulators, a row of the wave's tile is 32 bytes an instruction (two weight
+    // gradients of 2048 x 1024 x 768: 45 us that way, 42 element by element, 41 like this)
+    constexpr int kRow = BN / 2 + 4;
+    static_assert(4 * (BM / 2) * kRow * 4 <= (int)sizeof(lds), "the fp32 tile fits where the slices were");
+    float* stage = reinterpret_cast<float*>(lds) + wave * (BM / 2) * kRow;
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      const int n = col0 + 32 * j + r;
+    for (int j = 0; j < NI; ++j)
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int m = row0 + 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
-          BufIo<float>::store(acc[i][j][v], rc, n < n_left ? ((unsigned)m * (unsigned)ld + (unsigned)n) * 4u : kOutOfRange, 0u);
+        for (int g = 0; g < 4; ++g) {
+          f32x4 c;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) c[e] = acc[i][j][4 * g + e];
+          *reinterpret_cast<f32x4*>(stage + (32 * i + r) * kRow + 32 * j + 8 * g + 4 * hf) = c;
         }
+    wave_lds_fence();
+    constexpr int VPR = (BN / 2) / 4, ROWS = 64 / VPR;
+#pragma unroll
+    for (int q = 0; q < (BM / 2) / ROWS; ++q) {
+      const int m = q * ROWS + lane / VPR, cv = lane % VPR, row = row0 + m, n = col0 + cv * 4;
+      const i32x4 c = *reinterpret_cast<const i32x4*>(stage + m * kRow + cv * 4);
+      buf_store_b128(c, rc, n < n_left && row < m_left ? ((unsigned)row * (unsigned)ld + (unsigned)n) * 4u : kOutOfRange);
     }
     return;
   }
   // result in the storage type: through LDS (the slices have been read), then 16-byte vectors of rows
-  float bias[NI];
-#pragma unroll
-  for (int j = 0; j < NI; ++j) {
-    const int n = col0 + 32 * j + r;
-    bias[j] = (p.bias[problem] && n < n_left) ? (float)((const IO*)p.bias[problem])[n0 + n] : 0.f;
-  }
+  const rsrc_t rb = make_rsrc((const IO*)p.bias[problem] + n0, p.bias[problem] ? (unsigned)n_left * (unsigned)sizeof(IO) : 0u);
   IO* stage = lds + wave * (BM / 2) * kStageRow;
 #pragma unroll
-  for (int i = 0; i < MI; ++i)
+  for (int j = 0; j < NI; ++j)
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
+    for (int g = 0; g < 4; ++g) {
+      const int n = 32 * j + 8 * g + 4 * hf;
+      const io4 bias = buf_load_four<IO>(rb, (unsigned)(col0 + n) * (unsigned)sizeof(IO));
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = 32 * i + 8 * (v >> 2) + 4 * hf + (v & 3);
-        stage[m * kStageRow + 32 * j + r] = (IO)(acc[i][j][v] + bias[j]);
+      for (int i = 0; i < MI; ++i) {
+        io4 c;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[e] = (IO)(acc[i][j][4 * g + e] + (float)bias[e]);
+        *reinterpret_cast<io4*>(stage + (32 * i + r) * kStageRow + n) = c;
       }
+    }
   wave_lds_fence();
   const rsrc_t rc = make_rsrc((IO*)p.c[problem] + item * p.c_step + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
   constexpr int VPR = (BN / 2) / Tr::HW, ROWS = 64 / VPR;
