@@ -1068,3 +1068,23 @@ def test_forward_of_batches_that_fill_the_chip_with_sequences(bw, nb, B, T, mask
     errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
     for name, err in errs.items():
         assert err < BF16_TOL, (name, err)
+
+
+@pytest.mark.parametrize("B", [1016, 1018])
+def test_scan_op_gradients_below_and_above_the_cache(B):
+    """From 256 MB of gradients on they are stored past the caches: two runs of tokens, either side of the line, against the loop."""
+    from griffin_amd import hip_rglru_scan
+
+    T, W = 129, 256
+    assert (8 * B * T * W >= 256 << 20) == (B == 1018)
+    _say("scan gradients", B)
+    gen = torch.Generator().manual_seed(0)
+    a = torch.sigmoid(torch.randn(B, T, W, generator=gen) + 2.0)
+    z, dh = torch.randn(B, T, W, generator=gen), torch.randn(B, T, W, generator=gen)
+    h0 = torch.randn(B, W, generator=gen)
+    want = orc.scan_autograd(a, z, h0, dh)
+    leaves = [t.cuda().requires_grad_(True) for t in (a, z, h0)]
+    h = hip_rglru_scan(*leaves)
+    grads = torch.autograd.grad(h, leaves, dh.cuda())
+    errs = [rel_err(h, want[0])] + [rel_err(g, w) for g, w in zip(grads, want[1:])]
+    assert max(errs) < FP32_TOL, errs
