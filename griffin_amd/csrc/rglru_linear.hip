@@ -8,25 +8,30 @@
 //
 // Why not the BLAS library alone: a call of it costs the host 17 us, seven calls of it are a third of the host time of a
 // training step of the block, which is what bounds such a step up to several thousand tokens; and it takes no row mask and
-// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 59 us against 70 us, 735 TFLOP/s,
+// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 52 us against 65 us, 795 TFLOP/s,
 // here; the split weight gradient of the same 52 us against 91 us), so callers choose by the size of the product.
 //
-// A workgroup of four waves owns a BM x BN tile of C; K is walked in slices of 128 bytes.  A slice of both operands goes
-// through registers (requested one slice ahead) into one of two LDS buffers, one barrier a slice.  An operand that lies in
-// memory with its contraction index contiguous is read from LDS as 16-byte rows (row stride 144 bytes: no bank conflicts);
-// one that lies the other way round is read with the transposing LDS loads (16-bit types), or element by element (fp32).
+// A workgroup of four waves owns a BM x BN tile of C; K is walked in slices of 128 bytes, one barrier a slice.  Where both operands
+// lie with their contraction index contiguous (forward) a slice goes from memory to LDS directly (DirectTile), one slice ahead
+// (128 x 128) or two (64 x 64).  Otherwise it goes through registers (requested one slice ahead) into one of two LDS buffers: an
+// operand with its contraction index contiguous is read back as 16-byte rows (row stride 144 bytes: no bank conflicts); one that
+// lies the other way round is read with the transposing LDS loads (16-bit types), or element by element (fp32).
 // Edges of M, N and K are masked through the offsets of buffer loads, so any size works as long as rows are whole 16-byte
 // vectors.
-// What bounds it: neither the matrix unit nor memory.  With the products or the loads taken out (timing builds) two products of
-// 2331 x 1024 x 768 in bf16 take the same 20 us: 3.7 us until the first slice is there, 6 us for one slice and the result, then
-// 0.9 us a slice, of which the LDS writes (13.8 clocks a KB on a compute unit, reads 4.3) and the barrier are most; 304 tiles leave
-// 48 compute units with two.  us before -> with the order of a slice below, operand pointers outside the loop and results staged
-// four columns at a time: 2331 x 2 x 1024 x 768 21.3 -> 20.2, x 768 x 1024 13.1 -> 11.6; 800 tokens, both 23.6 -> 19.8;
-// gate gradients of B4 T1024 W1024 in fp32 39.5 -> 37.  More slices in flight (3, 4 or 6) and tiles of 128 x 64: no gain.
+// What bounds it, forward: with slices through registers the LDS writes (13.8 clocks a KB on a compute unit, reads 4.3) were most
+// of the 0.9 us a slice.  Direct, two products of 2331 x 1024 x 768 in bf16 take 14.8 us: 1.5 us launch, 3 us until the first slice is
+// there, 4 us for the results (timing builds), the rest MFMAs of the 48 compute units that have two of the 304 tiles.  us before ->
+// with direct slices, bias asked for in front of them: 2331 x 2 x 1024 x 768 20.3 -> 14.8, x 768 x 1024 11.6 -> 9.8; 4096 x 2 x 1024 x 768
+// 22.4 -> 18.9; 8192 41.5 -> 34.4; 16384 x 2048 x 2048 166 -> 136 (1012 TFLOP/s).  fp32, bound by its MFMAs: 34.1 -> 32.8 at 800
+// x 2 x 1024 x 768, 389 -> 387 at 16384.  Three or four slices of 128 x 128 (one workgroup a compute unit): 23.0, 16.4 against 16.6; tiles of
+// 128 x 64: 16.5; both operands' tiles per XCD in another order: no change.
+// The gradients, through registers: the order of a slice below, operand pointers outside the loop and results staged four columns
+// at a time took the gate gradients of B4 T1024 W1024 in fp32 from 39.5 to 37 us; more slices in flight (3, 4 or 6) gained nothing.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
 #include <initializer_list>
+#include <type_traits>
 
 #include "rglru_device.h"
 #include "rglru_host.h"
@@ -124,6 +129,49 @@ struct OperandTile {
 
 constexpr int kLinearThreads = 256;
 
+// Tile of an operand whose rows are result indices, moved from memory to LDS without passing through registers (1 KB a wave
+// instruction: eight rows of 128 bytes).  The rows lie without padding, so the 16-byte vectors of row r are permuted: vector c is at
+// place c ^ ((r / 2) % 8), and the sixteen rows that the LDS serves at once fall on different banks.
+template <typename IO, int ROWS>
+struct DirectTile {
+  typedef Io<IO> Tr;
+  typedef typename Tr::Frag Frag;
+  static constexpr int HW = Tr::HW, BK = 8 * HW, kBytes = ROWS * 128, NV = ROWS / 32;
+  unsigned off, cv;                  // the lane's first vector: offset in memory, its place in the slice
+  unsigned place[4];                 // the lane's vector of a fragment in LDS, by K group
+  RGLRU_DEVICE void setup(int wave, int lane, long long ld) {
+    const unsigned row = (unsigned)wave * 8u + (unsigned)(lane >> 3);
+    cv = (unsigned)(lane & 7) ^ ((row >> 1) & 7u);
+    off = row * (unsigned)(ld * (int)sizeof(IO)) + cv * 16u;
+    const unsigned r = lane & 31, hf = lane >> 5;
+#pragma unroll
+    for (unsigned kg = 0; kg < 4; ++kg) place[kg] = r * 128u + (((2u * kg + hf) ^ ((r >> 1) & 7u)) * 16u);
+  }
+  // Slice at `base` with k_left contraction indices into LDS at byte address `lds` (below 64 KB: M0 holds 16 bits of it); rows past
+  // `limit` and indices past k_left become zeros, as masked loads do everywhere.  The compiler neither counts these loads nor knows
+  // their hazards: the caller waits for them, and the descriptor has its wait states here.
+  RGLRU_DEVICE void request(const IO* base, long long ld, int k_left, int limit, unsigned lds, int wave) const {
+    const int lines = limit < ROWS ? limit : ROWS;
+    const unsigned long long at = (unsigned long long)base;
+    i32x4 r;
+    r[0] = __builtin_amdgcn_readfirstlane((int)(unsigned)at);
+    r[1] = __builtin_amdgcn_readfirstlane((int)((unsigned)(at >> 32) & 0xffffu));
+    r[2] = __builtin_amdgcn_readfirstlane(k_left > 0 ? (int)((unsigned)((long long)lines * ld) * (unsigned)sizeof(IO)) : 0);
+    r[3] = 0x00020000;
+    asm volatile("s_nop 4" :: "s"(r));
+    const unsigned step = 32u * (unsigned)(ld * (int)sizeof(IO));
+    const unsigned first = (int)cv * HW < k_left ? off : kOutOfRange;
+    const unsigned to = __builtin_amdgcn_readfirstlane(lds + (unsigned)wave * 1024u);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                   :: "s"(to + (unsigned)i * 4096u), "v"(first + (unsigned)i * step), "s"(r) : "memory", "m0");
+  }
+  RGLRU_DEVICE Frag fragment(const unsigned char* lds, int first, int kg) const {
+    return *reinterpret_cast<const Frag*>(lds + first * 128 + place[kg]);
+  }
+};
+
 // Four consecutive elements (N is a multiple of a 16-byte vector, so they lie wholly inside or outside a row).
 template <typename IO> RGLRU_DEVICE auto buf_load_four(rsrc_t r, unsigned voff) {
   typedef IO io4 __attribute__((ext_vector_type(4)));
@@ -131,7 +179,8 @@ template <typename IO> RGLRU_DEVICE auto buf_load_four(rsrc_t r, unsigned voff) 
   else return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
 
-template <typename IO, bool TA, bool TB, int BM, int BN>
+// DIRECT: both operands' rows are result indices and go to LDS directly (DirectTile).
+template <typename IO, bool TA, bool TB, int BM, int BN, bool DIRECT = !TA && !TB>
 __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
@@ -141,7 +190,9 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   constexpr int MI = BM / 64, NI = BN / 64;                  // 32 x 32 accumulator tiles of a wave (2 x 2 waves)
   constexpr int kStageRow = BN / 2 + Tr::HW;                 // epilogue: the wave's half tile, row by row
   constexpr int kStage = 4 * (BM / 2) * kStageRow;
-  constexpr int kBuffers = 2 * (TileA::kElems + TileB::kElems);
+  // two slices of 32 KB or three of 16 KB: two and three workgroups on a compute unit (64 x 64 with two or four slices: 11.8 and 10.2 us for 10)
+  constexpr int STAGES = BM == 128 ? 2 : 3;
+  constexpr int kBuffers = DIRECT ? STAGES * (BM + BN) * BK : 2 * (TileA::kElems + TileB::kElems);
   __shared__ __attribute__((aligned(16))) IO lds[kBuffers > kStage ? kBuffers : kStage];
 
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
@@ -213,11 +264,73 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
           for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)c[e];
         }
   }
+  io4 bias[NI][4];                                           // asked for here: behind the last slice it would be waited for
+  if constexpr (!TA) {
+    const rsrc_t rb = make_rsrc((const IO*)p.bias[problem] + n0, p.bias[problem] ? (unsigned)n_left * (unsigned)sizeof(IO) : 0u);
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) bias[j][g] = buf_load_four<IO>(rb, (unsigned)(wn * (BN / 2) + 32 * j + 8 * g + 4 * hf) * (unsigned)sizeof(IO));
+  } else {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) bias[j][g] = io4{};
+  }
   float sum[MI];                                             // column sums of A over the lane's share of K
 #pragma unroll
   for (int i = 0; i < MI; ++i) sum[i] = 0.f;
   const bool sums = TA && p.colsum && tn == 0 && wn == 0;
 
+  if constexpr (DIRECT) {
+    DirectTile<IO, BM> da;
+    DirectTile<IO, BN> db;
+    da.setup(wave, lane, lda);
+    db.setup(wave, lane, ldb);
+    constexpr unsigned kBytesA = DirectTile<IO, BM>::kBytes, kStageBytes = kBytesA + DirectTile<IO, BN>::kBytes;
+    constexpr int LOADS = DirectTile<IO, BM>::NV + DirectTile<IO, BN>::NV;     // of a wave and slice
+    unsigned char* const bytes = reinterpret_cast<unsigned char*>(lds);
+    const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)bytes;
+    auto fetch = [&](int s, int stage) {
+      const int k = k_begin + s * BK, left = s < total_slices ? k_end - k : 0;
+      const long long ks = s < total_slices ? k : 0;
+      da.request(a_first + m0 * lda + ks, lda, left, m_left, lds0 + (unsigned)stage * kStageBytes, wave);
+      db.request(b_first + n0 * ldb + ks, ldb, left, n_left, lds0 + (unsigned)stage * kStageBytes + kBytesA, wave);
+    };
+    // a slice has landed when every wave has waited for its own part of it
+    auto landed = [&](auto younger) {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(decltype(younger)::value) : "memory");
+    };
+#pragma unroll
+    for (int q = 0; q < STAGES - 1; ++q) fetch(q, q);
+    landed(std::integral_constant<int, (STAGES - 2) * LOADS>{});
+    int stage = 0;
+    for (int s = 0; s < total_slices; ++s) {
+      const int last = stage == 0 ? STAGES - 1 : stage - 1;                      // read in the pass before
+      fetch(s + STAGES - 1, last);
+      const unsigned char* cur = bytes + (unsigned)stage * kStageBytes;
+      Frag fa[2][MI], fb[2][NI];
+      auto read = [&](int kg) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[kg & 1][i] = da.fragment(cur, wm * (BM / 2) + 32 * i, kg);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) fb[kg & 1][j] = db.fragment(cur + kBytesA, wn * (BN / 2) + 32 * j, kg);
+      };
+      read(0);
+#pragma unroll
+      for (int kg = 0; kg < KGS; ++kg) {
+        if (kg + 1 < KGS) read(kg + 1);
+        __builtin_amdgcn_sched_barrier(0);               // or the reads sink to their use, and the products wait for them
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) Tr::mma(acc[i][j], fb[kg & 1][j], fa[kg & 1][i]);
+      }
+      landed(std::integral_constant<int, (STAGES - 2) * LOADS>{});
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+    landed(std::integral_constant<int, 0>{});                                  // nothing may land over the epilogue's staging
+  } else {
   request(0, 0);
   request(1, 1);
   ta.deposit(0, lds, tid, masked);
@@ -263,6 +376,8 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     }
   }
 
+  }
+
   if (sums) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -272,7 +387,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     }
   }
   const int col0 = wn * (BN / 2), row0 = wm * (BM / 2);
-  if (p.partial) {
+  if constexpr (TA) if (p.partial) {                         // weight gradients
     const int ld = p.partial_ld ? p.partial_ld : p.N, rows = p.partial_ld ? p.partial_ld : p.M;
     float* part = p.partial + ((((long long)split * p.batch + item) * p.problems + problem) * rows + m0) * ld + n0;
     const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * ld) * 4u);
@@ -303,19 +418,17 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     return;
   }
   // result in the storage type: through LDS (the slices have been read), then 16-byte vectors of rows
-  const rsrc_t rb = make_rsrc((const IO*)p.bias[problem] + n0, p.bias[problem] ? (unsigned)n_left * (unsigned)sizeof(IO) : 0u);
   IO* stage = lds + wave * (BM / 2) * kStageRow;
 #pragma unroll
   for (int j = 0; j < NI; ++j)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int n = 32 * j + 8 * g + 4 * hf;
-      const io4 bias = buf_load_four<IO>(rb, (unsigned)(col0 + n) * (unsigned)sizeof(IO));
 #pragma unroll
       for (int i = 0; i < MI; ++i) {
         io4 c;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) c[e] = (IO)(acc[i][j][4 * g + e] + (float)bias[e]);
+        for (int e = 0; e < 4; ++e) c[e] = (IO)(acc[i][j][4 * g + e] + (float)bias[j][g][e]);
         *reinterpret_cast<io4*>(stage + (32 * i + r) * kStageRow + n) = c;
       }
     }

@@ -912,6 +912,32 @@ def test_right_padded_block_in_one_launch_matches_the_separate_kernels(cfg, pack
 # matrix products of the Linear layers (C ABI: rglru_hip_linear) and the block as one training operator
 # ----------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(67, 72, 8), (130, 200, 200), (130, 200, 456), (2050, 2056, 8), (2050, 2056, 200), (2050, 2056, 456)])
+def test_forward_product_reads_only_its_operands(M, N, K, dtype):
+    """Rows and contraction indices past the operands' edges, which lie inside larger tensors of NaN, leave no trace: one, some and
+    many slices of the contraction, none of them a whole number, with small and with large tiles."""
+    from griffin_amd import _lib
+
+    lib = _lib.load()
+    _say("inside NaN", M, N, K, dtype)
+    gen = torch.Generator().manual_seed(11)
+    nan = lambda rows, cols: torch.full((rows + 130, cols), float("nan"), dtype=dtype, device="cuda")
+    x, w, c = nan(M, K + 64), nan(N, K + 16), nan(M, N + 24)
+    x[1:M + 1, 16:16 + K] = torch.randn(M, K, generator=gen).to(dtype).cuda()
+    w[1:N + 1, 8:8 + K] = torch.randn(N, K, generator=gen).to(dtype).cuda()
+    _lib.check(lib.rglru_hip_linear(0, x[1, 16:].data_ptr(), None, K + 64, w[1, 8:].data_ptr(), None, K + 16, None, None, None, c[1, 8:].data_ptr(),
+                                    None, N + 24, None, None, M, N, K, _lib.RGLRU_BF16 if dtype == torch.bfloat16 else _lib.RGLRU_F32,
+                                    torch.cuda.current_stream().cuda_stream), "linear")
+    torch.cuda.synchronize()
+    a, b = x[1:M + 1, 16:16 + K].double(), w[1:N + 1, 8:8 + K].double()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0         # rounding of the result; then K additions in fp32
+    bound = unit * (a @ b.t()).abs() + (K + 2) * 2.0 ** -24 * (a.abs() @ b.abs().t())
+    got = c[1:M + 1, 8:8 + N].double()
+    assert ((got - a @ b.t()).abs() <= bound).all()
+    assert torch.isnan(c[0]).all() and torch.isnan(c[M + 1:]).all() and torch.isnan(c[:, :8]).all() and torch.isnan(c[:, 8 + N:]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 72, 64), (65, 64, 136), (64, 128, 40), (700, 200, 328), (2050, 2056, 72), (1100, 136, 2304)])
 def test_linear_products_match_fp64(M, N, K, dtype):
     """All three kinds at edges of tiles, slices and splits, one and two products a launch, with and without masked rows."""
