@@ -112,11 +112,11 @@ __global__ __launch_bounds__(kThreads) void step16_kernel(FusedArgs p) {
   // A fragments: row m = lane % 16 is sequence row0 + m, element j of K step ks is input channel 32 ks + 8 q + j
   const long long arow = row0 + n;
   const bool arow_ok = arow < p.B;
-  const IO* xr = (const IO*)p.x + (arow_ok ? arow : 0) * W + k * p.bw + 8 * q;
+  const IO* xr = (const IO*)p.x + (arow_ok ? arow : 0) * W + k * p.bw;
   Frag xa[NKS], fa[NKS], fx[NKS];
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks)                         // a row past the end reads row 0: its products are not used
-    xa[ks] = *reinterpret_cast<const Frag*>(xr + (32 * ks + 8 * q < p.bw ? 32 * ks : 0));
+    xa[ks] = *reinterpret_cast<const Frag*>(xr + (32 * ks + 8 * q < p.bw ? 32 * ks + 8 * q : 0));
   // B fragments: column n is output channel o, same K elements: rows of the two weight matrices
   const IO* wa = (const IO*)p.wg + ((long long)(0 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
   const IO* wx = (const IO*)p.wg + ((long long)(1 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kThreads) void steps16_kernel(FusedArgs p) {
   const int steps = p.T;
   const long long arow = row0 + n;
   const bool arow_ok = arow < p.B;
-  const IO* xr = (const IO*)p.x + (arow_ok ? arow : 0) * W + k * p.bw + 8 * q;
+  const IO* xr = (const IO*)p.x + (arow_ok ? arow : 0) * W + k * p.bw;
   Frag fa[NKS], fx[NKS];
   const IO* wa = (const IO*)p.wg + ((long long)(0 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
   const IO* wx = (const IO*)p.wg + ((long long)(1 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kThreads) void steps16_kernel(FusedArgs p) {
     const long long tt = t < steps ? t : 0;                // a step past the end re-reads step 0
     const long long base = tt * step_elems;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + (32 * ks + 8 * q < p.bw ? 32 * ks : 0));
+    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + (32 * ks + 8 * q < p.bw ? 32 * ks + 8 * q : 0));
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       s.xv[v] = ((const IO*)p.x)[base + at[v]];

@@ -105,12 +105,12 @@ __global__ __launch_bounds__(kThreads) void decode_linear_kernel(DecodeLinearArg
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const long long r = row0 + 16 * t + n;
-    xr[t] = (const IO*)p.x + (r < p.B ? r : p.B - 1) * p.ldx + q * HW;
+    xr[t] = (const IO*)p.x + (r < p.B ? r : p.B - 1) * p.ldx;
   }
 #pragma unroll
   for (int t = 0; t < CT; ++t) {
     const int c = col0 + 16 * t + n;
-    wr[t] = (const IO*)p.w[which] + (long long)(c < p.N ? c : p.N - 1) * p.K + q * HW;
+    wr[t] = (const IO*)p.w[which] + (long long)(c < p.N ? c : p.N - 1) * p.K;
   }
   f32x4 acc[RT][CT];
 #pragma unroll
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kThreads) void decode_linear_kernel(DecodeLinearArg
     for (int u = 0; u < BATCH; ++u) {
       const int k = (s0 + u * kWaves) * M::STEP;
       const bool ok = k + q * HW < p.K;                                     // K is a multiple of a lane's vector
-      const int kk = ok ? k : 0;
+      const int kk = ok ? k + q * HW : 0;                                   // else the row's first vector, whatever K is
 #pragma unroll
       for (int t = 0; t < CT; ++t) wb[u][t] = *reinterpret_cast<const Frag*>(wr[t] + kk);
 #pragma unroll
