@@ -162,7 +162,8 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
 #pragma unroll
     for (int e = 0; e < EL; ++e) {
       h = fmaf(t.a[e], h, t.z[e]);
-      BufIo<IO>::store((IO)h, ry, voff + (unsigned)e * row_bytes, 0u);
+      // 32-bit results are written through (kWriteThrough): 27.0 -> 25.0 us at B4 T1024 W1024
+      BufIo<IO>::template store<sizeof(IO) == 4 ? kWriteThrough : kWriteBack>((IO)h, ry, voff + (unsigned)e * row_bytes, 0u);
       if ((e & 15) == 15) BufIo<float>::store(h, rck, ck_off[e >> 4], 0u);
     }
   }

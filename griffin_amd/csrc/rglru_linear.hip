@@ -413,10 +413,12 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     for (int q = 0; q < (BM / 2) / ROWS; ++q) {
       const int m = q * ROWS + lane / VPR, cv = lane % VPR, row = row0 + m, n = col0 + cv * 4;
       const i32x4 c = *reinterpret_cast<const i32x4*>(stage + m * kRow + cv * 4);
-      buf_store_b128(c, rc, n < n_left && row < m_left ? ((unsigned)row * (unsigned)ld + (unsigned)n) * 4u : kOutOfRange);
+      buf_store_b128<kWriteThrough>(c, rc, n < n_left && row < m_left ? ((unsigned)row * (unsigned)ld + (unsigned)n) * 4u : kOutOfRange);
     }
     return;
   }
+  // Results are written through the L2s (kWriteThrough): 16.6 -> 15.8 us for 2331 x 2 x 1024 x 768 in bf16, weight gradient of 2048 x 2 x 1024 x
+  // 768 41.6 -> 39.6, fp32 gate gradients of B4 T1024 W1024 37.5 -> 34.8; the largest tried, 134 MB, 183 -> 181.
   // result in the storage type: through LDS (the slices have been read), then 16-byte vectors of rows
   IO* stage = lds + wave * (BM / 2) * kStageRow;
 #pragma unroll
@@ -442,7 +444,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     const int row = row0 + m, n = col0 + cv * Tr::HW;
     if (!TA && p.active && row < m_left && !p.active[m0 + row]) f = Tr::zero();
     const unsigned off = n < n_left && row < m_left ? ((unsigned)row * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange;
-    buf_store_b128(__builtin_bit_cast(i32x4, f), rc, off);
+    buf_store_b128<kWriteThrough>(__builtin_bit_cast(i32x4, f), rc, off);
   }
 }
 
