@@ -1370,8 +1370,8 @@ Tensor sum_sets(const Tensor& sets) {
 // training step of the block has seven.  The line lies where both ways take equally long per layer in a stack of eight blocks,
 // alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
 // alone / with MLPs).  bf16, training 768 -> 1024: at 3.0e9 269 : 316 / 716 : 728, at 6.0e9 401 : 440 / 1106 : 1150, at 1.3e10 651 : 532 / 1847 : 1703;
-// 2560 -> 2560 at 4.5e9 373 : 384 / 963 : 952, at 6.0e9 431 : 419 / 1121 : 1108; prefill 768 -> 1024 at 6.0e9 109 : 105 / 299 : 296, 2560 at 4.5e9
-// 120 : 129 / 266 : 254.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
+// 2560 -> 2560 at 4.5e9 373 : 384 / 963 : 952, at 6.0e9 431 : 419 / 1121 : 1108; a block's prefill alone 768 -> 1024 at 6.4e9 86 : 90, at 9.7e9
+// 119 : 118, 2560 at 6.7e9 118 : 107.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
 // host time is nothing: there the line lies where the kernels take equally long.
 bool own_products(double macs, at::ScalarType dtype) {
   if (!known(dtype)) return false;
