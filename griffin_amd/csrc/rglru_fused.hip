@@ -355,10 +355,12 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
     const rsrc_t rticket = make_rsrc(q.counter, 4u);
     const unsigned rec_stride = (unsigned)W * 8u;
     // The first records of a walk are requested behind the tile's own map, across the barrier and the next tile's loads, where a
-    // sequence has at most two workgroups on it.  With more of them the chunk in front is not out yet and the early look comes back
+    // sequence has at most four workgroups on it.  With more of them the chunk in front is not out yet and the early look comes back
     // empty; so does one at the top of the tile, the place it had before.  Forward alone, us, with the priority above: B16 T2048
     // W2560 238 -> 228, the block's forward at B8 T2048 W1024 53 -> 49 (16 gate blocks), B1 T32768 W2560 294 (315 when it looked).
-    const unsigned rec_lane = (slab_ok && w.ch_ok) && p.wg_per_unit <= 2 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
+    // The line, 320-wide blocks, never : up to four (workgroups on a sequence in brackets): B8 T2048 W2560 (2.6) 130 : 114, B6 (3.5)
+    // 101 : 97; up to six: B4 (5.3) 73.9 : 75.3.
+    const unsigned rec_lane = (slab_ok && w.ch_ok) && p.wg_per_unit <= 4 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
     // A dead finalize in front of the loop: the loop is entered with the same memory operations in
     // flight as its back edge has, so the waits at its top are exact instead of worst case.
     bf16x8 gate_rows[BLOCK ? TR / 16 : 1];               // the lane's vectors of the second projection

@@ -346,10 +346,10 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
     }
     return;
   }
-  // The first records of a walk are requested as soon as the tile's own map is out where a sequence has at most two workgroups on
-  // it: the tile behind is then long finished (B16 T2048 W2560, 320-wide blocks: 321 against 343 us).  With more of them on one
-  // chain it is not, and the early look only comes back empty (B1 T32768: 458 against 420 us).
-  const unsigned ahead_lane = ch_ok && p.wg_per_unit <= 2 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
+  // The first records of a walk are requested as soon as the tile's own map is out where a sequence has at most four workgroups on
+  // it: the tile behind is then finished (320-wide blocks, W2560: B16 T2048 321 against 343 us, B8 T1024 97 against 100).  With more of
+  // them on one chain it is not, and the early look only comes back empty (B4 T2048 108 against 104.5, B1 T32768 458 against 420 us).
+  const unsigned ahead_lane = ch_ok && p.wg_per_unit <= 4 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
   // Everything that the next tile needs early -- its tile, the state in front of it, the ticket after it -- is requested in front
   // of the stores of this one: the counter that loads are waited for with counts in issue order, so whatever is requested
   // behind the stores is waited for together with them.
@@ -2283,8 +2283,13 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   a.aligned = 1;
   const int nkg = wide_groups(g, dtype, 1);
   const bool pad = wide_padded(g);
-  // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums
+  // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums.  Two workgroups a compute unit where each
+  // has two tiles or more: with fewer what they load first, the weights, is most of their time (320-wide blocks of W2560, us, two : one:
+  // 1.5 tiles each at B2 T512 29.4 : 27.1, 1.9 at B4 T300 33.0 : 31.8, 3 at B4 T512 39.0 : 39.9, 3.8 at B8 T300 43.5 : 47.5; 160-wide, 2.5 at
+  // B4 T300 25.7 : 29.6).
   a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, bwd_wide_occ(nkg), L.max_wg);
+  if (B * (long long)a.nC < 2 * (long long)pick_wg_per_unit(a.units, 1ll << 40, bwd_wide_occ(nkg), L.max_wg))
+    a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 1, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
   const bool masked = (flags != nullptr) || a.first_reset || (T % kChunk != 0);
   a.xcd_map = 1;

@@ -1030,7 +1030,7 @@ def test_padded_wide_blocks_match_oracle(bw, nb, B, T, masks, carried):
 @pytest.mark.parametrize("bw", [160, 192, 224, 256, 288, 320])
 @pytest.mark.parametrize("B,T,masks", [(1, 512, False), (33, 64, False), (1, 500, True), (33, 49, True)])
 def test_wide_backward_with_few_and_many_workgroups_on_a_sequence(bw, B, T, masks):
-    """The reverse scan of wide blocks looks for its neighbours' records early where a sequence has at most two workgroups (33
+    """The reverse scan of wide blocks looks for its neighbours' records early where a sequence has at most four workgroups (33
     sequences of two tiles) and not where it has more (one sequence of sixteen): every width that runs two workgroups a
     compute unit, whole and ragged tiles, against the oracle."""
     _say("wide backward", bw, B, T, masks)
@@ -1039,6 +1039,23 @@ def test_wide_backward_with_few_and_many_workgroups_on_a_sequence(bw, B, T, mask
     dh_last = torch.randn(B, bw, generator=torch.Generator().manual_seed(6))
     y, h_last, grads = hip_run(case, torch.bfloat16, reset, active, dh_last)
     ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, active, dh_last)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
+
+
+@pytest.mark.parametrize("bw", [160, 320])
+@pytest.mark.parametrize("B,masks", [(5, False), (16, True)])
+def test_wide_backward_with_several_tiles_a_workgroup(bw, B, masks):
+    """The reverse scan of wide blocks runs two workgroups a compute unit where each has two tiles or more, one elsewhere: batches on
+    either side of the line (175 and 560 tiles for 171 or 256 workgroups), against the oracle."""
+    T = 1100
+    _say("several tiles", bw, B, masks)
+    case = orc.make_case(B, T, bw, 1, seed=bw + B, h0_std=0.5, bias_std=0.5)
+    reset, active = _masks(B, T, masks)
+    y, h_last, grads = hip_run(case, torch.bfloat16, reset, active)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, active)
     errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
     errs.update({name: rel_err(grads[name].float(), rgrads[name]) for name in grads})
     for name, err in errs.items():
