@@ -264,9 +264,13 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
           for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = (float)c[e];
         }
   }
-  io4 bias[NI][4];                                           // asked for here: behind the last slice it would be waited for
+  // A bias may start at any element (a view of a longer tensor).  Vectors of it are asked for here, since behind the last slice they
+  // would be waited for; one that starts off their boundaries is loaded there, by elements.
+  const IO* const bias_from = TA ? nullptr : (const IO*)p.bias[problem];
+  const bool bias_vectors = bias_from != nullptr && (unsigned long long)bias_from % sizeof(io4) == 0;
+  io4 bias[NI][4];
   if constexpr (!TA) {
-    const rsrc_t rb = make_rsrc((const IO*)p.bias[problem] + n0, p.bias[problem] ? (unsigned)n_left * (unsigned)sizeof(IO) : 0u);
+    const rsrc_t rb = make_rsrc(bias_from + n0, bias_vectors ? (unsigned)n_left * (unsigned)sizeof(IO) : 0u);
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
@@ -378,6 +382,16 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
 
   }
 
+  if constexpr (!TA) if (bias_from != nullptr && !bias_vectors) {
+    const rsrc_t rb = make_rsrc(bias_from + n0, (unsigned)n_left * (unsigned)sizeof(IO));
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          bias[j][g][e] = (IO)BufIo<IO>::load(rb, (unsigned)(wn * (BN / 2) + 32 * j + 8 * g + 4 * hf + e) * (unsigned)sizeof(IO), 0u);
+  }
   if (sums) {
 #pragma unroll
     for (int i = 0; i < MI; ++i) {

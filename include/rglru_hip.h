@@ -377,7 +377,8 @@ int rglru_hip_sum_sets(const void* x, void* out, int64_t sets, int64_t n, int dt
 
 /* Products of the block's Linear layers (griffin/griffin.py:379-389) on the matrix unit, fp32 accumulation, all matrices in
  * `dtype`, their rows whole 16-byte vectors on 16-byte boundaries, lda / ldb / ldc elements apart:
- *   RGLRU_LINEAR_FORWARD      c_i[M, N] = a0[M, K] b_i[N, K]^T + bias_i[N]     i = 0, and 1 where b1 is given; biases may be NULL
+ *   RGLRU_LINEAR_FORWARD      c_i[M, N] = a0[M, K] b_i[N, K]^T + bias_i[N]     i = 0, and 1 where b1 is given; biases may be NULL,
+ *                             and start at any element
  *   RGLRU_LINEAR_INPUT_GRAD   c0[M, N]  = a0[M, K] b0[K, N] + a1[M, K] b1[K, N]     a1 NULL: the first product alone
  *   RGLRU_LINEAR_WEIGHT_GRAD  c_i[M, N] = a_i[K, M]^T b0[K, N]                 i = 0, and 1 where a1 is given
  * `active`: one byte per token or NULL; the results of inactive tokens (rows of c) are zero, and in a weight gradient the

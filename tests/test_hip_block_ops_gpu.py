@@ -985,6 +985,36 @@ def test_forward_product_reads_only_its_operands(M, N, K, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("first", [(0, 1), (3, 2), (5, 0)])
+@pytest.mark.parametrize("M,N,K", [(67, 72, 8), (1100, 2056, 72)])
+def test_bias_of_a_forward_product_may_start_at_any_element(M, N, K, first, dtype):
+    """Biases that are views into longer tensors, on and off the boundaries of the vectors they are loaded as, one of each in a launch;
+    what lies around them is NaN.  Small and large tiles, the last of them not full."""
+    from griffin_amd import _lib
+    from griffin_amd.hip_block_ops import hip_linear
+
+    _say("bias at", first, M, N, K, dtype)
+    gen = torch.Generator().manual_seed(first[0])
+    make = lambda *shape: torch.randn(*shape, generator=gen).to(dtype).cuda()
+    x, weights, biases = make(M, K), [make(N, K) for _ in first], []
+    for at in first:
+        b = torch.full((at + N + 8,), float("nan"), dtype=dtype, device="cuda")[at:at + N]
+        biases.append(b.copy_(make(N)))
+        assert b.data_ptr() % 16 == (at * b.element_size()) % 16
+    out = [torch.empty(M, N, dtype=dtype, device="cuda") for _ in first]
+    _lib.check(_lib.load().rglru_hip_linear(0, x.data_ptr(), None, K, weights[0].data_ptr(), weights[1].data_ptr(), K, biases[0].data_ptr(),
+                                            biases[1].data_ptr(), None, out[0].data_ptr(), out[1].data_ptr(), N, None, None, M, N, K,
+                                            _lib.RGLRU_BF16 if dtype == torch.bfloat16 else _lib.RGLRU_F32,
+                                            torch.cuda.current_stream().cuda_stream), "linear")
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0         # rounding of the result; then K + 1 additions in fp32
+    for w, b, got in zip(weights, biases, out):
+        want = x.double() @ w.double().t() + b.double()
+        bound = unit * want.abs() + (K + 3) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + b.double().abs())
+        assert ((got.double() - want).abs() <= bound).all()
+        assert torch.equal(hip_linear(x, w, b), got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 72, 64), (65, 64, 136), (64, 128, 40), (700, 200, 328), (2050, 2056, 72), (1100, 136, 2304)])
 def test_linear_products_match_fp64(M, N, K, dtype):
     """All three kinds at edges of tiles, slices and splits, one and two products a launch, with and without masked rows."""
