@@ -887,16 +887,28 @@ struct BlockFwd {
 
 
 // Workgroups per unit of the kernel whose workgroups own whole sequences (rglru_fwd_rows.hip), or 0 where the tiled kernel is the
-// better one.  It needs a sequence for every workgroup that fits the chip, and rounds of sequences that are mostly full, or the
-// last round idles: forward at T512 W1024 in 128-wide blocks, us, tiled -> rows, 64 workgroups a unit: 64 sequences 53 -> 49, 96 (two
-// rounds, three quarters full) 74 -> 66, 129 111 -> 108, 80 63 -> 64, 65 54 -> 61; 48 sequences 44 -> 47.  Tiles with flags cost the tiled
-// kernel a third more and this one only where a flag is: B96 T700 W1024 packed 141 -> 104.
-static int fwd_row_workgroups(int64_t B, const Geometry& g, int nkg, bool flags) {
+// better one.  It needs a sequence for every workgroup that fits the chip, and then its time grows in steps: the workgroups of a unit
+// that have one sequence more than the others lie on different compute units until every unit of the chip has one, then a second one
+// joins them, and so on.  `rounds` counts such steps of one sequence a compute unit; the last of them has to be nearly full.  How full
+// depends on the tiled kernel.  Forward, T512 unless said, us, tiled : rows (part of the rounds that is filled):
+//   128-wide, W1024 (64 workgroups a unit), odd rounds   B80 62.7 : 63.0 (83 %), 90 68.9 : 63.2 (94), 140 103.1 : 103.0 (88), 160 122 : 112
+//             even rounds, whose last sequence shares its compute unit   97 72.8 : 86.9 (76), 104 78.4 : 88.3 (81), 120 93.3 : 93.7 (94), 128 100 :
+//             96, 161 119 : 131 (84), 240 170 : 171 (94), 256 181 : 171; T2048 112 326 : 343, 120 352 : 350, 256 727 : 699
+//             20 units of them (25 workgroups each)   B38 78.5 : 91.1 (74), 48 93.5 : 89.6 (94), 51 94.9 : 101.1 (80), 64 125 : 134 (83)
+//   32- and 64-wide (three workgroups a compute unit)   B98 71.7 : 75.8 (77), 112 82.0 : 78.7 (88), 128 86.3 : 76.2, 161 112 : 119 (84), 176 120 : 118
+//             (92), 225 150 : 146 (88); T2048 98 262 : 282, 113 300 : 294, 170 448 : 451 (89)
+// Flags, ragged lengths and padded blocks cost the tiled kernel, whose variant for them is one for all three, up to a third; this one
+// only where a flag is.  96- and 128-wide   B70 68.9 : 68.5 (73), 77 74.7 : 68.0 (80), 97 91.1 : 93.6 (76), 104 96.5 : 96.2 (81), 128 118 : 98;
+// narrower ones always (48-wide B97 83.5 : 75.0, 64-wide with flags B98 88 : 78).
+static int fwd_row_workgroups(int64_t B, const Geometry& g, int nkg, bool masked) {
   FusedArgs a;
   a.units = (int)g.units;
   pack_units(a, g, nkg);
-  const int64_t slots = pick_wg_per_unit(a.units, 1ll << 40, fwd_rows_per_cu(nkg), 1 << 20), rounds = (B + slots - 1) / slots;
-  return B >= slots && 100 * B >= (flags ? 60 : 75) * slots * rounds ? (int)slots : 0;
+  const int64_t cus = num_compute_units(), per_cu = fwd_rows_per_cu(nkg), slots = cus * per_cu / a.units;
+  if (slots < 1 || B < slots) return 0;
+  const int64_t left = B % slots, rounds = B / slots * per_cu + (left * a.units + cus - 1) / cus;
+  const int need = per_cu == 3 ? (masked ? 0 : 88) : masked ? 80 : rounds % 2 ? 88 : 93;
+  return 100 * B * a.units >= need * rounds * cus ? (int)slots : 0;
 }
 
 static int fwd_impl(const void* x, const void* prep, const float* h0, const uint8_t* flags,
@@ -957,7 +969,10 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   // The tiled kernels need the forward records, tickets and failure word zeroed; the chain kernel needs the
   // failure word only and clears it itself.  (Every backward entry point that uses records clears its own.)
   const bool chain = !blk && !pre && narrow && fwd_chain_pays(B, T, g.Wp);
-  const int row_wg = blk || pre || !narrow || chain ? 0 : fwd_row_workgroups(B, g, nkg, flags != nullptr);
+  // the tiled kernels with register-held weights of whole blocks know first_reset and whole tiles; anything else is their masked variant
+  const int tile_tokens = 32 * fwd_mt(nkg);
+  const int masked = pad || flags != nullptr || T % tile_tokens != 0 || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
+  const int row_wg = blk || pre || !narrow || chain ? 0 : fwd_row_workgroups(B, g, nkg, masked);
   if (!cleared && !chain && !row_wg) {
     rc = launch_clear(wb, L.f_begin, L.f_end, s);
     if (rc) return rc;
@@ -1008,7 +1023,6 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     KernelTimer timer(0, s);
     return launch_fwd_rows(a, nkg, pad, s);
   }
-  const int tile_tokens = 32 * fwd_mt(nkg);
   a.nCf = (int)((T + tile_tokens - 1) / tile_tokens);
   // without weights in registers three workgroups fit a compute unit
   a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nCf, blk ? 2 : nkg < 0 ? RGLRU_GIVEN_OCC : ((nkg == 4 || nkg == 2) ? RGLRU_NARROW_OCC : nkg > 8 ? fwd_wide_occ(nkg) : 2), 1 << 20);
@@ -1020,9 +1034,6 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   }
   {
     KernelTimer timer(0, s);
-    // the plain kernels with register-held weights of up to 128 channels know first_reset; the others take it
-    // through the flag logic of their masked variant
-    const int masked = (flags != nullptr) || (T % tile_tokens != 0) || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
     if (pad) {
 #define RGLRU_PAD_CASE(N)                                                                                              \
       if (nkg == N) {                                                                                                  \
