@@ -195,9 +195,9 @@ constexpr int kVecThreads = 64 * kVecWaves;
 
 struct Map4 { float4 a, h; };
 
-// Accesses that leave nothing in the caches: z and dh are read once, and holding them puts out what is read again -- a by both
-// passes, h by the backward (fwd + bwd, us: B8 T2048 W1024 122 -> 114, B16 T1024 W2048 248 -> 240).
-RGLRU_DEVICE float4 load_once(const float* p) {
+// ONCE, STREAM: accesses that leave nothing in the caches (see read_once_pays and scan_bwd).
+template <bool ONCE> RGLRU_DEVICE float4 load4(const float* p) {
+  if constexpr (!ONCE) return *reinterpret_cast<const float4*>(p);
   const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
   return make_float4(v[0], v[1], v[2], v[3]);
 }
@@ -275,8 +275,8 @@ RGLRU_DEVICE void rec_store4(rec_t* rec, float4 a, float4 h, bool final) {
 
 // FORWARD = true: h_t = a_t h_{t-1} + z_t (out0 = h).  FORWARD = false: the reverse scan
 // delta_t = dh_t + a_{t+1} delta_{t+1}; out0 = da = delta * h_{t-1}, out1 = dz = delta, dh0 = a_0 delta_0.
-// STREAM: da and dz together are larger than the memory-side cache (see scan_bwd), so they leave as they would anyway.
-template <bool FORWARD, bool STREAM = false>
+// ONCE: z and dh bypass the caches.  STREAM: da and dz together are larger than the memory-side cache, so they leave as they would anyway.
+template <bool FORWARD, bool ONCE, bool STREAM = false>
 __global__ __launch_bounds__(kVecThreads, 2) void scan_vec_kernel(ScanArgs p) {
   __shared__ float4 s_a[kVecWaves][64], s_h[kVecWaves][64];
   __shared__ float4 s_carry[64];
@@ -310,12 +310,12 @@ __global__ __launch_bounds__(kVecThreads, 2) void scan_vec_kernel(ScanArgs p) {
       // copy of `zero` in scratch memory and loaded through the result: 31 flat loads of 4 and 12 bytes in place of
       // 16 global loads of 16.)
       const long long at = in ? base + e * W : 0;
-      const float4 av = *reinterpret_cast<const float4*>(p.a + at), zv = load_once(p.z + at);
+      const float4 av = *reinterpret_cast<const float4*>(p.a + at), zv = load4<ONCE>(p.z + at);
       a[e] = make_float4(in ? av.x : 1.f, in ? av.y : 1.f, in ? av.z : 1.f, in ? av.w : 1.f);
       v[e] = make_float4(in ? zv.x : 0.f, in ? zv.y : 0.f, in ? zv.z : 0.f, in ? zv.w : 0.f);
     } else {
       a[e] = in ? *reinterpret_cast<const float4*>(p.a + base + e * W) : one;
-      v[e] = in ? load_once(p.dh + base + e * W) : zero;
+      v[e] = in ? load4<ONCE>(p.dh + base + e * W) : zero;
       hp[e] = zero;
       if (in) hp[e] = (t0 + e == 0) ? *reinterpret_cast<const float4*>(p.h0 + (long long)b * W + ch)
                                     : *reinterpret_cast<const float4*>(p.h_saved + base + (e - 1) * W);
@@ -381,6 +381,13 @@ __global__ __launch_bounds__(kVecThreads, 2) void scan_vec_kernel(ScanArgs p) {
     }
   }
 }
+
+// z and dh are read once; holding large ones puts out what is read again: a by both passes, h by the backward.  Small ones come from the
+// caches, where their producer has left them, unless they are told not to.  Forward and backward, us, held : bypassed, inputs just
+// written or read : inputs out of the caches, by the size of one tensor:  1.8 MB (B5 T115 W808) 19.0 : 21.2, 22.7 : 22.2;  4.5 MB 25.8 : 30.6,
+// 30.0 : 30.0;  16 MB (B4 T1024 W1024) 37.0 : 39.0, 39.2 : 38.6;  32 MB 60.1 : 59.8, 62.0 : 61.2;  48 MB 91.4 : 83.1, 91.5 : 85.2;  64 MB (B8 T2048 W1024) 123.3 :
+// 118.4, 123.5 : 118.7;  128 MB 233 : 221, 235 : 219.
+static bool read_once_pays(int64_t B, int64_t T, int64_t W) { return 4 * B * T * W >= (32ll << 20); }
 
 static bool pointers_aligned16(const void* const* ptrs, int n) {
   for (int i = 0; i < n; ++i) if ((uintptr_t)ptrs[i] % 16 != 0) return false;
@@ -450,7 +457,8 @@ int rglru_hip_scan_fwd(const float* a, const float* z, const float* h0, float* h
   p.a = a; p.z = z; p.h0 = h0; p.h = h;
   if (vec) {
     const long long runs = (long long)B * ((W + 255) / 256) * ((T + kVecRun - 1) / kVecRun);
-    hipLaunchKernelGGL(scan_vec_kernel<true>, dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
+    if (read_once_pays(B, T, W)) hipLaunchKernelGGL((scan_vec_kernel<true, true>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
+    else hipLaunchKernelGGL((scan_vec_kernel<true, false>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
     return check_launch("scan_fwd");
   }
   unsigned blocks = (unsigned)((p.tiles + kWaves - 1) / kWaves);
@@ -473,8 +481,10 @@ int rglru_hip_scan_bwd(const float* a, const float* h0, const float* h, const fl
   if (vec) {
     const long long runs = (long long)B * ((W + 255) / 256) * ((T + kVecRun - 1) / kVecRun);
     // Beyond 256 MB, what the memory-side cache holds, the start of the gradients is gone from it by the time their reader comes:
-    // stored past it, B16 T1024 W2048 takes 223 us forward and backward (240 otherwise).  Smaller ones are left in it.
-    if (8ll * B * T * W >= (256ll << 20)) hipLaunchKernelGGL((scan_vec_kernel<false, true>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
+    // stored past it, B16 T1024 W2048 takes 222 us forward and backward (251 otherwise).  Smaller ones are left in it for their reader: by
+    // itself the operator would gain there too (B8 T2048 W1024 119 : 111, 192 MB 176 : 161; none at 96 MB).
+    if (8ll * B * T * W >= (256ll << 20)) hipLaunchKernelGGL((scan_vec_kernel<false, true, true>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
+    else if (read_once_pays(B, T, W)) hipLaunchKernelGGL((scan_vec_kernel<false, true>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
     else hipLaunchKernelGGL((scan_vec_kernel<false, false>), dim3((unsigned)runs), dim3(kVecThreads), 0, s, p);
     return check_launch("scan_bwd");
   }

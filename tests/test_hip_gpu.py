@@ -1103,14 +1103,15 @@ def test_forward_of_batches_that_fill_the_chip_with_sequences(bw, nb, B, owned, 
         assert err < BF16_TOL, (name, err)
 
 
-@pytest.mark.parametrize("B", [1016, 1018])
-def test_scan_op_gradients_below_and_above_the_cache(B):
-    """From 256 MB of gradients on they are stored past the caches: two runs of tokens, either side of the line, against the loop."""
+@pytest.mark.parametrize("B,W,once,stream", [(250, 260, False, False), (251, 260, True, False), (1016, 256, True, False), (1018, 256, True, True)])
+def test_scan_op_gradients_below_and_above_the_cache(B, W, once, stream):
+    """From 32 MB a tensor on the inputs that are read once bypass the caches, and from 256 MB of gradients on these are stored past
+    them: two runs of tokens, either side of the lines, against the loop."""
     from griffin_amd import hip_rglru_scan
 
-    T, W = 129, 256
-    assert (8 * B * T * W >= 256 << 20) == (B == 1018)
-    _say("scan gradients", B)
+    T = 129
+    assert (4 * B * T * W >= 32 << 20) == once and (8 * B * T * W >= 256 << 20) == stream
+    _say("scan gradients", B, W)
     gen = torch.Generator().manual_seed(0)
     a = torch.sigmoid(torch.randn(B, T, W, generator=gen) + 2.0)
     z, dh = torch.randn(B, T, W, generator=gen), torch.randn(B, T, W, generator=gen)
