@@ -194,10 +194,10 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
   constexpr bool GIVEN = NKG < 0;
   constexpr bool WIDE = NKG > 8;
   constexpr int KC = (GIVEN ? 8 : NKG) * Tr::KG;         // block width (held weights)
-  constexpr int TW = WIDE ? KC : kPackedWidth;           // tile width (narrow blocks are packed)
+  constexpr int TW = KC;                                 // tile width
   constexpr int LDSROW = TW + Tr::HW;
   constexpr int DYROW = kPackedWidth + Tr::HW;
-  static_assert(sizeof(IO) == 2 && NKG != 0, "fast backward is for 16-bit storage");
+  static_assert(sizeof(IO) == 2 && (NKG < 0 || NKG > 8), "16-bit storage; narrower blocks with weights run bwd_delta_kernel and its gradient kernel");
   constexpr bool SHARED = WIDE && bwd_wide_occ(NKG) == 2;
   constexpr int kDuStage = GIVEN ? 2 * WaveStage<TR>::kBytes : PairStage<TR>::kBytes;
   constexpr int kTileBytes = 2 * TR * (LDSROW + DYROW), kStageBytes = kWaves * (WaveStage<TR>::kBytes + kDuStage);
@@ -244,9 +244,9 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
   static_assert(RP_DY * VPR_DY == kThreads && NV_DY * RP_DY == TR, "a pass over the dy tile fills the workgroup");
   Frag pre_x[NV], pre_dy[NV_DY], pre_ua[GIVEN ? NV : 1], pre_ux[GIVEN ? NV : 1];
   // GIVEN: the tiles hold the 128 channels of this workgroup's four slabs
-  const int group_col = (GIVEN || WIDE) ? (w.unit % p.groups) * kPackedWidth : 0;
+  const int group_col = (w.unit % p.groups) * kPackedWidth;
   const int x_col = GIVEN ? w.k * p.bw + group_col : w.tile_col;
-  const int dy_col = WIDE ? w.k * p.bw + group_col : x_col;
+  const int dy_col = w.k * p.bw + group_col;
   const int own_col = WIDE ? group_col : 0;              // the dy tile's first column inside the x tile
   const unsigned u_row_bytes = 4u * (unsigned)p.bw;      // a row of `pre` and of du: two halves of bw 16-bit values
   const int x_row = tid / VPR, x_cv = tid - x_row * VPR, dy_row = tid / VPR_DY, dy_cv = tid - dy_row * VPR_DY;
