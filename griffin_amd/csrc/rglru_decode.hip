@@ -2,6 +2,7 @@
 // teacher-forced steps in one launch (rglru_hip_steps).  Rows are sequences; there is no scan.
 
 #include "rglru_fused.h"
+#include "rglru_rows.h"
 
 namespace rglru {
 
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(kThreads) void step16_kernel(FusedArgs p) {
   Frag xa[NKS], fa[NKS], fx[NKS];
 #pragma unroll
   for (int ks = 0; ks < NKS; ++ks)                         // a row past the end reads row 0: its products are not used
-    xa[ks] = *reinterpret_cast<const Frag*>(xr + (32 * ks + 8 * q < p.bw ? 32 * ks + 8 * q : 0));
+    xa[ks] = *reinterpret_cast<const Frag*>(xr + row_vector(32 * ks, q, 8, p.bw));
   // B fragments: column n is output channel o, same K elements: rows of the two weight matrices
   const IO* wa = (const IO*)p.wg + ((long long)(0 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
   const IO* wx = (const IO*)p.wg + ((long long)(1 * p.nb + k) * p.bwp + o) * p.bwp + 8 * q;
@@ -244,7 +245,7 @@ __global__ __launch_bounds__(kThreads) void steps16_kernel(FusedArgs p) {
     const long long tt = t < steps ? t : 0;                // a step past the end re-reads step 0
     const long long base = tt * step_elems;
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + (32 * ks + 8 * q < p.bw ? 32 * ks + 8 * q : 0));
+    for (int ks = 0; ks < NKS; ++ks) s.xa[ks] = *reinterpret_cast<const Frag*>(xr + base + row_vector(32 * ks, q, 8, p.bw));
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       s.xv[v] = ((const IO*)p.x)[base + at[v]];

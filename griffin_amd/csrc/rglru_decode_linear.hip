@@ -10,6 +10,7 @@
 //
 // Measured (MI355X, eager, one token of RMSNorm + RecurrentBlock(768, 1024)): see decode_project / decode_linear below.
 #include "rglru_fused.h"
+#include "rglru_rows.h"
 
 namespace rglru {
 
@@ -123,8 +124,7 @@ __global__ __launch_bounds__(kThreads) void decode_linear_kernel(DecodeLinearArg
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
       const int k = (s0 + u * kWaves) * M::STEP;
-      const bool ok = k + q * HW < p.K;                                     // K is a multiple of a lane's vector
-      const int kk = ok ? k + q * HW : 0;                                   // else the row's first vector, whatever K is
+      const int kk = row_vector(k, q, HW, p.K);                             // K is a multiple of a lane's vector
 #pragma unroll
       for (int t = 0; t < CT; ++t) wb[u][t] = *reinterpret_cast<const Frag*>(wr[t] + kk);
 #pragma unroll

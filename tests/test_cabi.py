@@ -4,6 +4,8 @@ on the host before touching a GPU (no kernel is launched here)."""
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -151,3 +153,43 @@ def test_scratch_sizes_do_not_depend_on_the_kernel_choice():
             assert got[0][1] >= B * W * 4                    # one row a sequence in the chain kernel
     finally:
         lib.rglru_hip_set_chain_forward(was)
+
+
+ROW_VECTORS = r"""
+#include <cstdio>
+#include "rglru_rows.h"
+
+// Every vector that the lanes of the decode kernels read of a row, over the widths that the kernels take.
+static int check(int first, int q, int per_lane, int width) {
+  const int at = rglru::row_vector(first, q, per_lane, width), own = first + q * per_lane;
+  const bool inside = at >= 0 && at % per_lane == 0 && at + per_lane <= width;
+  if (inside && at == (own < width ? own : 0)) return 0;
+  std::printf("step at %d quarter %d vector %d of a row of %d: %d\n", first, q, per_lane, width, at);
+  return 1;
+}
+
+int main() {
+  int wrong = 0;
+  // projections of a decode step: four waves take steps of four vectors in turn, up to six of them in flight past the last one
+  for (int per_lane = 4; per_lane <= 8; per_lane += 4)
+    for (int width = per_lane; width <= 4096; width += per_lane)
+      for (int step = 0; step * 4 * per_lane < width + 6 * 4 * 4 * per_lane; ++step)
+        for (int q = 0; q < 4; ++q) wrong += check(step * 4 * per_lane, q, per_lane, width);
+  // steps of the layer: gate blocks of 16 to 384 channels, as many steps of 32 as the padded block has
+  for (int width = 16; width <= 384; width += 16)
+    for (int step = 0; step < (width + 31) / 32; ++step)
+      for (int q = 0; q < 4; ++q) wrong += check(32 * step, q, 8, width);
+  return wrong != 0;
+}
+"""
+
+
+def test_lanes_of_the_decode_kernels_read_inside_their_rows(tmp_path):
+    """The offsets at which the decode kernels read their operands' rows (csrc/rglru_rows.h), compiled for the host and run for every lane:
+    whole vectors, none of them past the row's end."""
+    compiler = shutil.which("g++") or shutil.which("clang++") or "/opt/rocm/llvm/bin/clang++"
+    source, program = tmp_path / "rows.cpp", tmp_path / "rows"
+    source.write_text(ROW_VECTORS)
+    subprocess.run([compiler, "-std=c++17", "-O1", "-I", os.path.join(ROOT, "griffin_amd", "csrc"), str(source), "-o", str(program)], check=True)
+    ran = subprocess.run([str(program)], capture_output=True, text=True)
+    assert ran.returncode == 0, ran.stdout[:2000]
