@@ -94,6 +94,7 @@ _SIGNATURES = {
     "rglru_hip_set_reproducible": (ctypes.c_int, [ctypes.c_int]),
     "rglru_hip_reproducible": (ctypes.c_int, []),
     "rglru_hip_set_chain_forward": (ctypes.c_int, [ctypes.c_int]),
+    "rglru_hip_forward_owns_sequences": (ctypes.c_int, [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int]),
     "rglru_hip_set_timing": (ctypes.c_int, [ctypes.c_int]),
     "rglru_hip_kernel_ms": (ctypes.c_float, [ctypes.c_int]),
     "rglru_hip_workspace_status": (ctypes.c_int, [_P, _I, _I, _I, _I, ctypes.c_int, _P, ctypes.POINTER(ctypes.c_int)]),

@@ -911,6 +911,17 @@ static int fwd_row_workgroups(int64_t B, const Geometry& g, int nkg, bool masked
   return 100 * B * a.units >= need * rounds * cus ? (int)slots : 0;
 }
 
+// Kernel of a forward without block and without given pre-activations.
+struct FwdRoute { bool chain, masked; int row_wg; };
+static FwdRoute fwd_route(int64_t B, int64_t T, const Geometry& g, int nkg, bool narrow, bool pad, bool flags, bool first_reset) {
+  FwdRoute r;
+  r.chain = narrow && fwd_chain_pays(B, T, g.Wp);
+  // the tiled kernels with register-held weights of whole blocks know first_reset and whole tiles; anything else is their masked variant
+  r.masked = pad || flags || T % (32 * fwd_mt(nkg)) != 0 || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
+  r.row_wg = narrow && !r.chain ? fwd_row_workgroups(B, g, nkg, r.masked) : 0;
+  return r;
+}
+
 static int fwd_impl(const void* x, const void* prep, const float* h0, const uint8_t* flags,
                     void* y, float* h_last, void* ws,
                     int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, bool cleared, void* stream,
@@ -968,11 +979,9 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   }
   // The tiled kernels need the forward records, tickets and failure word zeroed; the chain kernel needs the
   // failure word only and clears it itself.  (Every backward entry point that uses records clears its own.)
-  const bool chain = !blk && !pre && narrow && fwd_chain_pays(B, T, g.Wp);
-  // the tiled kernels with register-held weights of whole blocks know first_reset and whole tiles; anything else is their masked variant
-  const int tile_tokens = 32 * fwd_mt(nkg);
-  const int masked = pad || flags != nullptr || T % tile_tokens != 0 || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
-  const int row_wg = blk || pre || !narrow || chain ? 0 : fwd_row_workgroups(B, g, nkg, masked);
+  const FwdRoute route = fwd_route(B, T, g, nkg, narrow && !blk && !pre, pad, flags != nullptr, first_reset);
+  const bool chain = route.chain;
+  const int masked = route.masked, row_wg = route.row_wg, tile_tokens = 32 * fwd_mt(nkg);
   if (!cleared && !chain && !row_wg) {
     rc = launch_clear(wb, L.f_begin, L.f_end, s);
     if (rc) return rc;
@@ -1058,6 +1067,13 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
     }
   }
   return check_launch("fwd");
+}
+
+int rglru_hip_forward_owns_sequences(int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int flags) {
+  if (check_geometry("forward_owns_sequences", W, nb, dtype) || B <= 0 || T <= 0 || check_extents("forward_owns_sequences", B, T, W)) return 0;
+  const Geometry g = make_geometry(W, nb);
+  const int nkg = narrow_groups(g, dtype, 1);
+  return nkg && fwd_route(B, T, g, nkg, true, narrow_padded(g), flags == 1, flags == 2).row_wg > 0;
 }
 
 int rglru_hip_fwd(const void* x, const void* prep, const float* h0, const uint8_t* flags,

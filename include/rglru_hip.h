@@ -522,6 +522,10 @@ int rglru_hip_reproducible(void);
  * tiled kernel.  2: the chain kernel whenever it covers the storage type and block width (tests).  Applies to
  * launches made after the call; returns the previous setting. */
 int rglru_hip_set_chain_forward(int mode);
+/* Whether rglru_hip_fwd takes a batch of 16-byte aligned tensors to the kernel whose workgroups own whole sequences (large batches,
+ * in place of the tiled kernel; no counterpart in the reference): what a test asserts.  `flags`: 0 = none, 1 = an array of them,
+ * 2 = RGLRU_FLAGS_FIRST_RESET.  1 or 0; 0 too for what rglru_hip_fwd refuses. */
+int rglru_hip_forward_owns_sequences(int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, int flags);
 /* Synchronising debug helper: copies the failure word of a workspace to the host (0 = clean). */
 int rglru_hip_workspace_status(const void* ws, int64_t B, int64_t T, int64_t W, int64_t nb,
                                int scan_only, void* stream, int* status);

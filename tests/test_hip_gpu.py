@@ -1062,17 +1062,7 @@ def test_wide_backward_with_several_tiles_a_workgroup(bw, B, masks):
         assert err < BF16_TOL, (name, err)
 
 
-def _sequences_fill_the_chip(bw, nb, B, masked):
-    """Whether the forward whose workgroups own whole sequences takes a batch (fwd_row_workgroups in rglru_fused.hip)."""
-    wide, cus = -(-bw // 32) * 32, torch.cuda.get_device_properties(0).multi_processor_count
-    units, per_cu = (nb, 2) if wide > 64 else (-(-nb * wide // 128), 3)
-    slots = cus * per_cu // units
-    rounds = B // slots * per_cu + -(-(B % slots) * units // cus)
-    need = (0 if masked else 88) if per_cu == 3 else 80 if masked else 88 if rounds % 2 else 93
-    return B >= slots and 100 * B * units >= need * rounds * cus
-
-
-# one round of sequences, two and more, the last unit not full, three units (170 workgroups each on 256 compute units); the batches of
+# on 256 compute units: one round of sequences, two and more, the last unit not full, three units (170 workgroups each); the batches of
 # the last line lie on the other side of the line, at least without flags and in whole tiles
 @pytest.mark.parametrize("bw,nb,B,owned", [(128, 1, 512, True), (128, 1, 700, True), (128, 3, 400, True), (88, 1, 512, True), (96, 1, 720, True),
                                            (64, 2, 768, True), (64, 3, 600, True), (40, 2, 770, True), (32, 4, 768, True), (8, 1, 768, True),
@@ -1082,12 +1072,17 @@ def test_forward_of_batches_that_fill_the_chip_with_sequences(bw, nb, B, owned, 
     """Batches with a sequence for every workgroup run the forward whose workgroups own whole sequences: full and ragged tiles,
     flags in some tiles, further rounds of sequences, packed and padded blocks, a last unit that is not full, and batches that leave too
     much of a round empty; outputs, final state and the gradients that the backward computes from its checkpoints."""
-    from griffin_amd import set_chain_forward
+    from griffin_amd import _lib, set_chain_forward
 
     W = bw * nb
     _say("sequences per workgroup", bw, nb, B, T, masks, with_h0)
-    masked = masks or T % 64 != 0 or bw % 32 != 0 or bw == 96
-    assert _sequences_fill_the_chip(bw, nb, B, masked) == (masked if owned is None else owned)
+    masked = masks or T % 64 != 0                            # the tiled kernel would run its masked variant
+    was = set_chain_forward(1)
+    try:
+        runs = _lib.load().rglru_hip_forward_owns_sequences(B, T, W, nb, _lib.RGLRU_BF16, 1 if masks else 0)
+    finally:
+        set_chain_forward(was)
+    assert runs == (masked if owned is None else owned)
     case = orc.make_case(B, T, W, nb, seed=bw + T, h0_std=0.5 if with_h0 else 0.0, bias_std=0.5)
     reset, active = _masks(B, T, masks)
     dh_last = torch.randn(B, W, generator=torch.Generator().manual_seed(6)) if with_h0 else None
