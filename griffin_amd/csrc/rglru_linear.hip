@@ -462,17 +462,30 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   }
 }
 
-// How a product is cut up.  Tiles of 128 x 128 where they give every compute unit one, else 64 x 64 (four times the workgroups
-// at half the reuse): at 2331 x 1024 x 768 in bf16 two forward products take 20 us either way (304 large tiles), one of
-// 2331 x 768 x 1024 12 us in small tiles and 18 us in 114 large ones.  A weight gradient contracts over the tokens, so its
-// tiles are few and its contraction long: it is split over workgroups until there are about two to a compute unit, at
-// least four slices each and at most eight splits (every split costs a pass over the result in fp32; 2331 tokens,
-// 768 x 1024: 67 us whole, 24 us in four, 19 us in eight).
+// How a product is cut up: tiles of 128 x 128, or 64 x 64 (four times the workgroups at half the reuse).
+// Forward and input gradients: time goes in steps of one tile a compute unit, and steps of large tiles are four times as coarse.
+// In bf16 three small tiles on a compute unit take about as long as one large one, so the line lies where there are more than three.
+// On 256 compute units, us, small : large (small tiles in brackets), two problems or segments unless said:
+//   forward  1527 x 1024 x 768 (768) 11.2 : 10.6, 1655 (832) 14.3 : 11.0, 2331 16.5 : 14.3;  2039 x 768 x 1024 (768) 12.6 : 12.7, 2167 (816) 17.1 : 13.6;
+//            1883 x 768 x 1024 (720) 12.3 : 14.6;  one of 4087 x 768 x 1024 (768) 12.7 : 12.6, 4215 (792) 16.6 : 12.7;  503 x 2560 x 2560 (640) 37.4 :
+//            37.9, 631 (800) 47.0 : 38.1;  beyond, 4087 x 1024 x 768 (2048) 26.7 : 18.0, 5495 x 768 x 1024 (2064) 32.7 : 32.7
+//   input    3063 x 1024 x 768 (768) 22.1 : 25.0, 3191 (800) 29.1 : 25.0;  4087 x 768 x 1024 (768) 27.7 : 31.5, 4215 (792) 36.4 : 31.6
+// fp32 is bound by its MFMAs, and a small tile takes 1 / 4 of a large one and 6 % more, so the number of steps decides (M x 256 x 256, two
+// problems; steps small : large x 4):  8183 (4 : 4) 22.1 : 22.2, 8439 (5 : 8) 26.3 : 36.0, 14071 (7 : 8) 35.8 : 36.9, 15991 (8 : 8) 40.3 : 37.8, 16631
+// (9 : 12) 44.2 : 54.9, 24567 (12 : 12) 58.9 : 56.3;  input gradient 8183 (2 : 4) 24.6 : 40.8, 16375 (4 : 4)
+// 39.9 : 42.5.
+// A weight gradient contracts over the tokens, so its tiles are few and its contraction long: it is split over workgroups until there
+// are about two to a compute unit, at least four slices each and at most eight splits (every split costs a pass over the result in
+// fp32).  With that pass, us, small : large (splits), bf16, 2331 tokens unless said: 768 x 1024 whole 31.4, 23.2 (3) : 25.0 (8), 4096 tokens 32.0 :
+// 28.4, 8192 52.6 : 38.0; 2 x 256 x 256 31.4 whole, 15.0 (4), 12.0 (8), 13.9 (9), always small; 2560 x 2560 88.3 (1) : 74.3 (2).  Two of 1024 x 768
+// are large from 1024 tokens on and would be faster in small tiles up to 4096: 30.0 (2) : 37.5 (6), 4096 tokens 42.4 : 45.3, 8192 74.4 : 71.3; in
+// fp32 83 : 108.
 struct LinearPlan { bool large; int splits; };
 static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
   auto tiles = [&](int64_t edge) { return ((M + edge - 1) / edge) * ((N + edge - 1) / edge) * problems; };
   const int64_t units = num_compute_units();
-  LinearPlan p = {tiles(128) >= units, 1};
+  auto steps = [&](int64_t edge) { return (tiles(edge) + units - 1) / units; };
+  LinearPlan p = {dtype == RGLRU_BF16 ? tiles(64) > 3 * units : tiles(128) > units && 106 * steps(64) >= 400 * steps(128), 1};
   if (kind != RGLRU_LINEAR_WEIGHT_GRAD) return p;
   const int64_t slices = (K + (dtype == RGLRU_BF16 ? 63 : 31)) / (dtype == RGLRU_BF16 ? 64 : 32);
   auto splits = [&](int64_t t) {

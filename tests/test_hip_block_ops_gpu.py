@@ -1007,6 +1007,31 @@ def test_bias_of_a_forward_product_may_start_at_any_element(M, N, K, first, dtyp
         assert torch.equal(hip_linear(x, w, b), got)
 
 
+# On 256 compute units, small tiles : large: bf16 768 small ones (small), 800 (large); fp32 1024 : 256 (small), 1056 : 264 (small), 2016 : 512
+# (large), 2112 : 528 (small)
+@pytest.mark.parametrize("dtype,N,M", [(torch.bfloat16, 1024, 3070), (torch.bfloat16, 1024, 3200), (torch.float32, 1024, 4090),
+                                       (torch.float32, 1024, 4200), (torch.float32, 2048, 3970), (torch.float32, 2048, 4200)])
+@pytest.mark.parametrize("kind,K", [(0, 72), (1, 136)])
+def test_linear_products_either_side_of_the_line_between_tiles(kind, K, dtype, N, M):
+    """Forward products and input gradients whose rows end inside a tile, on both sides of each line that chooses between small and large
+    tiles; what lies behind the operands and around the result is NaN."""
+    from griffin_amd import _lib
+
+    _say("tiles", kind, M, N, K, dtype)
+    gen = torch.Generator().manual_seed(M)
+    nan = lambda rows, cols: torch.full((rows + 130, cols), float("nan"), dtype=dtype, device="cuda")
+    a, b, c = nan(M, K), nan(N if kind == 0 else K, K if kind == 0 else N), nan(M, N)
+    a[:M] = torch.randn(M, K, generator=gen).to(dtype).cuda()
+    b[:-130] = torch.randn(b.size(0) - 130, b.size(1), generator=gen).to(dtype).cuda()
+    _lib.check(_lib.load().rglru_hip_linear(kind, a.data_ptr(), None, K, b.data_ptr(), None, b.size(1), None, None, None, c.data_ptr(), None, N, None,
+                                            None, M, N, K, _lib.RGLRU_BF16 if dtype == torch.bfloat16 else _lib.RGLRU_F32,
+                                            torch.cuda.current_stream().cuda_stream), "linear")
+    x, w = a[:M].double(), (b[:N].t() if kind == 0 else b[:K]).double()
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0         # rounding of the result; then K additions in fp32
+    bound = unit * (x @ w).abs() + (K + 2) * 2.0 ** -24 * (x.abs() @ w.abs())
+    assert ((c[:M].double() - x @ w).abs() <= bound).all() and torch.isnan(c[M:]).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K", [(1, 8, 8), (63, 72, 64), (65, 64, 136), (64, 128, 40), (700, 200, 328), (2050, 2056, 72), (1100, 136, 2304)])
 def test_linear_products_match_fp64(M, N, K, dtype):
