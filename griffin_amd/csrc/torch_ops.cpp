@@ -1367,12 +1367,15 @@ Tensor sum_sets(const Tensor& sets) {
 
 // Whether products of `macs` multiply-adds each (tokens x width x model width) run on the library's own kernels.  The BLAS
 // library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us and a
-// training step of the block has seven.  The line lies where both ways take equally long per layer in a stack of eight blocks,
+// training step of the block has seven.  The line lies where both ways take about equally long per layer in a stack of eight blocks,
 // alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
-// alone / with MLPs).  bf16, training 768 -> 1024: at 3.0e9 269 : 316 / 716 : 728, at 6.0e9 401 : 440 / 1106 : 1150, at 1.3e10 651 : 532 / 1847 : 1703;
-// 2560 -> 2560 at 4.5e9 373 : 384 / 963 : 952, at 6.0e9 431 : 419 / 1121 : 1108; a block's prefill alone 768 -> 1024 at 6.4e9 86 : 90, at 9.7e9
-// 119 : 118, 2560 at 6.7e9 118 : 107.  fp32, training 768 -> 1024: at 8e8 358 : 503 / 773 : 757, at 1.6e9 521 : 492 / 1257 : 1178.  Inside a captured graph
-// host time is nothing: there the line lies where the kernels take equally long.
+// alone / with MLPs).  bf16, training 768 -> 1024: at 3.0e9 250 : 273 / 702 : 721, at 6.0e9 363 : 423 / 1067 : 1124, at 6.4e9 368 : 344 / 1069 : 1036 (8192
+// tokens: the BLAS library has its best tiles at powers of two), at 8.0e9 445 : 506 / 1269 : 1338, at 1.3e10 620 : 527 / 1821 : 1707;  2560 -> 2560 at
+// 5.0e9 373 : 404 / 987 : 992, at 6.0e9 429 : 459 / 1121 : 1100, at 8.0e9 478 : 466 / 1234 : 1183;  prefill 768 -> 1024 at 4.0e9 82 : 86 / 201 : 199, at 6.0e9
+// 96 : 102 / 281 : 287, at 8.0e9 116 : 117 / 325 : 336, at 1.3e10 163 : 149 / 453 : 442;  2560 at 6.0e9 126 : 135 / 306 : 303, at 6.7e9 141 : 127 / 327 : 311.  So
+// between 6e9 and 9e9 either way wins somewhere.  fp32, training 768 -> 1024: at 8e8 326 : 469 / 759 : 755, at 9e8 362 : 468 / 843 : 824, at 1.2e9
+// 430 : 463, at 1.6e9 484 : 452;  wide and short ones lose below the line: 2560 -> 2560 at 5.8e8 (88 tokens) 481 : 466 / 1004 : 865, prefill
+// 151 : 123.  Inside a captured graph host time is nothing: there the line lies where the kernels take equally long.
 bool own_products(double macs, at::ScalarType dtype) {
   if (!known(dtype)) return false;
   const bool bf16 = dtype == at::kBFloat16;
