@@ -175,18 +175,19 @@ RGLRU_DEVICE void fwd_finalize(const FusedArgs& p, const WaveId& w, const FwdTil
 // 32768 tokens).
 constexpr int kFwdMT = 2;
 // ... except where a block wider than 128 channels needs the registers: each wave holds 8 NKG registers of
-// weights, and with one wave a SIMD nothing covers a tile's latency chain.  Measured per block width at
-// B1 T32768 and B4 T2048 (forward, ms; 64-token tiles and one workgroup a compute unit first):
-//   160: 0.185 -> 0.147, 192: 0.224 -> 0.161, 224: 0.199 -> 0.176 with 64-token tiles and two workgroups
-//   (224: 7 spilled registers); 288: 0.370 -> 0.302, 320: 0.390 -> 0.347 with 32-token tiles and two
-//   workgroups (320: 14 spilled registers); 256, 352, 384 are fastest as they were.
+// weights, and with one wave a SIMD nothing covers a tile's latency chain.  Forward at B1 T32768 in eight blocks, us, without flags / with
+// them, as chosen against the other tile and the other number of workgroups on a compute unit:
+//   160-wide 113 / 129, 32-token tiles 172 / 173, one workgroup 165 / 183;  192 130 / 139, 188 / 183, 192 / 210;  224 133 / 153, 192 / 199, 179 / 201
+//   288 254 / 282, 64-token tiles 389 / 289, one workgroup 380 / 404;  320 277 / 300, 322 / 337, 392 / 416
+//   352 298 / 328, 32-token tiles 406 / 441, two workgroups 501 / 523;  384 322 / 387, 421 / 468, 607 / 654
+//   256 187 / 207, 32-token tiles 265 / 283, two workgroups 167 / 282 (without flags they would gain; B4 T2048 48.6 : 50.6, B16 158 : 139)
 constexpr int fwd_mt(int nkg) { return (nkg == 18 || nkg == 20) ? 1 : kFwdMT; }
 constexpr int fwd_wide_occ(int nkg) { return (nkg == 16 || nkg > 20) ? 1 : 2; }
 // K groups of the weights that a wave keeps in LDS instead of registers (HeldWeights) where two workgroups a
 // compute unit leave too few registers.  The compiler's own spill goes to scratch memory: its reloads sit at the top of
 // the gate products and wait for every vector memory operation in flight, the record prefetch of the look-back
-// included.  Chosen so that nothing spills (224-wide masked: 4 registers still do) and two workgroups still fit the
-// LDS (8 KB per group and workgroup).  Forward at B1 T32768, us: 224-wide 163 -> 158, 320-wide 314 -> 292.
+// included.  Chosen so that nothing spills and two workgroups still fit the LDS (8 KB per group and workgroup).  Forward at B1 T32768, us,
+// without -> with, and with flags: 224-wide 135 -> 133, 159 -> 153; 288-wide with flags 296 -> 282; 320-wide 286 -> 277, 354 -> 300.
 constexpr int fwd_lds_groups(int nkg, bool masked) {
   return nkg == 14 ? (masked ? 4 : 3) : nkg == 18 ? (masked ? 5 : 0) : nkg == 20 ? (masked ? 6 : 4) : 0;
 }
@@ -358,8 +359,11 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
     // sequence has at most four workgroups on it.  With more of them the chunk in front is not out yet and the early look comes back
     // empty; so does one at the top of the tile, the place it had before.  Forward alone, us, with the priority above: B16 T2048
     // W2560 238 -> 228, the block's forward at B8 T2048 W1024 53 -> 49 (16 gate blocks), B1 T32768 W2560 294 (315 when it looked).
-    // The line, 320-wide blocks, never : up to four (workgroups on a sequence in brackets): B8 T2048 W2560 (2.6) 130 : 114, B6 (3.5)
-    // 101 : 97; up to six: B4 (5.3) 73.9 : 75.3.
+    // The line, never : up to four : up to six (workgroups on a sequence in brackets).  320-wide blocks: B8 T2048 W2560 (2.6) 130 : 114, B6
+    // (3.5) 101 : 97; B4 (5.3) 73.9 up to four, 75.3 up to six.  Narrower ones: 128-wide W1024, B22 T2048 (2.9) 69.2 : 65.0 : 64.6, B12 (5.3) 41.9 : 42.0 :
+    // 43.3, with flags B22 T640 34.0 : 33.7 : 33.4; 20 blocks of them, B7 T2048 (3.7) 57.2 : 53.6 : 53.9; 96-wide B30 T2048 W768 (2.8) 94.0 : 89.9 : 90.0;
+    // 48-wide B24 T2048 W768 (5.3) 76.6 : 75.5 : 77.6, B48 (2.7) 149 : 145 : 150; 64-wide B30 T2048 W1024 (3.2) 84.8 : 84.7 : 85.1, B24 W2560 (1.6) 161 :
+    // 155 : 155; 32-wide B32 T2048 W1024 (3) 87.4 : 81.5 : 82.4.
     const unsigned rec_lane = (slab_ok && w.ch_ok) && p.wg_per_unit <= 4 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
     // A dead finalize in front of the loop: the loop is entered with the same memory operations in
     // flight as its back edge has, so the waits at its top are exact instead of worst case.

@@ -8,11 +8,14 @@ namespace rglru {
 // blocks side by side) like the tiled kernel; x is double-buffered in LDS, so a tile costs one barrier, and the next tile is requested
 // as soon as this one is in LDS.  Flags come as one byte a lane and become two words by ballot; a tile without any takes the plain
 // gate math whether or not the call has flags.
-// Bound by latency and issue: two waves a SIMD (243 registers, 64 of them weights) cover each other's products, LDS round
-// trips and chains only in part (VALU 54 %); without the loads and stores 595 of 759 us would be left.
-// Forward at B256 T2048 W1024, 128-wide blocks, same device: 834 us tiled (+ 19 us clearing 134 MB of records), 759 here.  64-wide and
-// narrower blocks have registers for three workgroups with 32-token tiles: B256 T512 W1024 198 (+ 9) -> 179 us, with 64-token tiles 186.
-// For 128-wide blocks three workgroups spill (845 us).
+// Bound by vector issue: 24.5 vector instructions an element, six of them transcendental, keep the vector unit active on 73 % of the
+// SIMD clocks; two waves a SIMD (243 registers, 64 of them weights) cover each other's chains and LDS round trips for the rest.  The
+// 2.3 GB it moves take 3.4 TB/s; without loads and stores 560 of 680 us would be left.
+// Forward of B256 W1024 in calls behind each other (the clock follows the load: a launch between lighter ones says little), us, tiled with
+// the clearing of its records : here:  T2048 in 128-wide blocks 714 : 680, with flags 829 : 686, T512 185 : 177.  64-wide and narrower blocks
+// have registers for three workgroups with 32-token tiles: T2048 643 : 588, with flags 750 : 583, T512 165 : 149 (two workgroups with 64-token
+// tiles 4 % more).  For 128-wide blocks three workgroups spill (11 % more).  Without the checkpoints, 134 MB that only a backward pass reads,
+// it takes as long (686).
 constexpr int rows_mt(int nkg) { return nkg <= 4 ? 1 : 2; }
 constexpr int rows_occ(int nkg) { return nkg <= 4 ? 3 : 2; }
 

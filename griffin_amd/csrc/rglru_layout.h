@@ -60,8 +60,8 @@ inline PrepLayout make_prep_layout(const Geometry& g, size_t elem) {
 // of 64 tokens.
 //   ckpt        [B][2 nC][W]    fp32 state after every 16 tokens (kept for backward: each lane of the
 //                               backward scan owns 16 consecutive tokens and starts from one of these)
-//   --- [f_begin, f_end) is cleared at the start of a forward pass that uses records (the kernels with one
-//       workgroup per chain use none and clear the failure word only) ---
+//   --- [f_begin, f_end) is cleared at the start of a forward pass that uses records (the kernels whose workgroups own a
+//       chain or whole sequences use none and clear the failure word only) ---
 //   f_rec_a     [B][<=nC][W]    64-bit carry records of the forward chain
 //   f_ticket    [units][kMaxQueues]
 //   fail        [1]             failure word (either pass sets it; only forward clears it)
