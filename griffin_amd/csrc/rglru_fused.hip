@@ -364,7 +364,9 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
     // 43.3, with flags B22 T640 34.0 : 33.7 : 33.4; 20 blocks of them, B7 T2048 (3.7) 57.2 : 53.6 : 53.9; 96-wide B30 T2048 W768 (2.8) 94.0 : 89.9 : 90.0;
     // 48-wide B24 T2048 W768 (5.3) 76.6 : 75.5 : 77.6, B48 (2.7) 149 : 145 : 150; 64-wide B30 T2048 W1024 (3.2) 84.8 : 84.7 : 85.1, B24 W2560 (1.6) 161 :
     // 155 : 155; 32-wide B32 T2048 W1024 (3) 87.4 : 81.5 : 82.4.
-    const unsigned rec_lane = (slab_ok && w.ch_ok) && p.wg_per_unit <= 4 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
+    // Short sequences of wide blocks are looked at early in any case, the tiles in front are then done or close to it (at most 12 : 48 : all
+    // chunks): 320-wide B2 T512 W2560 25.5 : 24.5 : 25.1, B1 T640 W5120 26.8 : 26.1 : 26.4, B1 T4500 W5120 84.0 : 83.9 : 91.2; 288-wide B2 T900 27.2 : 26.4 : 26.3.
+    const unsigned rec_lane = (slab_ok && w.ch_ok) && (p.wg_per_unit <= 4 * p.B || (NKG > 8 && p.nCf <= 48)) ? (unsigned)w.ch * 8u : kOutOfRange;
     // A dead finalize in front of the loop: the loop is entered with the same memory operations in
     // flight as its back edge has, so the waits at its top are exact instead of worst case.
     bf16x8 gate_rows[BLOCK ? TR / 16 : 1];               // the lane's vectors of the second projection
@@ -384,8 +386,10 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
       // next ticket: one instruction for the whole workgroup, live only in its first lane
       const unsigned next_raw = (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, rticket, tid == 0 ? 0u : kOutOfRange, 0, 0);
       // From here until its carry is out, the tile is what other workgroups wait for: its waves go before those of the
-      // workgroup that shares their SIMDs and is storing (forward alone, us: B256 T2048 W1024 831 -> 808, B8 T2048 W2560 109 -> 106).
-      __builtin_amdgcn_s_setprio(1);
+      // workgroup that shares their SIMDs and is storing (forward alone, us: B256 T2048 W1024 831 -> 808, B1 T32768 W1024 71.6 -> 68.3, B3 T3818 W1536 48.1
+      // -> 43.3).  Nothing waits in sequences of one tile (B36 T40 W1536 15.8 -> 15.0 without), and 32-token tiles gain nothing (B1 T32768 W2560
+      // 269.0 with it, 266.6 without).
+      if (MT > 1 && p.nCf > 1) __builtin_amdgcn_s_setprio(1);
       if constexpr (BLOCK) {
         const int t0 = cur.c * TR;
         const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
@@ -501,8 +505,10 @@ __global__ __launch_bounds__(kThreads, (BLOCK ? 2 : NKG < 0 ? RGLRU_GIVEN_OCC : 
                                                    (unsigned)(w.k * p.bw + w.slab * 32) * 2u + (unsigned)(w.lane & 3) * 16u);
       }
       // The next tile is requested behind the look-back: loads return in issue order, so requested in front of it, as it was, its
-      // latency is part of every round trip of the walk (block forward at B8 T2048 W1024 49.9 -> 47.6 us, B8 T2048 W2560 98.8 -> 95.8).
-      auto next = [&]() { issue(tk_next); };
+      // latency is part of every round trip of the walk (block forward at B8 T2048 W1024 49.9 -> 47.6 us).  32-token tiles have half the time to
+      // cover it and request it in front (B1 T32768 W2560 277 behind, 266 in front; with flags 297, 288).
+      if constexpr (MT == 1) issue(tk_next);
+      auto next = [&]() { if constexpr (MT != 1) issue(tk_next); };
       fwd_finalize<IO, MT, MASKED, sizeof(IO) == 2, BLOCK, PAD>(p, w, cur, stage, &ahead, slab_ok, gate_rows, next);
       tk = tk_next;
     }
