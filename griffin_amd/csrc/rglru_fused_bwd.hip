@@ -172,9 +172,9 @@ RGLRU_DEVICE void hold_in_loop(unsigned& v) { asm volatile("" : "+v"(v)); }
 // 6.6 clocks, two waves together every 2.5 to 4.4).  So two workgroups share a compute unit, which leaves a wave 256 registers:
 // up to 96 for the weights of twelve K groups, the others' (8 KB each) in LDS, where the outputs are staged over the x and dy
 // tiles.  A wave keeps per token r, a, the input gate's pre-activation, x and dy; the rest is computed behind the
-// look-back, two tokens at a time.  Forward state, ticket and tile of the next pass are requested in front of this pass's stores.
+// look-back, two tokens at a time.  Forward state and tile of the next pass are requested in front of this pass's stores.
 // Until then a compute unit had one workgroup of four waves with 300 to 430 registers each.  Reverse scan, us, before -> now:
-//   320-wide blocks: B1 T32768 508 -> 420, B16 T2048 458 -> 321; 160-wide blocks: B8 T2048 W2560 270 -> 185.
+//   320-wide blocks: B1 T32768 498 -> 404, B16 T2048 447 -> 305; 160-wide blocks: B8 T2048 W2560 270 -> 185.
 // Without the look-back the first would take 314, without the memory behind the stores 370 (timing builds).  Blocks of 352 and 384
 // channels need 264 and more registers this way and stay with one workgroup.
 constexpr int bwd_wide_occ(int nkg) { return nkg <= 20 ? 2 : 1; }
@@ -350,11 +350,11 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
   // it: the tile behind is then finished (320-wide blocks, W2560: B16 T2048 321 against 343 us, B8 T1024 97 against 100).  With more of
   // them on one chain it is not, and the early look only comes back empty (B4 T2048 108 against 104.5, B1 T32768 458 against 420 us).
   const unsigned ahead_lane = ch_ok && p.wg_per_unit <= 4 * p.B ? (unsigned)w.ch * 8u : kOutOfRange;
-  // Everything that the next tile needs early -- its tile, the state in front of it, the ticket after it -- is requested in front
-  // of the stores of this one: the counter that loads are waited for with counts in issue order, so whatever is requested
-  // behind the stores is waited for together with them.
+  // What the next tile needs early -- its tile and the state in front of it -- is requested in front of the stores of this one: the
+  // counter that loads are waited for with counts in issue order, so whatever is requested behind the stores is waited for together
+  // with them.  The next ticket is taken behind the stores to LDS: a tile early, a workgroup holds one that an idle one could have started
+  // (us, early : here: B1 T32768 W2560 414 : 404, B1 T3000 W2048 47.7 : 41.9, B1 T322 W2432 19.6 : 18.5).
   request_state(tk);
-  unsigned next_raw = request_ticket();
   six_dropped_stores();
   while ((long long)tk < q.tiles) {
     int c, b;
@@ -366,6 +366,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
       lds_barrier();                                     // the stages of the tile before have been read
     }
     deposit();
+    const unsigned next_raw = request_ticket();
     unsigned flbits = 0u;                                // the token flags (two bits per local step)
     if constexpr (MASKED) flbits = flag_run(p, trow, t0 + hf * EL);
     const float h_start = h_ckpt + h_init;               // state in front of this lane's 16 tokens
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
                                    : carry_lookback(chain, c, +1, p.nC, 0.f, ch_ok, p.limit, p.fail);
     // the next tile's loads go out behind the look-back: loads return in issue order, so requested in front of it
     // they would put their latency into every round trip of the walk
-    if constexpr (!SHARED) { issue(tk_next); request_state(tk_next); next_raw = request_ticket(); }
+    if constexpr (!SHARED) { issue(tk_next); request_state(tk_next); }
     const float d_out = fmaf(A_t, d_in, D_t);
     if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
     if constexpr (SHARED) __builtin_amdgcn_s_setprio(0);
@@ -507,7 +508,7 @@ __global__ __launch_bounds__(kThreads, (NKG > 8 ? bwd_wide_occ(NKG) : 2)) void b
       }
       if constexpr (SHARED) { if (e & 1) __builtin_amdgcn_sched_barrier(0); }
     }
-    if constexpr (SHARED) { issue(tk_next); request_state(tk_next); next_raw = request_ticket(); }
+    if constexpr (SHARED) { issue(tk_next); request_state(tk_next); }
     wave_lds_fence();
     {
       unsigned fl_lane = (unsigned)w.lane;               // the offsets of the stores: a register each if they stayed between tiles
@@ -2283,13 +2284,19 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   a.aligned = 1;
   const int nkg = wide_groups(g, dtype, 1);
   const bool pad = wide_padded(g);
-  // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums.  Two workgroups a compute unit where each
-  // has two tiles or more: with fewer what they load first, the weights, is most of their time (320-wide blocks of W2560, us, two : one:
-  // 1.5 tiles each at B2 T512 29.4 : 27.1, 1.9 at B4 T300 33.0 : 31.8, 3 at B4 T512 39.0 : 39.9, 3.8 at B8 T300 43.5 : 47.5; 160-wide, 2.5 at
-  // B4 T300 25.7 : 29.6).
-  a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, bwd_wide_occ(nkg), L.max_wg);
-  if (B * (long long)a.nC < 2 * (long long)pick_wg_per_unit(a.units, 1ll << 40, bwd_wide_occ(nkg), L.max_wg))
-    a.wg_per_unit = pick_wg_per_unit(a.units, B * (long long)a.nC, 1, L.max_wg);
+  // reverse scan and gate math: direct part of dx, du2, per-workgroup bias and Lambda sums.  Two workgroups a compute unit where one
+  // each would have more than two tiles: with fewer what they load first, the weights, is most of their time.  us, one : two (tiles that
+  // one each would have; 288- and 320-wide ones round the number of workgroups up):
+  //   136-wide  W1088 (1.5) 16.8 : 17.5, (2) 20.6 : 18.8, (2.4) 23.9 : 20.3   160  W2560 (1.6) 17.1 : 16.4, (2) 15.9 : 16.1 and 17.9 : 17.0, (2.4) 20.9 : 18.2
+  //   192       W1536 (1.7) 20.0 : 20.4, (2) 20.8 : 21.9, (2.4) 25.2 : 22.8   224  W1792 (1.7) 19.5 : 19.4, (2) 20.5 : 20.6, (2.4) 23.4 : 21.8
+  //   256       W2048 (1.7) 21.6 : 24.5, (2) 22.5 : 24.7, (2.4) 27.0 : 25.5   288  W2304 (1.6) 19.5 : 19.8, (2) 24.1 : 21.2, (2.4) 24.2 : 21.7
+  //   320       W2560 (1.5) 19.6 : 22.9, (1.6) 21.9 : 23.1, (2) 26.0 : 24.7, (2.4) 27.4 : 25.7, (2.9) 27.1 : 28.9 and 28.1 : 28.5; W5120 (1.7) 25.4 : 23.3, (3.3) 40.0 :
+  //             33.2;  B1 T32768 W2560 520 : 402
+  // The rule before asked for two tiles of each of two workgroups: B1 T640 W5120 39.7 us, now 33.2.
+  const long long tiles = B * (long long)a.nC;
+  const long long spare = tiles - 2 * (long long)pick_wg_per_unit(a.units, 1ll << 40, 1, L.max_wg);
+  const bool share = spare > 0 || (spare == 0 && (nkg < 12 || nkg > 16));
+  a.wg_per_unit = pick_wg_per_unit(a.units, tiles, share ? bwd_wide_occ(nkg) : 1, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
   const bool masked = (flags != nullptr) || a.first_reset || (T % kChunk != 0);
   a.xcd_map = 1;

@@ -1046,10 +1046,10 @@ def test_wide_backward_with_few_and_many_workgroups_on_a_sequence(bw, B, T, mask
 
 
 @pytest.mark.parametrize("bw", [160, 320])
-@pytest.mark.parametrize("B,masks", [(5, False), (16, True)])
+@pytest.mark.parametrize("B,masks", [(4, True), (5, False), (16, True)])
 def test_wide_backward_with_several_tiles_a_workgroup(bw, B, masks):
-    """The reverse scan of wide blocks runs two workgroups a compute unit where each has two tiles or more, one elsewhere: batches on
-    either side of the line (175 and 560 tiles for 171 or 256 workgroups), against the oracle."""
+    """The reverse scan of wide blocks runs two workgroups a compute unit where one each would have more than two tiles, one elsewhere:
+    batches on either side of the line (140, 175 and 560 tiles; one each are 128 or 86), against the oracle."""
     T = 1100
     _say("several tiles", bw, B, masks)
     case = orc.make_case(B, T, bw, 1, seed=bw + B, h0_std=0.5, bias_std=0.5)
