@@ -603,6 +603,17 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
   constexpr int TW = kPackedWidth;                       // tile width (narrow blocks are packed)
   constexpr int LDSROW = TW + Tr::HW;
   static_assert(sizeof(IO) == 2 && NKG > 0, "fast backward is for 16-bit storage and register-held weights");
+  // Where the next tile is requested: behind the look-back, where no round trip of the walk waits for it (loads return in issue order),
+  // or in front of the chunk's map (FRONT), where its latency is covered earlier.  And when its ticket is taken: behind the tile's stores
+  // to LDS, or a tile early (AHEAD), where the request costs nothing but a workgroup then holds a tile that an idle one could have started.
+  // Reverse scan, us, before all of this : everything behind and ahead : as it is (of runs on different days the same kernels differ by 5 %):
+  //   16- to 64-wide   B87 T90 W256 (16) 16.4 : 17.5 : 16.8;  B543 T42 W384 (24) 28.4 : 30.1 : 29.1;  B1 T5905 W384 (48) 18.5 : 20.2 : 18.2;  B4 T4096 W1024 (64)
+  //                    33.5 : 29.4 : 29.8 (FRONT 31.3)
+  //   behind a gate    B87 T90 30.3 : 29.3 : 26.3;  B5 T4844 W640 (40) 82.0 : 88.3 : 83.0;  B219 T56 W1024 (64) 45.9 : 48.7 : 45.3;  B3 T7963 W640 (80) 87.8 :
+  //                    93.2 : 90.7
+  //   wider            B3 T3818 W1536 (96) 42.2 : 37.8, ticket late 38.6, FRONT 40.1;  B1 T32768 W1024 (128) 74.5 : 75.1, 77.5, 75.7;  gated B16 T2048 W2560
+  //                    (128) 249 : 224, 225, 260
+  constexpr bool FRONT = GATED && (NKG == 4 || NKG == 6), AHEAD = NKG == 8 || (NKG == 6 && !GATED);
   __shared__ __attribute__((aligned(16))) IO lds_x[TR * LDSROW];
   __shared__ __attribute__((aligned(16))) IO lds_dy[TR * LDSROW];
   __shared__ __attribute__((aligned(16))) unsigned char stage_all[PAD ? 16 : kWaves * WaveStage<TR>::kBytes];
@@ -676,17 +687,19 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
   unsigned tk = s_ticket[0];
   int par = 0;
   issue(tk);
-  // the next ticket: one atomic instruction for the workgroup, live in its first lane only (atomicAdd would combine the lanes'
-  // operations first and wait for the result on the spot)
+  // one atomic instruction for the workgroup, live in its first lane only (atomicAdd would combine the lanes' operations first and wait
+  // for the result on the spot)
   auto request_ticket = [&]() {
     return (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(1, make_rsrc(q.counter, 4u), tid == 0 ? 0u : kOutOfRange, 0, 0);
   };
-  unsigned next_raw = request_ticket();
+  unsigned raw_ahead = 0u;
+  if constexpr (AHEAD) raw_ahead = request_ticket();
   while ((long long)tk < q.tiles) {
     int c, b;
     decode(tk, c, b);
     const int t0 = c * TR;
     const long long trow = (long long)b * p.T + t0 + hf * EL;
+    unsigned next_raw = raw_ahead;
     __builtin_amdgcn_s_setprio(1);                         // until its carry is out, the tile is what others wait for
     unsigned flbits[MT];
 #pragma unroll
@@ -708,6 +721,7 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
         *reinterpret_cast<Frag*>(lds_dy + row * LDSROW + cv * Tr::HW) = pre_dy[i];
       }
     }
+    if constexpr (!AHEAD) next_raw = request_ticket();
     __syncthreads();
     float a[EL], gy[EL];
     if (w.slab_ok) {
@@ -735,10 +749,11 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     const unsigned tk_next = s_ticket[par];
     if (!w.slab_ok) {                                    // a wave without a slab only helps with the loads
       issue(tk_next);
-      next_raw = request_ticket();
+      if constexpr (AHEAD) raw_ahead = request_ticket();
       tk = tk_next;
       continue;
     }
+    if constexpr (FRONT) issue(tk_next);
     // reverse affine map of this lane's run and of the chunk: carry_out = A carry_in + D
     float A = 1.f, carry = 0.f;
 #pragma unroll
@@ -759,11 +774,9 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
     if (hf == 0 && ch_ok) carry_publish(chain, c, 0.f, d_out, true);
     if (hf == 0 && c == 0 && p.dh0 && ch_ok) p.dh0[(long long)b * W + w.ch] = d_out;
     __builtin_amdgcn_s_setprio(0);
-    // The next tile and ticket are requested behind the look-back, whose every round trip would wait for them otherwise (loads return
-    // in issue order), and in front of the stores, which they would wait for.  With the priority, us, before -> now: B1 T32768 W1024
-    // 80 -> 77, B2 T8192 34.9 -> 33.5, B128 T128 26.3 -> 25.1, B40 T409 (64-wide blocks) 30.5 -> 27.3, gated B1 T8192 37.6 -> 34.2.
-    issue(tk_next);
-    next_raw = request_ticket();
+    // in front of the stores, which it would wait for
+    if constexpr (!FRONT) issue(tk_next);
+    if constexpr (AHEAD) raw_ahead = request_ticket();
 
     carry = hf ? d_in : fmaf(A_hi, d_in, D_hi);
     const int rows = (p.T - t0) < TR ? (p.T - t0) : TR;
