@@ -606,7 +606,7 @@ __global__ __launch_bounds__(kThreads, (MT == 1 ? 4 : RGLRU_DELTA_OCC)) void bwd
   // Where the next tile is requested: behind the look-back, where no round trip of the walk waits for it (loads return in issue order),
   // or in front of the chunk's map (FRONT), where its latency is covered earlier.  And when its ticket is taken: behind the tile's stores
   // to LDS, or a tile early (AHEAD), where the request costs nothing but a workgroup then holds a tile that an idle one could have started.
-  // Reverse scan, us, before all of this : everything behind and ahead : as it is (of runs on different days the same kernels differ by 5 %):
+  // Reverse scan, us, before all of this : everything behind and ahead : as it is (the same code differs by up to 5 % between builds):
   //   16- to 64-wide   B87 T90 W256 (16) 16.4 : 17.5 : 16.8;  B543 T42 W384 (24) 28.4 : 30.1 : 29.1;  B1 T5905 W384 (48) 18.5 : 20.2 : 18.2;  B4 T4096 W1024 (64)
   //                    33.5 : 29.4 : 29.8 (FRONT 31.3)
   //   behind a gate    B87 T90 30.3 : 29.3 : 26.3;  B5 T4844 W640 (40) 82.0 : 88.3 : 83.0;  B219 T56 W1024 (64) 45.9 : 48.7 : 45.3;  B3 T7963 W640 (80) 87.8 :
@@ -2305,7 +2305,7 @@ int rglru_hip_bwd_wide(const void* x, const void* prep, const float* h0,
   //   256       W2048 (1.7) 21.6 : 24.5, (2) 22.5 : 24.7, (2.4) 27.0 : 25.5   288  W2304 (1.6) 19.5 : 19.8, (2) 24.1 : 21.2, (2.4) 24.2 : 21.7
   //   320       W2560 (1.5) 19.6 : 22.9, (1.6) 21.9 : 23.1, (2) 26.0 : 24.7, (2.4) 27.4 : 25.7, (2.9) 27.1 : 28.9 and 28.1 : 28.5; W5120 (1.7) 25.4 : 23.3, (3.3) 40.0 :
   //             33.2;  B1 T32768 W2560 520 : 402
-  // The rule before asked for two tiles of each of two workgroups: B1 T640 W5120 39.7 us, now 33.2.
+  // At exactly two the widths differ, see (2).  The rule before asked for two tiles of each of two workgroups: B1 T640 W5120 39.7, now 33.2.
   const long long tiles = B * (long long)a.nC;
   const long long spare = tiles - 2 * (long long)pick_wg_per_unit(a.units, 1ll << 40, 1, L.max_wg);
   const bool share = spare > 0 || (spare == 0 && (nkg < 12 || nkg > 16));
