@@ -608,8 +608,8 @@ inline int pick_queues(long long B, int wg) {
 
 // rglru_fwd_rows.hip: the forward of batches large enough that every workgroup can own whole sequences (16-bit storage, blocks of
 // up to 128 channels).
-int fwd_rows_tile(int nkg);
-int fwd_rows_per_cu(int nkg);
+int fwd_rows_tile(int nkg, bool flags, int64_t workgroups);
+int fwd_rows_per_cu(int nkg, bool flags);
 int launch_fwd_rows(const FusedArgs& a, int nkg, bool pad, hipStream_t s);
 
 // Whether the forward runs one workgroup per chain (fwd_chain_kernel) instead of tiles with look-back:

@@ -897,28 +897,48 @@ struct BlockFwd {
 
 
 // Workgroups per unit of the kernel whose workgroups own whole sequences (rglru_fwd_rows.hip), or 0 where the tiled kernel is the
-// better one.  It needs a sequence for every workgroup that fits the chip, and then its time grows in steps: the workgroups of a unit
-// that have one sequence more than the others lie on different compute units until every unit of the chip has one, then a second one
-// joins them, and so on.  `rounds` counts such steps of one sequence a compute unit; the last of them has to be nearly full.  How full
-// depends on the tiled kernel.  Forward, T512 unless said, us, tiled : rows (part of the rounds that is filled):
-//   128-wide, W1024 (64 workgroups a unit), odd rounds   B80 62.7 : 63.0 (83 %), 90 68.9 : 63.2 (94), 140 103.1 : 103.0 (88), 160 122 : 112
-//             even rounds, whose last sequence shares its compute unit   97 72.8 : 86.9 (76), 104 78.4 : 88.3 (81), 120 93.3 : 93.7 (94), 128 100 :
-//             96, 161 119 : 131 (84), 240 170 : 171 (94), 256 181 : 171; T2048 112 326 : 343, 120 352 : 350, 256 727 : 699
-//             20 units of them (25 workgroups each)   B38 78.5 : 91.1 (74), 48 93.5 : 89.6 (94), 51 94.9 : 101.1 (80), 64 125 : 134 (83)
-//   32- and 64-wide (three workgroups a compute unit)   B98 71.7 : 75.8 (77), 112 82.0 : 78.7 (88), 128 86.3 : 76.2, 161 112 : 119 (84), 176 120 : 118
-//             (92), 225 150 : 146 (88); T2048 98 262 : 282, 113 300 : 294, 170 448 : 451 (89)
-// Flags, ragged lengths and padded blocks cost the tiled kernel, whose variant for them is one for all three, up to a third; this one
-// only where a flag is.  96- and 128-wide   B70 68.9 : 68.5 (73), 77 74.7 : 68.0 (80), 97 91.1 : 93.6 (76), 104 96.5 : 96.2 (81), 128 118 : 98;
-// narrower ones always (48-wide B97 83.5 : 75.0, 64-wide with flags B98 88 : 78).
-static int fwd_row_workgroups(int64_t B, const Geometry& g, int nkg, bool masked) {
+// better one.  Its time grows in steps: sequences beyond one for every compute unit join those that are there, up to the workgroups
+// that fit.  `rounds` counts such steps of one sequence a compute unit; the last of them has to be nearly full.  How full depends on
+// the tiled kernel.  Forward, T512 unless said, us, tiled : rows (part of the rounds that is filled):
+//   no flags, three workgroups a compute unit.  128-wide, W1024, one round   B16 23.3 : 31.5 (50 %), 32 30.2 : 31.1 (100), T2048 32 94.1 : 109.7
+//             two rounds   B48 39.3 : 42.5 (75), 56 44.3 : 42.9 (88), 64 48.5 : 43.4, T2048 60 171 : 165 (94)
+//             more   B66 50.0 : 56.7 (69), 72 53.7 : 56.9 (75), 80 59.3 : 57.8 (83), 90 66.7 : 62.2 (94), 97 72.9 : 72.0 (76), 104 77.2 : 73.2 (81),
+//             128 99.1 : 83.3, 176 127 : 123 (92), 256 185 : 162; T2048 112 313 : 303 (88), 256 708 : 628
+//             20 units of them   B24 47.8 : 43.1 (94), 30 57.2 : 57.7 (78), 38 76.5 : 62.4, 51 93.8 : 90.1 (80), 64 118 : 114 (83)
+//             64-wide, W1024   B48 38.8 : 39.5 (75), 64 45.4 : 40.1, 80 56.7 : 53.1 (83), 112 75.7 : 68.0 (88), 161 105.7 : 106.9 (84), 256 171 : 146
+//             short sequences, which pay most for the clearing of the tiled kernel's records   T256 20 units B16 24.1 : 24.9 (63), 12 20.9 : 18.4
+//             (94), W1024 B32 20.2 : 18.5; T128 20 units B12 16.2 : 11.5 (94), 48-wide W768 B32 14.6 : 10.2
+//             ragged lengths and padded blocks, which cost the tiled kernel up to a third   T300 B40 31.0 : 30.2 (63), 48 33.1 : 29.9 (75), T777
+//             64 89.6 : 70.2, 128 181 : 127; 96-wide B48 41.0 : 40.6 (75), 64 50.7 : 40.7, 72 56.7 : 53.9 (75), one round 32 30.4 : 30.4
+//   flags, two workgroups a compute unit, from a sequence for each of them on (three, 64-wide and narrower, always): 96- and 128-wide   B70
+//             68.9 : 68.5 (73), 77 74.7 : 68.0 (80), 97 91.1 : 93.6 (76), 104 96.5 : 96.2 (81), 128 118 : 98; 48-wide B97 83.5 : 75.0, 64-wide B98
+//             88 : 78
+// Sequences of fewer than 128 tokens have the line of the kernel with flags with or without them, and fuller rounds where the tiled
+// kernel runs its plain variant (88 %; 93 where the last round's sequences share their compute units): both kernels are done in 7 to 25 us
+// there, mostly launch (T64 W1024 B32 11.1 : 8.1, left to the tiled one).
+static int fwd_row_workgroups(int64_t B, int64_t T, const Geometry& g, int nkg, bool masked, bool flags) {
   FusedArgs a;
   a.units = (int)g.units;
   pack_units(a, g, nkg);
-  const int64_t cus = num_compute_units(), per_cu = fwd_rows_per_cu(nkg), slots = cus * per_cu / a.units;
-  if (slots < 1 || B < slots) return 0;
-  const int64_t left = B % slots, rounds = B / slots * per_cu + (left * a.units + cus - 1) / cus;
-  const int need = per_cu == 3 ? (masked ? 0 : 88) : masked ? 80 : rounds % 2 ? 88 : 93;
-  return 100 * B * a.units >= need * rounds * cus ? (int)slots : 0;
+  const int64_t cus = num_compute_units();
+  auto filled = [&](int64_t slots, int64_t per_cu, int64_t& rounds) {          // part of the rounds, in percent
+    const int64_t left = B % slots;
+    rounds = B / slots * per_cu + (left * a.units + cus - 1) / cus;
+    return 100 * B * a.units / (rounds * cus);
+  };
+  const int64_t per_cu = fwd_rows_per_cu(nkg, flags), slots = cus * per_cu / a.units;
+  int64_t rounds;
+  if (flags || T < 128) {
+    const int64_t line_per_cu = fwd_rows_per_cu(nkg, true), line = cus * line_per_cu / a.units;
+    if (line < 1 || B < line) return 0;
+    const int64_t part = filled(line, line_per_cu, rounds);
+    if (part < (line_per_cu == 3 ? (masked ? 0 : 88) : masked ? 80 : rounds % 2 ? 88 : 93)) return 0;
+  } else {
+    if (slots < 1) return 0;
+    const int64_t part = filled(slots, per_cu, rounds);
+    if ((rounds < 2 && T > 256) || part < (masked || T <= 256 ? 70 : rounds % 2 ? 80 : 85)) return 0;
+  }
+  return (int)(slots < B ? slots : B);
 }
 
 // Kernel of a forward without block and without given pre-activations.
@@ -928,7 +948,7 @@ static FwdRoute fwd_route(int64_t B, int64_t T, const Geometry& g, int nkg, bool
   r.chain = narrow && fwd_chain_pays(B, T, g.Wp);
   // the tiled kernels with register-held weights of whole blocks know first_reset and whole tiles; anything else is their masked variant
   r.masked = pad || flags || T % (32 * fwd_mt(nkg)) != 0 || (first_reset && !(nkg == 8 || nkg == 4 || nkg == 2));
-  r.row_wg = narrow && !r.chain ? fwd_row_workgroups(B, g, nkg, r.masked) : 0;
+  r.row_wg = narrow && !r.chain ? fwd_row_workgroups(B, T, g, nkg, r.masked, flags) : 0;
   return r;
 }
 
@@ -1037,7 +1057,8 @@ static int fwd_impl(const void* x, const void* prep, const float* h0, const uint
   }
   pack_units(a, g, nkg);
   if (row_wg) {
-    a.nCf = (int)((T + fwd_rows_tile(nkg) - 1) / fwd_rows_tile(nkg));
+    const int64_t tile = fwd_rows_tile(nkg, flags != nullptr, (int64_t)row_wg * a.units);
+    a.nCf = (int)((T + tile - 1) / tile);
     a.wg_per_unit = row_wg;
     KernelTimer timer(0, s);
     return launch_fwd_rows(a, nkg, pad, s);

@@ -6,20 +6,24 @@ namespace rglru {
 // Tiles of a sequence run one after the other in one workgroup, the state stays in a register: no tickets, no records, no look-back,
 // nothing to clear, and the order of the sums is fixed.  A workgroup of four waves holds the unit's 128 channels (or its
 // blocks side by side) like the tiled kernel; x is double-buffered in LDS, so a tile costs one barrier, and the next tile is requested
-// as soon as this one is in LDS.  Flags come as one byte a lane and become two words by ballot; a tile without any takes the plain
-// gate math whether or not the call has flags.
-// Bound by vector issue: 24.5 vector instructions an element, six of them transcendental, keep the vector unit active on 73 % of the
-// SIMD clocks; two waves a SIMD (243 registers, 64 of them weights) cover each other's chains and LDS round trips for the rest.  The
-// 2.3 GB it moves take 3.4 TB/s; without loads and stores 560 of 680 us would be left.
+// as soon as this one is in LDS.  Calls with flags have a variant of their own: they come as one byte a lane and become two words by
+// ballot, and a tile without any takes the plain gate math.  Two versions of that math in one kernel cost 40 registers and the
+// scheduler its freedom, so calls without flags do not have them (128-wide: 243 -> 208 registers with 64-token tiles, 142 with 32).
+// Bound by power: 24.5 vector instructions an element, six of them transcendental, and the matrix products beside them draw the
+// clock down to 2.0-2.1 GHz.  Without its loads and stores the kernel takes 500 of 650 us, without its gate math 530, and every
+// arrangement tried takes the same 650-660: tiles of 32 or 64 tokens, tiles requested two ahead, x or y brought into their layout by
+// products with the identity instead of two-byte LDS accesses.
 // Forward of B256 W1024 in calls behind each other (the clock follows the load: a launch between lighter ones says little), us, tiled with
-// the clearing of its records : here:  T2048 in 128-wide blocks 714 : 680, with flags 829 : 686, T512 185 : 177.  64-wide and narrower blocks
-// have registers for three workgroups with 32-token tiles: T2048 643 : 588, with flags 750 : 583, T512 165 : 149 (two workgroups with 64-token
-// tiles 4 % more).  For 128-wide blocks three workgroups spill (11 % more).  Without the checkpoints, 134 MB that only a backward pass reads,
-// it takes as long (686).
-constexpr int rows_mt(int nkg) { return nkg <= 4 ? 1 : 2; }
-constexpr int rows_occ(int nkg) { return nkg <= 4 ? 3 : 2; }
+// the clearing of its records : two workgroups a compute unit with 64-token tiles and both versions of the math : three with 32-token
+// tiles and one: T2048 in 128-wide blocks 708 : 672 : 628, T512 185 : 175 : 162.  With flags 829 : 686, the three-workgroup form
+// spills (11 % more).  64-wide blocks, three workgroups and 32-token tiles: T512 171 : 150 : 146, with flags T2048 750 : 583.
+// Where no more than two workgroups a compute unit have a sequence, the tiles of 96- and 128-wide blocks have 64 tokens without flags, too
+// (B64 T2048 W1024 176.7 -> 172).
+constexpr int rows_occ(int nkg, bool flags) { return nkg <= 4 || !flags ? 3 : 2; }
+static bool rows_long_tiles(int nkg, bool flags, int64_t workgroups) { return nkg > 4 && (flags || workgroups <= 2 * (int64_t)num_compute_units()); }
 
-// Gate outputs of 16 consecutive tokens (bits at .. at + 15 of the reset and padding words belong to them).
+// Gate outputs of 16 consecutive tokens (bits at .. at + 15 of the reset and padding words belong to them; without MASKED, bit 0 of
+// `resets` to the first of them).
 template <bool MASKED>
 RGLRU_DEVICE void rows_gates(const f32x16& ua, const f32x16& ux, const float (&xv)[16], float sp, float nba, float nbx,
                              unsigned resets, unsigned pads, int at, float* a, float* z) {
@@ -32,18 +36,21 @@ RGLRU_DEVICE void rows_gates(const f32x16& ua, const f32x16& ux, const float (&x
       unsigned u = __builtin_bit_cast(unsigned, l2);
       u = (u & ~m_reset) | (__builtin_bit_cast(unsigned, kResetLog2) & m_reset);
       l2 = __builtin_bit_cast(float, u & ~m_pad);
+    } else if (v == 0) {
+      l2 = resets & 1u ? kResetLog2 : l2;
     }
     const GateOut o = gate_outputs<false>(r, i, xv[v], l2);
     a[v] = o.a; z[v] = o.z;
   }
 }
 
-template <int NKG, bool PAD>
-__global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(FusedArgs p) {
+// FLAGS: the call has an array of them; else only a sequence's first token may carry one (p.first_reset).
+template <int NKG, bool PAD, bool FLAGS, int MT>
+__global__ __launch_bounds__(kThreads, MT == 1 ? 3 : 2) void fwd_rows_kernel(FusedArgs p) {
   typedef __bf16 IO;
   typedef Io<IO> Tr;
   typedef Tr::Frag Frag;
-  constexpr int MT = rows_mt(NKG), TR = 32 * MT, EL = 16 * MT;
+  constexpr int TR = 32 * MT, EL = 16 * MT;
   constexpr int KC = kPackedWidth, LDSROW = KC + Tr::HW;
   constexpr int VPR = KC / Tr::HW, RP = kThreads / VPR, NV = TR / RP;      // a pass of the workgroup loads RP rows
   __shared__ __attribute__((aligned(16))) IO lds[2][TR * LDSROW];
@@ -70,7 +77,7 @@ __global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(Fused
   IO* const x_at = &lds[0][0] + x_row * LDSROW + x_cv * Tr::HW;
   const rsrc_t rh0 = make_rsrc(p.h0, p.h0 ? (unsigned)p.B * uW * 4u : 0u), rhl = make_rsrc(p.h_last, p.h_last ? (unsigned)p.B * uW * 4u : 0u);
   Frag pre[NV];
-  unsigned pre_fl;
+  unsigned pre_fl = 0;
   float pre_h0;
   // a tile past the last sequence keeps valid addresses but an empty extent: nothing is fetched
   auto issue = [&](int b, int c) {
@@ -82,8 +89,10 @@ __global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(Fused
     asm volatile("" : "+v"(xo));
 #pragma unroll
     for (int i = 0; i < NV; ++i) pre[i] = buf_load_frag<Frag>(rx, xo + (unsigned)(i * RP) * row_bytes);
-    const rsrc_t rf = make_rsrc(p.flags + row0, p.flags ? (unsigned)rows : 0u);
-    pre_fl = (unsigned)__builtin_amdgcn_raw_buffer_load_b8(rf, (unsigned)(w.lane & (TR - 1)), 0, 0);
+    if constexpr (FLAGS) {
+      const rsrc_t rf = make_rsrc(p.flags + row0, (unsigned)rows);
+      pre_fl = (unsigned)__builtin_amdgcn_raw_buffer_load_b8(rf, (unsigned)(w.lane & (TR - 1)), 0, 0);
+    }
     pre_h0 = BufIo<float>::load(rh0, live && c == 0 ? ((unsigned)b * uW + ch) * 4u : kOutOfRange, 0u);
   };
   int b = w.wg_in_unit, c = 0;
@@ -103,7 +112,8 @@ __global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(Fused
 #pragma unroll
     for (int i = 0; i < NV; ++i) *reinterpret_cast<Frag*>(x_at + buf * (TR * LDSROW) + i * RP * LDSROW) = pre[i];
     // one bit per token; tokens past the end read as padding
-    unsigned long long resets = __ballot(pre_fl & RGLRU_FLAG_RESET), pads = __ballot(pre_fl & RGLRU_FLAG_INACTIVE);
+    unsigned long long resets = 0ull, pads = 0ull;
+    if constexpr (FLAGS) { resets = __ballot(pre_fl & RGLRU_FLAG_RESET); pads = __ballot(pre_fl & RGLRU_FLAG_INACTIVE); }
     if (p.T - t0 < TR) pads |= ~0ull << (p.T - t0);
     if (p.first_reset && c == 0) resets |= 1ull;
     if (c == 0) h_in = pre_h0;
@@ -119,8 +129,20 @@ __global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(Fused
       f32x16 ua, ux;
       float xv[16];
       gate_mfma_held<IO, MT, NKG, KC>(tile, hw, mt, w.slab, w.r, hf, 0.0f, 0.0f, ua, ux, xv, NKG >= 8 ? 0 : w.kb);
-      if (plain) rows_gates<false>(ua, ux, xv, sp, nba, nbx, 0u, 0u, 0, a + 16 * mt, z + 16 * mt);
+      if (!FLAGS) rows_gates<false>(ua, ux, xv, sp, nba, nbx, mt == 0 ? my_resets : 0u, 0u, 0, a + 16 * mt, z + 16 * mt);
+      else if (plain) rows_gates<false>(ua, ux, xv, sp, nba, nbx, 0u, 0u, 0, a + 16 * mt, z + 16 * mt);
       else rows_gates<true>(ua, ux, xv, sp, nba, nbx, my_resets, my_pads, 16 * mt, a + 16 * mt, z + 16 * mt);
+    }
+    if constexpr (!FLAGS) {
+      // tokens past the end leave the state alone
+      if (p.T - t0 < TR) {
+#pragma unroll
+        for (int e = 0; e < EL; ++e) {
+          const bool past = (my_pads >> e) & 1u;
+          a[e] = past ? 1.0f : a[e];
+          z[e] = past ? 0.0f : z[e];
+        }
+      }
     }
     // the carry is known, so the lower half-wave's run is walked for its end, then both for their states
     float h = h_in;
@@ -150,17 +172,21 @@ __global__ __launch_bounds__(kThreads, rows_occ(NKG)) void fwd_rows_kernel(Fused
   }
 }
 
-int fwd_rows_tile(int nkg) { return 32 * rows_mt(nkg); }
-int fwd_rows_per_cu(int nkg) { return rows_occ(nkg); }
+int fwd_rows_tile(int nkg, bool flags, int64_t workgroups) { return rows_long_tiles(nkg, flags, workgroups) ? 64 : 32; }
+int fwd_rows_per_cu(int nkg, bool flags) { return rows_occ(nkg, flags); }
 
 int launch_fwd_rows(const FusedArgs& a, int nkg, bool pad, hipStream_t s) {
   const dim3 grid((unsigned)(a.wg_per_unit * a.units));
-#define RGLRU_ROWS_CASE(N)                                                                                             \
-  if (nkg == N) {                                                                                                      \
-    if (pad) hipLaunchKernelGGL((fwd_rows_kernel<N, true>), grid, dim3(kThreads), 0, s, a);                            \
-    else hipLaunchKernelGGL((fwd_rows_kernel<N, false>), grid, dim3(kThreads), 0, s, a);                               \
+  const bool flags = a.flags != nullptr;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, s, a); };
+#define RGLRU_ROWS_CASE(N, F, MT) pad ? launch(fwd_rows_kernel<N, true, F, MT>) : launch(fwd_rows_kernel<N, false, F, MT>)
+  if (nkg == 2) flags ? (RGLRU_ROWS_CASE(2, true, 1)) : (RGLRU_ROWS_CASE(2, false, 1));
+  else if (nkg == 4) flags ? (RGLRU_ROWS_CASE(4, true, 1)) : (RGLRU_ROWS_CASE(4, false, 1));
+  else {
+    const bool long_tiles = rows_long_tiles(nkg, flags, (int64_t)a.wg_per_unit * a.units);
+    if (nkg == 6) flags ? (RGLRU_ROWS_CASE(6, true, 2)) : long_tiles ? (RGLRU_ROWS_CASE(6, false, 2)) : (RGLRU_ROWS_CASE(6, false, 1));
+    else flags ? (RGLRU_ROWS_CASE(8, true, 2)) : long_tiles ? (RGLRU_ROWS_CASE(8, false, 2)) : (RGLRU_ROWS_CASE(8, false, 1));
   }
-  RGLRU_ROWS_CASE(8) RGLRU_ROWS_CASE(6) RGLRU_ROWS_CASE(4) RGLRU_ROWS_CASE(2)
 #undef RGLRU_ROWS_CASE
   return check_launch("fwd");
 }

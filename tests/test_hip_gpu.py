@@ -1098,6 +1098,37 @@ def test_forward_of_batches_that_fill_the_chip_with_sequences(bw, nb, B, owned, 
         assert err < BF16_TOL, (name, err)
 
 
+# without flags, on 256 compute units: two rounds (64-token tiles), three, a workgroup with two sequences, one round of short sequences, several
+# units, packed and padded blocks; the batches of the last line leave too much of a round empty
+@pytest.mark.parametrize("bw,nb,B,T,owned", [(128, 1, 512, 300, True), (128, 1, 768, 289, True), (128, 1, 900, 257, True), (128, 1, 250, 129, True),
+                                             (128, 3, 220, 320, True), (96, 1, 700, 161, True), (40, 2, 600, 159, True), (64, 3, 230, 288, True),
+                                             (128, 1, 256, 300, False), (64, 1, 330, 288, False), (128, 1, 516, 272, False)])
+@pytest.mark.parametrize("first_reset", [False, True])
+def test_forward_without_flags_of_batches_that_fill_rounds(bw, nb, B, T, owned, first_reset):
+    """The variant of the whole-sequence forward without flags, either side of its line: ragged tiles (tokens past the end leave the state
+    alone) and a document start at token 0 only, which the backward kernels take from the same checkpoints."""
+    from griffin_amd import _lib, hip_rglru, set_chain_forward
+
+    W = bw * nb
+    _say("sequences per workgroup, no flags", bw, nb, B, T, first_reset)
+    case = orc.make_case(B, T, W, nb, seed=bw + T, h0_std=0.5, bias_std=0.5)
+    reset = (torch.arange(T) == 0).expand(B, T) if first_reset else None
+    leaves = [case[k].to(torch.bfloat16).cuda().requires_grad_(True) for k in PARAMS]
+    was = set_chain_forward(1)
+    try:
+        assert _lib.load().rglru_hip_forward_owns_sequences(B, T, W, nb, _lib.RGLRU_BF16, 2 if first_reset else 0) == owned
+        y, h_last = hip_rglru(*leaves, 8.0, case["h0"].cuda(), first_token_reset=first_reset)
+        grads = torch.autograd.grad(y, leaves, case["dy"].to(torch.bfloat16).cuda())
+        torch.cuda.synchronize()
+    finally:
+        set_chain_forward(was)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(g.float(), rgrads[name]) for name, g in zip(PARAMS, grads)})
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
+
+
 @pytest.mark.parametrize("B,W,once,stream", [(250, 260, False, False), (251, 260, True, False), (1016, 256, True, False), (1018, 256, True, True)])
 def test_scan_op_gradients_below_and_above_the_cache(B, W, once, stream):
     """From 32 MB a tensor on the inputs that are read once bypass the caches, and from 256 MB of gradients on these are stored past
