@@ -21,7 +21,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_NAME = "librglru_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 SOURCES = ["rglru_scan.hip", "rglru_fused.hip", "rglru_fwd_rows.hip", "rglru_fused_bwd.hip", "rglru_decode.hip", "rglru_decode_linear.hip",
-           "rglru_gate_gemm.hip", "rglru_linear.hip", "rglru_block_ops.hip", "rglru_tokens.hip"]
+           "rglru_gate_gemm.hip", "rglru_linear.hip", "rglru_linear16.hip", "rglru_block_ops.hip", "rglru_tokens.hip"]
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 NATIVE_SOURCE = "torch_ops.cpp"
 ARCH = "gfx950"

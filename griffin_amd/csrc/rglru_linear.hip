@@ -8,14 +8,15 @@
 //
 // Why not the BLAS library alone: a call of it costs the host 17 us, seven calls of it are a third of the host time of a
 // training step of the block, which is what bounds such a step up to several thousand tokens; and it takes no row mask and
-// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 52 us against 65 us, 795 TFLOP/s,
-// here; the split weight gradient of the same 52 us against 91 us), so callers choose by the size of the product.
+// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 52 us against 63 us), so callers choose by the
+// size of the product.
 //
-// A workgroup of four waves owns a BM x BN tile of C; K is walked in slices of 128 bytes, one barrier a slice.  Where both operands
+// Here: fp32, and the forward in bf16 (the gradients in bf16: rglru_linear16.hip).  A workgroup of four waves owns a BM x BN tile of C; K is
+// walked in slices of 128 bytes, one barrier a slice.  Where both operands
 // lie with their contraction index contiguous (forward) a slice goes from memory to LDS directly (DirectTile), one slice ahead
 // (128 x 128) or two (64 x 64).  Otherwise it goes through registers (requested one slice ahead) into one of two LDS buffers: an
 // operand with its contraction index contiguous is read back as 16-byte rows (row stride 144 bytes: no bank conflicts); one that
-// lies the other way round is read with the transposing LDS loads (16-bit types), or element by element (fp32).
+// lies the other way round is read element by element.
 // Edges of M, N and K are masked through the offsets of buffer loads, so any size works as long as rows are whole 16-byte
 // vectors.
 // What bounds it, forward: with slices through registers the LDS writes (13.8 clocks a KB on a compute unit, reads 4.3) were most
@@ -36,22 +37,9 @@
 #include "rglru_device.h"
 #include "rglru_host.h"
 #include "rglru_layout.h"
+#include "rglru_linear.h"
 
 namespace rglru {
-
-struct LinearArgs {
-  // `batch` equal problem sets side by side, operands a_step, b_step and c_step elements on: the gate blocks of the RG-LRU
-  long long a_step, b_step, c_step;
-  int batch, accumulate;             // accumulate: c += product, rounded once
-  int partial_ld;                    // partial: [split][batch][problem][partial_ld][partial_ld] where set, else [split][problem][M][N]
-  const void* a[2]; const void* b[2]; const void* bias[2]; void* c[2];
-  const unsigned char* active;       // one byte per token, or null: inactive rows of the result are zero (weight gradient: rows of A count as zero)
-  float* partial;                    // [split][problem][M][N] instead of c where the contraction is split
-  float* colsum;                     // weight gradient: [split][problem][M] column sums of A, or null
-  long long lda, ldb, ldc;           // elements between rows in memory
-  int M, N, K;                       // of one problem; K of one segment (input gradient)
-  int tiles_m, tiles_n, problems, segments, splits, k_per_split, total;
-};
 
 // Tile of one operand: ROWS rows of the result's index (m or n) x BK of the contraction index.  T: in memory (and in LDS) a row
 // is one contraction index, else one result index.
@@ -62,9 +50,8 @@ struct OperandTile {
   typedef typename Tr::Frag Frag;
   static constexpr int HW = Tr::HW, BK = 8 * HW;                              // 128 bytes
   static constexpr int kLines = T ? BK : ROWS, kLineElems = T ? ROWS : BK;    // memory rows of the tile, elements of each
-  // 16-bit transposed rows: 64 bytes more than a multiple of 128, so that the four rows of a transposing read fall on
-  // different banks; fp32: the two halves of a wave read rows four apart, half the banks away
-  static constexpr int kStride = T ? (sizeof(IO) == 2 ? ROWS + 32 : ROWS + 8) : BK + HW;
+  // transposed: the two halves of a wave read rows four apart, half the banks away
+  static constexpr int kStride = T ? ROWS + 8 : BK + HW;
   static constexpr int kElems = kLines * kStride;
   static constexpr int VPR = kLineElems / HW, NV = kLines * VPR / THREADS;
   static_assert(kLines * VPR % THREADS == 0, "whole vectors per thread");
@@ -116,9 +103,8 @@ struct OperandTile {
     const int r = lane & 31, hf = lane >> 5;
     if constexpr (!T) {
       return *reinterpret_cast<const Frag*>(lds + (first + r) * kStride + kg * Tr::KG + hf * HW);
-    } else if constexpr (sizeof(IO) == 2) {
-      return lds_transposed_frag(lds, kStride, kg * Tr::KG, first, lane);
     } else {
+      static_assert(sizeof(IO) == 4, "16-bit types: rglru_linear16.hip");
       Frag f;
 #pragma unroll
       for (int i = 0; i < HW; ++i) f[i] = lds[(kg * Tr::KG + hf * HW + i) * kStride + first + r];
@@ -147,7 +133,7 @@ struct DirectTile {
 #pragma unroll
     for (unsigned kg = 0; kg < 4; ++kg) place[kg] = r * 128u + (((2u * kg + hf) ^ ((r >> 1) & 7u)) * 16u);
   }
-  // Slice at `base` with k_left contraction indices into LDS at byte address `lds` (below 64 KB: M0 holds 16 bits of it); rows past
+  // Slice at `base` with k_left contraction indices into LDS at byte address `lds`; rows past
   // `limit` and indices past k_left become zeros, as masked loads do everywhere.  The compiler neither counts these loads nor knows
   // their hazards: the caller waits for them, and the descriptor has its wait states here.
   RGLRU_DEVICE void request(const IO* base, long long ld, int k_left, int limit, unsigned lds, int wave) const {
@@ -171,13 +157,6 @@ struct DirectTile {
     return *reinterpret_cast<const Frag*>(lds + first * 128 + place[kg]);
   }
 };
-
-// Four consecutive elements (N is a multiple of a 16-byte vector, so they lie wholly inside or outside a row).
-template <typename IO> RGLRU_DEVICE auto buf_load_four(rsrc_t r, unsigned voff) {
-  typedef IO io4 __attribute__((ext_vector_type(4)));
-  if constexpr (sizeof(IO) == 2) return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
-  else return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-}
 
 // DIRECT: both operands' rows are result indices and go to LDS directly (DirectTile).
 template <typename IO, bool TA, bool TB, int BM, int BN, bool DIRECT = !TA && !TB>
@@ -406,7 +385,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     float* part = p.partial + ((((long long)split * p.batch + item) * p.problems + problem) * rows + m0) * ld + n0;
     const rsrc_t rc = make_rsrc(part, (unsigned)((long long)(m_left < BM ? m_left : BM) * ld) * 4u);
     // through LDS like the result: stored from the accumulators, a row of the wave's tile is 32 bytes an instruction (two weight
-    // gradients of 2048 x 1024 x 768: 45 us that way, 42 element by element, 41 like this)
+    // gradients of 2048 x 1024 x 768, when bf16 ran here: 45 us that way, 42 element by element, 41 like this)
     constexpr int kRow = BN / 2 + 4;
     static_assert(4 * (BM / 2) * kRow * 4 <= (int)sizeof(lds), "the fp32 tile fits where the slices were");
     float* stage = reinterpret_cast<float*>(lds) + wave * (BM / 2) * kRow;
@@ -432,7 +411,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     return;
   }
   // result in the storage type: through LDS (the slices have been read), then 16-byte vectors of rows, written through the L2s
-  // (kWriteThrough).  Kernel times: 2331 x 2 x 1024 x 768 in bf16 16.6 -> 15.8 us, weight gradient of 2048 x 2 x 1024 x 768 41.6 -> 39.6, fp32
+  // (kWriteThrough).  Kernel times: 2331 x 2 x 1024 x 768 in bf16 16.6 -> 15.8 us, fp32
   // gate gradients of B4 T1024 W1024 37.5 -> 34.8; the largest tried, 134 MB, 183 -> 181.
   IO* stage = lds + wave * (BM / 2) * kStageRow;
 #pragma unroll
@@ -462,39 +441,72 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   }
 }
 
-// How a product is cut up: tiles of 128 x 128, or 64 x 64 (four times the workgroups at half the reuse).
-// Forward and input gradients: time goes in steps of one tile a compute unit, and steps of large tiles are four times as coarse.
+// How a product is cut up: tiles of 64 x 64, 128 x 128 (four times the work at half the reads) or, in bf16 gradients, 256 x 256.
+// Forward products: time goes in steps of one tile a compute unit, and steps of large tiles are four times as coarse.
 // In bf16 three small tiles on a compute unit take about as long as one large one, so the line lies where there are more than three.
-// On 256 compute units, us, small : large (small tiles in brackets), two problems or segments unless said:
-//   forward  1527 x 1024 x 768 (768) 11.2 : 10.6, 1655 (832) 14.3 : 11.0, 2331 16.5 : 14.3;  2039 x 768 x 1024 (768) 12.6 : 12.7, 2167 (816) 17.1 : 13.6;
-//            1883 x 768 x 1024 (720) 12.3 : 14.6;  one of 4087 x 768 x 1024 (768) 12.7 : 12.6, 4215 (792) 16.6 : 12.7;  503 x 2560 x 2560 (640) 37.4 :
-//            37.9, 631 (800) 47.0 : 38.1;  beyond, 4087 x 1024 x 768 (2048) 26.7 : 18.0, 5495 x 768 x 1024 (2064) 32.7 : 32.7
-//   input    3063 x 1024 x 768 (768) 22.1 : 25.0, 3191 (800) 29.1 : 25.0;  4087 x 768 x 1024 (768) 27.7 : 31.5, 4215 (792) 36.4 : 31.6
+// On 256 compute units, us, small : large (small tiles in brackets), two problems unless said:
+//   1527 x 1024 x 768 (768) 11.2 : 10.6, 1655 (832) 14.3 : 11.0, 2331 16.5 : 14.3;  2039 x 768 x 1024 (768) 12.6 : 12.7, 2167 (816) 17.1 : 13.6;
+//   1883 x 768 x 1024 (720) 12.3 : 14.6;  one of 4087 x 768 x 1024 (768) 12.7 : 12.6, 4215 (792) 16.6 : 12.7;  503 x 2560 x 2560 (640) 37.4 :
+//   37.9, 631 (800) 47.0 : 38.1;  beyond, 4087 x 1024 x 768 (2048) 26.7 : 18.0, 5495 x 768 x 1024 (2064) 32.7 : 32.7
 // fp32 is bound by its MFMAs, and a small tile takes 1 / 4 of a large one and 6 % more, so the number of steps decides (M x 256 x 256, two
 // problems; steps small : large x 4):  8183 (4 : 4) 22.1 : 22.2, 8439 (5 : 8) 26.3 : 36.0, 14071 (7 : 8) 35.8 : 36.9, 15991 (8 : 8) 40.3 : 37.8, 16631
 // (9 : 12) 44.2 : 54.9, 24567 (12 : 12) 58.9 : 56.3;  input gradient 8183 (2 : 4) 24.6 : 40.8, 16375 (4 : 4)
 // 39.9 : 42.5.
-// A weight gradient contracts over the tokens, so its tiles are few and its contraction long: it is split over workgroups until there
-// are about two to a compute unit, at least four slices each and at most eight splits (every split costs a pass over the result in
-// fp32).  With that pass, us, small : large (splits), bf16, 2331 tokens unless said: 768 x 1024 whole 31.4, 23.2 (3) : 25.0 (8), 4096 tokens 32.0 :
-// 28.4, 8192 52.6 : 38.0; 2 x 256 x 256 31.4 whole, 15.0 (4), 12.0 (8), 13.9 (9), always small; 2560 x 2560 88.3 (1) : 74.3 (2).  Two of 1024 x 768
-// are large from 1024 tokens on and would be faster in small tiles up to 4096: 30.0 (2) : 37.5 (6), 4096 tokens 42.4 : 45.3, 8192 74.4 : 71.3; in
-// fp32 83 : 108.
-struct LinearPlan { bool large; int splits; };
-static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
+// A weight gradient contracts over the tokens, so its tiles are few and its contraction long: it is split over workgroups (every split
+// costs a pass over the result in fp32).  In fp32 until there are about two to a compute unit, at least four slices each and at most
+// eight splits (two of 1024 x 768 at 2331 tokens 83 us in small tiles, 108 in large ones).
+struct TileCost { int edge; unsigned per_cu; double start, slice[3]; };
+// Gradients in bf16: the cheapest by a model of the time in us.  A workgroup of a tile size takes `start` and `slice[n - 1]` for 64 contraction
+// indices with n of them on a compute unit; the units run their tiles in rounds of `per_cu`.  Constants from 64, 128 and 256 on
+// 1000 to 16384 tokens of 768 and 1024 channels.  What it picks, us, sizes 64 : 128 : 256 (* taken; splits behind the slash):
+//   input, two segments of 1024 into 768   2331 *17.9 : 23.2 : 48.8, 4096 25.1 : *23.6, 8704 50.2 : *32.8 : 52.7, 16384 84 : *55.3 : 57.7
+//   input, 768 into 1024   2331 *11.1 : 11.3, 6000 20.6 : *15.9 : 23.2, 8704 28.0 : 25.1 : *24.8, 16384 46.4 : 40.0 : *29.3
+//   weight, two of 1024 x 768   1000 *10.4/2 : 10.5/2, 2331 18.1/2 : *17.0/3 : 19.0/8, 8704 51.7/2 : *39.8/5 : 36.1/10 (and ten sets to add up),
+//          16384 91/6 : 68.1/5 : *57.0/10
+//   weight, 768 x 1024   1000 8.1/4 : 8.3/5, 2331 11.4/4 : *10.7/5, 8704 28.2/4 : *26.1/5 : 30.8/10, 16384 49/4 : *36.6/10 : 36.5/16
+// The kernels they replace, whose slices went through registers: 40.2, 29.8, 64.5 and 31.8 us at 8704 tokens, in the order above.
+static LinearPlan linear16_plan(bool weight, int64_t M, int64_t N, int64_t K, int problems, int segments) {
+  static const TileCost input[] = {{64, 3, 2.5, {0.36, 0.47, 0.69}}, {128, 2, 4.5, {0.58, 0.87, 0.0}}, {256, 1, 10.0, {1.43, 0.0, 0.0}}};
+  static const TileCost weights[] = {{64, 3, 3.0, {0.39, 0.52, 0.71}}, {128, 2, 6.0, {0.70, 1.18, 0.0}}, {256, 1, 12.0, {1.74, 0.0, 0.0}}};
+  static const unsigned some[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24};
+  const unsigned units = (unsigned)num_compute_units(), slices = (unsigned)((K + 63) / 64);
+  LinearPlan best = {64, 1};
+  double least = 1e30;
+  for (const TileCost& c : weight ? weights : input) {
+    if (c.edge == 256 && N >= (1 << 20)) continue;           // 256 lines of fp32 within a lane's reach
+    const double all = (double)((M + c.edge - 1) / c.edge) * (double)((N + c.edge - 1) / c.edge) * problems;
+    if (all > 1e6) {                                         // far more tiles than units: by their throughput
+      const double t = all / units * c.slice[c.per_cu - 1] / c.per_cu * slices * segments;
+      if (t < least) { least = t; best = {c.edge, 1}; }
+      continue;
+    }
+    const unsigned tiles = (unsigned)all;
+    for (unsigned splits : some) {
+      if (splits > 1 && (!weight || splits * 4 > slices)) break;
+      const unsigned each = (tiles * splits + units - 1) / units, rounds = each / c.per_cu, rest = each - rounds * c.per_cu;
+      const double part = (double)((slices + splits - 1) / splits) * segments;
+      double t = rounds * (c.start + c.slice[c.per_cu - 1] * part) + (rest ? c.start + c.slice[rest - 1] * part : 0.0);
+      if (splits > 1) t += (double)splits * problems * M * N * (4.0 / 4.5e6);        // the sets are read again
+      if (t < least) { least = t; best = {c.edge, (int)splits}; }
+    }
+  }
+  return best;
+}
+static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int problems, int segments, int dtype) {
+  if (dtype == RGLRU_BF16 && kind != RGLRU_LINEAR_FORWARD) return linear16_plan(kind == RGLRU_LINEAR_WEIGHT_GRAD, M, N, K, problems, segments);
   auto tiles = [&](int64_t edge) { return ((M + edge - 1) / edge) * ((N + edge - 1) / edge) * problems; };
   const int64_t units = num_compute_units();
   auto steps = [&](int64_t edge) { return (tiles(edge) + units - 1) / units; };
-  LinearPlan p = {dtype == RGLRU_BF16 ? tiles(64) > 3 * units : tiles(128) > units && 106 * steps(64) >= 400 * steps(128), 1};
+  LinearPlan p = {(dtype == RGLRU_BF16 ? tiles(64) > 3 * units : tiles(128) > units && 106 * steps(64) >= 400 * steps(128)) ? 128 : 64, 1};
   if (kind != RGLRU_LINEAR_WEIGHT_GRAD) return p;
-  const int64_t slices = (K + (dtype == RGLRU_BF16 ? 63 : 31)) / (dtype == RGLRU_BF16 ? 64 : 32);
+  const int64_t slices = (K + 31) / 32;
   auto splits = [&](int64_t t) {
     int64_t s = (2 * units + t - 1) / t;
     if (s > slices / 4) s = slices / 4;
     return s > 8 ? (int64_t)8 : s < 1 ? (int64_t)1 : s;
   };
-  p.large = tiles(128) * splits(tiles(128)) >= units;
-  p.splits = (int)splits(tiles(p.large ? 128 : 64));
+  p.edge = tiles(128) * splits(tiles(128)) >= units ? 128 : 64;
+  p.splits = (int)splits(tiles(p.edge));
   return p;
 }
 
@@ -509,15 +521,14 @@ static void linear_launch(LinearArgs& a, bool large, hipStream_t s) {
   else hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 64, 64>), grid, dim3(kLinearThreads), 0, s, a);
 }
 
-static void linear_launch(LinearArgs& a, int kind, bool large, int dtype, hipStream_t s) {
+static void linear_launch(LinearArgs& a, int kind, int edge, int dtype, hipStream_t s) {
   if (dtype == RGLRU_BF16) {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, large, s);
-    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<__bf16, false, true>(a, large, s);
-    else linear_launch<__bf16, true, true>(a, large, s);
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, edge > 64, s);
+    else linear16_launch(a, kind, edge, s);
   } else {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, large, s);
-    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, large, s);
-    else linear_launch<float, true, true>(a, large, s);
+    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, edge > 64, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, edge > 64, s);
+    else linear_launch<float, true, true>(a, edge > 64, s);
   }
 }
 
@@ -544,7 +555,7 @@ int gate_pre_product(const void* x, const void* wg, void* pre, long long N, cons
   a.lda = g.W; a.ldb = g.bwp; a.ldc = 2 * g.bw; a.a_step = g.bw; a.b_step = g.bwp * g.bwp; a.c_step = N * 2 * g.bw;
   a.batch = (int)g.nb; a.problems = 2; a.segments = 1; a.splits = 1;
   a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
-  linear_launch(a, RGLRU_LINEAR_FORWARD, batch_large(g, N, 2), RGLRU_BF16, s);
+  linear_launch(a, RGLRU_LINEAR_FORWARD, batch_large(g, N, 2) ? 128 : 64, RGLRU_BF16, s);
   return check_launch("gate pre-activations");
 }
 
@@ -557,7 +568,7 @@ int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long lo
   a.lda = du_ld; a.ldb = g.bwp; a.ldc = g.W; a.a_step = du_blk; a.b_step = g.bwp * g.bwp; a.c_step = g.bw;
   a.batch = (int)g.nb; a.problems = 1; a.segments = 2; a.splits = 1; a.accumulate = 1;
   a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
-  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, batch_large(g, N, 1), dtype, s);
+  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, batch_large(g, N, 1) ? 128 : 64, dtype, s);
   return check_launch("gate input gradient");
 }
 
@@ -571,7 +582,7 @@ int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long l
   a.M = a.N = (int)g.bw; a.K = (int)N;
   const long long bk = dtype == RGLRU_BF16 ? 64 : 32;
   a.k_per_split = (int)(((N + splits - 1) / splits + bk - 1) / bk * bk);
-  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, batch_large(g, g.bw, 2 * splits), dtype, s);
+  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, batch_large(g, g.bw, 2 * splits) ? 128 : 64, dtype, s);
   return check_launch("gate weight gradients");
 }
 
@@ -583,7 +594,7 @@ extern "C" {
 
 int64_t rglru_hip_linear_splits(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return linear_plan(kind, M, N, K, problems, dtype).splits;
+  return linear_plan(kind, M, N, K, problems, 1, dtype).splits;
 }
 
 int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
@@ -598,7 +609,8 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
   a.batch = 1; a.active = active; a.colsum = colsum; a.lda = lda; a.ldb = ldb; a.ldc = ldc;
   a.problems = kind == RGLRU_LINEAR_FORWARD ? (b1 ? 2 : 1) : kind == RGLRU_LINEAR_WEIGHT_GRAD ? (a1 ? 2 : 1) : 1;
   a.segments = kind == RGLRU_LINEAR_INPUT_GRAD && a1 ? 2 : 1;
-  const LinearPlan plan = linear_plan(kind, M, N, K, a.problems, dtype);
+  LinearPlan plan = linear_plan(kind, M, N, K, a.problems, a.segments, dtype);
+  if (plan.edge == 256 && (lda >= (1 << 21) || ldc >= (1 << 21))) plan.edge = 128;        // 256 lines within a lane's reach
   a.splits = plan.splits;
   if (plan.splits > 1) a.partial = partial;
   if (!a0 || !b0 || (a.segments == 2 && !b1) || (plan.splits > 1 ? !partial : (!c0 || (a.problems == 2 && !c1)))) return fail(RGLRU_E_ARG, "linear: null pointer");
@@ -617,7 +629,7 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
   const int64_t bk = dtype == RGLRU_BF16 ? 64 : 32;
   a.k_per_split = (int)(((K + a.splits - 1) / a.splits + bk - 1) / bk * bk);
   hipStream_t s = (hipStream_t)stream;
-  linear_launch(a, kind, plan.large, dtype, s);
+  linear_launch(a, kind, plan.edge, dtype, s);
   return check_launch("linear");
 }
 

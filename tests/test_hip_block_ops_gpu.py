@@ -1080,6 +1080,59 @@ def test_linear_products_match_fp64(M, N, K, dtype):
         compare(sums.double().sum(0).view(-1), live.sum(0), "column sums")
 
 
+# On 256 compute units, tiles of 64, 128 and 256: input gradients of one and two segments, weight gradients whole and split (the last split
+# short); no edge is a whole tile, slice or vector of them
+@pytest.mark.parametrize("kind,pair,M,N,K", [(1, 1, 700, 1016, 776), (1, 2, 8200, 776, 1000), (1, 1, 16300, 1016, 776), (1, 2, 33000, 1016, 200),
+                                             (2, 1, 1016, 776, 130), (2, 2, 1016, 776, 2331), (2, 1, 776, 1016, 9001), (2, 2, 1016, 776, 16381), (2, 2, 264, 136, 20007)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_gradient_products_in_every_tile_read_only_their_operands(kind, pair, M, N, K, masked):
+    """bf16 gradients against fp64, with operands inside larger tensors of NaN; column sums and masked rows."""
+    from griffin_amd import _lib
+
+    lib = _lib.load()
+    _say("gradient products", kind, pair, M, N, K, masked)
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    rows_a, cols_a = (M, K) if kind == 1 else (K, M)
+    a = torch.full((rows_a + 2, 2 * cols_a + 16), float("nan"), dtype=torch.bfloat16, device="cuda")
+    b = torch.full((pair if kind == 1 else 1, K + 2, N + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+    a[1:-1, 8:-8] = torch.randn(rows_a, 2 * cols_a, generator=gen, device="cuda")
+    b[:, 1:-1, 8:-16] = torch.randn(b.size(0), K, N, generator=gen, device="cuda")
+    if pair == 1:
+        a[1:-1, 8 + cols_a:] = float("nan")
+    keep = torch.rand(rows_a, generator=gen, device="cuda") < 0.6 if masked else torch.ones(rows_a, dtype=torch.bool, device="cuda")
+    active = keep.to(torch.uint8) if masked else None
+    at = lambda t: None if t is None else t.data_ptr()
+    first, second = a[1, 8:], a[1, 8 + cols_a:] if pair == 2 else None
+    ld = a.size(1)
+    stream = torch.cuda.current_stream().cuda_stream
+    halves = [a[1:-1, 8 + i * cols_a:8 + (i + 1) * cols_a].double() for i in range(pair)]
+    if kind == 1:
+        c = torch.full((M + 2, N + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+        _lib.check(lib.rglru_hip_linear(1, at(first), at(second), ld, at(b[0, 1, 8:]), at(b[1, 1, 8:]) if pair == 2 else None, b.size(2), None, None,
+                                        at(active), at(c[1, 8:]), None, c.size(1), None, None, M, N, K, _lib.RGLRU_BF16, stream), "linear")
+        torch.cuda.synchronize()
+        want = sum(h @ b[i, 1:-1, 8:-16].double() for i, h in enumerate(halves)) * keep[:, None]
+        size = sum(h.abs() @ b[i, 1:-1, 8:-16].double().abs() for i, h in enumerate(halves))
+        got = c[1:-1, 8:-16].double()
+        # rounding of the result, then 2 K additions in fp32
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + (pair * K + 2) * 2.0 ** -24 * size).all()
+        assert torch.isnan(c[0]).all() and torch.isnan(c[-1]).all() and torch.isnan(c[:, :8]).all() and torch.isnan(c[:, -16:]).all()
+        return
+    splits = lib.rglru_hip_linear_splits(2, M, N, K, pair, _lib.RGLRU_BF16)
+    dw = torch.full((splits, pair, M, N), float("nan"), device="cuda", dtype=torch.float32 if splits > 1 else torch.bfloat16)
+    sums = torch.full((splits, pair, M), float("nan"), device="cuda")
+    _lib.check(lib.rglru_hip_linear(2, at(first), at(second), ld, at(b[0, 1, 8:]), None, b.size(2), None, None, at(active), at(dw[0, 0]),
+                                    at(dw[0, 1]) if pair == 2 else None, N, at(dw) if splits > 1 else None, at(sums), M, N, K, _lib.RGLRU_BF16, stream), "linear")
+    torch.cuda.synchronize()
+    x = b[0, 1:-1, 8:-16].double()
+    for i, h in enumerate(halves):
+        live = h * keep[:, None]
+        want, size = live.t() @ x, live.abs().t() @ x.abs()
+        unit = 2.0 ** -8 if splits == 1 else 0.0
+        assert ((dw.double().sum(0)[i] - want).abs() <= unit * want.abs() + (K + 2) * 2.0 ** -24 * size).all()
+        assert ((sums.double().sum(0)[i] - live.sum(0)).abs() <= (K + 2) * 2.0 ** -24 * live.abs().sum(0)).all()
+
+
 @pytest.mark.parametrize("padded", [False, True])
 @pytest.mark.parametrize("B,T,D,W,nb", [(2, 1, 64, 96, 3), (3, 37, 72, 128, 2), (2, 333, 192, 256, 16), (2, 4097, 768, 1024, 16), (4, 2048, 1536, 2048, 16)])
 def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded):
