@@ -1367,20 +1367,24 @@ Tensor sum_sets(const Tensor& sets) {
 
 // Whether products of `macs` multiply-adds each (tokens x width x model width) run on the library's own kernels.  The BLAS
 // library is the faster one on long products (see rglru_linear.hip), but each call of it keeps the host for 17 us and a
-// training step of the block has seven.  The line lies where both ways take about equally long per layer in a stack of eight blocks,
-// alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
-// alone / with MLPs).  bf16, training 768 -> 1024: at 3.0e9 250 : 273 / 702 : 721, at 6.0e9 363 : 423 / 1067 : 1124, at 6.4e9 368 : 344 / 1069 : 1036 (8192
-// tokens: the BLAS library has its best tiles at powers of two), at 8.0e9 445 : 506 / 1269 : 1338, at 1.3e10 620 : 527 / 1821 : 1707;  2560 -> 2560 at
-// 5.0e9 373 : 404 / 987 : 992, at 6.0e9 429 : 459 / 1121 : 1100, at 8.0e9 478 : 466 / 1234 : 1183;  prefill 768 -> 1024 at 4.0e9 82 : 86 / 201 : 199, at 6.0e9
+// training step of the block has seven.  Without gradients and in fp32 the line lies where both ways take about equally long per layer in a
+// stack of eight blocks, alone or with an MLP of three products behind each (profiles/block_products_own_vs_blas_in_stacks.txt, us own : BLAS,
+// alone / with MLPs).  bf16, prefill 768 -> 1024: at 4.0e9 82 : 86 / 201 : 199, at 6.0e9
 // 96 : 102 / 281 : 287, at 8.0e9 116 : 117 / 325 : 336, at 1.3e10 163 : 149 / 453 : 442;  2560 at 6.0e9 126 : 135 / 306 : 303, at 6.7e9 141 : 127 / 327 : 311.  So
 // between 6e9 and 9e9 either way wins somewhere.  fp32, training 768 -> 1024: at 8e8 326 : 469 / 759 : 755, at 9e8 362 : 468 / 843 : 824, at 1.2e9
 // 430 : 463, at 1.6e9 484 : 452;  wide and short ones lose below the line: 2560 -> 2560 at 5.8e8 (88 tokens) 481 : 466 / 1004 : 865, prefill
 // 151 : 123.  Inside a captured graph host time is nothing: there the line lies where the kernels take equally long.
-bool own_products(double macs, at::ScalarType dtype) {
+// In a training step of the block in bf16, steps queued behind each other, us: gradients on the BLAS library : own, then the forward own as well.
+// 768 -> 1024 at 6.3e9 374 : 317 : 305, 7.9e9 453 : 385 : 377, 9.7e9 442 : 443 : 439, 1.02e10 603 : 475 : 471, 1.3e10 516 : - : 542;  2560 -> 2560 at 6.0e9 482 :
+// 401 : 340, 8.5e9 485 : 395 : 388, 1.18e10 541 : 460 : 474, 1.3e10 542 : - : 516;  1536 -> 2048 at 6.4e9 317 : 278 : 273, 7.5e9 346 : 318 : 331, 9.4e9 388 :
+// 371 : 387, 1.3e10 447 : - : 477.
+enum class Product { kInference, kTrainingForward, kGradient };
+bool own_products(double macs, at::ScalarType dtype, Product use = Product::kInference) {
   if (!known(dtype)) return false;
   const bool bf16 = dtype == at::kBFloat16;
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return macs < (bf16 ? 2e9 : 4e8);
-  return macs < (bf16 ? 6e9 : 9e8);
+  if (!bf16) return macs < 9e8;
+  return macs < (use == Product::kInference ? 6e9 : use == Product::kTrainingForward ? 9e9 : 1.2e10);
 }
 
 // Contiguous rows of whole 16-byte vectors, as rglru_hip_linear takes them.
@@ -1393,10 +1397,10 @@ bool vector_rows(const Tensor& t) {
 bool plain(const Tensor& t) { return !t.defined() || !t.key_set().has(c10::DispatchKey::Python); }
 
 // Whether the library takes y = x w^T + b (and its gradients) for these operands.
-bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b) {
+bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b, Product use = Product::kInference) {
   const auto dtype = x.scalar_type();
   return plain(x) && plain(w) && plain(b) && w.dim() == 2 && x.size(-1) == w.size(1) && on_device_of(x, w) && on_device_of(x, b) && w.scalar_type() == dtype && has(b, w.size(0)) && (!b.defined() || (b.scalar_type() == dtype && b.is_contiguous())) &&
-         x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype) && vector_rows(w) && vector_rows(x) &&
+         x.numel() > 0 && own_products(double(x.numel()) * w.size(0), dtype, use) && vector_rows(w) && vector_rows(x) &&
          (w.size(0) * x.element_size()) % 16 == 0 && !at::autocast::is_autocast_enabled(at::kCUDA);
 }
 
@@ -1406,6 +1410,9 @@ void linear_forward(const Tensor& x, const Tensor& w0, const Tensor& b0, const T
   check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, ptr(x), nullptr, K, ptr(w0), ptr(w1), K, ptr(b0), ptr(b1), bptr(active), y0, y1, N,
                          nullptr, nullptr, x.numel() / K, N, K, code_of(x.scalar_type()), stream_of(x)), "rglru_hip_linear");
 }
+
+// Sizes that rglru_hip_linear addresses.
+bool own_rows(int64_t rows, int64_t n, int64_t k) { return rows < (int64_t(1) << 30) && n < (1 << 22) && k < (1 << 22); }
 
 // Weight and bias gradients of one or two Linear layers on one input x [rows, K]: dy_i [rows, N], rows `ld` elements apart.
 struct WeightGrad {
@@ -1428,7 +1435,8 @@ struct WeightGrad {
 
 // dW = dy^T x contracts over all tokens: one GEMM of the BLAS library with K = rows runs at a fraction of the rate of the same
 // work as a batch of GEMMs with K = 2048 whose results are added (100 us against 43 us for 16384 x 1024 x 768 in bf16), so
-// long contractions are split into this many.
+// long contractions are split into this many.  Other numbers of tokens (1) take the library's own kernel in bf16: two of 1024 x 768 at 8704 tokens 39
+// us, the BLAS library 66; at 8192 37 : 34, at 16384 59 : 52.
 int64_t contraction_chunks(int64_t rows) {
   int64_t chunks = rows % 2048 == 0 ? rows / 2048 : 1;
   while (chunks > 16 && chunks % 2 == 0) chunks /= 2;
@@ -1443,7 +1451,16 @@ std::tuple<Tensor, Tensor> linear_parameter_grads(const Tensor& x, at::ScalarTyp
   if (need_w) {
     Tensor x2 = x.reshape({-1, x.size(-1)}).to(dy.scalar_type());
     const int64_t chunks = dy2.is_contiguous() && x2.is_contiguous() ? contraction_chunks(rows) : 1;
-    if (chunks > 1) {
+    if (chunks == 1 && rows >= 2048 && own_rows(rows, width, x2.size(1)) && x2.scalar_type() == at::kBFloat16 && plain(x) && plain(dy) && on_device_of(x2, dy2) && vector_rows(x2) && vector_rows(dy2)) {
+      const WeightGrad own(rows, width, x2.size(1), 1, at::kBFloat16);
+      Tensor sets = own.splits > 1 ? fresh({own.splits, width, x2.size(1)}, at::kFloat, dy2) : Tensor();
+      dw = fresh({width, x2.size(1)}, at::kBFloat16, dy2);
+      own.run(ptr(dy2), nullptr, width, ptr(x2), nullptr, ptr(dw), ptr(sets), nullptr, rows, at::kBFloat16, stream_of(dy2));
+      if (own.splits > 1) {
+        const rglru_sum job = own.weight_sum(ptr(sets), ptr(dw));
+        check(rglru_hip_sums(&job, 1, RGLRU_BF16, stream_of(dy2)), "rglru_hip_sums");
+      }
+    } else if (chunks > 1) {
       const int64_t per = rows / chunks;
       dw = sum_sets(at::bmm(dy2.view({chunks, per, width}).transpose(1, 2), x2.view({chunks, per, x2.size(1)})));
     } else {
@@ -1505,7 +1522,7 @@ struct Linear : torch::autograd::Function<Linear> {
       c10::DeviceGuard guard(x.device());
       Needs need(ctx);
       const int64_t bias_type = unpack(ctx)[0];
-      if (own_linear(x, weight, Tensor()) && grads[0].scalar_type() == x.scalar_type() && (bias_type == kNone || bias_type == (int64_t)x.scalar_type())) {
+      if (own_linear(x, weight, Tensor(), Product::kGradient) && grads[0].scalar_type() == x.scalar_type() && (bias_type == kNone || bias_type == (int64_t)x.scalar_type())) {
         std::tie(dx, dw, db) = own_backward(x, weight, grads[0], s[2], need(0), need(1), need(2));
         return once({dx, dw, db, Tensor()});
       }
@@ -1591,8 +1608,8 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
     auto [u, v] = known != nullptr ? *known : values(x, w1, opt(b1), w2, opt(b2));
     return {u, v};
   }
-  static bool own(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
-    return own_linear(x, w1, b1) && own_linear(x, w2, b2) && w1.sizes() == w2.sizes() && b1.defined() == b2.defined();
+  static bool own(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2, Product use = Product::kInference) {
+    return own_linear(x, w1, b1, use) && own_linear(x, w2, b2, use) && w1.sizes() == w2.sizes() && b1.defined() == b2.defined();
   }
   static std::tuple<Tensor, Tensor> values(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
     if (!own(x, w1, b1, w2, b2)) return {at::linear(x, w1, maybe(b1)), at::linear(x, w2, maybe(b2))};
@@ -1617,7 +1634,7 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
       const auto dtype = x.scalar_type();
       auto usual = [&](int64_t t) { return t == kNone || t == (int64_t)dtype; };
       if (grads[0].defined() && grads[1].defined() && grads[0].scalar_type() == dtype && grads[1].scalar_type() == dtype &&
-          own(x, w1, Tensor(), w2, Tensor()) && usual(m[0]) && usual(m[1])) {
+          own(x, w1, Tensor(), w2, Tensor(), Product::kGradient) && usual(m[0]) && usual(m[1])) {
         Tensor g0 = grads[0], g1 = grads[1];
         const int64_t N = w1.size(0), K = w1.size(1), rows = x.numel() / K;
         const int64_t ld = both.defined() ? 2 * N : N;
@@ -1730,12 +1747,13 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     const size_t tensor_bytes = round_up(M * W * 2);
     const int own = u.defined() ? 3 : 5;
     const size_t ws_bytes = round_up(rglru_hip_workspace_bytes(B, T, W, nb));
-    const bool stack = !own_linear(x, wx, bx);               // the weights stacked for the backward's GEMM of the BLAS library
+    const bool own_forward = own_linear(x, wx, bx, Product::kTrainingForward);
+    const bool stack = !own_linear(x, wx, bx, Product::kGradient);               // the weights stacked for the backward's GEMM of the BLAS library
     Tensor buffer = bytes(own * tensor_bytes + image_bytes + ws_bytes + (stack ? 2 * W * D * 2 : 0), x);
     Saved s(buffer, M, W);
     if (!first_reset && !flags.defined()) flags = block_flags(pos);
     if (!u.defined()) {
-      if (!stack) {
+      if (own_forward) {
         linear_forward(x, wx, bx, wy, by, Tensor(), s[3], s[4]);
       } else {
         Tensor x2 = x.view({M, D});
@@ -1754,7 +1772,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
                                       RGLRU_BF16 | (clears ? RGLRU_BACKWARD_CLEAR : 0), stream),
           "rglru_hip_prepare_block_fwd");
     Tensor out;
-    if (!stack) {
+    if (own_forward) {
       out = fresh_like(x);
       check(rglru_hip_linear(RGLRU_LINEAR_FORWARD, s[2], nullptr, W, ptr(wo), nullptr, W, ptr(bo), nullptr, bptr(active), ptr(out), nullptr, D,
                              nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
@@ -1785,6 +1803,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       char *image = s[u.defined() ? 3 : 5], *ws = image + round_up(prep_bytes(W, nb, RGLRU_BF16));
       Tensor dy = aligned(grads[0].to(kType));
       const bool own = !m[2];
+      const bool own_weights = own || (contraction_chunks(M) == 1 && own_rows(M, 2 * W, D));       // the library's own weight gradients
       if (!own && active.defined()) dy = masked_rows(dy, active, false);
 
       // parameter gradients; those of the two input projections are the halves of one sum each
@@ -1800,8 +1819,8 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       Parts scratch;
       scratch.add(M * W * 2), scratch.add(2 * M * W * 2);
       scratch.add(rglru_hip_bwd_scratch_bytes(B, T, W, nb, RGLRU_BF16)), scratch.add(rglru_hip_conv_scratch_bytes(B, T, W, K));
-      scratch.add(own ? go.sets_bytes : 0), scratch.add(own ? go.sums_bytes : column_bytes_o);
-      scratch.add(own ? gp.sets_bytes : 0), scratch.add(rglru_hip_block_sums_bytes(B, T, W, nb));
+      scratch.add(own_weights ? go.sets_bytes : 0), scratch.add(own_weights ? go.sums_bytes : column_bytes_o);
+      scratch.add(own_weights ? gp.sets_bytes : 0), scratch.add(rglru_hip_block_sums_bytes(B, T, W, nb));
       scratch.allocate(x);
       char *dgated = scratch.raw(), *du = scratch.raw(), *gate_scratch = scratch.raw(), *conv_scratch = scratch.raw(), *sets_o = scratch.raw(),
            *sums_o = scratch.raw(), *sets_p = scratch.raw(), *sums_p = scratch.raw();
@@ -1811,14 +1830,17 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
 
       // output projection
       if (own) {
-        go.run(ptr(dy), nullptr, D, s[2], bptr(active), ptr(g[WO]), sets_o, sums_o, M, kType, stream);
         check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, ptr(dy), nullptr, D, ptr(wo), nullptr, W, nullptr, nullptr, bptr(active), dgated, nullptr, W,
                                nullptr, nullptr, M, W, D, RGLRU_BF16, stream), "rglru_hip_linear");
+      } else {
+        Tensor dg = part(scratch.buffer, scratch.offsets[0], {M, W}, kType);
+        at::mm_out(dg, dy.view({M, D}), wo);
+      }
+      if (own_weights) {
+        go.run(ptr(dy), nullptr, D, s[2], own ? bptr(active) : nullptr, ptr(g[WO]), sets_o, sums_o, M, kType, stream);
         sums[0] = go.weight_sum(sets_o, ptr(g[WO])), sums[1] = go.bias_sum(sums_o, ptr(g[BO]));
       } else {
         Tensor dy2 = dy.view({M, D});
-        Tensor dg = part(scratch.buffer, scratch.offsets[0], {M, W}, kType);
-        at::mm_out(dg, dy2, wo);
         held_o = contraction(dy2, part(buffer, 2 * s.tensor_bytes, {M, W}, kType));
         check(rglru_hip_colsum(ptr(dy), sums_o, nullptr, M, D, RGLRU_BF16, RGLRU_BF16, stream), "rglru_hip_colsum");
         sums[0] = {ptr(held_o), ptr(g[WO]), held_o.size(0), D * W, RGLRU_BF16};
@@ -1836,13 +1858,16 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
           check(rglru_hip_linear(RGLRU_LINEAR_INPUT_GRAD, du, dv, 2 * W, ptr(wx), ptr(wy), D, nullptr, nullptr, nullptr, ptr(g[X]), nullptr, D,
                                  nullptr, nullptr, M, D, W, RGLRU_BF16, stream), "rglru_hip_linear");
         }
-        gp.run(du, dv, 2 * W, ptr(x), nullptr, ptr(dw_pair), sets_p, nullptr, M, kType, stream);
-        sums[2] = gp.weight_sum(sets_p, ptr(dw_pair));
       } else {
         Tensor both = part(scratch.buffer, scratch.offsets[1], {M, 2 * W}, kType);
         const size_t stacked = static_cast<size_t>(ws - s.at) + round_up(rglru_hip_workspace_bytes(B, T, W, nb));
         if (need_x) g[X] = at::mm(both, part(buffer, stacked, {2 * W, D}, kType)).view(x.sizes());
-        held_p = contraction(both, x.view({M, D}));
+      }
+      if (own_weights) {
+        gp.run(du, dv, 2 * W, ptr(x), nullptr, ptr(dw_pair), sets_p, nullptr, M, kType, stream);
+        sums[2] = gp.weight_sum(sets_p, ptr(dw_pair));
+      } else {
+        held_p = contraction(part(scratch.buffer, scratch.offsets[1], {M, 2 * W}, kType), x.view({M, D}));
         sums[2] = {ptr(held_p), ptr(dw_pair), held_p.size(0), 2 * W * D, RGLRU_BF16};
       }
       check(rglru_hip_block_finish(image, gate_scratch, conv_scratch, sums_p, ptr(g[WA]), ptr(g[WI]), ptr(g[BA]), ptr(g[BI]), ptr(g[LAM]),

@@ -1169,6 +1169,14 @@ def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, p
         assert err < 1e-2, name
 
 
+# multiply-adds of a product: 1.04e10 (gradients by the library, forward by the BLAS library), 2.6e10 with tokens that do not divide into the
+# BLAS library's batches (weight gradients by the library alone)
+@pytest.mark.parametrize("padded", [False, True])
+@pytest.mark.parametrize("B,T,D,W,nb", [(3, 1100, 1536, 2048, 16), (3, 2777, 1536, 2048, 16)])
+def test_block_training_between_the_lines_of_its_products(B, T, D, W, nb, padded):
+    test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded)
+
+
 @pytest.mark.parametrize("tokens", ["all", "positions", "padded"])
 @pytest.mark.parametrize("B,T,D,W,nb,carried", [(2, 2, 64, 96, 3, True), (3, 77, 72, 128, 2, True), (1, 1000, 192, 256, 16, False), (3, 2777, 1536, 2048, 16, True)])
 def test_block_inference_in_one_call_matches_layer_by_layer(B, T, D, W, nb, carried, tokens):
