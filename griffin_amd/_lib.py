@@ -59,6 +59,8 @@ _SIGNATURES = {
     "rglru_hip_token_facts": (ctypes.c_int, [_P] * 9 + [_I, _I, _P]),
     "rglru_hip_pack_flags": (ctypes.c_int, [_P] * 3 + [_I, _P]),
     "rglru_hip_mask_rows": (ctypes.c_int, [_P] * 3 + [_I, _I, ctypes.c_int, _P]),
+    "rglru_hip_pack_rows": (ctypes.c_int, [_P] * 3 + [_I] + [_P] * 2 + [_I] + [_P] * 2 + [_I] * 3 + [_P]),
+    "rglru_hip_unpack_rows": (ctypes.c_int, [_P] * 3 + [_I] * 4 + [_P]),
     "rglru_hip_conv_padded_scratch_bytes": (ctypes.c_size_t, [_I, _I]),
     "rglru_hip_conv_padded_fwd": (ctypes.c_int, [_P] * 9 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, _P]),
     "rglru_hip_conv_padded_bwd": (ctypes.c_int, [_P] * 12 + [_I, _I, _I, _I, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),

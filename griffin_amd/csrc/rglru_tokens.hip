@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstring>
+
 #include "rglru_device.h"
 #include "rglru_host.h"
 
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(kTokenThreads) void token_facts_kernel(TokenArgs p)
     const int prefix = count == s_last_t + 1 ? 1 : 0;           // the active tokens are the row's first ones
     p.rows[b] = count; p.rows[p.B + b] = doc; p.rows[2 * p.B + b] = prefix;
     if (p.last) p.last[b] = s_last_pos;
-    if (p.host) p.host[b] = (count == p.T ? 1u : 0u) | (prefix ? 2u : 0u);
+    if (p.host) p.host[b] = (count == p.T ? 1u : 0u) | (prefix ? 2u : 0u) | ((unsigned)count << 2);
   }
 }
 
@@ -171,6 +173,60 @@ __global__ __launch_bounds__(256) void mask_rows_kernel(MaskRowsArgs p) {
     for (int q = 0; q < AHEAD; ++q) {
       const long long i = i0 + q * stride;
       if (i < n && !(live[q] && p.in_place)) dst[i] = live[q] ? v[q] : V{};
+    }
+  }
+}
+
+// Right-padded rows without their padding, one behind the other: rows of `bytes` bytes (whole 16-byte vectors) of [B, T] tokens to
+// `packed` rows and back.  A workgroup has sixteen tokens of a row; where the row lies follows from the counts of the rows in front of it.  What
+// is left behind the last row is one more row, of zeros.  PACK: up to two arrays, and the positions and flags (as
+// rglru_hip_block_fwd takes them) of tokens whose rows are documents from their beginning.  Else: one array, padding becomes zero.
+// Streaming, a batch of eight vectors in flight per thread; what lies past the ends is dropped by the descriptors.
+struct PackArgs {
+  const int* counts; const f32x4* src[2]; f32x4* dst[2]; int per_row[2];
+  long long* pos; unsigned char* flags; int B, T, packed, chunks;
+};
+constexpr int kPackTokens = 16;
+template <bool PACK>
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p) {
+  constexpr int kTokens = kPackTokens, AHEAD = 8;
+  __shared__ int lds[4];
+  const int b = blockIdx.x / p.chunks, chunk = blockIdx.x - b * p.chunks;
+  int before = 0;
+  for (int i = threadIdx.x; i < b; i += 256) before += p.counts[i];
+#pragma unroll
+  for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = before;
+  __syncthreads();
+  const int first = lds[0] + lds[1] + lds[2] + lds[3];
+  const bool tail = b == p.B;                   // PACK only
+  // tokens of the row that exist, and those that this launch writes
+  const int there = tail ? 0 : p.counts[b], rows = PACK ? (tail ? p.packed - first : there) : p.T;
+  for (int t0 = chunk * kTokens; t0 < rows; t0 += p.chunks * kTokens) {
+    const int n = rows - t0 < kTokens ? rows - t0 : kTokens;
+    const long long wide = (long long)b * p.T + t0, narrow = (long long)first + t0;
+#pragma unroll
+    for (int a = 0; a < (PACK ? 2 : 1); ++a) {
+      if (!p.dst[a]) continue;
+      const unsigned per_row = (unsigned)p.per_row[a], all = (unsigned)n * per_row;
+      const f32x4* src = p.src[a] + (PACK ? wide : narrow) * per_row;
+      f32x4* dst = p.dst[a] + (PACK ? narrow : wide) * per_row;
+      // vectors that exist, and that may be written (counts that do not fit `packed` lose their tail)
+      const int left = there - t0 < n ? there - t0 : n, fit = PACK && p.packed - narrow < n ? (int)(p.packed - narrow) : n;
+      const unsigned live = left > 0 ? (unsigned)left * per_row : 0u, room = fit > 0 ? (unsigned)fit * per_row : 0u;
+      const rsrc_t from = make_rsrc(src, live * 16u), to = make_rsrc(dst, room * 16u);
+      for (unsigned i0 = threadIdx.x; i0 < all; i0 += 256 * AHEAD) {
+        i32x4 v[AHEAD];
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) v[q] = __builtin_amdgcn_raw_buffer_load_b128(from, (i0 + q * 256) * 16u, 0, 0);
+#pragma unroll
+        for (int q = 0; q < AHEAD; ++q) buf_store_b128(v[q], to, (i0 + q * 256) * 16u);
+      }
+    }
+    if (PACK && p.pos && (int)threadIdx.x < n && narrow + threadIdx.x < p.packed) {
+      const int t = t0 + (int)threadIdx.x;
+      p.pos[narrow + threadIdx.x] = t;
+      p.flags[narrow + threadIdx.x] = (unsigned char)((t == 0 ? RGLRU_FLAG_RESET : 0u) | ((t < 3 ? 3u - (unsigned)t : 0u) << RGLRU_FLAG_CONV_SHIFT));
     }
   }
 }
@@ -238,6 +294,46 @@ int rglru_hip_mask_rows(const void* src, const uint8_t* active, void* dst, int64
   else if (es == 2) hipLaunchKernelGGL((mask_rows_kernel<short>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((mask_rows_kernel<float>), grid, dim3(256), 0, s, a);
   return check_launch("mask_rows");
+}
+
+static int pack_args(const char* who, PackArgs& a, const int32_t* counts, int64_t B, int64_t T, int64_t packed) {
+  if (!counts) return fail(RGLRU_E_ARG, "%s: null pointer", who);
+  if (B <= 0 || T <= 0 || packed <= 0) return fail(RGLRU_E_ARG, "%s: empty shape", who);
+  if (B * T >= (1ll << 30) || packed >= (1ll << 30)) return fail(RGLRU_E_UNSUPPORTED, "%s: too large", who);
+  a.counts = counts; a.B = (int)B; a.T = (int)T; a.packed = (int)packed; a.chunks = (int)((T + kPackTokens - 1) / kPackTokens);
+  return RGLRU_OK;
+}
+static int pack_array(const char* who, PackArgs& a, int i, const void* src, void* dst, int64_t bytes) {
+  if (!src || !dst) return fail(RGLRU_E_ARG, "%s: null pointer", who);
+  if (bytes <= 0 || bytes % 16 || (uintptr_t)src % 16 || (uintptr_t)dst % 16) return fail(RGLRU_E_UNSUPPORTED, "%s: rows must be whole 16-byte vectors", who);
+  if (bytes >= (1ll << 28)) return fail(RGLRU_E_UNSUPPORTED, "%s: too large", who);
+  a.src[i] = (const f32x4*)src; a.dst[i] = (f32x4*)dst; a.per_row[i] = (int)(bytes / 16);
+  return RGLRU_OK;
+}
+
+int rglru_hip_pack_rows(const int32_t* counts, const void* src0, void* dst0, int64_t bytes0, const void* src1, void* dst1, int64_t bytes1,
+                        int64_t* pos, uint8_t* flags, int64_t B, int64_t T, int64_t packed, void* stream) {
+  PackArgs a;
+  memset(&a, 0, sizeof(a));
+  int rc = pack_args("pack_rows", a, counts, B, T, packed);
+  if (!rc) rc = pack_array("pack_rows", a, 0, src0, dst0, bytes0);
+  if (!rc && dst1) rc = pack_array("pack_rows", a, 1, src1, dst1, bytes1);
+  if (rc) return rc;
+  if (!pos != !flags) return fail(RGLRU_E_ARG, "pack_rows: positions and flags go together");
+  a.pos = (long long*)pos; a.flags = flags;
+  const long long blocks = (long long)(B + 1) * a.chunks;
+  hipLaunchKernelGGL((pack_rows_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
+  return check_launch("pack_rows");
+}
+
+int rglru_hip_unpack_rows(const int32_t* counts, const void* src, void* dst, int64_t bytes, int64_t B, int64_t T, int64_t packed, void* stream) {
+  PackArgs a;
+  memset(&a, 0, sizeof(a));
+  int rc = pack_args("unpack_rows", a, counts, B, T, packed);
+  if (!rc) rc = pack_array("unpack_rows", a, 0, src, dst, bytes);
+  if (rc) return rc;
+  hipLaunchKernelGGL((pack_rows_kernel<false>), dim3((unsigned)(B * a.chunks)), dim3(256), 0, (hipStream_t)stream, a);
+  return check_launch("unpack_rows");
 }
 
 int rglru_hip_conv_carry(const void* u, int64_t u_stride, const void* state, const int32_t* rows, void* new_state, int64_t B, int64_t T,

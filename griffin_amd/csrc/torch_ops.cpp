@@ -708,9 +708,12 @@ struct TokenFacts {
     }
     bool all_active = true, prefix = true;
     const int32_t* a = static_cast<const int32_t*>(answer_.data_ptr());
-    for (int64_t b = 0; b < answer_.size(0); ++b) all_active &= (a[b] & 1) != 0, prefix &= (a[b] & 2) != 0;
+    active_tokens = 0;
+    for (int64_t b = 0; b < answer_.size(0); ++b)
+      all_active &= (a[b] & 1) != 0, prefix &= (a[b] & 2) != 0, active_tokens += static_cast<uint32_t>(a[b]) >> 2;
     return {all_active, prefix};
   }
+  int64_t active_tokens = 0;                               // of all rows, once resolved
 
  private:
   void wait() {
@@ -1738,8 +1741,35 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
                         const Tensor& cw, const Tensor& cb, const Tensor& wa, const Tensor& ba, const Tensor& wi, const Tensor& bi,
                         const Tensor& lam, const Tensor& wo, const Tensor& bo, const Tensor& pos, const MaybeTensor& flags_,
                         const MaybeTensor& rows_, const MaybeTensor& active_, const MaybeTensor& u_, const MaybeTensor& v_, bool first_reset,
-                        double c) {
-    Tensor flags = opt(flags_), rows = opt(rows_), active = opt(active_), u = opt(u_), v = opt(v_);
+                        double c, int64_t packed) {
+    if (packed == 0)
+      return run(ctx, x, wx, bx, wy, by, cw, cb, wa, ba, wi, bi, lam, wo, bo, pos, opt(flags_), opt(rows_), opt(active_), opt(u_), opt(v_), first_reset, c,
+                 Packed());
+    // Right-padded rows that are documents from their beginning become ONE row of documents without the padding, so that every product
+    // and scan runs on the tokens that count; rows_ starts with the number of them in each row, u_ is the first projection of all tokens.
+    c10::DeviceGuard guard(x.device());
+    const Packed p = {x.size(0), x.size(1), packed, *rows_, x, *u_};
+    Tensor tokens = fresh({1, packed, x.size(2)}, kType, x);
+    Tensor positions = fresh({1, packed}, at::kLong, x), flags = fresh({1, packed}, at::kByte, x);
+    Tensor live = run(ctx, tokens, wx, bx, wy, by, cw, cb, wa, ba, wi, bi, lam, wo, bo, positions, flags, Tensor(), Tensor(), Tensor(), Tensor(), false, c, p);
+    return p.unpack(live);
+  }
+
+  struct Packed {
+    int64_t B = 0, T = 0, rows = 0;                          // of the padded batch; rows: 0 where it was not packed
+    Tensor counts, x, u;
+    Tensor unpack(const Tensor& src) const {
+      Tensor dst = fresh({B, T, src.size(-1)}, kType, src);
+      check(rglru_hip_unpack_rows(static_cast<const int32_t*>(ptr(counts)), ptr(src), ptr(dst), src.size(-1) * 2, B, T, rows, stream_of(src)),
+            "rglru_hip_unpack_rows");
+      return dst;
+    }
+  };
+
+  static Tensor run(AutogradContext* ctx, const Tensor& x, const Tensor& wx, const Tensor& bx, const Tensor& wy, const Tensor& by, const Tensor& cw,
+                    const Tensor& cb, const Tensor& wa, const Tensor& ba, const Tensor& wi, const Tensor& bi, const Tensor& lam, const Tensor& wo,
+                    const Tensor& bo, const Tensor& pos, Tensor flags, const Tensor& rows, const Tensor& active, const Tensor& u, const Tensor& v,
+                    bool first_reset, double c, const Packed& packed) {
     c10::DeviceGuard guard(x.device());
     const int64_t B = x.size(0), T = x.size(1), D = x.size(2), W = wx.size(0), K = cw.size(2), nb = wa.size(0), M = B * T;
     void* stream = stream_of(x);
@@ -1751,8 +1781,20 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     const bool stack = !own_linear(x, wx, bx, Product::kGradient);               // the weights stacked for the backward's GEMM of the BLAS library
     Tensor buffer = bytes(own * tensor_bytes + image_bytes + ws_bytes + (stack ? 2 * W * D * 2 : 0), x);
     Saved s(buffer, M, W);
-    if (!first_reset && !flags.defined()) flags = block_flags(pos);
-    if (!u.defined()) {
+    if (packed.rows) {
+      check(rglru_hip_pack_rows(static_cast<const int32_t*>(ptr(packed.counts)), ptr(packed.x), ptr(x), D * 2, ptr(packed.u), s[3], W * 2,
+                                static_cast<int64_t*>(pos.data_ptr()), static_cast<uint8_t*>(flags.data_ptr()), packed.B, packed.T, packed.rows, stream),
+            "rglru_hip_pack_rows");
+      if (own_forward) {
+        linear_forward(x, wy, by, Tensor(), Tensor(), Tensor(), s[4], nullptr);
+      } else {
+        Tensor out_v = part(buffer, 4 * tensor_bytes, {M, W}, kType);
+        at::addmm_out(out_v, by, x.view({M, D}), wy.t());
+      }
+    } else if (!first_reset && !flags.defined()) {
+      flags = block_flags(pos);
+    }
+    if (!u.defined() && !packed.rows) {
       if (own_forward) {
         linear_forward(x, wx, bx, wy, by, Tensor(), s[3], s[4]);
       } else {
@@ -1780,8 +1822,8 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       out = at::linear(part(buffer, 2 * tensor_bytes, {B, T, W}, kType), wo, bo);
       if (active.defined()) masked_rows(out, active, true);
     }
-    ctx->save_for_backward({x, wx, wy, wo, cw, pos, flags, rows, active, u, v, buffer});
-    pack(ctx, {first_reset, nb, stack});
+    ctx->save_for_backward({x, wx, wy, wo, cw, pos, flags, rows, active, u, v, buffer, packed.counts});
+    pack(ctx, {first_reset, nb, stack, packed.B, packed.T, packed.rows});
     return out;
   }
 
@@ -1792,7 +1834,8 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
                  &rows = saved[7], &active = saved[8], &u = saved[9], &v = saved[10], &buffer = saved[11];
     const bool first_reset = m[0];
     const int64_t nb = m[1];
-    variable_list g(22);
+    const Packed packed = {m[3], m[4], m[5], saved[12], Tensor(), Tensor()};
+    variable_list g(23);
     {
       at::NoGradGuard no_grad;
       c10::DeviceGuard guard(x.device());
@@ -1802,6 +1845,12 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       void *up = u.defined() ? ptr(u) : s[3], *vp = v.defined() ? ptr(v) : s[4];
       char *image = s[u.defined() ? 3 : 5], *ws = image + round_up(prep_bytes(W, nb, RGLRU_BF16));
       Tensor dy = aligned(grads[0].to(kType));
+      if (packed.rows) {
+        Tensor live = fresh({1, packed.rows, D}, kType, x);
+        check(rglru_hip_pack_rows(static_cast<const int32_t*>(ptr(packed.counts)), ptr(dy), ptr(live), D * 2, nullptr, nullptr, 0, nullptr, nullptr, packed.B,
+                                  packed.T, packed.rows, stream), "rglru_hip_pack_rows");
+        dy = live;
+      }
       const bool own = !m[2];
       const bool own_weights = own || (contraction_chunks(M) == 1 && own_rows(M, 2 * W, D));       // the library's own weight gradients
       if (!own && active.defined()) dy = masked_rows(dy, active, false);
@@ -1872,6 +1921,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       }
       check(rglru_hip_block_finish(image, gate_scratch, conv_scratch, sums_p, ptr(g[WA]), ptr(g[WI]), ptr(g[BA]), ptr(g[BI]), ptr(g[LAM]),
                                    ptr(g[CW]), ptr(g[CB]), ptr(g[BX]), ptr(g[BY]), sums, 3, B, T, W, nb, K, stream), "rglru_hip_block_finish");
+      if (packed.rows && need_x) g[X] = packed.unpack(g[X]);
       for (int i = 1; i < kTensors; ++i)
         if (!ctx->needs_input_grad(i)) g[i] = Tensor();
     }
@@ -1911,8 +1961,8 @@ bool token_shapes(int64_t B, int64_t T, int64_t W, const Tensor& pos, const Tens
 }
 
 // Nothing is returned where the node does not take the operands; the caller then goes layer by layer.
-MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const MaybeTensor& flags, const MaybeTensor& rows,
-                        const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
+MaybeTensor block_train_node(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const MaybeTensor& flags, const MaybeTensor& rows,
+                        const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c, int64_t packed) {
   typedef BlockTrain N;
   const int64_t B = x.size(0), T = x.size(1), D = x.size(2);
   refuse_tangents("the recurrent block", p);
@@ -1927,7 +1977,10 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
   // p: the node's tensors behind x
   const Tensor &wx = p[N::WX - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
   const int64_t W = wx.size(0);
-  if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 || !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), opt(v)) ||
+  // packed: the number of rows that the tokens that count are packed to; u is then there alone
+  if (packed > 0 && (!u.has_value() || !rows.has_value() || packed > B * T || rglru_hip_reproducible())) return std::nullopt;
+  if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 ||
+      !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), packed > 0 ? opt(u) : opt(v)) ||
       (u.has_value() && u->scalar_type() != N::kType) || (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
     return std::nullopt;
   // the gated reverse scan in tiles adds the gradient of linear_y's bias up in the order of its tickets
@@ -1937,7 +1990,38 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
   Tensor positions = pos.to(at::kLong).contiguous();
   auto contiguous = [](const MaybeTensor& t) { return t.has_value() ? MaybeTensor(aligned(*t)) : t; };
   return BlockTrain::apply(x, p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11], p[12], positions, flags, rows, live,
-                           contiguous(u), contiguous(v), first_reset, c);
+                           contiguous(u), contiguous(v), first_reset, c, packed);
+}
+
+MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const MaybeTensor& flags, const MaybeTensor& rows,
+                        const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
+  return block_train_node(x, p, pos, flags, rows, active, u, v, first_reset, c, 0);
+}
+MaybeTensor block_train_packed(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const Tensor& rows, const Tensor& u, int64_t packed,
+                               double c) {
+  return packed <= 0 ? std::nullopt : block_train_node(x, p, pos, std::nullopt, rows, std::nullopt, u, std::nullopt, false, c, packed);
+}
+
+// Right-padded batches are packed (BlockTrain::Packed) where products are long enough for the launches around it to pay, and a tenth of
+// the tokens or more is padding.  Training step of the block, half of the tokens padding, us, not packed : packed (multiply-adds of a product of
+// all tokens): 768 -> 1024 at 2.2e9 226 : 237, 3.1e9 243 : 237, 4.1e9 269 : 247, 6.8e9 374 : 296, 1.0e10 (64 rows) 507 : 359, 1.3e10 538 : 434; 512 ->
+// 512 at 4.3e9 302 : 269.  Rows: multiples of 64, and of 512 from 8192 on, where the BLAS library may take products (a size it has not seen
+// costs it a search).
+bool block_may_pack(const Tensor& x, const Tensor& w) {
+  return x.dim() == 3 && x.size(0) > 1 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && double(x.numel()) * w.size(0) >= 3e9 && !rglru_hip_reproducible();
+}
+int64_t block_packed_rows(int64_t B, int64_t T, int64_t active_tokens) {
+  const int64_t grain = active_tokens >= 8192 ? 512 : 64, rows = (std::max<int64_t>(active_tokens, 1) + grain - 1) / grain * grain;
+  return 10 * rows <= 9 * B * T ? rows : 0;
+}
+
+// x w^T + b without a graph.
+Tensor linear_values(const Tensor& x, const Tensor& w, const MaybeTensor& b) {
+  const Tensor bias = opt(b);
+  refuse_tangents("hip_linear", std::initializer_list<Tensor>{x, w, bias});
+  require_device_of("hip_linear", x, {&w, &bias});
+  at::NoGradGuard no_grad;
+  return Linear::values(x, w, bias, Tensor());
 }
 
 // The whole block over sequences without gradients (griffin/griffin.py:459-528): projections, positions, convolution, RG-LRU
@@ -2122,7 +2206,8 @@ PYBIND11_MODULE(_native, m) {
       .def_readonly("flags", &TokenFacts::flags)
       .def_readonly("conv_positions", &TokenFacts::conv_positions)
       .def_readonly("rows", &TokenFacts::rows)
-      .def_readonly("last_position", &TokenFacts::last_position);
+      .def_readonly("last_position", &TokenFacts::last_position)
+      .def_readonly("active_tokens", &TokenFacts::active_tokens);
   EXPORT(causal_conv);
   EXPORT(causal_conv_padded);
   EXPORT(gelu_gate);
@@ -2136,7 +2221,11 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(linear);
   EXPORT(linear_pair);
   EXPORT(linear_pair_values);
+  EXPORT(linear_values);
+  EXPORT(block_may_pack);
+  EXPORT(block_packed_rows);
   EXPORT(block_train);
+  EXPORT(block_train_packed);
   EXPORT(block_infer);
   EXPORT(rmsnorm);
 #undef EXPORT

@@ -114,6 +114,23 @@ def hip_block_forward(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: T
     return gated, h_last, new_conv
 
 
+def hip_block_may_pack(x: Tensor, w: Tensor) -> bool:
+    """Whether a right-padded batch ``x`` [B, T, D] trains without its padding (``hip_block_train_packed``) if there is enough of it."""
+    return _lib.native().block_may_pack(x, w)
+
+
+def hip_block_train_packed(x: Tensor, parameters, facts, u: Tensor, c: float) -> Tensor | None:
+    """``hip_block_forward`` with ``around`` on a batch whose rows are right-padded documents from their beginning: products and scans
+    run on the active tokens alone, packed one row behind the other.  ``facts``: resolved ``token_facts`` of the mask; ``u``: the
+    values of linear_x on all tokens.  Returns the output [B, T, D], or None where there is too little padding, or the operator does not
+    take the operands."""
+    native = _lib.native()
+    rows = native.block_packed_rows(x.shape[0], x.shape[1], facts.active_tokens)
+    if rows == 0:
+        return None
+    return native.block_train_packed(x, parameters, facts.conv_positions, facts.rows, u, rows, c)
+
+
 def hip_block_decode_step(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: Tensor, bias: Tensor | None,
                           prev_pos: Tensor | None, segment_pos: Tensor | None, active: Tensor | None,
                           prep, rnn_state: Tensor | None):
@@ -205,6 +222,11 @@ def hip_linear_pair(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Te
 def hip_linear_pair_values(x: Tensor, w1: Tensor, b1: Tensor | None, w2: Tensor, b2: Tensor | None) -> tuple[Tensor, Tensor]:
     """The values of ``hip_linear_pair`` without a graph behind them."""
     return _lib.native().linear_pair_values(x, w1, b1, w2, b2)
+
+
+def hip_linear_values(x: Tensor, w: Tensor, b: Tensor | None) -> Tensor:
+    """The value of ``hip_linear`` without a graph behind it."""
+    return _lib.native().linear_values(x, w, b)
 
 
 @lru_cache(maxsize=None)

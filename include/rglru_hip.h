@@ -16,7 +16,7 @@
  *   (no counterpart: forward for callers that cannot allocate)              rglru_hip_fwd_static
  *   griffin/griffin.py:379-389 and autograd   the block's Linear layers      rglru_hip_linear, rglru_hip_sums
  *   griffin/griffin.py:379-389, :474-487 with T == 1   the same for a decode step, with its convolution   rglru_hip_decode_project, rglru_hip_decode_linear
- *   griffin/griffin.py:309-358, :488-510   what an activity mask says about the tokens   rglru_hip_token_facts, rglru_hip_pack_flags, rglru_hip_mask_rows
+ *   griffin/griffin.py:309-358, :488-510   what an activity mask says about the tokens   rglru_hip_token_facts, rglru_hip_pack_flags, rglru_hip_mask_rows, rglru_hip_pack_rows
  *   autograd of griffin/griffin.py:464-520   reverse scan with the output gate, convolution, last sums   rglru_hip_block_bwd, rglru_hip_block_finish
  *   griffin/griffin.py:474-487      causal depthwise convolution of the caller   rglru_hip_conv_fwd
  *   autograd of griffin/griffin.py:474-487                                   rglru_hip_conv_bwd
@@ -264,7 +264,7 @@ int rglru_hip_steps(const void* x, const void* prep, float* h, const uint8_t* fl
  * rglru_hip_conv_rows_bwd needs, tokens since the document start or unbounded where none lies in this call; rows[3 B]: active
  * tokens of the row, ordinal of its last document start (-1: none), 1 where its active tokens are its first ones;
  * last_pos[B] (NULL to skip): position of the row's last active token, or prev_pos; host_facts[B] (NULL to skip; may be
- * memory of the host): bit 0 = every token of the row is active, bit 1 = rows' third word. */
+ * memory of the host): bit 0 = every token of the row is active, bit 1 = rows' third word, from bit 2 on its first word. */
 int rglru_hip_token_facts(const uint8_t* active, const int64_t* segment_pos, const int64_t* prev_pos, int64_t* pos, uint8_t* flags,
                           int64_t* conv_pos, int32_t* rows, int64_t* last_pos, uint32_t* host_facts, int64_t B, int64_t T,
                           void* stream);
@@ -275,6 +275,14 @@ int rglru_hip_pack_flags(const uint8_t* reset, const uint8_t* active, uint8_t* f
 /* dst[r, :] = active[r] ? src[r, :] : 0 over rows of D elements (griffin/griffin.py:522-523).  With dst == src only the rows
  * that become zero are written. */
 int rglru_hip_mask_rows(const void* src, const uint8_t* active, void* dst, int64_t rows, int64_t D, int dtype, void* stream);
+
+/* Rows of `bytes` bytes of [B, T] tokens whose first counts[b] (rglru_hip_token_facts) are active, packed one row behind the other without
+ * their padding, and back (padding becomes zero).  `packed` >= the sum of the counts; what is left of it is filled with zeros.  src1 / dst1
+ * / bytes1: a second array, or NULL.  pos[packed], flags[packed] (both or neither): positions and the flags of rglru_hip_block_fwd where every
+ * row is a document from its beginning; what is left is one more.  Rows are whole 16-byte vectors on a 16-byte boundary. */
+int rglru_hip_pack_rows(const int32_t* counts, const void* src0, void* dst0, int64_t bytes0, const void* src1, void* dst1, int64_t bytes1,
+                        int64_t* pos, uint8_t* flags, int64_t B, int64_t T, int64_t packed, void* stream);
+int rglru_hip_unpack_rows(const int32_t* counts, const void* src, void* dst, int64_t bytes, int64_t B, int64_t T, int64_t packed, void* stream);
 
 /* The carried rows new_state[B,K-1,W] of the padded convolution (griffin/griffin.py:488-510) for rows whose active tokens are
  * their first ones; `rows` from rglru_hip_token_facts. */

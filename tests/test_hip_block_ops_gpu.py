@@ -1177,6 +1177,87 @@ def test_block_training_between_the_lines_of_its_products(B, T, D, W, nb, padded
     test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded)
 
 
+@pytest.mark.parametrize("B,T,counts,packed", [(1, 1, [1], 1), (3, 16, [16, 0, 5], 64), (5, 37, [1, 0, 37, 17, 16], 71), (300, 70, None, 11520), (2, 5000, [4999, 3], 5056),
+                                               (2, 3, [1, 2], 700)])
+def test_rows_are_packed_and_unpacked(B, T, counts, packed):
+    """Rows without their padding and back, for counts at the edges of a workgroup's tokens, empty rows, and a rest longer than a row: two
+    arrays of different widths, positions and flags; nothing outside the results is written."""
+    from griffin_amd import _lib
+
+    lib = _lib.load()
+    _say("pack", B, T, packed)
+    gen = torch.Generator().manual_seed(T)
+    if counts is None:
+        counts = torch.randint(0, T + 1, (B,), generator=gen).tolist()
+    assert sum(counts) <= packed
+    stream = torch.cuda.current_stream().cuda_stream
+    device = torch.tensor(counts, dtype=torch.int32, device="cuda")
+    live = torch.arange(T)[None] < torch.tensor(counts)[:, None]
+    wide = [torch.randn(B, T, n, generator=gen).cuda() for n in (4, 92)]
+    narrow = [torch.full((packed + 1, n), 7.0, device="cuda") for n in (4, 92)]
+    pos, flags = torch.full((packed + 1,), -7, device="cuda"), torch.full((packed + 1,), 77, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.rglru_hip_pack_rows(device.data_ptr(), wide[0].data_ptr(), narrow[0].data_ptr(), 16, wide[1].data_ptr(), narrow[1].data_ptr(), 368,
+                                       pos.data_ptr(), flags.data_ptr(), B, T, packed, stream), "pack_rows")
+    rest = packed - sum(counts)
+    for x, y in zip(wide, narrow):
+        want = torch.cat((x.cpu()[live], torch.zeros(rest, x.size(2)), torch.full((1, x.size(2)), 7.0)))
+        assert torch.equal(y.cpu(), want)
+        back = torch.full((B * T + 1, x.size(2)), 7.0, device="cuda")
+        _lib.check(lib.rglru_hip_unpack_rows(device.data_ptr(), y.data_ptr(), back.data_ptr(), 4 * x.size(2), B, T, packed, stream), "unpack_rows")
+        assert torch.equal(back[:-1].cpu().view(B, T, -1), x.cpu() * live[:, :, None]) and (back[-1] == 7.0).all()
+    want = torch.cat([torch.arange(n) for n in (*counts, rest)])
+    assert torch.equal(pos.cpu(), torch.cat((want, torch.tensor([-7]))))
+    near = (3 - want.clamp(max=3)) << 2                          # RGLRU_FLAG_CONV_SHIFT
+    assert torch.equal(flags.cpu(), torch.cat(((near | (want == 0)), torch.tensor([77]))).to(torch.uint8))
+
+
+@pytest.mark.parametrize("B,T,D,W,nb,lengths", [(5, 1700, 768, 1024, 8, [0, 1, 2, 3, 1700]), (150, 33, 768, 1024, 16, None), (3, 2000, 640, 832, 8, [2000, 1, 1500]),
+                                                (9, 2048, 768, 1024, 16, [2048, 2048, 5, 2048, 64, 128, 2047, 1, 513]), (4, 1100, 768, 1024, 8, [0, 0, 0, 0])])
+def test_block_trains_on_right_padded_batches_without_their_padding(B, T, D, W, nb, lengths):
+    """Long right-padded batches run on their active tokens alone: output and gradients against the block taken layer by layer, whatever
+    lies in the padding; a second backward pass over the same forward repeats."""
+    from griffin_amd import RecurrentBlock, hip_block_ops
+
+    _say("packed block", B, T, D, W, nb)
+    torch.manual_seed(5)
+    lengths = torch.tensor(lengths if lengths is not None else [(7 * i) % (T + 1) for i in range(B)])
+    block = RecurrentBlock(D, W, gate_blocks=nb, scan_mode="hip").cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            if name.endswith("bias"):
+                p.normal_(std=0.1)
+    active = (torch.arange(T)[None] < lengths[:, None]).cuda()
+    x = torch.randn(B, T, D, device="cuda", dtype=torch.bfloat16)
+    dy = torch.randn_like(x)
+    names, leaves = zip(*block.named_parameters())
+    calls, real = [], hip_block_ops.hip_block_train_packed
+
+    def spy(*args):
+        calls.append(real(*args))
+        return calls[-1]
+
+    hip_block_ops.hip_block_train_packed = spy
+    try:
+        dirty = x.masked_fill(~active[:, :, None], float("nan")).requires_grad_(True)
+        whole = block(dirty, active_mask=active)
+    finally:
+        hip_block_ops.hip_block_train_packed = real
+    assert len(calls) == 1 and calls[0] is not None
+    got = torch.autograd.grad(whole, (dirty, *leaves), dy.masked_fill(~active[:, :, None], float("nan")), retain_graph=True)
+    again = torch.autograd.grad(whole, (dirty, *leaves), dy)
+    x.requires_grad_(True)
+    layered, _ = block(x, active_mask=active, return_cache=True)
+    want = torch.autograd.grad(layered, (x, *leaves), dy)
+    torch.cuda.synchronize()
+    assert (whole[~active] == 0).all() and (got[0][~active] == 0).all()
+    assert rel_err(whole.float(), layered.float()) < 1e-2
+    for name, g, a, w in zip(("x", *names), got, again, want):
+        norm = w.float().norm().clamp_min(1e-30)
+        err = float((g.float() - w.float()).norm() / norm)
+        _say("  d%s rel error: %.2e" % (name, err))
+        assert err < 1e-2 and float((a.float() - w.float()).norm() / norm) < 1e-2, name
+
+
 @pytest.mark.parametrize("tokens", ["all", "positions", "padded"])
 @pytest.mark.parametrize("B,T,D,W,nb,carried", [(2, 2, 64, 96, 3, True), (3, 77, 72, 128, 2, True), (1, 1000, 192, 256, 16, False), (3, 2777, 1536, 2048, 16, True)])
 def test_block_inference_in_one_call_matches_layer_by_layer(B, T, D, W, nb, carried, tokens):
