@@ -2082,13 +2082,17 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
   const long long chunks = (T + 32 * kDeltaMT - 1) / (32 * kDeltaMT);
   a.wg_per_unit = pick_wg_per_unit(a.units, B * chunks, kDeltaMT == 1 ? 4 : RGLRU_DELTA_OCC, L.max_wg);
   a.queues = pick_queues(B, a.wg_per_unit);
-  const bool masked = (flags != nullptr) || (T % (32 * kDeltaMT) != 0);
+  // Tokens past the end: dy reads as zero there, so nothing comes out of them; only a gradient at the final state, which enters behind them,
+  // has to pass them unchanged, as in the masked variants.  (Their decays patched in the plain ones: up to 18 registers and two spills
+  // in every call for this one.)  Reverse scan, us, masked : plain: B8 T2049 W1024
+  // (128) 27.3 : 25.8, B1 T8191 (64) 25.0 : 23.1; the gradient kernel of the same 63.0 : 57.5, 31.1 : 28.6.
+  const bool masked = flags || (dh_last && T % (32 * kDeltaMT) != 0);
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
   const bool chain_scan = fwd_chain_pays(B, T, g.Wp);
   if (chain_scan) {
     // enough chains to give every compute unit one of its own (see fwd_impl)
     const dim3 cgrid((unsigned)(8 * ((B * nb + 7) / 8) * g.S));
-    const bool cmasked = (flags != nullptr) || (T % 32 != 0);
+    const bool cmasked = flags || (dh_last && T % 32 != 0);
     KernelTimer timer(1, s);
 #define RGLRU_LAUNCH_DELTA_CHAIN(N, M, P)                                                                            \
     do {                                                                                                             \
@@ -2116,7 +2120,8 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
   if (rc) return rc;
   // gradients: one workgroup per compute unit, the same units
   const int n_wg = grad_workgroups(B, T, a.units);
-  const bool masked_grad = (flags != nullptr) || (T % 32 != 0);
+  // tokens past the end: delta, x and h read as zero there, so every gradient of them is zero without a mask
+  const bool masked_grad = flags != nullptr;
   dim3 grid2((unsigned)(n_wg * a.units));
   {
     KernelTimer timer(3, s);

@@ -1129,6 +1129,36 @@ def test_forward_without_flags_of_batches_that_fill_rounds(bw, nb, B, T, owned, 
         assert err < BF16_TOL, (name, err)
 
 
+@pytest.mark.parametrize("bw,nb", [(128, 2), (64, 3), (32, 4), (160, 1), (320, 1)])
+@pytest.mark.parametrize("B,T", [(3, 1), (2, 31), (2, 33), (3, 63), (2, 65), (1, 127), (2, 300)])
+@pytest.mark.parametrize("how", ["plain", "first_reset", "dh_last"])
+@pytest.mark.parametrize("chain", [1, 2])
+def test_lengths_that_end_inside_a_tile_without_flags(bw, nb, B, T, how, chain):
+    """Without flags a length may end anywhere in a tile of the tiled and of the chain kernels: final state, output and gradients, also with a
+    gradient at the final state, which enters behind the tokens that are not there."""
+    from griffin_amd import hip_rglru, set_chain_forward
+
+    W = bw * nb
+    _say("ragged", bw, nb, B, T, how, chain)
+    case = orc.make_case(B, T, W, nb, seed=bw + T, h0_std=0.5, bias_std=0.5)
+    reset = (torch.arange(T) == 0).expand(B, T) if how == "first_reset" else None
+    dh_last = torch.randn(B, W, generator=torch.Generator().manual_seed(6)) if how == "dh_last" else None
+    leaves = [case[k].to(torch.bfloat16).cuda().requires_grad_(True) for k in PARAMS]
+    was = set_chain_forward(chain)
+    try:
+        y, h_last = hip_rglru(*leaves, 8.0, case["h0"].cuda(), first_token_reset=reset is not None)
+        grads = torch.autograd.grad([y] if dh_last is None else [y, h_last], leaves,
+                                    [case["dy"].to(torch.bfloat16).cuda()] + ([] if dh_last is None else [dh_last.cuda()]))
+        torch.cuda.synchronize()
+    finally:
+        set_chain_forward(was)
+    ry, rh, rgrads = oracle_run(case, torch.bfloat16, reset, None, dh_last)
+    errs = {"y": rel_err(y.float(), ry), "h_last": rel_err(h_last, rh)}
+    errs.update({name: rel_err(g.float(), rgrads[name]) for name, g in zip(PARAMS, grads)})
+    for name, err in errs.items():
+        assert err < BF16_TOL, (name, err)
+
+
 @pytest.mark.parametrize("B,W,once,stream", [(250, 260, False, False), (251, 260, True, False), (1016, 256, True, False), (1018, 256, True, True)])
 def test_scan_op_gradients_below_and_above_the_cache(B, W, once, stream):
     """From 32 MB a tensor on the inputs that are read once bypass the caches, and from 256 MB of gradients on these are stored past
