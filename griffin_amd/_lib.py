@@ -91,6 +91,8 @@ _SIGNATURES = {
                                     + [_I, _I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_block_infer": (ctypes.c_int, [_P, _I, _P, _I, _P, _P, _P, _I, ctypes.c_int] + [_P] * 10
                               + [_I, _I, _I, _I, ctypes.c_int, _P]),
+    "rglru_hip_block_project": (ctypes.c_int, [_P] * 12 + [_I] * 5 + [ctypes.c_int, _P]),
+    "rglru_hip_block_infer_projected": (ctypes.c_int, [_P, _I, _P, _I] + [_P] * 3 + [_I, ctypes.c_int] + [_P] * 7 + [_I] * 4 + [ctypes.c_int, _P]),
     "rglru_hip_step_gated": (ctypes.c_int, [_P] * 6 + [_I, _P] + [_I, _I, _I, ctypes.c_int, _P]),
     "rglru_hip_set_spin_limit": (ctypes.c_int64, [_I]),
     "rglru_hip_set_reproducible": (ctypes.c_int, [ctypes.c_int]),

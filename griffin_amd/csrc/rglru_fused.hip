@@ -16,6 +16,7 @@
 
 
 #include "rglru_fused.h"
+#include "rglru_linear.h"
 
 namespace rglru {
 
@@ -780,27 +781,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 1) void fwd_chain_kernel(FusedArg
   if (gave_up && lane == 0) atomicOr(p.fail, 1u);
 }
 
-// What the block forward of an inference call needs in front of it, in one launch: the flag bytes of every token (reset at
-// position 0, in bits 2-3 the lags that reach in front of the document), each row's last position and the cleared part of
-// the workspace.  (Five launches of 2 us each and two casts before: 12 us of GPU time and 25 us of the host's.)
-struct PositionArgs {
-  const long long* prev; const long long* segpos; unsigned char* flags; long long* last;
-  uint4* clear; long long clear_n;
-  int B, T;
-};
+// The positions of an inference call as a launch of its own (in front of products of the BLAS library).
 __global__ __launch_bounds__(256) void block_positions_kernel(PositionArgs p) {
-  const long long n = p.flags ? (long long)p.B * p.T : 0, stride = (long long)gridDim.x * 256;
-  const long long first = (long long)blockIdx.x * 256 + threadIdx.x;
-  for (long long i = first; i < p.clear_n; i += stride) p.clear[i] = make_uint4(0u, 0u, 0u, 0u);
-  for (long long i = first; i < n; i += stride) {
-    const int b = (int)(i / p.T), t = (int)(i - (long long)b * p.T);
-    const long long pos = p.segpos ? p.segpos[i] : p.prev[b] + 1 + t;
-    const unsigned near = pos < 0 ? 3u : pos < 3 ? (unsigned)(3 - pos) : 0u;
-    p.flags[i] = (unsigned char)((pos == 0 ? RGLRU_FLAG_RESET : 0u) | (near << RGLRU_FLAG_CONV_SHIFT));
-  }
-  if (p.last)
-    for (long long b = first; b < p.B; b += stride)
-      p.last[b] = p.segpos ? p.segpos[b * p.T + p.T - 1] : (p.prev ? p.prev[b] : -1ll) + p.T;
+  token_positions(p, (long long)blockIdx.x * 256 + threadIdx.x, (long long)gridDim.x * 256);
 }
 
 #define RGLRU_FWD_WIDE_CASE(N, grid, stream, args, dtype, nkg, masked)                                              \
@@ -1210,31 +1193,55 @@ int rglru_hip_block_fwd(const void* u, int64_t u_stride, const void* v, int64_t 
   return fwd_impl(u, prep, h0, flags, y, h_last, ws, B, T, W, nb, dtype, false, stream, nullptr, &blk);
 }
 
+// What an inference call derives from the positions it continues at, and the part of the workspace its forward needs cleared.
+static int position_args(const char* who, const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes, int64_t* last_pos, void* ws,
+                         int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, PositionArgs& a) {
+  int rc = check_geometry(who, W, nb, dtype);
+  if (rc) return rc;
+  if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "%s: B and T must be positive (got %lld, %lld)", who, (long long)B, (long long)T);
+  const bool first_reset = !prev_pos && !segment_pos;
+  if (!ws || (!first_reset && !flag_bytes)) return fail(RGLRU_E_ARG, "%s: null pointer", who);
+  rc = check_extents(who, B, T, W);
+  if (rc) return rc;
+  const WorkLayout L = make_work_layout(B, T, make_geometry(W, nb));
+  a.prev = (const long long*)prev_pos; a.segpos = (const long long*)segment_pos; a.flags = first_reset ? nullptr : flag_bytes;
+  a.last = (long long*)last_pos; a.B = (int)B; a.T = (int)T;
+  a.clear = (uint4*)((char*)ws + L.f_begin); a.clear_n = (long long)(L.f_end - L.f_begin) / 16;
+  return RGLRU_OK;
+}
+
+int rglru_hip_block_project(const void* x, const void* w0, const void* w1, const void* bias0, const void* bias1, void* u, void* v,
+                            const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes, int64_t* last_pos, void* ws,
+                            int64_t B, int64_t T, int64_t D, int64_t W, int64_t nb, int dtype, void* stream) {
+  PositionArgs a;
+  const int rc = position_args("block_project", prev_pos, segment_pos, flag_bytes, last_pos, ws, B, T, W, nb, dtype, a);
+  return rc ? rc : linear_pair_with_positions(x, w0, w1, bias0, bias1, u, v, B * T, W, D, dtype, a, stream);
+}
+
+int rglru_hip_block_infer_projected(const void* u, int64_t u_stride, const void* v, int64_t v_stride,
+                                    const void* conv_state, const void* taps, const void* conv_bias, int64_t K, int vec_dtype,
+                                    const void* prep, const float* h0, const uint8_t* flag_bytes, void* gated, void* new_conv_state,
+                                    float* h_last, void* ws, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream) {
+  const BlockFwd blk = {v, u_stride, v_stride, conv_state, taps, conv_bias, K, vec_dtype, nullptr, gated, new_conv_state};
+  return fwd_impl(u, prep, h0, flag_bytes ? flag_bytes : RGLRU_FLAGS_FIRST_RESET, nullptr, h_last, ws, B, T, W, nb, dtype, true, stream, nullptr, &blk);
+}
+
 int rglru_hip_block_infer(const void* u, int64_t u_stride, const void* v, int64_t v_stride,
                           const void* conv_state, const void* taps, const void* conv_bias, int64_t K, int vec_dtype,
                           const void* prep, const float* h0, const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes,
                           void* gated, void* new_conv_state, float* h_last, int64_t* last_pos, void* ws,
                           int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream) {
-  int rc = check_geometry("block_infer", W, nb, dtype);
-  if (rc) return rc;
-  if (B <= 0 || T <= 0) return fail(RGLRU_E_ARG, "block_infer: B and T must be positive (got %lld, %lld)", (long long)B, (long long)T);
-  const bool first_reset = !prev_pos && !segment_pos;
-  if (!ws || (!first_reset && !flag_bytes)) return fail(RGLRU_E_ARG, "block_infer: null pointer");
-  rc = check_extents("block_infer", B, T, W);
-  if (rc) return rc;
-  const WorkLayout L = make_work_layout(B, T, make_geometry(W, nb));
   PositionArgs a;
-  a.prev = (const long long*)prev_pos; a.segpos = (const long long*)segment_pos; a.flags = first_reset ? nullptr : flag_bytes;
-  a.last = (long long*)last_pos; a.B = (int)B; a.T = (int)T;
-  a.clear = (uint4*)((char*)ws + L.f_begin); a.clear_n = (long long)(L.f_end - L.f_begin) / 16;
-  long long items = first_reset ? B : B * T;
+  int rc = position_args("block_infer", prev_pos, segment_pos, flag_bytes, last_pos, ws, B, T, W, nb, dtype, a);
+  if (rc) return rc;
+  long long items = a.flags ? B * T : B;
   if (a.clear_n > items) items = a.clear_n;
   long long blocks = (items + 255) / 256; if (blocks > 2048) blocks = 2048;
   hipLaunchKernelGGL(block_positions_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, a);
   rc = check_launch("block_infer positions");
   if (rc) return rc;
-  const BlockFwd blk = {v, u_stride, v_stride, conv_state, taps, conv_bias, K, vec_dtype, nullptr, gated, new_conv_state};
-  return fwd_impl(u, prep, h0, first_reset ? RGLRU_FLAGS_FIRST_RESET : flag_bytes, nullptr, h_last, ws, B, T, W, nb, dtype, true, stream, nullptr, &blk);
+  return rglru_hip_block_infer_projected(u, u_stride, v, v_stride, conv_state, taps, conv_bias, K, vec_dtype, prep, h0, a.flags, gated,
+                                         new_conv_state, h_last, ws, B, T, W, nb, dtype, stream);
 }
 
 int rglru_hip_prepare_block_fwd(const void* w_a, const void* b_a, const void* w_x, const void* b_x,

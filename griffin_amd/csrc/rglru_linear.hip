@@ -177,6 +177,9 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
+  if constexpr (DIRECT && sizeof(IO) == 2) {
+    if (p.positions.B > 0) token_positions(p.positions, (long long)blockIdx.x * kLinearThreads + threadIdx.x, (long long)gridDim.x * kLinearThreads);
+  }
   // Workgroups go to the eight XCDs round-robin; each XCD gets a contiguous run of tiles (columns fastest), so that
   // the rows they share come from memory once and the weights stay in its L2.
   const int per_xcd = (p.total + 7) >> 3;
@@ -590,16 +593,9 @@ int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long l
 
 using namespace rglru;
 
-extern "C" {
-
-int64_t rglru_hip_linear_splits(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
-  if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return linear_plan(kind, M, N, K, problems, 1, dtype).splits;
-}
-
-int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
-                     const void* bias0, const void* bias1, const uint8_t* active, void* c0, void* c1, int64_t ldc,
-                     float* partial, float* colsum, int64_t M, int64_t N, int64_t K, int dtype, void* stream) {
+static int linear_product(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
+                          const void* bias0, const void* bias1, const uint8_t* active, void* c0, void* c1, int64_t ldc,
+                          float* partial, float* colsum, int64_t M, int64_t N, int64_t K, int dtype, void* stream, const PositionArgs* positions) {
   if (dtype != RGLRU_F32 && dtype != RGLRU_BF16) return fail(RGLRU_E_ARG, "linear: dtype must be RGLRU_F32 or RGLRU_BF16, got %d", dtype);
   if (kind < RGLRU_LINEAR_FORWARD || kind > RGLRU_LINEAR_WEIGHT_GRAD) return fail(RGLRU_E_ARG, "linear: unknown kind %d", kind);
   if (M <= 0 || N <= 0 || K <= 0) return fail(RGLRU_E_ARG, "linear: empty product %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
@@ -628,9 +624,32 @@ int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, cons
   a.M = (int)M; a.N = (int)N; a.K = (int)K;
   const int64_t bk = dtype == RGLRU_BF16 ? 64 : 32;
   a.k_per_split = (int)(((K + a.splits - 1) / a.splits + bk - 1) / bk * bk);
+  if (positions) a.positions = *positions;
   hipStream_t s = (hipStream_t)stream;
   linear_launch(a, kind, plan.edge, dtype, s);
   return check_launch("linear");
+}
+
+namespace rglru {
+int linear_pair_with_positions(const void* x, const void* w0, const void* w1, const void* bias0, const void* bias1, void* u, void* v, int64_t M,
+                               int64_t N, int64_t K, int dtype, const PositionArgs& positions, void* stream) {
+  if (dtype != RGLRU_BF16) return fail(RGLRU_E_UNSUPPORTED, "block_project: needs bf16 storage");
+  if (!w1 || !v) return fail(RGLRU_E_ARG, "block_project: null pointer");
+  return linear_product(RGLRU_LINEAR_FORWARD, x, nullptr, K, w0, w1, K, bias0, bias1, nullptr, u, v, N, nullptr, nullptr, M, N, K, dtype, stream, &positions);
+}
+}  // namespace rglru
+
+extern "C" {
+
+int64_t rglru_hip_linear_splits(int kind, int64_t M, int64_t N, int64_t K, int problems, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  return linear_plan(kind, M, N, K, problems, 1, dtype).splits;
+}
+
+int rglru_hip_linear(int kind, const void* a0, const void* a1, int64_t lda, const void* b0, const void* b1, int64_t ldb,
+                     const void* bias0, const void* bias1, const uint8_t* active, void* c0, void* c1, int64_t ldc,
+                     float* partial, float* colsum, int64_t M, int64_t N, int64_t K, int dtype, void* stream) {
+  return linear_product(kind, a0, a1, lda, b0, b1, ldb, bias0, bias1, active, c0, c1, ldc, partial, colsum, M, N, K, dtype, stream, nullptr);
 }
 
 }  // extern "C"

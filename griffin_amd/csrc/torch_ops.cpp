@@ -2025,7 +2025,7 @@ Tensor linear_values(const Tensor& x, const Tensor& w, const MaybeTensor& b) {
 }
 
 // The whole block over sequences without gradients (griffin/griffin.py:459-528): projections, positions, convolution, RG-LRU
-// and gate, output projection in four launches.  Every token active: positions follow prev_pos (or are segment_pos);
+// and gate, output projection in three launches (four behind the BLAS library's products).  Every token active: positions follow prev_pos (or are segment_pos);
 // right-padded: flags, rows, active and the projections u, v as the caller has them from TokenFacts.  Returns (output, final
 // state, convolution state, last position); nothing where the kernels do not take the operands.
 std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
@@ -2068,14 +2068,22 @@ std::optional<std::tuple<Tensor, Tensor, Tensor, Tensor>> block_infer(
   uint8_t* flag_bytes = reinterpret_cast<uint8_t*>(s.raw());
   if (u.defined()) {
     u = aligned(u), v = aligned(v);
-  } else if (own) {
-    linear_forward(x, wx, bx, wy, by, Tensor(), up, vp);
-  } else {
+  } else if (!own) {
     u = at::linear(x, wx, bx), v = at::linear(x, wy, by);
   }
+  const bool projects = !u.defined() && !flags.defined();  // in one launch with the positions
+  if (!u.defined() && !projects) linear_forward(x, wx, bx, wy, by, Tensor(), up, vp);
   if (u.defined()) up = static_cast<char*>(ptr(u)), vp = static_cast<char*>(ptr(v));
   Tensor h_last = fresh({B, W}, at::kFloat, x), new_conv = fresh({B, K - 1, W}, dtype, x), last;
-  if (!flags.defined()) {
+  if (projects) {
+    uint8_t* bytes_of_flags = prev.defined() || seg.defined() ? flag_bytes : nullptr;
+    last = fresh({B}, at::kLong, x);
+    check(rglru_hip_block_project(ptr(x), ptr(wx), ptr(wy), ptr(bx), ptr(by), up, vp, iptr(prev), iptr(seg), bytes_of_flags,
+                                  static_cast<int64_t*>(last.data_ptr()), ws, B, T, D, W, nb, code, stream), "rglru_hip_block_project");
+    check(rglru_hip_block_infer_projected(up, W, vp, W, ptr(state), ptr(cw), ptr(cb), K, code, ptr(image), fptr(h0), bytes_of_flags,
+                                          gated, K > 1 ? ptr(new_conv) : nullptr, fptr(h_last), ws, B, T, W, nb, code, stream),
+          "rglru_hip_block_infer_projected");
+  } else if (!flags.defined()) {
     last = fresh({B}, at::kLong, x);
     check(rglru_hip_block_infer(up, W, vp, W, ptr(state), ptr(cw), ptr(cb), K, code, ptr(image), fptr(h0), iptr(prev), iptr(seg), flag_bytes, gated,
                                 K > 1 ? ptr(new_conv) : nullptr, fptr(h_last), static_cast<int64_t*>(last.data_ptr()), ws, B, T, W, nb, code, stream),

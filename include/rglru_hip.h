@@ -503,6 +503,17 @@ int rglru_hip_block_infer(const void* u, int64_t u_stride, const void* v, int64_
                           const void* prep, const float* h0, const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes,
                           void* gated, void* new_conv_state, float* h_last, int64_t* last_pos, void* ws,
                           int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
+/* The same call with the two input projections u = x w0^T + bias0, v = x w1^T + bias1 of x[B*T,D] in front of it (bf16, rows of whole
+ * 16-byte vectors): rglru_hip_block_project is one launch for both products, the positions and the clearing;
+ * rglru_hip_block_infer_projected the forward behind it (flag_bytes NULL where rglru_hip_block_project got neither positions). */
+int rglru_hip_block_project(const void* x, const void* w0, const void* w1, const void* bias0, const void* bias1, void* u, void* v,
+                            const int64_t* prev_pos, const int64_t* segment_pos, uint8_t* flag_bytes, int64_t* last_pos, void* ws,
+                            int64_t B, int64_t T, int64_t D, int64_t W, int64_t nb, int dtype, void* stream);
+int rglru_hip_block_infer_projected(const void* u, int64_t u_stride, const void* v, int64_t v_stride,
+                                    const void* conv_state, const void* taps, const void* conv_bias, int64_t K, int vec_dtype,
+                                    const void* prep, const float* h0, const uint8_t* flag_bytes, void* gated, void* new_conv_state,
+                                    float* h_last, void* ws, int64_t B, int64_t T, int64_t W, int64_t nb, int dtype, void* stream);
+
 
 /* Test hook: number of polls a wave may spend waiting for a neighbouring chunk's carry before it
  * gives up, records the failure in the workspace and finishes with unspecified results.  The

@@ -1298,3 +1298,62 @@ def test_block_inference_in_one_call_matches_layer_by_layer(B, T, D, W, nb, carr
     assert rel_err(got_cache.rnn_state, want_cache.rnn_state) < 1e-2
     assert torch.equal(got_cache.segment_position, want_cache.segment_position)
     assert rel_err(got_cache.conv_state.float(), want_cache.conv_state.float()) < 1e-2
+
+
+# one tile and the smallest width; rows that end inside tiles of 64; tiles of 128
+@pytest.mark.parametrize("B,T,D,W,nb", [(1, 1, 8, 96, 3), (9, 77, 72, 128, 2), (3, 1537, 136, 2048, 16)])
+@pytest.mark.parametrize("tokens", ["fresh", "continued", "positions"])
+def test_projections_carry_the_positions_of_an_inference_call(B, T, D, W, nb, tokens):
+    """rglru_hip_block_project: flag bytes and last positions for every kind of position, the products of rglru_hip_linear bit for bit, and a
+    workspace that held anything is cleared for the forward behind it."""
+    from griffin_amd import _lib
+
+    _say("projections with positions", B, T, D, W, nb, tokens)
+    lib, code = _lib.load(), _lib.RGLRU_BF16
+    gen = torch.Generator().manual_seed(11)
+    make = lambda *shape: torch.randn(*shape, generator=gen).to(torch.bfloat16).cuda()
+    x, w0, w1, b0, b1 = make(B, T, D), make(W, D), make(W, D), make(W), make(W)
+    prev = torch.tensor([-1, 0, 1, 2, 3, 2 ** 40, -2, -3, -2 ** 40])[:B].cuda() if tokens == "continued" else None
+    seg = torch.randint(-3, 6, (B, T), generator=gen).cuda() if tokens == "positions" else None
+    pos = seg if seg is not None else (prev[:, None] + 1 if prev is not None else 0) + torch.arange(T, device="cuda").repeat(B, 1)
+    bytes_ = lambda n: torch.full((n,), 0xff, dtype=torch.uint8, device="cuda")
+    ws, flags = bytes_(lib.rglru_hip_workspace_bytes(B, T, W, nb)), bytes_(B * T + 8)
+    last = torch.full((B + 1,), -7, device="cuda")
+    u, v, u2, v2 = (torch.full((B * T + 1, W), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(4))
+    at = lambda t: None if t is None else t.data_ptr()
+    stream = torch.cuda.current_stream().cuda_stream
+    held = None if tokens == "fresh" else at(flags)
+    _lib.check(lib.rglru_hip_block_project(at(x), at(w0), at(w1), at(b0), at(b1), at(u), at(v), at(prev), at(seg), held, at(last), at(ws), B, T, D,
+                                           W, nb, code, stream), "project")
+    _lib.check(lib.rglru_hip_linear(0, at(x), None, D, at(w0), at(w1), D, at(b0), at(b1), None, at(u2), at(v2), W, None, None, B * T, W, D, code,
+                                    stream), "linear")
+    torch.cuda.synchronize()
+    for got, want in ((u, u2), (v, v2)):
+        assert torch.equal(got[:-1], want[:-1]) and torch.isnan(got[-1]).all()
+    want = (pos == 0).to(torch.uint8) | ((3 - pos).clamp(0, 3) << 2).to(torch.uint8)
+    assert torch.equal(flags[:B * T].view(B, T), want) if held else (flags == 0xff).all()
+    assert (flags[B * T:] == 0xff).all() and torch.equal(last[:-1], pos[:, -1]) and int(last[-1]) == -7
+    # the forward behind it, against the one that launches its own positions
+    gates = [make(nb, W // nb, W // nb) * 0.1, make(nb, W // nb) * 0.1, make(nb, W // nb, W // nb) * 0.1, make(nb, W // nb) * 0.1]
+    a_param = torch.rand(W, generator=gen).to(torch.bfloat16).cuda()
+    prep = bytes_(lib.rglru_hip_prep_bytes(W, nb, code))
+    _lib.check(lib.rglru_hip_prepare(*(at(t) for t in gates), at(a_param), 8.0, W, nb, code, code, at(prep), stream), "prepare")
+    taps, bias, state, h0 = make(W, 4), make(W), make(B, 3, W), torch.randn(B, W, generator=gen).cuda()
+    results = []
+    for own in (True, False):
+        gated, new_state, h = (torch.full(s, float("nan"), dtype=t, device="cuda") for s, t in
+                               (((B, T, W), torch.bfloat16), ((B, 3, W), torch.bfloat16), ((B, W), torch.float32)))
+        common = (at(u), W, at(v), W, at(state), at(taps), at(bias), 4, code, at(prep), at(h0))
+        if own:
+            _lib.check(lib.rglru_hip_block_infer_projected(*common, held, at(gated), at(new_state), at(h), at(ws), B, T, W, nb, code, stream), "behind")
+        else:
+            again = bytes_(B * T)
+            _lib.check(lib.rglru_hip_block_infer(*common, at(prev), at(seg), at(again) if held else None, at(gated), at(new_state), at(h), at(last),
+                                                 at(ws), B, T, W, nb, code, stream), "infer")
+        torch.cuda.synchronize()
+        results.append((gated, new_state, h))
+    for got, want in zip(*results):
+        assert rel_err(got.float(), want.float()) < 4e-3      # one rounding to bf16; the order in which tiles pass the state may differ
+    # refused: no workspace, no place for the flags
+    refused = lambda *edit: lib.rglru_hip_block_project(at(x), at(w0), at(w1), at(b0), at(b1), at(u), at(v), None, *edit, B, T, D, W, nb, code, stream)
+    assert refused(None, None, at(last), None) != 0 and refused(at(pos.contiguous()), None, at(last), at(ws)) != 0
