@@ -54,8 +54,8 @@ template <typename IO> RGLRU_DEVICE auto buf_load_four(rsrc_t r, unsigned voff) 
   else return __builtin_bit_cast(io4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
 
-// How a product is cut up: edge of the square tiles, and workgroups that share a contraction.
-struct LinearPlan { int edge, splits; };
+// How a product is cut up: rows (and columns, where no others are given) of a tile, and workgroups that share a contraction.
+struct LinearPlan { int edge, splits, columns = 0; };
 
 // rglru_linear.hip: two products of one input, u and v, with the positions of an inference call
 int linear_pair_with_positions(const void* x, const void* w0, const void* w1, const void* bias0, const void* bias1, void* u, void* v, int64_t M,

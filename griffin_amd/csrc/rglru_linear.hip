@@ -8,13 +8,13 @@
 //
 // Why not the BLAS library alone: a call of it costs the host 17 us, seven calls of it are a third of the host time of a
 // training step of the block, which is what bounds such a step up to several thousand tokens; and it takes no row mask and
-// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 52 us against 63 us), so callers choose by the
+// returns no column sums.  For long products it is faster (16384 x 1024 x 768 twice in bf16: 57 us against 67 us), so callers choose by the
 // size of the product.
 //
 // Here: fp32, and the forward in bf16 (the gradients in bf16: rglru_linear16.hip).  A workgroup of four waves owns a BM x BN tile of C; K is
 // walked in slices of 128 bytes, one barrier a slice.  Where both operands
 // lie with their contraction index contiguous (forward) a slice goes from memory to LDS directly (DirectTile), one slice ahead
-// (128 x 128) or two (64 x 64).  Otherwise it goes through registers (requested one slice ahead) into one of two LDS buffers: an
+// or (64 x 64) two.  Otherwise it goes through registers (requested one slice ahead) into one of two LDS buffers: an
 // operand with its contraction index contiguous is read back as 16-byte rows (row stride 144 bytes: no bank conflicts); one that
 // lies the other way round is read element by element.
 // Edges of M, N and K are masked through the offsets of buffer loads, so any size works as long as rows are whole 16-byte
@@ -158,8 +158,9 @@ struct DirectTile {
   }
 };
 
-// DIRECT: both operands' rows are result indices and go to LDS directly (DirectTile).
-template <typename IO, bool TA, bool TB, int BM, int BN, bool DIRECT = !TA && !TB>
+// DIRECT: both operands' rows are result indices and go to LDS directly (DirectTile).  STAGES: slices of them in LDS; two and three workgroups
+// on a compute unit (64 x 64 with two or four slices: 11.8 and 10.2 us for 10).
+template <typename IO, bool TA, bool TB, int BM, int BN, int STAGES = BN == 64 ? 3 : 2, bool DIRECT = !TA && !TB>
 __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
@@ -169,8 +170,6 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   constexpr int MI = BM / 64, NI = BN / 64;                  // 32 x 32 accumulator tiles of a wave (2 x 2 waves)
   constexpr int kStageRow = BN / 2 + Tr::HW;                 // epilogue: the wave's half tile, row by row
   constexpr int kStage = 4 * (BM / 2) * kStageRow;
-  // two slices of 32 KB or three of 16 KB: two and three workgroups on a compute unit (64 x 64 with two or four slices: 11.8 and 10.2 us for 10)
-  constexpr int STAGES = BM == 128 ? 2 : 3;
   constexpr int kBuffers = DIRECT ? STAGES * (BM + BN) * BK : 2 * (TileA::kElems + TileB::kElems);
   __shared__ __attribute__((aligned(16))) IO lds[kBuffers > kStage ? kBuffers : kStage];
 
@@ -433,6 +432,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   wave_lds_fence();
   const rsrc_t rc = make_rsrc((IO*)p.c[problem] + item * p.c_step + (long long)m0 * p.ldc + n0, (unsigned)((long long)(m_left < BM ? m_left : BM) * p.ldc) * (unsigned)sizeof(IO));
   constexpr int VPR = (BN / 2) / Tr::HW, ROWS = 64 / VPR;
+  static_assert(64 % VPR == 0 && (BM / 2) % ROWS == 0, "whole rows an instruction");
 #pragma unroll
   for (int q = 0; q < (BM / 2) / ROWS; ++q) {
     const int m = q * ROWS + lane / VPR, cv = lane % VPR;
@@ -444,13 +444,18 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
   }
 }
 
-// How a product is cut up: tiles of 64 x 64, 128 x 128 (four times the work at half the reads) or, in bf16 gradients, 256 x 256.
-// Forward products: time goes in steps of one tile a compute unit, and steps of large tiles are four times as coarse.
-// In bf16 three small tiles on a compute unit take about as long as one large one, so the line lies where there are more than three.
-// On 256 compute units, us, small : large (small tiles in brackets), two problems unless said:
-//   1527 x 1024 x 768 (768) 11.2 : 10.6, 1655 (832) 14.3 : 11.0, 2331 16.5 : 14.3;  2039 x 768 x 1024 (768) 12.6 : 12.7, 2167 (816) 17.1 : 13.6;
-//   1883 x 768 x 1024 (720) 12.3 : 14.6;  one of 4087 x 768 x 1024 (768) 12.7 : 12.6, 4215 (792) 16.6 : 12.7;  503 x 2560 x 2560 (640) 37.4 :
-//   37.9, 631 (800) 47.0 : 38.1;  beyond, 4087 x 1024 x 768 (2048) 26.7 : 18.0, 5495 x 768 x 1024 (2064) 32.7 : 32.7
+// How a product is cut up.  Forward in bf16: the cheapest of four tiles by a model of the time in us, whose constants come from 100 sizes (60 to 16000
+// rows, 256 to 2560 columns, 128 to 2560 contraction indices, one and two problems) on 256 compute units, every product behind a kernel that
+// writes its input.  A launch takes `launch`; the units run their tiles in rounds of `per_cu`, each of which takes `start` and `slice[n - 1]` for
+// 64 contraction indices with n workgroups on a compute unit; and `moved` for every 256,000 operand lines that go to LDS (what the L2s
+// give).  It picks within 1 % (at most 10) of the best of the four, and is 3 % (-4 to 44) faster than two tiles (64 x 64 up to three to a compute unit,
+// else 128 x 128).  Kernel us, 64 x 64 : 128 x 64 : 128 x 128 : 192 x 128 (* taken, + by the two-tile rule), two problems unless said:
+//   600 x 1024 x 768 +9.1 : *9.0 : 14.2 : 15.6, 2331 18.8 : 18.7 : *+15.7 : 16.6, 4096 27.5 : 23.0 : *+17.8 : 21.2, 6216 38.8 : 34.6 : *+29.0 : 32.6;
+//   415 x 2048 x 1536 +17.4 : *14.6 : 23.2 : 25.4;  2668 x 768 x 512 14.0 : *10.0 : +11.2 : 12.4;  11981 x 384 x 384 20.2 : 18.4 : +18.7 : *14.5;
+//   one of 2331 x 768 x 1024 +11.0 : *10.4 : 15.7 : 18.0, 8704 28.4 : 24.2 : *+20.3 : 24.0;  8704 x 1024 x 768 28.9 : 26.7 : +26.2 : *21.4;
+//   7012 x 1280 x 1024 34.9 : 32.0 : +31.2 : *24.8;  4518 x 2560 x 512 29.7 : 24.6 : +22.1 : *17.9;  901 x 1536 x 2560 +21.4 : *19.3 : 34.9 : 37.4
+// 64 x 128 is 128 x 64 but for few rows (415 x 2048 x 1536 16.6); 192 x 192, 256 x 128 and 128 x 192 are the better ones nowhere by more than 4 %.
+// From six tiles of 128 x 128 to a compute unit on the largest are taken without the model (two of 16384 x 1024 x 768 109.8 : 92 : +75 : *66.7).
 // fp32 is bound by its MFMAs, and a small tile takes 1 / 4 of a large one and 6 % more, so the number of steps decides (M x 256 x 256, two
 // problems; steps small : large x 4):  8183 (4 : 4) 22.1 : 22.2, 8439 (5 : 8) 26.3 : 36.0, 14071 (7 : 8) 35.8 : 36.9, 15991 (8 : 8) 40.3 : 37.8, 16631
 // (9 : 12) 44.2 : 54.9, 24567 (12 : 12) 58.9 : 56.3;  input gradient 8183 (2 : 4) 24.6 : 40.8, 16375 (4 : 4)
@@ -458,6 +463,24 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
 // A weight gradient contracts over the tokens, so its tiles are few and its contraction long: it is split over workgroups (every split
 // costs a pass over the result in fp32).  In fp32 until there are about two to a compute unit, at least four slices each and at most
 // eight splits (two of 1024 x 768 at 2331 tokens 83 us in small tiles, 108 in large ones).
+struct ForwardCost { int rows, columns; unsigned per_cu; float launch, start, slice[3], moved; };
+static LinearPlan forward16_plan(int64_t M, int64_t N, int64_t K, int problems) {
+  static const ForwardCost costs[] = {{64, 64, 3, 2.23f, 2.12f, {0.219f, 0.329f, 0.398f}, 0.49f}, {128, 64, 2, 2.31f, 2.38f, {0.304f, 0.435f, 0.0f}, 0.48f},
+                                      {128, 128, 2, 1.68f, 3.30f, {0.644f, 0.789f, 0.0f}, 0.41f}, {192, 128, 2, 0.63f, 4.93f, {0.726f, 1.030f, 0.0f}, 0.67f}};
+  const float slices = (float)((K + 63) / 64);
+  const unsigned units = (unsigned)num_compute_units();
+  if (M * N * problems >= (int64_t)units * 6 * 128 * 128) return {192, 1, 128};
+  LinearPlan best = {64, 1, 64};
+  float least = 1e30f;
+  for (const ForwardCost& c : costs) {
+    const unsigned tiles = (unsigned)((M + c.rows - 1) / c.rows) * (unsigned)((N + c.columns - 1) / c.columns) * (unsigned)problems;
+    const unsigned each = (tiles + units - 1) / units, rounds = each / c.per_cu, rest = each - rounds * c.per_cu;
+    const float t = c.launch + (float)rounds * (c.start + c.slice[c.per_cu - 1] * slices) + (rest ? c.start + c.slice[rest - 1] * slices : 0.0f) +
+                    c.moved * (float)(c.rows + c.columns) * (1.0f / 256e3f) * (float)tiles * slices;
+    if (t < least) { least = t; best = {c.rows, 1, c.columns}; }
+  }
+  return best;
+}
 struct TileCost { int edge; unsigned per_cu; double start, slice[3]; };
 // Gradients in bf16: the cheapest by a model of the time in us.  A workgroup of a tile size takes `start` and `slice[n - 1]` for 64 contraction
 // indices with n of them on a compute unit; the units run their tiles in rounds of `per_cu`.  Constants from 64, 128 and 256 on
@@ -496,11 +519,12 @@ static LinearPlan linear16_plan(bool weight, int64_t M, int64_t N, int64_t K, in
   return best;
 }
 static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int problems, int segments, int dtype) {
-  if (dtype == RGLRU_BF16 && kind != RGLRU_LINEAR_FORWARD) return linear16_plan(kind == RGLRU_LINEAR_WEIGHT_GRAD, M, N, K, problems, segments);
+  if (dtype == RGLRU_BF16 && kind == RGLRU_LINEAR_FORWARD) return forward16_plan(M, N, K, problems);
+  if (dtype == RGLRU_BF16) return linear16_plan(kind == RGLRU_LINEAR_WEIGHT_GRAD, M, N, K, problems, segments);
   auto tiles = [&](int64_t edge) { return ((M + edge - 1) / edge) * ((N + edge - 1) / edge) * problems; };
   const int64_t units = num_compute_units();
   auto steps = [&](int64_t edge) { return (tiles(edge) + units - 1) / units; };
-  LinearPlan p = {(dtype == RGLRU_BF16 ? tiles(64) > 3 * units : tiles(128) > units && 106 * steps(64) >= 400 * steps(128)) ? 128 : 64, 1};
+  LinearPlan p = {tiles(128) > units && 106 * steps(64) >= 400 * steps(128) ? 128 : 64, 1};
   if (kind != RGLRU_LINEAR_WEIGHT_GRAD) return p;
   const int64_t slices = (K + 31) / 32;
   auto splits = [&](int64_t t) {
@@ -513,25 +537,29 @@ static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int pro
   return p;
 }
 
-template <typename IO, bool TA, bool TB>
-static void linear_launch(LinearArgs& a, bool large, hipStream_t s) {
-  const int edge = large ? 128 : 64;
-  a.tiles_m = (a.M + edge - 1) / edge;
-  a.tiles_n = (a.N + edge - 1) / edge;
+template <typename IO, bool TA, bool TB, int BM, int BN>
+static void linear_launch(LinearArgs& a, hipStream_t s) {
+  a.tiles_m = (a.M + BM - 1) / BM;
+  a.tiles_n = (a.N + BN - 1) / BN;
   a.total = a.tiles_m * a.tiles_n * a.problems * a.batch * a.splits;
-  const dim3 grid((unsigned)(8 * ((a.total + 7) / 8)));
-  if (large) hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 128, 128>), grid, dim3(kLinearThreads), 0, s, a);
-  else hipLaunchKernelGGL((linear_kernel<IO, TA, TB, 64, 64>), grid, dim3(kLinearThreads), 0, s, a);
+  hipLaunchKernelGGL((linear_kernel<IO, TA, TB, BM, BN>), dim3((unsigned)(8 * ((a.total + 7) / 8))), dim3(kLinearThreads), 0, s, a);
+}
+template <bool TA, bool TB>
+static void linear32_launch(LinearArgs& a, int edge, hipStream_t s) {
+  edge > 64 ? linear_launch<float, TA, TB, 128, 128>(a, s) : linear_launch<float, TA, TB, 64, 64>(a, s);
 }
 
-static void linear_launch(LinearArgs& a, int kind, int edge, int dtype, hipStream_t s) {
+static void linear_launch(LinearArgs& a, int kind, LinearPlan plan, int dtype, hipStream_t s) {
   if (dtype == RGLRU_BF16) {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<__bf16, false, false>(a, edge > 64, s);
-    else linear16_launch(a, kind, edge, s);
+    if (kind != RGLRU_LINEAR_FORWARD) linear16_launch(a, kind, plan.edge, s);
+    else if (plan.edge == 192) linear_launch<__bf16, false, false, 192, 128>(a, s);
+    else if (plan.edge == 64) linear_launch<__bf16, false, false, 64, 64>(a, s);
+    else if (plan.columns == 64) linear_launch<__bf16, false, false, 128, 64>(a, s);
+    else linear_launch<__bf16, false, false, 128, 128>(a, s);
   } else {
-    if (kind == RGLRU_LINEAR_FORWARD) linear_launch<float, false, false>(a, edge > 64, s);
-    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear_launch<float, false, true>(a, edge > 64, s);
-    else linear_launch<float, true, true>(a, edge > 64, s);
+    if (kind == RGLRU_LINEAR_FORWARD) linear32_launch<false, false>(a, plan.edge, s);
+    else if (kind == RGLRU_LINEAR_INPUT_GRAD) linear32_launch<false, true>(a, plan.edge, s);
+    else linear32_launch<true, true>(a, plan.edge, s);
   }
 }
 
@@ -558,7 +586,7 @@ int gate_pre_product(const void* x, const void* wg, void* pre, long long N, cons
   a.lda = g.W; a.ldb = g.bwp; a.ldc = 2 * g.bw; a.a_step = g.bw; a.b_step = g.bwp * g.bwp; a.c_step = N * 2 * g.bw;
   a.batch = (int)g.nb; a.problems = 2; a.segments = 1; a.splits = 1;
   a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
-  linear_launch(a, RGLRU_LINEAR_FORWARD, batch_large(g, N, 2) ? 128 : 64, RGLRU_BF16, s);
+  linear_launch(a, RGLRU_LINEAR_FORWARD, {batch_large(g, N, 2) ? 128 : 64, 1}, RGLRU_BF16, s);
   return check_launch("gate pre-activations");
 }
 
@@ -571,7 +599,7 @@ int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long lo
   a.lda = du_ld; a.ldb = g.bwp; a.ldc = g.W; a.a_step = du_blk; a.b_step = g.bwp * g.bwp; a.c_step = g.bw;
   a.batch = (int)g.nb; a.problems = 1; a.segments = 2; a.splits = 1; a.accumulate = 1;
   a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
-  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, batch_large(g, N, 1) ? 128 : 64, dtype, s);
+  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, {batch_large(g, N, 1) ? 128 : 64, 1}, dtype, s);
   return check_launch("gate input gradient");
 }
 
@@ -585,7 +613,7 @@ int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long l
   a.M = a.N = (int)g.bw; a.K = (int)N;
   const long long bk = dtype == RGLRU_BF16 ? 64 : 32;
   a.k_per_split = (int)(((N + splits - 1) / splits + bk - 1) / bk * bk);
-  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, batch_large(g, g.bw, 2 * splits) ? 128 : 64, dtype, s);
+  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, {batch_large(g, g.bw, 2 * splits) ? 128 : 64, 1}, dtype, s);
   return check_launch("gate weight gradients");
 }
 
@@ -626,7 +654,7 @@ static int linear_product(int kind, const void* a0, const void* a1, int64_t lda,
   a.k_per_split = (int)(((K + a.splits - 1) / a.splits + bk - 1) / bk * bk);
   if (positions) a.positions = *positions;
   hipStream_t s = (hipStream_t)stream;
-  linear_launch(a, kind, plan.edge, dtype, s);
+  linear_launch(a, kind, plan, dtype, s);
   return check_launch("linear");
 }
 

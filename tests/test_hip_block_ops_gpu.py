@@ -1357,3 +1357,38 @@ def test_projections_carry_the_positions_of_an_inference_call(B, T, D, W, nb, to
     # refused: no workspace, no place for the flags
     refused = lambda *edit: lib.rglru_hip_block_project(at(x), at(w0), at(w1), at(b0), at(b1), at(u), at(v), None, *edit, B, T, D, W, nb, code, stream)
     assert refused(None, None, at(last), None) != 0 and refused(at(pos.contiguous()), None, at(last), at(ws)) != 0
+
+
+# On 256 compute units, tiles of 64 x 64, 128 x 64, 128 x 128 and 192 x 128; no edge is a whole tile or slice of them
+@pytest.mark.parametrize("pair,M,N,K", [(1, 700, 1016, 776), (2, 777, 1016, 776), (1, 2331, 776, 1000), (2, 2331, 1016, 776), (1, 8200, 1016, 776), (2, 6000, 1000, 264), (2, 14000, 1016, 72)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_forward_products_in_every_tile_read_only_their_operands(pair, M, N, K, masked):
+    """bf16 forward products against fp64, with operands inside larger tensors of NaN; biases on and off the boundaries of vectors; masked rows."""
+    from griffin_amd import _lib
+
+    _say("forward products", pair, M, N, K, masked)
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    nan = lambda *shape: torch.full(shape, float("nan"), dtype=torch.bfloat16, device="cuda")
+    x, w, c, bias = nan(M + 2, K + 24), nan(pair, N + 2, K + 16), nan(pair, M + 2, N + 24), nan(pair, N + 11)
+    x[1:-1, 8:-16] = torch.randn(M, K, generator=gen, device="cuda")
+    w[:, 1:-1, 8:-8] = torch.randn(pair, N, K, generator=gen, device="cuda")
+    starts = (8, 3)
+    for i in range(pair):
+        bias[i, starts[i]:starts[i] + N] = torch.randn(N, generator=gen, device="cuda")
+    keep = torch.rand(M, generator=gen, device="cuda") < 0.6 if masked else torch.ones(M, dtype=torch.bool, device="cuda")
+    active = keep.to(torch.uint8) if masked else None
+    at = lambda t: None if t is None else t.data_ptr()
+    second = lambda t: at(t) if pair == 2 else None
+    _lib.check(_lib.load().rglru_hip_linear(0, at(x[1, 8:]), None, x.size(1), at(w[0, 1, 8:]), second(w[-1, 1, 8:]), w.size(2), at(bias[0, 8:]), second(bias[-1, 3:]),
+                                            at(active), at(c[0, 1, 8:]), second(c[-1, 1, 8:]), c.size(2), None, None, M, N, K, _lib.RGLRU_BF16,
+                                            torch.cuda.current_stream().cuda_stream), "linear")
+    torch.cuda.synchronize()
+    xs = x[1:-1, 8:-16].double()
+    for i in range(pair):
+        ws, b = w[i, 1:-1, 8:-8].double(), bias[i, starts[i]:starts[i] + N].double()
+        want = (xs @ ws.t() + b) * keep[:, None]
+        size = xs.abs() @ ws.abs().t() + b.abs()
+        got = c[i, 1:-1, 8:-16].double()
+        # rounding of the result, then K additions in fp32
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + (K + 2) * 2.0 ** -24 * size).all()
+        assert torch.isnan(c[i, 0]).all() and torch.isnan(c[i, -1]).all() and torch.isnan(c[i, :, :8]).all() and torch.isnan(c[i, :, -16:]).all()
