@@ -226,10 +226,8 @@ int launch_gate_gemms(const void* x, const void* du_a, const void* du_x, long lo
                       const void* wg, const void* w2t, void* dx, float* dw_partial, long long N, const Geometry& g, int dtype,
                       int n_split, hipStream_t s) {
   // B4 T1024 W1024 in fp32 (64-wide blocks): 27 + 56 us in the kernels of this file, latency of the operands' loads
-  if (gate_products_cover(g, dtype, {x, du_a, du_x, wg, dx}, {g.W, du_ld}) && du_blk % (dtype == RGLRU_BF16 ? 8 : 4) == 0) {
-    const int rc = gate_input_grad(du_a, du_x, du_ld, du_blk, wg, dx, N, g, dtype, s);
-    return rc ? rc : gate_weight_grad(du_a, du_x, du_ld, du_blk, x, dw_partial, n_split, N, g, dtype, s);
-  }
+  if (gate_products_cover(g, dtype, {x, du_a, du_x, wg, dx}, {g.W, du_ld}) && du_blk % (dtype == RGLRU_BF16 ? 8 : 4) == 0)
+    return gate_grads(x, du_a, du_x, du_ld, du_blk, wg, dx, dw_partial, n_split, N, g, dtype, s);
   GateGemmArgs a;
   memset(&a, 0, sizeof(a));
   a.x = x; a.du_a = du_a; a.du_x = du_x; a.w2t = w2t; a.dx = dx; a.dw_partial = dw_partial;

@@ -38,12 +38,10 @@ int launch_gate_gemms(const void* x, const void* du_a, const void* du_x, long lo
 bool gate_products_cover(const Geometry& g, int dtype, std::initializer_list<const void*> tensors, std::initializer_list<long long> strides);
 // pre[k][n][g bw + o] = sum_j x[n, k bw + j] W_g[k][o][j] (bf16)
 int gate_pre_product(const void* x, const void* wg, void* pre, long long N, const Geometry& g, hipStream_t s);
-// dx[n, k bw + j] += sum over gates and o of du_g[n, k, o] W_g[k][o][j];  du_g[n, k, o] at du_g + k du_blk + n du_ld + o
-int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, long long N,
-                    const Geometry& g, int dtype, hipStream_t s);
-// partial[split][k][g][o][j] (blocks of bwp x bwp, the padding is not written) = sum over the split's n of du_g[n, k, o] x[n, k bw + j]
-int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* x, float* partial, int splits,
-                     long long N, const Geometry& g, int dtype, hipStream_t s);
+// dx[n, k bw + j] += sum over gates and o of du_g[n, k, o] W_g[k][o][j], and partial[split][k][g][o][j] (blocks of bwp x bwp, the padding is not
+// written) = sum over the split's n of du_g[n, k, o] x[n, k bw + j];  du_g[n, k, o] at du_g + k du_blk + n du_ld + o
+int gate_grads(const void* x, const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, float* partial, int splits,
+               long long N, const Geometry& g, int dtype, hipStream_t s);
 
 // The same for two ranges in one launch.
 static __global__ void clear_two_kernel(unsigned* p0, long long n0, unsigned* p1, long long n1) {

@@ -161,29 +161,28 @@ struct DirectTile {
 // DIRECT: both operands' rows are result indices and go to LDS directly (DirectTile).  STAGES: slices of them in LDS; two and three workgroups
 // on a compute unit (64 x 64 with two or four slices: 11.8 and 10.2 us for 10).
 template <typename IO, bool TA, bool TB, int BM, int BN, int STAGES = BN == 64 ? 3 : 2, bool DIRECT = !TA && !TB>
-__global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
+struct LinearTile {
   typedef Io<IO> Tr;
   typedef typename Tr::Frag Frag;
   typedef OperandTile<IO, TA, BM, kLinearThreads> TileA;
   typedef OperandTile<IO, TB, BN, kLinearThreads> TileB;
-  constexpr int BK = TileA::BK, KGS = BK / Tr::KG;
-  constexpr int MI = BM / 64, NI = BN / 64;                  // 32 x 32 accumulator tiles of a wave (2 x 2 waves)
-  constexpr int kStageRow = BN / 2 + Tr::HW;                 // epilogue: the wave's half tile, row by row
-  constexpr int kStage = 4 * (BM / 2) * kStageRow;
-  constexpr int kBuffers = DIRECT ? STAGES * (BM + BN) * BK : 2 * (TileA::kElems + TileB::kElems);
-  __shared__ __attribute__((aligned(16))) IO lds[kBuffers > kStage ? kBuffers : kStage];
+  static constexpr int BK = TileA::BK, KGS = BK / Tr::KG;
+  static constexpr int MI = BM / 64, NI = BN / 64;           // 32 x 32 accumulator tiles of a wave (2 x 2 waves)
+  static constexpr int kStageRow = BN / 2 + Tr::HW;          // epilogue: the wave's half tile, row by row
+  static constexpr int kStage = 4 * (BM / 2) * kStageRow;
+  static constexpr int kBuffers = DIRECT ? STAGES * (BM + BN) * BK : 2 * (TileA::kElems + TileB::kElems);
+  static constexpr int kElems = kBuffers > kStage ? kBuffers : kStage;         // of the workgroup's LDS
 
+  // The tile of workgroup `block` of the product.
+  static RGLRU_DEVICE void run(const LinearArgs& p, unsigned block, IO* lds) {
   const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
-  if constexpr (DIRECT && sizeof(IO) == 2) {
-    if (p.positions.B > 0) token_positions(p.positions, (long long)blockIdx.x * kLinearThreads + threadIdx.x, (long long)gridDim.x * kLinearThreads);
-  }
   // Workgroups go to the eight XCDs round-robin; each XCD gets a contiguous run of tiles (columns fastest), so that
   // the rows they share come from memory once and the weights stay in its L2.
   const int per_xcd = (p.total + 7) >> 3;
-  int t = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per_xcd || t >= p.total) return;
+  int t = (block & 7) * per_xcd + (block >> 3);
+  if ((int)(block >> 3) >= per_xcd || t >= p.total) return;
   const int tn = t % p.tiles_n; t /= p.tiles_n;
   const int problem = t % p.problems; t /= p.problems;
   const int tm = t % p.tiles_m; t /= p.tiles_m;
@@ -389,7 +388,7 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     // through LDS like the result: stored from the accumulators, a row of the wave's tile is 32 bytes an instruction (two weight
     // gradients of 2048 x 1024 x 768, when bf16 ran here: 45 us that way, 42 element by element, 41 like this)
     constexpr int kRow = BN / 2 + 4;
-    static_assert(4 * (BM / 2) * kRow * 4 <= (int)sizeof(lds), "the fp32 tile fits where the slices were");
+    static_assert(4 * (BM / 2) * kRow * 4 <= kElems * (int)sizeof(IO), "the fp32 tile fits where the slices were");
     float* stage = reinterpret_cast<float*>(lds) + wave * (BM / 2) * kRow;
 #pragma unroll
     for (int j = 0; j < NI; ++j)
@@ -442,6 +441,28 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
     const unsigned off = n < n_left && row < m_left ? ((unsigned)row * (unsigned)p.ldc + (unsigned)n) * (unsigned)sizeof(IO) : kOutOfRange;
     buf_store_b128<kWriteThrough>(__builtin_bit_cast(i32x4, f), rc, off);
   }
+  }
+};
+
+template <typename IO, bool TA, bool TB, int BM, int BN>
+__global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p) {
+  typedef LinearTile<IO, TA, TB, BM, BN> Tile;
+  __shared__ __attribute__((aligned(16))) IO lds[Tile::kElems];
+  if constexpr (!TA && !TB && sizeof(IO) == 2) {
+    if (p.positions.B > 0) token_positions(p.positions, (long long)blockIdx.x * kLinearThreads + threadIdx.x, (long long)gridDim.x * kLinearThreads);
+  }
+  Tile::run(p, blockIdx.x, lds);
+}
+
+// The weight and input gradients of the gates' products in fp32, in small tiles, in one launch: neither reads what the other writes.  The
+// weight gradients' workgroups have twice the slices and go first.  Steps of the layer in fp32, two launches and one, us: B4 T1024 W1024 (16 gate
+// blocks) 97.9 and 95.8, B8 T2048 338 and 324, B2 T256 W256, which the host bounds, 54.6 and 52.7.
+__global__ __launch_bounds__(kLinearThreads, 2) void gate_grads_kernel(LinearArgs weights, LinearArgs input, unsigned first) {
+  typedef LinearTile<float, true, true, 64, 64> Weights;
+  typedef LinearTile<float, false, true, 64, 64> Input;
+  __shared__ __attribute__((aligned(16))) float lds[Weights::kElems > Input::kElems ? Weights::kElems : Input::kElems];
+  if (blockIdx.x < first) Weights::run(weights, blockIdx.x, lds);
+  else Input::run(input, blockIdx.x - first, lds);
 }
 
 // How a product is cut up.  Forward in bf16: the cheapest of four tiles by a model of the time in us, whose constants come from 100 sizes (60 to 16000
@@ -537,12 +558,17 @@ static LinearPlan linear_plan(int kind, int64_t M, int64_t N, int64_t K, int pro
   return p;
 }
 
-template <typename IO, bool TA, bool TB, int BM, int BN>
-static void linear_launch(LinearArgs& a, hipStream_t s) {
+template <int BM, int BN>
+static unsigned linear_grid(LinearArgs& a) {
   a.tiles_m = (a.M + BM - 1) / BM;
   a.tiles_n = (a.N + BN - 1) / BN;
   a.total = a.tiles_m * a.tiles_n * a.problems * a.batch * a.splits;
-  hipLaunchKernelGGL((linear_kernel<IO, TA, TB, BM, BN>), dim3((unsigned)(8 * ((a.total + 7) / 8))), dim3(kLinearThreads), 0, s, a);
+  return (unsigned)(8 * ((a.total + 7) / 8));
+}
+template <typename IO, bool TA, bool TB, int BM, int BN>
+static void linear_launch(LinearArgs& a, hipStream_t s) {
+  const unsigned grid = linear_grid<BM, BN>(a);
+  hipLaunchKernelGGL((linear_kernel<IO, TA, TB, BM, BN>), dim3(grid), dim3(kLinearThreads), 0, s, a);
 }
 template <bool TA, bool TB>
 static void linear32_launch(LinearArgs& a, int edge, hipStream_t s) {
@@ -590,31 +616,31 @@ int gate_pre_product(const void* x, const void* wg, void* pre, long long N, cons
   return check_launch("gate pre-activations");
 }
 
-int gate_input_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, long long N,
-                    const Geometry& g, int dtype, hipStream_t s) {
-  LinearArgs a;
-  memset(&a, 0, sizeof(a));
+int gate_grads(const void* x, const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* wg, void* dx, float* partial, int splits,
+               long long N, const Geometry& g, int dtype, hipStream_t s) {
+  LinearArgs in, w;
+  memset(&in, 0, sizeof(in));
   const long long gate = g.nb * g.bwp * g.bwp;
-  a.a[0] = du_a; a.a[1] = du_x; a.b[0] = wg; a.b[1] = (const char*)wg + gate * (dtype == RGLRU_BF16 ? 2 : 4); a.c[0] = dx;
-  a.lda = du_ld; a.ldb = g.bwp; a.ldc = g.W; a.a_step = du_blk; a.b_step = g.bwp * g.bwp; a.c_step = g.bw;
-  a.batch = (int)g.nb; a.problems = 1; a.segments = 2; a.splits = 1; a.accumulate = 1;
-  a.M = (int)N; a.N = a.K = a.k_per_split = (int)g.bw;
-  linear_launch(a, RGLRU_LINEAR_INPUT_GRAD, {batch_large(g, N, 1) ? 128 : 64, 1}, dtype, s);
-  return check_launch("gate input gradient");
-}
-
-int gate_weight_grad(const void* du_a, const void* du_x, long long du_ld, long long du_blk, const void* x, float* partial, int splits,
-                     long long N, const Geometry& g, int dtype, hipStream_t s) {
-  LinearArgs a;
-  memset(&a, 0, sizeof(a));
-  a.a[0] = du_a; a.a[1] = du_x; a.b[0] = x; a.partial = partial; a.partial_ld = (int)g.bwp;
-  a.lda = du_ld; a.ldb = g.W; a.a_step = du_blk; a.b_step = g.bw;
-  a.batch = (int)g.nb; a.problems = 2; a.segments = 1; a.splits = splits;
-  a.M = a.N = (int)g.bw; a.K = (int)N;
+  in.a[0] = du_a; in.a[1] = du_x; in.b[0] = wg; in.b[1] = (const char*)wg + gate * (dtype == RGLRU_BF16 ? 2 : 4); in.c[0] = dx;
+  in.lda = du_ld; in.ldb = g.bwp; in.ldc = g.W; in.a_step = du_blk; in.b_step = g.bwp * g.bwp; in.c_step = g.bw;
+  in.batch = (int)g.nb; in.problems = 1; in.segments = 2; in.splits = 1; in.accumulate = 1;
+  in.M = (int)N; in.N = in.K = in.k_per_split = (int)g.bw;
+  memset(&w, 0, sizeof(w));
+  w.a[0] = du_a; w.a[1] = du_x; w.b[0] = x; w.partial = partial; w.partial_ld = (int)g.bwp;
+  w.lda = du_ld; w.ldb = g.W; w.a_step = du_blk; w.b_step = g.bw;
+  w.batch = (int)g.nb; w.problems = 2; w.segments = 1; w.splits = splits;
+  w.M = w.N = (int)g.bw; w.K = (int)N;
   const long long bk = dtype == RGLRU_BF16 ? 64 : 32;
-  a.k_per_split = (int)(((N + splits - 1) / splits + bk - 1) / bk * bk);
-  linear_launch(a, RGLRU_LINEAR_WEIGHT_GRAD, {batch_large(g, g.bw, 2 * splits) ? 128 : 64, 1}, dtype, s);
-  return check_launch("gate weight gradients");
+  w.k_per_split = (int)(((N + splits - 1) / splits + bk - 1) / bk * bk);
+  const bool large_in = batch_large(g, N, 1), large_w = batch_large(g, g.bw, 2 * splits);
+  if (dtype == RGLRU_F32 && !large_in && !large_w) {
+    const unsigned first = linear_grid<64, 64>(w), second = linear_grid<64, 64>(in);
+    hipLaunchKernelGGL(gate_grads_kernel, dim3(first + second), dim3(kLinearThreads), 0, s, w, in, first);
+    return check_launch("gate gradients");
+  }
+  linear_launch(in, RGLRU_LINEAR_INPUT_GRAD, {large_in ? 128 : 64, 1}, dtype, s);
+  linear_launch(w, RGLRU_LINEAR_WEIGHT_GRAD, {large_w ? 128 : 64, 1}, dtype, s);
+  return check_launch("gate gradients");
 }
 
 }  // namespace rglru

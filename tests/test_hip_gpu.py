@@ -1178,3 +1178,17 @@ def test_scan_op_gradients_below_and_above_the_cache(B, W, once, stream):
     grads = torch.autograd.grad(h, leaves, dh.cuda())
     errs = [rel_err(h, want[0])] + [rel_err(g, w) for g, w in zip(grads, want[1:])]
     assert max(errs) < FP32_TOL, errs
+
+
+# blocks of one and two small tiles, whole and not, and of a large one (two launches); tokens about a tile, a slice and a split
+@pytest.mark.parametrize("bw,nb", [(8, 5), (32, 4), (64, 3), (96, 2), (136, 2)])
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 63), (2, 33), (5, 77), (1, 2111)])
+def test_gate_gradients_in_fp32_at_the_edges_of_their_tiles(bw, nb, B, T):
+    """Both products of the gate gradients, one launch where the tiles are small, against the oracle in fp64."""
+    _say("gate gradients", bw, nb, B, T)
+    case = orc.make_case(B, T, bw * nb, nb, seed=bw + T, h0_std=0.5, bias_std=0.5)
+    y, _, grads = hip_run(case, torch.float32)
+    ry, _, rgrads = oracle_run(case, torch.float64)
+    assert rel_err(y, ry) < FP32_TOL
+    for name, g in grads.items():
+        assert rel_err(g, rgrads[name]) < FP32_TOL, name
