@@ -848,7 +848,8 @@ static int build_prep_args(const void* w_a, const void* b_a, const void* w_x, co
 
 static int launch_prepare(const PrepArgs& a, int dtype, void* stream) {
   const long long cells = (long long)a.nb * a.bwp * a.bwp;
-  long long total = a.vec_ok ? 4 * cells / 8 + a.Wp : 4 * cells + a.Wp;
+  const long long turned = (long long)a.nb * ((a.bw + 63) / 64) * ((a.bw + 31) / 32) * 64;
+  long long total = a.vec_ok ? turned + 2 * cells / 8 + a.Wp : 4 * cells + a.Wp;
   if (a.clear_n > total) total = a.clear_n;
   if (2 * a.stack_n > total) total = 2 * a.stack_n;
   int blocks = (int)((total + 255) / 256); if (blocks > 2048) blocks = 2048;

@@ -1192,3 +1192,26 @@ def test_gate_gradients_in_fp32_at_the_edges_of_their_tiles(bw, nb, B, T):
     assert rel_err(y, ry) < FP32_TOL
     for name, g in grads.items():
         assert rel_err(g, rgrads[name]) < FP32_TOL, name
+
+
+@pytest.mark.parametrize("bw,nb", [(32, 3), (64, 2), (96, 2), (160, 1), (320, 2)])
+def test_prepared_image_does_not_depend_on_the_alignment_of_the_weights(bw, nb):
+    """Weights on a 16-byte boundary are copied and turned by vectors, others element by element: the same image, byte for byte."""
+    from griffin_amd import _lib
+
+    lib, W = _lib.load(), bw * nb
+    _say("image", bw, nb)
+    gen = torch.Generator().manual_seed(bw)
+    stream = torch.cuda.current_stream().cuda_stream
+    wide = torch.randn(2, nb * bw * bw + 8, generator=gen).bfloat16().cuda()
+    b_a, b_x, lam = (torch.randn(W, generator=gen).cuda() for _ in range(3))
+    images = []
+    for first in (0, 1):
+        w = torch.empty_like(wide)
+        w[:, first:first + nb * bw * bw] = wide[:, :nb * bw * bw]
+        image = torch.full((lib.rglru_hip_prep_bytes(W, nb, _lib.RGLRU_BF16),), 0x5A, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.rglru_hip_prepare(w[0, first:].data_ptr(), b_a.data_ptr(), w[1, first:].data_ptr(), b_x.data_ptr(), lam.data_ptr(), 8.0,
+                                         W, nb, _lib.RGLRU_BF16, _lib.RGLRU_F32, image.data_ptr(), stream), "prepare")
+        torch.cuda.synchronize()
+        images.append(image)
+    assert torch.equal(*images) and not (images[0] == 0x5A).all()
