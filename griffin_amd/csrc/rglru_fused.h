@@ -24,7 +24,7 @@ struct PrepArgs {
   const void* w_a; const void* w_x; const void* b_a; const void* b_x; const void* lambda;
   void* wg; float* bias; float* sp; float* cs; float* dsp; void* w2t;
   int W, nb, bw, bwp, Wp, vec_dtype;
-  int vec_ok;                          // 16-bit weights, unpadded blocks, 16-byte aligned: eight elements per thread
+  int vec_ok;                          // 16-bit weights, blocks of a multiple of 8 channels, 16-byte aligned: eight elements per thread
   int rows_ok;                         // 16-bit weights whose rows are whole 16-byte vectors (blocks of a multiple of 8 channels)
   float c;
   uint4* clear; long long clear_n;     // optional: a workspace region to zero in the same launch
@@ -71,12 +71,13 @@ __global__ void prepare_kernel(PrepArgs p) {
   for (long long z = i; z < p.clear_n; z += stride) p.clear[z] = make_uint4(0u, 0u, 0u, 0u);
   for (long long z = i; z < 2 * p.stack_n; z += stride) p.stack_to[z] = z < p.stack_n ? p.stack_from[0][z] : p.stack_from[1][z - p.stack_n];
   if (sizeof(IO) == 2 && p.vec_ok) {
-    // wg is a copy of [w_a ; w_x], 16 bytes a thread.  w2t[k][j][2 o + gate] is the transpose of both: a thread turns eight j of four o, and the
+    // wg is a copy of [w_a ; w_x], 16 bytes a thread; the padding is zero in both.  w2t[k][j][2 o + gate] is the transpose of both: a thread turns eight j of four o, and the
     // lanes of a wave cover 64 j x 32 o, so that both sides move in runs of 128 bytes.  With a thread a vector of w2t, its eight elements gathered
     // one by one, W2560 in 8 gate blocks took 15.5 us with the clearing for B1 T32768, so 10.9; a training step of B2 T2048 W2560 167 and 160.
+    const int row8 = p.bwp / 8, tiles_j = (p.bwp + 63) / 64, tiles_o = p.bwp / 32;             // row8: vectors per row of wg
     const long long per_gate8 = per_gate / 8, n_w8 = 2 * per_gate8;
-    const int tiles_j = (p.bw + 63) / 64, tiles_o = (p.bw + 31) / 32, row8 = 2 * p.bw / 8;      // row8: vectors per row j of w2t
     const long long turned = (long long)p.nb * tiles_j * tiles_o * 64;
+    const bf16x8 zero = Io<__bf16>::zero();
     for (; i < turned + n_w8 + p.Wp; i += stride) {
       if (i < turned) {
         const int lane = (int)i & 63;
@@ -84,23 +85,29 @@ __global__ void prepare_kernel(PrepArgs p) {
         const int to = (int)(tile % tiles_o); tile /= tiles_o;
         const int tj = (int)(tile % tiles_j), k = (int)(tile / tiles_j);
         const int j = tj * 64 + (lane >> 3) * 8, o = to * 32 + (lane & 7) * 4;
-        if (j >= p.bw || o >= p.bw) continue;
-        const long long at = ((long long)k * p.bw + o) * p.bw + j;                    // W[k][o][j]
+        if (j >= p.bwp) continue;
+        const bool there = j < p.bw && o < p.bw;                                      // whole vectors: bw is a multiple of 8
+        const long long at = there ? ((long long)k * p.bw + o) * p.bw + j : 0;        // W[k][o][j]
+        const int next = there ? p.bw : 0;
         bf16x8 a[4], x[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          a[u] = *(const bf16x8*)((const __bf16*)p.w_a + at + (long long)u * p.bw);
-          x[u] = *(const bf16x8*)((const __bf16*)p.w_x + at + (long long)u * p.bw);
+          a[u] = *(const bf16x8*)((const __bf16*)p.w_a + at + (long long)u * next);
+          x[u] = *(const bf16x8*)((const __bf16*)p.w_x + at + (long long)u * next);
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const bf16x8 v = {a[0][e], x[0][e], a[1][e], x[1][e], a[2][e], x[2][e], a[3][e], x[3][e]};
-          ((bf16x8*)p.w2t)[((long long)k * p.bw + j + e) * row8 + o / 4] = v;
+          ((bf16x8*)p.w2t)[((long long)k * p.bwp + j + e) * (2 * row8) + o / 4] = there ? v : zero;
         }
       } else if (i < turned + n_w8) {
         const long long e8 = i - turned;
         const int gate = e8 >= per_gate8;
-        ((uint4*)p.wg)[e8] = ((const uint4*)(gate ? p.w_x : p.w_a))[e8 - gate * per_gate8];
+        const unsigned rem = (unsigned)(e8 - gate * per_gate8), row = rem / (unsigned)row8, j = (rem - row * (unsigned)row8) * 8u;
+        const unsigned k = row / (unsigned)p.bwp, o = row - k * (unsigned)p.bwp;
+        const bool there = (int)o < p.bw && (int)j < p.bw;
+        const bf16x8 v = *(const bf16x8*)((const __bf16*)(gate ? p.w_x : p.w_a) + (there ? ((long long)k * p.bw + o) * p.bw + j : 0));
+        ((bf16x8*)p.wg)[e8] = there ? v : zero;
       } else {
         prepare_channel(p, (int)(i - turned - n_w8));
       }

@@ -839,8 +839,9 @@ static int build_prep_args(const void* w_a, const void* b_a, const void* w_x, co
   a.w2t = pb + pl.w2t;
   a.W = (int)W; a.nb = (int)nb; a.bw = (int)g.bw; a.bwp = (int)g.bwp; a.Wp = (int)g.Wp; a.c = c;
   a.clear = (uint4*)clear; a.clear_n = (long long)(clear_bytes / 16);
+  const long long cells8 = (long long)g.nb * g.bwp * g.bwp / 8;
   a.stack_from[0] = a.stack_from[1] = nullptr; a.stack_to = nullptr; a.stack_n = 0;
-  a.vec_ok = dtype == RGLRU_BF16 && g.bw == g.bwp && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0 &&
+  a.vec_ok = dtype == RGLRU_BF16 && g.bw % 8 == 0 && g.bwp % 32 == 0 && cells8 < (1ll << 31) && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0 &&
              (uintptr_t)a.wg % 16 == 0 && (uintptr_t)a.w2t % 16 == 0;
   a.rows_ok = dtype == RGLRU_BF16 && g.bw % 8 == 0 && (uintptr_t)w_a % 16 == 0 && (uintptr_t)w_x % 16 == 0;
   return RGLRU_OK;
@@ -848,7 +849,7 @@ static int build_prep_args(const void* w_a, const void* b_a, const void* w_x, co
 
 static int launch_prepare(const PrepArgs& a, int dtype, void* stream) {
   const long long cells = (long long)a.nb * a.bwp * a.bwp;
-  const long long turned = (long long)a.nb * ((a.bw + 63) / 64) * ((a.bw + 31) / 32) * 64;
+  const long long turned = (long long)a.nb * ((a.bwp + 63) / 64) * (a.bwp / 32) * 64;
   long long total = a.vec_ok ? turned + 2 * cells / 8 + a.Wp : 4 * cells + a.Wp;
   if (a.clear_n > total) total = a.clear_n;
   if (2 * a.stack_n > total) total = 2 * a.stack_n;

@@ -1194,7 +1194,7 @@ def test_gate_gradients_in_fp32_at_the_edges_of_their_tiles(bw, nb, B, T):
         assert rel_err(g, rgrads[name]) < FP32_TOL, name
 
 
-@pytest.mark.parametrize("bw,nb", [(32, 3), (64, 2), (96, 2), (160, 1), (320, 2)])
+@pytest.mark.parametrize("bw,nb", [(32, 3), (64, 2), (96, 2), (160, 1), (320, 2), (8, 5), (40, 3), (104, 1), (240, 2)])
 def test_prepared_image_does_not_depend_on_the_alignment_of_the_weights(bw, nb):
     """Weights on a 16-byte boundary are copied and turned by vectors, others element by element: the same image, byte for byte."""
     from griffin_amd import _lib
