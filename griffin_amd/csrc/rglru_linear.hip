@@ -24,8 +24,8 @@
 // there, 4 us for the results (timing builds), the rest MFMAs of the 48 compute units that have two of the 304 tiles.  us before ->
 // with direct slices, bias asked for in front of them: 2331 x 2 x 1024 x 768 20.3 -> 14.8, x 768 x 1024 11.6 -> 9.8; 4096 x 2 x 1024 x 768
 // 22.4 -> 18.9; 8192 41.5 -> 34.4; 16384 x 2048 x 2048 166 -> 136 (1012 TFLOP/s).  fp32, bound by its MFMAs: 34.1 -> 32.8 at 800
-// x 2 x 1024 x 768, 389 -> 387 at 16384.  Three or four slices of 128 x 128 (one workgroup a compute unit): 23.0, 16.4 against 16.6; tiles of
-// 128 x 64: 16.5; both operands' tiles per XCD in another order: no change.
+// x 2 x 1024 x 768, 389 -> 387 at 16384.  Three or four slices of 128 x 128 (one workgroup a compute unit): 23.0, 16.4 against 16.6;
+// both operands' tiles per XCD in another order: no change.  Sizes of the tiles: forward16_plan.
 // The gradients, through registers: the order of a slice below, operand pointers outside the loop and results staged four columns
 // at a time took the gate gradients of B4 T1024 W1024 in fp32 from 39.5 to 37 us; more slices in flight (3, 4 or 6) gained nothing.
 #include <hip/hip_runtime.h>

@@ -2002,17 +2002,18 @@ MaybeTensor block_train_packed(const Tensor& x, const std::vector<Tensor>& p, co
   return packed <= 0 ? std::nullopt : block_train_node(x, p, pos, std::nullopt, rows, std::nullopt, u, std::nullopt, false, c, packed);
 }
 
-// Right-padded batches are packed (BlockTrain::Packed) where products are long enough for the launches around it to pay, and a tenth of
+// Right-padded batches are packed (BlockTrain::Packed) where products are long enough for the launches around it to pay, and a quarter of
 // the tokens or more is padding.  Training step of the block, half of the tokens padding, us, not packed : packed (multiply-adds of a product of
 // all tokens): 768 -> 1024 at 2.2e9 226 : 237, 3.1e9 243 : 237, 4.1e9 269 : 247, 6.8e9 374 : 296, 1.0e10 (64 rows) 507 : 359, 1.3e10 538 : 434; 512 ->
-// 512 at 4.3e9 302 : 269.  Rows: multiples of 64, and of 512 from 8192 on, where the BLAS library may take products (a size it has not seen
-// costs it a search).
+// 512 at 4.3e9 302 : 269.  With 30, 50, 60, 70 and 80 % of the tokens active: B8 T2048 768 -> 1024 537 : 307, 389, 449, 512, 547; B16 T2048 960 : 513,
+// 656, 775, 898, 995; B6 T1000 2048 -> 2048 710 : 375, 493, 551, 616, 685.  Rows: multiples of 64, and of 512 from 8192 on, where the BLAS
+// library may take products (a size it has not seen costs it a search).
 bool block_may_pack(const Tensor& x, const Tensor& w) {
   return x.dim() == 3 && x.size(0) > 1 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && double(x.numel()) * w.size(0) >= 3e9 && !rglru_hip_reproducible();
 }
 int64_t block_packed_rows(int64_t B, int64_t T, int64_t active_tokens) {
   const int64_t grain = active_tokens >= 8192 ? 512 : 64, rows = (std::max<int64_t>(active_tokens, 1) + grain - 1) / grain * grain;
-  return 10 * rows <= 9 * B * T ? rows : 0;
+  return 4 * rows <= 3 * B * T ? rows : 0;
 }
 
 // x w^T + b without a graph.

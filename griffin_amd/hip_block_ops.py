@@ -171,7 +171,7 @@ def hip_block_step_captured(batch: int, width: int, dim: int) -> bool:
 def hip_block_infer(x: Tensor, parameters, prep, conv_state: Tensor | None, rnn_state: Tensor | None, prev_pos: Tensor | None,
                     segment_pos: Tensor | None, flags: Tensor | None, rows: Tensor | None, active: Tensor | None, u: Tensor | None,
                     v: Tensor | None, need_state: bool):
-    """The whole recurrent block over sequences without gradients (griffin/griffin.py:459-528), four launches.  ``parameters``:
+    """The whole recurrent block over sequences without gradients (griffin/griffin.py:459-528), three launches (four behind the BLAS library's products).  ``parameters``:
     weights and biases of linear_x, linear_y and the convolution, the five of the RG-LRU, weight and bias of linear_out; ``prep`` the
     image of the RG-LRU's.  Every token active: positions follow ``prev_pos`` [B] or are ``segment_pos`` [B, T].  Right-padded:
     ``flags`` and ``rows`` of ``token_facts``, ``active`` the mask.  ``u``, ``v``: the projections if the caller has them.  Returns

@@ -448,3 +448,10 @@ def test_operands_on_different_gpus_are_refused():
             moved = list(step)
             moved[at] = moved[at].to("cuda:1")
             assert native.block_step(*moved) is None
+
+
+@pytest.mark.parametrize("active,rows", [(0, 64), (1, 64), (65, 128), (8191, 8192), (8192, 8192), (8193, 8704), (12288, 12288), (12289, 0), (16384, 0)])
+def test_right_padded_batches_are_packed_from_a_quarter_of_padding_on(active, rows):
+    from griffin_amd import _lib
+
+    assert _lib.native().block_packed_rows(8, 2048, active) == rows
