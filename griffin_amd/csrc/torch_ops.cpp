@@ -1395,9 +1395,9 @@ bool vector_rows(const Tensor& t) {
   return t.is_contiguous() && (t.size(-1) * t.element_size()) % 16 == 0 && is_aligned(t);
 }
 
-// A tensor that dispatches itself (a subclass with __torch_dispatch__: quantised or distributed weights, wrapped inputs) has no
-// memory for a kernel to read; PyTorch's product takes it.
-bool plain(const Tensor& t) { return !t.defined() || !t.key_set().has(c10::DispatchKey::Python); }
+// A tensor that dispatches itself (a subclass with __torch_dispatch__: quantised or distributed weights, wrapped inputs) or stands for a batch of
+// them (vmap, batched gradients) has no memory for a kernel to read; PyTorch's product takes it.
+bool plain(const Tensor& t) { return !t.defined() || (!t.key_set().has(c10::DispatchKey::Python) && t.has_storage()); }
 
 // Whether the library takes y = x w^T + b (and its gradients) for these operands.
 bool own_linear(const Tensor& x, const Tensor& w, const Tensor& b, Product use = Product::kInference) {
@@ -1525,7 +1525,7 @@ struct Linear : torch::autograd::Function<Linear> {
       c10::DeviceGuard guard(x.device());
       Needs need(ctx);
       const int64_t bias_type = unpack(ctx)[0];
-      if (own_linear(x, weight, Tensor(), Product::kGradient) && grads[0].scalar_type() == x.scalar_type() && (bias_type == kNone || bias_type == (int64_t)x.scalar_type())) {
+      if (own_linear(x, weight, Tensor(), Product::kGradient) && plain(grads[0]) && grads[0].scalar_type() == x.scalar_type() && (bias_type == kNone || bias_type == (int64_t)x.scalar_type())) {
         std::tie(dx, dw, db) = own_backward(x, weight, grads[0], s[2], need(0), need(1), need(2));
         return once({dx, dw, db, Tensor()});
       }
@@ -1636,7 +1636,7 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
       Tensor both = stacked_halves(grads[0], grads[1]);
       const auto dtype = x.scalar_type();
       auto usual = [&](int64_t t) { return t == kNone || t == (int64_t)dtype; };
-      if (grads[0].defined() && grads[1].defined() && grads[0].scalar_type() == dtype && grads[1].scalar_type() == dtype &&
+      if (grads[0].defined() && grads[1].defined() && plain(grads[0]) && plain(grads[1]) && grads[0].scalar_type() == dtype && grads[1].scalar_type() == dtype &&
           own(x, w1, Tensor(), w2, Tensor(), Product::kGradient) && usual(m[0]) && usual(m[1])) {
         Tensor g0 = grads[0], g1 = grads[1];
         const int64_t N = w1.size(0), K = w1.size(1), rows = x.numel() / K;

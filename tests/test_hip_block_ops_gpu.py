@@ -1133,6 +1133,23 @@ def test_gradient_products_in_every_tile_read_only_their_operands(kind, pair, M,
         assert ((sums.double().sum(0)[i] - live.sum(0)).abs() <= (K + 2) * 2.0 ** -24 * live.abs().sum(0)).all()
 
 
+# multiply-adds between the lines of inference and of gradients, and past both with tokens that do not divide into 2048
+@pytest.mark.parametrize("rows,N,K", [(1100, 2048, 2816), (2200, 2048, 2816)])
+def test_linear_layers_take_batches_of_gradients(rows, N, K):
+    """Batched gradients have no memory for a kernel to read: hip_linear and hip_linear_pair give them to PyTorch's products, one by one the same."""
+    from griffin_amd.hip_block_ops import hip_linear, hip_linear_pair
+
+    _say("batched gradients", rows, N, K)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x, w1, w2 = (torch.randn(*s, generator=gen, device="cuda").bfloat16().requires_grad_(True) for s in ((rows, K), (N, K), (N, K)))
+    dy = torch.randn(2, 2, rows, N, generator=gen, device="cuda").bfloat16()
+    for outs, leaves in (([hip_linear(x, w1, None)], (x, w1)), (list(hip_linear_pair(x, w1, None, w2, None)), (x, w1, w2))):
+        both = torch.autograd.grad(outs, leaves, [dy[i] for i in range(len(outs))], retain_graph=True, is_grads_batched=True)
+        for i in range(2):
+            for got, want in zip(both, torch.autograd.grad(outs, leaves, [dy[j, i] for j in range(len(outs))], retain_graph=True)):
+                assert rel_err(got[i].float(), want.float()) < 1e-2      # two roundings to bf16, sums in another order
+
+
 @pytest.mark.parametrize("padded", [False, True])
 @pytest.mark.parametrize("B,T,D,W,nb", [(2, 1, 64, 96, 3), (3, 37, 72, 128, 2), (2, 333, 192, 256, 16), (2, 4097, 768, 1024, 16), (4, 2048, 1536, 2048, 16)])
 def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded):
