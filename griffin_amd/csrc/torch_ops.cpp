@@ -1616,6 +1616,9 @@ struct LinearPair : torch::autograd::Function<LinearPair> {
   }
   static std::tuple<Tensor, Tensor> values(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
     if (!own(x, w1, b1, w2, b2)) return {at::linear(x, w1, maybe(b1)), at::linear(x, w2, maybe(b2))};
+    return own_values(x, w1, b1, w2, b2);
+  }
+  static std::tuple<Tensor, Tensor> own_values(const Tensor& x, const Tensor& w1, const Tensor& b1, const Tensor& w2, const Tensor& b2) {
     c10::DeviceGuard guard(x.device());
     at::DimVector size(x.sizes());
     size.back() = w1.size(0);
@@ -1746,9 +1749,10 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       return run(ctx, x, wx, bx, wy, by, cw, cb, wa, ba, wi, bi, lam, wo, bo, pos, opt(flags_), opt(rows_), opt(active_), opt(u_), opt(v_), first_reset, c,
                  Packed());
     // Right-padded rows that are documents from their beginning become ONE row of documents without the padding, so that every product
-    // and scan runs on the tokens that count; rows_ starts with the number of them in each row, u_ is the first projection of all tokens.
+    // and scan runs on the tokens that count; rows_ starts with the number of them in each row, u_ is the first projection of all tokens, v_ the
+    // second where it is there already.
     c10::DeviceGuard guard(x.device());
-    const Packed p = {x.size(0), x.size(1), packed, *rows_, x, *u_};
+    const Packed p = {x.size(0), x.size(1), packed, *rows_, x, *u_, opt(v_)};
     Tensor tokens = fresh({1, packed, x.size(2)}, kType, x);
     Tensor positions = fresh({1, packed}, at::kLong, x), flags = fresh({1, packed}, at::kByte, x);
     Tensor live = run(ctx, tokens, wx, bx, wy, by, cw, cb, wa, ba, wi, bi, lam, wo, bo, positions, flags, Tensor(), Tensor(), Tensor(), Tensor(), false, c, p);
@@ -1757,7 +1761,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
 
   struct Packed {
     int64_t B = 0, T = 0, rows = 0;                          // of the padded batch; rows: 0 where it was not packed
-    Tensor counts, x, u;
+    Tensor counts, x, u, v;
     Tensor unpack(const Tensor& src) const {
       Tensor dst = fresh({B, T, src.size(-1)}, kType, src);
       check(rglru_hip_unpack_rows(static_cast<const int32_t*>(ptr(counts)), ptr(src), ptr(dst), src.size(-1) * 2, B, T, rows, stream_of(src)),
@@ -1785,7 +1789,10 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
       check(rglru_hip_pack_rows(static_cast<const int32_t*>(ptr(packed.counts)), ptr(packed.x), ptr(x), D * 2, ptr(packed.u), s[3], W * 2,
                                 static_cast<int64_t*>(pos.data_ptr()), static_cast<uint8_t*>(flags.data_ptr()), packed.B, packed.T, packed.rows, stream),
             "rglru_hip_pack_rows");
-      if (own_forward) {
+      if (packed.v.defined()) {
+        check(rglru_hip_pack_rows(static_cast<const int32_t*>(ptr(packed.counts)), ptr(packed.v), s[4], W * 2, nullptr, nullptr, 0, nullptr, nullptr, packed.B,
+                                  packed.T, packed.rows, stream), "rglru_hip_pack_rows");
+      } else if (own_forward) {
         linear_forward(x, wy, by, Tensor(), Tensor(), Tensor(), s[4], nullptr);
       } else {
         Tensor out_v = part(buffer, 4 * tensor_bytes, {M, W}, kType);
@@ -1834,7 +1841,7 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
                  &rows = saved[7], &active = saved[8], &u = saved[9], &v = saved[10], &buffer = saved[11];
     const bool first_reset = m[0];
     const int64_t nb = m[1];
-    const Packed packed = {m[3], m[4], m[5], saved[12], Tensor(), Tensor()};
+    const Packed packed = {m[3], m[4], m[5], saved[12], Tensor(), Tensor(), Tensor()};
     variable_list g(23);
     {
       at::NoGradGuard no_grad;
@@ -1977,10 +1984,10 @@ MaybeTensor block_train_node(const Tensor& x, const std::vector<Tensor>& p, cons
   // p: the node's tensors behind x
   const Tensor &wx = p[N::WX - 1], &cw = p[N::CW - 1], &wa = p[N::WA - 1];
   const int64_t W = wx.size(0);
-  // packed: the number of rows that the tokens that count are packed to; u is then there alone
+  // packed: the number of rows that the tokens that count are packed to; u may then be there alone
   if (packed > 0 && (!u.has_value() || !rows.has_value() || packed > B * T || rglru_hip_reproducible())) return std::nullopt;
   if (x.scalar_type() != N::kType || !vector_rows(x) || W % 8 ||
-      !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), packed > 0 ? opt(u) : opt(v)) ||
+      !token_shapes(B, T, W, pos, opt(flags), opt(rows), opt(active), opt(u), packed > 0 && !v.has_value() ? opt(u) : opt(v)) ||
       (u.has_value() && u->scalar_type() != N::kType) || (B * T + 64) * 2 * W * 2 >= (int64_t(1) << 31) || B * T * W * 2 > (int64_t(1) << 30) || !rglru_hip_block_fwd_path(W, wa.size(0), cw.size(2), RGLRU_BF16))
     return std::nullopt;
   // the gated reverse scan in tiles adds the gradient of linear_y's bias up in the order of its tickets
@@ -1997,9 +2004,9 @@ MaybeTensor block_train(const Tensor& x, const std::vector<Tensor>& p, const Ten
                         const MaybeTensor& active, const MaybeTensor& u, const MaybeTensor& v, bool first_reset, double c) {
   return block_train_node(x, p, pos, flags, rows, active, u, v, first_reset, c, 0);
 }
-MaybeTensor block_train_packed(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const Tensor& rows, const Tensor& u, int64_t packed,
-                               double c) {
-  return packed <= 0 ? std::nullopt : block_train_node(x, p, pos, std::nullopt, rows, std::nullopt, u, std::nullopt, false, c, packed);
+MaybeTensor block_train_packed(const Tensor& x, const std::vector<Tensor>& p, const Tensor& pos, const Tensor& rows, const Tensor& u, const MaybeTensor& v,
+                               int64_t packed, double c) {
+  return packed <= 0 ? std::nullopt : block_train_node(x, p, pos, std::nullopt, rows, std::nullopt, u, v, false, c, packed);
 }
 
 // Right-padded batches are packed (BlockTrain::Packed) where products are long enough for the launches around it to pay, and a quarter of
@@ -2023,6 +2030,21 @@ Tensor linear_values(const Tensor& x, const Tensor& w, const MaybeTensor& b) {
   require_device_of("hip_linear", x, {&w, &bias});
   at::NoGradGuard no_grad;
   return Linear::values(x, w, bias, Tensor());
+}
+
+// The input projections of a training batch that may be packed, queued before the mask's answer is there: both where they are one launch of the
+// library, else the first alone, and the second follows on the tokens that turn out to count.  The first alone everywhere leaves the device idle
+// until the host has woken up: steps, us, alone : together, every token active (half of them in brackets): 768 -> 1024 at 3.2e9 multiply-adds 218 : 197 (211 :
+// 181), 4.1e9 250 : 232 (220 : 202), 5.5e9 271 : 266 (244 : 236), 7.1e9 346 : 319 (271 : 268); 1536 -> 2048 at 4.1e9 243 : 227 (227 : 212), 5.5e9 272 :
+// 256 (233 : 221).  Past the library's line a BLAS product covers most of the wait (1.3e10, every token active: 490 to 500 either way).
+std::tuple<Tensor, MaybeTensor> block_projections(const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2, const MaybeTensor& b2) {
+  const Tensor bias1 = opt(b1), bias2 = opt(b2);
+  refuse_tangents("hip_linear_pair", std::initializer_list<Tensor>{x, w1, bias1, w2, bias2});
+  require_device_of("hip_linear_pair", x, {&w1, &bias1, &w2, &bias2});
+  at::NoGradGuard no_grad;
+  if (!LinearPair::own(x, w1, bias1, w2, bias2, Product::kTrainingForward)) return {Linear::values(x, w1, bias1, Tensor()), std::nullopt};
+  auto [u, v] = LinearPair::own_values(x, w1, bias1, w2, bias2);
+  return {u, v};
 }
 
 // The whole block over sequences without gradients (griffin/griffin.py:459-528): projections, positions, convolution, RG-LRU
@@ -2231,6 +2253,7 @@ PYBIND11_MODULE(_native, m) {
   EXPORT(linear_pair);
   EXPORT(linear_pair_values);
   EXPORT(linear_values);
+  EXPORT(block_projections);
   EXPORT(block_may_pack);
   EXPORT(block_packed_rows);
   EXPORT(block_train);

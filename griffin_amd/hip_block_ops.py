@@ -119,16 +119,22 @@ def hip_block_may_pack(x: Tensor, w: Tensor) -> bool:
     return _lib.native().block_may_pack(x, w)
 
 
-def hip_block_train_packed(x: Tensor, parameters, facts, u: Tensor, c: float) -> Tensor | None:
+def hip_block_projections(x: Tensor, w_u: Tensor, b_u: Tensor | None, w_v: Tensor, b_v: Tensor | None):
+    """The values of linear_x and linear_y for ``hip_block_train_packed``; the second is None where it would be a launch of its own and is
+    better made for the active tokens alone."""
+    return _lib.native().block_projections(x, w_u, b_u, w_v, b_v)
+
+
+def hip_block_train_packed(x: Tensor, parameters, facts, u: Tensor, v: Tensor | None, c: float) -> Tensor | None:
     """``hip_block_forward`` with ``around`` on a batch whose rows are right-padded documents from their beginning: products and scans
-    run on the active tokens alone, packed one row behind the other.  ``facts``: resolved ``token_facts`` of the mask; ``u``: the
-    values of linear_x on all tokens.  Returns the output [B, T, D], or None where there is too little padding, or the operator does not
+    run on the active tokens alone, packed one row behind the other.  ``facts``: resolved ``token_facts`` of the mask; ``u``, ``v``:
+    ``hip_block_projections``.  Returns the output [B, T, D], or None where there is too little padding, or the operator does not
     take the operands."""
     native = _lib.native()
     rows = native.block_packed_rows(x.shape[0], x.shape[1], facts.active_tokens)
     if rows == 0:
         return None
-    return native.block_train_packed(x, parameters, facts.conv_positions, facts.rows, u, rows, c)
+    return native.block_train_packed(x, parameters, facts.conv_positions, facts.rows, u, v, rows, c)
 
 
 def hip_block_decode_step(u: Tensor, v: Tensor, conv_state: Tensor | None, weight: Tensor, bias: Tensor | None,

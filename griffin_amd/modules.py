@@ -654,16 +654,14 @@ class RecurrentBlock(_HoldsLeaves):
             facts = hip_block_ops.token_facts(active_mask, segment_pos, None)
             # queued before the facts are asked for: the answer arrives while the projections run
             packs = segment_pos is None and hip_block_ops.hip_block_may_pack(x, w_u)
-            if packs:
-                u = hip_block_ops.hip_linear_values(x, w_u, b_u)
-            else:
-                u, v = hip_block_ops.hip_linear_pair_values(x, w_u, b_u, w_v, b_v)
+            project = hip_block_ops.hip_block_projections if packs else hip_block_ops.hip_linear_pair_values
+            u, v = project(x, w_u, b_u, w_v, b_v)
             dense, right_padded = facts.resolve()
-            if packs:
-                if right_padded and not dense:
-                    done = hip_block_ops.hip_block_train_packed(x, parameters, facts, u, self.rg_lru.c)
-                    if done is not None:
-                        return done, facts, None
+            if packs and right_padded and not dense:
+                done = hip_block_ops.hip_block_train_packed(x, parameters, facts, u, v, self.rg_lru.c)
+                if done is not None:
+                    return done, facts, None
+            if v is None:
                 v = hip_block_ops.hip_linear_values(x, w_v, b_v)
             if dense:
                 positions = facts.positions

@@ -1275,6 +1275,33 @@ def test_block_trains_on_right_padded_batches_without_their_padding(B, T, D, W, 
         assert err < 1e-2 and float((a.float() - w.float()).norm() / norm) < 1e-2, name
 
 
+# multiply-adds of a projection: 3.1e9, 7.1e9, 1.3e10
+@pytest.mark.parametrize("B,T,together", [(4, 1000, True), (8, 1125, True), (8, 2048, False)])
+def test_projections_of_a_batch_that_may_be_packed_are_one_launch_where_they_can(B, T, together):
+    """Both projections are queued in front of the wait for the mask where they are one launch, and an all-true mask then asks for no other; the
+    values are those of the two layers."""
+    from griffin_amd import RecurrentBlock, hip_block_ops
+
+    _say("projections in front of the mask", B, T)
+    torch.manual_seed(2)
+    block = RecurrentBlock(768, 1024, gate_blocks=16, scan_mode="hip").cuda().to(torch.bfloat16)
+    x = torch.randn(B, T, 768, device="cuda", dtype=torch.bfloat16)
+    layers = block.linear_x, block.linear_y
+    assert hip_block_ops.hip_block_may_pack(x, layers[0].weight)
+    u, v = hip_block_ops.hip_block_projections(x, *(t for m in layers for t in (m.weight, m.bias)))
+    assert (v is not None) == together
+    for got, m in zip((u, v), layers):
+        if got is not None:
+            assert rel_err(got.float(), torch.nn.functional.linear(x.float(), m.weight.float(), m.bias.float())) < 4e-3      # one rounding to bf16
+    alone, real = [], hip_block_ops.hip_linear_values
+    hip_block_ops.hip_linear_values = lambda *args: alone.append(1) or real(*args)
+    try:
+        block(x.requires_grad_(True), active_mask=torch.ones(B, T, dtype=torch.bool, device="cuda"))
+    finally:
+        hip_block_ops.hip_linear_values = real
+    assert len(alone) == (0 if together else 1)
+
+
 @pytest.mark.parametrize("tokens", ["all", "positions", "padded"])
 @pytest.mark.parametrize("B,T,D,W,nb,carried", [(2, 2, 64, 96, 3, True), (3, 77, 72, 128, 2, True), (1, 1000, 192, 256, 16, False), (3, 2777, 1536, 2048, 16, True)])
 def test_block_inference_in_one_call_matches_layer_by_layer(B, T, D, W, nb, carried, tokens):
