@@ -181,7 +181,8 @@ __global__ __launch_bounds__(256) void mask_rows_kernel(MaskRowsArgs p) {
 // `packed` rows and back.  A workgroup has sixteen tokens of a row; where the row lies follows from the counts of the rows in front of it.  What
 // is left behind the last row is one more row, of zeros.  PACK: up to two arrays, and the positions and flags (as
 // rglru_hip_block_fwd takes them) of tokens whose rows are documents from their beginning.  Else: one array, padding becomes zero.
-// Streaming, a batch of eight vectors in flight per thread; what lies past the ends is dropped by the descriptors.
+// Streaming, a batch of eight vectors in flight per thread; what lies past the ends is dropped by the descriptors.  Counts that do not fit (more
+// than T, or more than `packed` together) lose their tail: nothing outside the arrays is read or written whatever they say.
 struct PackArgs {
   const int* counts; const f32x4* src[2]; f32x4* dst[2]; int per_row[2];
   long long* pos; unsigned char* flags; int B, T, packed, chunks;
@@ -192,8 +193,9 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p) {
   constexpr int kTokens = kPackTokens, AHEAD = 8;
   __shared__ int lds[4];
   const int b = blockIdx.x / p.chunks, chunk = blockIdx.x - b * p.chunks;
+  auto count = [&](int i) { return min(max(p.counts[i], 0), p.T); };
   int before = 0;
-  for (int i = threadIdx.x; i < b; i += 256) before += p.counts[i];
+  for (int i = threadIdx.x; i < b; i += 256) before += count(i);
 #pragma unroll
   for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d);
   if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = before;
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p) {
   const int first = lds[0] + lds[1] + lds[2] + lds[3];
   const bool tail = b == p.B;                   // PACK only
   // tokens of the row that exist, and those that this launch writes
-  const int there = tail ? 0 : p.counts[b], rows = PACK ? (tail ? p.packed - first : there) : p.T;
+  const int there = tail ? 0 : count(b), rows = PACK ? (tail ? p.packed - first : there) : p.T;
   for (int t0 = chunk * kTokens; t0 < rows; t0 += p.chunks * kTokens) {
     const int n = rows - t0 < kTokens ? rows - t0 : kTokens;
     const long long wide = (long long)b * p.T + t0, narrow = (long long)first + t0;
@@ -211,9 +213,10 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p) {
       const unsigned per_row = (unsigned)p.per_row[a], all = (unsigned)n * per_row;
       const f32x4* src = p.src[a] + (PACK ? wide : narrow) * per_row;
       f32x4* dst = p.dst[a] + (PACK ? narrow : wide) * per_row;
-      // vectors that exist, and that may be written (counts that do not fit `packed` lose their tail)
-      const int left = there - t0 < n ? there - t0 : n, fit = PACK && p.packed - narrow < n ? (int)(p.packed - narrow) : n;
-      const unsigned live = left > 0 ? (unsigned)left * per_row : 0u, room = fit > 0 ? (unsigned)fit * per_row : 0u;
+      // vectors that exist, and that may be written
+      const int left = there - t0 < n ? there - t0 : n, fit = p.packed - narrow < n ? (int)(p.packed - narrow) : n;
+      const int from_rows = PACK ? left : min(left, fit), to_rows = PACK ? fit : n;
+      const unsigned live = from_rows > 0 ? (unsigned)from_rows * per_row : 0u, room = to_rows > 0 ? (unsigned)to_rows * per_row : 0u;
       const rsrc_t from = make_rsrc(src, live * 16u), to = make_rsrc(dst, room * 16u);
       for (unsigned i0 = threadIdx.x; i0 < all; i0 += 256 * AHEAD) {
         i32x4 v[AHEAD];

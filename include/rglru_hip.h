@@ -277,9 +277,10 @@ int rglru_hip_pack_flags(const uint8_t* reset, const uint8_t* active, uint8_t* f
 int rglru_hip_mask_rows(const void* src, const uint8_t* active, void* dst, int64_t rows, int64_t D, int dtype, void* stream);
 
 /* Rows of `bytes` bytes of [B, T] tokens whose first counts[b] (rglru_hip_token_facts) are active, packed one row behind the other without
- * their padding, and back (padding becomes zero).  `packed` >= the sum of the counts; what is left of it is filled with zeros.  src1 / dst1
- * / bytes1: a second array, or NULL.  pos[packed], flags[packed] (both or neither): positions and the flags of rglru_hip_block_fwd where every
- * row is a document from its beginning; what is left is one more.  Rows are whole 16-byte vectors on a 16-byte boundary. */
+ * their padding, and back (padding becomes zero).  `packed` >= the sum of the counts (rows that do not fit are dropped); what is left of it is
+ * filled with zeros.  src1 / dst1 / bytes1: a second array, or NULL.  pos[packed], flags[packed] (both or neither): positions and the flags of
+ * rglru_hip_block_fwd where every row is a document from its beginning; what is left is one more.  Rows are whole 16-byte vectors on a 16-byte
+ * boundary. */
 int rglru_hip_pack_rows(const int32_t* counts, const void* src0, void* dst0, int64_t bytes0, const void* src1, void* dst1, int64_t bytes1,
                         int64_t* pos, uint8_t* flags, int64_t B, int64_t T, int64_t packed, void* stream);
 int rglru_hip_unpack_rows(const int32_t* counts, const void* src, void* dst, int64_t bytes, int64_t B, int64_t T, int64_t packed, void* stream);

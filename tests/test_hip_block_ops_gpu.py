@@ -1228,6 +1228,25 @@ def test_rows_are_packed_and_unpacked(B, T, counts, packed):
     assert torch.equal(flags.cpu(), torch.cat(((near | (want == 0)), torch.tensor([77]))).to(torch.uint8))
 
 
+def test_rows_past_the_packed_ones_are_not_touched():
+    """Counts that say more than there is: a row has at most T tokens, and what does not fit the packed rows is dropped by either direction (every array
+    here has memory behind its end)."""
+    from griffin_amd import _lib
+
+    _say("pack", "counts that do not fit")
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    B, T, packed = 2, 5, 8
+    counts = torch.tensor([4, 9], dtype=torch.int32, device="cuda")                      # 4 and T; 8 of the 9 rows fit
+    wide = torch.full((B * T + 8, 4), float("nan"), device="cuda")
+    wide[:B * T] = torch.arange(1.0, B * T + 1)[:, None]
+    narrow, back = torch.full((packed + 8, 4), 7.0, device="cuda"), torch.full((B * T + 8, 4), 7.0, device="cuda")
+    _lib.check(lib.rglru_hip_pack_rows(counts.data_ptr(), wide.data_ptr(), narrow.data_ptr(), 16, None, None, 0, None, None, B, T, packed, stream), "pack_rows")
+    narrow[packed:] = float("nan")
+    _lib.check(lib.rglru_hip_unpack_rows(counts.data_ptr(), narrow.data_ptr(), back.data_ptr(), 16, B, T, packed, stream), "unpack_rows")
+    assert narrow[:, 0].tolist()[:packed] == [1, 2, 3, 4, 6, 7, 8, 9]
+    assert back[:, 0].tolist() == [1, 2, 3, 4, 0, 6, 7, 8, 9, 0] + [7] * 8
+
+
 @pytest.mark.parametrize("B,T,D,W,nb,lengths", [(5, 1700, 768, 1024, 8, [0, 1, 2, 3, 1700]), (150, 33, 768, 1024, 16, None), (3, 2000, 640, 832, 8, [2000, 1, 1500]),
                                                 (9, 2048, 768, 1024, 16, [2048, 2048, 5, 2048, 64, 128, 2047, 1, 513]), (4, 1100, 768, 1024, 8, [0, 0, 0, 0])])
 def test_block_trains_on_right_padded_batches_without_their_padding(B, T, D, W, nb, lengths):
