@@ -55,7 +55,7 @@
 extern "C" {
 #endif
 
-#define RGLRU_ABI_VERSION 23
+#define RGLRU_ABI_VERSION 24
 
 enum { RGLRU_F32 = 0, RGLRU_BF16 = 1 };
 

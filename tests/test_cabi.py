@@ -51,6 +51,11 @@ def test_library_exports_every_declared_symbol(lib):
     assert lib.rglru_hip_max_block_width() == 512
 
 
+def test_version_tells_of_the_counts_in_the_words_for_the_host(lib):
+    """rglru_hip_token_facts writes more than its two bits since version 24; a caller built against 23 compares the whole word."""
+    assert lib.rglru_hip_abi_version() >= 24
+
+
 def test_size_queries(lib):
     assert lib.rglru_hip_prep_bytes(1024, 8, _lib.RGLRU_BF16) > 2 * 8 * 128 * 128 * 2
     assert lib.rglru_hip_prep_bytes(1024, 8, _lib.RGLRU_F32) > lib.rglru_hip_prep_bytes(1024, 8, _lib.RGLRU_BF16)
