@@ -1187,11 +1187,57 @@ def test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, p
 
 
 # multiply-adds of a product: 1.04e10 (gradients by the library, forward by the BLAS library), 2.6e10 with tokens that do not divide into the
-# BLAS library's batches (weight gradients by the library alone)
+# BLAS library's batches (weight gradients by the library alone).  The padded batches are packed to 1984 and 5056 rows: 6.2e9, all products by the
+# library, and 1.6e10; padding that stays is the next test's.
 @pytest.mark.parametrize("padded", [False, True])
 @pytest.mark.parametrize("B,T,D,W,nb", [(3, 1100, 1536, 2048, 16), (3, 2777, 1536, 2048, 16)])
 def test_block_training_between_the_lines_of_its_products(B, T, D, W, nb, padded):
     test_block_as_one_training_operator_matches_layer_by_layer(B, T, D, W, nb, padded)
+
+
+# multiply-adds of a product, tokens: 1.04e10 and 1.03e10 (gradients by the library, forward by the BLAS library), 3300 and 2 x 2048;  2.6e10 and
+# 1.3e10 (input gradients by the BLAS library; weight gradients by the library in 8331 tokens, by the BLAS library in 8 x 2048)
+@pytest.mark.parametrize("B,T,D,W,nb", [(3, 1100, 1536, 2048, 16), (4, 1024, 1408, 1792, 16), (3, 2777, 1536, 2048, 16), (8, 2048, 768, 1024, 8)])
+@pytest.mark.parametrize("how", ["little padding", "positions"])
+def test_block_trains_on_long_right_padded_batches_with_their_padding(B, T, D, W, nb, how):
+    """Right-padded batches that are not packed, for little padding (90 % active) or because the caller gives positions: the node with masked
+    products and row masks against the block taken layer by layer, on either side of the lines of its products."""
+    from griffin_amd import RecurrentBlock, hip_block_ops
+
+    _say("padded block, not packed", B, T, D, W, nb, how)
+    torch.manual_seed(6)
+    block = RecurrentBlock(D, W, gate_blocks=nb, scan_mode="hip").cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        for name, p in block.named_parameters():
+            if name.endswith("bias"):
+                p.normal_(std=0.1)
+    x = torch.randn(B, T, D, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    dy = torch.randn_like(x)
+    positions = torch.arange(T, device="cuda").repeat(B, 1) if how == "positions" else None
+    active = torch.arange(T, device="cuda")[None] < torch.linspace(T // 5 if how == "positions" else 4 * T // 5, T, B, device="cuda").long()[:, None]
+    names, leaves = zip(*([("x", x)] + list(block.named_parameters())))
+    calls, real = [], hip_block_ops.hip_block_train_packed
+
+    def spy(*args):
+        calls.append(real(*args))
+        return calls[-1]
+
+    hip_block_ops.hip_block_train_packed = spy
+    try:
+        whole = block(x, segment_pos=positions, active_mask=active)
+    finally:
+        hip_block_ops.hip_block_train_packed = real
+    assert calls == ([None] if positions is None else []) and "BlockTrain" in type(whole.grad_fn).__name__ + str(whole.grad_fn.name())
+    got = torch.autograd.grad(whole, leaves, dy)
+    layered, _ = block(x, segment_pos=positions, active_mask=active, return_cache=True)
+    want = torch.autograd.grad(layered, leaves, dy)
+    torch.cuda.synchronize()
+    assert (whole[~active] == 0).all() and (got[0][~active] == 0).all()
+    assert rel_err(whole.float(), layered.float()) < 1e-2
+    for name, g, w in zip(names, got, want):
+        err = float((g.float() - w.float()).norm() / w.float().norm().clamp_min(1e-30))
+        _say("  d%s rel error: %.2e" % (name, err))
+        assert err < 1e-2, name
 
 
 @pytest.mark.parametrize("B,T,counts,packed", [(1, 1, [1], 1), (3, 16, [16, 0, 5], 64), (5, 37, [1, 0, 37, 17, 16], 71), (300, 70, None, 11520), (2, 5000, [4999, 3], 5056),
