@@ -1935,10 +1935,9 @@ struct BlockTrain : torch::autograd::Function<BlockTrain> {
     return once(std::move(g));
   }
 
-  // a^T b over the rows, as the partial products [chunks, columns of a, columns of b] of the BLAS library
+  // a^T b over the rows, as the partial products [chunks, columns of a, columns of b] of the BLAS library (one chunk: the library's own kernel)
   static Tensor contraction(const Tensor& a, const Tensor& b) {
     const int64_t rows = a.size(0), chunks = contraction_chunks(rows), per = rows / chunks;
-    if (chunks == 1) return at::mm(a.t(), b).unsqueeze(0);
     return at::bmm(a.view({chunks, per, a.size(1)}).transpose(1, 2), b.view({chunks, per, b.size(1)}));
   }
 };
