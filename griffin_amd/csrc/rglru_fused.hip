@@ -913,14 +913,18 @@ struct BlockFwd {
 //             64-wide, W1024   B48 38.8 : 39.5 (75), 64 45.4 : 40.1, 80 56.7 : 53.1 (83), 112 75.7 : 68.0 (88), 161 105.7 : 106.9 (84), 256 171 : 146
 //             short sequences, which pay most for the clearing of the tiled kernel's records   T256 20 units B16 24.1 : 24.9 (63), 12 20.9 : 18.4
 //             (94), W1024 B32 20.2 : 18.5; T128 20 units B12 16.2 : 11.5 (94), 48-wide W768 B32 14.6 : 10.2
-//             ragged lengths and padded blocks, which cost the tiled kernel up to a third   T300 B40 31.0 : 30.2 (63), 48 33.1 : 29.9 (75), T777
-//             64 89.6 : 70.2, 128 181 : 127; 96-wide B48 41.0 : 40.6 (75), 64 50.7 : 40.7, 72 56.7 : 53.9 (75), one round 32 30.4 : 30.4
+//             lengths that end inside a tile, which run the plain tiled kernel too   W1024, 128-wide T300 B48 32.4 : 33.4 (75), 56 34.9 : 33.7 (88), 104 55.4 :
+//             52.1 (81, even), T777 56 70.6 : 71.3 (88), 64 83.4 : 78.3, 72 91.5 : 98.7 (75), 128 159 : 129, T1001 56 88.6 : 90.1 (88), 128 194 : 163; 64-wide
+//             T777 48 62.3 : 64.0 (75), 56 69.0 : 66.8 (88), 128 142 : 120
+//             padded blocks, which cost the tiled kernel its masked variant   96-wide, W768 T300 B40 29.8 : 30.3 (63), 48 32.7 : 31.0 (75), 72 41.9 :
+//             39.8 (75), T777 40 56.2 : 62.8 (63), 48 64.4 : 63.5 (75), 64 81.8 : 67.5, T1001 48 76.9 : 76.7 (75), 72 110 : 108 (75)
 //   flags, two workgroups a compute unit, from a sequence for each of them on (three, 64-wide and narrower, always): 96- and 128-wide   B70
 //             68.9 : 68.5 (73), 77 74.7 : 68.0 (80), 97 91.1 : 93.6 (76), 104 96.5 : 96.2 (81), 128 118 : 98; 48-wide B97 83.5 : 75.0, 64-wide B98
 //             88 : 78
-// Sequences of fewer than 128 tokens have the line of the kernel with flags with or without them, and fuller rounds where the tiled
-// kernel runs its plain variant (88 %; 93 where the last round's sequences share their compute units): both kernels are done in 7 to 25 us
-// there, mostly launch (T64 W1024 B32 11.1 : 8.1, left to the tiled one).
+// Sequences of fewer than 128 tokens have the line of the kernel with flags with or without them: both kernels are done in 7 to 25 us
+// there, mostly launch (T64 W1024 B32 12.6 : 11.1, left to the tiled one).  Without flags whole tiles ask for fuller rounds (88 %; 93 where the last
+// round's sequences share their compute units) than lengths that end inside one, whose last tile is as long for the tiled kernel as a whole
+// one: T100 W1024, 128-wide B80 25.3 : 25.4 (83), 112 29.0 : 28.4 (88), 161 38.9 : 37.7 (84); 64-wide B97 27.5 : 25.0 (76), 161 36.2 : 34.2 (84).
 static int fwd_row_workgroups(int64_t B, int64_t T, const Geometry& g, int nkg, bool masked, bool flags) {
   FusedArgs a;
   a.units = (int)g.units;

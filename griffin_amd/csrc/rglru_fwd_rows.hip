@@ -9,10 +9,10 @@ namespace rglru {
 // as soon as this one is in LDS.  Calls with flags have a variant of their own: they come as one byte a lane and become two words by
 // ballot, and a tile without any takes the plain gate math.  Two versions of that math in one kernel cost 40 registers and the
 // scheduler its freedom, so calls without flags do not have them (128-wide: 243 -> 208 registers with 64-token tiles, 142 with 32).
-// Bound by power: 24.5 vector instructions an element, six of them transcendental, and the matrix products beside them draw the
-// clock down to 2.0-2.1 GHz.  Without its loads and stores the kernel takes 500 of 650 us, without its gate math 530, and every
-// arrangement tried takes the same 650-660: tiles of 32 or 64 tokens, tiles requested two ahead, x or y brought into their layout by
-// products with the identity instead of two-byte LDS accesses.
+// Bound by power: 24.8 vector instructions an element, six of them transcendental, and the matrix products beside them draw the
+// clock down to 2.0-2.1 GHz.  In a series where the kernel took 650 us (B256 T2048 W1024; 628 in the one below) it took 500 without its
+// loads and stores, 530 without its gate math, and 650 to 660 in every arrangement tried: tiles requested two ahead, x or y brought into
+// their layout by products with the identity instead of two-byte LDS accesses.
 // Forward of B256 W1024 in calls behind each other (the clock follows the load: a launch between lighter ones says little), us, tiled with
 // the clearing of its records : two workgroups a compute unit with 64-token tiles and both versions of the math : three with 32-token
 // tiles and one: T2048 in 128-wide blocks 708 : 672 : 628, T512 185 : 175 : 162.  With flags 829 : 686, the three-workgroup form

@@ -455,8 +455,8 @@ __global__ __launch_bounds__(kLinearThreads, 2) void linear_kernel(LinearArgs p)
 }
 
 // The weight and input gradients of the gates' products in fp32, in small tiles, in one launch: neither reads what the other writes.  The
-// weight gradients' workgroups have twice the slices and go first.  Steps of the layer in fp32, two launches and one, us: B4 T1024 W1024 (16 gate
-// blocks) 97.9 and 95.8, B8 T2048 338 and 324, B2 T256 W256, which the host bounds, 54.6 and 52.7.
+// weight gradients' workgroups have twice the slices and go first.  Steps of the layer in fp32, two launches and one, us, four processes each: B4 T1024
+// W1024 (16 gate blocks) 97.1 to 100.1 and 96.7 to 97.5, B8 T2048 333 to 335 and 322; B2 T256 W256 is the host's, whose spread (60 to 100) hides it.
 __global__ __launch_bounds__(kLinearThreads, 2) void gate_grads_kernel(LinearArgs weights, LinearArgs input, unsigned first) {
   typedef LinearTile<float, true, true, 64, 64> Weights;
   typedef LinearTile<float, false, true, 64, 64> Input;
@@ -505,13 +505,17 @@ static LinearPlan forward16_plan(int64_t M, int64_t N, int64_t K, int problems) 
 struct TileCost { int edge; unsigned per_cu; double start, slice[3]; };
 // Gradients in bf16: the cheapest by a model of the time in us.  A workgroup of a tile size takes `start` and `slice[n - 1]` for 64 contraction
 // indices with n of them on a compute unit; the units run their tiles in rounds of `per_cu`.  Constants from 64, 128 and 256 on
-// 1000 to 16384 tokens of 768 and 1024 channels.  What it picks, us, sizes 64 : 128 : 256 (* taken; splits behind the slash):
-//   input, two segments of 1024 into 768   2331 *17.9 : 23.2 : 48.8, 4096 25.1 : *23.6, 8704 50.2 : *32.8 : 52.7, 16384 84 : *55.3 : 57.7
-//   input, 768 into 1024   2331 *11.1 : 11.3, 6000 20.6 : *15.9 : 23.2, 8704 28.0 : 25.1 : *24.8, 16384 46.4 : 40.0 : *29.3
-//   weight, two of 1024 x 768   1000 *10.4/2 : 10.5/2, 2331 18.1/2 : *17.0/3 : 19.0/8, 8704 51.7/2 : *39.8/5 : 36.1/10 (and ten sets to add up),
-//          16384 91/6 : 68.1/5 : *57.0/10
-//   weight, 768 x 1024   1000 8.1/4 : 8.3/5, 2331 11.4/4 : *10.7/5, 8704 28.2/4 : *26.1/5 : 30.8/10, 16384 49/4 : *36.6/10 : 36.5/16
-// The kernels they replace, whose slices went through registers: 40.2, 29.8, 64.5 and 31.8 us at 8704 tokens, in the order above.
+// 1000 to 16384 tokens of 768 and 1024 channels.  What it picks, us in calls behind each other, weight gradients with the launch that adds up their sets and the
+// column sums, sizes 64 : 128 : 256 (* taken; splits of that size behind the slash):
+//   input, two segments of 1024 into 768   1000 *12.5 : 21.0 : 48.9, 2331 *17.3 : 22.1 : 48.9, 4096 23.9 : *22.7 : 49.1, 8704 47.8 : *31.1 : 50.4, 16384 79.6 :
+//          *53.6 : 55.5
+//   input, 768 into 1024   1000 *6.9 : 10.1 : 22.2, 2331 *10.9 : 10.4 : 22.4, 6000 19.6 : *15.1 : 22.8, 8704 26.9 : *23.0 : 23.3, 16384 46.1 : 29.8 : *29.0
+//   weight, two of 1024 x 768   1000 *15.2/1 : 19.1/2 : 27.3/4, 2331 *23.9/2 : 24.9/2 : 30.7/8, 4096 32.4/2 : *29.4/5 : 34.8/8, 8704 57.2/2 : *46.2/5 :
+//          47.5/10, 16384 103.9/2 : 76.5/5 : *71.8/10
+//   weight, 768 x 1024   1000 *13.2/2 : 16.2/4 : 20.8/4, 2331 *17.9/4 : 19.5/5 : 26.9/8, 4096 *21.2/4 : 20.5/5 : 29.1/16, 8704 32.9/4 : *30.6/5 : 36.5/20, 16384
+//          54.3/4 : *43.3/10 : 47.4/20
+// Kernels alone at 8704 tokens, in the order above: 30.9, 22.7, 39.1 and 26.1; those they replace, whose slices went through registers, 40.2, 29.8, 64.5 and
+// 31.8.
 static LinearPlan linear16_plan(bool weight, int64_t M, int64_t N, int64_t K, int problems, int segments) {
   static const TileCost input[] = {{64, 3, 2.5, {0.36, 0.47, 0.69}}, {128, 2, 4.5, {0.58, 0.87, 0.0}}, {256, 1, 10.0, {1.43, 0.0, 0.0}}};
   static const TileCost weights[] = {{64, 3, 3.0, {0.39, 0.52, 0.71}}, {128, 2, 6.0, {0.70, 1.18, 0.0}}, {256, 1, 12.0, {1.74, 0.0, 0.0}}};

@@ -1376,11 +1376,17 @@ Tensor sum_sets(const Tensor& sets) {
 // 96 : 102 / 281 : 287, at 8.0e9 116 : 117 / 325 : 336, at 1.3e10 163 : 149 / 453 : 442;  2560 at 6.0e9 126 : 135 / 306 : 303, at 6.7e9 141 : 127 / 327 : 311.  So
 // between 6e9 and 9e9 either way wins somewhere.  fp32, training 768 -> 1024: at 8e8 326 : 469 / 759 : 755, at 9e8 362 : 468 / 843 : 824, at 1.2e9
 // 430 : 463, at 1.6e9 484 : 452;  wide and short ones lose below the line: 2560 -> 2560 at 5.8e8 (88 tokens) 481 : 466 / 1004 : 865, prefill
-// 151 : 123.  Inside a captured graph host time is nothing: there the line lies where the kernels take equally long.
+// 151 : 123.
 // In a training step of the block in bf16, steps queued behind each other, us: gradients on the BLAS library : own, then the forward own as well.
 // 768 -> 1024 at 6.3e9 374 : 317 : 305, 7.9e9 453 : 385 : 377, 9.7e9 442 : 443 : 439, 1.02e10 603 : 475 : 471, 1.3e10 516 : - : 542;  2560 -> 2560 at 6.0e9 482 :
 // 401 : 340, 8.5e9 485 : 395 : 388, 1.18e10 541 : 460 : 474, 1.3e10 542 : - : 516;  1536 -> 2048 at 6.4e9 317 : 278 : 273, 7.5e9 346 : 318 : 331, 9.4e9 388 :
 // 371 : 387, 1.3e10 447 : - : 477.
+// A Linear layer by itself in bf16, forward and backward, gradients own : BLAS: 1024 x 768 at 7884 tokens 69 : 110, 8192 69 : 85, 14336 99 : 118; 2560 x 2560 at
+// 948 79 : 84, 1812 107 : 126; 4096 x 1024 at 2836 109 : 110; the other way at 1024 x 4096, 2836 tokens, 111 : 107 and 4096 x 4096, 372 tokens, 85 : 82.
+// Inside a captured graph host time is nothing.  The line there is where kernels took equally long whose slices went through registers; with those of
+// today it is early.  Captured step in bf16, us, own : gradients alone own : BLAS: 768 -> 1024 at 2.0e9 155 : 167 : 175, 4.8e9 235 : 244 : 264, 9.7e9 406 :
+// 421 : 424; 1536 -> 2048 at 4.7e9 229 : 233 : 229, 9.4e9 330 : 330 : 331, 1.3e10 432 : 428 : 406; 2560 -> 2560 at 5.0e9 270 : 272 : 292, 1.3e10 438 : 444 :
+// 477; without gradients 768 -> 1024 at 4.8e9 66 : 76, 9.7e9 102 : 114; 2560 -> 2560 at 3.3e9 83 : 74, 6.7e9 106 : 95.
 enum class Product { kInference, kTrainingForward, kGradient };
 bool own_products(double macs, at::ScalarType dtype, Product use = Product::kInference) {
   if (!known(dtype)) return false;
@@ -1439,7 +1445,9 @@ struct WeightGrad {
 // dW = dy^T x contracts over all tokens: one GEMM of the BLAS library with K = rows runs at a fraction of the rate of the same
 // work as a batch of GEMMs with K = 2048 whose results are added (100 us against 43 us for 16384 x 1024 x 768 in bf16), so
 // long contractions are split into this many.  Other numbers of tokens (1) take the library's own kernel in bf16: two of 1024 x 768 at 8704 tokens 39
-// us, the BLAS library 66; at 8192 37 : 34, at 16384 59 : 52.
+// us, the BLAS library 66; at 8192 37 : 34, at 16384 59 : 52.  Own : one product of the BLAS library over 90 sizes of 512 to 10000 channels and 2063 to 60000
+// tokens: 0.27 to 0.98 of its time in 84 of them (1024 x 768 at 4851 24 : 39, 2 x 2560 x 2496 at 5539 155 : 188, 4992 x 4608 at 43097 1932 : 2622), 1.03 to
+// 1.12 in six that have no size in common (2 x 3968 x 2688 at 5707 304 : 270); 1.02 to 1.05 at 4096 x 4096 and 8192 x 4096 from 20000 tokens on.
 int64_t contraction_chunks(int64_t rows) {
   int64_t chunks = rows % 2048 == 0 ? rows / 2048 : 1;
   while (chunks > 16 && chunks % 2 == 0) chunks /= 2;
@@ -2012,8 +2020,9 @@ MaybeTensor block_train_packed(const Tensor& x, const std::vector<Tensor>& p, co
 // the tokens or more is padding.  Training step of the block, half of the tokens padding, us, not packed : packed (multiply-adds of a product of
 // all tokens): 768 -> 1024 at 2.2e9 226 : 237, 3.1e9 243 : 237, 4.1e9 269 : 247, 6.8e9 374 : 296, 1.0e10 (64 rows) 507 : 359, 1.3e10 538 : 434; 512 ->
 // 512 at 4.3e9 302 : 269.  With 30, 50, 60, 70 and 80 % of the tokens active: B8 T2048 768 -> 1024 537 : 307, 389, 449, 512, 547; B16 T2048 960 : 513,
-// 656, 775, 898, 995; B6 T1000 2048 -> 2048 710 : 375, 493, 551, 616, 685.  Rows: multiples of 64, and of 512 from 8192 on, where the BLAS
-// library may take products (a size it has not seen costs it a search).
+// 656, 775, 898, 995; B6 T1000 2048 -> 2048 710 : 375, 493, 551, 616, 685.  Rows: multiples of 64, and of 512 from 8192 on.  A size
+// that the BLAS library has not seen costs it 20 to 35 us once, a coarser grain up to 1 % of every step: 60 lengths, 1024 -> 2048, us a step the first time and
+// later, 64 498 and 448, 512 476 and 452; 2560 -> 2560 838 and 822, 830 and 815.
 bool block_may_pack(const Tensor& x, const Tensor& w) {
   return x.dim() == 3 && x.size(0) > 1 && w.dim() == 2 && x.scalar_type() == at::kBFloat16 && double(x.numel()) * w.size(0) >= 3e9 && !rglru_hip_reproducible();
 }
@@ -2033,9 +2042,10 @@ Tensor linear_values(const Tensor& x, const Tensor& w, const MaybeTensor& b) {
 
 // The input projections of a training batch that may be packed, queued before the mask's answer is there: both where they are one launch of the
 // library, else the first alone, and the second follows on the tokens that turn out to count.  The first alone everywhere leaves the device idle
-// until the host has woken up: steps, us, alone : together, every token active (half of them in brackets): 768 -> 1024 at 3.2e9 multiply-adds 218 : 197 (211 :
-// 181), 4.1e9 250 : 232 (220 : 202), 5.5e9 271 : 266 (244 : 236), 7.1e9 346 : 319 (271 : 268); 1536 -> 2048 at 4.1e9 243 : 227 (227 : 212), 5.5e9 272 :
-// 256 (233 : 221).  Past the library's line a BLAS product covers most of the wait (1.3e10, every token active: 490 to 500 either way).
+// until the host has woken up: steps, us, two processes each, alone : together, every token active (half of them in brackets): 768 -> 1024 at 3.2e9
+// multiply-adds 218-234 : 197-222 (211-225 : 181-215), 4.1e9 250-254 : 232-241 (220-235 : 202-223), 5.5e9 271 : 266-269 (244 : 236-241), 7.1e9 346-349 :
+// 319-321 (271 : 268-270); 1536 -> 2048 at 4.1e9 243-245 : 227-239 (227 : 212-226), 5.5e9 272 : 256-262 (234 : 221-233).  Past the library's line a BLAS product
+// covers most of the wait (1.3e10, every token active: 489 to 500 with the first alone, 494 to 497 with both queued).
 std::tuple<Tensor, MaybeTensor> block_projections(const Tensor& x, const Tensor& w1, const MaybeTensor& b1, const Tensor& w2, const MaybeTensor& b2) {
   const Tensor bias1 = opt(b1), bias2 = opt(b2);
   refuse_tangents("hip_linear_pair", std::initializer_list<Tensor>{x, w1, bias1, w2, bias2});

@@ -8,6 +8,7 @@ import shutil
 import subprocess
 
 import pytest
+import torch
 
 from griffin_amd import _lib
 
@@ -49,6 +50,14 @@ def test_library_exports_every_declared_symbol(lib):
         assert hasattr(raw, name), name
     assert lib.rglru_hip_abi_version() == _lib.ABI_VERSION
     assert lib.rglru_hip_max_block_width() == 512
+
+
+@pytest.mark.parametrize("N,K,problems,splits", [(1024, 768, 2, {1000: 1, 2331: 2, 4096: 5, 8704: 5, 16384: 10}),
+                                                 (768, 1024, 1, {1000: 2, 2331: 4, 4096: 4, 8704: 5, 16384: 10})])
+def test_weight_gradients_are_split_as_the_table_beside_their_plan_says(lib, N, K, problems, splits):
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the table is for 256 compute units")
+    assert {rows: lib.rglru_hip_linear_splits(2, N, K, rows, problems, _lib.RGLRU_BF16) for rows in splits} == splits
 
 
 def test_version_tells_of_the_counts_in_the_words_for_the_host(lib):
