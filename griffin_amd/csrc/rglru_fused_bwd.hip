@@ -2084,7 +2084,8 @@ static int bwd_full_kernels(const void* x, const void* y, const void* prep, cons
   a.queues = pick_queues(B, a.wg_per_unit);
   // Tokens past the end: dy reads as zero there, so nothing comes out of them; only a gradient at the final state, which enters behind them,
   // has to pass them unchanged, as in the masked variants.  (Their decays patched in the plain ones: up to 18 registers and two spills
-  // in every call for this one.)  Reverse scan, us, masked : plain: B8 T2049 W1024
+  // in every call for this one.  Their gates are those of x = 0, finite for finite weights; an infinite one, whose gradients are NaN in part at any
+  // length, makes them NaN and so dh0 and the gradients of its block here, too.)  Reverse scan, us, masked : plain: B8 T2049 W1024
   // (128) 27.3 : 25.8, B1 T8191 (64) 25.0 : 23.1; the gradient kernel of the same 63.0 : 57.5, 31.1 : 28.6.
   const bool masked = flags || (dh_last && T % (32 * kDeltaMT) != 0);
   dim3 grid((unsigned)(a.wg_per_unit * a.units));
